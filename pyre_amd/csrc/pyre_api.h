@@ -90,6 +90,16 @@ int pyre_gemm_mid_silu_blocks(int M, int two_i);
 int pyre_gemm_mid_silu_bf16(const void* X, long ldx, const void* W, long ldw, void* out, int M, int two_i,
                             int K, hipStream_t stream);
 
+// The same for any number of rows (prompts, mixed steps), in tiles of up to 256 x 256: out float32 [parts][M][N], where
+// `parts` is what pyre_gemm_tile_parts says for these sizes; the second with a gated unit in its epilogue (see GateShape),
+// out bfloat16 [M][two_i / 2]. N (two_i) a multiple of 16, K of 64.
+int pyre_gemm_tile_supports(int M, int N, int K, long ldx, long ldw);
+int pyre_gemm_tile_parts(int M, int N, int K);
+int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long ldw, float* out, int M, int N, int K, int parts,
+                        hipStream_t stream);
+int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, long ldw, void* out, int M, int two_i, int K, float limit,
+                            float slope, float shift, float cubic, hipStream_t stream);
+
 // tokens: the n tokens of the flat batch to attend for, or null for tokens 0..n-1. max_keys: a
 // bound on the keys that any of them sees (the block table's width in tokens will do); part:
 // n * nq * pyre_attn_generic_spans(max_keys) * (hd + 2) floats of scratch when that is more than one span.

@@ -54,6 +54,10 @@ _SIGNATURES = {
     "pyre_sample": [P, L, P, P, P, I, I, P],
     "pyre_feed_tokens": [P, P, P, I, P],
     "pyre_gemm_skinny_glu_bf16": [P, L, P, L, P, I, I, I, F, F, F, F, P],
+    "pyre_gemm_tile_supports": [I, I, I, L, L],
+    "pyre_gemm_tile_parts": [I, I, I],
+    "pyre_gemm_tile_bf16": [P, L, P, L, P, I, I, I, I, P],
+    "pyre_gemm_tile_glu_bf16": [P, L, P, L, P, I, I, I, F, F, F, F, P],
     "pyre_gemm_mid_glu_bf16": [P, L, P, L, P, I, I, I, F, F, F, F, P],
     "pyre_add_layernorm": [P, P, I, I, L, P, I, P, I, P, I, F, P, P, I, P, I, P, I, I, F, P],
     "pyre_clipped_glu": [P, I, I, L, P, I, I, I, F, F, F, F, P],

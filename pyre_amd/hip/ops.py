@@ -1018,6 +1018,45 @@ def gemm_mid_silu_bf16(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tens
          out.data_ptr(), m, two_i, w_gate_up.shape[1], _stream())
 
 
+@lru_cache(maxsize=4096)
+def gemm_tile_supports(m: int, n: int, k: int, ldx: int, ldw: int) -> bool:
+    from pyre_amd.hip.lib import lib
+
+    return bool(lib().pyre_gemm_tile_supports(m, n, k, ldx, ldw))
+
+
+@lru_cache(maxsize=4096)
+def gemm_tile_parts(m: int, n: int, k: int) -> int:
+    """Into how many parts of k :func:`gemm_tile_bf16` splits a product of these sizes."""
+    from pyre_amd.hip.lib import lib
+
+    return int(lib().pyre_gemm_tile_parts(m, n, k))
+
+
+def gemm_tile_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, parts: int) -> None:
+    """out[s] (float32 [parts, m, N]) = partial sums over k of x[0:m] @ w.T, in tiles of up to 256 x 256;
+    ``parts`` as :func:`gemm_tile_parts` says (or another number that leaves every part 256 k)."""
+    _skinny_common(x, w, m)
+    n = w.shape[0]
+    if out.dtype != torch.float32 or not out.is_contiguous() or out.numel() < parts * m * n or not out.is_cuda:
+        raise KernelError("gemm_tile: out must be contiguous float32 [parts, m, N] on the GPU")
+    call("pyre_gemm_tile_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), m, n, w.shape[1], parts,
+         _stream())
+
+
+def gemm_tile_glu_bf16(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, m: int,
+                       unit: tuple[float, float, float] | None = None) -> None:
+    """out[0:m] (bfloat16 [m, I]) = the gated unit of x @ gate.T and x @ up.T with w_gate_up = [gate; up], in tiles of up
+    to 256 x 256; ``unit`` as for :func:`gemm_skinny_silu_bf16`."""
+    _skinny_common(x, w_gate_up, m)
+    two_i = w_gate_up.shape[0]
+    if (out.dtype != torch.bfloat16 or not out.is_contiguous() or not out.is_cuda or out.dim() != 2
+            or out.shape[1] * 2 != two_i or out.shape[0] < m):
+        raise KernelError("gemm_tile_glu: out must be contiguous bfloat16 [>= m, I] on the GPU")
+    call("pyre_gemm_tile_glu_bf16", x.data_ptr(), x.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), out.data_ptr(), m,
+         two_i, w_gate_up.shape[1], *(_gate_shape(unit) if unit is not None else (0.0, 1.0, 0.0, 0.0)), _stream())
+
+
 def read_bandwidth(device: str = "cuda:0", gib: float = 2.0, blocks: int = 4096, repeats: int = 10) -> float:
     """Measured streaming-read bandwidth in GB/s (a buffer larger than every cache)."""
     import time

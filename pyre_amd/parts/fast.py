@@ -2,10 +2,10 @@
 
 Each function returns None / False when its fast path does not take the case
 (element type, sizes, alignment); the caller then runs the general kernel.
-Nothing here changes what is computed, only by which kernel. Plain matrix
-products with many rows go to the vendor's BLAS through ``torch.mm``, as the
-reference's do (`pyre/model.py:84-87` are ``nn.Linear``); the true 32-bit path
-never comes here.
+Nothing here changes what is computed, only by which kernel. Sizes that no kernel
+of this framework takes go to the vendor's BLAS through ``torch.mm``, as the
+reference's products do (`pyre/model.py:84-87` are ``nn.Linear``), and so do the
+head's logits of many rows; the true 32-bit path never comes here.
 """
 
 from __future__ import annotations
@@ -15,7 +15,7 @@ import torch
 from pyre_amd.hip.ops import DEFAULT_UNITS, Partials
 
 #: most rows the weight-streaming MFMA kernel takes; above, 16-bit products go to the kernel that keeps
-#: up to 256 rows in a block where it pays and else to the BLAS library
+#: up to 256 rows in a block where it pays and else to the one that takes tiles of rows and columns
 SKINNY_MAX_ROWS = 64
 #: the most partial sums of a weight-streaming product
 SKINNY_MAX_KSPLIT = 12
@@ -96,6 +96,23 @@ LIBRARY_F32_ROLES = frozenset({"attn.qkv", "attn.out", "mix.in", "mix.out", "cat
                                "stmoe.router", "stmoe.down", "side.gate", "side.proj", "lattn.q_up", "poly.up",
                                "poly.down", "light.in", "light.out", "ssm.in", "ssm.out", "ssm.x", "ssm.dt", "reglu.down",
                                "pass.start", "pass.stream"})
+
+
+#: products of many rows that are handed on in 16 bits, where the library takes them (the products of tiles hand on
+#: float32 sums like those of few rows): activations that the next kernel reads once and rounds anyway
+TILE_ROLES = LIBRARY_F32_ROLES | {"ffn.down"}
+
+
+def takes_tiles(rt, n: int, n_out: int, k: int, ldx: int, ldw: int) -> bool:
+    """Whether a 16-bit product of ``n`` rows goes to the kernel of tiles of up to 256 x 256 (`gemm_tile.hip`): all of more
+    rows than the weight-streaming kernel takes whose sizes it supports. Against the BLAS library's products (weights from
+    memory, in us): the 7B shape's way down 171 against 253 at 1,500 rows, 227 against 353 at 2,048;
+    q/k/v 27 against 39 at 566, 52 against 58 at 1,500, 75 against 68 at 2,048; gate/up with the SiLU-gate 464 against
+    508 + 37 at 2,048, 157 against 137 + 11 at 566; the 1.5B shape's way down 25 against 46 at 566, 58 against 83 at 2,109,
+    gate/up 118 against 114 + 17 at 2,109. The few sizes at which one product is slower have others that gain more."""
+    from pyre_amd.hip import ops
+
+    return bool(rt.options.get("tile_gemm", True)) and n > SKINNY_MAX_ROWS and ops.gemm_tile_supports(n, n_out, k, ldx, ldw)
 
 
 def _is_bf16(ctx, lin, x) -> bool:
@@ -181,6 +198,11 @@ def linear(lin, ctx, x, n, out):
         else:
             ops.gemm_mid_bf16(x, lin.weight, buf, n, ks, wide=wide)
         return Partials(buf, lin.bias)
+    if lin.role in TILE_ROLES and takes_tiles(rt, n, n_out, k, x.stride(0), lin.weight.stride(0)):
+        parts = ops.gemm_tile_parts(n, n_out, k)
+        buf = ctx.workspace.get(f"linear.{lin.role}.partials", (parts, n, n_out), torch.float32)
+        ops.gemm_tile_bf16(x, lin.weight, buf, n, parts)
+        return Partials(buf, lin.bias)
     if not library:
         return None
     if lin.role in rt.options.get("library_f32_roles", LIBRARY_F32_ROLES):
@@ -195,8 +217,8 @@ def linear(lin, ctx, x, n, out):
 def gate_up_silu(lin, ctx, x, n, act, unit=None) -> bool:
     """silu(x gate^T) * (x up^T) in one kernel (``unit`` = (limit, slope, shift): the gated unit
     g sigmoid(slope g) (u + shift) with clipped inputs instead, in the same epilogues): the kernel that keeps all rows in a block for up to
-    256 rows where one round of blocks holds the features, else the weight-streaming kernel for a
-    decode step's few rows."""
+    256 rows where one round of blocks holds the features, else the kernel of tiles for many rows and the weight-streaming
+    kernel for a decode step's few."""
     from pyre_amd.hip import ops
 
     if not _is_bf16(ctx, lin, x) or lin.bias is not None:
@@ -215,6 +237,9 @@ def gate_up_silu(lin, ctx, x, n, act, unit=None) -> bool:
         if fits and (ops.gemm_mid_silu_blocks(n, lin.out_features) <= ctx.runtime.compute_units or int(mid) == 2):
             ops.gemm_mid_silu_bf16(x, lin.weight, act, n, unit)
             return True
+    if takes_tiles(ctx.runtime, n, lin.out_features, lin.in_features, x.stride(0), lin.weight.stride(0)):
+        ops.gemm_tile_glu_bf16(x, lin.weight, act, n, unit)
+        return True
     if n > FUSED_SILU_MAX_ROWS or not ctx.runtime.options.get("skinny_gemm", True):
         return False
     if not ops.gemm_skinny_supports(n, lin.out_features, lin.in_features, x.stride(0), lin.weight.stride(0)):

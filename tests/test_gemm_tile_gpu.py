@@ -1,0 +1,124 @@
+"""The product of many rows in tiles (`gemm_tile.hip`) against the product of the same 16-bit values in float64: at the edges
+of its tiles, with every number of parts of k, with rows apart from each other, and in an engine's step against the library's
+products."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def rnd(*shape, seed=0, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale).to(torch.bfloat16).to(DEV)
+
+
+#: float32 sums of k products of values around one: a rounding of 2^-24 of the running sum for every addition, the sums
+#: growing as the root of k, k roundings at random: 2^-24 sqrt(k) of the result's size; eight times that for the largest
+def bound(k: int) -> float:
+    return 8.0 * 2.0 ** -24 * k ** 0.5
+
+
+@pytest.mark.parametrize("n,k", [(16, 64), (144, 128), (272, 448), (1536, 192), (2064, 1536)])
+@pytest.mark.parametrize("m", [1, 65, 128, 129, 255, 257, 600])
+def test_sums(m, n, k):
+    from pyre_amd.hip import ops
+
+    assert ops.gemm_tile_supports(m, n, k, k, k)
+    x, w = rnd(m, k, seed=m), rnd(n, k, seed=n)
+    want = x.double() @ w.double().T
+    for parts in sorted({1, ops.gemm_tile_parts(m, n, k), *([2, 6] if k == 1536 else [])}):
+        out = torch.full((parts, m, n), float("nan"), device=DEV)
+        ops.gemm_tile_bf16(x, w, out, m, parts)
+        assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * float(want.std()) * 4, parts
+
+
+@pytest.mark.parametrize("m,n,k,bm,bn", [(3000, 3584, 1536, 256, 256), (2048, 5560 // 16 * 16, 512, 256, 192), (500, 2064, 1024, 128, 192),
+                                         (260, 4608, 640, 128, 128), (70, 4624, 1024, 64, 128)])
+def test_every_tile_size(m, n, k, bm, bn):
+    """Sizes that fill one round of each tile size, one row and sixteen columns past it."""
+    from pyre_amd.hip import ops
+
+    for mm in (m, m // bm * bm + 1):
+        x, w = rnd(mm, k + 24, seed=1)[:, 8:k + 8], rnd(n, k + 8, seed=2)[:, :k]   # rows 48 and 16 bytes apart
+        parts = ops.gemm_tile_parts(mm, n, k)
+        out = torch.full((parts, mm, n), float("nan"), device=DEV)
+        ops.gemm_tile_bf16(x, w, out, mm, parts)
+        want = x.double() @ w.double().T
+        assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * float(want.std()) * 4
+
+
+@pytest.mark.parametrize("unit", [None, (7.0, 1.702, 1.0), (0.0, float("inf"), 0.0, 0.0)])
+@pytest.mark.parametrize("m,inter,k", [(1, 8, 64), (70, 8960, 128), (130, 18944, 64), (200, 18936, 64), (257, 136, 256), (300, 8960, 64),
+                                       (520, 18944, 64), (1100, 1000, 128), (2049, 8968, 64)])
+def test_gated_units(m, inter, k, unit):
+    from pyre_amd.hip import ops
+
+    x, w = rnd(m, k, seed=3), rnd(2 * inter, k, seed=4, scale=0.2)
+    out = torch.full((m, inter), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.gemm_tile_glu_bf16(x, w, out, m, unit)
+    gate, up = (x.double() @ w.double().T).split(inter, 1)
+    if unit is None:
+        want = torch.nn.functional.silu(gate) * up
+    elif unit[1] == float("inf"):
+        want = gate.clamp(min=0) * up
+    else:
+        gate, up = gate.clamp(max=unit[0]), up.clamp(-unit[0], unit[0])
+        want = gate * torch.sigmoid(unit[1] * gate) * (up + unit[2])
+    # half a unit of the 8 bits that bfloat16 keeps, and the sums' rounding through factors of up to 16
+    assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 64 * bound(k)).all())
+
+
+def test_not_numbers_and_infinities_stay_in_their_rows():
+    from pyre_amd.hip import ops
+
+    x, w = rnd(300, 128, seed=5), rnd(512, 128, seed=6)
+    x[7, 3], x[299, 127] = float("nan"), float("inf")
+    out = torch.zeros(1, 300, 512, device=DEV)
+    ops.gemm_tile_bf16(x, w, out, 300, 1)
+    clean = torch.ones(300, dtype=torch.bool, device=DEV)
+    clean[7] = clean[299] = False
+    assert bool(torch.isnan(out[0, 7]).all()) and not bool(torch.isfinite(out[0, 299]).any())
+    assert bool(torch.isfinite(out[0, clean]).all())
+
+
+def test_what_it_refuses():
+    from pyre_amd.hip import ops
+    from pyre_amd.hip.lib import KernelError
+
+    assert not ops.gemm_tile_supports(100, 24, 64, 64, 64) and not ops.gemm_tile_supports(100, 32, 96, 96, 96)
+    assert not ops.gemm_tile_supports(100, 32, 64, 60, 64) and not ops.gemm_tile_supports(1 << 20, 32, 4096, 4096, 4096)
+    x, w = rnd(100, 96), rnd(32, 96)
+    with pytest.raises(KernelError):
+        ops.gemm_tile_bf16(x, w, torch.empty(1, 100, 32, device=DEV), 100, 1)
+    x, w = rnd(100, 128), rnd(32, 128)
+    with pytest.raises(KernelError):
+        ops.gemm_tile_bf16(x, w, torch.empty(3, 100, 32, device=DEV), 100, 3)     # parts of less than 256 k
+    with pytest.raises(KernelError):
+        ops.gemm_tile_bf16(x[:, 1:65], w[:, :64], torch.empty(1, 100, 32, device=DEV), 100, 1)
+
+
+@pytest.mark.parametrize("n", [65, 300])
+def test_a_step_against_the_librarys_products(n):
+    """The whole prompt of a small model through both: 16-bit activations, three layers."""
+    from pyre_amd.config import EngineConfig, preset
+    from pyre_amd.engine.batch import Entry
+    from pyre_amd.engine.engine import Engine
+    from pyre_amd.weights import model_tensor_specs, random_state
+
+    cfg = preset("tiny-a", hidden_size=128, head_dim=32, intermediate_size=320, num_hidden_layers=3)
+    state = random_state(model_tensor_specs(cfg), 3, 0.08, 0.1, torch.bfloat16, device=DEV)
+    eng = Engine.from_state(cfg, state, EngineConfig(max_cached_tokens=1024, max_num_batched_tokens=512, max_model_len=512))
+    ids = [(7 * i + 3) % 512 for i in range(n)]
+    rows = []
+    for tile in (True, False):
+        eng.runtime.options["tile_gemm"] = tile
+        eng.runtime.options["mid_gemm"] = False
+        rows.append(eng.step([Entry("a", ids, list(range(n)))]).clone())
+        eng.finish("a")
+    scale = rows[1].abs().amax(1)
+    assert float(((rows[0] - rows[1]).abs().amax(1) / scale).max()) <= 2e-2
