@@ -148,8 +148,165 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
   }
 }
 
-// The same product for a decode step's rows (M <= 64), as a stream over the weights. A block
-// is one wave with 32 output columns, so there is no barrier. It has a ring of R slots in LDS, a
+// 16 bytes per lane from `base + off` straight into LDS: lane x's piece lands at lds_addr + 16 x (see load_to_lds below).
+__device__ inline void load_rows(const void* base, unsigned off, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+template <int N>
+__device__ inline void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+constexpr int kSlotK = 32;  // k of a slot (two stages) of the rings below: rows of 128 bytes
+
+// The same product for more than 16 rows whose k comes in whole stages, bit for bit. A slot of the ring in LDS holds 32 k of the
+// block's BN rows of W and BM rows of A, filled by loads that go from memory straight into LDS; the 16-byte pieces of a row
+// are exchanged among themselves by the row's number. The operands of the next stage are read while the present one is
+// multiplied; the one barrier of a slot stands before its second stage: every wave has read the slot for the last time by
+// then, so the loads of S slots further on go into it, and the next slot, which everybody has waited for, is read from.
+//
+// What bounds it are the matrix cores (64 cycles for 4,096 multiply-adds): a block's loads are a tenth of what a compute unit
+// can take. So the tiles are small enough that all compute units have equally many, several blocks to a unit, whose waves
+// hide each other's waits. Against one buffer in LDS behind two barriers a stage and tiles of 128 x 128 (the 1.5B shape's
+// weights, us): q/k/v 55 -> 40 and the way down 169 -> 130 at 566 rows, gate/up 321 -> 241; 149 -> 81 at 72; 952 -> 834
+// at 2,048 (135 of 157 TFLOP/s). Against waves that stream the weights with a barrier a slot, at 40 rows: q/k/v 24 -> 14, way
+// down 46 -> 28, gate/up 64 -> 59; at 20 rows 15.0 -> 14.3, 29.6 -> 27.9, 41.5 -> 39.2 (the 7B shape's q/k/v 20.8 -> 17.0).
+template <int BM, int BN, int WM, int WN, int S, int OCC>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
+    const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const void* __restrict__ bias,
+    int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int mt, int nt) {
+  constexpr int NW = WM * WN, SLOT = (BM + BN) * 128, LX = BM / 8 / NW, LW = BN / 8 / NW, L = LX + LW;
+  constexpr int CT = BM / WM / 32, RT = BN / WN / 32, RD = 2 * (RT + CT), MF = 8 * RT * CT;
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "rows divide over the waves");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[S * SLOT];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 31, half = lane >> 5, wm = wave % WM, wn = wave / WM;
+  // Blocks are dealt to the eight dies in turn: a die's blocks are neighbours, eight tiles along m by some along n.
+  const int die = blockIdx.x & 7, share = gridDim.x >> 3, rest = gridDim.x & 7;
+  int t = die * share + min(die, rest) + (blockIdx.x >> 3);
+  const int per = mt * nt, ks = t / per;
+  t -= ks * per;
+  const int group = t / (8 * nt), first = 8 * group, gm = min(8, mt - first);
+  t -= 8 * nt * group;
+  const int m0 = (first + t % gm) * BM, n0 = (t / gm) * BN;
+  const int kbeg = ks * kper, kend = min(K, kbeg + kper), slots = (kend - kbeg + kSlotK - 1) / kSlotK;
+  out += ks * part_stride;
+  if (ks) bias = nullptr;  // the bias belongs to one part only
+  const unsigned base = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
+  const int lrow = lane >> 3, lpiece = lane & 7;
+  unsigned offx[LX], offw[LW];
+  int piece[L];
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {
+    const int row = 8 * (NW * i + wave) + lrow;  // rows past the end are the last one once more, and are not stored
+    piece[i] = lpiece ^ ((row >> 1) & 7);
+    offx[i] = static_cast<unsigned>(min(m0 + row, M - 1)) * static_cast<unsigned>(4 * lda);
+  }
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    const int row = 8 * (NW * i + wave) + lrow;
+    piece[LX + i] = lpiece ^ ((row >> 1) & 7);
+    offw[i] = static_cast<unsigned>(min(n0 + row, N - 1)) * static_cast<unsigned>(4 * ldw);
+  }
+  const char* xb = reinterpret_cast<const char*>(A + kbeg);
+  const char* wb = reinterpret_cast<const char*>(W + kbeg);
+  auto issue = [&](int i, int st, unsigned slot_base) {
+    // the last slot may hold 16 k only: the pieces behind them are the row's first once more, and are not multiplied
+    const int pc = 4 * piece[i] < kend - kbeg - kSlotK * st ? piece[i] : 0;
+    if (i < LX) load_rows(xb, offx[i < LX ? i : 0] + 16 * pc, slot_base + (NW * i + wave) * 1024);
+    else load_rows(wb, offw[i < LX ? 0 : i - LX] + 16 * pc, slot_base + BM * 128 + (NW * (i - LX) + wave) * 1024);
+  };
+  const unsigned char* const xrow = lds + (wm * 32 * CT + c) * 128;
+  const unsigned char* const wrow = lds + BM * 128 + (wn * 32 * RT + c) * 128;
+  const int swz = (c >> 1) & 7;
+  f32x4 a[2][RT][2], b[2][CT][2];
+  auto read = [&](int x, int run, int buf, int slot) {
+    const int h = x & 1, y = x >> 1, at = slot * SLOT + 16 * ((4 * run + half + 2 * h) ^ swz);
+    if (y < RT) a[buf][y < RT ? y : 0][h] = *reinterpret_cast<const f32x4*>(wrow + at + y * 32 * 128);
+    else b[buf][y < RT ? 0 : y - RT][h] = *reinterpret_cast<const f32x4*>(xrow + at + (y - RT) * 32 * 128);
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < slots) {
+#pragma unroll
+      for (int i = 0; i < L; ++i) issue(i, s, base + s * SLOT);
+      xb += 128;
+      wb += 128;
+    }
+  if (slots < S) wait_loads<0>();
+  else wait_loads<(S - 1) * L>();
+  asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+  for (int x = 0; x < RD; ++x) read(x, 0, 0, 0);
+  f32x16 acc[RT][CT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int q = 0; q < CT; ++q)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[r][q][i] = 0.f;
+  int slot = 0;
+  for (int st = 0; st < slots; ++st) {
+    const int next = slot + 1 == S ? 0 : slot + 1;
+#pragma unroll
+    for (int run = 0; run < 2; ++run) {
+      bool more = false;
+      if (run == 1) {
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        if (st + S > slots) wait_loads<0>();
+        else wait_loads<(S - 2) * L>();
+        asm volatile("s_barrier" ::: "memory");
+        more = st + S < slots;
+        if (kbeg + kSlotK * st + BK >= kend) break;  // a part that ends with half a slot
+      }
+#pragma unroll
+      for (int g = 0; g < MF; ++g) {
+        const int s = g / (RT * CT), r = g % (RT * CT) / CT, q = g % CT;
+#pragma unroll
+        for (int x = 0; x < RD; ++x)
+          if (x * MF / RD / 2 == g) read(x, run == 0 ? 1 : 0, run ^ 1, run == 0 ? slot : next);
+        acc[r][q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[run][r][s & 1][s >> 1], b[run][q][s & 1][s >> 1], acc[r][q], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (run == 1 && more) {
+#pragma unroll
+          for (int i = 0; i < L; ++i)
+            if (i * MF / L == g) issue(i, st + S, base + slot * SLOT);
+        }
+      }
+      if (run == 1 && more) {
+        xb += 128;
+        wb += 128;
+      }
+    }
+    slot = next;
+  }
+#pragma unroll
+  for (int q = 0; q < CT; ++q) {
+    const int m = m0 + 32 * (wm * CT + q) + c;
+    if (m >= M) continue;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int n = n0 + 32 * (wn * RT + r) + 8 * i + 4 * half;
+        if (n >= N) continue;
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = acc[r][q][4 * i + j];
+          if (bias && n + j < N) v[j] += load_as_float(bias, bias_dt, n + j);
+        }
+        float* dst = out + static_cast<size_t>(m) * ldo + n;
+        if (n + 3 < N && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+        } else {
+          for (int j = 0; j < 4 && n + j < N; ++j) dst[j] = v[j];
+        }
+      }
+  }
+}
+
+// The same product for a decode step's rows (M <= 16; up to 64 where k does not come in whole stages), as a stream over the
+// weights. A block is one wave with 32 output columns, so there is no barrier. It has a ring of R slots in LDS, a
 // slot being 32 k (two stages) of its 32 rows of W (4 KB) and of XR rows of A (XR = 8, 16, 32 or 64,
 // whichever holds M: 1 to 8 KB), filled by loads that go from memory straight into LDS: while
 // slot j is multiplied, slot j + 1 is read from LDS into registers and the R - 2 after it are on
@@ -163,18 +320,13 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
 // cores' float32 rate does; a small ring lets several blocks share a compute unit.
 constexpr int kStreamMaxRows = 64;
 constexpr int kMaxDevices = 64;
-constexpr int kSlotK = 32;
 
 __device__ inline void load_to_lds(const void* src, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_addr) : "memory", "m0");
 }
-template <int N>
-__device__ inline void wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
-}
 __device__ __attribute__((aligned(16))) const unsigned kZeroPiece[4] = {0u, 0u, 0u, 0u};
 
-// NW = 4 (steps of 17 to 64 rows): four such waves, one on each SIMD, share the step's rows: a slot
+// NW = 4 (17 to 64 rows): four such waves, one on each SIMD, share the step's rows: a slot
 // holds the four waves' weights and one copy of the rows, of which every wave loads a quarter, and
 // a barrier per slot tells a wave that the others' quarters are there. A wave alone reads the rows
 // from L2 once per 32 output columns, more bytes than its weights at 64 rows, and has LDS for one
@@ -413,7 +565,30 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
   // 16-byte loads along k need rows that start on 16 bytes
   const int vec_ok = lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(W) % 16 == 0;
-  if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows: the weights as a stream
+  if (M > 16 && vec_ok && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32)) {
+    // Tiles whose rows are few where the step's are; beyond 64 rows the size with the least work on the busiest unit (a block
+    // of several shares its matrix cores' time, so that is its tiles), smaller ones costing a little more for the same.
+    const auto tile = [&](auto kernel, int bm, int bn, int threads) {
+      const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * nt * ksplit), dim3(threads), 0, stream, A, lda, W, ldw, bias, bias_dt, out,
+                         static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, mt, nt);
+    };
+    constexpr struct { int bm, bn; double cost; } kTiles[4] = {{128, 128, 0.98}, {64, 128, 1.0}, {96, 128, 1.03}, {64, 64, 1.07}};
+    int best = 0;
+    double least = 1e300;
+    for (int i = 0; i < 4; ++i) {
+      const long tiles = static_cast<long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((N + kTiles[i].bn - 1) / kTiles[i].bn) * ksplit;
+      const double work = kTiles[i].cost * kTiles[i].bm * kTiles[i].bn * ((tiles + compute_units() - 1) / compute_units());
+      if (work < least) least = work, best = i;
+    }
+    PYRE_REQUIRE(static_cast<long>((M + 31) / 32) * ((N + 63) / 64) * ksplit < (1L << 30), "gemm_f32: M=%d N=%d too large for one launch", M, N);
+    if (M <= 32) tile(gemm_f32_tile_kernel<32, 128, 1, 4, 4, 1>, 32, 128, 256);
+    else if (M <= 64) tile(gemm_f32_tile_kernel<64, 64, 2, 2, 3, 1>, 64, 64, 256);
+    else if (best == 0) tile(gemm_f32_tile_kernel<128, 128, 2, 2, 2, 2>, 128, 128, 256);
+    else if (best == 1) tile(gemm_f32_tile_kernel<64, 128, 2, 2, 2, 3>, 64, 128, 256);
+    else if (best == 2) tile(gemm_f32_tile_kernel<96, 128, 1, 4, 2, 2>, 96, 128, 256);
+    else tile(gemm_f32_tile_kernel<64, 64, 2, 2, 2, 5>, 64, 64, 256);
+  } else if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows: the weights as a stream
     const dim3 grid((N + 31) / 32, 1, ksplit);
 #define PYRE_STREAM(R, XR)                                                                                         \
   hipLaunchKernelGGL((gemm_f32_stream_kernel<R, XR, 1>), grid, dim3(64), 0, stream, A, static_cast<size_t>(lda), W, \

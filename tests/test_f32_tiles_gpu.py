@@ -1,0 +1,70 @@
+"""The 32-bit path's products of more than 16 rows in tiles and its prompts' attention with pieces of 16 bytes: at the edges
+of their tiles, slots and pages."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def rnd(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV)
+
+
+@pytest.mark.parametrize("n,k,ks", [(48, 16, 1), (130, 1520, 2), (200, 80, 1), (1536, 1104, 3), (4608, 48, 1)])
+def test_products_at_every_row_count_have_the_bits_of_one_row(n, k, ks):
+    """Parts of k that end with half a slot among them (1520 / 2 = 760 -> 768 + 752; 1104 / 3 = 368)."""
+    from pyre_amd.hip import ops
+
+    m = 600
+    a, w = rnd(m, k, seed=1), rnd(n, k, seed=2)
+    one = torch.empty(ks, 16, n, device=DEV)
+    want = torch.empty(ks, m, n, device=DEV)
+    for r in range(0, m, 16):                                  # the kernel that streams the weights
+        rows = min(16, m - r)
+        part = one[:, :rows].contiguous() if rows < 16 else one
+        ops.gemm_f32(a[r:r + rows], w, None, part if ks > 1 else part[0], rows, ks)
+        want[:, r:r + rows] = part
+    exact = a.double() @ w.double().T
+    # k additions of products of values around one, each rounded to 2^-24 of a sum that grows as the root of k
+    assert float((want.double().sum(0) - exact).abs().max()) <= 8 * 2.0 ** -24 * k ** 0.5 * float(exact.std()) * 4
+    for rows in (17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 129, 200, 400, 600):
+        out = torch.full((ks, rows, n), float("nan"), device=DEV)
+        ops.gemm_f32(a[:rows], w, None, out if ks > 1 else out[0], rows, ks)
+        assert torch.equal(out, want[:, :rows]), rows
+
+
+@pytest.mark.parametrize("hd,page,window", [(128, 16, 0), (128, 32, 40), (64, 8, 0), (36, 4, 50), (96, 12, 33), (256, 16, 0), (20, 16, 7),
+                                            (30, 16, 0), (64, 6, 0)])
+def test_attention_of_prompts(hd, page, window):
+    """Against float64; what lies behind a step's last key in its page is not a number."""
+    from pyre_amd.hip import ops
+
+    nq, nkv, T = 6, 2, 77
+    pages = -(-T // page) + 2
+    k, v = rnd(T, nkv, hd, seed=1), rnd(T, nkv, hd, seed=2)
+    q = rnd(T, nq, hd, seed=3)
+    kc = torch.full((pages, nkv, page, hd), float("nan"), device=DEV)
+    vc = torch.full((pages, nkv, hd, page), float("nan"), device=DEV)
+    order = torch.randperm(pages, generator=torch.Generator().manual_seed(4)).tolist()
+    for t in range(T):
+        kc[order[t // page], :, t % page] = k[t]
+        vc[order[t // page], :, :, t % page] = v[t]
+    table = torch.tensor([order], dtype=torch.int32, device=DEV)
+    first = 5                                                  # the step brings tokens 5 .. 76
+    n = T - first
+    pos = torch.arange(first, T, dtype=torch.int32, device=DEV)
+    seq = torch.zeros(n, dtype=torch.int32, device=DEV)
+    tiles = torch.tensor([[t, min(32, n - t)] for t in range(0, n, 32)], dtype=torch.int32, device=DEV)
+    out = torch.full((n, nq, hd), float("nan"), device=DEV)
+    ops.attn_prefill_f32(q[first:].contiguous(), out, kc, vc, tiles, len(tiles), pos, seq, table, nq, nkv, hd, page, hd ** -0.5, window)
+    i, j = torch.arange(first, T, device=DEV)[:, None], torch.arange(T, device=DEV)[None]
+    hidden = (j > i) | ((i - j >= window) if window else torch.zeros_like(j > i))
+    for h in range(nq):
+        s = (q[first:, h].double() @ k[:, h // 3].double().T * hd ** -0.5).masked_fill(hidden, float("-inf"))
+        want = torch.softmax(s, 1) @ v[:, h // 3].double()
+        assert float((out[:, h].double() - want).abs().max()) <= 2e-5
