@@ -18,12 +18,15 @@
 #include "pyre_common.h"
 #include "pyre_vec4.h"
 
+#include <algorithm>
+
 using namespace pyre;
 
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxRank = 512;
+constexpr int kMaxSegments = 16;
 
 __device__ inline float silu_of(float z) { return z / (1.f + expf(-z)); }
 
@@ -151,6 +154,12 @@ __global__ __launch_bounds__(kThreads) void gla_scan_kernel(
 // instruction's operands) and the kernel that walks the chunks (gla_chunk_walk: a wave per request,
 // head and 16 columns of the state, nothing shared between waves) is left with three small matrix
 // products per chunk, whose operands it asks for one chunk ahead.
+// A walk is a chain of dependent instructions (2.2 us a chunk) and a prompt's heads are few waves: 112 of 1,024 SIMDs for 14 heads of
+// 128 columns. So the chunks of a prompt are dealt to segments that are walked at the same time: gla_chunk_ends first
+// walks all segments but the last, the first of them from the request's state and the others from zero, and leaves the states at their
+// ends and the products of their decays; in gla_chunk_walk a segment's wave makes the state before it from those of the
+// segments before it, S = diag(decays) S + end, in their order. Two walks of a ninth of the length: 251 -> 25 + 58 us a layer for a
+// prompt of 1,777 tokens on 14 heads of 128 x 128.
 // Chunks are counted from the first token that the request brings in this step. A chunk's operands
 // lie at "slots": token t of request s of the step has slot t + 16 s, so that the 16 slots of a
 // request's last, shorter chunk do not reach into the next request's.
@@ -163,9 +172,17 @@ struct ChunkScratch {
   float* vt;     // per chunk [head][dvp][16 tokens]:  v
   float* pairs;  // [slot][head][16]:                  row of A
   float* eb;     // per chunk [head][256]:             exp(B)
+  float* ends;   // per segment [head][tile of 16 columns][2][DT][lane][4]: the state at its end; its decays, or of a request's
+                 // first segment the state before it
 };
+// A segment is kSegment chunks at least, so token t0, with which one begins that is not a request's last, has a place of its
+// own at t0 / (16 kSegment).
+constexpr int kSegment = 4;
 __host__ __device__ inline size_t chunk_scratch_floats(size_t slots, int heads, int dkp, int dvp) {
-  return slots * heads * (2 * static_cast<size_t>(dkp) + dvp + 2 * kChunk);
+  return (slots * heads * (2 * static_cast<size_t>(dkp) + dvp + 2 * kChunk) + 3) / 4 * 4;
+}
+__host__ __device__ inline size_t ends_floats(size_t n_tokens, int heads, int dkp, int dv) {
+  return (n_tokens / (kChunk * kSegment) + 1) * heads * ((dv + 15) / 16) * 2 * (dkp / 16) * kWave * 4;
 }
 __host__ __device__ inline ChunkScratch carve(float* base, size_t slots, int heads, int dkp, int dvp) {
   ChunkScratch c;
@@ -174,6 +191,7 @@ __host__ __device__ inline ChunkScratch carve(float* base, size_t slots, int hea
   c.vt = c.kdt + slots * heads * dkp;
   c.pairs = c.vt + slots * heads * dvp;
   c.eb = c.pairs + slots * heads * kChunk;
+  c.ends = base + chunk_scratch_floats(slots, heads, dkp, dvp);
   return c;
 }
 
@@ -229,6 +247,115 @@ __global__ __launch_bounds__(kThreads) void gla_chunk_prep_kernel(
   for (int d = tid; d < dkp; d += kThreads) sc.eb[region * kChunk + d] = d < dk ? expf(bs[(nc - 1) * dk + d]) : 0.f;
 }
 
+// The same where heads are multiples of four elements, with fewer exponentials and no sums across waves. A[t][s] takes the
+// exponent b_t - b_s apart at the last token m of the lower half of the smallest aligned run of 2, 4, 8 or 16 tokens that
+// holds both: exp(b_t - b_m) goes with the query, exp(b_m - b_s) with the key, both exponents <= 0. So a level (a half of 8,
+// 4, 2 or 1 tokens) needs one exponential for each of the 16 tokens and a channel, 64 a channel in all instead of one for
+// each of 120 pairs, and its pairs are plain products of rows in LDS. Values cross LDS on their way to [column][token].
+// 79 -> 33 us for 1,777 tokens of 14 heads of 128 x 128, 32 -> 12 for 300 tokens of six (a chain of 64 sums over a wave).
+__global__ __launch_bounds__(kThreads) void gla_chunk_prep_vec_kernel(
+    const float* __restrict__ x, ChunkScratch sc, const int* __restrict__ q_start, int heads, int dk, int dv, int dkp,
+    int dvp) {
+  extern __shared__ __attribute__((aligned(16))) float prep_lds[];
+  const int ld = dk + 4;  // rows on distinct banks
+  float* qs = prep_lds;
+  float* ks = qs + kChunk * ld;
+  float* bs = ks + kChunk * ld;
+  float* f = bs + kChunk * ld;
+  const int s = blockIdx.z, hd = blockIdx.y, tid = threadIdx.x;
+  const int t0 = q_start[s] + blockIdx.x * kChunk, t_end = q_start[s + 1];
+  if (t0 >= t_end) return;
+  const int nc = min(kChunk, t_end - t0);
+  const size_t slot0 = static_cast<size_t>(t0) + kChunk * s;
+  const size_t region = slot0 * heads + static_cast<size_t>(hd) * kChunk;  // of this chunk and head, in slots
+  const int hk = heads * dk, hv = heads * dv, width = 3 * hk + 2 * hv, quads = dk / 4;
+  for (int i = tid; i < kChunk * quads; i += kThreads) {
+    const int t = i / quads, d = 4 * (i % quads);
+    const float* xr = x + static_cast<size_t>(t0 + min(t, nc - 1)) * width + hd * dk + d;
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};  // tokens that are not there: no query, no key, no decay
+    *reinterpret_cast<f32x4*>(qs + t * ld + d) = t < nc ? *reinterpret_cast<const f32x4*>(xr) : none;
+    *reinterpret_cast<f32x4*>(ks + t * ld + d) = t < nc ? *reinterpret_cast<const f32x4*>(xr + hk) : none;
+    *reinterpret_cast<f32x4*>(bs + t * ld + d) = t < nc ? *reinterpret_cast<const f32x4*>(xr + 2 * hk) : none;
+  }
+  for (int c0 = 0; c0 < dvp; c0 += dk) {
+    const int cols = min(dk, dvp - c0), vq = cols / 4;
+    __syncthreads();
+    for (int i = tid; i < kChunk * vq; i += kThreads) {
+      const int t = i / vq, cc = 4 * (i % vq);
+      *reinterpret_cast<f32x4*>(f + t * ld + cc) =
+          t < nc ? *reinterpret_cast<const f32x4*>(x + static_cast<size_t>(t0 + t) * width + 3 * hk + hd * dv + c0 + cc) : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+    for (int i = tid; i < cols * 4; i += kThreads) {
+      const int cc = i >> 2, t = 4 * (i & 3);
+      *reinterpret_cast<f32x4*>(sc.vt + region * dvp + static_cast<size_t>(c0) * kChunk + 4 * i) =
+          f32x4{f[t * ld + cc], f[(t + 1) * ld + cc], f[(t + 2) * ld + cc], f[(t + 3) * ld + cc]};
+    }
+  }
+  for (int d = tid; d < dk; d += kThreads) {  // behind the first barrier above
+    float b = bs[d];
+    for (int t = 1; t < kChunk; ++t) bs[t * ld + d] = b += bs[t * ld + d];
+  }
+  __syncthreads();
+  // Pairs of one level: 64, 32, 16, 8 of them, each by as many neighbouring lanes as there are for it; then the 16 of a
+  // token with itself, whose exponent is zero.
+  auto pair_of = [&](const float* q, const float* k, int t, int u, int lanes) {
+    const int part = tid % lanes;
+    float sum = 0.f;
+    for (int d = 4 * part; d < dk; d += 4 * lanes) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(q + t * ld + d), b = *reinterpret_cast<const f32x4*>(k + u * ld + d);
+      sum = fmaf(a[0], b[0], fmaf(a[1], b[1], fmaf(a[2], b[2], fmaf(a[3], b[3], sum))));
+    }
+    for (int o = lanes / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
+    if (part == 0) sc.pairs[((slot0 + t) * heads + hd) * kChunk + u] = t < nc ? sum : 0.f;
+  };
+#pragma unroll
+  for (int level = 3; level >= 0; --level) {
+    const int half = 1 << level;
+    if (level < 3) __syncthreads();
+    for (int i = tid; i < kChunk * quads; i += kThreads) {
+      const int t = i / quads, d = 4 * (i % quads);
+      const bool upper = t & half;
+      const int m = (t & ~(2 * half - 1)) + half - 1;
+      const f32x4 bt = *reinterpret_cast<const f32x4*>(bs + t * ld + d), bm = *reinterpret_cast<const f32x4*>(bs + m * ld + d);
+      f32x4 y = *reinterpret_cast<const f32x4*>((upper ? qs : ks) + t * ld + d);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] *= expf(upper ? bt[j] - bm[j] : bm[j] - bt[j]);
+      *reinterpret_cast<f32x4*>(f + t * ld + d) = y;
+    }
+    __syncthreads();
+    const int lanes = kThreads / (8 * half), p = tid / lanes;  // 8 half pairs: 8 / half runs of half x half
+    const int run = p / (half * half), in = p % (half * half);
+    pair_of(f, f, run * 2 * half + half + in / half, run * 2 * half + in % half, lanes);
+  }
+  pair_of(qs, ks, tid >> 4, tid >> 4, 16);
+  for (int i = tid; i < kChunk * kChunk; i += kThreads) {
+    const int t = i / kChunk, u = i % kChunk;
+    if (u > t) sc.pairs[((slot0 + t) * heads + hd) * kChunk + u] = 0.f;
+  }
+  for (int i = tid; i < kChunk * (dkp / 4); i += kThreads) {
+    const int t = i / (dkp / 4), d = 4 * (i % (dkp / 4));
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};
+    if (d < dk) {
+      y = *reinterpret_cast<const f32x4*>(qs + t * ld + d);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] *= expf(bs[t * ld + d + j]);
+    }
+    *reinterpret_cast<f32x4*>(sc.qd + ((slot0 + t) * heads + hd) * dkp + d) = y;
+  }
+  const float* const total = bs + (kChunk - 1) * ld;  // tokens that are not there do not decay
+  for (int i = tid; i < 4 * dkp; i += kThreads) {
+    const int d = i >> 2, t = 4 * (i & 3);
+    f32x4 y = {0.f, 0.f, 0.f, 0.f};
+    if (d < dk) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = ks[(t + j) * ld + d] * expf(total[d] - bs[(t + j) * ld + d]);
+    }
+    *reinterpret_cast<f32x4*>(sc.kdt + region * dkp + 4 * i) = y;
+  }
+  for (int d = tid; d < dkp; d += kThreads) sc.eb[region * kChunk + d] = d < dk ? expf(total[d]) : 0.f;
+}
+
 // DT: tiles of 16 rows of the state (dk <= 16 DT; the rows beyond dk are zeros and stay so). The wave
 // keeps its 16 columns' rows in the layout of the instruction's result: lane (g = lane / 16,
 // c = lane % 16) holds rows 16 j + 4 g + i (i < 4) of column c in S[j][i]. The sums over the rows take
@@ -239,71 +366,194 @@ struct ChunkOperands {
   f32x4 q[DT], k[DT], e[DT], v, a;
 };
 
-template <int DT>
-__global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
-    ChunkScratch sc, float* __restrict__ state, float* __restrict__ o, const int* __restrict__ q_start,
-    const int* __restrict__ state_slots, int heads, int dk, int dv, int dvp, float qscale) {
+// Chunk t0 of request s: for the states alone (OUT false) its keys, values and decays.
+template <int DT, bool OUT>
+__device__ inline void fetch_chunk(const ChunkScratch& sc, int t0, int s, int hd, int heads, int col, int dv, int dvp, int g, int c,
+                                   ChunkOperands<DT>& r) {
   constexpr int dkp = 16 * DT;
-  // the blocks of one request lie together in the grid and not those of one head: neighbours go to different dies, and a
-  // long prompt beside many single tokens is then not one die's alone. Heads are padded to a multiple of eight, so that the
-  // blocks of a head, which read the same operands, share a die and its cache
-  const int s = blockIdx.z, hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  if (hd >= heads) return;
-  const int col = blockIdx.y * 16 + c;
-  const bool has_col = col < dv;
-  const int t_begin = q_start[s], t_end = q_start[s + 1], hv = heads * dv;
-  float* st = state + (static_cast<size_t>(state_slots[s]) * heads + hd) * dk * dv;
-  f32x4 S[DT];
+  const size_t slot0 = static_cast<size_t>(t0) + kChunk * s;
+  const size_t region = slot0 * heads + static_cast<size_t>(hd) * kChunk;
+  const float* qp = sc.qd + ((slot0 + c) * heads + hd) * dkp + 4 * g;
+  const float* kp = sc.kdt + region * dkp + c * kChunk + 4 * g;
+  const float* ep = sc.eb + region * kChunk + 4 * g;
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    if (OUT) r.q[j] = *reinterpret_cast<const f32x4*>(qp + 16 * j);
+    r.k[j] = *reinterpret_cast<const f32x4*>(kp + 16 * j * kChunk);
+    r.e[j] = *reinterpret_cast<const f32x4*>(ep + 16 * j);
+  }
+  r.v = *reinterpret_cast<const f32x4*>(sc.vt + region * dvp + static_cast<size_t>(min(col, dvp - 1)) * kChunk + 4 * g);
+  if (col >= dv) r.v = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (OUT) r.a = *reinterpret_cast<const f32x4*>(sc.pairs + ((slot0 + c) * heads + hd) * kChunk + 4 * g);
+}
+
+// `step` on every chunk from `first` to `last`, its operands asked for two chunks ahead: three sets of registers that take turns
+// (a set copied into another would be waited for at the copy; heads beyond 128 have no registers for that many).
+template <int DT, bool OUT>
+struct ChunkSets {
+  static constexpr int N = DT > 8 ? (OUT ? 1 : 2) : 3;
+  ChunkOperands<DT> r[N];
+  template <typename Fetch>
+  __device__ void begin(int first, int last, Fetch fetch) {
+#pragma unroll
+    for (int b = 0; b < N; ++b)
+      if (first + b * kChunk < last) fetch(first + b * kChunk, r[b]);
+  }
+  template <typename Fetch, typename Step>
+  __device__ void walk(int first, int last, Fetch fetch, Step step) {
+    for (int t0 = first; t0 < last; t0 += N * kChunk) {
+#pragma unroll
+      for (int b = 0; b < N; ++b) {
+        const int t = t0 + b * kChunk;
+        if (t >= last) return;
+        step(t, r[b]);
+        if (t + N * kChunk < last) fetch(t + N * kChunk, r[b]);
+      }
+    }
+  }
+};
+
+// The state's rows and columns of a lane.
+template <int DT>
+__device__ inline void load_state(const float* st, int dk, int dv, int col, int g, f32x4 (&S)[DT]) {
 #pragma unroll
   for (int j = 0; j < DT; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 16 * j + 4 * g + i;
-      S[j][i] = has_col && row < dk ? st[static_cast<size_t>(row) * dv + col] : 0.f;
+      S[j][i] = col < dv && row < dk ? st[static_cast<size_t>(row) * dv + col] : 0.f;
     }
-  auto fetch = [&](int t0, ChunkOperands<DT>& r) {
-    const size_t slot0 = static_cast<size_t>(t0) + kChunk * s;
-    const size_t region = slot0 * heads + static_cast<size_t>(hd) * kChunk;
-    const float* qp = sc.qd + ((slot0 + c) * heads + hd) * dkp + 4 * g;
-    const float* kp = sc.kdt + region * dkp + c * kChunk + 4 * g;
-    const float* ep = sc.eb + region * kChunk + 4 * g;
+}
+
+// Where the wave of head hd and columns 16 tile .. finds or leaves what belongs to the segment that begins with token t0.
+template <int DT>
+__device__ inline f32x4* segment_end(const ChunkScratch& sc, int t0, int hd, int heads, int tile, int tiles, int lane) {
+  return reinterpret_cast<f32x4*>(sc.ends) +
+         ((static_cast<size_t>(t0 / (kChunk * kSegment)) * heads + hd) * tiles + tile) * 2 * DT * kWave + lane;
+}
+
+// grid: (heads, tiles of columns, requests x segments) in both kernels; `per`: chunks of a segment, `segments` of the longest
+// request. The blocks of one request lie together in the grid and not those of one head: neighbours go to different dies, and a
+// long prompt beside many single tokens is then not one die's alone. Heads are padded to a multiple of eight, so that the
+// blocks of a head, which read the same operands, share a die and its cache.
+template <int DT>
+__global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, const float* __restrict__ state,
+                                                               const int* __restrict__ q_start,
+                                                               const int* __restrict__ state_slots, int heads, int dk, int dv,
+                                                               int dvp, int per, int segments) {
+  const int s = blockIdx.z / segments, seg = blockIdx.z % segments, hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  if (hd >= heads) return;
+  const int t_begin = q_start[s], t_end = q_start[s + 1];
+  const int first = t_begin + seg * per * kChunk, last = first + per * kChunk;
+  if (last >= t_end) return;  // the request's last segment, or none of its
+  const int col = blockIdx.y * 16 + c;
+  f32x4 S[DT], D[DT];
+  if (seg == 0) {
+    load_state<DT>(state + (static_cast<size_t>(state_slots[s]) * heads + hd) * dk * dv, dk, dv, col, g, S);
+#pragma unroll
+    for (int j = 0; j < DT; ++j) D[j] = S[j];
+  } else {
 #pragma unroll
     for (int j = 0; j < DT; ++j) {
-      r.q[j] = *reinterpret_cast<const f32x4*>(qp + 16 * j);
-      r.k[j] = *reinterpret_cast<const f32x4*>(kp + 16 * j * kChunk);
-      r.e[j] = *reinterpret_cast<const f32x4*>(ep + 16 * j);
+      S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      D[j] = f32x4{1.f, 1.f, 1.f, 1.f};
     }
-    r.v = *reinterpret_cast<const f32x4*>(sc.vt + region * dvp + static_cast<size_t>(min(col, dvp - 1)) * kChunk + 4 * g);
-    if (!has_col) r.v = f32x4{0.f, 0.f, 0.f, 0.f};
-    r.a = *reinterpret_cast<const f32x4*>(sc.pairs + ((slot0 + c) * heads + hd) * kChunk + 4 * g);
-  };
-  ChunkOperands<DT> now, next;
-  if (t_begin < t_end) fetch(t_begin, now);
-  for (int t0 = t_begin; t0 < t_end; t0 += kChunk) {
-    const int nc = min(kChunk, t_end - t0);
-    const bool more = t0 + kChunk < t_end;
-    if (more) fetch(t0 + kChunk, next);
-    f32x4 out = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < DT; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[j][i], S[j][i], out, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a[i], now.v[i], out, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 4 * g + i;
-      if (t < nc && has_col) o[static_cast<size_t>(t0 + t) * hv + hd * dv + col] = out[i] * qscale;
-    }
-#pragma unroll
-    for (int j = 0; j < DT; ++j) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) S[j][i] *= now.e[j][i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
-    }
-    if (more) now = next;
   }
+  const auto fetch = [&](int t0, ChunkOperands<DT>& r) { fetch_chunk<DT, false>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
+  ChunkSets<DT, false> sets;
+  sets.begin(first, last, fetch);
+  sets.walk(first, last, fetch, [&](int, const ChunkOperands<DT>& now) {
+#pragma unroll
+        for (int j = 0; j < DT; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            S[j][i] *= now.e[j][i];
+            if (seg) D[j][i] *= now.e[j][i];
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < DT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
+      });
+  f32x4* end = segment_end<DT>(sc, first, hd, heads, blockIdx.y, gridDim.y, lane);
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+    end[j * kWave] = S[j];
+    end[(DT + j) * kWave] = D[j];
+  }
+}
+
+template <int DT>
+__global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
+    ChunkScratch sc, float* __restrict__ state, float* __restrict__ o, const int* __restrict__ q_start,
+    const int* __restrict__ state_slots, int heads, int dk, int dv, int dvp, float qscale, int per, int segments) {
+  const int s = blockIdx.z / segments, seg = blockIdx.z % segments, hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  if (hd >= heads) return;
+  const int col = blockIdx.y * 16 + c;
+  const bool has_col = col < dv;
+  const int t_begin = q_start[s], t_end = q_start[s + 1], hv = heads * dv;
+  const int first = t_begin + seg * per * kChunk;
+  const bool whole = seg + 1 < segments && first + per * kChunk < t_end;  // another segment comes after this one
+  const int last = whole ? first + per * kChunk : t_end;
+  if (first >= t_end) return;
+  const auto fetch = [&](int t0, ChunkOperands<DT>& r) { fetch_chunk<DT, true>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
+  ChunkSets<DT, true> sets;
+  sets.begin(first, last, fetch);
+  float* st = state + (static_cast<size_t>(state_slots[s]) * heads + hd) * dk * dv;
+  f32x4 S[DT];
+  if (seg == 0 && !whole) {  // a request of one segment: its state is this wave's alone
+    load_state<DT>(st, dk, dv, col, g, S);
+  } else {
+    const f32x4* end = segment_end<DT>(sc, t_begin, hd, heads, blockIdx.y, gridDim.y, lane);
+#pragma unroll
+    for (int j = 0; j < DT; ++j) S[j] = end[(seg == 0 ? DT + j : j) * kWave];
+    // a segment's end is asked for before the one before it is used
+    f32x4 e[2][DT], d[2][DT];
+    const auto ask = [&](int b, int set) {
+      if (b >= seg) return;
+      end = segment_end<DT>(sc, t_begin + b * per * kChunk, hd, heads, blockIdx.y, gridDim.y, lane);
+#pragma unroll
+      for (int j = 0; j < DT; ++j) e[set][j] = end[j * kWave], d[set][j] = end[(DT + j) * kWave];
+    };
+    const auto add = [&](int b, int set) {
+      if (b >= seg) return;
+#pragma unroll
+      for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[j][i] = fmaf(d[set][j][i], S[j][i], e[set][j][i]);
+    };
+    ask(1, 0);
+    for (int b = 1; b < seg; b += 2) {
+      ask(b + 1, 1);
+      add(b, 0);
+      ask(b + 2, 0);
+      add(b + 1, 1);
+    }
+  }
+  sets.walk(first, last, fetch, [&](int t0, const ChunkOperands<DT>& now) {
+        const int nc = min(kChunk, t_end - t0);
+        f32x4 out = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < DT; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[j][i], S[j][i], out, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a[i], now.v[i], out, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = 4 * g + i;
+          if (t < nc && has_col) o[static_cast<size_t>(t0 + t) * hv + hd * dv + col] = out[i] * qscale;
+        }
+#pragma unroll
+        for (int j = 0; j < DT; ++j) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[j][i] *= now.e[j][i];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
+        }
+      });
+  if (whole) return;
 #pragma unroll
   for (int j = 0; j < DT; ++j)
 #pragma unroll
@@ -512,7 +762,8 @@ static int chunk_tiles(int dk) { return dk <= 32 ? 2 : dk <= 64 ? 4 : dk <= 128 
 // Floats of scratch that pyre_gla_chunks needs for a step of n_tokens tokens of n_seqs requests.
 extern "C" long pyre_gla_chunks_scratch(int n_tokens, int n_seqs, int heads, int dk, int dv) {
   const size_t slots = static_cast<size_t>(n_tokens) + static_cast<size_t>(kChunk) * n_seqs;
-  return static_cast<long>(chunk_scratch_floats(slots, heads, 16 * chunk_tiles(dk), (dv + 3) / 4 * 4));
+  return static_cast<long>(chunk_scratch_floats(slots, heads, 16 * chunk_tiles(dk), (dv + 3) / 4 * 4) +
+                           ends_floats(n_tokens, heads, 16 * chunk_tiles(dk), dv));
 }
 
 extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, float* o, const int* q_start,
@@ -524,13 +775,31 @@ extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, flo
   if (n_seqs <= 0 || max_tokens == 0) return 0;
   const int DTs = chunk_tiles(dk), dkp = 16 * DTs, dvp = (dv + 3) / 4 * 4;
   const ChunkScratch sc = carve(scratch, static_cast<size_t>(n_tokens) + static_cast<size_t>(kChunk) * n_seqs, heads, dkp, dvp);
-  hipLaunchKernelGGL(gla_chunk_prep_kernel, dim3((max_tokens + kChunk - 1) / kChunk, heads, n_seqs), dim3(kThreads),
-                     sizeof(float) * 3 * kChunk * dk, stream, x, sc, q_start, heads, dk, dv, dkp, dvp);
+  const dim3 prep_grid((max_tokens + kChunk - 1) / kChunk, heads, n_seqs);
+  const size_t prep_bytes = sizeof(float) * 4 * kChunk * (dk + 4);
+  if (dk % 4 == 0 && dv % 4 == 0 && prep_bytes <= 65536 && reinterpret_cast<uintptr_t>(x) % 16 == 0)
+    hipLaunchKernelGGL(gla_chunk_prep_vec_kernel, prep_grid, dim3(kThreads), prep_bytes, stream, x, sc, q_start, heads, dk, dv, dkp, dvp);
+  else
+    hipLaunchKernelGGL(gla_chunk_prep_kernel, prep_grid, dim3(kThreads), sizeof(float) * 3 * kChunk * dk, stream, x, sc, q_start,
+                       heads, dk, dv, dkp, dvp);
   if (check_launch("gla_chunk_prep")) return 1;
-  const dim3 grid((heads + 7) / 8 * 8, (dv + 15) / 16, n_seqs);
-#define PYRE_WALK(DT)                                                                                                  \
-  hipLaunchKernelGGL(gla_chunk_walk_kernel<DT>, grid, dim3(kWave), 0, stream, sc, state, o, q_start, state_slots, heads, \
-                     dk, dv, dvp, qscale)
+  // As many segments as put a wave on every SIMD, counting the requests that may be as long as the longest; a segment costs
+  // its waves a walk for its end and the reading of those before it, so it has four chunks at least.
+  const int chunks = (max_tokens + kChunk - 1) / kChunk, tiles = (dv + 15) / 16;
+  const long waves = static_cast<long>((n_tokens + max_tokens - 1) / max_tokens) * heads * tiles;
+  int segments = static_cast<int>(std::max(1L, std::min(static_cast<long>(kMaxSegments), 4L * compute_units() / waves)));
+  int per = std::max(kSegment, (chunks + segments - 1) / segments);
+  segments = (chunks + per - 1) / per;
+  if (static_cast<long>(n_seqs) * segments > 65535) segments = 1, per = chunks;
+  const dim3 grid((heads + 7) / 8 * 8, tiles, n_seqs * segments);
+#define PYRE_WALK(DT)                                                                                                      \
+  do {                                                                                                                     \
+    if (segments > 1)                                                                                                      \
+      hipLaunchKernelGGL(gla_chunk_ends_kernel<DT>, grid, dim3(kWave), 0, stream, sc, state, q_start, state_slots, heads,   \
+                         dk, dv, dvp, per, segments);                                                                      \
+    hipLaunchKernelGGL(gla_chunk_walk_kernel<DT>, grid, dim3(kWave), 0, stream, sc, state, o, q_start, state_slots, heads, \
+                       dk, dv, dvp, qscale, per, segments);                                                                \
+  } while (0)
   switch (DTs) {
     case 2: PYRE_WALK(2); break;
     case 4: PYRE_WALK(4); break;

@@ -1,0 +1,46 @@
+"""The walk of gated linear attention in chunks, whose prompts are cut into segments that are walked at the same time: against
+the recurrence in float64, token by token."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("heads,dk,dv", [(3, 128, 128), (5, 40, 24), (1, 17, 250), (2, 200, 16), (1, 12, 100), (2, 256, 36)])
+@pytest.mark.parametrize("lengths", [[1, 700, 3], [64], [65], [80, 81, 79, 1, 1], [1300], [129, 5, 512]])
+def test_segments(heads, dk, dv, lengths):
+    from pyre_amd.hip import ops
+
+    n, hk, hv = sum(lengths), heads * dk, heads * dv
+    g = torch.Generator().manual_seed(n + dk)
+    x = torch.randn(n, 3 * hk + 2 * hv, generator=g)
+    # decays from one that forgets at once to one that keeps all
+    x[:, 2 * hk:3 * hk] = -torch.rand(n, hk, generator=g) ** 4 * torch.logspace(-4, 1.2, hk)[torch.randperm(hk, generator=g)]
+    slots = torch.randperm(len(lengths) + 2, generator=g)[:len(lengths)]
+    state = torch.randn(len(lengths) + 2, heads, dk, dv, generator=g)
+    starts = [0]
+    for m in lengths:
+        starts.append(starts[-1] + m)
+    out = torch.full((n, hv), float("nan"), device=DEV)
+    after = state.to(DEV)
+    scratch = torch.full((ops.gla_chunks_scratch(n, len(lengths), heads, dk, dv),), float("nan"), device=DEV)
+    ops.gla_scan(x.to(DEV), after, out, torch.tensor(starts, dtype=torch.int32, device=DEV),
+                 torch.tensor(slots.tolist(), dtype=torch.int32, device=DEV), len(lengths), heads, dk, dv, dk ** -0.5, scratch, max(lengths))
+    q, k, ld, v = (x[:, a:b].double().view(n, heads, -1) for a, b in ((0, hk), (hk, 2 * hk), (2 * hk, 3 * hk), (3 * hk, 3 * hk + hv)))
+    want, wanted_state = torch.empty(n, heads, dv, dtype=torch.float64), state.double().clone()
+    for s, m in enumerate(lengths):
+        S = wanted_state[slots[s]]
+        for t in range(starts[s], starts[s] + m):
+            S = torch.exp(ld[t])[:, :, None] * S + k[t][:, :, None] * v[t][:, None, :]
+            want[t] = torch.einsum("hdv,hd->hv", S, q[t]) * dk ** -0.5
+        wanted_state[slots[s]] = S
+    # sums of up to `reach` tokens of products of values around one, in float32; the exponents of a chunk are sums of sixteen logarithms
+    for got, ref in ((out.cpu().double().view(n, heads, dv), want), (after.cpu().double(), wanted_state)):
+        assert bool(torch.isfinite(got).all())
+        assert float((got - ref).abs().max() / ref.pow(2).mean().sqrt()) <= 1e-4
+        assert float((got - ref).norm() / ref.norm()) <= 4e-6
