@@ -323,9 +323,9 @@ __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_b
 // sums [n_partials][rows][(nq + 2 nkv) HD] float32 with its bias, the rotary tables, and where each
 // token's key and value go. Every block sums, biases and rotates the queries of its heads into LDS
 // (the arithmetic of rope_kv_write, so the same bits); of the waves that attend for a token and
-// key/value head, the one whose chunks hold the token's own position first writes its rotated key
-// and its value into the cache, zeroes the values behind it in the page as rope_kv_write does, waits
-// for the stores and then loads its chunks: no other wave reads that position. A step of single
+// key/value head, the one whose chunks hold the token's own position writes its rotated key
+// and its value into the cache, zeroes the values behind it in the page as rope_kv_write does, and takes them
+// for its own chunk from LDS: no other wave reads that position. A step of single
 // tokens then needs no kernel between the product and the attention.
 struct RopeIn {
   const float* qkv;
@@ -395,15 +395,12 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
     TableWindow tw{kv.table, min(table_stride, (last * kChunk + 16) / page_size + 1), 0, -1};
     if (begin < end) tw.fill(begin * kChunk / page_size);
     // FUSED: of the waves that attend for a token and key/value head (the first group of query heads
-    // only), the one whose chunks hold the token's own position writes its key and value; it loads
-    // that chunk only when its stores have arrived.
+    // only), the one whose chunks hold the token's own position writes its key and value; it does not read
+    // them back but puts them into that chunk's registers (see own_key).
     const bool may_write = FUSED && qt == 0 && rope.write_kv && begin <= last && last < end;
     bool writes = false;
-    auto arrived = [&](int c) {
-      if (FUSED && writes && c == last) asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-    };
-    const bool ask_a = begin < end && !(may_write && begin == last);
-    const bool ask_b = begin + 1 < end && !(may_write && begin + 1 == last);
+    const bool ask_a = begin < end, ask_b = begin + 1 < end;
+    __shared__ __attribute__((aligned(16))) bf16 own_s[2][FUSED ? HD : 8];
     if constexpr (FUSED) {
       constexpr int half = HD / 2;
       const int width = (nq + 2 * nkv) * HD;
@@ -453,16 +450,22 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
         Vec4<bf16>::store(&q_s[h][j], a4);
         Vec4<bf16>::store(&q_s[h][j + half], b4);
       }
+      // the token's own key and value, rounded likewise
+      float4 ka = zero4, kb = zero4;
+      if (key_lane) {
+        rotate(kp, ka, kb);
+        Vec4<bf16>::store(&own_s[0][4 * lane], ka);
+        Vec4<bf16>::store(&own_s[0][4 * lane + half], kb);
+      } else if (value_lane) {
+        Vec4<bf16>::store(&own_s[1][4 * (lane - HD / 8)], vv);
+      }
       lds_barrier();  // waits for LDS alone: the chunks' loads stay on their way
 #pragma unroll
       for (int c = 0; c < HD / 32; ++c) qr[0][c] = r < nheads ? load_b128(&q_s[r][32 * c + 8 * g]) : zero_b128();
-      // the token's own key and value
       writes = may_write && slot >= 0;
       if (writes) {
         const int page = slot / page_size, off = slot % page_size;
         if (key_lane) {
-          float4 ka, kb;
-          rotate(kp, ka, kb);
           bf16* dst = k_cache + ((static_cast<size_t>(page) * nkv + kvh) * page_size + off) * HD + 4 * lane;
           Vec4<bf16>::store(dst, ka);
           Vec4<bf16>::store(dst + half, kb);
@@ -483,26 +486,44 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
       if (ask_a) load_chunk<HD, STREAM_V>(kv, tw, begin * kChunk, ra);
       if (ask_b) load_chunk<HD, STREAM_V>(kv, tw, (begin + 1) * kChunk, rb);
     }
-    if (begin < end && !ask_a) {
-      arrived(begin);
-      load_chunk<HD, STREAM_V>(kv, tw, begin * kChunk, ra);
-    }
-    if (begin + 1 < end && !ask_b) {
-      arrived(begin + 1);
-      load_chunk<HD, STREAM_V>(kv, tw, (begin + 1) * kChunk, rb);
-    }
-    for (int c = begin; c < end; c += 2) {
-      attend_regs<HD, 1>(ra, c * kChunk, c == first || c == last, bd, scale_log2, qr, o, m, l);
-      if (c + 2 < end) {
-        arrived(c + 2);
-        load_chunk<HD, STREAM_V>(kv, tw, (c + 2) * kChunk, ra);
-      }
-      if (c + 1 < end) {
-        attend_regs<HD, 1>(rb, (c + 1) * kChunk, c + 1 == first || c + 1 == last, bd, scale_log2, qr, o, m, l);
-        if (c + 3 < end) {
-          arrived(c + 3);
-          load_chunk<HD, STREAM_V>(kv, tw, (c + 3) * kChunk, rb);
+    // The chunk that holds the token's own position was read from the cache as the step found it: its key and value go
+    // into the registers that stand for them, and the values behind it, which nobody has written, become zero. (Waiting
+    // for the stores and reading them back was two trips through memory on the way of the last wave.)
+    auto own_key = [&](int c, ChunkRegs<HD>& cr) {
+      if (!FUSED || !writes || c != last) return;
+      const int p = pos - c * kChunk;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        if (t == ((p >> 2) & 1) && r == 4 * (p >> 3) + (p & 3)) {
+#pragma unroll
+          for (int cc = 0; cc < HD / 32; ++cc) cr.k[t][cc] = load_b128(&own_s[0][32 * cc + 8 * g]);
         }
+      unsigned keep[4], own[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int key = 8 * g + 2 * j;  // and the one after it
+        keep[j] = (key < p ? 0xffffu : 0u) | (key + 1 < p ? 0xffff0000u : 0u);
+        own[j] = (key == p ? 0xffffu : 0u) | (key + 1 == p ? 0xffff0000u : 0u);
+      }
+#pragma unroll
+      for (int dt = 0; dt < HD / 16; ++dt) {
+        const unsigned v = own_s[1][16 * dt + r].bits * 0x10001u;
+        uint4 u = __builtin_bit_cast(uint4, cr.v[dt]);
+        u.x = (u.x & keep[0]) | (v & own[0]);
+        u.y = (u.y & keep[1]) | (v & own[1]);
+        u.z = (u.z & keep[2]) | (v & own[2]);
+        u.w = (u.w & keep[3]) | (v & own[3]);
+        cr.v[dt] = __builtin_bit_cast(bf16x8, u);
+      }
+    };
+    for (int c = begin; c < end; c += 2) {
+      own_key(c, ra);
+      attend_regs<HD, 1>(ra, c * kChunk, c == first || c == last, bd, scale_log2, qr, o, m, l);
+      if (c + 2 < end) load_chunk<HD, STREAM_V>(kv, tw, (c + 2) * kChunk, ra);
+      if (c + 1 < end) {
+        own_key(c + 1, rb);
+        attend_regs<HD, 1>(rb, (c + 1) * kChunk, c + 1 == first || c + 1 == last, bd, scale_log2, qr, o, m, l);
+        if (c + 3 < end) load_chunk<HD, STREAM_V>(kv, tw, (c + 3) * kChunk, rb);
       }
     }
   } else {
