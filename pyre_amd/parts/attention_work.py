@@ -21,6 +21,10 @@ DEFAULT_UNITS = 256
 #: keys per chunk of the decode kernel, and the fewest chunks a block is given if its request has them
 DECODE_CHUNK = 32
 DECODE_MIN_CHUNKS_PER_BLOCK = 8
+#: a request of up to this many chunks is one block's: three chunks a wave in a row take less than a second block whose
+#: result goes through memory (11.2 us against 13.4 for one request of ten chunks, 13.4 against 16.6 for 30; at 16 chunks
+#: the two are alike)
+DECODE_ONE_BLOCK_CHUNKS = 12
 #: the same when the blocks take several rounds anyway: every block has a start and an end worth
 #: several chunks' time, and nothing is idle that more blocks could fill (measured in the serving
 #: workload of 256 requests: 2.73 ms a captured step with 16, 2.77 with 8, 2.75 with 24, 2.80 with 32)
@@ -79,7 +83,8 @@ def decode_work(tokens: np.ndarray, positions: np.ndarray, rows: int, window: in
     padding = max(0, rows - n)
     total, longest = int(chunks.sum()) + padding, int(chunks.max())
     slots = _decode_slots(rows, nq, nkv, units)
-    if size is None:
+    planned = size is None
+    if planned:
         size = -(-total // (2 * slots))  # many rounds: half a slot's share
         least = DECODE_MIN_CHUNKS_MANY_ROUNDS
         if n + padding <= slots:
@@ -96,7 +101,7 @@ def decode_work(tokens: np.ndarray, positions: np.ndarray, rows: int, window: in
                 size, least = max(a, math.isqrt(longest // 2)), DECODE_MIN_CHUNKS_PER_BLOCK
         size = max(size, least)
     size = max(size, -(-longest // DECODE_MAX_BLOCKS_PER_REQUEST))
-    nb = -(-chunks // size)
+    nb = np.where(chunks <= (DECODE_ONE_BLOCK_CHUNKS if planned else 0), 1, -(-chunks // size))
     per = -(-chunks // (4 * nb))
     nb = -(-chunks // (4 * per))  # blocks that are left without a chunk by the rounding are dropped
     order = np.argsort(-chunks, kind="stable")
