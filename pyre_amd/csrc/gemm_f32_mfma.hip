@@ -170,7 +170,9 @@ constexpr int kSlotK = 32;  // k of a slot (two stages) of the rings below: rows
 // weights, us): q/k/v 55 -> 40 and the way down 169 -> 130 at 566 rows, gate/up 321 -> 241; 149 -> 81 at 72; 952 -> 834
 // at 2,048 (135 of 157 TFLOP/s). Against waves that stream the weights with a barrier a slot, at 40 rows: q/k/v 24 -> 14, way
 // down 46 -> 28, gate/up 64 -> 59; at 20 rows 15.0 -> 14.3, 29.6 -> 27.9, 41.5 -> 39.2 (the 7B shape's q/k/v 20.8 -> 17.0).
-template <int BM, int BN, int WM, int WN, int S, int OCC>
+// WHOLE: a block walks all parts of k and adds their sums up in their order, as the consumer of partial sums does (the same
+// bits), where the rows alone fill the chip: the parts of a prompt do not go through memory.
+template <int BM, int BN, int WM, int WN, int S, int OCC, bool WHOLE>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
     const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const void* __restrict__ bias,
     int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int mt, int nt) {
@@ -188,7 +190,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
   const int group = t / (8 * nt), first = 8 * group, gm = min(8, mt - first);
   t -= 8 * nt * group;
   const int m0 = (first + t % gm) * BM, n0 = (t / gm) * BN;
-  const int kbeg = ks * kper, kend = min(K, kbeg + kper), slots = (kend - kbeg + kSlotK - 1) / kSlotK;
+  const int kbeg = WHOLE ? 0 : ks * kper, kend = WHOLE ? K : min(K, kbeg + kper), slots = (kend - kbeg + kSlotK - 1) / kSlotK;
   out += ks * part_stride;
   if (ks) bias = nullptr;  // the bias belongs to one part only
   const unsigned base = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
@@ -244,6 +246,28 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
     for (int q = 0; q < CT; ++q)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[r][q][i] = 0.f;
+  f32x16 total[WHOLE ? RT : 1][WHOLE ? CT : 1];
+  int left = kper / BK;  // stages until the part ends
+  if (WHOLE) {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int q = 0; q < CT; ++q)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) total[WHOLE ? r : 0][WHOLE ? q : 0][i] = 0.f;
+  }
+  auto end_part = [&]() {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int q = 0; q < CT; ++q)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          total[WHOLE ? r : 0][WHOLE ? q : 0][i] += acc[r][q][i];
+          acc[r][q][i] = 0.f;
+        }
+    left = kper / BK;
+  };
   int slot = 0;
   for (int st = 0; st < slots; ++st) {
     const int next = slot + 1 == S ? 0 : slot + 1;
@@ -276,8 +300,16 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
         xb += 128;
         wb += 128;
       }
+      if (WHOLE && --left == 0) end_part();
     }
     slot = next;
+  }
+  if (WHOLE) {
+    end_part();  // a last, shorter part (or nothing)
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int q = 0; q < CT; ++q) acc[r][q] = total[WHOLE ? r : 0][WHOLE ? q : 0];
   }
 #pragma unroll
   for (int q = 0; q < CT; ++q) {
@@ -551,6 +583,81 @@ __global__ __launch_bounds__(64 * NW) void gemm_f32_stream_kernel(
 
 }  // namespace
 
+namespace {
+
+// Tiles whose rows are few where the step's are; beyond 64 rows the size with the least work on the busiest unit (a block of
+// several shares its matrix cores' time, so that is its tiles), smaller ones costing a little more for the same.
+struct TileRows {
+  int bm, bn;
+  double cost;
+};
+constexpr TileRows kTiles[4] = {{128, 128, 0.98}, {64, 128, 1.0}, {96, 128, 1.03}, {64, 64, 1.07}};
+constexpr double kMacsPerUs = 2.8e5;    // of a compute unit
+constexpr double kBytesPerUs = 5e6;     // of memory, both ways
+constexpr double kFillUs = 0.006;       // a k of a block's chain before the unit's other blocks hide it
+
+// The tile size for so many rows and `parts` parts of kper, and what it takes in microseconds.
+int best_tile(int M, int N, int kper, int parts, double* us) {
+  int best = 0;
+  double least = 1e300;
+  for (int i = 0; i < 4; ++i) {
+    const long tiles = static_cast<long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((N + kTiles[i].bn - 1) / kTiles[i].bn) * parts;
+    const double work = kTiles[i].cost * kTiles[i].bm * kTiles[i].bn * kper * ((tiles + compute_units() - 1) / compute_units());
+    if (work < least) least = work, best = i;
+  }
+  if (us) *us = least / kMacsPerUs + 8.0 * parts * M * static_cast<double>(N) / kBytesPerUs + kFillUs * kper;
+  return best;
+}
+
+bool takes_tiles(int M, int N, int K, long lda, long ldw) {
+  return M > 16 && lda % 4 == 0 && ldw % 4 == 0 && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32) &&
+         static_cast<long>((M + 31) / 32) * ((N + 63) / 64) < (1L << 24);
+}
+
+template <bool WHOLE>
+void launch_tiles(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
+                  int M, int N, int K, int kper, int ksplit, hipStream_t stream) {
+  const int parts = WHOLE ? 1 : ksplit;
+  const auto tile = [&](auto kernel, int bm, int bn) {
+    const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * nt * parts), dim3(256), 0, stream, A, lda, W, ldw, bias, bias_dt, out,
+                       static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, mt, nt);
+  };
+  const int best = best_tile(M, N, WHOLE ? K : kper, parts, nullptr);
+  if (M <= 32) tile(gemm_f32_tile_kernel<32, 128, 1, 4, 4, 1, WHOLE>, 32, 128);
+  else if (M <= 64) tile(gemm_f32_tile_kernel<64, 64, 2, 2, 3, 1, WHOLE>, 64, 64);
+  else if (best == 0) tile(gemm_f32_tile_kernel<128, 128, 2, 2, 2, 2, WHOLE>, 128, 128);
+  else if (best == 1) tile(gemm_f32_tile_kernel<64, 128, 2, 2, 2, 3, WHOLE>, 64, 128);
+  else if (best == 2) tile(gemm_f32_tile_kernel<96, 128, 1, 4, 2, 2, WHOLE>, 96, 128);
+  else tile(gemm_f32_tile_kernel<64, 64, 2, 2, 2, 5, WHOLE>, 64, 64);
+}
+
+int part_of(int K, int ksplit) { return ((K + ksplit - 1) / ksplit + BK - 1) / BK * BK; }
+
+}  // namespace
+
+// Whether the sums of all parts of k are better made by the blocks themselves: where that takes less than the same work in
+// parts with their way through memory, there and back (the 1.5B shape's q/k/v in 8 parts, us with the consumer's reading: 28 apart
+// and 38 whole at 300 rows, 45 and 61 at 566, 96 and 83 at 1,200, 148 and 111 at 2,000; the 7B shape's o in 9: 120 and 138 at
+// 400, 148 and 140 at 566, 926 and 799 at 4,000).
+extern "C" int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int ksplit) {
+  if (ksplit <= 1 || M <= 64 || !takes_tiles(M, N, K, lda, ldw)) return 0;
+  double apart, whole;
+  best_tile(M, N, part_of(K, ksplit), ksplit, &apart);
+  best_tile(M, N, K, 1, &whole);
+  return whole < apart;
+}
+
+extern "C" int pyre_gemm_f32_whole(const float* A, long lda, const float* W, long ldw, float* out, long ldo, int M, int N, int K,
+                                   int ksplit, hipStream_t stream) {
+  PYRE_REQUIRE(takes_tiles(M, N, K, lda, ldw) && lda >= K && ldw >= K && ldo >= N && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(W) % 16 == 0,
+               "gemm_f32_whole: M=%d (more than 16) N=%d K=%d (a multiple of 16) lda=%ld ldw=%ld (of 4) are not supported", M, N, K, lda, ldw);
+  PYRE_REQUIRE(ksplit >= 1 && ksplit <= 64 && static_cast<long>(ksplit - 1) * part_of(K, ksplit) < K, "gemm_f32_whole: ksplit=%d", ksplit);
+  launch_tiles<true>(A, lda, W, ldw, nullptr, 0, out, ldo, 0, M, N, K, part_of(K, ksplit), ksplit, stream);
+  return check_launch("gemm_f32_whole");
+}
+
 extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt,
                              float* out, long ldo, long part_stride, int M, int N, int K, int ksplit,
                              hipStream_t stream) {
@@ -560,34 +667,13 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
   PYRE_REQUIRE(ksplit >= 1 && ksplit <= 64 && (ksplit == 1 || part_stride >= static_cast<long>(M) * ldo),
                "gemm_f32: ksplit=%d, partial sums %ld apart", ksplit, part_stride);
   if (M == 0) return 0;
-  const int kper = ((K + ksplit - 1) / ksplit + BK - 1) / BK * BK;
+  const int kper = part_of(K, ksplit);
   PYRE_REQUIRE(static_cast<long>(ksplit - 1) * kper < K, "gemm_f32: a part of k would be empty (K=%d, ksplit=%d)", K, ksplit);
   // 16-byte loads along k need rows that start on 16 bytes
   const int vec_ok = lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(W) % 16 == 0;
-  if (M > 16 && vec_ok && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32)) {
-    // Tiles whose rows are few where the step's are; beyond 64 rows the size with the least work on the busiest unit (a block
-    // of several shares its matrix cores' time, so that is its tiles), smaller ones costing a little more for the same.
-    const auto tile = [&](auto kernel, int bm, int bn, int threads) {
-      const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
-      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * nt * ksplit), dim3(threads), 0, stream, A, lda, W, ldw, bias, bias_dt, out,
-                         static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, mt, nt);
-    };
-    constexpr struct { int bm, bn; double cost; } kTiles[4] = {{128, 128, 0.98}, {64, 128, 1.0}, {96, 128, 1.03}, {64, 64, 1.07}};
-    int best = 0;
-    double least = 1e300;
-    for (int i = 0; i < 4; ++i) {
-      const long tiles = static_cast<long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((N + kTiles[i].bn - 1) / kTiles[i].bn) * ksplit;
-      const double work = kTiles[i].cost * kTiles[i].bm * kTiles[i].bn * ((tiles + compute_units() - 1) / compute_units());
-      if (work < least) least = work, best = i;
-    }
-    PYRE_REQUIRE(static_cast<long>((M + 31) / 32) * ((N + 63) / 64) * ksplit < (1L << 30), "gemm_f32: M=%d N=%d too large for one launch", M, N);
-    if (M <= 32) tile(gemm_f32_tile_kernel<32, 128, 1, 4, 4, 1>, 32, 128, 256);
-    else if (M <= 64) tile(gemm_f32_tile_kernel<64, 64, 2, 2, 3, 1>, 64, 64, 256);
-    else if (best == 0) tile(gemm_f32_tile_kernel<128, 128, 2, 2, 2, 2>, 128, 128, 256);
-    else if (best == 1) tile(gemm_f32_tile_kernel<64, 128, 2, 2, 2, 3>, 64, 128, 256);
-    else if (best == 2) tile(gemm_f32_tile_kernel<96, 128, 1, 4, 2, 2>, 96, 128, 256);
-    else tile(gemm_f32_tile_kernel<64, 64, 2, 2, 2, 5>, 64, 64, 256);
+  if (vec_ok && takes_tiles(M, N, K, lda, ldw)) {
+    launch_tiles<false>(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, stream);
   } else if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows: the weights as a stream
     const dim3 grid((N + 31) / 32, 1, ksplit);
 #define PYRE_STREAM(R, XR)                                                                                         \

@@ -67,6 +67,13 @@ int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw, const void
                   float* out, long ldo, long part_stride, int M, int N, int K, int ksplit,
                   hipStream_t stream);
 
+// 1 if a product of so many rows in ksplit parts of k is better made by pyre_gemm_f32_whole: out [M][N] (rows ldo apart) =
+// the sum of the parts in their order, as a consumer of pyre_gemm_f32's partial sums forms it, bit for bit. More than 16
+// rows, K a multiple of 16, rows on 16 bytes.
+int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int ksplit);
+int pyre_gemm_f32_whole(const float* A, long lda, const float* W, long ldw, float* out, long ldo, int M, int N, int K, int ksplit,
+                        hipStream_t stream);
+
 // bfloat16 products with 1..64 rows (decode): 1 if the kernel takes the shape.
 int pyre_gemm_skinny_supports(int M, int N, int K, long ldx, long ldw);
 

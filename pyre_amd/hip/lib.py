@@ -54,6 +54,8 @@ _SIGNATURES = {
     "pyre_sample": [P, L, P, P, P, I, I, P],
     "pyre_feed_tokens": [P, P, P, I, P],
     "pyre_gemm_skinny_glu_bf16": [P, L, P, L, P, I, I, I, F, F, F, F, P],
+    "pyre_gemm_f32_adds": [I, I, I, L, L, I],
+    "pyre_gemm_f32_whole": [P, L, P, L, P, L, I, I, I, I, P],
     "pyre_gemm_tile_supports": [I, I, I, L, L],
     "pyre_gemm_tile_parts": [I, I, I],
     "pyre_gemm_tile_bf16": [P, L, P, L, P, I, I, I, I, P],

@@ -590,7 +590,12 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, ou
          out.data_ptr(), dtype_code(out), out.stride(0), m, n_out, k, _stream())
 
 
-F32_KSPLIT_MAX = 8
+#: the most parts of k of a float32 product, and the fewest k of a part: a wave of a decode step's product is a chain of
+#: matrix instructions along its part (20 rows on the 1.5B shape's weights, us: q/k/v in 3, 6, 8 parts 14.7, 9.3, 8.2, the way
+#: down in 8, 12, 14, 16 28.7, 22.2, 18.7, 18.4; one row 9.4, 6.5, 6.1 and 18.0, 14.6, 12.9, 13.3), while a prompt pays for more
+#: parts with their way through memory (566 rows, the way down: 139, 176, 131, 143)
+F32_KSPLIT_MAX = 14
+F32_KSPLIT_MIN_K = 192
 
 
 def compute_units(device=None) -> int:
@@ -606,11 +611,33 @@ def compute_units(device=None) -> int:
 
 def gemm_f32_ksplit(n_out: int, k: int, units: int = DEFAULT_UNITS) -> int:
     """Into how many parts of k the float32 product is split: enough blocks of 128 output
-    columns for the ``units`` compute units, parts of at least 512. A function of the weight's
+    columns for the ``units`` compute units, parts of at least 192. A function of the weight's
     shape (and the engine's device) alone, never of the rows, so that a row's result does not
     depend on its step."""
     blocks = -(-n_out // 128)
-    return max(1, min(F32_KSPLIT_MAX, units // blocks, k // 512))
+    return max(1, min(F32_KSPLIT_MAX, units // blocks, k // F32_KSPLIT_MIN_K))
+
+
+@lru_cache(maxsize=4096)
+def gemm_f32_adds(m: int, n_out: int, k: int, lda: int, ldw: int, ksplit: int) -> bool:
+    """Whether :func:`gemm_f32_whole` is the better form of such a product in ``ksplit`` parts."""
+    from pyre_amd.hip.lib import lib
+
+    return bool(lib().pyre_gemm_f32_adds(m, n_out, k, lda, ldw, ksplit))
+
+
+def gemm_f32_whole(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, ksplit: int) -> None:
+    """out[0:m] (float32 [>= m, N]) = the sum, in their order, of the ``ksplit`` parts that :func:`gemm_f32` would make."""
+    _dev(a, w, out)
+    n_out, k = w.shape
+    if a.dtype != torch.float32 or w.dtype != torch.float32 or out.dtype != torch.float32:
+        raise KernelError("gemm_f32: float32 operands and result expected")
+    if a.dim() != 2 or a.shape[1] != k or out.dim() != 2 or out.shape[1] != n_out or out.shape[0] < m or a.shape[0] < m:
+        raise KernelError(f"gemm_f32: a {tuple(a.shape)} @ w {tuple(w.shape)}.T -> out {tuple(out.shape)} do not fit {m} rows")
+    if a.stride(1) != 1 or w.stride(1) != 1 or out.stride(1) != 1:
+        raise KernelError("gemm_f32: rows must be contiguous")
+    call("pyre_gemm_f32_whole", a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), m, n_out, k,
+         ksplit, _stream())
 
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, m: int,

@@ -42,6 +42,12 @@ class Linear:
         if f32 and out is None:
             # the true 32-bit path: the matrix cores' float32 instruction, k split by the weight's shape alone
             ks = ops.gemm_f32_ksplit(self.out_features, self.in_features, ctx.runtime.compute_units)
+            lda, ldw = x.stride(0), self.weight.stride(0)
+            if x.data_ptr() % 16 == 0 and self.weight.data_ptr() % 16 == 0 and \
+                    ops.gemm_f32_adds(n, self.out_features, self.in_features, lda, ldw, ks):
+                buf = ctx.workspace.get(f"linear.{self.role}", (1, n, self.out_features), torch.float32)
+                ops.gemm_f32_whole(x, self.weight, buf[0], n, ks)
+                return Partials(buf, self.bias)
             buf = ctx.workspace.get(f"linear.{self.role}", (ks, n, self.out_features), torch.float32)
             ops.gemm_f32(x, self.weight, None, buf if ks > 1 else buf[0], n, ks)
             return Partials(buf, self.bias)

@@ -68,3 +68,21 @@ def test_attention_of_prompts(hd, page, window):
         s = (q[first:, h].double() @ k[:, h // 3].double().T * hd ** -0.5).masked_fill(hidden, float("-inf"))
         want = torch.softmax(s, 1) @ v[:, h // 3].double()
         assert float((out[:, h].double() - want).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("n,k,ks", [(130, 1520, 2), (1536, 1104, 3), (200, 8960, 16), (48, 80, 3), (300, 640, 40)])
+def test_parts_added_where_they_are_made(n, k, ks):
+    """The same bits as the parts added up in their order (parts that end with half a slot, a last part shorter than the
+    others)."""
+    from pyre_amd.hip import ops
+
+    for m in (17, 40, 65, 100, 200, 520):
+        a, w = rnd(m, k, seed=m), rnd(n, k, seed=n)
+        parts = torch.empty(ks, m, n, device=DEV)
+        ops.gemm_f32(a, w, None, parts, m, ks)
+        want = parts[0].clone()
+        for p in parts[1:]:
+            want += p
+        out = torch.full((m, n), float("nan"), device=DEV)
+        ops.gemm_f32_whole(a, w, out, m, ks)
+        assert torch.equal(out, want), m
