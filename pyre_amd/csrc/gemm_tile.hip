@@ -53,6 +53,8 @@ enum Out { kF32Out = 0, kGated = 1 };
 struct TileShape {
   int M, N, K, kper;  // kper: k of a part, a multiple of 64
   int mt, nt, parts;  // tiles along m and n, parts of k
+  int ldo, up;        // length of a row of the results, rows of W from a feature's gate to its up row
+  size_t plane;       // results of a part of k
 };
 
 template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC>
@@ -105,7 +107,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
       int n;
       if (OUT == kGated) {  // 32 gate rows, then the up rows of the same features
         const int f = in * (BN / 2) + 32 * (row >> 6) + (row & 31);
-        n = min(f, inter - 1) + ((row >> 5) & 1) * inter;
+        n = min(f, inter - 1) + ((row >> 5) & 1) * sh.up;
       } else {
         n = min(in * BN + row, sh.N - 1);
       }
@@ -252,11 +254,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
             const int f = fcol + 16 * (wn * RT + r) + 8 * lpiece;
             if (!stored && (m >= sh.M || f >= inter)) continue;
             if (RT - r < 4 && lpiece >= 4) continue;  // a lone pair of tiles: half a row
-            *reinterpret_cast<uint4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * inter + f) = y;
+            *reinterpret_cast<uint4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * sh.ldo + f) = y;
           } else {
             const int n = n0 + 32 * (wn * RT + r) + 4 * lpiece;
             if (!stored && (m >= sh.M || n >= sh.N)) continue;
-            *reinterpret_cast<uint4*>(static_cast<float*>(out) + (static_cast<size_t>(part) * sh.M + m) * sh.N + n) = y;
+            *reinterpret_cast<uint4*>(static_cast<float*>(out) + part * sh.plane + static_cast<size_t>(m) * sh.ldo + n) = y;
           }
         }
       }
@@ -292,42 +294,91 @@ constexpr TileCost kUnits[] = {{256, 256, 3.1, 0.0, 1.471, 0.291, 0.000},
                                {96, 192, 4.1, 0.9, 0.586, 0.768, 0.041}};
 constexpr int kMaxParts = 6;
 constexpr double kReadMb = 0.2;              // the consumer's reading of a further part, a megabyte
+// A product cut in two (see TileChoice) pays for a second launch, and full rounds run at lower clocks than a nearly empty one:
+// of twenty sizes, what these sums promise came out 4.5 % lower on average, so a cut has to look that much better. One launch
+// against two, us: the 7B shape's gate/up 440 -> 417 at 1,777 rows and 278 -> 259 at 1,000, its q/k/v 135 -> 127 at 4,000 and
+// 353 -> 339 at 12,001, the 1.5B shape's gate/up 116 -> 108 at 2,048; not cut, the former's gate/up at 800 rows (262 against 281).
+constexpr double kSecondLaunchUs = 2.0, kCutCost = 1.045;
 constexpr double kMostPartsBytes = 536870912.0;  // parts of k together take no more scratch memory than this
 
+// Which tiles, in how many parts of k; and, where that leaves the last round of blocks nearly empty, a cut: tiles of `cfg`
+// make the first `cut` rows of X (by_rows) or of W (gated: features), which fill their rounds, tiles of `rest` the others in a
+// launch of its own.
 struct TileChoice {
   int cfg, parts, kper;
   double us;
+  int cut, by_rows, rest;
 };
 
-TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, int K, int only_parts) {
-  TileChoice best{0, 1, K, 1e30};
+double tile_us(const TileCost& c, bool gated, int M, int N, int K, int kper, int parts) {
   const double units = compute_units(), rows_mb = static_cast<double>(M) * N * 1e-6;
+  const double tiles = static_cast<double>((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * parts;
+  const double rounds = static_cast<double>(static_cast<long>((tiles + units - 1) / units));
+  const double out_mb = rows_mb * (gated ? 1.0 : 4.0 * parts);
+  return c.launch + rounds * (c.round + kper / BK * c.stage) + out_mb * c.out_mb + 2e-6 * N * static_cast<double>(K) * c.weight_mb +
+         (parts - 1) * 4.0 * rows_mb * kReadMb;
+}
+
+TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, int K, int only_parts) {
+  TileChoice best{0, 1, K, 1e30, 0, 0, 0};
+  const int units = compute_units();
   for (int parts = 1; parts <= (gated ? 1 : kMaxParts); ++parts) {
     if (only_parts && parts != only_parts) continue;
     const int kper = ((K + parts - 1) / parts + BK - 1) / BK * BK;
     // A part is at least 256 k, none is empty; a caller that names the number of parts has asked here before.
     if (parts > 1 && (K / parts < 256 || static_cast<long>(parts - 1) * kper >= K)) continue;
-    if (parts > 1 && 4e6 * rows_mb * parts > kMostPartsBytes) continue;
+    if (parts > 1 && 4.0 * M * N * parts > kMostPartsBytes) continue;
     for (int i = 0; i < n_costs; ++i) {
       const TileCost& c = costs[i];
-      const double tiles = static_cast<double>((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * parts;
-      const double rounds = static_cast<double>(static_cast<long>((tiles + units - 1) / units));
-      const double out_mb = rows_mb * (gated ? 1.0 : 4.0 * parts);
-      const double us = c.launch + rounds * (c.round + kper / BK * c.stage) + out_mb * c.out_mb +
-                        2e-6 * N * static_cast<double>(K) * c.weight_mb + (parts - 1) * 4.0 * rows_mb * kReadMb;
-      if (us < best.us) best = TileChoice{i, parts, kper, us};
+      const double us = tile_us(c, gated, M, N, K, kper, parts);
+      if (us < best.us) best = TileChoice{i, parts, kper, us, 0, 0, 0};
+      const long mt = (M + c.bm - 1) / c.bm, nt = (N + c.bn - 1) / c.bn, rounds = (mt * nt * parts + units - 1) / units;
+      for (long full = rounds - 1; full >= 1 && full >= rounds - 2; --full) {
+        for (int by_rows = 0; by_rows < 2; ++by_rows) {
+          const long cut = full * units / parts / (by_rows ? nt : mt);
+          if (cut < 1 || cut >= (by_rows ? mt : nt)) continue;
+          const int m1 = by_rows ? static_cast<int>(cut) * c.bm : M, n1 = by_rows ? N : static_cast<int>(cut) * c.bn;
+          const int m2 = by_rows ? M - m1 : M, n2 = by_rows ? N : N - n1;
+          const double first = kCutCost * (tile_us(c, gated, m1, n1, K, kper, parts) + kSecondLaunchUs);
+          if (first >= best.us) continue;
+          for (int j = 0; j < n_costs; ++j) {
+            const double both = first + kCutCost * tile_us(costs[j], gated, m2, n2, K, kper, parts);
+            if (both < best.us) best = TileChoice{i, parts, kper, both, by_rows ? m1 : gated ? n1 / 2 : n1, by_rows, j};
+          }
+        }
+      }
     }
   }
   return best;
 }
 
+// Rows [m0, m0 + M) of X against rows (gated: features) [n0, n0 + N) of W, of a product of all_m x all_n.
+struct Region {
+  int m0, M, n0, N, all_m, all_n;
+};
+
 template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC>
-void launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, int M, int N, int K, int kper, int parts, GateShape act,
+void launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, const Region& r, int K, int kper, int parts, GateShape act,
             hipStream_t stream) {
-  const TileShape sh{M, N, K, kper, (M + BM - 1) / BM, (N + BN - 1) / BN, parts};
+  const bool gated = OUT == kGated;
+  const int rows = gated ? 2 * r.N : r.N;  // of W
+  const TileShape sh{r.M, rows, K, kper, (r.M + BM - 1) / BM, (rows + BN - 1) / BN, parts, r.all_n, r.all_n,
+                     static_cast<size_t>(r.all_m) * r.all_n};
   const int tiles = sh.mt * sh.nt * parts;
+  const size_t at = static_cast<size_t>(r.m0) * r.all_n + r.n0;
+  void* to = gated ? static_cast<void*>(static_cast<bf16*>(out) + at) : static_cast<void*>(static_cast<float*>(out) + at);
   hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, S, OUT, OCC>), dim3(tiles < compute_units() ? tiles : compute_units()),
-                     dim3(64 * WM * WN), 0, stream, X, ldx, W, ldw, out, sh, act);
+                     dim3(64 * WM * WN), 0, stream, X + static_cast<size_t>(r.m0) * ldx, ldx, W + static_cast<size_t>(r.n0) * ldw, ldw, to,
+                     sh, act);
+}
+
+// The whole product, or its two regions.
+template <typename Launch>
+void launch_regions(const TileChoice& c, int M, int N, const Launch& go) {
+  if (!c.cut) return go(c.cfg, Region{0, M, 0, N, M, N});
+  go(c.cfg, Region{0, c.by_rows ? c.cut : M, 0, c.by_rows ? N : c.cut, M, N});
+  if (c.by_rows) go(c.rest, Region{c.cut, M - c.cut, 0, N, M, N});
+  else go(c.rest, Region{0, M, c.cut, N - c.cut, M, N});
 }
 
 int check_tile(const char* name, const void* X, const void* W, const void* out, int M, int N, int K, long ldx, long ldw) {
@@ -351,6 +402,12 @@ extern "C" int pyre_gemm_tile_parts(int M, int N, int K) {
   return choose(kSums, sizeof(kSums) / sizeof(kSums[0]), false, M, N, K, 0).parts;
 }
 
+extern "C" int pyre_gemm_tile_launches(int M, int N, int K, int gated) {
+  const TileChoice c = gated ? choose(kUnits, sizeof(kUnits) / sizeof(kUnits[0]), true, M, N, K, 0)
+                             : choose(kSums, sizeof(kSums) / sizeof(kSums[0]), false, M, N, K, 0);
+  return c.cut ? 2 : 1;
+}
+
 // out: float32 [parts][M][N].
 extern "C" int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long ldw, float* out, int M, int N, int K, int parts,
                                    hipStream_t stream) {
@@ -360,11 +417,13 @@ extern "C" int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long 
   const bf16* x = static_cast<const bf16*>(X);
   const bf16* w = static_cast<const bf16*>(W);
   const GateShape act{};
-  if (c.cfg == 0) launch<256, 256, 4, 2, 2, kF32Out, 2>(x, ldx, w, ldw, out, M, N, K, c.kper, parts, act, stream);
-  else if (c.cfg == 1) launch<256, 192, 4, 2, 2, kF32Out, 2>(x, ldx, w, ldw, out, M, N, K, c.kper, parts, act, stream);
-  else if (c.cfg == 2) launch<128, 192, 2, 2, 3, kF32Out, 1>(x, ldx, w, ldw, out, M, N, K, c.kper, parts, act, stream);
-  else if (c.cfg == 3) launch<128, 128, 2, 4, 4, kF32Out, 2>(x, ldx, w, ldw, out, M, N, K, c.kper, parts, act, stream);
-  else launch<64, 128, 1, 4, 6, kF32Out, 1>(x, ldx, w, ldw, out, M, N, K, c.kper, parts, act, stream);
+  launch_regions(c, M, N, [&](int cfg, const Region& r) {
+    if (cfg == 0) launch<256, 256, 4, 2, 2, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else if (cfg == 1) launch<256, 192, 4, 2, 2, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else if (cfg == 2) launch<128, 192, 2, 2, 3, kF32Out, 1>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else if (cfg == 3) launch<128, 128, 2, 4, 4, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else launch<64, 128, 1, 4, 6, kF32Out, 1>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+  });
   return check_launch("gemm_tile_bf16");
 }
 
@@ -377,11 +436,13 @@ extern "C" int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, l
   const bf16* x = static_cast<const bf16*>(X);
   const bf16* w = static_cast<const bf16*>(W);
   const GateShape act{limit, slope, shift, cubic};
-  if (c.cfg == 0) launch<256, 256, 4, 2, 2, kGated, 2>(x, ldx, w, ldw, out, M, two_i, K, c.kper, 1, act, stream);
-  else if (c.cfg == 1) launch<192, 256, 2, 4, 2, kGated, 2>(x, ldx, w, ldw, out, M, two_i, K, c.kper, 1, act, stream);
-  else if (c.cfg == 2) launch<192, 192, 2, 3, 2, kGated, 2>(x, ldx, w, ldw, out, M, two_i, K, c.kper, 1, act, stream);
-  else if (c.cfg == 3) launch<128, 256, 2, 2, 3, kGated, 1>(x, ldx, w, ldw, out, M, two_i, K, c.kper, 1, act, stream);
-  else if (c.cfg == 4) launch<96, 256, 1, 4, 3, kGated, 1>(x, ldx, w, ldw, out, M, two_i, K, c.kper, 1, act, stream);
-  else launch<96, 192, 1, 3, 3, kGated, 1>(x, ldx, w, ldw, out, M, two_i, K, c.kper, 1, act, stream);
+  launch_regions(c, M, two_i / 2, [&](int cfg, const Region& r) {
+    if (cfg == 0) launch<256, 256, 4, 2, 2, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 1) launch<192, 256, 2, 4, 2, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 2) launch<192, 192, 2, 3, 2, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 3) launch<128, 256, 2, 2, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 4) launch<96, 256, 1, 4, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else launch<96, 192, 1, 3, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+  });
   return check_launch("gemm_tile_glu_bf16");
 }

@@ -102,6 +102,8 @@ int pyre_gemm_mid_silu_bf16(const void* X, long ldx, const void* W, long ldw, vo
 // out bfloat16 [M][two_i / 2]. N (two_i) a multiple of 16, K of 64.
 int pyre_gemm_tile_supports(int M, int N, int K, long ldx, long ldw);
 int pyre_gemm_tile_parts(int M, int N, int K);
+// Launches of the product (gated: N = gate and up rows): 2 where a region of smaller tiles makes what would be a nearly empty round.
+int pyre_gemm_tile_launches(int M, int N, int K, int gated);
 int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long ldw, float* out, int M, int N, int K, int parts,
                         hipStream_t stream);
 int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, long ldw, void* out, int M, int two_i, int K, float limit,

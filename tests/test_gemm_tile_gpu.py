@@ -122,3 +122,25 @@ def test_a_step_against_the_librarys_products(n):
         eng.finish("a")
     scale = rows[1].abs().amax(1)
     assert float(((rows[0] - rows[1]).abs().amax(1) / scale).max()) <= 2e-2
+
+
+@pytest.mark.parametrize("m,n,k,gated", [(1777, 37904, 1024, True), (2101, 17936, 1536, True), (5501, 3600, 2048, True), (2101, 9040, 2048, False),
+                                         (4501, 3600, 2048, False), (7501, 2064, 2048, False)])
+def test_a_last_round_in_smaller_tiles(m, n, k, gated):
+    """Products cut in two launches, along the rows of either operand: every element is the product of its own rows."""
+    from pyre_amd.hip import ops
+    from pyre_amd.hip.lib import lib
+
+    assert lib().pyre_gemm_tile_launches(m, n, k, int(gated)) == 2
+    x, w = rnd(m, k + 8, seed=8)[:, :k], rnd(n, k + 8, seed=9, scale=0.2)[:, :k]
+    want = x.double() @ w.double().T
+    if gated:
+        out = torch.full((m, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops.gemm_tile_glu_bf16(x, w, out, m)
+        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
+        assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 64 * bound(k)).all())
+    else:
+        parts = ops.gemm_tile_parts(m, n, k)
+        out = torch.full((parts, m, n), float("nan"), device=DEV)
+        ops.gemm_tile_bf16(x, w, out, m, parts)
+        assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * float(want.std()) * 4
