@@ -596,6 +596,8 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, ou
 #: parts with their way through memory (566 rows, the way down: 139, 176, 131, 143)
 F32_KSPLIT_MAX = 14
 F32_KSPLIT_MIN_K = 192
+#: what the kernels round a part of k up to
+F32_K_STAGE = 16
 
 
 def compute_units(device=None) -> int:
@@ -611,11 +613,20 @@ def compute_units(device=None) -> int:
 
 def gemm_f32_ksplit(n_out: int, k: int, units: int = DEFAULT_UNITS) -> int:
     """Into how many parts of k the float32 product is split: enough blocks of 128 output
-    columns for the ``units`` compute units, parts of at least 192. A function of the weight's
+    columns for the ``units`` compute units, parts of at least 192, none of them empty (a part is rounded up to
+    16 k: fourteen parts of 208 would leave the last of 2,704 nothing). A function of the weight's
     shape (and the engine's device) alone, never of the rows, so that a row's result does not
     depend on its step."""
     blocks = -(-n_out // 128)
-    return max(1, min(F32_KSPLIT_MAX, units // blocks, k // F32_KSPLIT_MIN_K))
+    ks = max(1, min(F32_KSPLIT_MAX, units // blocks, k // F32_KSPLIT_MIN_K))
+    while ks > 1 and (ks - 1) * f32_part(k, ks) >= k:
+        ks -= 1
+    return ks
+
+
+def f32_part(k: int, ksplit: int) -> int:
+    """The length of a part of k (the last one may be shorter), as the kernels form it."""
+    return -(-(-(-k // ksplit)) // F32_K_STAGE) * F32_K_STAGE
 
 
 @lru_cache(maxsize=4096)
