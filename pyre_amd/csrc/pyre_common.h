@@ -133,7 +133,12 @@ __device__ inline float gated_unit(float gate, float up, GateShape a) {
 }
 // Whether the unit is the SiLU-gate, which needs none of the above's other steps.
 __device__ inline bool is_silu(GateShape a) { return a.limit <= 0.f && a.slope == 1.f && a.shift == 0.f && a.cubic == 0.f; }
-__device__ inline float silu_unit(float gate, float up) { return gate / (1.f + __expf(-gate)) * up; }
+// In sixteenths, so that the hardware's reciprocal (an error of one unit in the last place of float32) stays a normal number as long
+// as the exponential is one: with the division above the 1.5B shape's gate/up product took 112.9 us instead of 109.2 at 2,048
+// rows, the 7B shape's 463.4 instead of 456.5.
+__device__ inline float silu_unit(float gate, float up) {
+  return 0.0625f * gate * __builtin_amdgcn_rcpf(fmaf(0.0625f, __expf(-gate), 0.0625f)) * up;
+}
 
 __device__ inline float wave_sum(float v) {
 #pragma unroll

@@ -44,3 +44,38 @@ def test_segments(heads, dk, dv, lengths):
         assert bool(torch.isfinite(got).all())
         assert float((got - ref).abs().max() / ref.pow(2).mean().sqrt()) <= 1e-4
         assert float((got - ref).norm() / ref.norm()) <= 4e-6
+
+
+@pytest.mark.parametrize("heads,dk,dv", [(14, 128, 128), (3, 40, 24), (2, 256, 36), (1, 17, 250)])
+@pytest.mark.parametrize("lengths", [[300, 1777], [700, 1, 65, 64, 1, 2, 700, 130], [1] * 70 + [513] + [40] * 70])
+def test_a_request_has_the_same_bits_alone_and_among_others(heads, dk, dv, lengths):
+    """Outputs and states of every request of a step, among them more than a wave has lanes, beside each by itself."""
+    from pyre_amd.hip import ops
+
+    n, hk, hv = sum(lengths), heads * dk, heads * dv
+    g = torch.Generator().manual_seed(n + dk)
+    x = torch.randn(n, 3 * hk + 2 * hv, generator=g)
+    x[:, 2 * hk:3 * hk] = -torch.rand(n, hk, generator=g) ** 4 * torch.logspace(-4, 1.2, hk)
+    x = x.to(DEV)
+    state = torch.randn(len(lengths), heads, dk, dv, generator=g).to(DEV)
+
+    def walk(first, lens, states):
+        starts = [0]
+        for m in lens:
+            starts.append(starts[-1] + m)
+        out = torch.full((starts[-1], hv), float("nan"), device=DEV)
+        after = states.clone()
+        scratch = torch.full((ops.gla_chunks_scratch(starts[-1], len(lens), heads, dk, dv),), float("nan"), device=DEV)
+        ops.gla_scan(x[first:first + starts[-1]].contiguous(), after, out, torch.tensor(starts, dtype=torch.int32, device=DEV),
+                     torch.arange(len(lens), dtype=torch.int32, device=DEV), len(lens), heads, dk, dv, dk ** -0.5, scratch, max(lens))
+        return out, after
+
+    out, after = walk(0, lengths, state)
+    at = 0
+    for s, m in enumerate(lengths):
+        if m > 1 or s < 2:
+            alone, state_alone = walk(at, [m], state[s:s + 1])
+            assert torch.equal(alone, out[at:at + m]), s
+            assert torch.equal(state_alone[0], after[s]), s
+        at += m
+    assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(after).all())
