@@ -432,24 +432,68 @@ __device__ inline f32x4* segment_end(const ChunkScratch& sc, int t0, int hd, int
          ((static_cast<size_t>(t0 / (kChunk * kSegment)) * heads + hd) * tiles + tile) * 2 * DT * kWave + lane;
 }
 
-// grid: (heads, tiles of columns, requests x segments) in both kernels; `per`: chunks of a segment, `segments` of the longest
-// request. The blocks of one request lie together in the grid and not those of one head: neighbours go to different dies, and a
-// long prompt beside many single tokens is then not one die's alone. Heads are padded to a multiple of eight, so that the
-// blocks of a head, which read the same operands, share a die and its cache.
+// A segment of a request. How a request is cut follows from its own tokens and `most`, the most segments that a model of these
+// heads is given: the state is summed segment by segment, so a request's bits are the same whatever else is in the step.
+struct Segment {
+  int s, slot;       // the request, its place among the states
+  int seg;           // which of its segments
+  int first, last;   // the segment's tokens
+  int t_begin, per;  // the request's first token, the chunks of its segments
+  bool ends;         // it is the request's last
+};
+// What place z of the grid has to do, found by a wave, a lane a request; false: nothing. A request has a place for every kSegment
+// chunks (2^shift tokens) and one more, which is what it can be cut into at most; where no request of the step is cut, one (a shift
+// that leaves nothing of a token's number); a request alone has all places. (With as many places for every request as for the
+// longest, 60 single tokens beside a prompt of nine segments would be 480 empty blocks a head and tile, each of which holds a
+// SIMD's registers for a microsecond.)
+constexpr int kUncut = 8;  // a request of up to so many chunks is one segment
+constexpr int kSegmentShift = 6, kNoShift = 30;
+static_assert(1 << kSegmentShift == kChunk * kSegment, "a place for every segment");
+__host__ __device__ inline int segment_place(int t_begin, int s, int shift) { return (t_begin >> shift) + s; }
+
+__device__ inline bool find_segment(const int* __restrict__ q_start, const int* __restrict__ state_slots, int n_seqs,
+                                    int most, int shift, int z, Segment& r) {
+  const int lane = threadIdx.x & (kWave - 1);
+  r.s = n_seqs == 1 ? 0 : z;
+  if (n_seqs > 1 && shift != kNoShift) {
+    int s = -1;  // the last request whose places begin at z or before
+    for (int s0 = 0; s0 < n_seqs; s0 += kWave) {
+      const int i = s0 + lane;
+      const int hits = __popcll(__ballot(i < n_seqs && segment_place(q_start[min(i, n_seqs)], i, shift) <= z));
+      s += hits;
+      if (hits < kWave) break;
+    }
+    if (s < 0) return false;
+    r.s = __builtin_amdgcn_readfirstlane(s);
+  }
+  r.t_begin = q_start[r.s];
+  r.slot = state_slots[r.s];
+  const int t_end = q_start[r.s + 1], chunks = (t_end - r.t_begin + kChunk - 1) / kChunk;
+  r.per = shift == kNoShift || chunks <= kUncut ? max(chunks, 1) : max(kSegment, (chunks + most - 1) / most);
+  r.seg = n_seqs == 1 ? z : z - segment_place(r.t_begin, r.s, shift);
+  r.first = r.t_begin + r.seg * r.per * kChunk;
+  r.last = min(t_end, r.first + r.per * kChunk);
+  r.ends = r.last == t_end;
+  return r.first < t_end;
+}
+
+// grid: (heads, tiles of columns, places from `z0` on, see find_segment) in both kernels. The blocks of one request lie together in the grid
+// and not those of one head: neighbours go to different dies, and a long prompt beside many single tokens is then not one die's
+// alone. Heads are padded to a multiple of eight, so that the blocks of a head, which read the same operands, share a die and
+// its cache.
 template <int DT>
 __global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, const float* __restrict__ state,
                                                                const int* __restrict__ q_start,
                                                                const int* __restrict__ state_slots, int heads, int dk, int dv,
-                                                               int dvp, int per, int segments) {
-  const int s = blockIdx.z / segments, seg = blockIdx.z % segments, hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  if (hd >= heads) return;
-  const int t_begin = q_start[s], t_end = q_start[s + 1];
-  const int first = t_begin + seg * per * kChunk, last = first + per * kChunk;
-  if (last >= t_end) return;  // the request's last segment, or none of its
+                                                               int dvp, int n_seqs, int most, int shift, int z0) {
+  const int hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  Segment sg;
+  if (hd >= heads || !find_segment(q_start, state_slots, n_seqs, most, shift, z0 + blockIdx.z, sg) || sg.ends) return;
+  const int s = sg.s, seg = sg.seg, first = sg.first, last = sg.last;
   const int col = blockIdx.y * 16 + c;
   f32x4 S[DT], D[DT];
   if (seg == 0) {
-    load_state<DT>(state + (static_cast<size_t>(state_slots[s]) * heads + hd) * dk * dv, dk, dv, col, g, S);
+    load_state<DT>(state + (static_cast<size_t>(sg.slot) * heads + hd) * dk * dv, dk, dv, col, g, S);
 #pragma unroll
     for (int j = 0; j < DT; ++j) D[j] = S[j];
   } else {
@@ -487,22 +531,19 @@ __global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, 
 template <int DT>
 __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
     ChunkScratch sc, float* __restrict__ state, float* __restrict__ o, const int* __restrict__ q_start,
-    const int* __restrict__ state_slots, int heads, int dk, int dv, int dvp, float qscale, int per, int segments) {
-  const int s = blockIdx.z / segments, seg = blockIdx.z % segments, hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  if (hd >= heads) return;
-  const int col = blockIdx.y * 16 + c;
+    const int* __restrict__ state_slots, int heads, int dk, int dv, int dvp, float qscale, int n_seqs, int most, int shift, int z0) {
+  const int hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  Segment sg;
+  if (hd >= heads || !find_segment(q_start, state_slots, n_seqs, most, shift, z0 + blockIdx.z, sg)) return;
+  const int s = sg.s, seg = sg.seg, first = sg.first, last = sg.last, t_begin = sg.t_begin, per = sg.per;
+  const int col = blockIdx.y * 16 + c, hv = heads * dv;
   const bool has_col = col < dv;
-  const int t_begin = q_start[s], t_end = q_start[s + 1], hv = heads * dv;
-  const int first = t_begin + seg * per * kChunk;
-  const bool whole = seg + 1 < segments && first + per * kChunk < t_end;  // another segment comes after this one
-  const int last = whole ? first + per * kChunk : t_end;
-  if (first >= t_end) return;
   const auto fetch = [&](int t0, ChunkOperands<DT>& r) { fetch_chunk<DT, true>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
   ChunkSets<DT, true> sets;
   sets.begin(first, last, fetch);
-  float* st = state + (static_cast<size_t>(state_slots[s]) * heads + hd) * dk * dv;
+  float* st = state + (static_cast<size_t>(sg.slot) * heads + hd) * dk * dv;
   f32x4 S[DT];
-  if (seg == 0 && !whole) {  // a request of one segment: its state is this wave's alone
+  if (seg == 0 && sg.ends) {  // a request of one segment: its state is this wave's alone
     load_state<DT>(st, dk, dv, col, g, S);
   } else {
     const f32x4* end = segment_end<DT>(sc, t_begin, hd, heads, blockIdx.y, gridDim.y, lane);
@@ -532,7 +573,7 @@ __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
     }
   }
   sets.walk(first, last, fetch, [&](int t0, const ChunkOperands<DT>& now) {
-        const int nc = min(kChunk, t_end - t0);
+        const int nc = min(kChunk, last - t0);
         f32x4 out = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < DT; ++j)
@@ -553,7 +594,7 @@ __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
           for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
         }
       });
-  if (whole) return;
+  if (!sg.ends) return;
 #pragma unroll
   for (int j = 0; j < DT; ++j)
 #pragma unroll
@@ -783,22 +824,24 @@ extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, flo
     hipLaunchKernelGGL(gla_chunk_prep_kernel, prep_grid, dim3(kThreads), sizeof(float) * 3 * kChunk * dk, stream, x, sc, q_start,
                        heads, dk, dv, dkp, dvp);
   if (check_launch("gla_chunk_prep")) return 1;
-  // As many segments as put a wave on every SIMD, counting the requests that may be as long as the longest; a segment costs
-  // its waves a walk for its end and the reading of those before it, so it has four chunks at least.
+  // A request gets as many segments as put a wave on every SIMD when it is alone in the step, whatever else is in it (see Segment):
+  // six prompts of 300 tokens on 14 heads of 128 x 128 take 116 us that way, 87 with segments counted over the whole step and
+  // 139 without any. A segment costs its waves a walk for its end and the reading of those before it, so it has four chunks at
+  // least, and eight are not cut: 16 requests of 100 tokens 83 us, 104 in two segments each.
   const int chunks = (max_tokens + kChunk - 1) / kChunk, tiles = (dv + 15) / 16;
-  const long waves = static_cast<long>((n_tokens + max_tokens - 1) / max_tokens) * heads * tiles;
-  int segments = static_cast<int>(std::max(1L, std::min(static_cast<long>(kMaxSegments), 4L * compute_units() / waves)));
-  int per = std::max(kSegment, (chunks + segments - 1) / segments);
-  segments = (chunks + per - 1) / per;
-  if (static_cast<long>(n_seqs) * segments > 65535) segments = 1, per = chunks;
-  const dim3 grid((heads + 7) / 8 * 8, tiles, n_seqs * segments);
-#define PYRE_WALK(DT)                                                                                                      \
-  do {                                                                                                                     \
-    if (segments > 1)                                                                                                      \
-      hipLaunchKernelGGL(gla_chunk_ends_kernel<DT>, grid, dim3(kWave), 0, stream, sc, state, q_start, state_slots, heads,   \
-                         dk, dv, dvp, per, segments);                                                                      \
-    hipLaunchKernelGGL(gla_chunk_walk_kernel<DT>, grid, dim3(kWave), 0, stream, sc, state, o, q_start, state_slots, heads, \
-                       dk, dv, dvp, qscale, per, segments);                                                                \
+  const int most = std::max(1, std::min(kMaxSegments, 4 * compute_units() / (heads * tiles)));
+  const bool cut = most > 1 && chunks > kUncut;  // some request may be
+  const int shift = cut ? kSegmentShift : kNoShift;
+  const long places = n_seqs == 1 ? (cut ? most : 1) : segment_place(n_tokens, n_seqs, shift);
+#define PYRE_WALK_Z(KERNEL, ...)                                                                                       \
+  for (long z0 = 0; z0 < places; z0 += 65535)                                                                        \
+  hipLaunchKernelGGL(KERNEL, dim3((heads + 7) / 8 * 8, tiles, static_cast<unsigned>(std::min(65535L, places - z0))), \
+                     dim3(kWave), 0, stream, __VA_ARGS__, n_seqs, most, shift, static_cast<int>(z0))
+#define PYRE_WALK(DT)                                                                                       \
+  do {                                                                                                      \
+    if (cut)                                                                                                \
+      PYRE_WALK_Z(gla_chunk_ends_kernel<DT>, sc, state, q_start, state_slots, heads, dk, dv, dvp);          \
+    PYRE_WALK_Z(gla_chunk_walk_kernel<DT>, sc, state, o, q_start, state_slots, heads, dk, dv, dvp, qscale); \
   } while (0)
   switch (DTs) {
     case 2: PYRE_WALK(2); break;
@@ -807,6 +850,7 @@ extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, flo
     default: PYRE_WALK(16); break;
   }
 #undef PYRE_WALK
+#undef PYRE_WALK_Z
   return check_launch("gla_chunks");
 }
 
