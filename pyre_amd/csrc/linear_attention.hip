@@ -153,12 +153,12 @@ __global__ __launch_bounds__(kThreads) void gla_scan_kernel(
 // chunk and head makes A, q * exp(b), k * exp(B - b), exp(B) and v in the layouts of the matrix
 // instruction's operands) and the kernel that walks the chunks (gla_chunk_walk: a wave per request,
 // head and 16 columns of the state, nothing shared between waves) is left with three small matrix
-// products per chunk, whose operands it asks for one chunk ahead.
+// products per chunk, whose operands it asks for two chunks ahead (see ChunkSets).
 // A walk is a chain of dependent instructions (2.2 us a chunk) and a prompt's heads are few waves: 112 of 1,024 SIMDs for 14 heads of
 // 128 columns. So the chunks of a prompt are dealt to segments that are walked at the same time: gla_chunk_ends first
 // walks all segments but the last, the first of them from the request's state and the others from zero, and leaves the states at their
 // ends and the products of their decays; in gla_chunk_walk a segment's wave makes the state before it from those of the
-// segments before it, S = diag(decays) S + end, in their order. Two walks of a ninth of the length: 251 -> 25 + 58 us a layer for a
+// segments before it, S = diag(decays) S + end, in their order. Two walks of a ninth of the length: 251 -> 23 + 48 us a layer for a
 // prompt of 1,777 tokens on 14 heads of 128 x 128.
 // Chunks are counted from the first token that the request brings in this step. A chunk's operands
 // lie at "slots": token t of request s of the step has slot t + 16 s, so that the 16 slots of a
@@ -366,52 +366,78 @@ struct ChunkOperands {
   f32x4 q[DT], k[DT], e[DT], v, a;
 };
 
-// Chunk t0 of request s: for the states alone (OUT false) its keys, values and decays.
-template <int DT, bool OUT>
-__device__ inline void fetch_chunk(const ChunkScratch& sc, int t0, int s, int hd, int heads, int col, int dv, int dvp, int g, int c,
-                                   ChunkOperands<DT>& r) {
+// Of chunk t0 of request s: what its outputs take besides the state before it, and what takes that state on.
+template <int DT>
+__device__ inline void fetch_queries(const ChunkScratch& sc, int t0, int s, int hd, int heads, int g, int c, ChunkOperands<DT>& r) {
   constexpr int dkp = 16 * DT;
-  const size_t slot0 = static_cast<size_t>(t0) + kChunk * s;
-  const size_t region = slot0 * heads + static_cast<size_t>(hd) * kChunk;
-  const float* qp = sc.qd + ((slot0 + c) * heads + hd) * dkp + 4 * g;
+  const size_t row = (static_cast<size_t>(t0) + kChunk * s + c) * heads + hd;
+  const float* qp = sc.qd + row * dkp + 4 * g;
+#pragma unroll
+  for (int j = 0; j < DT; ++j) r.q[j] = *reinterpret_cast<const f32x4*>(qp + 16 * j);
+  r.a = *reinterpret_cast<const f32x4*>(sc.pairs + row * kChunk + 4 * g);
+}
+template <int DT>
+__device__ inline void fetch_keys(const ChunkScratch& sc, int t0, int s, int hd, int heads, int col, int dv, int dvp, int g, int c,
+                                  ChunkOperands<DT>& r) {
+  constexpr int dkp = 16 * DT;
+  const size_t region = (static_cast<size_t>(t0) + kChunk * s) * heads + static_cast<size_t>(hd) * kChunk;
   const float* kp = sc.kdt + region * dkp + c * kChunk + 4 * g;
   const float* ep = sc.eb + region * kChunk + 4 * g;
 #pragma unroll
   for (int j = 0; j < DT; ++j) {
-    if (OUT) r.q[j] = *reinterpret_cast<const f32x4*>(qp + 16 * j);
     r.k[j] = *reinterpret_cast<const f32x4*>(kp + 16 * j * kChunk);
     r.e[j] = *reinterpret_cast<const f32x4*>(ep + 16 * j);
   }
+  // Columns past the last are the last one once more: nobody stores what comes of them (zeros in their place would be waited for here).
   r.v = *reinterpret_cast<const f32x4*>(sc.vt + region * dvp + static_cast<size_t>(min(col, dvp - 1)) * kChunk + 4 * g);
-  if (col >= dv) r.v = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (OUT) r.a = *reinterpret_cast<const f32x4*>(sc.pairs + ((slot0 + c) * heads + hd) * kChunk + 4 * g);
 }
 
-// `step` on every chunk from `first` to `last`, its operands asked for two chunks ahead: three sets of registers that take turns
-// (a set copied into another would be waited for at the copy; heads beyond 128 have no registers for that many).
-template <int DT, bool OUT>
+// Every chunk from `first` to `last`: `outputs` and then `state` on its operands. Three sets of registers take turns, so that a
+// chunk's operands are asked for two chunks ahead (a set copied into another would be waited for at the copy). Heads beyond 128
+// have registers for one set: its queries are asked for again when the chunk's outputs are made, before the state is taken on,
+// its keys behind that (1,777 tokens of two heads of 256 x 256, all kernels: 166 us; with two sets, which do not fit, and one asked
+// for whole behind the chunk 312).
+template <int DT>
 struct ChunkSets {
-  static constexpr int N = DT > 8 ? (OUT ? 1 : 2) : 3;
+  static constexpr int N = DT > 8 ? 1 : 3;
   ChunkOperands<DT> r[N];
-  template <typename Fetch>
-  __device__ void begin(int first, int last, Fetch fetch) {
+  template <typename FetchQ, typename FetchK>
+  __device__ void begin(int from, int to, int first, int last, FetchQ fetch_q, FetchK fetch_k) {  // the first operands of sets from .. to - 1
 #pragma unroll
     for (int b = 0; b < N; ++b)
-      if (first + b * kChunk < last) fetch(first + b * kChunk, r[b]);
+      if (b >= from && b < to && first + b * kChunk < last) {
+        fetch_q(first + b * kChunk, r[b]);
+        fetch_k(first + b * kChunk, r[b]);
+      }
   }
-  template <typename Fetch, typename Step>
-  __device__ void walk(int first, int last, Fetch fetch, Step step) {
+  template <typename FetchQ, typename FetchK, typename Outputs, typename State>
+  __device__ void walk(int first, int last, FetchQ fetch_q, FetchK fetch_k, Outputs outputs, State state) {
     for (int t0 = first; t0 < last; t0 += N * kChunk) {
 #pragma unroll
       for (int b = 0; b < N; ++b) {
         const int t = t0 + b * kChunk;
         if (t >= last) return;
-        step(t, r[b]);
-        if (t + N * kChunk < last) fetch(t + N * kChunk, r[b]);
+        const bool more = t + N * kChunk < last;
+        outputs(t, r[b]);
+        if (more) fetch_q(t + N * kChunk, r[b]);
+        state(r[b]);
+        if (more) fetch_k(t + N * kChunk, r[b]);
       }
     }
   }
 };
+
+// The state after a chunk from the one before it.
+template <int DT>
+__device__ inline void take_on(const ChunkOperands<DT>& now, f32x4 (&S)[DT]) {
+#pragma unroll
+  for (int j = 0; j < DT; ++j) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[j][i] *= now.e[j][i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
+  }
+}
 
 // The state's rows and columns of a lane.
 template <int DT>
@@ -503,23 +529,19 @@ __global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, 
       D[j] = f32x4{1.f, 1.f, 1.f, 1.f};
     }
   }
-  const auto fetch = [&](int t0, ChunkOperands<DT>& r) { fetch_chunk<DT, false>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
-  ChunkSets<DT, false> sets;
-  sets.begin(first, last, fetch);
-  sets.walk(first, last, fetch, [&](int, const ChunkOperands<DT>& now) {
+  const auto fetch = [&](int t0, ChunkOperands<DT>& r) { fetch_keys<DT>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
+  ChunkSets<DT> sets;
+  const auto state_on = [&](const ChunkOperands<DT>& now) {
+    take_on<DT>(now, S);
+    if (seg == 0) return;
 #pragma unroll
-        for (int j = 0; j < DT; ++j) {
+    for (int j = 0; j < DT; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            S[j][i] *= now.e[j][i];
-            if (seg) D[j][i] *= now.e[j][i];
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int j = 0; j < DT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
-      });
+      for (int i = 0; i < 4; ++i) D[j][i] *= now.e[j][i];
+  };
+  const auto no_queries = [](int, ChunkOperands<DT>&) {};
+  sets.begin(0, sets.N, first, last, no_queries, fetch);
+  sets.walk(first, last, no_queries, fetch, [](int, const ChunkOperands<DT>&) {}, state_on);
   f32x4* end = segment_end<DT>(sc, first, hd, heads, blockIdx.y, gridDim.y, lane);
 #pragma unroll
   for (int j = 0; j < DT; ++j) {
@@ -538,9 +560,12 @@ __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
   const int s = sg.s, seg = sg.seg, first = sg.first, last = sg.last, t_begin = sg.t_begin, per = sg.per;
   const int col = blockIdx.y * 16 + c, hv = heads * dv;
   const bool has_col = col < dv;
-  const auto fetch = [&](int t0, ChunkOperands<DT>& r) { fetch_chunk<DT, true>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
-  ChunkSets<DT, true> sets;
-  sets.begin(first, last, fetch);
+  const auto fetch_q = [&](int t0, ChunkOperands<DT>& r) { fetch_queries<DT>(sc, t0, s, hd, heads, g, c, r); };
+  const auto fetch_k = [&](int t0, ChunkOperands<DT>& r) { fetch_keys<DT>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
+  ChunkSets<DT> sets;
+  // on their way while the state is formed: as many as there are registers for beside it
+  constexpr int early = DT <= 8 ? 1 : 0;
+  sets.begin(0, early, first, last, fetch_q, fetch_k);
   float* st = state + (static_cast<size_t>(sg.slot) * heads + hd) * dk * dv;
   f32x4 S[DT];
   if (seg == 0 && sg.ends) {  // a request of one segment: its state is this wave's alone
@@ -572,28 +597,23 @@ __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
       add(b + 1, 1);
     }
   }
-  sets.walk(first, last, fetch, [&](int t0, const ChunkOperands<DT>& now) {
-        const int nc = min(kChunk, last - t0);
-        f32x4 out = {0.f, 0.f, 0.f, 0.f};
+  sets.begin(early, sets.N, first, last, fetch_q, fetch_k);
+  const auto outputs = [&](int t0, const ChunkOperands<DT>& now) {
+    const int nc = min(kChunk, last - t0);
+    f32x4 out = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < DT; ++j)
+    for (int j = 0; j < DT; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[j][i], S[j][i], out, 0, 0, 0);
+      for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.q[j][i], S[j][i], out, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a[i], now.v[i], out, 0, 0, 0);
+    for (int i = 0; i < 4; ++i) out = __builtin_amdgcn_mfma_f32_16x16x4f32(now.a[i], now.v[i], out, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = 4 * g + i;
-          if (t < nc && has_col) o[static_cast<size_t>(t0 + t) * hv + hd * dv + col] = out[i] * qscale;
-        }
-#pragma unroll
-        for (int j = 0; j < DT; ++j) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) S[j][i] *= now.e[j][i];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(now.k[j][i], now.v[i], S[j], 0, 0, 0);
-        }
-      });
+    for (int i = 0; i < 4; ++i) {
+      const int t = 4 * g + i;
+      if (t < nc && has_col) o[static_cast<size_t>(t0 + t) * hv + hd * dv + col] = out[i] * qscale;
+    }
+  };
+  sets.walk(first, last, fetch_q, fetch_k, outputs, [&](const ChunkOperands<DT>& now) { take_on<DT>(now, S); });
   if (!sg.ends) return;
 #pragma unroll
   for (int j = 0; j < DT; ++j)
@@ -825,17 +845,17 @@ extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, flo
                        heads, dk, dv, dkp, dvp);
   if (check_launch("gla_chunk_prep")) return 1;
   // A request gets as many segments as put a wave on every SIMD when it is alone in the step, whatever else is in it (see Segment):
-  // six prompts of 300 tokens on 14 heads of 128 x 128 take 116 us that way, 87 with segments counted over the whole step and
-  // 139 without any. A segment costs its waves a walk for its end and the reading of those before it, so it has four chunks at
-  // least, and eight are not cut: 16 requests of 100 tokens 83 us, 104 in two segments each.
+  // six prompts of 300 tokens on 14 heads of 128 x 128 take 103 us that way and 139 without any. A segment costs its waves a walk
+  // for its end and the reading of those before it, so it has four chunks at least, and eight are not cut: 16 requests of 100
+  // tokens 75 us, 99 in two segments each.
   const int chunks = (max_tokens + kChunk - 1) / kChunk, tiles = (dv + 15) / 16;
   const int most = std::max(1, std::min(kMaxSegments, 4 * compute_units() / (heads * tiles)));
   const bool cut = most > 1 && chunks > kUncut;  // some request may be
   const int shift = cut ? kSegmentShift : kNoShift;
   const long places = n_seqs == 1 ? (cut ? most : 1) : segment_place(n_tokens, n_seqs, shift);
 #define PYRE_WALK_Z(KERNEL, ...)                                                                                       \
-  for (long z0 = 0; z0 < places; z0 += 65535)                                                                        \
-  hipLaunchKernelGGL(KERNEL, dim3((heads + 7) / 8 * 8, tiles, static_cast<unsigned>(std::min(65535L, places - z0))), \
+  for (long z0 = 0; z0 < places; z0 += 65535)                                                                          \
+  hipLaunchKernelGGL(KERNEL, dim3((heads + 7) / 8 * 8, tiles, static_cast<unsigned>(std::min(65535L, places - z0))),   \
                      dim3(kWave), 0, stream, __VA_ARGS__, n_seqs, most, shift, static_cast<int>(z0))
 #define PYRE_WALK(DT)                                                                                       \
   do {                                                                                                      \
