@@ -755,9 +755,10 @@ constexpr int kKeys = 64;
 
 // 16 bytes per lane from global memory straight into LDS: lane x's piece lands at
 // lds_addr + 16 x. The compiler does not know of these loads; whoever reads the bytes
-// waits for them with wait_loads (they finish in the order of issue) and a barrier.
+// waits for them with wait_loads (they finish in the order of issue) and a barrier. The s_nop is the wait state that the instruction
+// needs behind a scalar write of m0; the compiler puts none into inline assembly.
 __device__ inline void load_to_lds(const void* src, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_addr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_addr) : "memory", "m0");
 }
 template <int N>
 __device__ inline void wait_loads() {

@@ -148,9 +148,10 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
   }
 }
 
-// 16 bytes per lane from `base + off` straight into LDS: lane x's piece lands at lds_addr + 16 x (see load_to_lds below).
+// 16 bytes per lane from `base + off` straight into LDS: lane x's piece lands at lds_addr + 16 x. The s_nop is the wait state that the instruction
+// needs behind a scalar write of m0; the compiler puts none into inline assembly.
 __device__ inline void load_rows(const void* base, unsigned off, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
 template <int N>
 __device__ inline void wait_loads() {
@@ -354,7 +355,7 @@ constexpr int kStreamMaxRows = 64;
 constexpr int kMaxDevices = 64;
 
 __device__ inline void load_to_lds(const void* src, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_addr) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_addr) : "memory", "m0");
 }
 __device__ __attribute__((aligned(16))) const unsigned kZeroPiece[4] = {0u, 0u, 0u, 0u};
 
