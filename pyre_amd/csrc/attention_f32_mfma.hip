@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     int hd, int page_size, float scale, int window) {
   __shared__ float Ks[kKeys][HDP + 1];   // rows on distinct banks for the lanes of a half-wave
   __shared__ float Vt[HDP][kKeys + 1];
-  __shared__ int page_s[kKeys];          // the page of each key of the chunk, -1 if it is not there
+  __shared__ int page_s[kKeys];          // the page of each key of the chunk, -1 if it is not there (VEC: see missing)
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int n_rep = nq / nkv, hgroups = (n_rep + 3) / 4;
   const int kvh = blockIdx.y / hgroups, hin = (blockIdx.y % hgroups) * 4 + wave;
@@ -80,25 +80,30 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   constexpr int PIECES = HDP / 32;  // 16-byte pieces of keys, and of values, of a thread and chunk
   f32x4 kp[VEC ? PIECES : 1], vp[VEC ? PIECES : 1];
   int kpage[VEC ? PIECES : 1], vpage = -1;
+  unsigned missing = 0, next_missing = 0;  // VEC: which fourths of the chunk's keys (of the next's) have no page though the step has them
   const int vkey = 4 * (tid & 7);  // the first of the four keys of this thread's pieces of values
+  // the key of this thread's piece i of a chunk's keys (heads of 256: a whole wave's, so that pages and rows are scalars)
+  const int wave_id = __builtin_amdgcn_readfirstlane(wave);
+  auto piece_key = [&](int i) { return HDP == 256 ? wave_id + 4 * i : (tid + 256 * i) / (HDP / 4); };
   auto page_of = [&](int key) {
     const int entry = key / page_size;
     return key <= hi_all && entry < table_stride ? table[entry] : -1;
   };
   auto look_up = [&](int chunk) {  // the pages of this thread's pieces of a chunk
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) kpage[i] = page_of(kKeys * chunk + (tid + 256 * i) / (HDP / 4));
+    for (int i = 0; i < PIECES; ++i) kpage[i] = page_of(kKeys * chunk + piece_key(i));
     vpage = page_of(kKeys * chunk + vkey);
   };
   auto fetch = [&](int chunk) {
     const int key0 = kKeys * chunk;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int key = key0 + (tid + 256 * i) / (HDP / 4), d = 4 * ((tid + 256 * i) % (HDP / 4));
+      const int key = key0 + piece_key(i), d = 4 * ((tid + 256 * i) % (HDP / 4));
       kp[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (kpage[i] >= 0 && d < hd)
         kp[i] = *reinterpret_cast<const f32x4*>(k_cache + ((static_cast<size_t>(kpage[i]) * nkv + kvh) * page_size + key % page_size) * hd + d);
     }
+    next_missing = __ballot(vpage < 0 && key0 + vkey <= hi_all) & 0xffu;
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int d = (tid >> 3) + 32 * i, key = key0 + vkey;
@@ -123,7 +128,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     if (VEC) {
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) {
-        const int key = (tid + 256 * i) / (HDP / 4), d = 4 * ((tid + 256 * i) % (HDP / 4));
+        const int key = piece_key(i), d = 4 * ((tid + 256 * i) % (HDP / 4));
 #pragma unroll
         for (int j = 0; j < 4; ++j) Ks[key][d + j] = kp[i][j];
       }
@@ -131,6 +136,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
       for (int i = 0; i < PIECES; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) Vt[(tid >> 3) + 32 * i][vkey + j] = vp[i][j];
+      missing = next_missing;
       __syncthreads();
       if (chunk < last_chunk) {
         fetch(chunk + 1);
@@ -168,8 +174,16 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int kk = 8 * (i >> 2) + 4 * h + (i & 3), key = key0 + kk;
-      s[i] = key < lo || key > hi ? -INFINITY : s[i] * scale;  // what a token sees is there
+      s[i] = key < lo || key > hi || (!VEC && page_s[kk] < 0) ? -INFINITY : s[i] * scale;
       mx = fmaxf(mx, s[i]);
+    }
+    if (VEC && missing) {
+      mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if (missing >> (2 * (i >> 2) + h) & 1) s[i] = -INFINITY;
+        mx = fmaxf(mx, s[i]);
+      }
     }
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float m_new = fmaxf(m, mx);

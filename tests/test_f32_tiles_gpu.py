@@ -70,6 +70,35 @@ def test_attention_of_prompts(hd, page, window):
         assert float((out[:, h].double() - want).abs().max()) <= 2e-5
 
 
+@pytest.mark.parametrize("hd,page", [(64, 16), (128, 8), (36, 4), (30, 16), (64, 6)])
+def test_keys_without_a_page_are_not_seen(hd, page):
+    """An entry of -1 in the block table, and a table that ends before the step's keys do: in both forms, as in the kernels of
+    the other attentions."""
+    from pyre_amd.hip import ops
+
+    nq, nkv, T = 4, 2, 70
+    pages = -(-T // page)
+    k, v, q = rnd(T, nkv, hd, seed=1), rnd(T, nkv, hd, seed=2), rnd(T, nq, hd, seed=3)
+    kc, vc = torch.zeros(pages, nkv, page, hd, device=DEV), torch.zeros(pages, nkv, hd, page, device=DEV)
+    for t in range(T):
+        kc[t // page, :, t % page] = k[t]
+        vc[t // page, :, :, t % page] = v[t]
+    pos, seq = torch.arange(T, dtype=torch.int32, device=DEV), torch.zeros(T, dtype=torch.int32, device=DEV)
+    tiles = torch.tensor([[t, min(32, T - t)] for t in range(0, T, 32)], dtype=torch.int32, device=DEV)
+    i, j = torch.arange(T, device=DEV)[:, None], torch.arange(T, device=DEV)[None]
+    for gone, width in ((2, pages), (pages - 1, pages), (None, pages - 1)):
+        table = torch.arange(width, dtype=torch.int32, device=DEV)[None].clone()
+        if gone is not None:
+            table[0, gone] = -1
+        lost = (j // page == gone) if gone is not None else (j // page >= width)
+        out = torch.full((T, nq, hd), float("nan"), device=DEV)
+        ops.attn_prefill_f32(q, out, kc, vc, tiles, len(tiles), pos, seq, table.contiguous(), nq, nkv, hd, page, hd ** -0.5, 0)
+        for h in range(nq):
+            s = (q[:, h].double() @ k[:, h // 2].double().T * hd ** -0.5).masked_fill((j > i) | lost, float("-inf"))
+            want = torch.softmax(s, 1) @ v[:, h // 2].double()
+            assert float((out[:, h].double() - want).abs().max()) <= 2e-5, (gone, width)
+
+
 @pytest.mark.parametrize("n,k,ks", [(130, 1520, 2), (1536, 1104, 3), (200, 8960, 16), (48, 80, 3), (300, 640, 40)])
 def test_parts_added_where_they_are_made(n, k, ks):
     """The same bits as the parts added up in their order (parts that end with half a slot, a last part shorter than the
