@@ -403,10 +403,14 @@ extern "C" int pyre_gemm_tile_parts(int M, int N, int K) {
   return choose(kSums, sizeof(kSums) / sizeof(kSums[0]), false, M, N, K, 0).parts;
 }
 
-extern "C" int pyre_gemm_tile_launches(int M, int N, int K, int gated) {
-  const TileChoice c = gated ? choose(kUnits, sizeof(kUnits) / sizeof(kUnits[0]), true, M, N, K, 0)
-                             : choose(kSums, sizeof(kSums) / sizeof(kSums[0]), false, M, N, K, 0);
-  return c.cut ? 2 : 1;
+extern "C" int pyre_gemm_tile_choice(int M, int N, int K, int gated, int parts, int* tiles) {
+  const TileCost* costs = gated ? kUnits : kSums;
+  const int n = gated ? sizeof(kUnits) / sizeof(kUnits[0]) : sizeof(kSums) / sizeof(kSums[0]);
+  const TileChoice c = choose(costs, n, gated, M, N, K, parts);
+  PYRE_REQUIRE(c.us < 1e30, "gemm_tile_choice: K=%d cannot be taken in %d parts", K, parts);
+  const int says[6] = {costs[c.cfg].bm, costs[c.cfg].bn, c.cut, c.by_rows, c.cut ? costs[c.rest].bm : 0, c.cut ? costs[c.rest].bn : 0};
+  for (int i = 0; i < 6; ++i) tiles[i] = says[i];
+  return 0;
 }
 
 // out: float32 [parts][M][N].

@@ -102,8 +102,10 @@ int pyre_gemm_mid_silu_bf16(const void* X, long ldx, const void* W, long ldw, vo
 // out bfloat16 [M][two_i / 2]. N (two_i) a multiple of 16, K of 64.
 int pyre_gemm_tile_supports(int M, int N, int K, long ldx, long ldw);
 int pyre_gemm_tile_parts(int M, int N, int K);
-// Launches of the product (gated: N = gate and up rows): 2 where a region of smaller tiles makes what would be a nearly empty round.
-int pyre_gemm_tile_launches(int M, int N, int K, int gated);
+// How the product (gated: N = gate and up rows) in `parts` parts (0: as many as pyre_gemm_tile_parts says) is made: tiles[0..5] =
+// rows of X and of W of a tile; if [2] is not 0, tiles of [4] x [5] in a launch of their own make what lies behind the first [2] rows
+// of X ([3] = 1) or of the result's columns ([3] = 0).
+int pyre_gemm_tile_choice(int M, int N, int K, int gated, int parts, int* tiles);
 int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long ldw, float* out, int M, int N, int K, int parts,
                         hipStream_t stream);
 int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, long ldw, void* out, int M, int two_i, int K, float limit,

@@ -57,7 +57,7 @@ _SIGNATURES = {
     "pyre_gemm_f32_adds": [I, I, I, L, L, I],
     "pyre_gemm_f32_whole": [P, L, P, L, P, L, I, I, I, I, P],
     "pyre_gemm_tile_supports": [I, I, I, L, L],
-    "pyre_gemm_tile_launches": [I, I, I, I],
+    "pyre_gemm_tile_choice": [I, I, I, I, I, P],
     "pyre_gemm_tile_parts": [I, I, I],
     "pyre_gemm_tile_bf16": [P, L, P, L, P, I, I, I, I, P],
     "pyre_gemm_tile_glu_bf16": [P, L, P, L, P, I, I, I, F, F, F, F, P],

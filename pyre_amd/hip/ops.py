@@ -1071,6 +1071,17 @@ def gemm_tile_parts(m: int, n: int, k: int) -> int:
     return int(lib().pyre_gemm_tile_parts(m, n, k))
 
 
+def gemm_tile_choice(m: int, n: int, k: int, gated: bool, parts: int = 0) -> tuple[tuple[int, int], int, bool, tuple[int, int]]:
+    """How such a product is made: its tiles (rows of x, rows of w), and where it is cut in two launches, the rows (or columns of
+    the result) of the first, whether they are rows, and the tiles of the second; (.., 0, False, (0, 0)) for one launch."""
+    from ctypes import addressof, c_int
+
+    says = (c_int * 6)()
+    call("pyre_gemm_tile_choice", m, n, k, int(gated), parts, addressof(says))
+    bm, bn, cut, by_rows, rest_m, rest_n = says
+    return (bm, bn), cut, bool(by_rows), (rest_m, rest_n)
+
+
 def gemm_tile_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, parts: int) -> None:
     """out[s] (float32 [parts, m, N]) = partial sums over k of x[0:m] @ w.T, in tiles of up to 256 x 256;
     ``parts`` as :func:`gemm_tile_parts` says (or another number that leaves every part 256 k)."""

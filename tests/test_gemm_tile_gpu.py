@@ -4,6 +4,10 @@ products."""
 
 from __future__ import annotations
 
+import functools
+import math
+import random
+
 import pytest
 import torch
 
@@ -37,19 +41,122 @@ def test_sums(m, n, k):
         assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * float(want.std()) * 4, parts
 
 
-@pytest.mark.parametrize("m,n,k,bm,bn", [(3000, 3584, 1536, 256, 256), (2048, 5560 // 16 * 16, 512, 256, 192), (500, 2064, 1024, 128, 192),
-                                         (260, 4608, 640, 128, 128), (70, 4624, 1024, 64, 128)])
-def test_every_tile_size(m, n, k, bm, bn):
-    """Sizes that fill one round of each tile size, one row and sixteen columns past it."""
+@pytest.mark.parametrize("m,n,k,rows", [(3000, 3584, 1536, 256), (2048, 5552, 512, 256), (500, 2064, 1024, 128), (260, 4608, 640, 128),
+                                        (70, 4624, 1024, 64)])
+def test_larger_sums(m, n, k, rows):
+    """Sizes of about one round, and a row more than whole tiles."""
     from pyre_amd.hip import ops
 
-    for mm in (m, m // bm * bm + 1):
+    for mm in (m, m // rows * rows + 1):
         x, w = rnd(mm, k + 24, seed=1)[:, 8:k + 8], rnd(n, k + 8, seed=2)[:, :k]   # rows 48 and 16 bytes apart
         parts = ops.gemm_tile_parts(mm, n, k)
         out = torch.full((parts, mm, n), float("nan"), device=DEV)
         ops.gemm_tile_bf16(x, w, out, mm, parts)
         want = x.double() @ w.double().T
         assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * float(want.std()) * 4
+
+
+#: the forms of the kernel: rows of x and of w of a tile, and the stages of 64 k that its ring holds
+SUMS = {(256, 256): 2, (256, 192): 2, (128, 192): 3, (128, 128): 4, (64, 128): 6}
+UNITS = {(256, 256): 2, (192, 256): 2, (192, 192): 2, (128, 256): 3, (96, 256): 3, (96, 192): 3}
+CASES = ("whole tiles", "a row more", "columns past the end", "fewer stages than slots", "an edge before a whole tile")
+
+
+def walks_from_an_edge(m, n, parts, bm, bn, units):
+    """Whether some block takes a whole tile after one that ends past the matrix (the kernel's order of tiles)."""
+    mt, nt = -(-m // bm), -(-n // bn)
+    tiles, blocks = mt * nt * parts, min(units, mt * nt * parts)
+
+    def whole(t):
+        t %= mt * nt
+        first = t // (8 * nt) * 8
+        t, gm = t - first * nt, min(8, mt - first)
+        return (first + t % gm + 1) * bm <= m and (t // gm + 1) * bn <= n
+
+    for die in range(min(8, blocks)):
+        begin = die * (tiles // 8) + min(die, tiles % 8)
+        end, step = begin + tiles // 8 + (die < tiles % 8), (blocks - die + 7) // 8
+        if any(not whole(t) and whole(t + step) for t in range(begin, end - step)):
+            return True
+    return False
+
+
+@functools.lru_cache(maxsize=None)
+def sizes_of_every_form(gated: bool):
+    """For every form and case the smallest size of many that the planner gives to it: {(tile, case): (m, n, k)}, in one launch;
+    {("first" or "rest", tile): (m, n, k)} of those that it cuts."""
+    from pyre_amd.hip import ops
+
+    forms, units = UNITS if gated else SUMS, ops.compute_units()
+    rng, found = random.Random(5), {}
+
+    def note(key, size):
+        if key not in found or math.prod(size) < math.prod(found[key]):
+            found[key] = size
+
+    for i in range(40000):
+        bm, bn = list(forms)[i % len(forms)]
+        m, n, k = rng.randint(1, 3000), 16 * rng.randint(1, 1600), 64 * rng.choice([1, 2, 3, 4, 5, 7, 16, 24, 40])
+        if i % 3 == 1:
+            m, n = -(-m // bm) * bm, -(-n // bn) * bn
+        elif i % 3 == 2:
+            m = m // bm * bm + 1
+        if m * n > 4e7:
+            continue
+        tile, cut, _, rest = ops.gemm_tile_choice(m, n, k, gated)
+        if cut:
+            note(("first", tile), (m, n, k))
+            note(("rest", rest), (m, n, k))
+            continue
+        parts = 1 if gated else ops.gemm_tile_parts(m, n, k)
+        per = -(-(-(-k // parts)) // 64)
+        is_so = (m % tile[0] == 0 and n % tile[1] == 0, m % tile[0] == 1, n % tile[1] != 0, per < forms[tile],
+                 m % tile[0] and n % tile[1] and walks_from_an_edge(m, n, parts, *tile, units))
+        for case, so in zip(CASES, is_so):
+            if so:
+                note((tile, case), (m, n, k))
+    return found
+
+
+def check_product(m, n, k, gated, tile, rest=None):
+    """A product whose rows lie 16 and 48 bytes further apart than they are long, made by the tiles that are named."""
+    from pyre_amd.hip import ops
+
+    says, cut, _, then = ops.gemm_tile_choice(m, n, k, gated)
+    assert (says == tile or tile is None) and (bool(cut), then) == ((False, (0, 0)) if rest is None else (True, rest))
+    x, w = rnd(m, k + 24, seed=1)[:, 8:k + 8], rnd(n, k + 8, seed=2, scale=0.2 if gated else 1.0)[:, :k]
+    want = x.double() @ w.double().T
+    if gated:
+        out = torch.full((m, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops.gemm_tile_glu_bf16(x, w, out, m)
+        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
+        # half a unit of the 8 bits that bfloat16 keeps, and the sums' rounding through factors that grow with the sums
+        assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 64 * bound(k)).all())
+    else:
+        parts = ops.gemm_tile_parts(m, n, k)
+        out = torch.full((parts, m, n), float("nan"), device=DEV)
+        ops.gemm_tile_bf16(x, w, out, m, parts)
+        assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * max(1.0, k ** 0.5) * 4
+
+
+#: what the planner gives to no form: its smallest tiles are for products of one round, some of them for longer k only
+NEVER = {(False, (64, 128), CASES[4]), (True, (96, 192), CASES[4]), (False, (128, 192), CASES[3]), (True, (192, 192), CASES[3]),
+         (True, (96, 256), CASES[3]), (True, (96, 192), CASES[3])}
+
+
+@pytest.mark.parametrize("gated,tile,case", [(g, t, c) for g, forms in ((False, SUMS), (True, UNITS)) for t in forms for c in CASES
+                                             if (g, t, c) not in NEVER])
+def test_every_form(gated, tile, case):
+    """Every form of the kernel at the edges of its tiles, rounds and ring, at sizes that the planner gives to it."""
+    check_product(*sizes_of_every_form(gated)[tile, case], gated, tile)
+
+
+@pytest.mark.parametrize("gated,tile", [(False, (256, 192)), (False, (128, 192)), (False, (128, 128)), (False, (64, 128)),
+                                        (True, (256, 256)), (True, (192, 256)), (True, (192, 192)),
+                                        (True, (128, 256)), (True, (96, 256)), (True, (96, 192))])
+def test_every_form_behind_a_cut(gated, tile):
+    size = sizes_of_every_form(gated)["rest", tile]
+    check_product(*size, gated, None, tile)
 
 
 @pytest.mark.parametrize("unit", [None, (7.0, 1.702, 1.0), (0.0, float("inf"), 0.0, 0.0)])
@@ -124,23 +231,13 @@ def test_a_step_against_the_librarys_products(n):
     assert float(((rows[0] - rows[1]).abs().amax(1) / scale).max()) <= 2e-2
 
 
-@pytest.mark.parametrize("m,n,k,gated", [(1777, 37904, 1024, True), (2101, 17936, 1536, True), (5501, 3600, 2048, True), (2101, 9040, 2048, False),
-                                         (4501, 3600, 2048, False), (7501, 2064, 2048, False)])
-def test_a_last_round_in_smaller_tiles(m, n, k, gated):
+@pytest.mark.parametrize("m,n,k,gated,by_rows", [(1777, 37904, 1024, True, False), (2101, 17936, 1536, True, False),
+                                                 (5501, 3600, 2048, True, True), (2101, 9040, 2048, False, False),
+                                                 (4501, 3600, 2048, False, False), (7501, 2064, 2048, False, True)])
+def test_a_last_round_in_smaller_tiles(m, n, k, gated, by_rows):
     """Products cut in two launches, along the rows of either operand: every element is the product of its own rows."""
     from pyre_amd.hip import ops
-    from pyre_amd.hip.lib import lib
 
-    assert lib().pyre_gemm_tile_launches(m, n, k, int(gated)) == 2
-    x, w = rnd(m, k + 8, seed=8)[:, :k], rnd(n, k + 8, seed=9, scale=0.2)[:, :k]
-    want = x.double() @ w.double().T
-    if gated:
-        out = torch.full((m, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
-        ops.gemm_tile_glu_bf16(x, w, out, m)
-        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
-        assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 64 * bound(k)).all())
-    else:
-        parts = ops.gemm_tile_parts(m, n, k)
-        out = torch.full((parts, m, n), float("nan"), device=DEV)
-        ops.gemm_tile_bf16(x, w, out, m, parts)
-        assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * float(want.std()) * 4
+    _, cut, rows, rest = ops.gemm_tile_choice(m, n, k, gated)
+    assert cut and rows == by_rows
+    check_product(m, n, k, gated, None, rest)
