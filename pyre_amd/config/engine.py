@@ -28,7 +28,8 @@ class EngineConfig:
     max_model_len: int | None = None  #: longest request; None: the model's max positions
     use_graphs: bool = True          #: capture decode-only steps in HIP graphs
     #: row counts (tokens in a step) for which the BLAS library is asked, once at start-up,
-    #: to time its kernels for this model's many-row 16-bit products and keep the fastest
+    #: to time its kernels for those of this model's many-row 16-bit products that are left to it
+    #: and keep the fastest
     tune_gemm_rows: tuple = ()
     #: debugging aid: fill every cache page and state slot with NaN when it goes back to its
     #: pool (and all of them at the start), so that a read of freed memory shows in the logits

@@ -127,19 +127,18 @@ class Engine:
     def tune_library_gemms(self, rows) -> int:
         """For steps of exactly ``rows`` tokens (any of them), let the BLAS front end
         time the vendor libraries' kernels for each distinct many-row 16-bit product of
-        this model and remember the fastest (torch's TunableOp). Other row counts keep
-        the libraries' own choice. Returns the number of products tuned."""
+        this model that is left to them (:func:`pyre_amd.parts.fast.library_takes`: of the
+        shapes that the framework's own kernels take none) and remember the fastest (torch's
+        TunableOp). Other row counts keep the libraries' own choice, and so do the head's
+        float32 logits. Returns the number of products tuned."""
         import os
         import tempfile
 
         import torch.cuda.tunable as tunable
 
-        from pyre_amd.parts.fast import SKINNY_MAX_ROWS
+        from pyre_amd.parts.fast import SKINNY_MAX_ROWS, library_takes
 
-        shapes = {}
-        for lin in self.model.linears():
-            if lin.weight is not None and lin.weight.dtype == torch.bfloat16:
-                shapes.setdefault((lin.out_features, lin.in_features), lin)
+        linears = [lin for lin in self.model.linears() if lin.weight is not None and lin.weight.dtype == torch.bfloat16]
         tunable.enable(True)
         if hasattr(tunable, "write_file_on_exit"):
             tunable.write_file_on_exit(False)
@@ -151,9 +150,9 @@ class Engine:
         try:
             with torch.cuda.device(self.device):
                 for m in sorted({int(r) for r in rows if int(r) > SKINNY_MAX_ROWS}):
+                    shapes = {(lin.out_features, lin.in_features): lin for lin in linears
+                              if lin.out_features != self.vocab_size and library_takes(lin, self.runtime, m)}
                     for (n_out, k), lin in shapes.items():
-                        if n_out == self.vocab_size:
-                            continue  # the head's float32 logits do not go through the library
                         x = torch.zeros(m, k, device=self.device, dtype=torch.bfloat16)
                         out = torch.empty(m, n_out, device=self.device, dtype=torch.bfloat16)
                         torch.mm(x, lin.weight.t(), out=out)

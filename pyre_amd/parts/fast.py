@@ -115,6 +115,13 @@ def takes_tiles(rt, n: int, n_out: int, k: int, ldx: int, ldw: int) -> bool:
     return bool(rt.options.get("tile_gemm", True)) and n > SKINNY_MAX_ROWS and ops.gemm_tile_supports(n, n_out, k, ldx, ldw)
 
 
+def library_takes(lin, rt, n: int) -> bool:
+    """Whether the 16-bit product of ``n`` rows (more than the weight-streaming kernel's) and this weight is left to the BLAS
+    library once no kernel for few rows takes it."""
+    by_tiles = lin.role in TILE_ROLES or (lin.role == "ffn.gate_up" and lin.bias is None)
+    return not (by_tiles and takes_tiles(rt, n, lin.out_features, lin.in_features, lin.in_features, lin.weight.stride(0)))
+
+
 def _is_bf16(ctx, lin, x) -> bool:
     return (ctx.runtime.dtype == torch.bfloat16 and lin.weight.dtype == torch.bfloat16
             and x.dtype == torch.bfloat16)

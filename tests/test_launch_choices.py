@@ -5,6 +5,7 @@ than it takes."""
 import random
 
 import numpy as np
+import pytest
 
 from pyre_amd.parts.attention_work import (DECODE_MAX_BLOCKS_PER_REQUEST, DEFAULT_UNITS, decode_alone, decode_capacity,
                                            decode_work, prefill_slots, prefill_work)
@@ -244,3 +245,24 @@ def test_which_kernel_takes_a_product_is_a_function_of_its_sizes():
     for shape in (qkv7, down7, (3584, 3584), (2048, 1536), (1536, 8960), (7168, 5120), (5120, 27648), (96, 64), (1000, 4096)):
         for lo, hi in zip(edges, edges[1:]):
             assert len({narrow_kernel(n, *shape) for n in range(lo + 1, hi + 1)}) == 1, (shape, lo, hi)
+
+
+@pytest.mark.parametrize("role,bias,k,left", [("attn.qkv", True, 1536, False), ("ffn.down", False, 8960, False), ("ffn.gate_up", False, 1536, False),
+                                              ("ffn.gate_up", True, 1536, True), ("moe.up", False, 1536, True), ("attn.out", False, 1000, True)])
+def test_what_is_left_to_the_library(role, bias, k, left):
+    """Tuning the library's kernels is for the products that it makes: not for those of the kernel of tiles (k a multiple of 64)."""
+    import torch
+
+    from pyre_amd.parts.fast import library_takes
+
+    class Lin:
+        out_features, in_features, weight = 2048, k, torch.empty(2048, k, dtype=torch.bfloat16, device="meta")
+
+    Lin.role, Lin.bias = role, torch.empty(2048) if bias else None
+
+    class Rt:
+        options = {}
+
+    assert library_takes(Lin, Rt, 2048) is left
+    Rt.options = {"tile_gemm": False}
+    assert library_takes(Lin, Rt, 2048)
