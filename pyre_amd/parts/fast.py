@@ -105,11 +105,17 @@ TILE_ROLES = LIBRARY_F32_ROLES | {"ffn.down"}
 
 def takes_tiles(rt, n: int, n_out: int, k: int, ldx: int, ldw: int) -> bool:
     """Whether a 16-bit product of ``n`` rows goes to the kernel of tiles of up to 256 x 256 (`gemm_tile.hip`): all of more
-    rows than the weight-streaming kernel takes whose sizes it supports. Against the BLAS library's products (weights from
-    memory, in us): the 7B shape's way down 171 against 253 at 1,500 rows, 227 against 353 at 2,048;
-    q/k/v 27 against 39 at 566, 52 against 58 at 1,500, 75 against 68 at 2,048; gate/up with the SiLU-gate 464 against
-    508 + 37 at 2,048, 157 against 137 + 11 at 566; the 1.5B shape's way down 25 against 46 at 566, 58 against 83 at 2,109,
-    gate/up 118 against 114 + 17 at 2,109. The few sizes at which one product is slower have others that gain more."""
+    rows than the weight-streaming kernel takes whose sizes it supports. Against the BLAS library's products (us here and there,
+    weights from memory, the gated unit and the reading of partial sums with them): the 7B shape's way down 107 and 141 at 566
+    rows, 241 and 360 at 2,048, 469 and 537 at 4,096, 936 and 880 at 8,192; its gate/up 156 and 153, 454 and 550, 888 and 868,
+    1,717 and 1,780; the 1.5B shape's way down 26 and 31 at 566, 60 and 67 at 2,048, 107 and 103 at 4,096; its gate/up 38 and 43,
+    109 and 138, 200 and 225; the 32B shape's way down 190 and 246, 496 and 447, 1,037 and 897, at 8,192 1,932 and 2,289.
+    Where the line could be drawn otherwise: q/k/v and attention output are ahead up to about 1,000 rows (7B: 28 and 33, 26 and
+    25 at 566) and behind from there on (71 and 65, 58 and 51 at 2,048; 128 and 123, 94 and 89 at 4,096; worst the 1.5B shape's
+    q/k/v, 32 and 25 at 3,000). All products of a layer together are 824 and 1,024 us for 2,048 rows of the 7B shape, 1,578 and
+    1,618 for 4,096, 3,070 and 3,047 for 8,192; 206 and 247, 367 and 383, 651 and 690 of the 1.5B shape; 1,654 and 1,729, 3,276
+    and 3,216, 6,286 and 6,804 of the 32B shape (at 3,000 rows 2,409 and 2,297: 1.23 PFLOP/s in its way down where the library
+    has 1.48)."""
     from pyre_amd.hip import ops
 
     return bool(rt.options.get("tile_gemm", True)) and n > SKINNY_MAX_ROWS and ops.gemm_tile_supports(n, n_out, k, ldx, ldw)
