@@ -175,14 +175,40 @@ struct ChunkScratch {
   float* ends;   // per segment [head][tile of 16 columns][2][DT][lane][4]: the state at its end; its decays, or of a request's
                  // first segment the state before it
 };
+
+// A segment of a request. How a request is cut follows from its own tokens and `most`, the most segments that a model of these
+// heads is given: the state is summed segment by segment, so a request's bits are the same whatever else is in the step.
+struct Segment {
+  int s, slot;       // the request (-1: nothing to do), its place among the states
+  int seg;           // which of its segments
+  int first, last;   // the segment's tokens
+  int t_begin, per;  // the request's first token, the chunks of its segments
+  int ends;          // it is the request's last
+};
 // A segment is kSegment chunks at least, so token t0, with which one begins that is not a request's last, has a place of its
 // own at t0 / (16 kSegment).
 constexpr int kSegment = 4;
+constexpr int kUncut = 8;  // a request of up to so many chunks is one segment
+constexpr int kSegmentShift = 6, kNoShift = 30;
+static_assert(1 << kSegmentShift == kChunk * kSegment, "a place for every segment");
+// The grid of the walk is a list of places. A request has one for every kSegment chunks (2^shift tokens) and one more, which is
+// what it can be cut into at most; where no request of the step is cut, one (a shift that leaves nothing of a token's number); a
+// request alone has as many as it may have segments. (With as many for every request as for the longest, 60 single tokens beside
+// a prompt of nine segments would be 480 empty blocks a head and tile, each of which holds a SIMD's registers for a microsecond.)
+__host__ __device__ inline int segment_place(int t_begin, int s, int shift) { return (t_begin >> shift) + s; }
+struct Places {
+  Segment* list;
+  const int* state_slots;
+  int n, n_seqs, most, shift;
+};
 __host__ __device__ inline size_t chunk_scratch_floats(size_t slots, int heads, int dkp, int dvp) {
   return (slots * heads * (2 * static_cast<size_t>(dkp) + dvp + 2 * kChunk) + 3) / 4 * 4;
 }
 __host__ __device__ inline size_t ends_floats(size_t n_tokens, int heads, int dkp, int dv) {
   return (n_tokens / (kChunk * kSegment) + 1) * heads * ((dv + 15) / 16) * 2 * (dkp / 16) * kWave * 4;
+}
+__host__ __device__ inline size_t places_floats(size_t n_tokens, size_t n_seqs) {
+  return (n_tokens / (kChunk * kSegment) + n_seqs + kMaxSegments) * (sizeof(Segment) / sizeof(float));
 }
 __host__ __device__ inline ChunkScratch carve(float* base, size_t slots, int heads, int dkp, int dvp) {
   ChunkScratch c;
@@ -195,8 +221,21 @@ __host__ __device__ inline ChunkScratch carve(float* base, size_t slots, int hea
   return c;
 }
 
+// What the places of request s have to do, by one block of the kernels that prepare the chunks.
+__device__ inline void lay_places(const Places& p, const int* __restrict__ q_start, int s) {
+  const int t_begin = q_start[s], t_end = q_start[s + 1], chunks = (t_end - t_begin + kChunk - 1) / kChunk;
+  const int per = p.shift == kNoShift || chunks <= kUncut ? max(chunks, 1) : max(kSegment, (chunks + p.most - 1) / p.most);
+  const int count = (chunks + per - 1) / per, from = p.n_seqs == 1 ? 0 : segment_place(t_begin, s, p.shift);
+  const int to = s + 1 < p.n_seqs ? segment_place(t_end, s + 1, p.shift) : p.n;
+  for (int z = (s ? from : 0) + threadIdx.x; z < to; z += kThreads) {
+    const bool there = z >= from && z - from < count;
+    const int seg = there ? z - from : 0, first = t_begin + seg * per * kChunk, last = min(t_end, first + per * kChunk);
+    p.list[z] = Segment{there ? s : -1, p.state_slots[s], seg, first, last, t_begin, per, last == t_end};
+  }
+}
+
 __global__ __launch_bounds__(kThreads) void gla_chunk_prep_kernel(
-    const float* __restrict__ x, ChunkScratch sc, const int* __restrict__ q_start, int heads, int dk, int dv, int dkp,
+    const float* __restrict__ x, ChunkScratch sc, Places places, const int* __restrict__ q_start, int heads, int dk, int dv, int dkp,
     int dvp) {
   extern __shared__ float prep_lds[];
   float* qs = prep_lds;
@@ -204,6 +243,7 @@ __global__ __launch_bounds__(kThreads) void gla_chunk_prep_kernel(
   float* bs = ks + kChunk * dk;
   const int s = blockIdx.z, hd = blockIdx.y, tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int t0 = q_start[s] + blockIdx.x * kChunk, t_end = q_start[s + 1];
+  if (blockIdx.x == 0 && hd == 0) lay_places(places, q_start, s);
   if (t0 >= t_end) return;
   const int nc = min(kChunk, t_end - t0);
   const size_t slot0 = static_cast<size_t>(t0) + kChunk * s;
@@ -254,7 +294,7 @@ __global__ __launch_bounds__(kThreads) void gla_chunk_prep_kernel(
 // each of 120 pairs, and its pairs are plain products of rows in LDS. Values cross LDS on their way to [column][token].
 // 79 -> 33 us for 1,777 tokens of 14 heads of 128 x 128, 32 -> 12 for 300 tokens of six (a chain of 64 sums over a wave).
 __global__ __launch_bounds__(kThreads) void gla_chunk_prep_vec_kernel(
-    const float* __restrict__ x, ChunkScratch sc, const int* __restrict__ q_start, int heads, int dk, int dv, int dkp,
+    const float* __restrict__ x, ChunkScratch sc, Places places, const int* __restrict__ q_start, int heads, int dk, int dv, int dkp,
     int dvp) {
   extern __shared__ __attribute__((aligned(16))) float prep_lds[];
   const int ld = dk + 4;  // rows on distinct banks
@@ -264,6 +304,7 @@ __global__ __launch_bounds__(kThreads) void gla_chunk_prep_vec_kernel(
   float* f = bs + kChunk * ld;
   const int s = blockIdx.z, hd = blockIdx.y, tid = threadIdx.x;
   const int t0 = q_start[s] + blockIdx.x * kChunk, t_end = q_start[s + 1];
+  if (blockIdx.x == 0 && hd == 0) lay_places(places, q_start, s);
   if (t0 >= t_end) return;
   const int nc = min(kChunk, t_end - t0);
   const size_t slot0 = static_cast<size_t>(t0) + kChunk * s;
@@ -442,12 +483,20 @@ __device__ inline void take_on(const ChunkOperands<DT>& now, f32x4 (&S)[DT]) {
 // The state's rows and columns of a lane.
 template <int DT>
 __device__ inline void load_state(const float* st, int dk, int dv, int col, int g, f32x4 (&S)[DT]) {
+  const float* const column = st + min(col, dv - 1);  // columns past the last are the last one once more
+  if (dk == 16 * DT) {  // no load under a condition: all of them on their way at once
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[j][i] = column[static_cast<size_t>(16 * j + 4 * g + i) * dv];
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < DT; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = 16 * j + 4 * g + i;
-      S[j][i] = col < dv && row < dk ? st[static_cast<size_t>(row) * dv + col] : 0.f;
+      S[j][i] = row < dk ? column[static_cast<size_t>(row) * dv] : 0.f;
     }
 }
 
@@ -458,63 +507,16 @@ __device__ inline f32x4* segment_end(const ChunkScratch& sc, int t0, int hd, int
          ((static_cast<size_t>(t0 / (kChunk * kSegment)) * heads + hd) * tiles + tile) * 2 * DT * kWave + lane;
 }
 
-// A segment of a request. How a request is cut follows from its own tokens and `most`, the most segments that a model of these
-// heads is given: the state is summed segment by segment, so a request's bits are the same whatever else is in the step.
-struct Segment {
-  int s, slot;       // the request, its place among the states
-  int seg;           // which of its segments
-  int first, last;   // the segment's tokens
-  int t_begin, per;  // the request's first token, the chunks of its segments
-  bool ends;         // it is the request's last
-};
-// What place z of the grid has to do, found by a wave, a lane a request; false: nothing. A request has a place for every kSegment
-// chunks (2^shift tokens) and one more, which is what it can be cut into at most; where no request of the step is cut, one (a shift
-// that leaves nothing of a token's number); a request alone has all places. (With as many places for every request as for the
-// longest, 60 single tokens beside a prompt of nine segments would be 480 empty blocks a head and tile, each of which holds a
-// SIMD's registers for a microsecond.)
-constexpr int kUncut = 8;  // a request of up to so many chunks is one segment
-constexpr int kSegmentShift = 6, kNoShift = 30;
-static_assert(1 << kSegmentShift == kChunk * kSegment, "a place for every segment");
-__host__ __device__ inline int segment_place(int t_begin, int s, int shift) { return (t_begin >> shift) + s; }
-
-__device__ inline bool find_segment(const int* __restrict__ q_start, const int* __restrict__ state_slots, int n_seqs,
-                                    int most, int shift, int z, Segment& r) {
-  const int lane = threadIdx.x & (kWave - 1);
-  r.s = n_seqs == 1 ? 0 : z;
-  if (n_seqs > 1 && shift != kNoShift) {
-    int s = -1;  // the last request whose places begin at z or before
-    for (int s0 = 0; s0 < n_seqs; s0 += kWave) {
-      const int i = s0 + lane;
-      const int hits = __popcll(__ballot(i < n_seqs && segment_place(q_start[min(i, n_seqs)], i, shift) <= z));
-      s += hits;
-      if (hits < kWave) break;
-    }
-    if (s < 0) return false;
-    r.s = __builtin_amdgcn_readfirstlane(s);
-  }
-  r.t_begin = q_start[r.s];
-  r.slot = state_slots[r.s];
-  const int t_end = q_start[r.s + 1], chunks = (t_end - r.t_begin + kChunk - 1) / kChunk;
-  r.per = shift == kNoShift || chunks <= kUncut ? max(chunks, 1) : max(kSegment, (chunks + most - 1) / most);
-  r.seg = n_seqs == 1 ? z : z - segment_place(r.t_begin, r.s, shift);
-  r.first = r.t_begin + r.seg * r.per * kChunk;
-  r.last = min(t_end, r.first + r.per * kChunk);
-  r.ends = r.last == t_end;
-  return r.first < t_end;
-}
-
-// grid: (heads, tiles of columns, places from `z0` on, see find_segment) in both kernels. The blocks of one request lie together in the grid
+// grid: (heads, tiles of columns, places, see segment_place) in both kernels. The blocks of one request lie together in the grid
 // and not those of one head: neighbours go to different dies, and a long prompt beside many single tokens is then not one die's
 // alone. Heads are padded to a multiple of eight, so that the blocks of a head, which read the same operands, share a die and
 // its cache.
 template <int DT>
-__global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, const float* __restrict__ state,
-                                                               const int* __restrict__ q_start,
-                                                               const int* __restrict__ state_slots, int heads, int dk, int dv,
-                                                               int dvp, int n_seqs, int most, int shift, int z0) {
+__global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, const Segment* __restrict__ places,
+                                                               const float* __restrict__ state, int heads, int dk, int dv, int dvp) {
   const int hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  Segment sg;
-  if (hd >= heads || !find_segment(q_start, state_slots, n_seqs, most, shift, z0 + blockIdx.z, sg) || sg.ends) return;
+  const Segment sg = places[blockIdx.z];
+  if (hd >= heads || sg.s < 0 || sg.ends) return;
   const int s = sg.s, seg = sg.seg, first = sg.first, last = sg.last;
   const int col = blockIdx.y * 16 + c;
   f32x4 S[DT], D[DT];
@@ -552,25 +554,29 @@ __global__ __launch_bounds__(kWave) void gla_chunk_ends_kernel(ChunkScratch sc, 
 
 template <int DT>
 __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
-    ChunkScratch sc, float* __restrict__ state, float* __restrict__ o, const int* __restrict__ q_start,
-    const int* __restrict__ state_slots, int heads, int dk, int dv, int dvp, float qscale, int n_seqs, int most, int shift, int z0) {
+    ChunkScratch sc, const Segment* __restrict__ places, float* __restrict__ state, float* __restrict__ o, int heads, int dk, int dv,
+    int dvp, float qscale) {
   const int hd = blockIdx.x, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
-  Segment sg;
-  if (hd >= heads || !find_segment(q_start, state_slots, n_seqs, most, shift, z0 + blockIdx.z, sg)) return;
+  const Segment sg = places[blockIdx.z];
+  if (hd >= heads || sg.s < 0) return;
   const int s = sg.s, seg = sg.seg, first = sg.first, last = sg.last, t_begin = sg.t_begin, per = sg.per;
   const int col = blockIdx.y * 16 + c, hv = heads * dv;
   const bool has_col = col < dv;
   const auto fetch_q = [&](int t0, ChunkOperands<DT>& r) { fetch_queries<DT>(sc, t0, s, hd, heads, g, c, r); };
   const auto fetch_k = [&](int t0, ChunkOperands<DT>& r) { fetch_keys<DT>(sc, t0, s, hd, heads, col, dv, dvp, g, c, r); };
   ChunkSets<DT> sets;
-  // on their way while the state is formed: as many as there are registers for beside it
-  constexpr int early = DT <= 8 ? 1 : 0;
-  sets.begin(0, early, first, last, fetch_q, fetch_k);
   float* st = state + (static_cast<size_t>(sg.slot) * heads + hd) * dk * dv;
   f32x4 S[DT];
-  if (seg == 0 && sg.ends) {  // a request of one segment: its state is this wave's alone
+  if (seg == 0 && sg.ends) {
+    // A request of one segment: its state is this wave's alone. All loads are on their way before one is waited for (with the first
+    // set before the branch, the registers that its two sides share made the state's loads wait: 64 requests of 33 tokens on 28
+    // heads of 128 x 128 walked 244 us instead of 196).
     load_state<DT>(st, dk, dv, col, g, S);
+    sets.begin(0, sets.N, first, last, fetch_q, fetch_k);
   } else {
+    // on their way while the state is formed: as many as there are registers for beside it
+    constexpr int early = DT <= 8 ? 1 : 0;
+    sets.begin(0, early, first, last, fetch_q, fetch_k);
     const f32x4* end = segment_end<DT>(sc, t_begin, hd, heads, blockIdx.y, gridDim.y, lane);
 #pragma unroll
     for (int j = 0; j < DT; ++j) S[j] = end[(seg == 0 ? DT + j : j) * kWave];
@@ -596,8 +602,8 @@ __global__ __launch_bounds__(kWave) void gla_chunk_walk_kernel(
       ask(b + 2, 0);
       add(b + 1, 1);
     }
+    sets.begin(early, sets.N, first, last, fetch_q, fetch_k);
   }
-  sets.begin(early, sets.N, first, last, fetch_q, fetch_k);
   const auto outputs = [&](int t0, const ChunkOperands<DT>& now) {
     const int nc = min(kChunk, last - t0);
     f32x4 out = {0.f, 0.f, 0.f, 0.f};
@@ -824,7 +830,7 @@ static int chunk_tiles(int dk) { return dk <= 32 ? 2 : dk <= 64 ? 4 : dk <= 128 
 extern "C" long pyre_gla_chunks_scratch(int n_tokens, int n_seqs, int heads, int dk, int dv) {
   const size_t slots = static_cast<size_t>(n_tokens) + static_cast<size_t>(kChunk) * n_seqs;
   return static_cast<long>(chunk_scratch_floats(slots, heads, 16 * chunk_tiles(dk), (dv + 3) / 4 * 4) +
-                           ends_floats(n_tokens, heads, 16 * chunk_tiles(dk), dv));
+                           ends_floats(n_tokens, heads, 16 * chunk_tiles(dk), dv) + places_floats(n_tokens, n_seqs));
 }
 
 extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, float* o, const int* q_start,
@@ -836,32 +842,33 @@ extern "C" int pyre_gla_chunks(const float* x, float* scratch, float* state, flo
   if (n_seqs <= 0 || max_tokens == 0) return 0;
   const int DTs = chunk_tiles(dk), dkp = 16 * DTs, dvp = (dv + 3) / 4 * 4;
   const ChunkScratch sc = carve(scratch, static_cast<size_t>(n_tokens) + static_cast<size_t>(kChunk) * n_seqs, heads, dkp, dvp);
-  const dim3 prep_grid((max_tokens + kChunk - 1) / kChunk, heads, n_seqs);
-  const size_t prep_bytes = sizeof(float) * 4 * kChunk * (dk + 4);
-  if (dk % 4 == 0 && dv % 4 == 0 && prep_bytes <= 65536 && reinterpret_cast<uintptr_t>(x) % 16 == 0)
-    hipLaunchKernelGGL(gla_chunk_prep_vec_kernel, prep_grid, dim3(kThreads), prep_bytes, stream, x, sc, q_start, heads, dk, dv, dkp, dvp);
-  else
-    hipLaunchKernelGGL(gla_chunk_prep_kernel, prep_grid, dim3(kThreads), sizeof(float) * 3 * kChunk * dk, stream, x, sc, q_start,
-                       heads, dk, dv, dkp, dvp);
-  if (check_launch("gla_chunk_prep")) return 1;
   // A request gets as many segments as put a wave on every SIMD when it is alone in the step, whatever else is in it (see Segment):
-  // six prompts of 300 tokens on 14 heads of 128 x 128 take 103 us that way and 139 without any. A segment costs its waves a walk
+  // six prompts of 300 tokens on 14 heads of 128 x 128 take 102 us that way and 139 without any. A segment costs its waves a walk
   // for its end and the reading of those before it, so it has four chunks at least, and eight are not cut: 16 requests of 100
-  // tokens 75 us, 99 in two segments each.
+  // tokens 73 us, about 97 in two segments each.
   const int chunks = (max_tokens + kChunk - 1) / kChunk, tiles = (dv + 15) / 16;
   const int most = std::max(1, std::min(kMaxSegments, 4 * compute_units() / (heads * tiles)));
   const bool cut = most > 1 && chunks > kUncut;  // some request may be
   const int shift = cut ? kSegmentShift : kNoShift;
-  const long places = n_seqs == 1 ? (cut ? most : 1) : segment_place(n_tokens, n_seqs, shift);
-#define PYRE_WALK_Z(KERNEL, ...)                                                                                       \
-  for (long z0 = 0; z0 < places; z0 += 65535)                                                                          \
-  hipLaunchKernelGGL(KERNEL, dim3((heads + 7) / 8 * 8, tiles, static_cast<unsigned>(std::min(65535L, places - z0))),   \
-                     dim3(kWave), 0, stream, __VA_ARGS__, n_seqs, most, shift, static_cast<int>(z0))
-#define PYRE_WALK(DT)                                                                                       \
-  do {                                                                                                      \
-    if (cut)                                                                                                \
-      PYRE_WALK_Z(gla_chunk_ends_kernel<DT>, sc, state, q_start, state_slots, heads, dk, dv, dvp);          \
-    PYRE_WALK_Z(gla_chunk_walk_kernel<DT>, sc, state, o, q_start, state_slots, heads, dk, dv, dvp, qscale); \
+  const Places places{reinterpret_cast<Segment*>(sc.ends + ends_floats(n_tokens, heads, dkp, dv)), state_slots,
+                      n_seqs == 1 ? (cut ? most : 1) : segment_place(n_tokens, n_seqs, shift), n_seqs, most, shift};
+  const dim3 prep_grid((max_tokens + kChunk - 1) / kChunk, heads, n_seqs);
+  const size_t prep_bytes = sizeof(float) * 4 * kChunk * (dk + 4);
+  if (dk % 4 == 0 && dv % 4 == 0 && prep_bytes <= 65536 && reinterpret_cast<uintptr_t>(x) % 16 == 0)
+    hipLaunchKernelGGL(gla_chunk_prep_vec_kernel, prep_grid, dim3(kThreads), prep_bytes, stream, x, sc, places, q_start, heads, dk,
+                       dv, dkp, dvp);
+  else
+    hipLaunchKernelGGL(gla_chunk_prep_kernel, prep_grid, dim3(kThreads), sizeof(float) * 3 * kChunk * dk, stream, x, sc, places,
+                       q_start, heads, dk, dv, dkp, dvp);
+  if (check_launch("gla_chunk_prep")) return 1;
+#define PYRE_WALK_Z(KERNEL, ...)                                                                                                  \
+  for (int z0 = 0; z0 < places.n; z0 += 65535)                                                                                    \
+  hipLaunchKernelGGL(KERNEL, dim3((heads + 7) / 8 * 8, tiles, std::min(65535, places.n - z0)), dim3(kWave), 0, stream, sc,         \
+                     places.list + z0, __VA_ARGS__)
+#define PYRE_WALK(DT)                                                                                        \
+  do {                                                                                                       \
+    if (cut) PYRE_WALK_Z(gla_chunk_ends_kernel<DT>, state, heads, dk, dv, dvp);                              \
+    PYRE_WALK_Z(gla_chunk_walk_kernel<DT>, state, o, heads, dk, dv, dvp, qscale);                            \
   } while (0)
   switch (DTs) {
     case 2: PYRE_WALK(2); break;
