@@ -22,8 +22,10 @@ DEFAULT_UNITS = 256
 DECODE_CHUNK = 32
 DECODE_MIN_CHUNKS_PER_BLOCK = 8
 #: a request of up to this many chunks is one block's: three chunks a wave in a row take less than a second block whose
-#: result goes through memory (11.2 us against 13.4 for one request of ten chunks, 13.4 against 16.6 for 30; at 16 chunks
-#: the two are alike)
+#: result goes through memory. One request on the 1.5B heads, us a layer in two blocks and in one: 9 chunks 11.5 and 11.0, 10
+#: 13.4 and 10.1, 11 12.4 and 11.0, 12 13.6 and 11.9, 13 11.0 and 11.4, 14 11.9 and 11.8, 16 12.9 and 13.3, 20 14.2 and 14.7;
+#: 30 requests on the 7B heads 14.4 and 13.6, 16.0 and 11.5, 14.9 and 13.0, 16.3 and 13.9, then 13.8 and 13.1, 15.4 and 14.5,
+#: 15.8 and 15.6, 15.7 and 17.1; with 100 requests the blocks take several rounds and the two are alike at all of them
 DECODE_ONE_BLOCK_CHUNKS = 12
 #: the same when the blocks take several rounds anyway: every block has a start and an end worth
 #: several chunks' time, and nothing is idle that more blocks could fill (measured in the serving
@@ -64,8 +66,8 @@ def decode_work(tokens: np.ndarray, positions: np.ndarray, rows: int, window: in
     number: the missing ones count as requests of one chunk, which is what the padding of a
     captured step is, so that an eager step and a replayed one split alike).
 
-    A request of c chunks of 32 keys gets ceil(c / size) blocks of four waves and deals its
-    chunks evenly to them. The chip runs ``slots`` blocks per key/value item at once. If all
+    A request of c chunks of 32 keys gets ceil(c / size) blocks of four waves (one up to
+    ``DECODE_ONE_BLOCK_CHUNKS``, unless ``size`` is given) and deals its chunks evenly to them. The chip runs ``slots`` blocks per key/value item at once. If all
     blocks can run in one round, ``size`` is the smallest at which they do (but not so small
     that joining a request's blocks takes longer than the blocks): the step then takes as long
     as one block. Otherwise (or if that is slower) ``size`` is half of what a
