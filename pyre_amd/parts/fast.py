@@ -103,9 +103,10 @@ LIBRARY_F32_ROLES = frozenset({"attn.qkv", "attn.out", "mix.in", "mix.out", "cat
 TILE_ROLES = LIBRARY_F32_ROLES | {"ffn.down"}
 
 
-def takes_tiles(rt, n: int, n_out: int, k: int, ldx: int, ldw: int) -> bool:
+def takes_tiles(rt, lin, n: int, x=None) -> bool:
     """Whether a 16-bit product of ``n`` rows goes to the kernel of tiles of up to 256 x 256 (`gemm_tile.hip`): all of more
-    rows than the weight-streaming kernel takes whose sizes it supports. Against the BLAS library's products (us here and there,
+    rows than the weight-streaming kernel takes whose sizes it supports and whose operands lie on 16 bytes (``x`` None: rows like a
+    workspace's; a weight that its owner hands over may be a view). Against the BLAS library's products (us here and there,
     weights from memory, the gated unit and the reading of partial sums with them): the 7B shape's way down 107 and 141 at 566
     rows, 241 and 360 at 2,048, 469 and 537 at 4,096, 936 and 880 at 8,192; its gate/up 156 and 153, 454 and 550, 888 and 868,
     1,717 and 1,780; the 1.5B shape's way down 26 and 31 at 566, 60 and 67 at 2,048, 107 and 103 at 4,096; its gate/up 38 and 43,
@@ -118,14 +119,16 @@ def takes_tiles(rt, n: int, n_out: int, k: int, ldx: int, ldw: int) -> bool:
     has 1.48)."""
     from pyre_amd.hip import ops
 
-    return bool(rt.options.get("tile_gemm", True)) and n > SKINNY_MAX_ROWS and ops.gemm_tile_supports(n, n_out, k, ldx, ldw)
+    if not rt.options.get("tile_gemm", True) or n <= SKINNY_MAX_ROWS or lin.weight.data_ptr() % 16 or (x is not None and x.data_ptr() % 16):
+        return False
+    return ops.gemm_tile_supports(n, lin.out_features, lin.in_features, lin.in_features if x is None else x.stride(0), lin.weight.stride(0))
 
 
 def library_takes(lin, rt, n: int) -> bool:
     """Whether the 16-bit product of ``n`` rows (more than the weight-streaming kernel's) and this weight is left to the BLAS
     library once no kernel for few rows takes it."""
     by_tiles = lin.role in TILE_ROLES or (lin.role == "ffn.gate_up" and lin.bias is None)
-    return not (by_tiles and takes_tiles(rt, n, lin.out_features, lin.in_features, lin.in_features, lin.weight.stride(0)))
+    return not (by_tiles and takes_tiles(rt, lin, n))
 
 
 def _is_bf16(ctx, lin, x) -> bool:
@@ -211,7 +214,7 @@ def linear(lin, ctx, x, n, out):
         else:
             ops.gemm_mid_bf16(x, lin.weight, buf, n, ks, wide=wide)
         return Partials(buf, lin.bias)
-    if lin.role in TILE_ROLES and takes_tiles(rt, n, n_out, k, x.stride(0), lin.weight.stride(0)):
+    if lin.role in TILE_ROLES and takes_tiles(rt, lin, n, x):
         parts = ops.gemm_tile_parts(n, n_out, k)
         buf = ctx.workspace.get(f"linear.{lin.role}.partials", (parts, n, n_out), torch.float32)
         ops.gemm_tile_bf16(x, lin.weight, buf, n, parts)
@@ -250,7 +253,7 @@ def gate_up_silu(lin, ctx, x, n, act, unit=None) -> bool:
         if fits and (ops.gemm_mid_silu_blocks(n, lin.out_features) <= ctx.runtime.compute_units or int(mid) == 2):
             ops.gemm_mid_silu_bf16(x, lin.weight, act, n, unit)
             return True
-    if takes_tiles(ctx.runtime, n, lin.out_features, lin.in_features, x.stride(0), lin.weight.stride(0)):
+    if takes_tiles(ctx.runtime, lin, n, x):
         ops.gemm_tile_glu_bf16(x, lin.weight, act, n, unit)
         return True
     if n > FUSED_SILU_MAX_ROWS or not ctx.runtime.options.get("skinny_gemm", True):

@@ -241,3 +241,24 @@ def test_a_last_round_in_smaller_tiles(m, n, k, gated, by_rows):
     _, cut, rows, rest = ops.gemm_tile_choice(m, n, k, gated)
     assert cut and rows == by_rows
     check_product(m, n, k, gated, None, rest)
+
+
+def test_a_step_with_weights_that_are_views():
+    """Weights that do not lie on 16 bytes: the step's products go to the library and give what they give there."""
+    from pyre_amd.config import EngineConfig, preset
+    from pyre_amd.engine.batch import Entry
+    from pyre_amd.engine.engine import Engine
+    from pyre_amd.weights import model_tensor_specs, random_state
+
+    cfg = preset("tiny-a", hidden_size=128, head_dim=32, intermediate_size=320, num_hidden_layers=2)
+    ids = [(7 * i + 3) % 512 for i in range(300)]
+    rows = []
+    for shift in (0, 4):
+        state = random_state(model_tensor_specs(cfg), 3, 0.08, 0.1, torch.bfloat16, device=DEV)
+        for name, t in state.items():
+            if name.endswith(("o_proj.weight", "down_proj.weight")):
+                state[name] = torch.cat([t.new_zeros(shift), t.flatten()])[shift:].view(t.shape)
+                assert state[name].data_ptr() % 16 == 2 * shift
+        eng = Engine.from_state(cfg, state, EngineConfig(max_cached_tokens=1024, max_num_batched_tokens=512, max_model_len=512))
+        rows.append(eng.step([Entry("a", ids, list(range(300)))]).clone())
+    assert float(((rows[0] - rows[1]).abs().amax(1) / rows[1].abs().amax(1)).max()) <= 2e-2

@@ -266,3 +266,23 @@ def test_what_is_left_to_the_library(role, bias, k, left):
     assert library_takes(Lin, Rt, 2048) is left
     Rt.options = {"tile_gemm": False}
     assert library_takes(Lin, Rt, 2048)
+
+
+def test_products_in_tiles_need_operands_on_16_bytes():
+    """What the kernel of tiles refuses goes to the library: weights and rows that are views of other tensors."""
+    import torch
+
+    from pyre_amd.parts.fast import library_takes, takes_tiles
+
+    class Lin:
+        role, bias, out_features, in_features = "ffn.down", None, 48, 128
+
+    class Rt:
+        options = {}
+
+    store, rows = (torch.zeros(129 * 128, dtype=torch.bfloat16) for _ in range(2))
+    for shift, aligned in ((0, True), (1, False), (4, False), (8, True)):
+        Lin.weight = store[shift:shift + 48 * 128].view(48, 128)
+        assert takes_tiles(Rt, Lin, 100) is aligned and library_takes(Lin, Rt, 100) is not aligned
+        Lin.weight = store[:48 * 128].view(48, 128)
+        assert takes_tiles(Rt, Lin, 100, rows[shift:shift + 100 * 128].view(100, 128)) is aligned
