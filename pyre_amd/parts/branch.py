@@ -54,6 +54,9 @@ class BranchMixer(Mixer):
     def attend(self, ctx, proj: Partials, col0: int, cache, o: torch.Tensor, scale: float) -> None:
         raise NotImplementedError
 
+    #: whether ``attend`` is better off with an input product of many rows that comes as one sum (see Linear)
+    whole_input = False
+
     def inner_linears(self) -> list:
         """Products that ``attend`` runs itself."""
         return []
@@ -78,7 +81,7 @@ class BranchMixer(Mixer):
             w = torch.cat([w, torch.zeros(pad, w.shape[1], dtype=w.dtype, device=w.device)], dim=0)
             if bias is not None:
                 bias.append(torch.zeros(pad, dtype=torch.float32, device=w.device))
-        self._in = Linear(self.hidden_size, w.shape[0], f"{self.role}.in")
+        self._in = Linear(self.hidden_size, w.shape[0], f"{self.role}.in", self.whole_input)
         self._out = Linear(self.inner, self.hidden_size, f"{self.role}.out")
         self._in.set(w, None if bias is None else torch.cat(bias))
         ob = self.out_bias()
@@ -179,7 +182,7 @@ class ParallelMixer(Mixer):
                                                                                   dtype=torch.float32, device=mine[0].device)]))
             parts += mine
             col += rows
-        self.proj = Linear(self.spec.hidden_size, col, "mix.in")
+        self.proj = Linear(self.spec.hidden_size, col, "mix.in", any(b.whole_input for b in self.branches))
         bias = None
         if any(x is not None for x in biases):  # one bias over all branches' columns, zero where a branch has none
             rows = [*self.first_column[1:], col]

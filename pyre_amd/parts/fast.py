@@ -215,7 +215,7 @@ def linear(lin, ctx, x, n, out):
             ops.gemm_mid_bf16(x, lin.weight, buf, n, ks, wide=wide)
         return Partials(buf, lin.bias)
     if lin.role in TILE_ROLES and takes_tiles(rt, lin, n, x):
-        parts = ops.gemm_tile_parts(n, n_out, k)
+        parts = 1 if lin.whole else ops.gemm_tile_parts(n, n_out, k)
         buf = ctx.workspace.get(f"linear.{lin.role}.partials", (parts, n, n_out), torch.float32)
         ops.gemm_tile_bf16(x, lin.weight, buf, n, parts)
         return Partials(buf, lin.bias)

@@ -16,10 +16,11 @@ from pyre_amd.parts.base import TensorSpec
 
 
 class Linear:
-    def __init__(self, in_features: int, out_features: int, role: str):
+    def __init__(self, in_features: int, out_features: int, role: str, whole: bool = False):
         self.in_features = in_features
         self.out_features = out_features
         self.role = role              #: names this product's scratch buffer
+        self.whole = whole            #: of many rows: handed on as one sum, for a consumer that loses more by partial sums
         self.weight: torch.Tensor | None = None   # [out, in]
         self.bias: torch.Tensor | None = None
 

@@ -23,6 +23,10 @@ class SelectiveScan(BranchMixer):
     (rounded, and what the rounding left) against W_dt twice; a step of single tokens makes them inside its scan's kernel."""
 
     role = "ssm"
+    # The scan's walk is a chain and its helping waves bring a tile while one is walked: loads alone, all on their way together,
+    # where each of its three products is one sum, 102 us for 2,048 tokens of 1,536 channels with a state of 16; 307 us where
+    # any comes in parts (7B shape: 108 and 317). The product itself takes a few us longer in one part (see Linear.whole).
+    whole_input = True
 
     def __init__(self, spec: SelectiveScanSpec):
         if spec.inner <= 0 or spec.dt_rank <= 0 or not (0 < spec.state <= ops.SSM_MAX_STATE):
@@ -76,12 +80,12 @@ class SelectiveScan(BranchMixer):
 
         width = s.dt_rank + 2 * s.state
         width += -width % COLUMN_ALIGN
-        self.select = Linear(s.inner, width, "ssm.x")
+        self.select = Linear(s.inner, width, "ssm.x", whole=True)
         self.select.set(padded(take(tensors, f"{p}.x"), width, s.inner))
         dt = padded(take(tensors, f"{p}.dt"), s.inner, self.padded_rank)
         if runtime.dtype != torch.float32:
             dt = torch.cat([dt, dt], dim=1)
-        self.steps = Linear(dt.shape[1], s.inner, "ssm.dt")
+        self.steps = Linear(dt.shape[1], s.inner, "ssm.dt", whole=True)
         self.steps.set(dt)
 
     def inner_linears(self) -> list:

@@ -876,3 +876,34 @@ def test_trace_run_as_a_process(dtype, extra, folders, tmp_path):
             assert d <= TOL[dtype], f"step {st} request {r} position {pos}: {d:.3e}"
             checked += 1
     assert checked > 50
+
+
+@pytest.mark.parametrize("n", [257, 300])
+def test_the_scan_of_a_prompt_gets_whole_sums(n, monkeypatch):
+    """In the 16-bit mode a prompt's products that the scan reads come in one part, also at sizes where the kernel of tiles
+    splits k: the scan's form without partial sums takes a third of the time. The result is the 32-bit mode's, rounded."""
+    from pyre_amd.config.engine import EngineConfig
+    from pyre_amd.engine.batch import Entry
+    from pyre_amd.engine.engine import Engine
+    from pyre_amd.hip import ops
+    from pyre_amd.registry import config_from_dict
+    from pyre_amd.weights import model_tensor_specs, random_state
+
+    cfg = config_from_dict(M.model(96, 512, [M.parallel(M.attention(2, 1, 32, 32, 0.2), M.scan(512, 16, 32, 4), 64)]))
+    assert ops.gemm_tile_parts(n, 64, 512) > 1 and ops.gemm_tile_parts(n, 1152, 512) > 1
+    parts, scan, rows = [], ops.ssm_scan, {}
+
+    def seen(z, dt_b, x, sel, rank, proj, *rest, **kw):
+        parts.append((x.dtype, len(z.data), len(sel.data), len(proj.data)))
+        return scan(z, dt_b, x, sel, rank, proj, *rest, **kw)
+
+    monkeypatch.setattr(ops, "ssm_scan", seen)
+    for dtype in (torch.float32, torch.bfloat16):
+        state = random_state(model_tensor_specs(cfg), 5, 0.05, 0.1, torch.bfloat16, device=DEV)
+        name = str(dtype).split(".")[1]
+        engine = Engine.from_state(cfg, {k: v.to(dtype) for k, v in state.items()},
+                                   EngineConfig(dtype=name, max_cached_tokens=1024, max_num_batched_tokens=512, max_model_len=400))
+        rows[dtype] = engine.step([Entry("a", [(7 * i + 3) % 96 for i in range(n)], list(range(n)))]).clone()
+    assert [p[1:] for p in parts if p[0] == torch.bfloat16] == [(1, 1, 1)]
+    off = (rows[torch.bfloat16] - rows[torch.float32]).abs().amax(1) / rows[torch.float32].abs().amax(1)
+    assert float(off.max()) <= TOL["bfloat16"] and float(off.median()) <= MEDIAN[TOL["bfloat16"]]
