@@ -141,7 +141,7 @@ def narrow_kernel(n: int, n_out: int, k: int, options: dict | None = None,
     """Which of our kernels takes a 16-bit product of ``n`` rows whose result is handed on as partial
     sums: ("stream", parts of k, False) for the weight-streaming kernel, ("block", parts, wide) for the
     kernel that keeps the step's rows in a block (``wide``: 128 rows of the weights a block instead
-    of 64), ("", 0, False) for neither (the BLAS library then). A function of the sizes (and of the
+    of 64), ("", 0, False) for neither (the kernel of tiles then, or the BLAS library). A function of the sizes (and of the
     device's compute units, which an engine reads once) alone; the
     thresholds in rows lie just above sizes at which decode steps are captured, so that an eager step
     and its replay at the padded size agree."""
@@ -244,7 +244,7 @@ def gate_up_silu(lin, ctx, x, n, act, unit=None) -> bool:
         # where one round of blocks holds them. Measured on the 1.5B shape: 17 us against the
         # library's product and the SiLU-gate kernel's 29 at 65 to 128 rows, 26 against 30 at 192, 28 at 256;
         # on the 7B shape 55 against 66 at 128, and at 256 rows, as on the 32B shape, two rounds of
-        # blocks: those stay with the library. With blocks of 32 and 64 rows of X for steps that
+        # blocks: those go to the kernel of tiles. With blocks of 32 and 64 rows of X for steps that
         # small it is ahead of the weight-streaming kernel at every size: on the 7B shape 3.20
         # against 3.23 ms a step at one request, 3.44 against 3.49 at 8, 3.77 against 3.87 at 16,
         # 4.46 against 4.56 at 32, 5.87 against 6.13 at 64; on the 1.5B shape by 1 to 4 %.
