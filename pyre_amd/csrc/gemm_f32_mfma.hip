@@ -1,27 +1,30 @@
-// out[m, n] = sum_k A[m, k] * W[n, k] (+ bias[n]) with all three in float32, on the matrix
-// cores' true 32-bit instruction (v_mfma_f32_32x32x2_f32: float32 operands, float32 products
-// and sums; no reduced-precision mode is involved). This is the product of the 32-bit path
+// out[m, n] = sum_k A[m, k] * W[n, k] (+ bias[n]) with all three in float32. This is the product of the 32-bit path
 // of the model (`pyre/model.py:92-94,125,139,201` are the products it stands for); operands
 // of mixed element types stay with gemm_generic.hip.
+//
+// The matrix cores' float32 instruction has a sixteenth of the 16-bit instruction's rate, so the products are made of bfloat16
+// pieces: a float32 is the sum of three, x = h + m + l with eight bits each, exactly, and a product of two bfloat16 is exact in
+// float32. Of the nine products of pieces the six largest are added, l h', h l', m m', m h', h m' and h h' in this order; what
+// is left out (m l', l m', l l') is below 2^-26 of the product, less than the rounding of a float32 product. An instruction
+// adds sixteen products of each kind at once, so that an element's sum is rounded six times for 16 k where a chain of fused
+// multiply-adds rounds 16 times, and the sum is made in pieces that are added in float32 (below). Distance from 64 bits,
+// root mean square over that of the values, against the float32 instruction on the same numbers: 1.9e-7 and 7.1e-7 for sums of
+// 1,536 products, 2.5e-7 and 1.6e-6 of 8,960, and 4.0e-7 and 4.8e-7 for a single chain of 640. Numbers that
+// a bfloat16 cannot hold the pieces of (infinities and those within 2^-9 of the largest) give a sum that is not finite: such an
+// element is made again as a chain of fused multiply-adds.
 //
 // As in the weight-streaming kernels the product is computed transposed, out^T = W A^T: the
 // 32 rows of an MFMA tile are output columns n, its 32 columns are rows m, so that a lane
 // holds runs of four consecutive n of one row m and stores them as one float4.
 //
-// The instruction adds an element's products one after the other, each with one fused
-// multiply-add, in the order of its k (for 32x32x2: lanes 0..31, then lanes 32..63; for 16x16x4:
-// the four groups of 16 lanes in turn), exactly as a chain of fmaf() does. k is walked in stages
-// of 16 through LDS, and within a stage in the order 0, 4, 8, 12, 1, 5, 9, 13, 2, ..., 15: step s
-// (0..7) of 32x32x2 multiplies k = 8 (s & 1) + (s >> 1) in lanes 0..31 and that k + 4 in lanes
-// 32..63, so that a lane reads its eight values of a stage as two 16-byte LDS loads (pieces
-// `half` and `half` + 2); step i (0..3) of 16x16x4 multiplies k = 4 g + i in its lane group g (one
-// 16-byte load). The order in which an element's products are added is a function of k alone and
-// the same for every tile shape and both instructions below, so an element's value does not depend
-// on the shape, on the number of rows in the step or on where the row lies in it, bit for bit.
+// All kernels below walk k in steps of 16, lanes 0..31 holding k 0..7 of a step and lanes 32..63 k 8..15, on
+// v_mfma_f32_32x32x16_bf16, so that an element's value does not depend on the kernel or the tile,
+// on the number of rows in the step or on where the row lies in it, bit for bit. Steps past the end of k add zeros.
 //
-// k may be split into `ksplit` parts (grid.z), each writing a partial sum out[s] that the
+// k may be split into `ksplit` parts (grid.z or tiles of their own), each writing a partial sum out[s] that the
 // consumer adds in the order 0..ksplit-1: products with few output columns and a long k would
-// otherwise leave most of the chip idle. The caller chooses ksplit from N and K alone.
+// otherwise leave most of the chip idle. The caller chooses ksplit from N and K alone. A part is one chain of
+// instructions; a product in one part is made in chains of 128 k, added in float32.
 #include "pyre_api.h"
 #include "pyre_common.h"
 
@@ -31,9 +34,72 @@ namespace {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
-constexpr int BK = 16;      // k per stage
-constexpr int LD = BK + 4;  // floats per LDS row: 80 bytes, so that eight rows' 16-byte pieces fall on distinct banks
+constexpr int BK = 16;        // k per step
+constexpr int LD = BK + 4;    // floats per LDS row of the general kernel
+constexpr int kChain = 8;     // steps of a chain of a product in one part
+
+// Eight float32 as three times eight bfloat16 that sum to them.
+struct Pieces {
+  u32x4 p[3];
+};
+__device__ inline Pieces split8(f32x4 lo, f32x4 hi) {
+  Pieces r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = i < 2 ? lo[2 * i] : hi[2 * i - 4], b = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const uint32_t w = pack_bf16x2(a, b);
+      r.p[t][i] = w;
+      a -= __uint_as_float(w << 16);
+      b -= __uint_as_float(w & 0xffff0000u);
+    }
+  }
+  return r;
+}
+
+// The six products of pieces, the smallest first: piece of W, piece of A.
+constexpr int kTerms = 6;
+constexpr int kTermW[kTerms] = {2, 0, 1, 1, 0, 0}, kTermA[kTerms] = {0, 2, 1, 0, 1, 0};
+__device__ inline f32x16 multiply(u32x4 w, u32x4 a, f32x16 acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), acc, 0, 0, 0);
+}
+
+// Output columns n .. n + 3 of a row; whether one of their sums is not finite.
+__device__ inline bool store4(f32x4 v, float* row, bool rows_of_16, int n, int N) {
+  bool bad = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) bad |= !(fabsf(v[j]) < INFINITY);
+  if (n + 3 < N && rows_of_16) {
+    *reinterpret_cast<f32x4*>(row + n) = v;
+  } else {
+#pragma unroll 1
+    for (int j = 0; j < 4 && n + j < N; ++j) row[n + j] = j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
+  }
+  return bad;
+}
+
+// What the usual product does not need, over the elements that this lane has stored (of rows m, m + 32, .., column groups of four
+// at n + 8 i): the sums that are not finite once more, without pieces (`a` and `w` are the rows of A and W at the part's first k of
+// `len`), and the bias.
+__device__ inline void finish(const float* a, size_t lda, const float* w, size_t ldw, const void* bias, int bias_dt, float* out,
+                              size_t ldo, int m, int mtiles, int M, int n, int ntiles, int N, int len) {
+#pragma unroll 1
+  for (int e = 0; e < 16 * mtiles * ntiles; ++e) {
+    const int row = m + 32 * (e / (16 * ntiles)), col = n + 8 * (e / 4 % (4 * ntiles)) + e % 4;
+    if (row >= M || col >= N) continue;
+    float s = out[row * ldo + col];
+    if (!(fabsf(s) < INFINITY)) {
+      s = 0.f;
+#pragma unroll 1
+      for (int k = 0; k < len; ++k) s = fmaf(a[row * lda + k], w[col * ldw + k], s);
+    }
+    out[row * ldo + col] = s + (bias ? load_as_float(bias, bias_dt, col) : 0.f);
+  }
+}
 
 // Four consecutive k of one row; zero where the row or the k is not there.
 __device__ inline f32x4 load_k4(const float* base, size_t ld, int row, int rows, int k, int K, bool vec_ok) {
@@ -45,12 +111,13 @@ __device__ inline f32x4 load_k4(const float* base, size_t ld, int row, int rows,
   return v;
 }
 
-// WN x WM waves (along n and along m), each on TN x TM tiles of 32 x 32.
+// Rows that do not start on 16 bytes, and k that is not a multiple of four: 16 k of both operands at a time through registers
+// and LDS as float32, split by the waves that multiply them. WN x WM waves (along n and along m), each on TN x TM tiles of 32 x 32.
 template <int WN, int WM, int TN, int TM>
 __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
     const float* __restrict__ A, size_t lda, const float* __restrict__ W, size_t ldw,
     const void* __restrict__ bias, int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M,
-    int N, int K, int kper, int vec_ok) {
+    int N, int K, int kper, int chain, int vec_ok) {
   constexpr int NT = 64 * WN * WM, BN = WN * TN * 32, BM = WM * TM * 32;
   constexpr int WP = (BN * 4 + NT - 1) / NT, AP = (BM * 4 + NT - 1) / NT;  // 16-byte pieces per thread and stage
   __shared__ __attribute__((aligned(16))) float Ws[BN][LD];
@@ -89,98 +156,95 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
     }
   };
 
-  f32x16 acc[TN][TM];
+  f32x16 acc[TN][TM], total[TN][TM];
 #pragma unroll
   for (int t = 0; t < TN; ++t)
 #pragma unroll
     for (int u = 0; u < TM; ++u)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[t][u][i] = 0.f;
+      for (int i = 0; i < 16; ++i) acc[t][u][i] = total[t][u][i] = 0.f;
 
+  const int kfirst = kbeg;
+  auto end_chain = [&]() {
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+      for (int u = 0; u < TM; ++u)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          total[t][u][i] += acc[t][u][i];
+          acc[t][u][i] = 0.f;
+        }
+  };
+  int left = chain;
   fetch(kbeg);
   for (int k0 = kbeg; k0 < K; k0 += BK) {
     stash();
     __syncthreads();
     if (k0 + BK < K) fetch(k0 + BK);  // in flight while this stage is multiplied
-    f32x4 a[TN][2], b[TM][2];
+    Pieces b[TM];
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
+    for (int u = 0; u < TM; ++u) {
+      const float* p = &As[(wm * TM + u) * 32 + c][8 * half];
+      b[u] = split8(*reinterpret_cast<const f32x4*>(p), *reinterpret_cast<const f32x4*>(p + 4));
+    }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) a[t][h] = *reinterpret_cast<const f32x4*>(&Ws[(wn * TN + t) * 32 + c][4 * half + 8 * h]);
+    for (int t = 0; t < TN; ++t) {
+      const float* p = &Ws[(wn * TN + t) * 32 + c][8 * half];
+      const Pieces a = split8(*reinterpret_cast<const f32x4*>(p), *reinterpret_cast<const f32x4*>(p + 4));
 #pragma unroll
-    for (int u = 0; u < TM; ++u)
+      for (int s = 0; s < kTerms; ++s)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) b[u][h] = *reinterpret_cast<const f32x4*>(&As[(wm * TM + u) * 32 + c][4 * half + 8 * h]);
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int t = 0; t < TN; ++t)
-#pragma unroll
-        for (int u = 0; u < TM; ++u)
-          acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][s & 1][s >> 1], b[u][s & 1][s >> 1], acc[t][u], 0, 0, 0);
+        for (int u = 0; u < TM; ++u) acc[t][u] = multiply(a.p[kTermW[s]], b[u].p[kTermA[s]], acc[t][u]);
+    }
+    if (--left == 0) {
+      end_chain();
+      left = chain;
+    }
     __syncthreads();
   }
+  end_chain();
 
-  // acc[t][u][4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = tile column c.
+  // total[t][u][4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = tile column c.
+  const bool rows_of_16 = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  const int m = m0 + wm * TM * 32 + c, n = n0 + wn * TN * 32 + 4 * half;
+  bool bad = false;
 #pragma unroll
   for (int u = 0; u < TM; ++u) {
-    const int m = m0 + (wm * TM + u) * 32 + c;
-    if (m >= M) continue;
+    if (m + 32 * u >= M) continue;
 #pragma unroll
     for (int t = 0; t < TN; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = n0 + (wn * TN + t) * 32 + 8 * i + 4 * half;
-        if (n >= N) continue;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v[j] = acc[t][u][4 * i + j];
-          if (bias && n + j < N) v[j] += load_as_float(bias, bias_dt, n + j);
-        }
-        float* dst = out + static_cast<size_t>(m) * ldo + n;
-        if (n + 3 < N && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
-          for (int j = 0; j < 4 && n + j < N; ++j) dst[j] = v[j];
-        }
-      }
+      for (int i = 0; i < 4; ++i)
+        bad |= store4(f32x4{total[t][u][4 * i], total[t][u][4 * i + 1], total[t][u][4 * i + 2], total[t][u][4 * i + 3]},
+                      out + static_cast<size_t>(m + 32 * u) * ldo, rows_of_16, n + 32 * t + 8 * i, N);
   }
+  if (bad || bias) finish(A + kfirst, lda, W + kfirst, ldw, bias, bias_dt, out, ldo, m, TM, M, n, TN, N, K - kfirst);
 }
 
-// 16 bytes per lane from `base + off` straight into LDS: lane x's piece lands at lds_addr + 16 x. The s_nop is the wait state that the instruction
-// needs behind a scalar write of m0; the compiler puts none into inline assembly.
-__device__ inline void load_rows(const void* base, unsigned off, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
-}
-template <int N>
-__device__ inline void wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
-}
-constexpr int kSlotK = 32;  // k of a slot (two stages) of the rings below: rows of 128 bytes
-
-// The same product for more than 16 rows whose k comes in whole stages, bit for bit. A slot of the ring in LDS holds 32 k of the
-// block's BN rows of W and BM rows of A, filled by loads that go from memory straight into LDS; the 16-byte pieces of a row
-// are exchanged among themselves by the row's number. The operands of the next stage are read while the present one is
-// multiplied; the one barrier of a slot stands before its second stage: every wave has read the slot for the last time by
-// then, so the loads of S slots further on go into it, and the next slot, which everybody has waited for, is read from.
+// More than 32 rows whose k comes in whole steps. A block of four waves keeps BM rows of A and BN rows of W; every thread brings
+// eight k of some rows, two steps ahead in registers, splits them once for the whole block and writes the pieces into one of two
+// buffers in LDS, while the pieces in the other are multiplied: one barrier a slot of SL steps.
 //
-// What bounds it are the matrix cores (64 cycles for 4,096 multiply-adds): a block's loads are a tenth of what a compute unit
-// can take. So the tiles are small enough that all compute units have equally many, several blocks to a unit, whose waves
-// hide each other's waits. Against one buffer in LDS behind two barriers a stage and tiles of 128 x 128 (the 1.5B shape's
-// weights, us): q/k/v 55 -> 40 and the way down 169 -> 130 at 566 rows, gate/up 321 -> 241; 149 -> 81 at 72; 952 -> 834
-// at 2,048 (135 of 157 TFLOP/s). Against waves that stream the weights with a barrier a slot, at 40 rows: q/k/v 24 -> 14, way
-// down 46 -> 28, gate/up 64 -> 59; at 20 rows 15.0 -> 14.3, 29.6 -> 27.9, 41.5 -> 39.2 (the 7B shape's q/k/v 20.8 -> 17.0).
-// WHOLE: a block walks all parts of k and adds their sums up in their order, as the consumer of partial sums does (the same
-// bits), where the rows alone fill the chip: the parts of a prompt do not go through memory.
-template <int BM, int BN, int WM, int WN, int S, int OCC, bool WHOLE>
-__global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
-    const float* __restrict__ A, long lda, const float* __restrict__ W, long ldw, const void* __restrict__ bias,
-    int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int mt, int nt) {
-  constexpr int NW = WM * WN, SLOT = (BM + BN) * 128, LX = BM / 8 / NW, LW = BN / 8 / NW, L = LX + LW;
-  constexpr int CT = BM / WM / 32, RT = BN / WN / 32, RD = 2 * (RT + CT), MF = 8 * RT * CT;
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "rows divide over the waves");
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[S * SLOT];
+// What bounds it: a step of 128 x 128 is 768 cycles of the matrix cores a SIMD, 580 cycles of LDS (24 KB written, 48 KB read) and
+// 350 of splitting; two blocks share a compute unit and fill each other's waits. At 2,000 rows of the 7B shape the gate/up product
+// runs at 197 TFLOP/s, 1.18 PFLOP/s of the 16-bit instruction, what that reaches at the clocks the card's power leaves. Against the float32
+// instruction (135 of its 157 TFLOP/s; us): gate/up 4,007 -> 2,748 there, 1,254 -> 885 at 566 rows, 316 -> 270 at 99; the 1.5B shape's
+// 844 -> 581, 245 -> 210 and 80 -> 72, its way down 446 -> 314, 127 -> 106 and 37 -> 35.
+// The eight k of a lane lie in arrays of their own, so that the lanes of a read are neighbours; each starts 64 bytes (32 of
+// slots of two steps) off the banks of the one before, since a write's lanes go to all of them in turn.
+//
+// A chain of instructions ends after `chain` steps and is added to the total in float32. A block that walks all parts of k
+// (where the rows alone fill the chip) ends its chains where the parts end: the bits of the consumer's sum of partial sums, which
+// then do not go through memory.
+template <int BM, int BN, int WM, int WN, int SL, int OCC>
+__global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
+    const float* A, long lda, const float* W, long ldw, const void* __restrict__ bias,
+    int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int chain, int mt, int nt) {
+  constexpr int R = BM + BN, KP = 2 * SL, P = KP * R / 256, ROWS = 16 * R + 64 / SL, PLANE = KP * ROWS, BUF = 3 * PLANE;
+  constexpr int CT = BM / WM / 32, RT = BN / WN / 32;
+  static_assert(WM * WN == 4 && KP * R % 256 == 0, "four waves, whose threads bring equally many pieces");
+  __shared__ __attribute__((aligned(64))) unsigned char lds[2 * BUF];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 31, half = lane >> 5, wm = wave % WM, wn = wave / WM;
   // Blocks are dealt to the eight dies in turn: a die's blocks are neighbours, eight tiles along m by some along n.
@@ -191,417 +255,375 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_f32_tile_kernel(
   const int group = t / (8 * nt), first = 8 * group, gm = min(8, mt - first);
   t -= 8 * nt * group;
   const int m0 = (first + t % gm) * BM, n0 = (t / gm) * BN;
-  const int kbeg = WHOLE ? 0 : ks * kper, kend = WHOLE ? K : min(K, kbeg + kper), slots = (kend - kbeg + kSlotK - 1) / kSlotK;
+  const int kbeg = ks * kper, kend = min(K, kbeg + kper), steps = (kend - kbeg) / BK;
+  const int slots = (steps + SL - 1) / SL;
   out += ks * part_stride;
   if (ks) bias = nullptr;  // the bias belongs to one part only
-  const unsigned base = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
-  const int lrow = lane >> 3, lpiece = lane & 7;
-  unsigned offx[LX], offw[LW];
-  int piece[L];
+
+  const float* src[P];
+  unsigned dst[P];
 #pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int row = 8 * (NW * i + wave) + lrow;  // rows past the end are the last one once more, and are not stored
-    piece[i] = lpiece ^ ((row >> 1) & 7);
-    offx[i] = static_cast<unsigned>(min(m0 + row, M - 1)) * static_cast<unsigned>(4 * lda);
+  for (int i = 0; i < P; ++i) {
+    const int p = threadIdx.x + 256 * i, row = p / KP, h = p % KP;  // rows past the end are the last one once more, and are not stored
+    src[i] = (row < BM ? A + static_cast<size_t>(min(m0 + row, M - 1)) * lda : W + static_cast<size_t>(min(n0 + row - BM, N - 1)) * ldw) +
+             kbeg + 8 * h;
+    dst[i] = h * ROWS + 16 * row;
   }
+  f32x4 st[2][P][2];
+  const bool short_end = SL > 1 && steps % SL;  // the last slot has fewer steps: what lies behind them is not multiplied
+  auto fetch = [&](int buf, int slot) {
+    const int at = min(slot, slots - 1);
 #pragma unroll
-  for (int i = 0; i < LW; ++i) {
-    const int row = 8 * (NW * i + wave) + lrow;
-    piece[LX + i] = lpiece ^ ((row >> 1) & 7);
-    offw[i] = static_cast<unsigned>(min(n0 + row, N - 1)) * static_cast<unsigned>(4 * ldw);
-  }
-  const char* xb = reinterpret_cast<const char*>(A + kbeg);
-  const char* wb = reinterpret_cast<const char*>(W + kbeg);
-  auto issue = [&](int i, int st, unsigned slot_base) {
-    // the last slot may hold 16 k only: the pieces behind them are the row's first once more, and are not multiplied
-    const int pc = 4 * piece[i] < kend - kbeg - kSlotK * st ? piece[i] : 0;
-    if (i < LX) load_rows(xb, offx[i < LX ? i : 0] + 16 * pc, slot_base + (NW * i + wave) * 1024);
-    else load_rows(wb, offw[i < LX ? 0 : i - LX] + 16 * pc, slot_base + BM * 128 + (NW * (i - LX) + wave) * 1024);
-  };
-  const unsigned char* const xrow = lds + (wm * 32 * CT + c) * 128;
-  const unsigned char* const wrow = lds + BM * 128 + (wn * 32 * RT + c) * 128;
-  const int swz = (c >> 1) & 7;
-  f32x4 a[2][RT][2], b[2][CT][2];
-  auto read = [&](int x, int run, int buf, int slot) {
-    const int h = x & 1, y = x >> 1, at = slot * SLOT + 16 * ((4 * run + half + 2 * h) ^ swz);
-    if (y < RT) a[buf][y < RT ? y : 0][h] = *reinterpret_cast<const f32x4*>(wrow + at + y * 32 * 128);
-    else b[buf][y < RT ? 0 : y - RT][h] = *reinterpret_cast<const f32x4*>(xrow + at + (y - RT) * 32 * 128);
-  };
-#pragma unroll
-  for (int s = 0; s < S; ++s)
-    if (s < slots) {
-#pragma unroll
-      for (int i = 0; i < L; ++i) issue(i, s, base + s * SLOT);
-      xb += 128;
-      wb += 128;
+    for (int i = 0; i < P; ++i) {
+      const int k = BK * SL * at - (short_end && at == slots - 1 && (threadIdx.x + 256 * i) % KP >= 2 ? BK : 0);
+      st[buf][i][0] = *reinterpret_cast<const f32x4*>(src[i] + k);
+      st[buf][i][1] = *reinterpret_cast<const f32x4*>(src[i] + k + 4);
     }
-  if (slots < S) wait_loads<0>();
-  else wait_loads<(S - 1) * L>();
-  asm volatile("s_barrier" ::: "memory");
+  };
+  auto convert = [&](int buf, int i) {
+    const Pieces v = split8(st[buf][i][0], st[buf][i][1]);
 #pragma unroll
-  for (int x = 0; x < RD; ++x) read(x, 0, 0, 0);
-  f32x16 acc[RT][CT];
+    for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x4*>(lds + buf * BUF + s * PLANE + dst[i]) = v.p[s];
+  };
+  const unsigned char* const arow = lds + half * ROWS + 16 * (wm * 32 * CT + c);
+  const unsigned char* const wrow = lds + half * ROWS + 16 * (BM + wn * 32 * RT + c);
+  f32x16 acc[RT][CT], total[RT][CT];
 #pragma unroll
   for (int r = 0; r < RT; ++r)
 #pragma unroll
     for (int q = 0; q < CT; ++q)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[r][q][i] = 0.f;
-  f32x16 total[WHOLE ? RT : 1][WHOLE ? CT : 1];
-  int left = kper / BK;  // stages until the part ends
-  if (WHOLE) {
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int q = 0; q < CT; ++q)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) total[WHOLE ? r : 0][WHOLE ? q : 0][i] = 0.f;
-  }
-  auto end_part = [&]() {
+      for (int i = 0; i < 16; ++i) acc[r][q][i] = total[r][q][i] = 0.f;
+  auto end_chain = [&]() {
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int q = 0; q < CT; ++q)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          total[WHOLE ? r : 0][WHOLE ? q : 0][i] += acc[r][q][i];
+          total[r][q][i] += acc[r][q][i];
           acc[r][q][i] = 0.f;
         }
-    left = kper / BK;
   };
-  int slot = 0;
-  for (int st = 0; st < slots; ++st) {
-    const int next = slot + 1 == S ? 0 : slot + 1;
+  int left = chain;
+  auto turn = [&](int buf, int slot) {
 #pragma unroll
-    for (int run = 0; run < 2; ++run) {
-      bool more = false;
-      if (run == 1) {
-        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-        if (st + S > slots) wait_loads<0>();
-        else wait_loads<(S - 2) * L>();
-        asm volatile("s_barrier" ::: "memory");
-        more = st + S < slots;
-        if (kbeg + kSlotK * st + BK >= kend) break;  // a part that ends with half a slot
+    for (int j = 0; j < SL; ++j) {
+      if (j > 0 && SL * slot + j >= steps) break;
+      u32x4 a[RT][3], b[CT][3];
+      const int at = buf * BUF + 2 * j * ROWS;
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) a[r][2 - s] = *reinterpret_cast<const u32x4*>(wrow + at + (2 - s) * PLANE + 512 * r);
+#pragma unroll
+        for (int q = 0; q < CT; ++q) b[q][s] = *reinterpret_cast<const u32x4*>(arow + at + s * PLANE + 512 * q);
       }
 #pragma unroll
-      for (int g = 0; g < MF; ++g) {
-        const int s = g / (RT * CT), r = g % (RT * CT) / CT, q = g % CT;
+      for (int s = 0; s < kTerms; ++s) {
 #pragma unroll
-        for (int x = 0; x < RD; ++x)
-          if (x * MF / RD / 2 == g) read(x, run == 0 ? 1 : 0, run ^ 1, run == 0 ? slot : next);
-        acc[r][q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[run][r][s & 1][s >> 1], b[run][q][s & 1][s >> 1], acc[r][q], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (run == 1 && more) {
+        for (int r = 0; r < RT; ++r)
 #pragma unroll
-          for (int i = 0; i < L; ++i)
-            if (i * MF / L == g) issue(i, st + S, base + slot * SLOT);
+          for (int q = 0; q < CT; ++q) acc[r][q] = multiply(a[r][kTermW[s]], b[q][kTermA[s]], acc[r][q]);
+        // the next slot's pieces meanwhile
+        if (j == 0) {
+#pragma unroll
+          for (int i = 0; i < P; ++i)
+            if (i * (kTerms - 1) / P == s) convert(buf ^ 1, i);
         }
       }
-      if (run == 1 && more) {
-        xb += 128;
-        wb += 128;
+      if (j == 0) fetch(buf ^ 1, slot + 3);
+      if (--left == 0) {
+        end_chain();
+        left = chain;
       }
-      if (WHOLE && --left == 0) end_part();
     }
-    slot = next;
-  }
-  if (WHOLE) {
-    end_part();  // a last, shorter part (or nothing)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  // in the order in which the turns ask, so that a turn waits for its own slot alone (the operands are not __restrict__: the
+  // compiler would move these loads behind one another)
+  fetch(0, 0);
+  asm volatile("" ::: "memory");
+  fetch(1, 1);
+  asm volatile("" ::: "memory");
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-      for (int q = 0; q < CT; ++q) acc[r][q] = total[WHOLE ? r : 0][WHOLE ? q : 0];
+  for (int i = 0; i < P; ++i) convert(0, i);
+  fetch(0, 2);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  int slot = 0;
+  for (; slot + 2 <= slots; slot += 2) {  // (no way round turn 1: the compiler's waits are those of the worst way)
+    turn(0, slot);
+    turn(1, slot + 1);
   }
+  if (slot < slots) turn(0, slot);
+  end_chain();  // a last, shorter chain (or nothing)
+  const bool rows_of_16 = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  const int m = m0 + 32 * wm * CT + c, n = n0 + 32 * wn * RT + 4 * half;
+  bool bad = false;
 #pragma unroll
   for (int q = 0; q < CT; ++q) {
-    const int m = m0 + 32 * (wm * CT + q) + c;
-    if (m >= M) continue;
+    if (m + 32 * q >= M) continue;
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = n0 + 32 * (wn * RT + r) + 8 * i + 4 * half;
-        if (n >= N) continue;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v[j] = acc[r][q][4 * i + j];
-          if (bias && n + j < N) v[j] += load_as_float(bias, bias_dt, n + j);
-        }
-        float* dst = out + static_cast<size_t>(m) * ldo + n;
-        if (n + 3 < N && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
-          for (int j = 0; j < 4 && n + j < N; ++j) dst[j] = v[j];
-        }
-      }
+      for (int i = 0; i < 4; ++i)
+        bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]},
+                      out + static_cast<size_t>(m + 32 * q) * ldo, rows_of_16, n + 32 * r + 8 * i, N);
   }
+  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, kend - kbeg);
 }
 
-// The same product for a decode step's rows (M <= 16; up to 64 where k does not come in whole stages), as a stream over the
-// weights. A block is one wave with 32 output columns, so there is no barrier. It has a ring of R slots in LDS, a
-// slot being 32 k (two stages) of its 32 rows of W (4 KB) and of XR rows of A (XR = 8, 16, 32 or 64,
-// whichever holds M: 1 to 8 KB), filled by loads that go from memory straight into LDS: while
-// slot j is multiplied, slot j + 1 is read from LDS into registers and the R - 2 after it are on
-// their way. A load instruction takes whole 128-byte lines (8 rows x 32 k); the 16-byte pieces
-// of a row are exchanged among themselves by the row's number so that the matrix instruction's
-// operand reads (a lane's row, eight k of a stage) spread over the banks. Stages, steps and
-// parts of k are those of the kernel above, and an element of the result depends on its own
-// row of A and row of W alone: the sums are the same bit for bit, however many of the
-// instruction's 32 columns carry a row. With few rows the chain of dependent instructions of a
-// wave, not memory, sets the pace (a slot of 4 KB in about 0.6 us), and with 64 rows the matrix
-// cores' float32 rate does; a small ring lets several blocks share a compute unit.
-constexpr int kStreamMaxRows = 64;
+constexpr int kStreamMaxRows = 32;
 constexpr int kMaxDevices = 64;
+constexpr int kSlotK = 32;  // k of a slot of the ring: rows of 128 bytes
+
+// 16 bytes per lane straight into LDS: lane x's piece lands at lds_addr + 16 x. The s_nop is the wait state that the instruction
+// needs behind a scalar write of m0; the compiler puts none into inline assembly.
 
 __device__ inline void load_to_lds(const void* src, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_addr) : "memory", "m0");
 }
+// (past the caches: weights that this launch reads once)
+__device__ inline void load_to_lds_nt(const void* src, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" : : "v"(src), "s"(lds_addr) : "memory", "m0");
+}
+template <int N>
+__device__ inline void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
 __device__ __attribute__((aligned(16))) const unsigned kZeroPiece[4] = {0u, 0u, 0u, 0u};
 
-// NW = 4 (17 to 64 rows): four such waves, one on each SIMD, share the step's rows: a slot
-// holds the four waves' weights and one copy of the rows, of which every wave loads a quarter, and
-// a barrier per slot tells a wave that the others' quarters are there. A wave alone reads the rows
-// from L2 once per 32 output columns, more bytes than its weights at 64 rows, and has LDS for one
-// slot on its way; four waves together have it for four (the ring is dynamic shared memory then).
-extern __shared__ __attribute__((aligned(1024))) unsigned char stream_ring[];
+// Up to 32 rows (k a multiple of four, rows on 16 bytes): the weights as a stream. A block has C times 32 output columns and a
+// ring of R slots in LDS; a slot is 32 k (two steps) of the block's rows of W and of 32 rows of A, filled by loads
+// that go from memory straight into LDS (whole 128-byte lines: 8 rows x 32 k an instruction; the 16-byte pieces of a row are
+// exchanged among themselves by the row's number so that the reads spread over the banks). Waves have one task each: C of them
+// multiply, 32 columns each, and split the weights that they multiply, a step's while the one before it is multiplied; C bring
+// the weights; four bring eight rows of A each and split them, once for the block, into one of two buffers. Behind the one barrier
+// of slot j the weights and pieces of slot j + 1 are read into registers and slot j is multiplied; R - 2 slots are on their way. The
+// loops are kept short: between other kernels' launches the instructions come from memory, and 2.7 KB of them less are 0.9 us less.
+//
+// What bounds it: a compute unit has about 32 KB of loads under way (27 GB/s from memory, 84 from L2), so that a stream
+// reaches the memory's rate only if all units pull, and equally much; C is chosen for that. Against the float32 instruction with
+// a wave a block up to 16 rows and four above (us, alone in a graph): the 1.5B shape's gate/up 37 -> 29 at 20 rows, its way down 18.6 -> 14.2,
+// q/k/v 8.5 -> 6.7, the 7B shape's gate/up 134 -> 97 and 106 -> 96 at 8 rows. Steps of few rows, whose kernels are start and end: 1,300 -> 1,275 us at one
+// request of the 1.5B shape (14 layers), 1,333 -> 1,336 at 8, 2,076 -> 1,901 at 4 of the 7B shape (8 layers); with the weights kept in
+// the caches on their way 1,358, 1,388 and 2,040.
+// (Weights straight into the registers that they are multiplied from, a lane's eight k at a time, take twice as long: a line is
+// asked for eight times there, and the lines that a block's waves have under way do not fit the vector cache.)
+constexpr int kRowWaves = 4;
+constexpr int kStreamPiece = 512 + 32, kStreamPlane = 4 * kStreamPiece;       // [8 k][row] of a plane of pieces, off each other's banks
+constexpr int ring_slots(int C) { return C == 3 || C == 4 ? 6 : 5; }
+constexpr int slot_bytes(int C) { return 4096 * (C + 1); }
+constexpr int stream_bytes(int C) { return ring_slots(C) * slot_bytes(C) + 2 * 3 * kStreamPlane; }
+extern __shared__ __attribute__((aligned(1024))) unsigned char stream_lds[];
 
-template <int R, int XR, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_f32_stream_kernel(
+template <int C>
+__global__ __launch_bounds__(64 * (2 * C + kRowWaves)) void gemm_f32_stream_kernel(
     const float* __restrict__ A, size_t lda, const float* __restrict__ W, size_t ldw,
     const void* __restrict__ bias, int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M,
-    int N, int K, int kper) {
-  static_assert(NW == 1 || (NW == 4 && XR >= 32), "four waves share 32 or 64 rows");
-  constexpr int XL = XR / 8 / NW;               // this wave's load instructions for a slot's rows of A
-  constexpr int MT = XR > 32 ? 2 : 1;           // tiles of 32 rows of A
-  constexpr int kSlotBytes = 4096 * NW + XR * 128;
-  constexpr int L = 4 + XL;                     // a wave's load instructions per slot
-  static_assert(L * (R - 2) <= 63, "the wait counter holds 63 loads");
-  __shared__ __attribute__((aligned(1024))) unsigned char own_ring[NW == 1 ? R * kSlotBytes : 16];
-  unsigned char* const ring = NW == 1 ? own_ring : stream_ring;
+    int N, int K, int kper, int chain) {
+  constexpr int R = ring_slots(C), SLOT = slot_bytes(C);
+  unsigned char* const ring = stream_lds;
+  unsigned char* const planes = stream_lds + R * SLOT;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, half = lane >> 5, c = lane & 31;
-  const int n0 = (blockIdx.x * NW + wave) * 32;
   const int kbeg = blockIdx.z * kper;
   K = min(K, kbeg + kper);  // this part's end
   out += blockIdx.z * part_stride;
   if (blockIdx.z) bias = nullptr;  // the bias belongs to one part only
   const int slots = (K - kbeg + kSlotK - 1) / kSlotK;
-
-  // This lane's share of a slot's loads: of load i, the piece that lands at row 8 i + lane / 8,
-  // place lane % 8, which is piece (place ^ swizzle of the row) of the row's 32 k. Columns past
-  // the end read the last one's weights and are not stored; rows of A past M read zeros.
-  const int lr = lane >> 3, lp = lane & 7;
-  const float* wsrc[4];
-  int wk[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 8 * i + lr;
-    wk[i] = 4 * (lp ^ ((r >> 1) & 7));
-    wsrc[i] = W + static_cast<size_t>(min(n0 + r, N - 1)) * ldw + kbeg + wk[i];
-  }
-  const float* xsrc[XL];
-  int xk[XL];
-  bool xrow[XL];
-#pragma unroll
-  for (int i = 0; i < XL; ++i) {
-    const int r = 8 * (NW * i + wave) + lr;  // of the slot's instructions for A, this wave's are wave, NW + wave, ...
-    xk[i] = 4 * (lp ^ ((r >> 1) & 7));
-    xrow[i] = r < M;
-    xsrc[i] = A + static_cast<size_t>(xrow[i] ? r : 0) * lda + kbeg + xk[i];
-  }
   const unsigned mine = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(ring)));
   const float* zero = reinterpret_cast<const float*>(kZeroPiece);
-
+  // A load instruction brings 8 rows: lane x's piece lands at row x / 8, place x % 8, and is piece (place ^ swizzle of the row)
+  // of the row's 32 k. Columns past the end are the last one once more and are not stored; rows of A past M are zeros.
+  const int lr = lane >> 3, lp = lane & 7;
   int fill = 0;  // ring position of the next slot to load
-  auto issue = [&](int j) {
-    const unsigned dst = mine + fill * kSlotBytes;
-    fill = fill + 1 == R ? 0 : fill + 1;
-    const int k0 = kSlotK * j, left = j < slots ? K - kbeg - k0 : 0;  // k of this part from the slot's start on
-#pragma unroll
-    for (int i = 0; i < 4; ++i) load_to_lds(wk[i] < left ? wsrc[i] + k0 : zero, dst + 4096 * wave + 1024 * i);
-#pragma unroll
-    for (int i = 0; i < XL; ++i)
-      load_to_lds(xrow[i] && xk[i] < left ? xsrc[i] + k0 : zero, dst + 4096 * NW + 1024 * (NW * i + wave));
-  };
-  // The slot that this wave's loads have just filled is whole when the other waves' are there too.
-  auto slot_whole = [&]() {
-    if (NW > 1) {
-      asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // and what this wave read of the slot that is filled next
-      __syncthreads();
-    }
-  };
-
-  if constexpr (XR <= 16) {
-    // Sixteen rows or fewer: 16x16x4, whose 16 columns hold the step's rows and whose 16 rows are
-    // output columns, two tiles of them a wave. It takes a weight once for 16 rows where 32x32x2
-    // takes it once for 32, so that a wave gets through its weights in half the time.
-    const int g = lane >> 4, c16 = lane & 15;
-    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    const int xr = XR == 8 ? c16 & 7 : c16;  // eight rows: the instruction's columns 8..15 read them again and are not stored
-    const unsigned char* wpiece0 = ring + c16 * 128;
-    const unsigned char* wpiece1 = ring + (16 + c16) * 128;
-    const unsigned char* xpiece = ring + 4096 + xr * 128;
-    const int swz = (c16 >> 1) & 7, xswz = (xr >> 1) & 7;  // rows c16 and 16 + c16 exchange their pieces alike
-    int at = 0;
-    auto read = [&](f32x4 (&a)[2][2], f32x4 (&b)[2]) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int piece = 4 * t + g;
-        a[0][t] = *reinterpret_cast<const f32x4*>(wpiece0 + at * kSlotBytes + 16 * (piece ^ swz));
-        a[1][t] = *reinterpret_cast<const f32x4*>(wpiece1 + at * kSlotBytes + 16 * (piece ^ swz));
-        b[t] = *reinterpret_cast<const f32x4*>(xpiece + at * kSlotBytes + 16 * (piece ^ xswz));
-      }
-      at = at + 1 == R ? 0 : at + 1;
+  auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  if (wave >= 2 * C) {
+    const int xr = 8 * (wave - 2 * C) + lr, xk = 4 * (lp ^ ((xr >> 1) & 7));
+    const float* const xsrc = A + static_cast<size_t>(xr < M ? xr : 0) * lda + kbeg + xk;
+    auto issue = [&](int j) {
+      const unsigned dst = mine + fill * SLOT + 4096 * C + 1024 * (wave - 2 * C);
+      fill = fill + 1 == R ? 0 : fill + 1;
+      const int k0 = kSlotK * j, left = j < slots ? K - kbeg - k0 : 0;  // k of this part from the slot's start on
+      load_to_lds(xr < M && xk < left ? xsrc + k0 : zero, dst);
     };
+    // Four k of a row a lane, of the rows that this wave has brought: the lane's own piece, and its place among the pieces of eight.
+    const unsigned char* const raw = ring + 4096 * C + 1024 * (wave - 2 * C) + 16 * lane;
+    unsigned char* const dst = planes + (xk >> 3) * kStreamPiece + 16 * xr + 2 * (xk & 4);
+    int at = 0;  // ring position of the next slot whose rows are split
+    auto split_rows = [&](int buf) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(raw + at * SLOT);
+      at = at + 1 == R ? 0 : at + 1;
+      const Pieces p = split8(v, v);
 #pragma unroll
+      for (int s = 0; s < 3; ++s)
+        *reinterpret_cast<uint2*>(dst + (3 * buf + s) * kStreamPlane) = make_uint2(p.p[s][0], p.p[s][1]);
+    };
+#pragma unroll 1
     for (int j = 0; j < R - 1; ++j) issue(j);
-    f32x4 a[2][2], b[2], an[2][2], bn[2];
-    wait_loads<L * (R - 2)>();
-    read(a, b);
+    wait_loads<R - 2>();
+    split_rows(0);
+    barrier();
     for (int j = 0; j < slots; ++j) {
-      issue(j + R - 1);
-      wait_loads<L * (R - 2)>();
-      read(an, bn);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if (kSlotK * j + BK * t >= K - kbeg) break;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][t][i], b[t][i], acc[u], 0, 0, 0);
-      }
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        a[0][t] = an[0][t];
-        a[1][t] = an[1][t];
-        b[t] = bn[t];
-      }
+      issue(j + R - 1);         // into the position of slot j - 1
+      wait_loads<R - 2>();      // slot j + 1 is there (loads finish in the order of issue)
+      split_rows((j + 1) & 1);  // where the multiplying waves have read those of slot j - 1
+      barrier();
     }
-    wait_loads<0>();
-    // acc[u][j]: output column n = 16 u + 4 g + j, output row m = c16.
-    if (c16 >= M || c16 >= XR) return;
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int n = n0 + 16 * u + 4 * g;
-      if (n >= N) continue;
-      float v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[j] = acc[u][j];
-        if (bias && n + j < N) v[j] += load_as_float(bias, bias_dt, n + j);
-      }
-      float* dst = out + static_cast<size_t>(c16) * ldo + n;
-      if (n + 3 < N && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-      } else {
-        for (int j = 0; j < 4 && n + j < N; ++j) dst[j] = v[j];
-      }
-    }
-  } else {
-  f32x16 acc[MT];
-#pragma unroll
-  for (int u = 0; u < MT; ++u)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[u][i] = 0.f;
-  const unsigned char* wpiece = ring + 4096 * wave + c * 128;
-  const unsigned char* xpiece = ring + 4096 * NW + c * 128;
-  const int swz = (c >> 1) & 7;  // rows c and 32 + c exchange their pieces alike
-  int at = 0;  // ring position of the next slot to read
-  auto read = [&](f32x4 (&a)[2][2], f32x4 (&b)[MT][2][2]) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int piece = 4 * t + half + 2 * h;
-        a[t][h] = *reinterpret_cast<const f32x4*>(wpiece + at * kSlotBytes + 16 * (piece ^ swz));
-#pragma unroll
-        for (int u = 0; u < MT; ++u) {
-          b[u][t][h] = *reinterpret_cast<const f32x4*>(xpiece + at * kSlotBytes + 4096 * u + 16 * (piece ^ swz));
-        }
-      }
-    at = at + 1 == R ? 0 : at + 1;
-  };
-
-  // Slot j + 1 is read from LDS while slot j is multiplied, so of the R slots of the ring one is
-  // in registers, one being read and R - 2 on their way.
-#pragma unroll
-  for (int j = 0; j < R - 1; ++j) issue(j);
-  f32x4 a[2][2], b[MT][2][2], an[2][2], bn[MT][2][2];
-  wait_loads<L * (R - 2)>();  // loads finish in the order of issue: slot 0 is there
-  slot_whole();
-  read(a, b);
-  for (int j = 0; j < slots; ++j) {
-    issue(j + R - 1);            // into the position of slot j - 1, read a turn ago (by every wave: the barrier since)
-    wait_loads<L * (R - 2)>();   // slot j + 1 is there
-    slot_whole();
-    read(an, bn);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if (kSlotK * j + BK * t >= K - kbeg) break;  // a part that ends with half a slot
-#pragma unroll
-      for (int s = 0; s < 8; ++s)
-#pragma unroll
-        for (int u = 0; u < MT; ++u)
-          acc[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][s & 1][s >> 1], b[u][t][s & 1][s >> 1], acc[u], 0, 0, 0);
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        a[t][h] = an[t][h];
-#pragma unroll
-        for (int u = 0; u < MT; ++u) b[u][t][h] = bn[u][t][h];
-      }
+    wait_loads<0>();  // the loads past the end
+    return;
   }
-  wait_loads<0>();  // the loads past the end
-
-  // acc[u][4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = 32 u + tile column c.
-#pragma unroll
-  for (int u = 0; u < MT; ++u) {
-    const int m = 32 * u + c;
-    if (m >= M) continue;
+  if (wave >= C) {
+    const int load = wave - C;
+    const float* wsrc[4];
+    int wk[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int n = n0 + 8 * i + 4 * half;
-      if (n >= N) continue;
-      float v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        v[j] = acc[u][4 * i + j];
-        if (bias && n + j < N) v[j] += load_as_float(bias, bias_dt, n + j);
-      }
-      float* dst = out + static_cast<size_t>(m) * ldo + n;
-      if (n + 3 < N && (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-      } else {
-        for (int j = 0; j < 4 && n + j < N; ++j) dst[j] = v[j];
-      }
+      const int r = 8 * i + lr;
+      wk[i] = 4 * (lp ^ ((r >> 1) & 7));
+      wsrc[i] = W + static_cast<size_t>(min((static_cast<int>(blockIdx.x) * C + load) * 32 + r, N - 1)) * ldw + kbeg + wk[i];
     }
+    auto issue = [&](int j) {
+      const unsigned dst = mine + fill * SLOT + 4096 * load;
+      fill = fill + 1 == R ? 0 : fill + 1;
+      const int k0 = kSlotK * j, left = j < slots ? K - kbeg - k0 : 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load_to_lds_nt(wk[i] < left ? wsrc[i] + k0 : zero, dst + 1024 * i);
+    };
+#pragma unroll 1
+    for (int j = 0; j < R - 1; ++j) issue(j);
+    wait_loads<4 * (R - 2)>();
+    barrier();
+    for (int j = 0; j < slots; ++j) {
+      issue(j + R - 1);           // into the position of slot j - 1
+      wait_loads<4 * (R - 2)>();  // slot j + 1 is there
+      barrier();
+    }
+    wait_loads<0>();  // the loads past the end
+    return;
   }
+  const int n0 = (blockIdx.x * C + wave) * 32;
+  const unsigned char* const wpiece = ring + 4096 * wave + c * 128;
+  const unsigned char* const xpiece = planes + half * kStreamPiece + 16 * c;
+  const int swz = (c >> 1) & 7;
+  int at = 0;  // ring position of the next slot whose weights are read
+  f32x4 w[2][2];
+  u32x4 x[2][3];
+  auto read_w = [&](int t) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[t][h] = *reinterpret_cast<const f32x4*>(wpiece + at * SLOT + 16 * ((4 * t + 2 * half + h) ^ swz));
+  };
+  auto read_x = [&](int t, int buf) {
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      x[t][s] = *reinterpret_cast<const u32x4*>(xpiece + (3 * buf + s) * kStreamPlane + 2 * t * kStreamPiece);
+  };
+  f32x16 acc, total;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = total[i] = 0.f;
+  auto end_chain = [&]() {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      total[i] += acc[i];
+      acc[i] = 0.f;
+    }
+  };
+  auto interleave = [] {
+#pragma unroll
+    for (int s = 0; s < kTerms; ++s) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // a matrix instruction,
+      __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);  // eight vector instructions
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  barrier();
+  read_w(0);
+  read_w(1);
+  read_x(0, 0);
+  read_x(1, 0);
+  Pieces p[2];  // of the two steps' weights
+  p[0] = split8(w[0][0], w[0][1]);
+#pragma unroll 1
+  for (int j = 0; j < slots; ++j) {
+    barrier();  // the weights and pieces of the next slot are there
+    at = at + 1 == R ? 0 : at + 1;
+    p[1] = split8(w[1][0], w[1][1]);
+#pragma unroll
+    for (int s = 0; s < kTerms; ++s) acc = multiply(p[0].p[kTermW[s]], x[0][kTermA[s]], acc);
+    interleave();
+    read_w(0);
+    read_x(0, (j + 1) & 1);
+    read_w(1);
+    p[0] = split8(w[0][0], w[0][1]);
+#pragma unroll
+    for (int s = 0; s < kTerms; ++s) acc = multiply(p[1].p[kTermW[s]], x[1][kTermA[s]], acc);
+    interleave();
+    read_x(1, (j + 1) & 1);
+    if (chain == kChain && j % (kChain / 2) == kChain / 2 - 1) end_chain();
   }
+  end_chain();
+
+  // total[4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = tile column c.
+  const bool rows_of_16 = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+  bool bad = false;
+  if (c < M) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, out + static_cast<size_t>(c) * ldo,
+                    rows_of_16, n0 + 4 * half + 8 * i, N);
+  }
+  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, c, 1, M, n0 + 4 * half, 1, N, K - kbeg);
 }
 
-}  // namespace
+template <int C>
+bool launch_stream(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
+                   int M, int N, int K, int kper, int parts, int chain, hipStream_t stream) {
+  static bool asked[kMaxDevices] = {};  // for that much LDS a block, once per device
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
+  if (!asked[dev]) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_stream_kernel<C>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            stream_bytes(C)) != hipSuccess)
+      return false;
+    asked[dev] = true;
+  }
+  hipLaunchKernelGGL(gemm_f32_stream_kernel<C>, dim3((N + 32 * C - 1) / (32 * C), 1, parts), dim3(64 * (2 * C + kRowWaves)), stream_bytes(C),
+                     stream, A, static_cast<size_t>(lda), W, static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),
+                     static_cast<size_t>(part_stride), M, N, K, kper, chain);
+  return true;
+}
 
-namespace {
+// How many times 32 columns a block has: the least time of the busiest unit, where a block costs half as much as 32 columns for its
+// start and its rows of A. (The 1.5B shape's head: 239 us with 32 columns a block, which leave the units least unequal.)
+int stream_columns(int N, int parts) {
+  int best = 1;
+  long least = 0;
+  for (int c = 1; c <= 5; ++c) {
+    const long blocks = static_cast<long>((N + 32 * c - 1) / (32 * c)) * parts, most = (blocks + compute_units() - 1) / compute_units() * (2 * c + 1);
+    if (c == 1 || most <= least) least = most, best = c;
+  }
+  return best;
+}
 
-// Tiles whose rows are few where the step's are; beyond 64 rows the size with the least work on the busiest unit (a block of
-// several shares its matrix cores' time, so that is its tiles), smaller ones costing a little more for the same.
+// The tile with the least work on the busiest unit (a block of two or three shares its matrix cores' time, so that is its
+// tiles), smaller ones costing more for the same: their operands come from LDS more often.
 struct TileRows {
   int bm, bn;
   double cost;
 };
-constexpr TileRows kTiles[4] = {{128, 128, 0.98}, {64, 128, 1.0}, {96, 128, 1.03}, {64, 64, 1.07}};
-constexpr double kMacsPerUs = 2.8e5;    // of a compute unit
+constexpr int kSizes = 3;
+constexpr TileRows kTiles[kSizes] = {{128, 128, 1.0}, {64, 128, 1.1}, {64, 64, 1.5}};
+constexpr double kMacsPerUs = 3.9e5;    // of a compute unit
 constexpr double kBytesPerUs = 5e6;     // of memory, both ways
-constexpr double kFillUs = 0.006;       // a k of a block's chain before the unit's other blocks hide it
+constexpr double kFillUs = 0.004;       // a k of a block's chain before the unit's other blocks hide it
 
 // The tile size for so many rows and `parts` parts of kper, and what it takes in microseconds.
 int best_tile(int M, int N, int kper, int parts, double* us) {
   int best = 0;
   double least = 1e300;
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < kSizes; ++i) {
     const long tiles = static_cast<long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((N + kTiles[i].bn - 1) / kTiles[i].bn) * parts;
     const double work = kTiles[i].cost * kTiles[i].bm * kTiles[i].bn * kper * ((tiles + compute_units() - 1) / compute_units());
     if (work < least) least = work, best = i;
@@ -615,25 +637,23 @@ bool takes_tiles(int M, int N, int K, long lda, long ldw) {
          static_cast<long>((M + 31) / 32) * ((N + 63) / 64) < (1L << 24);
 }
 
-template <bool WHOLE>
+// Chains of `chain` steps; `whole`: a block walks all of k.
 void launch_tiles(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
-                  int M, int N, int K, int kper, int ksplit, hipStream_t stream) {
-  const int parts = WHOLE ? 1 : ksplit;
+                  int M, int N, int K, int kper, int parts, int chain, hipStream_t stream) {
   const auto tile = [&](auto kernel, int bm, int bn) {
     const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * nt * parts), dim3(256), 0, stream, A, lda, W, ldw, bias, bias_dt, out,
-                       static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, mt, nt);
+                       static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, chain, mt, nt);
   };
-  const int best = best_tile(M, N, WHOLE ? K : kper, parts, nullptr);
-  if (M <= 32) tile(gemm_f32_tile_kernel<32, 128, 1, 4, 4, 1, WHOLE>, 32, 128);
-  else if (M <= 64) tile(gemm_f32_tile_kernel<64, 64, 2, 2, 3, 1, WHOLE>, 64, 64);
-  else if (best == 0) tile(gemm_f32_tile_kernel<128, 128, 2, 2, 2, 2, WHOLE>, 128, 128);
-  else if (best == 1) tile(gemm_f32_tile_kernel<64, 128, 2, 2, 2, 3, WHOLE>, 64, 128);
-  else if (best == 2) tile(gemm_f32_tile_kernel<96, 128, 1, 4, 2, 2, WHOLE>, 96, 128);
-  else tile(gemm_f32_tile_kernel<64, 64, 2, 2, 2, 5, WHOLE>, 64, 64);
+  const int best = best_tile(M, N, kper, parts, nullptr);
+  if (best == 0) tile(gemm_f32_tile_kernel<128, 128, 2, 2, 1, 2>, 128, 128);
+  else if (best == 1) tile(gemm_f32_tile_kernel<64, 128, 2, 2, 2, 2>, 64, 128);
+  else tile(gemm_f32_tile_kernel<64, 64, 2, 2, 2, 3>, 64, 64);
 }
 
 int part_of(int K, int ksplit) { return ((K + ksplit - 1) / ksplit + BK - 1) / BK * BK; }
+// Steps of a chain: a part, or less where there is one part only.
+int chain_of(int K, int ksplit) { return ksplit > 1 ? part_of(K, ksplit) / BK : kChain; }
 
 }  // namespace
 
@@ -655,7 +675,7 @@ extern "C" int pyre_gemm_f32_whole(const float* A, long lda, const float* W, lon
                    reinterpret_cast<uintptr_t>(W) % 16 == 0,
                "gemm_f32_whole: M=%d (more than 16) N=%d K=%d (a multiple of 16) lda=%ld ldw=%ld (of 4) are not supported", M, N, K, lda, ldw);
   PYRE_REQUIRE(ksplit >= 1 && ksplit <= 64 && static_cast<long>(ksplit - 1) * part_of(K, ksplit) < K, "gemm_f32_whole: ksplit=%d", ksplit);
-  launch_tiles<true>(A, lda, W, ldw, nullptr, 0, out, ldo, 0, M, N, K, part_of(K, ksplit), ksplit, stream);
+  launch_tiles(A, lda, W, ldw, nullptr, 0, out, ldo, 0, M, N, K, K, 1, chain_of(K, ksplit), stream);
   return check_launch("gemm_f32_whole");
 }
 
@@ -673,50 +693,29 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
   // 16-byte loads along k need rows that start on 16 bytes
   const int vec_ok = lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(W) % 16 == 0;
-  if (vec_ok && takes_tiles(M, N, K, lda, ldw)) {
-    launch_tiles<false>(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, stream);
-  } else if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows: the weights as a stream
-    const dim3 grid((N + 31) / 32, 1, ksplit);
-#define PYRE_STREAM(R, XR)                                                                                         \
-  hipLaunchKernelGGL((gemm_f32_stream_kernel<R, XR, 1>), grid, dim3(64), 0, stream, A, static_cast<size_t>(lda), W, \
-                     static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),                       \
-                     static_cast<size_t>(part_stride), M, N, K, kper)
-// four waves a block, the ring in dynamic shared memory (asked for once per device and kernel)
-#define PYRE_STREAM4(R, XR)                                                                                        \
-  do {                                                                                                             \
-    constexpr int kBytes = (R) * (4096 * 4 + (XR) * 128);                                                          \
-    static bool asked[kMaxDevices] = {};                                                                           \
-    int dev = 0;                                                                                                   \
-    PYRE_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices, "gemm_f32: no device");         \
-    if (!asked[dev]) {                                                                                             \
-      PYRE_REQUIRE(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_stream_kernel<R, XR, 4>),           \
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kBytes) == hipSuccess,          \
-                   "gemm_f32: %d bytes of LDS a block are refused", kBytes);                                       \
-      asked[dev] = true;                                                                                           \
-    }                                                                                                              \
-    hipLaunchKernelGGL((gemm_f32_stream_kernel<R, XR, 4>), dim3((N + 127) / 128, 1, ksplit), dim3(256), kBytes,    \
-                       stream, A, static_cast<size_t>(lda), W, static_cast<size_t>(ldw), bias, bias_dt, out,       \
-                       static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper);                 \
-  } while (0)
-    if (M <= 8) PYRE_STREAM(4, 8);
-    else if (M <= 16) PYRE_STREAM(4, 16);
-    else if (M <= 32 && N >= 128) PYRE_STREAM4(7, 32);
-    else if (M <= 32) PYRE_STREAM(4, 32);
-    else if (N >= 128) PYRE_STREAM4(6, 64);
-    else PYRE_STREAM(3, 64);
-#undef PYRE_STREAM
-#undef PYRE_STREAM4
+  const int chain = chain_of(K, ksplit);
+  if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows
+    const auto launch = [&](auto f) { return f(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, stream); };
+    const int c = stream_columns(N, ksplit);
+    PYRE_REQUIRE(c == 1   ? launch(launch_stream<1>)
+                 : c == 2 ? launch(launch_stream<2>)
+                 : c == 3 ? launch(launch_stream<3>)
+                 : c == 4 ? launch(launch_stream<4>)
+                          : launch(launch_stream<5>),
+                 "gemm_f32: no device, or too little LDS");
+  } else if (vec_ok && takes_tiles(M, N, K, lda, ldw)) {
+    launch_tiles(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, stream);
   } else if (M <= 32) {  // four waves side by side along n
     const dim3 grid((N + 127) / 128, (M + 31) / 32, ksplit);
     hipLaunchKernelGGL((gemm_f32_mfma_kernel<4, 1, 1, 1>), grid, dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
                        static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),
-                       static_cast<size_t>(part_stride), M, N, K, kper, vec_ok);
+                       static_cast<size_t>(part_stride), M, N, K, kper, chain, vec_ok);
   } else {
     const dim3 grid((N + 127) / 128, (M + 127) / 128, ksplit);
     PYRE_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d too large for one launch", M);
     hipLaunchKernelGGL((gemm_f32_mfma_kernel<2, 2, 2, 2>), grid, dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
                        static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),
-                       static_cast<size_t>(part_stride), M, N, K, kper, vec_ok);
+                       static_cast<size_t>(part_stride), M, N, K, kper, chain, vec_ok);
   }
   return check_launch("gemm_f32");
 }

@@ -1,0 +1,56 @@
+"""The 32-bit path's products, made of bfloat16 pieces: how far they are from 64 bits, and numbers whose pieces no bfloat16 holds."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+#: few rows, tiles of both sizes; with k in one part and in several, with rows that start on 16 bytes and that do not
+FORMS = [(m, n, k, ks, off) for m in (1, 32, 33, 300) for n, k, ks in ((33, 48, 1), (1537, 1040, 1), (200, 1536, 3)) for off in (0, 1)]
+
+
+def operands(m, n, k, off, scale=1.0):
+    g = torch.Generator().manual_seed(m + n + k)
+    a = torch.zeros(m, k + 4, device=DEV)
+    a[:, off:off + k] = torch.randn(m, k, generator=g).to(DEV) * scale
+    return a[:, off:off + k], (torch.randn(n, k, generator=g) * 0.02).to(DEV)
+
+
+@pytest.mark.parametrize("m,n,k,ks,off", FORMS)
+def test_no_further_from_64_bits_than_a_chain_of_fused_multiply_adds(m, n, k, ks, off):
+    from pyre_amd.hip import ops
+
+    a, w = operands(m, n, k, off, scale=3.0)
+    out, chain = torch.full((ks, m, n), float("nan"), device=DEV), torch.empty(m, n, device=DEV)
+    ops.gemm_f32(a, w, None, out if ks > 1 else out[0], m, ks)
+    ops.gemm_generic(a, w, None, chain, m)
+    want = a.double() @ w.double().T
+    err, err_chain = ((x.double() - want).square().mean().sqrt() for x in (out.sum(0), chain))
+    # what is left out of a product is below 2^-26 of it, the chain's own roundings are 2^-25 of the sum each; a few dozen
+    # elements (one row) scatter by some ten per cent, and a sum of 48 has few roundings of either kind
+    assert float(err) <= 1.1 * float(err_chain) + 2.0 ** -26 * float(want.square().mean().sqrt())
+
+
+@pytest.mark.parametrize("m,n,k,ks,off", FORMS)
+def test_infinities_and_the_largest_numbers(m, n, k, ks, off):
+    """As float32 arithmetic has them: a row with an infinity, one with a NaN, one with the largest number (whose upper piece
+    would round to infinity) times weights that keep its products finite."""
+    from pyre_amd.hip import ops
+
+    a, w = operands(m, n, k, off)
+    big = torch.finfo(torch.float32).max
+    for value, row in ((float("inf"), 0), (float("nan"), m // 2), (-float("inf"), m - 1), (big, m - 1)):
+        b = a.clone() if off == 0 else torch.nn.functional.pad(a, (off, 0))[:, off:]
+        b[row, k // 2] = value
+        out = torch.full((ks, m, n), float("nan"), device=DEV)
+        ops.gemm_f32(b, w, None, out if ks > 1 else out[0], m, ks)
+        got, want = out.double().sum(0), b.double() @ w.double().T
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()), (value, row)
+        fine = want.isfinite()
+        assert torch.equal(got[~fine & ~want.isnan()], want[~fine & ~want.isnan()])
+        # roundings of 2^-24 of the largest partial sum: the row's scale is that of its largest product
+        scale = (b.double().abs() @ w.double().abs().T)[fine]
+        assert bool(((got - want)[fine].abs() <= 2.0 ** -22 * scale + 1e-30).all()), (value, row)
