@@ -90,6 +90,7 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
   constexpr int NT = 64 * G * SL, TPR = NT / kKeys;     // threads that bring one key's row
   constexpr int E = 16 / sizeof(T);                      // elements of a 16-byte unit
   constexpr int KI = (2 * KQ * SL + TPR - 1) / TPR;      // units a thread brings of a row
+  constexpr bool kAhead = sizeof(T) == 2 && !SINGLE && SL > 1;  // the loop that is a chunk's score ahead
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const int steps = (a.dk + 2 * E - 1) / (2 * E), ldk = 2 * E * steps + E;
   T* Ks = reinterpret_cast<T*>(lds_raw);                                   // [1 or 2][32][ldk], then slack
@@ -100,6 +101,7 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
   int* tab_s = reinterpret_cast<int*>(Ps + (SL > 1 ? G * weight_bytes<T>() : 0));
   __shared__ int slot_s[kRing][kKeys];
   __shared__ float row_s[G * SL][32];  // the waves' maxima of their keys, per query; at the end their weights
+  __shared__ int jump_s;               // the last chunk (from 1 on) whose scores rise far above those before
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int g = wave / SL, sl = wave % SL;
@@ -196,8 +198,7 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
 
   // A chunk's rows go from the registers to LDS, and the next one's are asked for at once: they have a whole chunk's work to
   // arrive in (asked for at a chunk's start they had its score and softmax: 120 us instead of 116 for a prompt's last 952 of
-  // 3,000 tokens, 12 heads, rows of 576, a window of 1,024, 166 instead of 163 for its first 2,048). What is left, 3.5 us a
-  // chunk with 1.1 us of products, is three barriers a chunk that the two waves of a SIMD wait at together.
+  // 3,000 tokens, 12 heads, rows of 576, a window of 1,024, 166 instead of 163 for its first 2,048).
   auto bring = [&](int it) {
     if (it >= n_chunks) return;
     stash(it);
@@ -210,7 +211,111 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
   float m = -INFINITY, l = 0.f;
+  // This wave's part of the scores of a chunk: element i is of key 8 (i / 4) + 4 h + i % 4, query c.
+  auto score = [&](const T* K) {
+    // four steps' keys at a time, in two chains of sums; steps behind the row's last one meet a query of zeros
+    const T* krow = K + c * ldk + E * h;
+    f32x16 s, s2;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = s2[i] = 0.f;
+#pragma unroll
+    for (int st0 = 0; st0 < KQ; st0 += 4) {
+      if (!kAhead && st0 * SL + sl >= steps) continue;
+      uint4 k4[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (st0 + u < KQ) k4[u] = *reinterpret_cast<const uint4*>(krow + 2 * E * min((st0 + u) * SL + sl, steps - 1));
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (st0 + u < KQ) {
+          f32x16& sum = u & 1 ? s2 : s;
+          if constexpr (sizeof(T) == 2) {
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, k4[u]), __builtin_bit_cast(bf16x8, qf[st0 + u]), sum, 0, 0, 0);
+          } else {
+            const f32x4 kf = __builtin_bit_cast(f32x4, k4[u]), qq = __builtin_bit_cast(f32x4, qf[st0 + u]);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[v], qq[v], sum, 0, 0, 0);
+          }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] += s2[i];
+    return s;
+  };
+  // The waves of a row tile hand their parts of the scores round.
+  auto hand_round = [&](const f32x16& s) {
+    float* mine = sred + wave * 1024 + 4 * lane;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(mine + 256 * j) = f32x4{s[4 * j], s[4 * j + 1], s[4 * j + 2], s[4 * j + 3]};
+  };
+  // Of SL waves each turns EW = 16 / SL of a chunk's scores into weights: the parts of its own ones are added up (in order),
+  // scaled and masked; their maximum over both halves of the wave.
+  constexpr int EW = 16 / SL;
+  auto take = [&](const f32x16& s, int key0, float (&w)[EW]) {
+    float mx = -INFINITY;
+    if (SL > 1) {
+      const float* base = sred + g * SL * 1024 + 4 * lane + 256 * (EW / 4) * sl;
+#pragma unroll
+      for (int j = 0; j < EW / 4; ++j) {
+        f32x4 t = *reinterpret_cast<const f32x4*>(base + 256 * j);
+#pragma unroll
+        for (int o2 = 1; o2 < SL; ++o2) t += *reinterpret_cast<const f32x4*>(base + 1024 * o2 + 256 * j);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[4 * j + u] = t[u];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < EW; ++i) w[i] = s[i];
+    }
+    if (key0 >= lo_last && key0 + kKeys - 1 <= pos0) {
+#pragma unroll
+      for (int i = 0; i < EW; ++i) w[i] *= a.scale2, mx = fmaxf(mx, w[i]);
+    } else {
+      const unsigned seen = static_cast<unsigned>(hi - lo), first = static_cast<unsigned>(key0 + 8 * (EW / 4) * sl + 4 * h - lo);
+#pragma unroll
+      for (int i = 0; i < EW; ++i) {
+        w[i] = first + 8 * (i >> 2) + (i & 3) <= seen ? w[i] * a.scale2 : -INFINITY;
+        mx = fmaxf(mx, w[i]);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    return mx;
+  };
+  auto store_pieces = [&](const uint32_t (&w1)[EW / 2], const uint32_t (&w2)[EW / 2], const uint32_t (&w3)[EW / 2]) {
+#pragma unroll
+    for (int j = 0; j < EW / 4; ++j) {
+      const int quad = sl * (EW / 4) + j;  // elements 4 quad .. 4 quad + 3
+      unsigned char* dst = Ps + g * weight_bytes<T>() + (quad >> 1) * 1024 + 16 * lane + 8 * (quad & 1);
+      *reinterpret_cast<uint2*>(dst) = uint2{w1[2 * j], w1[2 * j + 1]};
+      *reinterpret_cast<uint2*>(dst + 2048) = uint2{w2[2 * j], w2[2 * j + 1]};
+      *reinterpret_cast<uint2*>(dst + 4096) = uint2{w3[2 * j], w3[2 * j + 1]};
+    }
+  };
+  auto read_pieces = [&](int b, uint4 (&pieces)[3][2]) {
+#pragma unroll
+    for (int pc = 0; pc < 3; ++pc) pieces[pc][b] = *reinterpret_cast<const uint4*>(Ps + g * weight_bytes<T>() + pc * 2048 + b * 1024 + 16 * lane);
+  };
+  // Keys 16 b .. 16 b + 15 of a chunk; the lane's eight are 16 b + 4 h + u and 16 b + 8 + 4 h + u. All columns' values first,
+  // then the pieces in turn, the smallest first: neighbouring products add to different sums (columns behind the last tile
+  // repeat it, and nobody reads their sums).
+  auto add_values = [&](const T* K, int b, const uint4 (&pieces)[3][2]) {
+    const int j16 = lane & 15, col16 = 16 * ((lane >> 4) & 1);
+    const bf16* vrow = reinterpret_cast<const bf16*>(K) + (16 * b + 4 * h + (j16 >> 2)) * ldk + col16 + 4 * (j16 & 3);
+    bf16x8 v8[NVT];
+#pragma unroll
+    for (int dt = 0; dt < NVT; ++dt) {
+      const int d0 = 32 * min(sl * NVT + dt, last_tile);
+      const uint2 v0 = read_transposed(vrow + d0), v1 = read_transposed(vrow + 8 * ldk + d0);
+      v8[dt] = __builtin_bit_cast(bf16x8, uint4{v0.x, v0.y, v1.x, v1.y});
+    }
+#pragma unroll
+    for (int pc = 2; pc >= 0; --pc)
+#pragma unroll
+      for (int dt = 0; dt < NVT; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v8[dt], __builtin_bit_cast(bf16x8, pieces[pc][b]), o[dt], 0, 0, 0);
+  };
 
+  if (tid == 0) jump_s = 0;
   if (tid < kKeys) {
     slot_s[0][tid] = slot_of(chunk0 * kKeys + tid);
     slot_s[1][tid] = slot_of((chunk0 + 1) * kKeys + tid);
@@ -219,82 +324,105 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
   __syncthreads();
   ask(0);
   stash(0);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the queries are there on every way, and no wait for them comes behind the rows asked for ahead
   if (n_chunks > 1) ask(1);
   __syncthreads();
+  // Row tiles that waves share, with both chunks in LDS: the score of chunk it + 1 is made beside the second product of chunk it,
+  // so that a chunk has one stretch of products and one of handing round, a barrier behind each. What bounds it are the products
+  // (33 instructions of 32 cycles a wave and chunk, two waves a SIMD: 2,100 cycles) and the handing round's latencies between. Against three
+  // barriers a chunk, the maxima going round before the weights are made (us for a prompt's first 2,048 and last 952 tokens of
+  // 3,000, 12 heads, rows of 576, a window of 1,024): 163 -> 154 and 116 -> 102 us.
+  //
+  // A chunk's weights are made against the maximum of the chunks before it, which needs no barrier of its own; a reference
+  // other than the maximum scales weights and sums alike. Where a query's scores rise by more than 2^kJump over it (as in the
+  // first chunk that it sees), its weights are made once more against the new maximum: all waves of the block see the flag behind the barrier.
+  if constexpr (kAhead) {
+    constexpr float kJump = 60.f;
+    float alpha = 1.f;  // what the sums so far are to be multiplied with
+    if (active) hand_round(score(Ks));
+    lds_barrier();
+    for (int it = 0; it < n_chunks; ++it) {
+      const int key0 = (chunk0 + it) * kKeys;
+      const T* K = Ks + (it & 1) * buffer;
+      if (tid < kKeys && it + 3 < n_chunks) slot_s[(it + 3) % kRing][tid] = slot_of(key0 + 3 * kKeys + tid);
+      float w[EW], sum = 0.f;
+      auto weigh = [&](float reference) {
+        const float m_use = reference == -INFINITY ? 0.f : reference;
+        uint32_t w1[EW / 2], w2[EW / 2], w3[EW / 2];
+        sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < EW / 2; ++u) {
+          const float p0 = exp2_hw(w[2 * u] - m_use), p1 = exp2_hw(w[2 * u + 1] - m_use);
+          sum += p0;
+          sum += p1;
+          split_pair(p0, p1, w1[u], w2[u], w3[u]);
+        }
+        store_pieces(w1, w2, w3);
+      };
+      if (active) {
+        const float mx = take(f32x16{}, key0, w);
+        if (h == 0) row_s[wave][c] = mx;
+        if (__ballot(mx > m + kJump) && lane == 0) jump_s = it + 1;
+        weigh(m);
+      }
+      bring(it + 1);  // into the buffer whose last readers, of the chunk before, have passed the barrier above
+      lds_barrier();
+      float top = -INFINITY;
+      if (active)
+#pragma unroll
+        for (int o2 = 0; o2 < SL; ++o2) top = fmaxf(top, row_s[g * SL + o2][c]);
+      if (jump_s == it + 1) {
+        if (active) {
+          const float reference = top > m + kJump ? top : m;
+          if (reference != m) alpha *= exp2_hw(m - reference), l *= exp2_hw(m - reference);
+          m = reference;
+          weigh(m);
+        }
+        lds_barrier();
+      }
+      if (active) {
+        if (__ballot(alpha != 1.f))
+#pragma unroll
+          for (int dt = 0; dt < NVT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+        l += sum;
+        // the reference of the next chunk
+        const float next = fmaxf(m, top);
+        alpha = next == m ? 1.f : exp2_hw(m - next);
+        l *= alpha;
+        m = next;
+        uint4 pieces[3][2];
+        const f32x16 s = score(Ks + ((it + 1) & 1) * buffer);  // (behind the last chunk: of whatever lies there, for nobody)
+        read_pieces(0, pieces);
+        read_pieces(1, pieces);
+        add_values(K, 0, pieces);
+        hand_round(s);
+        add_values(K, 1, pieces);
+      }
+      lds_barrier();
+    }
+    if (__ballot(alpha != 1.f))
+#pragma unroll
+      for (int dt = 0; dt < NVT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+  } else
   for (int it = 0; it < n_chunks; ++it) {
     const int key0 = (chunk0 + it) * kKeys;
     const T* K = Ks + (a.two_buffers ? (it & 1) * buffer : 0);
     if (tid < kKeys && it + 3 < n_chunks) slot_s[(it + 3) % kRing][tid] = slot_of(key0 + 3 * kKeys + tid);
 
     f32x16 s;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.f;
     if (active) {
-      // four steps' keys at a time, in two chains of sums; steps behind the row's last one meet a query of zeros
-      const T* krow = K + c * ldk + E * h;
-      f32x16 s2;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s2[i] = 0.f;
-#pragma unroll
-      for (int st0 = 0; st0 < KQ; st0 += 4) {
-        if (st0 * SL + sl >= steps) continue;
-        uint4 k4[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (st0 + u < KQ) k4[u] = *reinterpret_cast<const uint4*>(krow + 2 * E * min((st0 + u) * SL + sl, steps - 1));
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (st0 + u < KQ) {
-            f32x16& sum = u & 1 ? s2 : s;
-            if constexpr (sizeof(T) == 2) {
-              sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, k4[u]), __builtin_bit_cast(bf16x8, qf[st0 + u]), sum, 0, 0, 0);
-            } else {
-              const f32x4 kf = __builtin_bit_cast(f32x4, k4[u]), qq = __builtin_bit_cast(f32x4, qf[st0 + u]);
-#pragma unroll
-              for (int v = 0; v < 4; ++v) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[v], qq[v], sum, 0, 0, 0);
-            }
-          }
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] += s2[i];
-      if (SL > 1) {
-        float* mine = sred + wave * 1024 + 4 * lane;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(mine + 256 * j) = f32x4{s[4 * j], s[4 * j + 1], s[4 * j + 2], s[4 * j + 3]};
-      }
+      s = score(K);
+      if (SL > 1) hand_round(s);
     }
-    // Element i of s: key key0 + 8 (i / 4) + 4 h + i % 4, query c. Of SL waves each turns 16 / SL of them into weights:
-    // the parts of its own ones are added up (in order), the maxima and then the weights go round through LDS.
-    constexpr int EW = 16 / SL;
+    // the maxima and then the weights go round through LDS
     if (SL > 1) lds_barrier();
     float w[EW], mx = -INFINITY;
     if (active) {
-      if (SL > 1) {
-        const float* base = sred + g * SL * 1024 + 4 * lane + 256 * (EW / 4) * sl;
-#pragma unroll
-        for (int j = 0; j < EW / 4; ++j) {
-          f32x4 t = *reinterpret_cast<const f32x4*>(base + 256 * j);
-#pragma unroll
-          for (int o2 = 1; o2 < SL; ++o2) t += *reinterpret_cast<const f32x4*>(base + 1024 * o2 + 256 * j);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) w[4 * j + u] = t[u];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < EW; ++i) w[i] = s[i];
-      }
-      if (key0 >= lo_last && key0 + kKeys - 1 <= pos0) {
-#pragma unroll
-        for (int i = 0; i < EW; ++i) w[i] *= a.scale2, mx = fmaxf(mx, w[i]);
-      } else {
-        const unsigned seen = static_cast<unsigned>(hi - lo), first = static_cast<unsigned>(key0 + 8 * (EW / 4) * sl + 4 * h - lo);
-#pragma unroll
-        for (int i = 0; i < EW; ++i) {
-          w[i] = first + 8 * (i >> 2) + (i & 3) <= seen ? w[i] * a.scale2 : -INFINITY;
-          mx = fmaxf(mx, w[i]);
-        }
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = take(s, key0, w);
       if (SL > 1 && h == 0) row_s[wave][c] = mx;
     }
     if (SL > 1) lds_barrier();
@@ -324,14 +452,7 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
             pieces[2][b] = uint4{w3[4 * b], w3[4 * b + 1], w3[4 * b + 2], w3[4 * b + 3]};
           }
         } else {
-#pragma unroll
-          for (int j = 0; j < EW / 4; ++j) {
-            const int quad = sl * (EW / 4) + j;  // elements 4 quad .. 4 quad + 3
-            unsigned char* dst = Ps + g * weight_bytes<T>() + (quad >> 1) * 1024 + 16 * lane + 8 * (quad & 1);
-            *reinterpret_cast<uint2*>(dst) = uint2{w1[2 * j], w1[2 * j + 1]};
-            *reinterpret_cast<uint2*>(dst + 2048) = uint2{w2[2 * j], w2[2 * j + 1]};
-            *reinterpret_cast<uint2*>(dst + 4096) = uint2{w3[2 * j], w3[2 * j + 1]};
-          }
+          store_pieces(w1, w2, w3);
         }
       } else if constexpr (SL > 1) {
 #pragma unroll
@@ -351,27 +472,10 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
       if constexpr (sizeof(T) == 2) {
-        const int j16 = lane & 15, col16 = 16 * ((lane >> 4) & 1);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {  // keys 16 b .. 16 b + 15; the lane's eight are 16 b + 4 h + u and 16 b + 8 + 4 h + u
-          if constexpr (SL > 1)
-#pragma unroll
-            for (int pc = 0; pc < 3; ++pc) pieces[pc][b] = *reinterpret_cast<const uint4*>(Ps + g * weight_bytes<T>() + pc * 2048 + b * 1024 + 16 * lane);
-          const bf16* vrow = reinterpret_cast<const bf16*>(K) + (16 * b + 4 * h + (j16 >> 2)) * ldk + col16 + 4 * (j16 & 3);
-          // all columns' values first, then the pieces in turn, the smallest first: neighbouring products add to
-          // different sums (columns behind the last tile repeat it, and nobody reads their sums)
-          bf16x8 v8[NVT];
-#pragma unroll
-          for (int dt = 0; dt < NVT; ++dt) {
-            const int d0 = 32 * min(sl * NVT + dt, last_tile);
-            const uint2 v0 = read_transposed(vrow + d0), v1 = read_transposed(vrow + 8 * ldk + d0);
-            v8[dt] = __builtin_bit_cast(bf16x8, uint4{v0.x, v0.y, v1.x, v1.y});
-          }
-#pragma unroll
-          for (int pc = 2; pc >= 0; --pc)
-#pragma unroll
-            for (int dt = 0; dt < NVT; ++dt)
-              o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v8[dt], __builtin_bit_cast(bf16x8, pieces[pc][b]), o[dt], 0, 0, 0);
+        for (int b = 0; b < 2; ++b) {
+          if constexpr (SL > 1) read_pieces(b, pieces);
+          add_values(K, b, pieces);
         }
       } else {
         const float* v = reinterpret_cast<const float*>(K) + 4 * h * ldk + c;
@@ -521,6 +625,7 @@ int launch(const char* what, LatentArgs a, int blocks, int spans, hipStream_t st
   auto k_bytes = [&](int buffers) { return sizeof(T) * ((buffers * kKeys * static_cast<size_t>(ldk) + slack + 7) / 8 * 8); };
   const size_t budget = 156 * 1024;
   a.two_buffers = k_bytes(2) + exchange <= budget - 16 * 1024 ? 1 : 0;
+  PYRE_REQUIRE(a.two_buffers || sizeof(T) == 4 || SINGLE || SL == 1, "%s: two chunks of %d elements a row do not fit a block", what, a.dk);
   size_t lds = k_bytes(a.two_buffers ? 2 : 1) + exchange;
   // the block's part of the request's block table, if it is not too long
   const int seen = a.window > 0 ? a.window + kKeys : a.table_stride * a.page_size;
