@@ -11,31 +11,6 @@ using namespace pyre;
 
 namespace {
 
-// The same loads and stores past the caches, for rows that are read and written once in a step of
-// many rows (more bytes than the caches hold).
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
-template <typename T> struct Stream4;
-template <> struct Stream4<float> {
-  static __device__ inline float4 load(const float* p) {
-    const f32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(p));
-    return float4{v[0], v[1], v[2], v[3]};
-  }
-  static __device__ inline void store(float* p, float4 v) {
-    __builtin_nontemporal_store(f32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4_t*>(p));
-  }
-};
-template <> struct Stream4<bf16> {
-  static __device__ inline float4 load(const bf16* p) {
-    const u32x2_t u = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(p));
-    return float4{__uint_as_float(u[0] << 16), __uint_as_float(u[0] & 0xffff0000u), __uint_as_float(u[1] << 16),
-                  __uint_as_float(u[1] & 0xffff0000u)};
-  }
-  static __device__ inline void store(bf16* p, float4 v) {
-    __builtin_nontemporal_store(u32x2_t{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)}, reinterpret_cast<u32x2_t*>(p));
-  }
-};
-
 // ---------------------------------------------------------------------------
 // add + RMSNorm, one block per row, the row kept in registers between the passes.
 // ---------------------------------------------------------------------------

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kThreads) void add_layernorm_kernel(
 // The same with four elements to a load (the row's width and the partial sums' stride are multiples
 // of four, no bias), the partial sums of an element asked for together: a step of few rows is all
 // waiting for loads. THREADS x ITEMS float4 hold a row.
-template <typename TD, typename TG, typename TO, int THREADS, int ITEMS>
+template <typename TD, typename TG, typename TO, int THREADS, int ITEMS, bool STREAM = false>
 __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
     float* __restrict__ resid, const TD* __restrict__ delta, int n_partials, size_t partial_stride,
     const TG* __restrict__ post_gain, const TG* __restrict__ post_scale, float post_eps, const TG* __restrict__ gain,
@@ -132,7 +132,16 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
-      v[k] = i < hidden ? sum_partials4(delta + row + i, partial_stride, n_partials) : float4{0.f, 0.f, 0.f, 0.f};
+      v[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f}
+             : STREAM    ? sum_partials4_stream(delta + row + i, partial_stride, n_partials)
+                         : sum_partials4(delta + row + i, partial_stride, n_partials);
+    }
+    // the residual is asked for with the term, not behind the term's own norm: one trip through memory less in a row
+    float4 r[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+      const int i = 4 * (tid + k * THREADS);
+      r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
     }
     if (post_gain) {
       float mean, inv;
@@ -156,8 +165,11 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
       if (i < hidden) {
-        v[k] = add4(v[k], Vec4<float>::load(resid + row + i));
-        if (!rows) Vec4<float>::store(resid + row + i, v[k]);
+        v[k] = add4(v[k], r[k]);
+        if (!rows) {
+          if (STREAM) Stream4<float>::store(resid + row + i, v[k]);
+          else Vec4<float>::store(resid + row + i, v[k]);
+        }
       }
     }
   } else {
@@ -287,8 +299,8 @@ extern "C" int pyre_add_layernorm(float* resid, const void* delta, int delta_dt,
     // sums of per-thread sums either way, and the two shapes differ in how the elements are dealt to threads
     const int quads = hidden / 4;
     const bool few = n <= 128 && quads > 256;  // a decode step: spread each row over more threads
-#define PYRE_LNV(THREADS, ITEMS)                                                                                       \
-  hipLaunchKernelGGL((add_layernorm_vec_kernel<TD, TG, TO, THREADS, ITEMS>), dim3(n), dim3(THREADS), 0, stream, resid, \
+#define PYRE_LNV(THREADS, ...)                                                                                         \
+  hipLaunchKernelGGL((add_layernorm_vec_kernel<TD, TG, TO, THREADS, __VA_ARGS__>), dim3(n), dim3(THREADS), 0, stream, resid, \
                      static_cast<const TD*>(delta), n_partials, static_cast<size_t>(partial_stride),                   \
                      static_cast<const TG*>(post_gain), static_cast<const TG*>(post_scale), post_eps,                  \
                      static_cast<const TG*>(gain), static_cast<const TG*>(shift), static_cast<TO*>(out), rows, hidden, eps)
@@ -296,6 +308,7 @@ extern "C" int pyre_add_layernorm(float* resid, const void* delta, int delta_dt,
       if (few && quads <= 1024) PYRE_LNV(1024, 1);
       else if (few) PYRE_LNV(1024, 4);
       else if (quads <= 256) PYRE_LNV(256, 1);
+      else if (quads <= 1024 && static_cast<long>(n) * hidden >= kStreamElements) PYRE_LNV(256, 4, true);
       else if (quads <= 1024) PYRE_LNV(256, 4);
       else PYRE_LNV(256, 16);
     })));

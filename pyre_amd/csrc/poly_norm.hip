@@ -36,8 +36,8 @@ __device__ inline void add_powers(float z, float& s2, float& s4, float& s6) {
   s2 += q, s4 += r, s6 = fmaf(r, q, s6);
 }
 
-// A row in the block's registers: ITEMS groups of four elements a thread.
-template <typename TI, typename TO, int THREADS, int ITEMS>
+// A row in the block's registers: ITEMS groups of four elements a thread. STREAM: the row past the caches.
+template <typename TI, typename TO, int THREADS, int ITEMS, bool STREAM = false>
 __global__ __launch_bounds__(THREADS) void poly_norm_vec_kernel(const TI* __restrict__ z, int n_partials, size_t partial_stride,
                                                                 const float* __restrict__ abce, float eps,
                                                                 TO* __restrict__ out, int width) {
@@ -49,7 +49,8 @@ __global__ __launch_bounds__(THREADS) void poly_norm_vec_kernel(const TI* __rest
   for (int k = 0; k < ITEMS; ++k) {
     const int i = 4 * (threadIdx.x + k * THREADS);
     v[k] = float4{0.f, 0.f, 0.f, 0.f};
-    if (i < width) v[k] = n_partials == 1 ? Vec4<TI>::load(z + row + i) : sum_partials4(z + row + i, partial_stride, n_partials);
+    if (i < width && STREAM) v[k] = sum_partials4_stream(z + row + i, partial_stride, n_partials);
+    else if (i < width) v[k] = n_partials == 1 ? Vec4<TI>::load(z + row + i) : sum_partials4(z + row + i, partial_stride, n_partials);
   }
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
@@ -92,8 +93,9 @@ extern "C" int pyre_poly_norm(const void* z, int z_dt, int n_partials, long part
   const bool vec = width % 4 == 0 && partial_stride % 4 == 0 && reinterpret_cast<uintptr_t>(z) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(out) % 16 == 0 && width <= 4 * 1024 * 8;
   const int quads = width / 4;
-#define PYRE_PN(THREADS, ITEMS)                                                                                           \
-  hipLaunchKernelGGL((poly_norm_vec_kernel<TI, TO, THREADS, ITEMS>), dim3(n), dim3(THREADS), 0, stream,                   \
+  const bool many = static_cast<long>(n) * width >= kStreamElements;
+#define PYRE_PN(THREADS, ...)                                                                                             \
+  hipLaunchKernelGGL((poly_norm_vec_kernel<TI, TO, THREADS, __VA_ARGS__>), dim3(n), dim3(THREADS), 0, stream,                   \
                      static_cast<const TI*>(z), n_partials, static_cast<size_t>(partial_stride), abce, eps,               \
                      static_cast<TO*>(out), width)
   PYRE_DISPATCH(z_dt, TI, PYRE_DISPATCH(out_dt, TO, {
@@ -102,7 +104,9 @@ extern "C" int pyre_poly_norm(const void* z, int z_dt, int n_partials, long part
                          static_cast<size_t>(partial_stride), abce, eps, static_cast<TO*>(out), width);
     else if (quads <= 256) PYRE_PN(256, 1);
     else if (quads <= 1024) PYRE_PN(1024, 1);
+    else if (quads <= 3072 && many) PYRE_PN(1024, 3, true);
     else if (quads <= 3072) PYRE_PN(1024, 3);
+    else if (quads <= 5120 && many) PYRE_PN(1024, 5, true);
     else if (quads <= 5120) PYRE_PN(1024, 5);
     else PYRE_PN(1024, 8);
   }));

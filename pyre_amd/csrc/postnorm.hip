@@ -98,8 +98,9 @@ __global__ __launch_bounds__(kThreads) void add_rms_terms_kernel(
 }
 
 // The same with four elements to a load: the row's width and the partial sums' strides are multiples of four, all
-// gains share one element type, every pointer lies on 16 bytes. THREADS x ITEMS float4 hold a row.
-template <typename TA, typename TG, typename TO, int THREADS, int ITEMS>
+// gains share one element type, every pointer lies on 16 bytes. THREADS x ITEMS float4 hold a row. The
+// residual is asked for with the terms, not behind their norms. STREAM: terms and residual past the caches.
+template <typename TA, typename TG, typename TO, int THREADS, int ITEMS, bool STREAM = false>
 __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
     float* __restrict__ resid, Term a, Term b, float inner_eps, const TG* __restrict__ outer_gain, float outer_eps,
     const TG* __restrict__ out_gain, float out_eps, TO* __restrict__ out, const int* __restrict__ rows, int hidden) {
@@ -111,6 +112,12 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) y[k] = float4{0.f, 0.f, 0.f, 0.f};
 
+  float4 r[ITEMS];
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = 4 * (tid + k * THREADS);
+    r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
+  }
   auto inv_rms = [&](const float4 (&v)[ITEMS], float e) {
     float ss = 0.f;
 #pragma unroll
@@ -124,7 +131,9 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
-      v[k] = i < hidden ? sum_partials4(src + i, t.stride, t.n_partials) : float4{0.f, 0.f, 0.f, 0.f};
+      v[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f}
+             : STREAM    ? sum_partials4_stream(src + i, t.stride, t.n_partials)
+                         : sum_partials4(src + i, t.stride, t.n_partials);
     }
     const float f = t.gain ? inv_rms(v, inner_eps) * t.scale : t.scale;
 #pragma unroll
@@ -152,8 +161,11 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
   for (int k = 0; k < ITEMS; ++k) {
     const int i = 4 * (tid + k * THREADS);
     if (i < hidden) {
-      y[k] = add4(y[k], Vec4<float>::load(resid + row + i));
-      if (!rows && a.data) Vec4<float>::store(resid + row + i, y[k]);
+      y[k] = add4(y[k], r[k]);
+      if (!rows && a.data) {
+        if (STREAM) Stream4<float>::store(resid + row + i, y[k]);
+        else Vec4<float>::store(resid + row + i, y[k]);
+      }
     }
   }
   if (!out) return;
@@ -208,14 +220,15 @@ extern "C" int pyre_add_rms_terms(float* resid, const void* a, int a_dt, int a_p
   if (vec) {
     const int quads = hidden / 4;
     const bool few = n <= 128 && quads > 256;  // a decode step: spread each row over more threads
-#define PYRE_RTV(THREADS, ITEMS)                                                                                          \
-  hipLaunchKernelGGL((add_rms_terms_vec_kernel<TA, TG, TO, THREADS, ITEMS>), dim3(n), dim3(THREADS), 0, stream, resid, ta, \
+#define PYRE_RTV(THREADS, ...)                                                                                            \
+  hipLaunchKernelGGL((add_rms_terms_vec_kernel<TA, TG, TO, THREADS, __VA_ARGS__>), dim3(n), dim3(THREADS), 0, stream, resid, ta, \
                      tb, inner_eps, static_cast<const TG*>(outer_gain), outer_eps, static_cast<const TG*>(out_gain),      \
                      out_eps, static_cast<TO*>(out), rows, hidden)
     PYRE_DISPATCH(a ? a_dt : kF32, TA, PYRE_DISPATCH(gdt, TG, PYRE_DISPATCH(out ? out_dt : kF32, TO, {
       if (few && quads <= 1024) PYRE_RTV(1024, 1);
       else if (few) PYRE_RTV(1024, 4);
       else if (quads <= 256) PYRE_RTV(256, 1);
+      else if (quads <= 1024 && static_cast<long>(n) * hidden >= kStreamElements) PYRE_RTV(256, 4, true);
       else if (quads <= 1024) PYRE_RTV(256, 4);
       else PYRE_RTV(256, 16);
     })));

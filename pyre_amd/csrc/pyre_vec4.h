@@ -30,6 +30,35 @@ template <> struct Vec4<bf16> {
   }
 };
 
+// The same loads and stores past the caches, for rows that are read and written once in a step of
+// many rows (more bytes than the caches hold). The row kernels take them from kStreamElements elements on: 16 MB of float32 (us a
+// launch at 1,777 rows of 3,584, two partial sums: LayerNorm with its term's own norm 31.1 -> 25.4, sums of two terms with three norms
+// 36 -> 31; two streams of 1,536 at 2,048 rows 18.0 -> 15.7 and at 952 rows, 12 MB, 10.8 -> 11.5; PolyNorm of 8,960 at 2,048 and 952
+// rows 30.8 -> 22.0 and 16.5 -> 12.5).
+constexpr long kStreamElements = 1L << 22;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+template <typename T> struct Stream4;
+template <> struct Stream4<float> {
+  static __device__ inline float4 load(const float* p) {
+    const f32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(p));
+    return float4{v[0], v[1], v[2], v[3]};
+  }
+  static __device__ inline void store(float* p, float4 v) {
+    __builtin_nontemporal_store(f32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4_t*>(p));
+  }
+};
+template <> struct Stream4<bf16> {
+  static __device__ inline float4 load(const bf16* p) {
+    const u32x2_t u = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(p));
+    return float4{__uint_as_float(u[0] << 16), __uint_as_float(u[0] & 0xffff0000u), __uint_as_float(u[1] << 16),
+                  __uint_as_float(u[1] & 0xffff0000u)};
+  }
+  static __device__ inline void store(bf16* p, float4 v) {
+    __builtin_nontemporal_store(u32x2_t{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)}, reinterpret_cast<u32x2_t*>(p));
+  }
+};
+
 __device__ inline float4 add4(float4 a, float4 b) { return float4{a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w}; }
 
 // p[0] + p[1] + ... + p[n - 1] (in that order) of the float4 at `src` in each of n partial sums that
@@ -47,6 +76,14 @@ __device__ inline float4 sum_partials4(const T* src, size_t stride, int n) {
   for (int p = 1; p < kAtOnce; ++p)
     if (p < n) s = add4(s, v[p]);
   for (int p = kAtOnce; p < n; ++p) s = add4(s, Vec4<T>::load(src + p * stride));
+  return s;
+}
+
+// The same sum of loads past the caches, in the same order.
+template <typename T>
+__device__ inline float4 sum_partials4_stream(const T* src, size_t stride, int n) {
+  float4 s = Stream4<T>::load(src);
+  for (int p = 1; p < n; ++p) s = add4(s, Stream4<T>::load(src + p * stride));
   return s;
 }
 

@@ -20,8 +20,8 @@ namespace {
 constexpr int kMaxStreams = 8;
 
 // One row's elements are dealt to THREADS x ITEMS float4 (VEC) or single floats; an element's streams (up to S of
-// them) are in registers together.
-template <typename TD, typename TO, int S, int THREADS, int ITEMS, bool VEC>
+// them) are in registers together. STREAM: the streams and the result past the caches.
+template <typename TD, typename TO, int S, int THREADS, int ITEMS, bool VEC, bool STREAM = false>
 __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
     const float* __restrict__ src, int src_streams, float* __restrict__ dst, int streams, const TD* __restrict__ y, int n_partials,
     size_t partial_stride, const float* __restrict__ mix, const float* __restrict__ out_w, const float* __restrict__ in_w,
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
       if (s >= streams) continue;
       const float* p = src + (src_streams == 1 ? row : (static_cast<size_t>(r_in) * streams + s) * hidden) + i;
       if constexpr (VEC) {
-        const float4 v = Vec4<float>::load(p);
+        const float4 v = STREAM ? Stream4<float>::load(p) : Vec4<float>::load(p);
         x[s][0] = v.x, x[s][1] = v.y, x[s][2] = v.z, x[s][3] = v.w;
       } else {
         x[s][0] = *p;
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
     }
     if (y) {
       if constexpr (VEC) {
-        const float4 v = sum_partials4(y + row + i, partial_stride, n_partials);
+        const float4 v = STREAM ? sum_partials4_stream(y + row + i, partial_stride, n_partials) : sum_partials4(y + row + i, partial_stride, n_partials);
         d[0] = v.x, d[1] = v.y, d[2] = v.z, d[3] = v.w;
       } else {
         d[0] = 0.f;
@@ -85,7 +85,8 @@ __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
         for (int e = 0; e < W; ++e) x[t][e] = z[t][e];
         if (dst && t < streams) {
           float* p = dst + (static_cast<size_t>(r_in) * streams + t) * hidden + i;
-          if constexpr (VEC) Vec4<float>::store(p, float4{x[t][0], x[t][1], x[t][2], x[t][3]});
+          if constexpr (VEC && STREAM) Stream4<float>::store(p, float4{x[t][0], x[t][1], x[t][2], x[t][3]});
+          else if constexpr (VEC) Vec4<float>::store(p, float4{x[t][0], x[t][1], x[t][2], x[t][3]});
           else *p = x[t][0];
         }
       }
@@ -144,8 +145,8 @@ extern "C" int pyre_stream_norm(const float* src, int src_streams, float* dst, i
   if (n <= 0) return 0;
   const auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool vec = hidden % 4 == 0 && (!y || partial_stride % 4 == 0) && a16(src) && a16(dst) && a16(y) && a16(gain) && a16(shift) && a16(out);
-#define PYRE_SN(S, THREADS, ITEMS, VEC)                                                                                     \
-  hipLaunchKernelGGL((stream_norm_kernel<TD, TO, S, THREADS, ITEMS, VEC>), dim3(n), dim3(THREADS), 0, stream, src,          \
+#define PYRE_SN(S, THREADS, ITEMS, ...)                                                                                     \
+  hipLaunchKernelGGL((stream_norm_kernel<TD, TO, S, THREADS, ITEMS, __VA_ARGS__>), dim3(n), dim3(THREADS), 0, stream, src,          \
                      src_streams, dst, streams, static_cast<const TD*>(y), n_partials,                                      \
                      static_cast<size_t>(partial_stride), mix, out_w, in_w, gain, shift, center, eps,                       \
                      static_cast<TO*>(out), picked, hidden)
@@ -156,6 +157,7 @@ extern "C" int pyre_stream_norm(const float* src, int src_streams, float* dst, i
     const int quads = hidden / 4;                                   \
     if (quads <= 256) PYRE_SN(S, 256, 1, true);                     \
     else if (n <= 128 && quads <= 1024) PYRE_SN(S, 1024, 1, true);  \
+    else if (quads <= 1024 && static_cast<long>(n) * streams * hidden >= kStreamElements) PYRE_SN(S, 256, 4, true, true); \
     else if (quads <= 1024) PYRE_SN(S, 256, 4, true);               \
     else PYRE_SN(S, 1024, 4, true);                                 \
   } while (0)
