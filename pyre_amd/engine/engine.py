@@ -72,6 +72,7 @@ class Engine:
         self.meta = MetaBuffers(self.device, max(ec.max_num_batched_tokens, seq_cap), seq_cap,
                                 [width for _ in self.cache.page_groups], self.step_arrays)
         self.steps_run = 0
+        self._cells = None  # see _list_cells
         #: captured decode steps: (rows, table width) -> "warm" (ran eagerly once) or (graph, logits)
         self._graphs: dict[tuple[int, int], object] = {}
         self.graph_replays = 0
@@ -285,6 +286,22 @@ class Engine:
     def _layer_views(self, views) -> list[list]:
         """For every entry of the layer order the views of its caches (or of the entry's whose
         caches it reads), in the order of the layer's descriptions."""
+        if self._cells is None:
+            self._cells = self._list_cells()
+        out = []
+        for cells in self._cells:
+            mine = []
+            for gi, tensors, spec, writes in cells:
+                if spec is not None:
+                    mine.append(PagedLayerView(tensors, views[f"table{gi}"], views[f"slots{gi}"], spec[0], spec[1], writes=writes))
+                else:
+                    mine.append(StateLayerView(tensors, views["state_slots"]))
+            out.append(mine)
+        return out
+
+    def _list_cells(self) -> list[list]:
+        """What of the views does not change from step to step: the group, the layer's own part of its tensors (page size and
+        window, None for a state), and whether the entry writes them. The engine's caches are made once."""
         cache = self.cache
         out = []
         entries = [(call.cache_from if call.cache_from is not None else pos, call.cache_from is None)
@@ -298,12 +315,10 @@ class Engine:
                 if kind == "paged":
                     g = cache.page_groups[gi]
                     li = g.layer_index(src, k)
-                    mine.append(PagedLayerView({name: t[li] for name, t in g.tensors.items()}, views[f"table{gi}"],
-                                               views[f"slots{gi}"], g.page_size, g.spec.window,
-                                               writes=writes))
+                    mine.append((gi, {name: t[li] for name, t in g.tensors.items()}, (g.page_size, g.spec.window), writes))
                 else:
                     g = cache.state_groups[gi]
-                    mine.append(StateLayerView(g.tensor[g.layer_index(src, k)], views["state_slots"]))
+                    mine.append((gi, g.tensor[g.layer_index(src, k)], None, writes))
             out.append(mine)
         return out
 

@@ -22,7 +22,7 @@ DEFAULT_UNITS = 256
 
 
 def dtype_code(t: torch.Tensor | torch.dtype) -> int:
-    dt = t if isinstance(t, torch.dtype) else t.dtype
+    dt = t.dtype if isinstance(t, torch.Tensor) else t
     try:
         return _DT[dt]
     except KeyError:
@@ -117,12 +117,15 @@ class Partials:
         return self.data.stride(0)
 
     def _args(self, width: int):
-        if self.width != width:
-            raise KernelError(f"partials are {self.width} wide, {width} expected")
-        if self.bias is not None and self.bias.numel() != width:
-            raise KernelError(f"bias has {self.bias.numel()} entries, {width} expected")
-        return (self.data.data_ptr(), dtype_code(self.data), self.count, self.stride,
-                _ptr(self.bias), dtype_code(self.bias) if self.bias is not None else 0)
+        data, bias = self.data, self.bias
+        count, _, wide = data.shape
+        if wide != width:
+            raise KernelError(f"partials are {wide} wide, {width} expected")
+        if bias is None:
+            return data.data_ptr(), dtype_code(data), count, data.stride(0), None, 0
+        if bias.numel() != width:
+            raise KernelError(f"bias has {bias.numel()} entries, {width} expected")
+        return data.data_ptr(), dtype_code(data), count, data.stride(0), bias.data_ptr(), dtype_code(bias)
 
 
 def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0,
@@ -932,6 +935,7 @@ def attn_prefill_bf16(q, out, k_cache, v_cache, tiles, n_tiles, positions, seq_o
 
 
 @lru_cache(maxsize=4096)
+@lru_cache(maxsize=4096)
 def attn_prefill_waves(nq: int, nkv: int) -> int:
     from pyre_amd.hip.lib import lib
 
@@ -969,7 +973,7 @@ def _skinny_common(x, w, m):
     _dev(x, w)
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise KernelError("gemm_skinny: bfloat16 operands expected")
-    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.shape[0] < m:
+    if x.dim() != 2 or w.dim() != 2 or x.size(1) != w.size(1) or x.size(0) < m:
         raise KernelError(f"gemm_skinny: x {tuple(x.shape)} and w {tuple(w.shape)} do not fit {m} rows")
     if x.stride(1) != 1 or w.stride(1) != 1:
         raise KernelError("gemm_skinny: rows must be contiguous")

@@ -10,9 +10,13 @@ head's logits of many rows; the true 32-bit path never comes here.
 
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 
+from pyre_amd.hip import ops
 from pyre_amd.hip.ops import DEFAULT_UNITS, Partials
+from pyre_amd.parts import attention_work as plan
 
 #: most rows the weight-streaming MFMA kernel takes; above, 16-bit products go to the kernel that keeps
 #: up to 256 rows in a block where it pays and else to the one that takes tiles of rows and columns
@@ -117,8 +121,6 @@ def takes_tiles(rt, lin, n: int, x=None) -> bool:
     1,618 for 4,096, 3,070 and 3,047 for 8,192; 206 and 247, 367 and 383, 651 and 690 of the 1.5B shape; 1,654 and 1,729, 3,276
     and 3,216, 6,286 and 6,804 of the 32B shape (at 3,000 rows 2,409 and 2,297: 1.23 PFLOP/s in its way down where the library
     has 1.48)."""
-    from pyre_amd.hip import ops
-
     if not rt.options.get("tile_gemm", True) or n <= SKINNY_MAX_ROWS or lin.weight.data_ptr() % 16 or (x is not None and x.data_ptr() % 16):
         return False
     return ops.gemm_tile_supports(n, lin.out_features, lin.in_features, lin.in_features if x is None else x.stride(0), lin.weight.stride(0))
@@ -146,8 +148,14 @@ def narrow_kernel(n: int, n_out: int, k: int, options: dict | None = None,
     thresholds in rows lie just above sizes at which decode steps are captured, so that an eager step
     and its replay at the padded size agree."""
     opt = options or {}
-    block = opt.get("mid_gemm", True)
-    if block and opt.get("mid_wide_min_rows", MID_WIDE_MIN_ROWS) <= n <= MID_MAX_ROWS:
+    return _narrow_kernel(n, n_out, k, units, opt.get("mid_gemm", True), opt.get("mid_wide_min_rows", MID_WIDE_MIN_ROWS),
+                          opt.get("skinny_gemm", True), opt.get("mid_small", True))
+
+
+@lru_cache(maxsize=4096)
+def _narrow_kernel(n: int, n_out: int, k: int, units: int, block, wide_min_rows: int, stream, small) -> tuple[str, int, bool]:
+    """The rule itself, kept by its sizes: three products a layer ask for it, and the splits that it weighs take longer than a launch."""
+    if block and wide_min_rows <= n <= MID_MAX_ROWS:
         # With 128 rows of the weights a block, where such blocks fill three quarters of the chip at
         # least: a block's bytes are the step's rows of X and its rows of W, over its part of k, and
         # with as many of the one as of the other they are fewest (at few rows of X a stage, and the
@@ -162,9 +170,9 @@ def narrow_kernel(n: int, n_out: int, k: int, options: dict | None = None,
         ks = mid_ksplit(n_out, k, 128, units)
         if ks and 4 * -(-n_out // 128) * ks >= 3 * units:
             return "block", ks, True
-    if n <= SKINNY_MAX_ROWS and opt.get("skinny_gemm", True):
+    if n <= SKINNY_MAX_ROWS and stream:
         ks = skinny_ksplit(n, n_out, k, units)
-        if block and opt.get("mid_small", True) and -(-n_out // 64) * ks < units and mid_ksplit(n_out, k, 64, units):
+        if block and small and -(-n_out // 64) * ks < units and mid_ksplit(n_out, k, 64, units):
             # A product so small that the weight-streaming kernel's blocks do not fill the compute
             # units (the 1.5B shape's: 96, 72 and 240 blocks) is latency all the way, and the other
             # kernel, whose loads go straight into a ring in LDS, starts sooner: 1.7 % of a step of
@@ -182,8 +190,6 @@ def narrow_kernel(n: int, n_out: int, k: int, options: dict | None = None,
 
 
 def linear(lin, ctx, x, n, out):
-    from pyre_amd.hip import ops
-
     rt = ctx.runtime
     if not _is_bf16(ctx, lin, x):
         return None
@@ -235,8 +241,6 @@ def gate_up_silu(lin, ctx, x, n, act, unit=None) -> bool:
     g sigmoid(slope g) (u + shift) with clipped inputs instead, in the same epilogues): the kernel that keeps all rows in a block for up to
     256 rows where one round of blocks holds the features, else the kernel of tiles for many rows and the weight-streaming
     kernel for a decode step's few."""
-    from pyre_amd.hip import ops
-
     if not _is_bf16(ctx, lin, x) or lin.bias is not None:
         return False
     if ctx.runtime.options.get("mid_silu_min_rows", MID_SILU_MIN_ROWS) <= n <= MID_MAX_ROWS:
@@ -273,8 +277,6 @@ def rope_in_attention(mixer, ctx, qkv, cache, rotary_dim: int) -> bool:
     sums, bias, rotation, the cache write): a step of single tokens only, on the 16-bit path's decode
     kernel, full-head rotation, heads of up to 128 elements. The kernel between product and attention
     is then left out; the bits are the same. A function of the step's shape and the model's sizes."""
-    from pyre_amd.hip import ops
-
     s = mixer.spec
     hb = ctx.host
     if ctx.dtype != torch.bfloat16 or cache["k"].dtype != torch.bfloat16 or qkv.data.dtype != torch.float32:
@@ -290,10 +292,6 @@ def rope_in_attention(mixer, ctx, qkv, cache, rotary_dim: int) -> bool:
 def attention(mixer, ctx, q, o, cache, rope=None) -> bool:
     """``rope``: (the q/k/v product's partial sums, cos, sin) when :func:`rope_in_attention` said that
     the decode kernel finishes the product; ``q`` is then not read."""
-    from pyre_amd.hip import ops
-    from pyre_amd.parts.attention_work import (decode_alone, decode_capacity, decode_items, prefill_items,
-                                                prefill_slots)
-
     s = mixer.spec
     k_pages, v_pages = cache["k"], cache["v"]
     if ctx.dtype != torch.bfloat16 or k_pages.dtype != torch.bfloat16:
@@ -311,15 +309,15 @@ def attention(mixer, ctx, q, o, cache, rope=None) -> bool:
         # eagerly or as a replayed graph at those sizes.
         rows, _ = hb.decode_shape()
         units = mixer.units
-        capacity = decode_capacity(rows, s.num_heads, s.num_kv_heads, units)
+        capacity = plan.decode_capacity(rows, s.num_heads, s.num_kv_heads, units)
         listed_blocks = int(hb.arrays[mixer.decode_work_name].reshape(-1)[0])
         if listed_blocks > capacity:  # the kernel would leave the rest of the list undone, silently
             raise RuntimeError(f"the decode attention's work list has {listed_blocks} blocks, its launch {capacity}")
-        items = decode_items(s.num_heads, s.num_kv_heads)
+        items = plan.decode_items(s.num_heads, s.num_kv_heads)
         acc = ctx.workspace.get("attn.part_acc", (capacity, items, 16, s.head_dim), torch.float32)
         ml = ctx.workspace.get("attn.part_ml", (capacity, items, 16, 2), torch.float32)
         counters = ctx.workspace.get("attn.counters", (capacity, items), torch.int32, zeroed=True)
-        alone = decode_alone(rows, s.num_heads, s.num_kv_heads, units)
+        alone = plan.decode_alone(rows, s.num_heads, s.num_kv_heads, units)
         if rope is not None:
             qkv, cos, sin = rope
             ops.attn_decode_work_rope_bf16(qkv, cos, sin, cache.slots, o, k_pages, v_pages, cache.writes,
@@ -333,11 +331,11 @@ def attention(mixer, ctx, q, o, cache, rope=None) -> bool:
                                       cache.window)
     if n_tiles and s.head_dim <= 128:
         work = hb.arrays[mixer.prefill_work_name]
-        n_slots = prefill_slots(work)
+        n_slots = plan.prefill_slots(work)
         if 8 * len(work) > ctx.arrays[mixer.prefill_work_name].numel():
             raise RuntimeError(f"the prompt attention's work list has {len(work)} blocks, its step array holds "
                                f"{ctx.arrays[mixer.prefill_work_name].numel() // 8}")
-        per_slot = prefill_items(s.num_heads, s.num_kv_heads) * ops.attn_prefill_waves(s.num_heads, s.num_kv_heads)
+        per_slot = plan.prefill_items(s.num_heads, s.num_kv_heads) * ops.attn_prefill_waves(s.num_heads, s.num_kv_heads)
         partials = counters = None
         if n_slots:
             partials = ctx.workspace.get("attn.prefill_partials", (n_slots, per_slot, s.head_dim // 32 * 1024 + 128),

@@ -12,6 +12,7 @@ import torch
 
 from pyre_amd.hip import ops
 from pyre_amd.hip.ops import Partials
+from pyre_amd.parts import fast
 from pyre_amd.parts.base import TensorSpec
 
 
@@ -34,8 +35,6 @@ class Linear:
     def forward(self, ctx, x: torch.Tensor, n: int, out: torch.Tensor | None = None) -> Partials:
         """x: [>= n, in] -> partial sums of the n x out product. ``out`` (float32
         [n, out]) makes the product land there, complete but for the bias."""
-        from pyre_amd.parts import fast
-
         done = fast.linear(self, ctx, x, n, out)
         if done is not None:
             return done
