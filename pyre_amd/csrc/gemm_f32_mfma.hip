@@ -230,7 +230,7 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
 // 350 of splitting; two blocks share a compute unit and fill each other's waits. At 2,000 rows of the 7B shape the gate/up product
 // runs at 197 TFLOP/s, 1.18 PFLOP/s of the 16-bit instruction, what that reaches at the clocks the card's power leaves. Against the float32
 // instruction (135 of its 157 TFLOP/s; us): gate/up 4,007 -> 2,748 there, 1,254 -> 885 at 566 rows, 316 -> 270 at 99; the 1.5B shape's
-// 844 -> 581, 245 -> 210 and 80 -> 72, its way down 446 -> 314, 127 -> 106 and 37 -> 35.
+// 844 -> 581, 245 -> 197 and 80 -> 68, its way down 446 -> 314, 127 -> 108 and 37 -> 33.
 // The eight k of a lane lie in arrays of their own, so that the lanes of a read are neighbours; each starts 64 bytes (32 of
 // slots of two steps) off the banks of the one before, since a write's lanes go to all of them in turn.
 //
@@ -608,13 +608,15 @@ int stream_columns(int N, int parts) {
 }
 
 // The tile with the least work on the busiest unit (a block of two or three shares its matrix cores' time, so that is its
-// tiles), smaller ones costing more for the same: their operands come from LDS more often.
+// tiles), smaller ones costing more for the same: their operands come from LDS more often. The three sizes in turn (us): the 1.5B
+// shape's gate/up 68, 74, 66 at 99 rows, 187, 158, 176 at 400, 197, 207, 230 at 566; the 7B shape's way down 111, 116, 135, then 344,
+// 375, 414 and 440, 484, 545.
 struct TileRows {
   int bm, bn;
   double cost;
 };
 constexpr int kSizes = 3;
-constexpr TileRows kTiles[kSizes] = {{128, 128, 1.0}, {64, 128, 1.1}, {64, 64, 1.5}};
+constexpr TileRows kTiles[kSizes] = {{128, 128, 1.0}, {64, 128, 1.2}, {64, 64, 1.4}};
 constexpr double kMacsPerUs = 3.9e5;    // of a compute unit
 constexpr double kBytesPerUs = 5e6;     // of memory, both ways
 constexpr double kFillUs = 0.004;       // a k of a block's chain before the unit's other blocks hide it
