@@ -334,10 +334,11 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
   // 3,000, 12 heads, rows of 576, a window of 1,024): 163 -> 154 and 116 -> 102 us.
   //
   // A chunk's weights are made against the maximum of the chunks before it, which needs no barrier of its own; a reference
-  // other than the maximum scales weights and sums alike. Where a query's scores rise by more than 2^kJump over it (as in the
-  // first chunk that it sees), its weights are made once more against the new maximum: all waves of the block see the flag behind the barrier.
+  // other than the maximum scales weights and sums alike. Where a query's weights would rise above 2^kJump (as in the
+  // first chunk that it sees), they are made once more against the new maximum: all waves of the block see the flag behind the
+  // barrier. The bound keeps the sums within a thousand times what they are against the maximum, so that values near float32's end do not overflow.
   if constexpr (kAhead) {
-    constexpr float kJump = 60.f;
+    constexpr float kJump = 10.f;
     float alpha = 1.f;  // what the sums so far are to be multiplied with
     if (active) hand_round(score(Ks));
     lds_barrier();

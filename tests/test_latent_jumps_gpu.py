@@ -9,8 +9,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-#: what a chunk's scores are around, in turn: rises of less and of more than 2^60 in weight (60 ln 2 = 41.6), falls, repeats
-LEVELS = (0.0, 30.0, 75.0, -90.0, 74.0, 400.0, 399.0, 430.0, 900.0, 0.0, 1000.0)
+#: what a chunk's scores are around, in turn: rises of less and of more than 2^10 in weight (10 ln 2 = 6.9), falls, repeats
+LEVELS = (0.0, 5.0, 14.0, -90.0, 12.0, 17.0, 400.0, 399.0, 404.0, 900.0, 0.0)
 
 
 @pytest.mark.parametrize("heads,rank,rot,window", [(12, 512, 64, 0), (3, 512, 64, 100), (5, 256, 128, 0), (1, 200, 30, 70), (2, 512, 128, 0)])
