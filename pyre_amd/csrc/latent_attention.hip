@@ -101,7 +101,6 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
   int* tab_s = reinterpret_cast<int*>(Ps + (SL > 1 ? G * weight_bytes<T>() : 0));
   __shared__ int slot_s[kRing][kKeys];
   __shared__ float row_s[G * SL][32];  // the waves' maxima of their keys, per query; at the end their weights
-  __shared__ int jump_s;               // the last chunk (from 1 on) whose scores rise far above those before
 
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, c = lane & 31;
   const int g = wave / SL, sl = wave % SL;
@@ -315,7 +314,6 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v8[dt], __builtin_bit_cast(bf16x8, pieces[pc][b]), o[dt], 0, 0, 0);
   };
 
-  if (tid == 0) jump_s = 0;
   if (tid < kKeys) {
     slot_s[0][tid] = slot_of(chunk0 * kKeys + tid);
     slot_s[1][tid] = slot_of((chunk0 + 1) * kKeys + tid);
@@ -328,71 +326,49 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
   if (n_chunks > 1) ask(1);
   __syncthreads();
   // Row tiles that waves share, with both chunks in LDS: the score of chunk it + 1 is made beside the second product of chunk it,
-  // so that a chunk has one stretch of products and one of handing round, a barrier behind each. What bounds it are the products
-  // (33 instructions of 32 cycles a wave and chunk, two waves a SIMD: 2,100 cycles) and the handing round's latencies between. Against three
-  // barriers a chunk, the maxima going round before the weights are made (us for a prompt's first 2,048 and last 952 tokens of
-  // 3,000, 12 heads, rows of 576, a window of 1,024): 163 -> 154 and 116 -> 102 us.
-  //
-  // A chunk's weights are made against the maximum of the chunks before it, which needs no barrier of its own; a reference
-  // other than the maximum scales weights and sums alike. Where a query's weights would rise above 2^kJump (as in the
-  // first chunk that it sees), they are made once more against the new maximum: all waves of the block see the flag behind the
-  // barrier. The bound keeps the sums within a thousand times what they are against the maximum, so that values near float32's end do not overflow.
+  // so that a chunk has one stretch of products, and then the handing round of parts of scores, of maxima and of weights, a barrier
+  // behind each. What bounds it are the products (33 instructions of 32 cycles a wave and chunk, two waves a SIMD: 2,100 cycles) and
+  // the latencies between the barriers. Weights are never above 1: what they are made against includes the chunk's own maximum. (Against
+  // the maximum of the chunks before, a barrier less, sums of large values overflow where these do not, and scores that rise have their
+  // weights made twice.) Against a chunk's score made in its own turn, us a launch: 12 heads, rows of 576, a window of 1,024,
+  // 2,048 tokens 151 -> 148, the next 952 101 -> 101; 28 heads without a window, 1,777 tokens 280 -> 271; 8 heads, rows of 384, 900
+  // tokens 86 -> 84; scores that rise (12 heads, 1,400 tokens) 134 -> 131.
   if constexpr (kAhead) {
-    constexpr float kJump = 10.f;
-    float alpha = 1.f;  // what the sums so far are to be multiplied with
     if (active) hand_round(score(Ks));
     lds_barrier();
     for (int it = 0; it < n_chunks; ++it) {
       const int key0 = (chunk0 + it) * kKeys;
       const T* K = Ks + (it & 1) * buffer;
       if (tid < kKeys && it + 3 < n_chunks) slot_s[(it + 3) % kRing][tid] = slot_of(key0 + 3 * kKeys + tid);
-      float w[EW], sum = 0.f;
-      auto weigh = [&](float reference) {
-        const float m_use = reference == -INFINITY ? 0.f : reference;
-        uint32_t w1[EW / 2], w2[EW / 2], w3[EW / 2];
-        sum = 0.f;
-#pragma unroll
-        for (int u = 0; u < EW / 2; ++u) {
-          const float p0 = exp2_hw(w[2 * u] - m_use), p1 = exp2_hw(w[2 * u + 1] - m_use);
-          sum += p0;
-          sum += p1;
-          split_pair(p0, p1, w1[u], w2[u], w3[u]);
-        }
-        store_pieces(w1, w2, w3);
-      };
+      float w[EW], alpha = 1.f, mx = -INFINITY;
       if (active) {
-        const float mx = take(f32x16{}, key0, w);
+        mx = take(f32x16{}, key0, w);
         if (h == 0) row_s[wave][c] = mx;
-        if (__ballot(mx > m + kJump) && lane == 0) jump_s = it + 1;
-        weigh(m);
       }
-      bring(it + 1);  // into the buffer whose last readers, of the chunk before, have passed the barrier above
       lds_barrier();
-      float top = -INFINITY;
-      if (active)
+      if (active) {
 #pragma unroll
-        for (int o2 = 0; o2 < SL; ++o2) top = fmaxf(top, row_s[g * SL + o2][c]);
-      if (jump_s == it + 1) {
-        if (active) {
-          const float reference = top > m + kJump ? top : m;
-          if (reference != m) alpha *= exp2_hw(m - reference), l *= exp2_hw(m - reference);
-          m = reference;
-          weigh(m);
-        }
-        lds_barrier();
+        for (int o2 = 0; o2 < SL; ++o2) mx = fmaxf(mx, row_s[g * SL + o2][c]);
+        const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
+        alpha = exp2_hw(m - m_use);
+        m = m_new;
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < EW; ++i) w[i] = exp2_hw(w[i] - m_use), sum += w[i];
+        l = l * alpha + sum;
+        uint32_t w1[EW / 2], w2[EW / 2], w3[EW / 2];
+#pragma unroll
+        for (int u = 0; u < EW / 2; ++u) split_pair(w[2 * u], w[2 * u + 1], w1[u], w2[u], w3[u]);
+        store_pieces(w1, w2, w3);
       }
+      bring(it + 1);  // into the buffer whose last readers, of the chunk before, have passed the barriers above
+      lds_barrier();
       if (active) {
         if (__ballot(alpha != 1.f))
 #pragma unroll
           for (int dt = 0; dt < NVT; ++dt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-        l += sum;
-        // the reference of the next chunk
-        const float next = fmaxf(m, top);
-        alpha = next == m ? 1.f : exp2_hw(m - next);
-        l *= alpha;
-        m = next;
         uint4 pieces[3][2];
         const f32x16 s = score(Ks + ((it + 1) & 1) * buffer);  // (behind the last chunk: of whatever lies there, for nobody)
         read_pieces(0, pieces);
@@ -403,11 +379,6 @@ __global__ __launch_bounds__(64 * G * SL, sizeof(T) == 2 && !SINGLE ? 2 : 1) voi
       }
       lds_barrier();
     }
-    if (__ballot(alpha != 1.f))
-#pragma unroll
-      for (int dt = 0; dt < NVT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
   } else
   for (int it = 0; it < n_chunks; ++it) {
     const int key0 = (chunk0 + it) * kKeys;

@@ -1,5 +1,5 @@
-"""Attention over compressed rows by row tiles that waves share: a chunk's weights are made against the maximum of the chunks
-before it, and once more where the scores rise far above that."""
+"""Attention over compressed rows by row tiles that waves share: scores that rise from chunk to chunk, and values near the end of the
+range under them."""
 
 from __future__ import annotations
 
@@ -9,7 +9,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-#: what a chunk's scores are around, in turn: rises of less and of more than 2^10 in weight (10 ln 2 = 6.9), falls, repeats
+#: what a chunk's scores are around, in turn: small and large rises, falls, repeats
 LEVELS = (0.0, 5.0, 14.0, -90.0, 12.0, 17.0, 400.0, 399.0, 404.0, 900.0, 0.0)
 
 
@@ -50,3 +50,25 @@ def test_scores_that_rise_from_chunk_to_chunk(heads, rank, rot, window):
     share = torch.stack([torch.exp(torch.logsumexp(x, 1) - torch.logaddexp(torch.logsumexp(x, 1), torch.tensor(50.0, dtype=torch.float64)))
                          for x in s], 1)
     assert float((outs[1] - want * share[:, :, None]).abs().max()) < bound
+
+
+@pytest.mark.parametrize("heads,rank,rot", [(3, 512, 64), (2, 256, 128)])
+def test_values_near_the_end_of_the_range(heads, rank, rot):
+    """Scores that rise by 6 from chunk to chunk (8.7 in base two) over values of 2^118: no weight is above 1, so 340 keys stay below
+    2^127. The output is an average of the values, whatever the weights."""
+    from pyre_amd.hip import ops
+
+    page, length, dk = 16, 340, rank + rot
+    scale = 1.0 / dk ** 0.5
+    rows, q = torch.full((length, dk), 2.0 ** 118), torch.zeros(length, heads, dk)
+    rows[:, -1], q[:, :, -1] = torch.tensor([6.0 * (t // 32) for t in range(length)]) / scale, 1.0
+    n_pages = -(-length // page)
+    pool = torch.zeros(n_pages * page, dk)
+    pool[:length] = rows
+    tiles = torch.tensor([(t, min(32, length - t)) for t in range(0, length, 32)], dtype=torch.int32, device=DEV)
+    pos, seq = torch.arange(length, dtype=torch.int32, device=DEV), torch.zeros(length, dtype=torch.int32, device=DEV)
+    out = torch.full((length, heads, rank), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.latent_attn_tile(q.to(DEV).bfloat16(), pool.to(DEV).bfloat16().view(n_pages, 1, page, dk), out, tiles, tiles.shape[0], pos, seq,
+                         torch.arange(n_pages, dtype=torch.int32, device=DEV)[None], heads, rank, dk, page, scale, 0, None)
+    # 2^-9 of the result's own 16 bits, and the sums' roundings far below that
+    assert float((out.double() / 2.0 ** 118 - 1).abs().max()) <= 2.0 ** -8
