@@ -34,6 +34,7 @@ namespace {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef f32x4 f32x4_any __attribute__((aligned(4)));  // where rows may start on any float: one load all the same
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
@@ -101,102 +102,51 @@ __device__ inline void finish(const float* a, size_t lda, const float* w, size_t
   }
 }
 
-// Four consecutive k of one row; zero where the row or the k is not there.
-__device__ inline f32x4 load_k4(const float* base, size_t ld, int row, int rows, int k, int K, bool vec_ok) {
-  if (row >= rows || k >= K) return f32x4{0.f, 0.f, 0.f, 0.f};
-  const float* p = base + static_cast<size_t>(row) * ld + k;
-  if (vec_ok && k + 3 < K) return *reinterpret_cast<const f32x4*>(p);
-  f32x4 v = {0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < 4 && k + j < K; ++j) v[j] = p[j];
-  return v;
-}
-
-// Rows that do not start on 16 bytes, and k that is not a multiple of four: 16 k of both operands at a time through registers
-// and LDS as float32, split by the waves that multiply them. WN x WM waves (along n and along m), each on TN x TM tiles of 32 x 32.
-template <int WN, int WM, int TN, int TM>
-__global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
+// What the other kernels leave: fewer than eight k, or more tiles than a launch holds. 16 k of both operands at a time through
+// registers and LDS as float32, split by the waves that multiply them: 32 rows of A against 32 columns a wave.
+__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     const float* __restrict__ A, size_t lda, const float* __restrict__ W, size_t ldw,
     const void* __restrict__ bias, int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M,
-    int N, int K, int kper, int chain, int vec_ok) {
-  constexpr int NT = 64 * WN * WM, BN = WN * TN * 32, BM = WM * TM * 32;
-  constexpr int WP = (BN * 4 + NT - 1) / NT, AP = (BM * 4 + NT - 1) / NT;  // 16-byte pieces per thread and stage
-  __shared__ __attribute__((aligned(16))) float Ws[BN][LD];
-  __shared__ __attribute__((aligned(16))) float As[BM][LD];
+    int N, int K, int kper, int chain, int mt) {
+  __shared__ __attribute__((aligned(16))) float Ws[128][LD];
+  __shared__ __attribute__((aligned(16))) float As[32][LD];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, half = lane >> 5, c = lane & 31;
-  const int wn = wave % WN, wm = wave / WN;
-  const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
+  const int n0 = static_cast<int>(blockIdx.x / mt) * 128, m0 = static_cast<int>(blockIdx.x % mt) * 32;
   const int kbeg = blockIdx.z * kper;
   K = min(K, kbeg + kper);  // this part's end
   out += blockIdx.z * part_stride;
   if (blockIdx.z) bias = nullptr;  // the bias belongs to one part only
 
-  f32x4 wr[WP], ar[AP];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int i = 0; i < WP; ++i) {
-      const int p = tid + NT * i;
-      wr[i] = p < BN * 4 ? load_k4(W, ldw, n0 + p / 4, N, k0 + 4 * (p % 4), K, vec_ok) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int i = 0; i < AP; ++i) {
-      const int p = tid + NT * i;
-      ar[i] = p < BM * 4 ? load_k4(A, lda, m0 + p / 4, M, k0 + 4 * (p % 4), K, vec_ok) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+  // Four consecutive k of one row; zero where the row or the k is not there.
+  auto load_k4 = [&](const float* base, size_t ld, int row, int rows, int k) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (row < rows)
+      for (int j = 0; j < 4 && k + j < K; ++j) v[j] = base[row * ld + k + j];
+    return v;
   };
-  auto stash = [&]() {
+  f32x16 acc, total;
 #pragma unroll
-    for (int i = 0; i < WP; ++i) {
-      const int p = tid + NT * i;
-      if (p < BN * 4) *reinterpret_cast<f32x4*>(&Ws[p / 4][4 * (p % 4)]) = wr[i];
-    }
-#pragma unroll
-    for (int i = 0; i < AP; ++i) {
-      const int p = tid + NT * i;
-      if (p < BM * 4) *reinterpret_cast<f32x4*>(&As[p / 4][4 * (p % 4)]) = ar[i];
-    }
-  };
-
-  f32x16 acc[TN][TM], total[TN][TM];
-#pragma unroll
-  for (int t = 0; t < TN; ++t)
-#pragma unroll
-    for (int u = 0; u < TM; ++u)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[t][u][i] = total[t][u][i] = 0.f;
-
-  const int kfirst = kbeg;
+  for (int i = 0; i < 16; ++i) acc[i] = total[i] = 0.f;
   auto end_chain = [&]() {
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-      for (int u = 0; u < TM; ++u)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          total[t][u][i] += acc[t][u][i];
-          acc[t][u][i] = 0.f;
-        }
+    for (int i = 0; i < 16; ++i) {
+      total[i] += acc[i];
+      acc[i] = 0.f;
+    }
   };
   int left = chain;
-  fetch(kbeg);
   for (int k0 = kbeg; k0 < K; k0 += BK) {
-    stash();
+    for (int p = tid; p < 160 * 4; p += 256) {
+      const int row = p / 4, k = 4 * (p % 4);
+      if (row < 128) *reinterpret_cast<f32x4*>(&Ws[row][k]) = load_k4(W, ldw, n0 + row, N, k0 + k);
+      else *reinterpret_cast<f32x4*>(&As[row - 128][k]) = load_k4(A, lda, m0 + row - 128, M, k0 + k);
+    }
     __syncthreads();
-    if (k0 + BK < K) fetch(k0 + BK);  // in flight while this stage is multiplied
-    Pieces b[TM];
+    const float *w = &Ws[32 * wave + c][8 * half], *a = &As[c][8 * half];
+    const Pieces x = split8(*reinterpret_cast<const f32x4*>(w), *reinterpret_cast<const f32x4*>(w + 4));
+    const Pieces y = split8(*reinterpret_cast<const f32x4*>(a), *reinterpret_cast<const f32x4*>(a + 4));
 #pragma unroll
-    for (int u = 0; u < TM; ++u) {
-      const float* p = &As[(wm * TM + u) * 32 + c][8 * half];
-      b[u] = split8(*reinterpret_cast<const f32x4*>(p), *reinterpret_cast<const f32x4*>(p + 4));
-    }
-#pragma unroll
-    for (int t = 0; t < TN; ++t) {
-      const float* p = &Ws[(wn * TN + t) * 32 + c][8 * half];
-      const Pieces a = split8(*reinterpret_cast<const f32x4*>(p), *reinterpret_cast<const f32x4*>(p + 4));
-#pragma unroll
-      for (int s = 0; s < kTerms; ++s)
-#pragma unroll
-        for (int u = 0; u < TM; ++u) acc[t][u] = multiply(a.p[kTermW[s]], b[u].p[kTermA[s]], acc[t][u]);
-    }
+    for (int s = 0; s < kTerms; ++s) acc = multiply(x.p[kTermW[s]], y.p[kTermA[s]], acc);
     if (--left == 0) {
       end_chain();
       left = chain;
@@ -205,39 +155,40 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(
   }
   end_chain();
 
-  // total[t][u][4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = tile column c.
+  // total[4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = tile column c.
   const bool rows_of_16 = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  const int m = m0 + wm * TM * 32 + c, n = n0 + wn * TN * 32 + 4 * half;
+  const int m = m0 + c, n = n0 + 32 * wave + 4 * half;
   bool bad = false;
+  if (m < M) {
 #pragma unroll
-  for (int u = 0; u < TM; ++u) {
-    if (m + 32 * u >= M) continue;
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        bad |= store4(f32x4{total[t][u][4 * i], total[t][u][4 * i + 1], total[t][u][4 * i + 2], total[t][u][4 * i + 3]},
-                      out + static_cast<size_t>(m + 32 * u) * ldo, rows_of_16, n + 32 * t + 8 * i, N);
+    for (int i = 0; i < 4; ++i)
+      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, out + static_cast<size_t>(m) * ldo,
+                    rows_of_16, n + 8 * i, N);
   }
-  if (bad || bias) finish(A + kfirst, lda, W + kfirst, ldw, bias, bias_dt, out, ldo, m, TM, M, n, TN, N, K - kfirst);
+  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, 1, M, n, 1, N, K - kbeg);
 }
 
-// More than 32 rows whose k comes in whole steps. A block of four waves keeps BM rows of A and BN rows of W; every thread brings
-// eight k of some rows, two steps ahead in registers, splits them once for the whole block and writes the pieces into one of two
-// buffers in LDS, while the pieces in the other are multiplied: one barrier a slot of SL steps.
+// More than 32 rows, and fewer where they do not start on 16 bytes. A block of four waves keeps BM rows of A and BN rows of W; every
+// thread brings eight k of some rows, two steps ahead in registers, splits them once for the whole block and writes the pieces into one
+// of two buffers in LDS, while the pieces in the other are multiplied: one barrier a slot of SL steps. TAIL: k may end within a step
+// (at least eight k in all); the last step's loads lie as far before the end as keeps them in their rows, and what they bring is
+// moved to its place, zeros behind it, before it is split.
 //
 // What bounds it: a step of 128 x 128 is 768 cycles of the matrix cores a SIMD, 580 cycles of LDS (24 KB written, 48 KB read) and
 // 350 of splitting; two blocks share a compute unit and fill each other's waits. At 2,000 rows of the 7B shape the gate/up product
 // runs at 197 TFLOP/s, 1.18 PFLOP/s of the 16-bit instruction, what that reaches at the clocks the card's power leaves. Against the float32
 // instruction (135 of its 157 TFLOP/s; us): gate/up 4,007 -> 2,748 there, 1,254 -> 885 at 566 rows, 316 -> 270 at 99; the 1.5B shape's
 // 844 -> 581, 245 -> 197 and 80 -> 68, its way down 446 -> 314, 127 -> 108 and 37 -> 33.
+// Rows that start on any float cost two per cent, k that ends within a step five to ten. Against the float32 instruction in tiles that
+// went through registers, the 7B shape's gate/up with rows a float off: 713 -> 153 at one row, 1,132 -> 156 at 33, 2,357 -> 567 at 300; with
+// four k more: 271 -> 197 at 33 (there against a stream of 64 rows), 523 -> 271 at 99, 1,050 -> 592 at 300.
 // The eight k of a lane lie in arrays of their own, so that the lanes of a read are neighbours; each starts 64 bytes (32 of
 // slots of two steps) off the banks of the one before, since a write's lanes go to all of them in turn.
 //
 // A chain of instructions ends after `chain` steps and is added to the total in float32. A block that walks all parts of k
 // (where the rows alone fill the chip) ends its chains where the parts end: the bits of the consumer's sum of partial sums, which
 // then do not go through memory.
-template <int BM, int BN, int WM, int WN, int SL, int OCC>
+template <int BM, int BN, int WM, int WN, int SL, int OCC, bool TAIL>
 __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
     const float* A, long lda, const float* W, long ldw, const void* __restrict__ bias,
     int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int chain, int mt, int nt) {
@@ -255,7 +206,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
   const int group = t / (8 * nt), first = 8 * group, gm = min(8, mt - first);
   t -= 8 * nt * group;
   const int m0 = (first + t % gm) * BM, n0 = (t / gm) * BN;
-  const int kbeg = ks * kper, kend = min(K, kbeg + kper), steps = (kend - kbeg) / BK;
+  const int kbeg = ks * kper, kend = min(K, kbeg + kper), len = kend - kbeg, steps = (len + BK - 1) / BK;
   const int slots = (steps + SL - 1) / SL;
   out += ks * part_stride;
   if (ks) bias = nullptr;  // the bias belongs to one part only
@@ -271,17 +222,32 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
   }
   f32x4 st[2][P][2];
   const bool short_end = SL > 1 && steps % SL;  // the last slot has fewer steps: what lies behind them is not multiplied
+  auto last_k = [&](int i) { return len - 8 - 8 * static_cast<int>((threadIdx.x + 256 * i) % KP); };  // of a load in its row, from src[i] on
   auto fetch = [&](int buf, int slot) {
     const int at = min(slot, slots - 1);
 #pragma unroll
     for (int i = 0; i < P; ++i) {
-      const int k = BK * SL * at - (short_end && at == slots - 1 && (threadIdx.x + 256 * i) % KP >= 2 ? BK : 0);
-      st[buf][i][0] = *reinterpret_cast<const f32x4*>(src[i] + k);
-      st[buf][i][1] = *reinterpret_cast<const f32x4*>(src[i] + k + 4);
+      const int k = TAIL ? min(BK * SL * at, last_k(i)) : BK * SL * at - (short_end && at == slots - 1 && (threadIdx.x + 256 * i) % KP >= 2 ? BK : 0);
+      st[buf][i][0] = *reinterpret_cast<const f32x4_any*>(src[i] + k);
+      st[buf][i][1] = *reinterpret_cast<const f32x4_any*>(src[i] + k + 4);
     }
   };
-  auto convert = [&](int buf, int i) {
-    const Pieces v = split8(st[buf][i][0], st[buf][i][1]);
+  auto convert = [&](int buf, int i, int slot) {
+    f32x4 lo = st[buf][i][0], hi = st[buf][i][1];
+    if (TAIL && slot == slots - 1) {
+      const int by = BK * SL * slot - min(BK * SL * slot, last_k(i));  // places towards the front; from eight on nothing is left
+#pragma unroll
+      for (int b = 1; b < 8; b *= 2)
+        if (by & b)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float v = j + b < 4 ? lo[(j + b) & 3] : j + b < 8 ? hi[(j + b) & 3] : 0.f;
+            if (j < 4) lo[j] = v;
+            else hi[j - 4] = v;
+          }
+      if (by >= 8) lo = hi = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const Pieces v = split8(lo, hi);
 #pragma unroll
     for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x4*>(lds + buf * BUF + s * PLANE + dst[i]) = v.p[s];
   };
@@ -329,7 +295,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
         if (j == 0) {
 #pragma unroll
           for (int i = 0; i < P; ++i)
-            if (i * (kTerms - 1) / P == s) convert(buf ^ 1, i);
+            if (i * (kTerms - 1) / P == s) convert(buf ^ 1, i, slot + 1);
         }
       }
       if (j == 0) fetch(buf ^ 1, slot + 3);
@@ -347,7 +313,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
   fetch(1, 1);
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < P; ++i) convert(0, i);
+  for (int i = 0; i < P; ++i) convert(0, i, 0);
   fetch(0, 2);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   int slot = 0;
@@ -370,7 +336,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
         bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]},
                       out + static_cast<size_t>(m + 32 * q) * ldo, rows_of_16, n + 32 * r + 8 * i, N);
   }
-  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, kend - kbeg);
+  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len);
 }
 
 constexpr int kStreamMaxRows = 32;
@@ -634,12 +600,14 @@ int best_tile(int M, int N, int kper, int parts, double* us) {
   return best;
 }
 
-bool takes_tiles(int M, int N, int K, long lda, long ldw) {
-  return M > 16 && lda % 4 == 0 && ldw % 4 == 0 && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32) &&
-         static_cast<long>((M + 31) / 32) * ((N + 63) / 64) < (1L << 24);
+// (The last loads of a row lie up to eight k before its end.)
+bool takes_tiles(int M, int N, int K) { return K >= 8 && static_cast<long>((M + 31) / 32) * ((N + 63) / 64) < (1L << 24); }
+// What is offered as sums of all parts: rows on 16 bytes, whole steps.
+bool takes_whole(int M, int N, int K, long lda, long ldw) {
+  return M > 16 && lda % 4 == 0 && ldw % 4 == 0 && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32) && takes_tiles(M, N, K);
 }
 
-// Chains of `chain` steps; `whole`: a block walks all of k.
+// Chains of `chain` steps.
 void launch_tiles(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
                   int M, int N, int K, int kper, int parts, int chain, hipStream_t stream) {
   const auto tile = [&](auto kernel, int bm, int bn) {
@@ -648,9 +616,10 @@ void launch_tiles(const float* A, long lda, const float* W, long ldw, const void
                        static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, chain, mt, nt);
   };
   const int best = best_tile(M, N, kper, parts, nullptr);
-  if (best == 0) tile(gemm_f32_tile_kernel<128, 128, 2, 2, 1, 2>, 128, 128);
-  else if (best == 1) tile(gemm_f32_tile_kernel<64, 128, 2, 2, 2, 2>, 64, 128);
-  else tile(gemm_f32_tile_kernel<64, 64, 2, 2, 2, 3>, 64, 64);
+  const bool tail = K % BK != 0;
+  if (best == 0) tile(tail ? gemm_f32_tile_kernel<128, 128, 2, 2, 1, 2, true> : gemm_f32_tile_kernel<128, 128, 2, 2, 1, 2, false>, 128, 128);
+  else if (best == 1) tile(tail ? gemm_f32_tile_kernel<64, 128, 2, 2, 2, 2, true> : gemm_f32_tile_kernel<64, 128, 2, 2, 2, 2, false>, 64, 128);
+  else tile(tail ? gemm_f32_tile_kernel<64, 64, 2, 2, 2, 3, true> : gemm_f32_tile_kernel<64, 64, 2, 2, 2, 3, false>, 64, 64);
 }
 
 int part_of(int K, int ksplit) { return ((K + ksplit - 1) / ksplit + BK - 1) / BK * BK; }
@@ -664,7 +633,7 @@ int chain_of(int K, int ksplit) { return ksplit > 1 ? part_of(K, ksplit) / BK : 
 // and 38 whole at 300 rows, 45 and 61 at 566, 96 and 83 at 1,200, 148 and 111 at 2,000; the 7B shape's o in 9: 120 and 138 at
 // 400, 148 and 140 at 566, 926 and 799 at 4,000).
 extern "C" int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int ksplit) {
-  if (ksplit <= 1 || M <= 64 || !takes_tiles(M, N, K, lda, ldw)) return 0;
+  if (ksplit <= 1 || M <= 64 || !takes_whole(M, N, K, lda, ldw)) return 0;
   double apart, whole;
   best_tile(M, N, part_of(K, ksplit), ksplit, &apart);
   best_tile(M, N, K, 1, &whole);
@@ -673,7 +642,7 @@ extern "C" int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int k
 
 extern "C" int pyre_gemm_f32_whole(const float* A, long lda, const float* W, long ldw, float* out, long ldo, int M, int N, int K,
                                    int ksplit, hipStream_t stream) {
-  PYRE_REQUIRE(takes_tiles(M, N, K, lda, ldw) && lda >= K && ldw >= K && ldo >= N && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
+  PYRE_REQUIRE(takes_whole(M, N, K, lda, ldw) && lda >= K && ldw >= K && ldo >= N && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(W) % 16 == 0,
                "gemm_f32_whole: M=%d (more than 16) N=%d K=%d (a multiple of 16) lda=%ld ldw=%ld (of 4) are not supported", M, N, K, lda, ldw);
   PYRE_REQUIRE(ksplit >= 1 && ksplit <= 64 && static_cast<long>(ksplit - 1) * part_of(K, ksplit) < K, "gemm_f32_whole: ksplit=%d", ksplit);
@@ -692,8 +661,8 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
   if (M == 0) return 0;
   const int kper = part_of(K, ksplit);
   PYRE_REQUIRE(static_cast<long>(ksplit - 1) * kper < K, "gemm_f32: a part of k would be empty (K=%d, ksplit=%d)", K, ksplit);
-  // 16-byte loads along k need rows that start on 16 bytes
-  const int vec_ok = lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
+  // loads that go straight into LDS, 16 bytes a lane, need rows that start on 16 bytes
+  const bool vec_ok = lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(W) % 16 == 0;
   const int chain = chain_of(K, ksplit);
   if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows
@@ -705,19 +674,14 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
                  : c == 4 ? launch(launch_stream<4>)
                           : launch(launch_stream<5>),
                  "gemm_f32: no device, or too little LDS");
-  } else if (vec_ok && takes_tiles(M, N, K, lda, ldw)) {
+  } else if (takes_tiles(M, N, K)) {
     launch_tiles(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, stream);
-  } else if (M <= 32) {  // four waves side by side along n
-    const dim3 grid((N + 127) / 128, (M + 31) / 32, ksplit);
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<4, 1, 1, 1>), grid, dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
-                       static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),
-                       static_cast<size_t>(part_stride), M, N, K, kper, chain, vec_ok);
   } else {
-    const dim3 grid((N + 127) / 128, (M + 127) / 128, ksplit);
-    PYRE_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d too large for one launch", M);
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<2, 2, 2, 2>), grid, dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
-                       static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),
-                       static_cast<size_t>(part_stride), M, N, K, kper, chain, vec_ok);
+    const long mt = (M + 31) / 32, blocks = mt * ((N + 127) / 128);
+    PYRE_REQUIRE(blocks < (1L << 24), "gemm_f32: M=%d N=%d are more than a launch holds", M, N);
+    hipLaunchKernelGGL(gemm_f32_mfma_kernel, dim3(static_cast<unsigned>(blocks), 1, ksplit), dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
+                       static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper,
+                       chain, static_cast<int>(mt));
   }
   return check_launch("gemm_f32");
 }

@@ -115,3 +115,28 @@ def test_parts_added_where_they_are_made(n, k, ks):
         out = torch.full((m, n), float("nan"), device=DEV)
         ops.gemm_f32_whole(a, w, out, m, ks)
         assert torch.equal(out, want), m
+
+
+@pytest.mark.parametrize("n,k,ks,off", [(48, 20, 1, 0), (130, 1524, 2, 0), (200, 8, 1, 0), (130, 1529, 2, 1), (77, 23, 1, 3), (70, 9, 1, 1),
+                                        (1536, 1110, 3, 2), (200, 1104, 3, 1), (130, 272, 1, 0), (65, 5, 1, 0), (33, 7, 1, 1), (40, 1, 1, 0),
+                                        (4608, 60, 1, 1), (9000, 45, 1, 0)])
+def test_k_that_ends_within_a_step_and_rows_that_start_anywhere(n, k, ks, off):
+    """The bits of the same product with zeros behind k, up to whole steps, and with rows on 16 bytes. What lies behind the rows and
+    before them is not a number."""
+    from pyre_amd.hip import ops
+
+    m, whole = 600, -(-k // 16) * 16
+    assert ops.f32_part(k, ks) == ops.f32_part(whole, ks)
+    a, w = rnd(m, k, seed=1), rnd(n, k, seed=2)
+
+    def laid(x, step):
+        rows = torch.full((x.shape[0], off + k + step), float("nan"), device=DEV)
+        rows[:, off:off + k] = x
+        return rows[:, off:off + k]
+
+    pad = torch.nn.functional.pad
+    for rows in (1, 31, 32, 33, 64, 65, 129, 400, 600):
+        want, out = torch.empty(ks, rows, n, device=DEV), torch.full((ks, rows, n), float("nan"), device=DEV)
+        ops.gemm_f32(pad(a[:rows], (0, whole - k)), pad(w, (0, whole - k)), None, want if ks > 1 else want[0], rows, ks)
+        ops.gemm_f32(laid(a[:rows], 0), laid(w, 3 if off else 0), None, out if ks > 1 else out[0], rows, ks)
+        assert torch.equal(out, want), rows
