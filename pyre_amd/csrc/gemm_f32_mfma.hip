@@ -10,7 +10,7 @@
 // multiply-adds rounds 16 times, and the sum is made in pieces that are added in float32 (below). Distance from 64 bits,
 // root mean square over that of the values, against the float32 instruction on the same numbers: 1.9e-7 and 7.1e-7 for sums of
 // 1,536 products, 2.5e-7 and 1.6e-6 of 8,960, and 4.0e-7 and 4.8e-7 for a single chain of 640. Numbers that
-// a bfloat16 cannot hold the pieces of (infinities and those within 2^-9 of the largest) give a sum that is not finite: such an
+// a bfloat16 cannot hold the pieces of (infinities and, with the scale below, those from 2^104 on) give a sum that is not finite: such an
 // element is made again as a chain of fused multiply-adds.
 //
 // As in the weight-streaming kernels the product is computed transposed, out^T = W A^T: the
@@ -42,21 +42,39 @@ constexpr int BK = 16;        // k per step
 constexpr int LD = BK + 4;    // floats per LDS row of the general kernel
 constexpr int kChain = 8;     // steps of a chain of a product in one part
 
-// Eight float32 as three times eight bfloat16 that sum to them.
+// Operands are split 2^kUp times as large, so that the last piece of the smallest float32 (a multiple of 2^-149) is still a normal
+// bfloat16 (2^-126 and more); the sums come down again where a part ends. Below about 2^-110 the third piece would otherwise lose bits (an
+// operand around 2^-118 1.5e-5 of it, one around 2^-126 4e-3). It is two vector instructions of thirteen in the split and costs two to
+// four per cent of a product (us, the 7B shape's gate/up 2,805 -> 2,899 at 2,000 rows, 92 -> 96 at 8; the 1.5B shape's 28.3 -> 29.0 at 8).
+// Numbers from 2^104 and sums from 2^80 on are not finite on the way and are made again (`finish`). (A residual as one
+// v_dot2_f32_bf16 instead of a shift and a subtraction is exact too and slower: 2,849 -> 3,145.)
+constexpr int kUp = 24;
+__device__ inline float down(float sum) { return __builtin_amdgcn_ldexpf(sum, -2 * kUp); }
+
+// Eight float32 as three times eight bfloat16 that sum to 2^kUp times them.
 struct Pieces {
   u32x4 p[3];
 };
+// FUSED: the first residual straight from the operand, a shorter chain of larger instructions, for code that is not fetched anew
+// by every launch (tiles).
+template <bool FUSED = false>
 __device__ inline Pieces split8(f32x4 lo, f32x4 hi) {
+#pragma clang fp contract(off)
+  float up = 1 << kUp;  // these two from scalar registers: half the bytes of instructions that hold a constant
+  uint32_t high = 0xffff0000u;
+  if (!FUSED) asm("" : "+s"(up), "+s"(high));
   Pieces r;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float a = i < 2 ? lo[2 * i] : hi[2 * i - 4], b = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
+    const float a0 = i < 2 ? lo[2 * i] : hi[2 * i - 4], b0 = i < 2 ? lo[2 * i + 1] : hi[2 * i - 3];
+    float a = a0 * up, b = b0 * up;
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       const uint32_t w = pack_bf16x2(a, b);
       r.p[t][i] = w;
-      a -= __uint_as_float(w << 16);
-      b -= __uint_as_float(w & 0xffff0000u);
+      const float wa = __uint_as_float(w << 16), wb = __uint_as_float(w & high);
+      a = FUSED && t == 0 ? __builtin_fmaf(a0, up, -wa) : a - wa;
+      b = FUSED && t == 0 ? __builtin_fmaf(b0, up, -wb) : b - wb;
     }
   }
   return r;
@@ -69,9 +87,11 @@ __device__ inline f32x16 multiply(u32x4 w, u32x4 a, f32x16 acc) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, a), acc, 0, 0, 0);
 }
 
-// Output columns n .. n + 3 of a row; whether one of their sums is not finite.
-__device__ inline bool store4(f32x4 v, float* row, bool rows_of_16, int n, int N) {
+// Output columns n .. n + 3 of a row, their sums still `up`; whether one of them is not finite.
+__device__ inline bool store4(f32x4 v, bool up, float* row, bool rows_of_16, int n, int N) {
   bool bad = false;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = up ? down(v[j]) : v[j];
 #pragma unroll
   for (int j = 0; j < 4; ++j) bad |= !(fabsf(v[j]) < INFINITY);
   if (n + 3 < N && rows_of_16) {
@@ -162,7 +182,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   if (m < M) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, out + static_cast<size_t>(m) * ldo,
+      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, true, out + static_cast<size_t>(m) * ldo,
                     rows_of_16, n + 8 * i, N);
   }
   if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, 1, M, n, 1, N, K - kbeg);
@@ -187,8 +207,8 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
 //
 // A chain of instructions ends after `chain` steps and is added to the total in float32. A block that walks all parts of k
 // (where the rows alone fill the chip) ends its chains where the parts end: the bits of the consumer's sum of partial sums, which
-// then do not go through memory.
-template <int BM, int BN, int WM, int WN, int SL, int OCC, bool TAIL>
+// then do not go through memory (WHOLE: every part's sum comes down by itself, as in memory).
+template <int BM, int BN, int WM, int WN, int SL, int OCC, bool TAIL, bool WHOLE>
 __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
     const float* A, long lda, const float* W, long ldw, const void* __restrict__ bias,
     int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int chain, int mt, int nt) {
@@ -247,7 +267,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
           }
       if (by >= 8) lo = hi = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const Pieces v = split8(lo, hi);
+    const Pieces v = split8<true>(lo, hi);
 #pragma unroll
     for (int s = 0; s < 3; ++s) *reinterpret_cast<u32x4*>(lds + buf * BUF + s * PLANE + dst[i]) = v.p[s];
   };
@@ -267,7 +287,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
       for (int q = 0; q < CT; ++q)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          total[r][q][i] += acc[r][q][i];
+          total[r][q][i] += WHOLE ? down(acc[r][q][i]) : acc[r][q][i];
           acc[r][q][i] = 0.f;
         }
   };
@@ -333,7 +353,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
     for (int r = 0; r < RT; ++r)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]},
+        bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]}, !WHOLE,
                       out + static_cast<size_t>(m + 32 * q) * ldo, rows_of_16, n + 32 * r + 8 * i, N);
   }
   if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len);
@@ -500,7 +520,7 @@ __global__ __launch_bounds__(64 * (2 * C + kRowWaves)) void gemm_f32_stream_kern
 #pragma unroll
     for (int s = 0; s < kTerms; ++s) {
       __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // a matrix instruction,
-      __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);  // eight vector instructions
+      __builtin_amdgcn_sched_group_barrier(0x2, 9, 0);  // nine vector instructions
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -537,7 +557,7 @@ __global__ __launch_bounds__(64 * (2 * C + kRowWaves)) void gemm_f32_stream_kern
   if (c < M) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, out + static_cast<size_t>(c) * ldo,
+      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, true, out + static_cast<size_t>(c) * ldo,
                     rows_of_16, n0 + 4 * half + 8 * i, N);
   }
   if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, c, 1, M, n0 + 4 * half, 1, N, K - kbeg);
@@ -607,9 +627,9 @@ bool takes_whole(int M, int N, int K, long lda, long ldw) {
   return M > 16 && lda % 4 == 0 && ldw % 4 == 0 && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32) && takes_tiles(M, N, K);
 }
 
-// Chains of `chain` steps.
+// Chains of `chain` steps. `whole`: in one part, whose chains are the parts of a product in several.
 void launch_tiles(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
-                  int M, int N, int K, int kper, int parts, int chain, hipStream_t stream) {
+                  int M, int N, int K, int kper, int parts, int chain, bool whole, hipStream_t stream) {
   const auto tile = [&](auto kernel, int bm, int bn) {
     const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * nt * parts), dim3(256), 0, stream, A, lda, W, ldw, bias, bias_dt, out,
@@ -617,9 +637,14 @@ void launch_tiles(const float* A, long lda, const float* W, long ldw, const void
   };
   const int best = best_tile(M, N, kper, parts, nullptr);
   const bool tail = K % BK != 0;
-  if (best == 0) tile(tail ? gemm_f32_tile_kernel<128, 128, 2, 2, 1, 2, true> : gemm_f32_tile_kernel<128, 128, 2, 2, 1, 2, false>, 128, 128);
-  else if (best == 1) tile(tail ? gemm_f32_tile_kernel<64, 128, 2, 2, 2, 2, true> : gemm_f32_tile_kernel<64, 128, 2, 2, 2, 2, false>, 64, 128);
-  else tile(tail ? gemm_f32_tile_kernel<64, 64, 2, 2, 2, 3, true> : gemm_f32_tile_kernel<64, 64, 2, 2, 2, 3, false>, 64, 64);
+#define PYRE_F32_TILE(BM, BN, SL, OCC)                                                    \
+  tile(whole  ? gemm_f32_tile_kernel<BM, BN, 2, 2, SL, OCC, false, true>                  \
+       : tail ? gemm_f32_tile_kernel<BM, BN, 2, 2, SL, OCC, true, false>                  \
+              : gemm_f32_tile_kernel<BM, BN, 2, 2, SL, OCC, false, false>, BM, BN)
+  if (best == 0) PYRE_F32_TILE(128, 128, 1, 2);
+  else if (best == 1) PYRE_F32_TILE(64, 128, 2, 2);
+  else PYRE_F32_TILE(64, 64, 2, 3);
+#undef PYRE_F32_TILE
 }
 
 int part_of(int K, int ksplit) { return ((K + ksplit - 1) / ksplit + BK - 1) / BK * BK; }
@@ -646,7 +671,7 @@ extern "C" int pyre_gemm_f32_whole(const float* A, long lda, const float* W, lon
                    reinterpret_cast<uintptr_t>(W) % 16 == 0,
                "gemm_f32_whole: M=%d (more than 16) N=%d K=%d (a multiple of 16) lda=%ld ldw=%ld (of 4) are not supported", M, N, K, lda, ldw);
   PYRE_REQUIRE(ksplit >= 1 && ksplit <= 64 && static_cast<long>(ksplit - 1) * part_of(K, ksplit) < K, "gemm_f32_whole: ksplit=%d", ksplit);
-  launch_tiles(A, lda, W, ldw, nullptr, 0, out, ldo, 0, M, N, K, K, 1, chain_of(K, ksplit), stream);
+  launch_tiles(A, lda, W, ldw, nullptr, 0, out, ldo, 0, M, N, K, K, 1, chain_of(K, ksplit), ksplit > 1, stream);
   return check_launch("gemm_f32_whole");
 }
 
@@ -675,7 +700,7 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
                           : launch(launch_stream<5>),
                  "gemm_f32: no device, or too little LDS");
   } else if (takes_tiles(M, N, K)) {
-    launch_tiles(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, stream);
+    launch_tiles(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, false, stream);
   } else {
     const long mt = (M + 31) / 32, blocks = mt * ((N + 127) / 128);
     PYRE_REQUIRE(blocks < (1L << 24), "gemm_f32: M=%d N=%d are more than a launch holds", M, N);

@@ -54,3 +54,25 @@ def test_infinities_and_the_largest_numbers(m, n, k, ks, off):
         # roundings of 2^-24 of the largest partial sum: the row's scale is that of its largest product
         scale = (b.double().abs() @ w.double().abs().T)[fine]
         assert bool(((got - want)[fine].abs() <= 2.0 ** -22 * scale + 1e-30).all()), (value, row)
+
+
+@pytest.mark.parametrize("m,n,k,ks,off", FORMS)
+@pytest.mark.parametrize("low,high", [(-108, 100), (-113, 60), (-118, 100), (-126, 110), (-140, 100), (-70, -70), (45, 50)])
+def test_small_and_large_operands(m, n, k, ks, off, low, high):
+    """Small activations times large weights and the other way round, subnormal numbers among them; sums that are small themselves;
+    sums that leave the range of the scaled pieces (2^80) and not that of a float32."""
+    from pyre_amd.hip import ops
+
+    a, w = operands(m, n, k, off)
+    w = w * 50.0
+    for ea, ew in ((low, high), (high, low)):
+        x, y = torch.ldexp(a.double(), torch.tensor(float(ea), device=DEV)).float(), torch.ldexp(w.double(), torch.tensor(float(ew), device=DEV)).float()
+        if off:
+            x = torch.nn.functional.pad(x, (off, 0))[:, off:]
+        out, chain = torch.full((ks, m, n), float("nan"), device=DEV), torch.empty(m, n, device=DEV)
+        ops.gemm_f32(x, y, None, out if ks > 1 else out[0], m, ks)
+        ops.gemm_generic(x, y, None, chain, m)
+        want = x.double() @ y.double().T
+        err, err_chain, rms = (float(v.square().mean().sqrt()) for v in (out.double().sum(0) - want, chain.double() - want, want))
+        # what is left out of a product is at most 2^-24 of it, what a result below 2^-126 cannot hold at most 2^-149 for each part
+        assert err <= 1.1 * err_chain + 2.0 ** -24 * rms + ks * 2.0 ** -149, (ea, ew)
