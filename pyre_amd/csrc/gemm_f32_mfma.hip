@@ -11,7 +11,7 @@
 // root mean square over that of the values, against the float32 instruction on the same numbers: 1.9e-7 and 7.1e-7 for sums of
 // 1,536 products, 2.5e-7 and 1.6e-6 of 8,960, and 4.0e-7 and 4.8e-7 for a single chain of 640. Numbers that
 // a bfloat16 cannot hold the pieces of (infinities and, with the scale below, those from 2^104 on) give a sum that is not finite: such an
-// element is made again as a chain of fused multiply-adds.
+// element is made again on the float32 instruction.
 //
 // As in the weight-streaming kernels the product is computed transposed, out^T = W A^T: the
 // 32 rows of an MFMA tile are output columns n, its 32 columns are rows m, so that a lane
@@ -103,22 +103,78 @@ __device__ inline bool store4(f32x4 v, bool up, float* row, bool rows_of_16, int
   return bad;
 }
 
-// What the usual product does not need, over the elements that this lane has stored (of rows m, m + 32, .., column groups of four
-// at n + 8 i): the sums that are not finite once more, without pieces (`a` and `w` are the rows of A and W at the part's first k of
-// `len`), and the bias.
-__device__ inline void finish(const float* a, size_t lda, const float* w, size_t ldw, const void* bias, int bias_dt, float* out,
-                              size_t ldo, int m, int mtiles, int M, int n, int ntiles, int N, int len) {
+// What the usual product does not need: the sums that are not finite once more, and the bias, over a wave's tiles of 32 x 32 (this
+// lane's are rows m + 32 q and column groups of four at n + 32 r + 8 i; `a` and `w` are the operands at the part's first k of `len`).
+// Infinities, numbers that are not one and those beyond the pieces' range go through the float32 instruction as they are, the whole tile
+// in the same steps and chains, of which the elements are kept that were not finite. A row with such a number costs its own tiles
+// this much (us, a launch by itself without and with one such row: the 1.5B shape's gate/up 38 and 91 at 20 rows, the 7B shape's 97 and
+// 294, 937 and 1,360 at 566; all rows 3,801). An element made by one lane, k by k, held the step up for 2,142, 6,140, 13,530 and 160,351.
+constexpr int kAgain = 4;  // steps whose operands are asked for together
+__device__ inline void finish(bool bad, const float* a, size_t lda, const float* w, size_t ldw, const void* bias, int bias_dt, float* out,
+                              size_t ldo, int m, int mtiles, int M, int n, int ntiles, int N, int len, int chain) {
+  const int c = threadIdx.x & 31, half = threadIdx.x >> 5 & 1;
+  if (__ballot(bad)) {
+#pragma unroll 1
+    for (int t = 0; t < mtiles * ntiles; ++t) {
+      const int row = m + 32 * (t / ntiles), col = n + 32 * (t % ntiles);
+      bool again = false;
+#pragma unroll 1
+      for (int e = 0; e < 16; ++e) {
+        const int at = col + 8 * (e / 4) + e % 4;
+        if (row < M && at < N) again |= !(fabsf(out[row * ldo + at]) < INFINITY);
+      }
+      if (!__ballot(again)) continue;
+      // rows and columns past the end are the last one once more
+      const float* const x = a + static_cast<size_t>(min(row, M - 1)) * lda + 8 * half;
+      const float* const y = w + static_cast<size_t>(min(col - 4 * half + c, N - 1)) * ldw + 8 * half;
+      f32x16 acc, total;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] = total[i] = 0.f;
+      int left = chain;
+#pragma unroll 1
+      for (int k0 = 0; k0 < len; k0 += kAgain * BK) {
+        f32x4 xs[kAgain][2], ys[kAgain][2];
+#pragma unroll
+        for (int u = 0; u < kAgain; ++u)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int k = k0 + BK * u + 4 * h, there = len - 8 * half - k;
+            if (there >= 4) {
+              xs[u][h] = *reinterpret_cast<const f32x4_any*>(x + k);
+              ys[u][h] = *reinterpret_cast<const f32x4_any*>(y + k);
+            } else {
+#pragma unroll
+              for (int j = 0; j < 4; ++j) xs[u][h][j] = j < there ? x[k + j] : 0.f, ys[u][h][j] = j < there ? y[k + j] : 0.f;
+            }
+          }
+#pragma unroll
+        for (int u = 0; u < kAgain; ++u) {
+          if (k0 + BK * u >= len) break;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ys[u][j >> 2][j & 3], xs[u][j >> 2][j & 3], acc, 0, 0, 0);
+          if (--left == 0) {
+            left = chain;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              total[i] += acc[i];
+              acc[i] = 0.f;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int at = col + 8 * (i / 4) + i % 4;
+        float* const p = out + row * ldo + at;
+        if (row < M && at < N && !(fabsf(*p) < INFINITY)) *p = total[i] + acc[i];
+      }
+    }
+  }
+  if (!bias) return;
 #pragma unroll 1
   for (int e = 0; e < 16 * mtiles * ntiles; ++e) {
     const int row = m + 32 * (e / (16 * ntiles)), col = n + 8 * (e / 4 % (4 * ntiles)) + e % 4;
-    if (row >= M || col >= N) continue;
-    float s = out[row * ldo + col];
-    if (!(fabsf(s) < INFINITY)) {
-      s = 0.f;
-#pragma unroll 1
-      for (int k = 0; k < len; ++k) s = fmaf(a[row * lda + k], w[col * ldw + k], s);
-    }
-    out[row * ldo + col] = s + (bias ? load_as_float(bias, bias_dt, col) : 0.f);
+    if (row < M && col < N) out[row * ldo + col] += load_as_float(bias, bias_dt, col);
   }
 }
 
@@ -185,7 +241,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
       bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, true, out + static_cast<size_t>(m) * ldo,
                     rows_of_16, n + 8 * i, N);
   }
-  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, 1, M, n, 1, N, K - kbeg);
+  finish(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, 1, M, n, 1, N, K - kbeg, chain);
 }
 
 // More than 32 rows, and fewer where they do not start on 16 bytes. A block of four waves keeps BM rows of A and BN rows of W; every
@@ -356,7 +412,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
         bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]}, !WHOLE,
                       out + static_cast<size_t>(m + 32 * q) * ldo, rows_of_16, n + 32 * r + 8 * i, N);
   }
-  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len);
+  finish(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len, chain);
 }
 
 constexpr int kStreamMaxRows = 32;
@@ -560,7 +616,7 @@ __global__ __launch_bounds__(64 * (2 * C + kRowWaves)) void gemm_f32_stream_kern
       bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, true, out + static_cast<size_t>(c) * ldo,
                     rows_of_16, n0 + 4 * half + 8 * i, N);
   }
-  if (bad || bias) finish(A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, c, 1, M, n0 + 4 * half, 1, N, K - kbeg);
+  finish(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, c, 1, M, n0 + 4 * half, 1, N, K - kbeg, chain);
 }
 
 template <int C>

@@ -76,3 +76,29 @@ def test_small_and_large_operands(m, n, k, ks, off, low, high):
         err, err_chain, rms = (float(v.square().mean().sqrt()) for v in (out.double().sum(0) - want, chain.double() - want, want))
         # what is left out of a product is at most 2^-24 of it, what a result below 2^-126 cannot hold at most 2^-149 for each part
         assert err <= 1.1 * err_chain + 2.0 ** -24 * rms + ks * 2.0 ** -149, (ea, ew)
+
+
+@pytest.mark.parametrize("m,n,k", [(20, 17920, 1536), (300, 4608, 3584)])
+def test_a_row_that_is_not_finite_does_not_hold_up_the_others(m, n, k):
+    """Its elements are made again on a slower instruction: a few times the step's time (2 to 3 measured), not a hundred times."""
+    from pyre_amd.hip import ops
+
+    a, w = operands(m, n, k, 0)
+    out = torch.empty(m, n, device=DEV)
+
+    def least_time(x):
+        times = []
+        for _ in range(6):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            ops.gemm_f32(x, w, None, out, m)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(begin.elapsed_time(end))
+        return min(times)
+
+    fine = least_time(a)
+    for value in (float("nan"), float("inf"), 3e38):
+        b = a.clone()
+        b[m // 2, 5] = value
+        assert least_time(b) < 12 * fine, value
