@@ -109,9 +109,11 @@ __device__ inline bool store4(f32x4 v, bool up, float* row, bool rows_of_16, int
 // in the same steps and chains, of which the elements are kept that were not finite. A row with such a number costs its own tiles
 // this much (us, a launch by itself without and with one such row: the 1.5B shape's gate/up 38 and 91 at 20 rows, the 7B shape's 97 and
 // 294, 937 and 1,360 at 566; all rows 3,801). An element made by one lane, k by k, held the step up for 2,142, 6,140, 13,530 and 160,351.
-constexpr int kAgain = 4;  // steps whose operands are asked for together
+// PARTS: a chain is a part of k, whose sums are what the part would be by itself, of pieces where that is finite.
+template <bool PARTS = false>
 __device__ inline void finish(bool bad, const float* a, size_t lda, const float* w, size_t ldw, const void* bias, int bias_dt, float* out,
                               size_t ldo, int m, int mtiles, int M, int n, int ntiles, int N, int len, int chain) {
+  constexpr int kAgain = PARTS ? 1 : 4;  // steps whose operands are asked for together
   const int c = threadIdx.x & 31, half = threadIdx.x >> 5 & 1;
   if (__ballot(bad)) {
 #pragma unroll 1
@@ -127,9 +129,17 @@ __device__ inline void finish(bool bad, const float* a, size_t lda, const float*
       // rows and columns past the end are the last one once more
       const float* const x = a + static_cast<size_t>(min(row, M - 1)) * lda + 8 * half;
       const float* const y = w + static_cast<size_t>(min(col - 4 * half + c, N - 1)) * ldw + 8 * half;
-      f32x16 acc, total;
+      f32x16 acc, sum, total;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[i] = total[i] = 0.f;
+      for (int i = 0; i < 16; ++i) acc[i] = sum[i] = total[i] = 0.f;
+      auto end_chain = [&]() {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float of_pieces = down(sum[i]);
+          total[i] += PARTS && fabsf(of_pieces) < INFINITY ? of_pieces : acc[i];
+          acc[i] = sum[i] = 0.f;
+        }
+      };
       int left = chain;
 #pragma unroll 1
       for (int k0 = 0; k0 < len; k0 += kAgain * BK) {
@@ -149,24 +159,26 @@ __device__ inline void finish(bool bad, const float* a, size_t lda, const float*
           }
 #pragma unroll
         for (int u = 0; u < kAgain; ++u) {
-          if (k0 + BK * u >= len) break;
+          if (u > 0 && k0 + BK * u >= len) continue;
 #pragma unroll
           for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ys[u][j >> 2][j & 3], xs[u][j >> 2][j & 3], acc, 0, 0, 0);
+          if (PARTS) {
+            const Pieces p = split8<true>(ys[u][0], ys[u][1]), q = split8<true>(xs[u][0], xs[u][1]);
+#pragma unroll
+            for (int s = 0; s < kTerms; ++s) sum = multiply(p.p[kTermW[s]], q.p[kTermA[s]], sum);
+          }
           if (--left == 0) {
             left = chain;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              total[i] += acc[i];
-              acc[i] = 0.f;
-            }
+            end_chain();
           }
         }
       }
+      end_chain();  // a last, shorter one (or nothing)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int at = col + 8 * (i / 4) + i % 4;
         float* const p = out + row * ldo + at;
-        if (row < M && at < N && !(fabsf(*p) < INFINITY)) *p = total[i] + acc[i];
+        if (row < M && at < N && !(fabsf(*p) < INFINITY)) *p = total[i];
       }
     }
   }
@@ -412,7 +424,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
         bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]}, !WHOLE,
                       out + static_cast<size_t>(m + 32 * q) * ldo, rows_of_16, n + 32 * r + 8 * i, N);
   }
-  finish(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len, chain);
+  finish<WHOLE>(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len, chain);
 }
 
 constexpr int kStreamMaxRows = 32;
@@ -719,6 +731,13 @@ extern "C" int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int k
   best_tile(M, N, part_of(K, ksplit), ksplit, &apart);
   best_tile(M, N, K, 1, &whole);
   return whole < apart;
+}
+
+// Which of the tiles' sizes a product of more than 32 rows takes (`ksplit` parts, or 1: also for the sums of all parts).
+extern "C" int pyre_gemm_f32_tile_choice(int M, int N, int K, int ksplit) {
+  PYRE_REQUIRE(M > 0 && N > 0 && K > 0 && ksplit > 0, "gemm_f32_tile_choice: bad sizes");
+  const int i = best_tile(M, N, part_of(K, ksplit), ksplit, nullptr);
+  return 1000 * kTiles[i].bm + kTiles[i].bn;
 }
 
 extern "C" int pyre_gemm_f32_whole(const float* A, long lda, const float* W, long ldw, float* out, long ldo, int M, int N, int K,

@@ -55,6 +55,7 @@ _SIGNATURES = {
     "pyre_feed_tokens": [P, P, P, I, P],
     "pyre_gemm_skinny_glu_bf16": [P, L, P, L, P, I, I, I, F, F, F, F, P],
     "pyre_gemm_f32_adds": [I, I, I, L, L, I],
+    "pyre_gemm_f32_tile_choice": [I, I, I, I],
     "pyre_gemm_f32_whole": [P, L, P, L, P, L, I, I, I, I, P],
     "pyre_gemm_tile_supports": [I, I, I, L, L],
     "pyre_gemm_tile_choice": [I, I, I, I, I, P],

@@ -102,3 +102,37 @@ def test_a_row_that_is_not_finite_does_not_hold_up_the_others(m, n, k):
         b = a.clone()
         b[m // 2, 5] = value
         assert least_time(b) < 12 * fine, value
+
+
+#: sums of all parts in tiles of each size (rows x columns)
+WHOLES = [(100, 1536, 1104, 3, (64, 64)), (300, 6000, 560, 2, (64, 128)), (300, 8960, 560, 2, (128, 128))]
+
+
+@pytest.mark.parametrize("m,n,k,ks,tile", WHOLES)
+def test_numbers_beyond_the_pieces_have_the_bits_of_parts_added_in_order(m, n, k, ks, tile):
+    """Numbers from 2^104 on, the largest, infinities and not-a-numbers, in rows of several row tiles and in one part of k or in all:
+    whether a block adds the parts up itself or their consumer does."""
+    from pyre_amd.hip import ops
+    from pyre_amd.hip.lib import lib
+
+    assert lib().pyre_gemm_f32_tile_choice(m, n, k, 1) == 1000 * tile[0] + tile[1]
+    a, w = operands(m, n, k, 0)
+    w[:, 5] *= 1e-31  # under a number of 1e32 its products are as large as the others', whose parts the element keeps
+    for row, value, places in ((0, 3e38, (3,)), (33, 1e32, (5,)), (65, -3e32, (5,)), (m - 1, -3e38, (k - 2,)), (40, float("inf"), (k // 2,)),
+                               (70, float("nan"), (1,)), (m - 2, 2e35, range(0, k, 7)), (m // 2, 1e30, (2, k // 2))):
+        a[row, list(places)] = value
+    w[n - 1, 4], w[n // 2, k - 3] = 1e33, -2e31
+    parts, whole = torch.empty(ks, m, n, device=DEV), torch.full((m, n), float("nan"), device=DEV)
+    ops.gemm_f32(a, w, None, parts, m, ks)
+    ops.gemm_f32_whole(a, w, whole, m, ks)
+    want = parts[0].clone()
+    for p in parts[1:]:
+        want += p
+    assert torch.equal(whole.isnan(), want.isnan()) and torch.equal(whole.nan_to_num(), want.nan_to_num())
+    exact = a.double() @ w.double().T
+    fine, scale = exact.abs() < 1e38, a.double().abs() @ w.double().abs().T
+    assert bool(((want.double() - exact)[fine].abs() <= 2.0 ** -21 * scale[fine]).all())
+    rows = torch.tensor([0, 33, 40, 65, 70, m // 2, m - 1], device=DEV)  # in a step of few rows
+    few = torch.empty(ks, len(rows), n, device=DEV)
+    ops.gemm_f32(a[rows].contiguous(), w, None, few, len(rows), ks)
+    assert torch.equal(few.nan_to_num(), parts[:, rows].nan_to_num())
