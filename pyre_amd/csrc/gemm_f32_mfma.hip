@@ -3,13 +3,22 @@
 // of mixed element types stay with gemm_generic.hip.
 //
 // The matrix cores' float32 instruction has a sixteenth of the 16-bit instruction's rate, so the products are made of bfloat16
-// pieces: a float32 is the sum of three, x = h + m + l with eight bits each, exactly, and a product of two bfloat16 is exact in
-// float32. Of the nine products of pieces the six largest are added, l h', h l', m m', m h', h m' and h h' in this order; what
-// is left out (m l', l m', l l') is below 2^-26 of the product, less than the rounding of a float32 product. An instruction
-// adds sixteen products of each kind at once, so that an element's sum is rounded six times for 16 k where a chain of fused
-// multiply-adds rounds 16 times, and the sum is made in pieces that are added in float32 (below). Distance from 64 bits,
-// root mean square over that of the values, against the float32 instruction on the same numbers: 1.9e-7 and 7.1e-7 for sums of
-// 1,536 products, 2.5e-7 and 1.6e-6 of 8,960, and 4.0e-7 and 4.8e-7 for a single chain of 640. Numbers that
+// pieces: a float32 is the sum of three, x = h + m + l with eight bits each, exactly (with the scale below), and a product of two
+// bfloat16 is exact in float32 (G. Henry, P. Tang, A. Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", 2019). Of the nine products of pieces the six largest are added, l h', h l', m m', m h', h m' and
+// h h' in this order; what is left out (m l', l m', l l') is at most 2^-24 of the product, |m| being up to 2^-8 and |l| up to 2^-17 of
+// x, and 2^-27.4 in root mean square. An instruction adds sixteen products of each kind at once, so that an element's sum is rounded six
+// times for 16 k where a chain of fused multiply-adds rounds 16 times, and the sum is made in chains that are added in float32 (below).
+//
+// Measured distance from 64 bits, root mean square over that of the values, here and of the float32 instruction on the same numbers;
+// "repeated" is one pair of numbers in [1, 2) a sum, whose roundings all go one way:
+//   products            8          16          128         1,536       8,960     part of 640  part of 2,112  part of 4,608
+//   random signs  3.1 5.4e-8  3.3 7.1e-8  1.6 2.0e-7  1.8 7.1e-7  2.4 17e-7   3.8 4.5e-7    7.1 8.2e-7     1.1 1.2e-6
+//   positive      2.6 4.6e-8  3.3 6.2e-8  1.3 1.6e-7  0.7 5.8e-7  1.3 14e-7   2.8 3.9e-7    4.2 6.6e-7     0.6 1.0e-6
+//   repeated      2.5 5.4e-8  3.3 11e-8   3.0 9.2e-7  3.1 113e-7  6.0 658e-7  1.7 4.7e-6    3.9 15.6e-6    8.1 34.0e-6
+// The largest error of an element, over the sum of its products' sizes: 0.9e-7 and 2.3e-7 for 8 random products, 0.3e-6 and 2.6e-6
+// for 1,536 positive ones. Sums of one or two products are the exception (3.4e-8 and 2.6e-8 for one, at most 1.5e-7 and 6e-8), also where
+// all others of a longer sum are far smaller; fewer than eight k are left to the float32 instruction. Numbers that
 // a bfloat16 cannot hold the pieces of (infinities and, with the scale below, those from 2^104 on) give a sum that is not finite: such an
 // element is made again on the float32 instruction.
 //
@@ -39,7 +48,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 constexpr int BK = 16;        // k per step
-constexpr int LD = BK + 4;    // floats per LDS row of the general kernel
 constexpr int kChain = 8;     // steps of a chain of a product in one part
 
 // Operands are split 2^kUp times as large, so that the last piece of the smallest float32 (a multiple of 2^-149) is still a normal
@@ -190,70 +198,29 @@ __device__ inline void finish(bool bad, const float* a, size_t lda, const float*
   }
 }
 
-// What the other kernels leave: fewer than eight k, or more tiles than a launch holds. 16 k of both operands at a time through
-// registers and LDS as float32, split by the waves that multiply them: 32 rows of A against 32 columns a wave.
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
-    const float* __restrict__ A, size_t lda, const float* __restrict__ W, size_t ldw,
-    const void* __restrict__ bias, int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M,
-    int N, int K, int kper, int chain, int mt) {
-  __shared__ __attribute__((aligned(16))) float Ws[128][LD];
-  __shared__ __attribute__((aligned(16))) float As[32][LD];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, half = lane >> 5, c = lane & 31;
-  const int n0 = static_cast<int>(blockIdx.x / mt) * 128, m0 = static_cast<int>(blockIdx.x % mt) * 32;
-  const int kbeg = blockIdx.z * kper;
-  K = min(K, kbeg + kper);  // this part's end
-  out += blockIdx.z * part_stride;
-  if (blockIdx.z) bias = nullptr;  // the bias belongs to one part only
-
-  // Four consecutive k of one row; zero where the row or the k is not there.
-  auto load_k4 = [&](const float* base, size_t ld, int row, int rows, int k) {
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (row < rows)
-      for (int j = 0; j < 4 && k + j < K; ++j) v[j] = base[row * ld + k + j];
-    return v;
-  };
-  f32x16 acc, total;
+// Fewer than eight k, on the float32 instruction: a sum of one or two products of pieces is up to twice as far from 64 bits as one of
+// fused multiply-adds. A wave has 32 rows and 32 columns, straight from memory.
+constexpr int kShort = 8;
+__global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __restrict__ A, size_t lda, const float* __restrict__ W, size_t ldw,
+                                                             const void* __restrict__ bias, int bias_dt, float* __restrict__ out, size_t ldo,
+                                                             int M, int N, int K, int mt) {
+  const int wave = threadIdx.x >> 6, half = threadIdx.x >> 5 & 1, c = threadIdx.x & 31;
+  const int n0 = static_cast<int>(blockIdx.x / mt) * 128 + 32 * wave, m = static_cast<int>(blockIdx.x % mt) * 32 + c;
+  // rows and columns past the end are the last one once more and are not stored
+  const float *const a = A + min(m, M - 1) * lda, *const w = W + min(n0 + c, N - 1) * ldw;
+  f32x16 acc;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = total[i] = 0.f;
-  auto end_chain = [&]() {
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      total[i] += acc[i];
-      acc[i] = 0.f;
-    }
-  };
-  int left = chain;
-  for (int k0 = kbeg; k0 < K; k0 += BK) {
-    for (int p = tid; p < 160 * 4; p += 256) {
-      const int row = p / 4, k = 4 * (p % 4);
-      if (row < 128) *reinterpret_cast<f32x4*>(&Ws[row][k]) = load_k4(W, ldw, n0 + row, N, k0 + k);
-      else *reinterpret_cast<f32x4*>(&As[row - 128][k]) = load_k4(A, lda, m0 + row - 128, M, k0 + k);
-    }
-    __syncthreads();
-    const float *w = &Ws[32 * wave + c][8 * half], *a = &As[c][8 * half];
-    const Pieces x = split8(*reinterpret_cast<const f32x4*>(w), *reinterpret_cast<const f32x4*>(w + 4));
-    const Pieces y = split8(*reinterpret_cast<const f32x4*>(a), *reinterpret_cast<const f32x4*>(a + 4));
-#pragma unroll
-    for (int s = 0; s < kTerms; ++s) acc = multiply(x.p[kTermW[s]], y.p[kTermA[s]], acc);
-    if (--left == 0) {
-      end_chain();
-      left = chain;
-    }
-    __syncthreads();
+  for (int j = 0; j < kShort; j += 2) {
+    const int k = j + half;
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < K ? w[k] : 0.f, k < K ? a[k] : 0.f, acc, 0, 0, 0);
   }
-  end_chain();
-
-  // total[4 i + j]: output column n = tile row 8 i + 4 half + j, output row m = tile column c.
-  const bool rows_of_16 = (ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  const int m = m0 + c, n = n0 + 32 * wave + 4 * half;
-  bool bad = false;
-  if (m < M) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      bad |= store4(f32x4{total[4 * i], total[4 * i + 1], total[4 * i + 2], total[4 * i + 3]}, true, out + static_cast<size_t>(m) * ldo,
-                    rows_of_16, n + 8 * i, N);
+  for (int i = 0; i < 16; ++i) {
+    const int n = n0 + 8 * (i / 4) + 4 * half + i % 4;
+    if (m < M && n < N) out[m * ldo + n] = acc[i] + (bias ? load_as_float(bias, bias_dt, n) : 0.f);
   }
-  finish(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, 1, M, n, 1, N, K - kbeg, chain);
 }
 
 // More than 32 rows, and fewer where they do not start on 16 bytes. A block of four waves keeps BM rows of A and BN rows of W; every
@@ -689,7 +656,7 @@ int best_tile(int M, int N, int kper, int parts, double* us) {
 }
 
 // (The last loads of a row lie up to eight k before its end.)
-bool takes_tiles(int M, int N, int K) { return K >= 8 && static_cast<long>((M + 31) / 32) * ((N + 63) / 64) < (1L << 24); }
+bool takes_tiles(int M, int N, int K) { return K >= kShort && static_cast<long>((M + 63) / 64) * ((N + 63) / 64) < (1L << 24); }
 // What is offered as sums of all parts: rows on 16 bytes, whole steps.
 bool takes_whole(int M, int N, int K, long lda, long ldw) {
   return M > 16 && lda % 4 == 0 && ldw % 4 == 0 && K % BK == 0 && 4 * lda * M < (1L << 32) && 4 * ldw * N < (1L << 32) && takes_tiles(M, N, K);
@@ -765,7 +732,12 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
   const bool vec_ok = lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(W) % 16 == 0;
   const int chain = chain_of(K, ksplit);
-  if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows
+  if (K < kShort) {  // (one part: a part has 16 k)
+    const long mt = (M + 31) / 32, blocks = mt * ((N + 127) / 128);
+    PYRE_REQUIRE(blocks < (1L << 24), "gemm_f32: M=%d N=%d are more than a launch holds", M, N);
+    hipLaunchKernelGGL(gemm_f32_short_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
+                       static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo), M, N, K, static_cast<int>(mt));
+  } else if (M <= kStreamMaxRows && vec_ok && K % 4 == 0) {  // a decode step's rows
     const auto launch = [&](auto f) { return f(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, stream); };
     const int c = stream_columns(N, ksplit);
     PYRE_REQUIRE(c == 1   ? launch(launch_stream<1>)
@@ -774,14 +746,9 @@ extern "C" int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw,
                  : c == 4 ? launch(launch_stream<4>)
                           : launch(launch_stream<5>),
                  "gemm_f32: no device, or too little LDS");
-  } else if (takes_tiles(M, N, K)) {
-    launch_tiles(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, false, stream);
   } else {
-    const long mt = (M + 31) / 32, blocks = mt * ((N + 127) / 128);
-    PYRE_REQUIRE(blocks < (1L << 24), "gemm_f32: M=%d N=%d are more than a launch holds", M, N);
-    hipLaunchKernelGGL(gemm_f32_mfma_kernel, dim3(static_cast<unsigned>(blocks), 1, ksplit), dim3(256), 0, stream, A, static_cast<size_t>(lda), W,
-                       static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper,
-                       chain, static_cast<int>(mt));
+    PYRE_REQUIRE(takes_tiles(M, N, K), "gemm_f32: M=%d N=%d are more than a launch holds", M, N);
+    launch_tiles(A, lda, W, ldw, bias, bias_dt, out, ldo, part_stride, M, N, K, kper, ksplit, chain, false, stream);
   }
   return check_launch("gemm_f32");
 }

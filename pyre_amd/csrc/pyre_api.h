@@ -59,9 +59,9 @@ int pyre_gemm_generic(const void* A, int a_dt, long lda, const int* a_rows, cons
 int pyre_fill_rows(void* base, int elem_bytes, long outer_stride, int n_outer, int n_rows, long row_elems,
                    const int* ids_host, int n_ids, unsigned pattern, hipStream_t stream);
 
-// The same for float32 operands and results only, of bfloat16 pieces that sum to the operands exactly (no further from
-// 64 bits than fused multiply-adds): the product of the true 32-bit path. The order of an element's additions depends on k and
-// ksplit alone.
+// The same for float32 operands and results only, of bfloat16 pieces that sum to the operands exactly (measured no further from
+// 64 bits than a chain of fused multiply-adds from eight products on; fewer are one): the product of the true 32-bit path. The order
+// of an element's additions depends on k and ksplit alone.
 // ksplit > 1: partial sums out[s] (part_stride elements apart) over ksplit parts of k, the bias
 // in part 0; the consumer adds them in the order 0..ksplit-1.
 int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt,

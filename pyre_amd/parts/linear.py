@@ -40,7 +40,7 @@ class Linear:
             return done
         f32 = x.dtype == torch.float32 and self.weight.dtype == torch.float32
         if f32 and out is None:
-            # the true 32-bit path: no less precise than float32 fused multiply-adds, k split by the weight's shape alone
+            # the true 32-bit path, k split by the weight's shape alone
             ks = ops.gemm_f32_ksplit(self.out_features, self.in_features, ctx.runtime.compute_units)
             lda, ldw = x.stride(0), self.weight.stride(0)
             if x.data_ptr() % 16 == 0 and self.weight.data_ptr() % 16 == 0 and \

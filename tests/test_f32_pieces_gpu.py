@@ -29,8 +29,8 @@ def test_no_further_from_64_bits_than_a_chain_of_fused_multiply_adds(m, n, k, ks
     ops.gemm_generic(a, w, None, chain, m)
     want = a.double() @ w.double().T
     err, err_chain = ((x.double() - want).square().mean().sqrt() for x in (out.sum(0), chain))
-    # what is left out of a product is below 2^-26 of it, the chain's own roundings are 2^-25 of the sum each; a few dozen
-    # elements (one row) scatter by some ten per cent, and a sum of 48 has few roundings of either kind
+    # what is left out of a product is at most 2^-24 of it and in root mean square below 2^-26, the chain's own roundings are 2^-25 of
+    # the sum each; a few dozen elements (one row) scatter by some ten per cent, and a sum of 48 has few roundings of either kind
     assert float(err) <= 1.1 * float(err_chain) + 2.0 ** -26 * float(want.square().mean().sqrt())
 
 
@@ -136,3 +136,35 @@ def test_numbers_beyond_the_pieces_have_the_bits_of_parts_added_in_order(m, n, k
     few = torch.empty(ks, len(rows), n, device=DEV)
     ops.gemm_f32(a[rows].contiguous(), w, None, few, len(rows), ks)
     assert torch.equal(few.nan_to_num(), parts[:, rows].nan_to_num())
+
+
+@pytest.mark.parametrize("kind", ["random", "positive", "repeated", "one pair"])
+@pytest.mark.parametrize("k,ks", [(1, 1), (2, 1), (3, 1), (4, 1), (7, 1), (8, 1), (16, 1), (20, 1), (128, 1), (1536, 1), (8960, 14), (4224, 2), (9216, 2)])
+def test_sums_of_any_length_and_of_one_sign(kind, k, ks):
+    """From one product to parts of 4,608 (the 32B shape's way down), whose chains are the longest: no further from 64 bits than a chain
+    of fused multiply-adds. ``repeated``: an element's products are all the same, so that its roundings all go one way."""
+    from pyre_amd.hip import ops
+
+    g = torch.Generator().manual_seed(k)
+    for m in (4, 40, 300):
+        n = 256
+        if kind == "random":
+            a, w = torch.randn(m, k, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+        elif kind == "positive":
+            a, w = torch.rand(m, k, generator=g).to(DEV) + 0.01, torch.rand(n, k, generator=g).to(DEV) + 0.01
+        elif kind == "repeated":
+            a, w = ((1 + torch.rand(x, 1, generator=g)).to(DEV).expand(x, k).contiguous() for x in (m, n))
+        else:  # the numbers whose left-out products are largest: 2^-24.0 of each
+            a, w = (torch.full((x, k), 1.0038986206054688, device=DEV) for x in (m, n))
+        out, chain = torch.empty(ks, m, n, device=DEV), torch.empty(m, n, device=DEV)
+        ops.gemm_f32(a, w, None, out if ks > 1 else out[0], m, ks)
+        part = ops.f32_part(k, ks)
+        for p in range(ks):
+            x, y = a[:, p * part:(p + 1) * part].contiguous(), w[:, p * part:(p + 1) * part].contiguous()
+            ops.gemm_generic(x, y, None, chain, m)
+            want = x.double() @ y.double().T
+            err, err_chain, rms = (float(v.square().mean().sqrt()) for v in (out[p].double() - want, chain.double() - want, want))
+            # one pair has one error of either kind, its sums' roundings being all alike: those of 16 k are six, each of 2^-24
+            bound = 1.1 * err_chain if kind != "one pair" else 2.0 ** -24 * (1 + 6 * -(-part // 16) / 2) * rms
+            assert err <= bound, (m, p)
+            assert k >= 8 or torch.equal(out[p], chain)  # the float32 instruction: the same fused multiply-adds

@@ -118,7 +118,7 @@ def test_parts_added_where_they_are_made(n, k, ks):
 
 
 @pytest.mark.parametrize("n,k,ks,off", [(48, 20, 1, 0), (130, 1524, 2, 0), (200, 8, 1, 0), (130, 1529, 2, 1), (77, 23, 1, 3), (70, 9, 1, 1),
-                                        (1536, 1110, 3, 2), (200, 1104, 3, 1), (130, 272, 1, 0), (65, 5, 1, 0), (33, 7, 1, 1), (40, 1, 1, 0),
+                                        (1536, 1110, 3, 2), (200, 1104, 3, 1), (130, 272, 1, 0), (65, 9, 1, 0), (33, 15, 1, 1),
                                         (4608, 60, 1, 1), (9000, 45, 1, 0)])
 def test_k_that_ends_within_a_step_and_rows_that_start_anywhere(n, k, ks, off):
     """The bits of the same product with zeros behind k, up to whole steps, and with rows on 16 bytes. What lies behind the rows and
