@@ -136,12 +136,18 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
              : STREAM    ? sum_partials4_stream(delta + row + i, partial_stride, n_partials)
                          : sum_partials4(delta + row + i, partial_stride, n_partials);
     }
-    // the residual is asked for with the term, not behind the term's own norm: one trip through memory less in a row
-    float4 r[ITEMS];
+    // the residual is asked for with the term, not behind the term's own norm: one trip through memory less in a row (wider rows,
+    // which have no registers for it without a wave less on a SIMD, ask behind the norm: us, 1,777 and 4,000 rows of 5,120, 16-bit
+    // terms: together 47 and 93, one after the other 40 and 80)
+    constexpr bool kTogether = ITEMS <= 4;
+    auto residual = [&](int i) { return STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i); };
+    float4 r[kTogether ? ITEMS : 1];
+    if constexpr (kTogether) {
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const int i = 4 * (tid + k * THREADS);
-      r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
+      for (int k = 0; k < ITEMS; ++k) {
+        const int i = 4 * (tid + k * THREADS);
+        r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : residual(i);
+      }
     }
     if (post_gain) {
       float mean, inv;
@@ -165,7 +171,7 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
       if (i < hidden) {
-        v[k] = add4(v[k], r[k]);
+        v[k] = add4(v[k], kTogether ? r[kTogether ? k : 0] : residual(i));
         if (!rows) {
           if (STREAM) Stream4<float>::store(resid + row + i, v[k]);
           else Vec4<float>::store(resid + row + i, v[k]);

@@ -99,7 +99,9 @@ __global__ __launch_bounds__(kThreads) void add_rms_terms_kernel(
 
 // The same with four elements to a load: the row's width and the partial sums' strides are multiples of four, all
 // gains share one element type, every pointer lies on 16 bytes. THREADS x ITEMS float4 hold a row. The
-// residual is asked for with the terms, not behind their norms. STREAM: terms and residual past the caches.
+// residual is asked for with the terms, not behind their norms, but for wide rows of 16-bit terms, which have no registers for it without
+// a wave less on a SIMD (us, 1,777 and 4,000 rows of 5,120: together 135 and 304, one after the other 92 and 190; of float32 terms 76
+// and 160, 83 and 175). STREAM: terms and residual past the caches.
 template <typename TA, typename TG, typename TO, int THREADS, int ITEMS, bool STREAM = false>
 __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
     float* __restrict__ resid, Term a, Term b, float inner_eps, const TG* __restrict__ outer_gain, float outer_eps,
@@ -112,11 +114,15 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) y[k] = float4{0.f, 0.f, 0.f, 0.f};
 
-  float4 r[ITEMS];
+  constexpr bool kTogether = ITEMS <= 4 || sizeof(TA) == 4;  // float32 terms: 192 or 255 registers, two waves a SIMD either way
+  auto residual = [&](int i) { return STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i); };
+  float4 r[kTogether ? ITEMS : 1];
+  if constexpr (kTogether) {
 #pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const int i = 4 * (tid + k * THREADS);
-    r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
+    for (int k = 0; k < ITEMS; ++k) {
+      const int i = 4 * (tid + k * THREADS);
+      r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : residual(i);
+    }
   }
   auto inv_rms = [&](const float4 (&v)[ITEMS], float e) {
     float ss = 0.f;
@@ -161,7 +167,7 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
   for (int k = 0; k < ITEMS; ++k) {
     const int i = 4 * (tid + k * THREADS);
     if (i < hidden) {
-      y[k] = add4(y[k], r[k]);
+      y[k] = add4(y[k], kTogether ? r[kTogether ? k : 0] : residual(i));
       if (!rows && a.data) {
         if (STREAM) Stream4<float>::store(resid + row + i, y[k]);
         else Vec4<float>::store(resid + row + i, y[k]);

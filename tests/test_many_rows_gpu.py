@@ -89,3 +89,30 @@ def test_poly_norm(width, n, parts_of_k):
         return (out,)
 
     in_steps(run, n, 150)
+
+
+@pytest.mark.parametrize("hidden,n,dtype", [(4100, 200, torch.bfloat16), (5120, 400, torch.float32), (8192, 600, torch.bfloat16), (16384, 130, torch.float32)])
+def test_wide_rows(hidden, n, dtype):
+    """More than 4,096 columns, whose residual is read behind the term's norm, against float64."""
+    from pyre_amd.hip import ops
+
+    resid, data, more = rnd(n, hidden, seed=1), rnd(2, n, hidden, seed=2, dtype=dtype), rnd(2, n, hidden, seed=3, dtype=dtype)
+    gain, own = rnd(hidden, seed=4, dtype=torch.bfloat16), rnd(hidden, seed=5, dtype=torch.bfloat16)
+
+    def norm(x, kind):
+        x = x - x.mean(1, keepdim=True) if kind == "layer" else x
+        return x / (x.square().mean(1, keepdim=True) + 1e-6).sqrt()
+
+    r, out = resid.clone(), torch.full((n, hidden), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.add_layernorm(r, ops.Partials(data, post=ops.PostNorm(own, 1e-6)), gain, 1e-6, out)
+    want = resid.double() + norm(data.double().sum(0), "layer") * own.double()
+    checks = [(r, out, want, norm(want, "layer") * gain.double())]
+    r, out, post = resid.clone(), torch.full_like(out, float("nan")), ops.PostNorm(own, 1e-6, kind="rms")
+    ops.add_rms_terms(r, ops.Partials(data, post=post, more=ops.Partials(more, post=post, scale=0.5), outer=post), gain, 1e-6, out)
+    both = norm(data.double().sum(0), "rms") * own.double() + 0.5 * norm(more.double().sum(0), "rms") * own.double()
+    want = resid.double() + norm(both, "rms") * own.double()
+    checks.append((r, out, want, norm(want, "rms") * gain.double()))
+    for r, out, want, normed in checks:
+        # float32 sums of some ten thousand values around one, and the output's 16 bits
+        assert float((r.double() - want).abs().max()) <= 2.0 ** -19 * float(want.abs().max())
+        assert float((out.double() - normed).abs().max()) <= 2.0 ** -8 * float(normed.abs().max())
