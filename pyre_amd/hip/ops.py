@@ -657,7 +657,9 @@ def gemm_f32_whole(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, m: int,
              ksplit: int = 1) -> None:
     """out[0:m] = a[0:m] @ w.T (+ bias) with float32 operands and result, made of bfloat16 pieces that sum
-    to the operands exactly; the order of an element's additions depends on k and ``ksplit`` alone. With ``ksplit`` > 1, ``out`` is [ksplit, m, N]: partial sums over parts of k (the bias in part 0)."""
+    to the operands exactly (fewer than eight k as fused multiply-adds); the order of an element's additions
+    depends on k and ``ksplit`` alone. With ``ksplit`` > 1, ``out`` is [ksplit, m, N]: partial sums over parts
+    of k (the bias in part 0)."""
     _dev(a, w, bias, out)
     n_out, k = w.shape
     if a.dtype != torch.float32 or w.dtype != torch.float32 or out.dtype != torch.float32:
@@ -933,7 +935,6 @@ def attn_prefill_bf16(q, out, k_cache, v_cache, tiles, n_tiles, positions, seq_o
          block_table.stride(0), nq, nkv, hd, page_size, float(scale), int(window), _stream())
 
 
-@lru_cache(maxsize=4096)
 @lru_cache(maxsize=4096)
 def attn_prefill_waves(nq: int, nkv: int) -> int:
     from pyre_amd.hip.lib import lib
