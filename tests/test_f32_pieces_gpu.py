@@ -8,7 +8,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-#: few rows, tiles of both sizes; with k in one part and in several, with rows that start on 16 bytes and that do not
+#: few rows, the smallest tiles (the others below); with k in one part and in several, with rows that start on 16 bytes and that do not
 FORMS = [(m, n, k, ks, off) for m in (1, 32, 33, 300) for n, k, ks in ((33, 48, 1), (1537, 1040, 1), (200, 1536, 3)) for off in (0, 1)]
 
 
@@ -168,3 +168,39 @@ def test_sums_of_any_length_and_of_one_sign(kind, k, ks):
             bound = 1.1 * err_chain if kind != "one pair" else 2.0 ** -24 * (1 + 6 * -(-part // 16) / 2) * rms
             assert err <= bound, (m, p)
             assert k >= 8 or torch.equal(out[p], chain)  # the float32 instruction: the same fused multiply-adds
+
+
+@pytest.mark.parametrize("m,n,tile", [(100, 1500, (64, 64)), (290, 6000, (64, 128)), (290, 8960, (128, 128))])
+@pytest.mark.parametrize("k,off", [(160, 0), (157, 0), (157, 3)])
+def test_every_size_of_tiles(m, n, tile, k, off):
+    """The distance from 64 bits, and numbers that are not finite or beyond the pieces in the second of a wave's row tiles and column
+    tiles, alone and with a whole row, which leave all other elements as they are."""
+    from pyre_amd.hip import ops
+    from pyre_amd.hip.lib import lib
+
+    assert lib().pyre_gemm_f32_tile_choice(m, n, k, 1) == 1000 * tile[0] + tile[1]
+    a, w = operands(m, n, k, off)
+    if off:
+        w = torch.nn.functional.pad(w, (off, 0))[:, off:]
+    out, chain = torch.full((m, n), float("nan"), device=DEV), torch.empty(m, n, device=DEV)
+    ops.gemm_f32(a, w, None, out, m)
+    ops.gemm_generic(a, w, None, chain, m)
+    exact = a.double() @ w.double().T
+    assert float((out.double() - exact).square().mean()) <= 1.1 ** 2 * float((chain.double() - exact).square().mean())
+    b, v = a.clone() if off == 0 else torch.nn.functional.pad(a, (off, 0))[:, off:], w.clone()
+    rows, cols = (33, 97, m - 1), (32, 40, 95, 127, 161, n - 1)
+    b[33, 7], b[97, k - 1], b[m - 1, 0] = float("inf"), 2e38, float("nan")
+    for i, col in enumerate(cols):
+        v[col, (3 * i) % k] = (float("-inf"), 1e35, float("nan"))[i % 3]
+    if off:
+        v = torch.nn.functional.pad(v, (off, 0))[:, off:]
+    got = torch.full((m, n), float("nan"), device=DEV)
+    ops.gemm_f32(b, v, None, got, m)
+    want = b.double() @ v.double().T
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.abs() > torch.finfo(torch.float32).max)
+    fine = want.isfinite() & (want.abs() < 1e38)
+    scale = b.double().abs() @ v.double().abs().T
+    assert bool(((got.double() - want)[fine].abs() <= 2.0 ** -21 * scale[fine]).all())
+    same = torch.ones(m, n, dtype=torch.bool, device=DEV)
+    same[list(rows)], same[:, list(cols)] = False, False
+    assert torch.equal(got[same], out[same])

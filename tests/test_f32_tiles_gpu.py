@@ -1,4 +1,4 @@
-"""The 32-bit path's products of more than 16 rows in tiles and its prompts' attention with pieces of 16 bytes: at the edges
+"""The 32-bit path's products of more than 32 rows in tiles and its prompts' attention with pieces of 16 bytes: at the edges
 of their tiles, slots and pages."""
 
 from __future__ import annotations
