@@ -140,14 +140,12 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
     // which have no registers for it without a wave less on a SIMD, ask behind the norm: us, 1,777 and 4,000 rows of 5,120, 16-bit
     // terms: together 47 and 93, one after the other 40 and 80)
     constexpr bool kTogether = ITEMS <= 4;
-    auto residual = [&](int i) { return STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i); };
-    float4 r[kTogether ? ITEMS : 1];
-    if constexpr (kTogether) {
+    float4 r[ITEMS];
 #pragma unroll
-      for (int k = 0; k < ITEMS; ++k) {
-        const int i = 4 * (tid + k * THREADS);
-        r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : residual(i);
-      }
+    for (int k = 0; k < ITEMS; ++k) {
+      const int i = 4 * (tid + k * THREADS);
+      if constexpr (kTogether)
+        r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
     }
     if (post_gain) {
       float mean, inv;
@@ -171,7 +169,8 @@ __global__ __launch_bounds__(THREADS) void add_layernorm_vec_kernel(
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
       if (i < hidden) {
-        v[k] = add4(v[k], kTogether ? r[kTogether ? k : 0] : residual(i));
+        if constexpr (!kTogether) r[k] = Vec4<float>::load(resid + row + i);
+        v[k] = add4(v[k], r[k]);
         if (!rows) {
           if (STREAM) Stream4<float>::store(resid + row + i, v[k]);
           else Vec4<float>::store(resid + row + i, v[k]);

@@ -115,14 +115,12 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
   for (int k = 0; k < ITEMS; ++k) y[k] = float4{0.f, 0.f, 0.f, 0.f};
 
   constexpr bool kTogether = ITEMS <= 4 || sizeof(TA) == 4;  // float32 terms: 192 or 255 registers, two waves a SIMD either way
-  auto residual = [&](int i) { return STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i); };
-  float4 r[kTogether ? ITEMS : 1];
-  if constexpr (kTogether) {
+  float4 r[ITEMS];
 #pragma unroll
-    for (int k = 0; k < ITEMS; ++k) {
-      const int i = 4 * (tid + k * THREADS);
-      r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : residual(i);
-    }
+  for (int k = 0; k < ITEMS; ++k) {
+    const int i = 4 * (tid + k * THREADS);
+    if constexpr (kTogether)
+      r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
   }
   auto inv_rms = [&](const float4 (&v)[ITEMS], float e) {
     float ss = 0.f;
@@ -167,7 +165,8 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
   for (int k = 0; k < ITEMS; ++k) {
     const int i = 4 * (tid + k * THREADS);
     if (i < hidden) {
-      y[k] = add4(y[k], kTogether ? r[kTogether ? k : 0] : residual(i));
+      if constexpr (!kTogether) r[k] = Vec4<float>::load(resid + row + i);
+      y[k] = add4(y[k], r[k]);
       if (!rows && a.data) {
         if (STREAM) Stream4<float>::store(resid + row + i, y[k]);
         else Vec4<float>::store(resid + row + i, y[k]);
