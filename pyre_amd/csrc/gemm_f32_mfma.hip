@@ -230,10 +230,10 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __rest
 // moved to its place, zeros behind it, before it is split.
 //
 // What bounds it: a step of 128 x 128 is 768 cycles of the matrix cores a SIMD, 580 cycles of LDS (24 KB written, 48 KB read) and
-// 350 of splitting; two blocks share a compute unit and fill each other's waits. At 2,000 rows of the 7B shape the gate/up product
-// runs at 197 TFLOP/s, 1.18 PFLOP/s of the 16-bit instruction, what that reaches at the clocks the card's power leaves. Against the float32
-// instruction (135 of its 157 TFLOP/s; us): gate/up 4,007 -> 2,748 there, 1,254 -> 885 at 566 rows, 316 -> 270 at 99; the 1.5B shape's
-// 844 -> 581, 245 -> 197 and 80 -> 68, its way down 446 -> 314, 127 -> 108 and 37 -> 33.
+// 410 of splitting; two blocks share a compute unit and fill each other's waits. At 2,000 rows of the 7B shape the gate/up product
+// runs at 190 TFLOP/s, 1.14 PFLOP/s of the 16-bit instruction, what that reaches at the clocks the card's power leaves. Against the float32
+// instruction (135 of its 157 TFLOP/s; us): gate/up 4,035 -> 2,860 there, 1,240 -> 905 at 566 rows, 318 -> 273 at 99; the 1.5B shape's
+// 842 -> 600, 243 -> 207 and 80 -> 75, its way down 447 -> 320, 130 -> 110 and 38 -> 35.
 // Rows that start on any float cost two per cent, k that ends within a step five to ten. Against the float32 instruction in tiles that
 // went through registers, the 7B shape's gate/up with rows a float off: 713 -> 153 at one row, 1,132 -> 156 at 33, 2,357 -> 567 at 300; with
 // four k more: 271 -> 197 at 33 (there against a stream of 64 rows), 523 -> 271 at 99, 1,050 -> 592 at 300.
@@ -425,10 +425,11 @@ __device__ __attribute__((aligned(16))) const unsigned kZeroPiece[4] = {0u, 0u, 
 //
 // What bounds it: a compute unit has about 32 KB of loads under way (27 GB/s from memory, 84 from L2), so that a stream
 // reaches the memory's rate only if all units pull, and equally much; C is chosen for that. Against the float32 instruction with
-// a wave a block up to 16 rows and four above (us, alone in a graph): the 1.5B shape's gate/up 37 -> 29 at 20 rows, its way down 18.6 -> 14.2,
-// q/k/v 8.5 -> 6.7, the 7B shape's gate/up 134 -> 97 and 106 -> 96 at 8 rows. Steps of few rows, whose kernels are start and end: 1,300 -> 1,275 us at one
-// request of the 1.5B shape (14 layers), 1,333 -> 1,336 at 8, 2,076 -> 1,901 at 4 of the 7B shape (8 layers); with the weights kept in
-// the caches on their way 1,358, 1,388 and 2,040.
+// a wave a block up to 16 rows and four above (us, alone in a graph): the 1.5B shape's gate/up 38 -> 30 at 20 rows, its way down 18.4 -> 14.7,
+// q/k/v 8.2 -> 6.7, the 7B shape's gate/up 138 -> 97 and 109 -> 95 at 8 rows; at 1 to 16 rows the 1.5B shape's products, which are start
+// and end, take 5 to 10 % more (gate/up 27 -> 29, way down 13.1 -> 13.9). Whole steps: 1,299 -> 1,307 us at one request of the 1.5B shape
+// (14 layers), 1,334 -> 1,347 at 8, 2,132 -> 1,919 at one of the 7B shape (8 layers), 2,153 -> 1,976 at 8; with the weights kept in the
+// caches on their way 6 % more.
 // (Weights straight into the registers that they are multiplied from, a lane's eight k at a time, take twice as long: a line is
 // asked for eight times there, and the lines that a block's waves have under way do not fit the vector cache.)
 constexpr int kRowWaves = 4;
@@ -631,7 +632,7 @@ int stream_columns(int N, int parts) {
 // The tile with the least work on the busiest unit (a block of two or three shares its matrix cores' time, so that is its
 // tiles), smaller ones costing more for the same: their operands come from LDS more often. The three sizes in turn (us): the 1.5B
 // shape's gate/up 68, 74, 66 at 99 rows, 187, 158, 176 at 400, 197, 207, 230 at 566; the 7B shape's way down 111, 116, 135, then 344,
-// 375, 414 and 440, 484, 545.
+// 375, 414 and 440, 484, 545 (without the operands' scale, which adds three per cent to all).
 struct TileRows {
   int bm, bn;
   double cost;
