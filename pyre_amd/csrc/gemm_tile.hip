@@ -14,7 +14,8 @@
 // (eight tiles along m by four along n): its L2 then serves every row several times.
 //
 // kF32Out: float32 [ksplit][M][N], part `ks` of k; kGated: W = gate rows, then up rows; bfloat16 [M][N / 2], the gated
-// unit of the two. Results pass through four kilobytes of LDS of the wave's own, so that a store writes whole lines: a
+// unit of the two; kPaged: X's rows lie in the pages of a cache, 32 consecutive positions of a request at a time; bfloat16 [N / ldo][M][ldo].
+// Results pass through four kilobytes of LDS of the wave's own, so that a store writes whole lines: a
 // lane's own four elements are 8 or 16 bytes of a row, and 32 rows of such pieces to a store make the L2's rate of
 // requests the limit.
 #include "pyre_api.h"
@@ -49,13 +50,16 @@ __device__ inline void barrier() {
   asm volatile("s_barrier" : : : "memory");
 }
 
-enum Out { kF32Out = 0, kGated = 1 };
+enum Out { kF32Out = 0, kGated = 1, kPaged = 2 };
 
 struct TileShape {
   int M, N, K, kper;  // kper: k of a part, a multiple of 64
   int mt, nt, parts;  // tiles along m and n, parts of k
   int ldo, up;        // length of a row of the results, rows of W from a feature's gate to its up row
   size_t plane;       // results of a part of k
+  const int* groups;  // kPaged: of every 32 rows the request's row of the block table, its first and its last position
+  const int* table;
+  int table_stride, page_size;
 };
 
 template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC>
@@ -65,7 +69,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
   constexpr int NW = WM * WN, STAGE = (BM + BN) * ROW;
   constexpr int LX = BM / 8 / NW, LW = BN / 8 / NW, L = LX + LW;      // loads (of eight rows) of a wave and stage
   constexpr int CT = BM / WM / 32, RT = BN / WN / 32;                 // tiles of 32 rows of X and of W of a wave
-  constexpr int STORES = CT * (OUT == kGated ? (RT + 3) / 4 : RT) * 4;  // stores of a wave for a whole tile
+  constexpr int STORES = CT * (OUT == kGated ? (RT + 3) / 4 : OUT == kPaged ? (RT + 1) / 2 : RT) * 4;  // stores of a wave for a whole tile
   constexpr int MF = RT * CT, RD = RT + CT;
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && (OUT != kGated || RT % 2 == 0), "rows divide over the waves");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[S * STAGE + NW * 4096];
@@ -100,7 +104,13 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
 #pragma unroll
     for (int i = 0; i < LX; ++i) {
       const int row = 8 * (NW * i + wave) + lrow;
-      offx[i] = static_cast<unsigned>(min(im * BM + row, sh.M - 1)) * static_cast<unsigned>(2 * ldx) + 16 * (lpiece ^ ((row >> 1) & 7));
+      int at = min(im * BM + row, sh.M - 1);
+      if (OUT == kPaged) {  // (positions behind the request's last one are the last one once more)
+        const int* const group = sh.groups + 3 * (at / 32);
+        const int pos = min(group[1] + at % 32, group[2]);
+        at = max(sh.table[static_cast<size_t>(group[0]) * sh.table_stride + pos / sh.page_size], 0) * sh.page_size + pos % sh.page_size;
+      }
+      offx[i] = static_cast<unsigned>(at) * static_cast<unsigned>(2 * ldx) + 16 * (lpiece ^ ((row >> 1) & 7));
     }
 #pragma unroll
     for (int i = 0; i < LW; ++i) {
@@ -215,7 +225,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
 #pragma unroll
     for (int q = 0; q < CT; ++q)
 #pragma unroll
-      for (int r = 0; r < RT; r += OUT == kGated ? 2 : 1) {
+      for (int r = 0; r < RT; r += OUT == kF32Out ? 1 : 2) {
         if (OUT == kGated && r % 4 == 2) continue;  // written with the pair before it
         asm volatile("" : : : "memory");
         if (OUT == kGated) {
@@ -240,6 +250,16 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
           };
           if (is_silu(act)) finish(std::true_type{});
           else finish(std::false_type{});
+        } else if (OUT == kPaged) {
+#pragma unroll
+          for (int pair = 0; pair < 2; ++pair) {
+            if (r + pair >= RT) continue;
+            const f32x16& t = acc[r + pair < RT ? r + pair : 0][q];
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+              *reinterpret_cast<uint2*>(own + c * 128 + 16 * ((4 * pair + p) ^ (c & 7)) + 8 * half) =
+                  uint2{pack_bf16x2(t[4 * p], t[4 * p + 1]), pack_bf16x2(t[4 * p + 2], t[4 * p + 3])};
+          }
         } else {
 #pragma unroll
           for (int p = 0; p < 4; ++p)
@@ -256,6 +276,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
             if (!stored && (m >= sh.M || f >= inter)) continue;
             if (RT - r < 4 && lpiece >= 4) continue;  // a lone pair of tiles: half a row
             *reinterpret_cast<uint4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * sh.ldo + f) = y;
+          } else if (OUT == kPaged) {
+            const int n = n0 + 32 * (wn * RT + r) + 8 * lpiece;
+            if (!stored && (m >= sh.M || n >= sh.N)) continue;
+            if (RT - r < 2 && lpiece >= 4) continue;  // a lone tile: half a row
+            *reinterpret_cast<uint4*>(static_cast<bf16*>(out) + n / sh.ldo * sh.plane + static_cast<size_t>(m) * sh.ldo + n % sh.ldo) = y;
           } else {
             const int n = n0 + 32 * (wn * RT + r) + 4 * lpiece;
             if (!stored && (m >= sh.M || n >= sh.N)) continue;
@@ -293,6 +318,8 @@ constexpr TileCost kUnits[] = {{256, 256, 3.1, 0.0, 1.471, 0.291, 0.000},
                                {128, 256, 3.9, 0.0, 0.903, 0.430, 0.018},
                                {96, 256, 4.7, 1.1, 0.654, 0.660, 0.050},
                                {96, 192, 4.1, 0.9, 0.586, 0.768, 0.041}};
+// Paged rows: the sums' times (their results are half as many bytes); the product is short in k, what counts are its rounds.
+constexpr TileCost kPages[] = {kSums[0], kSums[2], kSums[3]};
 constexpr int kMaxParts = 6;
 constexpr double kReadMb = 0.2;              // the consumer's reading of a further part, a megabyte
 // A product cut in two (see TileChoice) pays for a second launch, and full rounds run at lower clocks than a nearly empty one:
@@ -311,16 +338,18 @@ struct TileChoice {
   int cut, by_rows, rest;
 };
 
-double tile_us(const TileCost& c, bool gated, int M, int N, int K, int kper, int parts) {
+// `bytes`: of a result of a part.
+double tile_us(const TileCost& c, int bytes, int M, int N, int K, int kper, int parts) {
   const double units = compute_units(), rows_mb = static_cast<double>(M) * N * 1e-6;
   const double tiles = static_cast<double>((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * parts;
   const double rounds = static_cast<double>(static_cast<long>((tiles + units - 1) / units));
-  const double out_mb = rows_mb * (gated ? 1.0 : 4.0 * parts);
+  const double out_mb = rows_mb * bytes * parts;
   return c.launch + rounds * (c.round + kper / BK * c.stage) + out_mb * c.out_mb + 2e-6 * N * static_cast<double>(K) * c.weight_mb +
          (parts - 1) * 4.0 * rows_mb * kReadMb;
 }
 
 TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, int K, int only_parts) {
+  const int bytes = gated ? 1 : 4;  // (a unit of two bytes is of two rows of W)
   TileChoice best{0, 1, K, 1e30, 0, 0, 0};
   const int units = compute_units();
   for (int parts = 1; parts <= (gated ? 1 : kMaxParts); ++parts) {
@@ -331,7 +360,7 @@ TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, 
     if (parts > 1 && 4.0 * M * N * parts > kMostPartsBytes) continue;
     for (int i = 0; i < n_costs; ++i) {
       const TileCost& c = costs[i];
-      const double us = tile_us(c, gated, M, N, K, kper, parts);
+      const double us = tile_us(c, bytes, M, N, K, kper, parts);
       if (us < best.us) best = TileChoice{i, parts, kper, us, 0, 0, 0};
       const long mt = (M + c.bm - 1) / c.bm, nt = (N + c.bn - 1) / c.bn, rounds = (mt * nt * parts + units - 1) / units;
       for (long full = rounds - 1; full >= 1 && full >= rounds - 2; --full) {
@@ -340,10 +369,10 @@ TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, 
           if (cut < 1 || cut >= (by_rows ? mt : nt)) continue;
           const int m1 = by_rows ? static_cast<int>(cut) * c.bm : M, n1 = by_rows ? N : static_cast<int>(cut) * c.bn;
           const int m2 = by_rows ? M - m1 : M, n2 = by_rows ? N : N - n1;
-          const double first = kCutCost * (tile_us(c, gated, m1, n1, K, kper, parts) + kSecondLaunchUs);
+          const double first = kCutCost * (tile_us(c, bytes, m1, n1, K, kper, parts) + kSecondLaunchUs);
           if (first >= best.us) continue;
           for (int j = 0; j < n_costs; ++j) {
-            const double both = first + kCutCost * tile_us(costs[j], gated, m2, n2, K, kper, parts);
+            const double both = first + kCutCost * tile_us(costs[j], bytes, m2, n2, K, kper, parts);
             if (both < best.us) best = TileChoice{i, parts, kper, both, by_rows ? m1 : gated ? n1 / 2 : n1, by_rows, j};
           }
         }
@@ -364,7 +393,7 @@ void launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, const R
   const bool gated = OUT == kGated;
   const int rows = gated ? 2 * r.N : r.N;  // of W
   const TileShape sh{r.M, rows, K, kper, (r.M + BM - 1) / BM, (rows + BN - 1) / BN, parts, r.all_n, r.all_n,
-                     static_cast<size_t>(r.all_m) * r.all_n};
+                     static_cast<size_t>(r.all_m) * r.all_n, nullptr, nullptr, 0, 0};
   const int tiles = sh.mt * sh.nt * parts;
   const size_t at = static_cast<size_t>(r.m0) * r.all_n + r.n0;
   void* to = gated ? static_cast<void*>(static_cast<bf16*>(out) + at) : static_cast<void*>(static_cast<float*>(out) + at);
@@ -450,4 +479,30 @@ extern "C" int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, l
     else launch<96, 192, 1, 3, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
   });
   return check_launch("gemm_tile_glu_bf16");
+}
+
+// X [pages][1][page][row]: rows of n_groups x 32 positions (see TileShape); out: bfloat16 [N / head][32 n_groups][head].
+extern "C" int pyre_gemm_tile_paged_bf16(const void* X, int pages, int page_size, int row, const int* groups, int n_groups,
+                                         const int* block_table, int table_stride, const void* W, void* out, int N, int K, int head,
+                                         hipStream_t stream) {
+  PYRE_REQUIRE(n_groups >= 0 && n_groups < (1 << 24) && pages > 0 && page_size > 0 && table_stride > 0 && head > 0 && head % 8 == 0 && N % head == 0, "gemm_tile_paged_bf16: bad geometry");
+  if (n_groups == 0) return 0;
+  const int M = 32 * n_groups;
+  if (int rc = check_tile("gemm_tile_paged_bf16", X, W, out, M, N, K, row, K)) return rc;
+  PYRE_REQUIRE(groups && block_table && 2L * pages * page_size * row < (1L << 32), "gemm_tile_paged_bf16: a cache of %d x %d rows of %d is not within 4 GiB",
+               pages, page_size, row);
+  int cfg = 0;
+  for (int i = 1; i < 3; ++i)
+    if (tile_us(kPages[i], 2, M, N, K, K, 1) < tile_us(kPages[cfg], 2, M, N, K, K, 1)) cfg = i;
+  const TileCost& c = kPages[cfg];
+  const TileShape sh{M, N, K, K, (M + c.bm - 1) / c.bm, (N + c.bn - 1) / c.bn, 1, head, 0, static_cast<size_t>(M) * head, groups, block_table, table_stride, page_size};
+  const int tiles = sh.mt * sh.nt, blocks = tiles < compute_units() ? tiles : compute_units();
+  const auto go = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, stream, static_cast<const bf16*>(X), static_cast<long>(row),
+                       static_cast<const bf16*>(W), static_cast<long>(K), out, sh, GateShape{});
+  };
+  if (cfg == 0) go(gemm_tile_kernel<256, 256, 4, 2, 2, kPaged, 2>, 512);
+  else if (cfg == 1) go(gemm_tile_kernel<128, 192, 2, 2, 3, kPaged, 1>, 256);
+  else go(gemm_tile_kernel<128, 128, 2, 2, 4, kPaged, 1>, 256);
+  return check_launch("gemm_tile_paged_bf16");
 }

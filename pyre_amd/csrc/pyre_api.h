@@ -113,6 +113,11 @@ int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long ldw, float*
                         hipStream_t stream);
 int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, long ldw, void* out, int M, int two_i, int K, float limit,
                             float slope, float shift, float cubic, hipStream_t stream);
+// The same over rows that lie in the pages of a cache, X [pages][1][page_size][row], of which the first K elements count:
+// groups: of every 32 rows of out a request's row of the block table, the first position and the request's last one (rows behind
+// it repeat it); W [N][K]; out bfloat16 [N / head][32 n_groups][head], `head` a divisor of N and a multiple of 8.
+int pyre_gemm_tile_paged_bf16(const void* X, int pages, int page_size, int row, const int* groups, int n_groups,
+                              const int* block_table, int table_stride, const void* W, void* out, int N, int K, int head, hipStream_t stream);
 
 // tokens: the n tokens of the flat batch to attend for, or null for tokens 0..n-1. max_keys: a
 // bound on the keys that any of them sees (the block table's width in tokens will do); part:
@@ -367,6 +372,15 @@ int pyre_latent_attn_single(const void* q, const void* rows, void* out, int dt, 
                             const int* positions, const int* seq_of_token, const int* block_table, int table_stride,
                             int heads, int rank, int dk, int page_size, float scale, int window, const float* sink,
                             float* part, hipStream_t stream);
+// Prompt portions over keys and values that were made of the rows (pyre_gemm_tile_paged_bf16), bfloat16: q [n][heads][key_dim], the
+// queries' turned parts `rot` elements each, kv [heads][kv_rows][key_dim | value_dim], a key's turned part the last `rot`
+// elements of its row in the cache; out [n][heads][value_dim], times the gate (float32, the same shape, or null). tiles: first token,
+// count (up to 64), the first token's position, its request's row of the block table, the row of kv that position 0 has or would have.
+int pyre_latent_heads_supports(int key_dim, int rot, int value_dim);
+int pyre_latent_heads(const void* q, const void* turned, long turned_token, long turned_head, const void* kv, int kv_rows, const void* rows,
+                      int row, int page_size, void* out, const float* gate, const int* tiles, int n_tiles, const int* block_table,
+                      int table_stride, int heads, int key_dim, int rot, int value_dim, float scale, int window, const float* sink,
+                      hipStream_t stream);
 
 // ---- a mixture of experts with a sigmoid router (moe.hip) ----
 // gates[n, experts + extra] float32: for the `top` experts of largest logit z, s / (sum of the chosen s + 1e-20) with

@@ -11,7 +11,7 @@ from ctypes import c_float, c_int, c_long, c_void_p
 
 from pyre_amd.hip import build as _build
 
-ABI_VERSION = 30
+ABI_VERSION = 31
 
 
 class KernelError(RuntimeError):
@@ -85,6 +85,9 @@ _SIGNATURES = {
     "pyre_latent_attn_tile": [P, P, P, I, P, I, P, P, P, I, I, I, I, I, F, I, P, P],
     "pyre_latent_attn_spans": [I, I],
     "pyre_latent_attn_single": [P, P, P, I, P, I, P, P, P, I, I, I, I, I, F, I, P, P, P],
+    "pyre_gemm_tile_paged_bf16": [P, I, I, I, P, I, P, I, P, P, I, I, I, P],
+    "pyre_latent_heads_supports": [I, I, I],
+    "pyre_latent_heads": [P, P, L, L, P, I, P, I, I, P, P, P, I, P, I, I, I, I, I, F, I, P, P],
     "pyre_route_topk": [P, I, I, L, P, I, P, I, I, I, I, I, P],
     "pyre_expert_act": [P, I, I, L, P, P, I, I, I, I, I, P],
     "pyre_add_rms_terms": [P, P, I, I, L, P, I, F, P, I, I, L, P, I, F, F, P, I, F, P, I, F, P, I, P, I, I, P],

@@ -1352,6 +1352,62 @@ def latent_attn_single(q, rows, out, tokens, n, positions, seq_of_token, block_t
          page_size, float(scale), int(window), _ptr(sink), _ptr(scratch) if spans > 1 else None, _stream())
 
 
+def gemm_tile_paged(rows, groups, n_groups, block_table, w, out) -> None:
+    """out (bfloat16 [heads, 32 n_groups, N / heads], head by head) = c @ w.T for the first ``w.shape[1]`` elements c of cached rows ``[pages, 1, page, row]``.
+    ``groups`` (int32 [n_groups, 3]): of every 32 rows of ``out`` the request's row of the block table, its first position and the
+    request's last one (rows behind that repeat it)."""
+    _dev(rows, groups, block_table, w, out)
+    for t, name in ((rows, "rows"), (w, "w"), (out, "out")):
+        _contig(name, t)
+        if t.dtype != torch.bfloat16:
+            raise KernelError(f"gemm_tile_paged: {name} is bfloat16")
+    _i32("groups", groups, 3 * n_groups), _i32("block_table", block_table)
+    if rows.dim() != 4 or rows.shape[1] != 1 or w.dim() != 2 or w.shape[1] > rows.shape[3]:
+        raise KernelError(f"gemm_tile_paged: rows [pages, 1, page, row] and w [N, <= row], not {tuple(rows.shape)} and {tuple(w.shape)}")
+    if out.dim() != 3 or out.shape[0] * out.shape[2] != w.shape[0] or out.shape[1] != 32 * n_groups:
+        raise KernelError(f"gemm_tile_paged: out is [heads, {32 * n_groups}, {w.shape[0]} / heads], not {tuple(out.shape)}")
+    call("pyre_gemm_tile_paged_bf16", rows.data_ptr(), rows.shape[0], rows.shape[2], rows.shape[3], groups.data_ptr(), n_groups,
+         block_table.data_ptr(), block_table.shape[1], w.data_ptr(), out.data_ptr(), w.shape[0], w.shape[1], out.shape[2], _stream())
+
+
+LATENT_HEADS_TOKENS = 64  #: queries of a tile of :func:`latent_heads`
+
+
+@lru_cache(maxsize=64)
+def latent_heads_supports(key_dim: int, rot: int, value_dim: int) -> bool:
+    from pyre_amd.hip.lib import lib
+
+    return bool(lib().pyre_latent_heads_supports(key_dim, rot, value_dim))
+
+
+def latent_heads(q, turned, kv, rows, out, tiles, n_tiles, block_table, scale, window=0, sink=None, gate=None) -> None:
+    """Prompt portions over keys and values made per head: ``q [N, heads, key_dim]`` and ``turned [N, heads, rot]`` (any strides of
+    tokens and heads) against ``kv [heads, keys, key_dim + value_dim]`` and the turned parts that end the cached rows
+    ``[pages, 1, page, row]``; ``out [N, heads, value_dim]``, times ``gate`` (float32, the same elements). ``tiles`` (int32
+    [n_tiles, 5]): first token, count, the first token's position, its request's row of the block table, the row of ``kv`` that
+    position 0 has or would have (the caller's rows hold every position that the tile's queries see)."""
+    _dev(q, turned, kv, rows, out, tiles, block_table, sink, gate)
+    for t, name in ((q, "q"), (turned, "turned"), (kv, "kv"), (rows, "rows"), (out, "out")):
+        if t.dtype != torch.bfloat16:
+            raise KernelError(f"latent_heads: {name} is bfloat16")
+    for t, name in ((q, "q"), (kv, "kv"), (rows, "rows"), (out, "out")):
+        _contig(name, t)
+    n, heads, key_dim = q.shape
+    rot, value_dim = turned.shape[2], out.shape[2]
+    if tuple(turned.shape[:2]) != (n, heads) or turned.stride(2) != 1 or tuple(out.shape[:2]) != (n, heads):
+        raise KernelError("latent_heads: q, turned and out are of the same tokens and heads")
+    if kv.dim() != 3 or kv.shape[0] != heads or kv.shape[2] != key_dim + value_dim or rows.dim() != 4 or rows.shape[1] != 1:
+        raise KernelError(f"latent_heads: kv {tuple(kv.shape)} or rows {tuple(rows.shape)} do not fit {heads} heads")
+    if gate is not None and (gate.dtype != torch.float32 or not gate.is_contiguous() or gate.numel() < out.numel()):
+        raise KernelError("latent_heads: the gate is float32 of the output's elements")
+    if sink is not None and (sink.dtype != torch.float32 or sink.numel() != heads or not sink.is_contiguous()):
+        raise KernelError("latent_heads: the sink is float32 [heads]")
+    _i32("tiles", tiles, 5 * n_tiles), _i32("block_table", block_table)
+    call("pyre_latent_heads", q.data_ptr(), turned.data_ptr(), turned.stride(0), turned.stride(1), kv.data_ptr(), kv.shape[1], rows.data_ptr(),
+         rows.shape[3], rows.shape[2], out.data_ptr(), _ptr(gate), tiles.data_ptr(), n_tiles, block_table.data_ptr(),
+         block_table.shape[1], heads, key_dim, rot, value_dim, float(scale), int(window), _ptr(sink), _stream())
+
+
 MAX_STREAMS = 8  #: streams of a residual that the kernel takes (streams.hip)
 
 

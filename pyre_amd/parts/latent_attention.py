@@ -2,20 +2,107 @@
 
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from pyre_amd.hip import ops
 from pyre_amd.parts.attention import STEP_ARRAYS
-from pyre_amd.parts.base import LatentAttentionSpec, Mixer, PagedCacheSpec, PagedTensorSpec, TensorSpec, make_part, take
+from pyre_amd.parts.base import (LatentAttentionSpec, Mixer, PagedCacheSpec, PagedTensorSpec, StepArraySpec, TensorSpec,
+                                 make_part, take)
 from pyre_amd.parts.linear import Linear
+
+#: rows of a request that keys and values are made of at a time (the product's groups)
+GROUP = 32
+#: keys of a portion, in multiples of its tokens, up to which keys and values are made of all of them (bounds the step's list of them)
+MOST_KEYS = 64
+#: keys and values that are made at a time: a portion with more of them runs over the rows, a step with more makes them in rounds
+MADE_BYTES = 256 << 20
+
+
+def portion_pairs(start: int, n: int, window: int) -> int:
+    """Pairs of a query and a key that it sees, of n tokens from position ``start`` on."""
+    if not window or start + n <= window:
+        return n * start + n * (n + 1) // 2
+    short = max(0, window - start)  # tokens that see less than a window
+    return short * start + short * (short + 1) // 2 + (n - short) * window
+
+
+def seen_keys(start: int, n: int, window: int) -> int:
+    return min(start + n, n + window - 1) if window else start + n
+
+
+def made_rows(start: int, n: int, window: int) -> int:
+    """Rows that the keys of a portion are made into: all that it sees, in whole groups."""
+    return -(-seen_keys(start, n, window) // GROUP) * GROUP
+
+
+def makes_heads(start: int, n: int, spec: LatentAttentionSpec) -> bool:
+    """Whether a portion's attention runs over keys and values made of the compressed rows that it sees, or over the rows
+    themselves. Multiply-adds of a pair and head (a weight is three pieces): row + 3 rank against key + 3 value elements; of
+    a key, or a token and head: rank x (key + value elements), for every key that is seen or for every token of the
+    portion, at two and a half times the rate. Decided by a portion's own sizes, so that its result does not depend on what runs
+    beside it.
+
+    Over the rows and over made keys and values, us a layer with what goes with each (rows of 512 + 64, heads of 128 + 64 and 128, a
+    window of 1,024): 12 heads, the first 2,048 tokens 183 and 55, the next 952 120 and 48, the first 512 70 and 31, the first 16 31 and
+    24, 64 behind 1,000 113 and 44; 28 heads 335 and 96, 221 and 70, 71 and 30, 30 and 24, 113 and 52; without a window 12 heads,
+    512 tokens behind 4,000 376 and 142, 28 heads, 1,000 behind 8,000 1,357 and 406. The line: 32 tokens behind 1,000 take 111 and
+    44 alone (50 with 28 heads), but where such portions fill the chip the two are alike."""
+    rows = made_rows(start, n, spec.window)
+    if rows > MOST_KEYS * n + GROUP or rows * spec.num_heads * (spec.key_dim + spec.value_dim) * 2 > MADE_BYTES:
+        return False
+    a_pair = 4 * spec.rank - spec.key_dim - 3 * spec.value_dim
+    return 5 * portion_pairs(start, n, spec.window) * a_pair > 2 * (seen_keys(start, n, spec.window) - n) * spec.rank * (spec.key_dim + spec.value_dim)
+
+
+def made_portions(hb, spec: LatentAttentionSpec):
+    """The portions that :func:`makes_heads`: round, request, first token, tokens, position, first key, the row that it is made into."""
+    counts = hb.q_start[1:] - hb.q_start[:-1]
+    most = MADE_BYTES // (spec.num_heads * (spec.key_dim + spec.value_dim) * 2)
+    rows = turn = 0
+    for s in np.nonzero(counts != 1)[0]:
+        t0, n = int(hb.q_start[s]), int(counts[s])
+        start = int(hb.positions[t0])
+        if makes_heads(start, n, spec):
+            more = made_rows(start, n, spec.window)
+            if rows + more > most:
+                rows, turn = 0, turn + 1
+            yield turn, int(s), t0, n, start, max(0, start - spec.window + 1) if spec.window else 0, rows
+            rows += more
+
+
+def plan_groups(hb, spec: LatentAttentionSpec) -> np.ndarray:
+    """[G, 3], see :func:`~pyre_amd.hip.ops.gemm_tile_paged`, round by round."""
+    out = [(s, p, start + n - 1) for _, s, _, n, start, lo, _ in made_portions(hb, spec) for p in range(lo, start + n, GROUP)]
+    return np.asarray(out, dtype=np.int32).reshape(-1, 3)
+
+
+def plan_tiles(hb, spec: LatentAttentionSpec) -> np.ndarray:
+    """[T, 5], see :func:`~pyre_amd.hip.ops.latent_heads`, round by round, those that see the most keys first."""
+    size = ops.LATENT_HEADS_TOKENS
+    out = [(turn, t0 + k, min(size, n - k), start + k, s, row - lo) for turn, s, t0, n, start, lo, row in made_portions(hb, spec)
+           for k in range(0, n, size)]
+    out.sort(key=lambda t: (t[0], -(t[3] + t[2])))
+    return np.asarray([t[1:] for t in out], dtype=np.int32).reshape(-1, 5)
+
+
+def plan_rounds(hb, spec: LatentAttentionSpec) -> np.ndarray:
+    """[R, 2]: groups and tiles of every round."""
+    out: list[list[int]] = []
+    for turn, _, _, n, start, _, _ in made_portions(hb, spec):
+        if turn == len(out):
+            out.append([0, 0])
+        out[turn][0] += made_rows(start, n, spec.window) // GROUP
+        out[turn][1] += -(-n // ops.LATENT_HEADS_TOKENS)
+    return np.asarray(out, dtype=np.int32).reshape(-1, 2)
 
 
 class LatentAttention(Mixer):
     """c = rms_norm(Wdkv h) gain; head i: k = Wuk_i c, v = Wuv_i c, out_i = softmax(q_i k^T scale) v; with a turned part
     r that all heads share, k = [Wuk_i c | r] and q_i = [unturned | turned].
 
-    Only [c | r] is kept, and neither keys nor values are ever made: q_i . (Wuk_i c) = (Wuk_i^T q_i) . c, so a head's
-    query is carried into the compressed row's space (a product per head), the attention kernels run with the kept
+    Only [c | r] is kept. 16-bit prompt portions make every head's keys and values of the rows that they see, in scratch memory
+    (:func:`makes_heads`). Elsewhere neither is ever made: q_i . (Wuk_i c) = (Wuk_i^T q_i) . c, so a head's query is carried into the compressed row's space (a product per head), the attention kernels run with the kept
     rows as the one shared key head and their first part as the value head, and the weighted sum of rows is carried out
     again, Wuv_i (sum_j a_j c_j), the output's gate applied on the way. Queries (or the compressed row that they are
     made of), the kept row and the gate are one input product. A layer without a row of its own (``own_latent`` False)
@@ -44,13 +131,27 @@ class LatentAttention(Mixer):
         self.inp = Linear(spec.hidden_size, self.gate_col + (self.o_dim if spec.gated else 0), "lattn.in")
         self.q_up = Linear(spec.q_rank, self.q_dim, "lattn.q_up") if spec.q_rank else None
         self.out = Linear(self.o_dim, spec.hidden_size, "lattn.out")
-        self.gain = self.q_gain = self.key_up = self.value_up = self.sink = None
+        self.gain = self.q_gain = self.key_up = self.value_up = self.heads_up = self.sink = None
+        self.plan_name = f"latent.{spec.num_heads}.{spec.window}.{spec.rank}.{spec.rot_dim}.{spec.key_dim}.{spec.value_dim}"
 
     def cache_spec(self):
         return PagedCacheSpec((PagedTensorSpec("c", (1, self.row), token_axis=1),), self.spec.window)
 
     def step_arrays(self):
-        return list(STEP_ARRAYS)
+        if self.heads_up is None:
+            return list(STEP_ARRAYS)
+        plan, spec = self.plan_name, self.spec
+
+        def row_tiles(hb):  # the tiles of the other portions
+            tiles = hb.arrays["attention.prefill_tiles"]
+            return tiles[~np.isin(hb.seq_of_token[tiles[:, 0]], hb.arrays[f"{plan}.tiles"][:, 3])]
+
+        return [*STEP_ARRAYS,
+                StepArraySpec(f"{plan}.groups", lambda n_cap, s_cap: 3 * (MOST_KEYS * n_cap // GROUP + 2 * s_cap), lambda hb: plan_groups(hb, spec)),
+                StepArraySpec(f"{plan}.tiles", lambda n_cap, s_cap: 5 * (n_cap // ops.LATENT_HEADS_TOKENS + s_cap),
+                              lambda hb: plan_tiles(hb, spec)),
+                StepArraySpec(f"{plan}.rounds", lambda n_cap, s_cap: 2 * s_cap, lambda hb: plan_rounds(hb, spec)),
+                StepArraySpec(f"{plan}.row_tiles", STEP_ARRAYS[1].capacity, row_tiles)]
 
     def linears(self) -> list:
         return [lin for lin in (self.inp, self.q_up, self.out) if lin is not None]
@@ -91,8 +192,17 @@ class LatentAttention(Mixer):
             self.sink = take(tensors, f"{p}.sink").float().contiguous()
         self.out.set(take(tensors, f"{p}.o"))
         # per head [outputs, inputs] both ways: [rank, key_dim] carries a query in, [value_dim, rank] a sum out
-        self.key_up = take(tensors, f"{p}.uk").view(s.num_heads, s.key_dim, s.rank).transpose(1, 2).contiguous()
-        self.value_up = take(tensors, f"{p}.uv").view(s.num_heads, s.value_dim, s.rank).contiguous()
+        uk, uv = take(tensors, f"{p}.uk"), take(tensors, f"{p}.uv")
+        self.key_up = uk.view(s.num_heads, s.key_dim, s.rank).transpose(1, 2).contiguous()
+        if uk.dtype == torch.bfloat16 and self._can_make_heads():
+            both = [t.view(s.num_heads, -1, s.rank) for t in (uk, uv)]
+            self.heads_up = torch.cat(both, dim=1).view(-1, s.rank)  # a head's key, then its value, of a row
+        self.value_up = uv.view(s.num_heads, s.value_dim, s.rank).contiguous()
+
+    def _can_make_heads(self) -> bool:
+        """Sizes that the kernels over made keys and values take."""
+        s = self.spec
+        return (ops.latent_heads_supports(s.key_dim, s.rot_dim, s.value_dim) and s.rank % 64 == 0 and self.row % 8 == 0)
 
     def forward(self, ctx, h, cache):
         s, n, ws = self.spec, ctx.n_tokens, ctx.workspace
@@ -114,21 +224,45 @@ class LatentAttention(Mixer):
                             queries=(0, heads, s.key_dim, q, wide), **turn)
         else:
             ops.latent_rows(proj, n, s.rank, s.rot_dim, ctx.dtype, queries=(0, heads, s.key_dim, q, wide), **latent)
-        ops.head_matmul(q, self.key_up, wide, n)
-        o_in = ws.get("lattn.o_in", (n, heads, s.rank), ctx.dtype)
-        self._attend(ctx, wide, rows, o_in, cache)
         o = ws.get("lattn.o", (n, heads, s.value_dim), ctx.dtype)
-        ops.head_matmul(o_in, self.value_up, o, n, gate)
+        made = 0
+        if self.heads_up is not None and rows.numel() < 1 << 31:  # (a product's operand lies within 4 GiB)
+            made = len(ctx.host.arrays[f"{self.plan_name}.tiles"])
+        a, b = self._plain_tokens(ctx.host, n) if made else (0, n)
+        if b > a:
+            ops.head_matmul(q[a:b], self.key_up, wide[a:b], b - a)
+            o_in = ws.get("lattn.o_in", (n, heads, s.rank), ctx.dtype)
+            self._attend(ctx, wide, rows, o_in, cache, f"{self.plan_name}.row_tiles" if made else "attention.prefill_tiles")
+            # (whatever lies between a and b besides is written again below)
+            ops.head_matmul(o_in[a:b], self.value_up, o[a:b], b - a, None if gate is None else gate[a:b])
+        if made:
+            self._attend_made(ctx, q, wide[:, :, s.rank:], rows, o, cache, gate)
         return self.out.forward(ctx, o.view(n, self.o_dim), n)
 
-    def _attend(self, ctx, q, rows, out, cache) -> None:
+    def _plain_tokens(self, host, n: int) -> tuple[int, int]:
+        """The range of tokens in which those lie whose attention runs over the rows themselves."""
+        singles, tiles = host.arrays["attention.decode_tokens"], host.arrays[f"{self.plan_name}.row_tiles"]
+        first = [int(x.min()) for x in (singles, tiles[:, 0]) if len(x)]
+        last = [int(x.max()) + 1 for x in (singles, tiles.sum(axis=1) - 1) if len(x)]
+        return (min(first), max(last)) if first else (0, 0)
+
+    def _attend_made(self, ctx, q, turned, rows, out, cache, gate) -> None:
+        s, g0, t0 = self.spec, 0, 0
+        groups, tiles = ctx.arrays[f"{self.plan_name}.groups"], ctx.arrays[f"{self.plan_name}.tiles"]
+        for g, t in ctx.host.arrays[f"{self.plan_name}.rounds"].tolist():
+            kv = ctx.workspace.get("lattn.kv", (s.num_heads, GROUP * g, s.key_dim + s.value_dim), ctx.dtype)
+            ops.gemm_tile_paged(rows, groups[3 * g0:], g, cache.table, self.heads_up, kv)
+            ops.latent_heads(q, turned, kv, rows, out, tiles[5 * t0:], t, cache.table, s.scale, s.window, self.sink, gate)
+            g0, t0 = g0 + g, t0 + t
+
+    def _attend(self, ctx, q, rows, out, cache, tile_list: str) -> None:
         s = self.spec
         step = (ctx.positions, ctx.seq_of_token, cache.table, s.num_heads, s.rank, self.row, cache.page_size, s.scale, s.window,
                 self.sink)
-        tiles = ctx.host.arrays["attention.prefill_tiles"]
+        tiles = ctx.host.arrays[tile_list]
         singles = ctx.host.arrays["attention.decode_tokens"]
         if len(tiles):
-            ops.latent_attn_tile(q, rows, out, ctx.arrays["attention.prefill_tiles"], len(tiles), *step)
+            ops.latent_attn_tile(q, rows, out, ctx.arrays[tile_list], len(tiles), *step)
         if len(singles):
             spans = ops.latent_attn_spans(cache.table.shape[1], cache.page_size, s.window)
             scratch = None
