@@ -25,6 +25,7 @@ from pathlib import Path
 CSRC = Path(__file__).resolve().parent.parent / "csrc"
 ARCH = "gfx950"
 LIB_NAME = "libpyre_hip.so"
+BINDING_NAME = "pyre_binding.so"
 
 # -packed-fp32-ops off: hipcc must not form packed fp32 instructions from float code.
 HIPCC_FLAGS = [
@@ -126,7 +127,8 @@ def _compile_one(hipcc: str, src: Path, obj: Path, digest: str, tree: str) -> tu
 
 
 def build(force: bool = False, quiet: bool = False) -> Path:
-    """Compile stale (or, with ``force``, all) sources and link the library."""
+    """Compile stale (or, with ``force``, all) sources and link the library; the binding as well."""
+    build_binding(force, quiet)
     out = build_dir()
     out.mkdir(parents=True, exist_ok=True)
     lib = out / LIB_NAME
@@ -164,6 +166,51 @@ def build(force: bool = False, quiet: bool = False) -> Path:
     if not quiet:
         _log(f"linked {lib}")
     return lib
+
+
+def _binding_command(out: Path) -> list[str]:
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(_hipcc()).resolve().parent.parent
+    includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
+                *(p for p in (rocm / "include", Path("/opt/rocm/include")) if p.exists()), CSRC]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{i}" for i in includes], str(CSRC / "binding.cpp"),
+            f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-ldl", "-o", str(out)]
+
+
+def _binding_digest() -> str:
+    """What the binding is built from: its source, the declarations, torch and the interpreter."""
+    import torch
+
+    return _digest([CSRC / "binding.cpp", CSRC / "pyre_api.h"], f"{torch.__version__} {sys.version}")
+
+
+def build_binding(force: bool = False, quiet: bool = False) -> Path:
+    """Compile the native half of the Python binding (host code alone)."""
+    out = build_dir()
+    out.mkdir(parents=True, exist_ok=True)
+    lib, digest = out / BINDING_NAME, _binding_digest()
+    if not force and lib.exists() and _stamp(lib) == digest:
+        return lib
+    t0 = time.time()
+    tmp = out / f".{os.getpid()}.{BINDING_NAME}"
+    proc = subprocess.run(_binding_command(tmp), capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise BuildError(f"the compiler failed on binding.cpp:\n{proc.stderr[-4000:]}")
+    os.replace(tmp, lib)
+    _write_stamp(lib, digest)
+    if not quiet:
+        _log(f"built {lib} ({time.time() - t0:.1f} s)")
+    return lib
+
+
+def ensure_binding() -> Path:
+    """Path of the binding; compiles only when it is missing or was built from something else."""
+    return build_binding()
 
 
 def ensure_built() -> Path:

@@ -14,19 +14,14 @@ from functools import lru_cache
 import torch
 
 from pyre_amd.hip.lib import KernelError, call
-
-_DT = {torch.float32: 0, torch.bfloat16: 1}
+from pyre_amd.hip.native import binding
 
 #: compute units that launch plans are made for when nobody names a device (an MI355X)
 DEFAULT_UNITS = 256
 
 
-def dtype_code(t: torch.Tensor | torch.dtype) -> int:
-    dt = t.dtype if isinstance(t, torch.Tensor) else t
-    try:
-        return _DT[dt]
-    except KeyError:
-        raise KernelError(f"unsupported element type {dt}; kernels take float32 and bfloat16") from None
+#: the element type's code of a tensor or a type; what the kernels do not take is refused
+dtype_code = binding.dtype_code
 
 
 _STREAM: int | None = None
@@ -43,27 +38,8 @@ def _stream() -> int:
     return _STREAM if _STREAM is not None else torch.cuda.current_stream().cuda_stream
 
 
-def _dev(*tensors: torch.Tensor | None) -> None:
-    for t in tensors:
-        if t is not None and not t.is_cuda:
-            raise KernelError("kernel operand is not on a GPU (there is no CPU path)")
-
-
-def _contig(name: str, t: torch.Tensor) -> None:
-    if not t.is_contiguous():
-        raise KernelError(f"{name} must be contiguous")
-
-
-def _i32(name: str, t: torch.Tensor, n: int | None = None) -> None:
-    if t.dtype != torch.int32:
-        raise KernelError(f"{name} must be int32, got {t.dtype}")
-    _contig(name, t)
-    if n is not None and t.numel() < n:
-        raise KernelError(f"{name} holds {t.numel()} entries, {n} needed")
-
-
-def _ptr(t: torch.Tensor | None) -> int | None:
-    return None if t is None else t.data_ptr()
+# Checks of operands: every tensor lies on a GPU; a tensor is contiguous; int32, contiguous and of enough entries; its address.
+_dev, _contig, _i32, _ptr = binding.dev, binding.contig, binding.i32, binding.ptr
 
 
 @dataclass
@@ -117,15 +93,7 @@ class Partials:
         return self.data.stride(0)
 
     def _args(self, width: int):
-        data, bias = self.data, self.bias
-        count, _, wide = data.shape
-        if wide != width:
-            raise KernelError(f"partials are {wide} wide, {width} expected")
-        if bias is None:
-            return data.data_ptr(), dtype_code(data), count, data.stride(0), None, 0
-        if bias.numel() != width:
-            raise KernelError(f"bias has {bias.numel()} entries, {width} expected")
-        return data.data_ptr(), dtype_code(data), count, data.stride(0), bias.data_ptr(), dtype_code(bias)
+        return binding.partials(self.data, self.bias, width)
 
 
 def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: float = 1.0,
@@ -141,8 +109,8 @@ def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: floa
         if places.dim() != 2 or places.shape[1] != hidden or places.dtype != table.dtype or places.shape[0] < 1 or positions is None:
             raise KernelError("embed: the table of positions is [rows, H] of the token table's type, with the tokens' positions")
         _contig("places", places), _i32("positions", positions, n)
-    call("pyre_embed", table.data_ptr(), dtype_code(table), ids.data_ptr(), _ptr(positions), _ptr(places),
-         places.shape[0] if places is not None else 0, out.data_ptr(), n, hidden, float(scale), _stream())
+    call("pyre_embed", table, dtype_code(table), ids, positions, places,
+         places.shape[0] if places is not None else 0, out, n, hidden, float(scale), _stream())
 
 
 def add_rmsnorm(resid: torch.Tensor, delta: Partials | None, gain: torch.Tensor, eps: float,
@@ -170,8 +138,8 @@ def add_rmsnorm(resid: torch.Tensor, delta: Partials | None, gain: torch.Tensor,
         d = delta._args(hidden)
     else:
         d = (None, 0, 0, 0, None, 0)
-    call("pyre_add_rmsnorm", resid.data_ptr(), *d, gain.data_ptr(), dtype_code(gain), out.data_ptr(),
-         dtype_code(out), _ptr(rows), n, hidden, float(eps), _stream())
+    call("pyre_add_rmsnorm", resid, *d, gain, dtype_code(gain), out,
+         dtype_code(out), rows, n, hidden, float(eps), _stream())
 
 
 def add_layernorm(resid: torch.Tensor, delta: Partials | None, gain: torch.Tensor, eps: float,
@@ -216,8 +184,8 @@ def add_layernorm(resid: torch.Tensor, delta: Partials | None, gain: torch.Tenso
                     dtype_code(pn.scale) if pn.scale is not None else 0, float(pn.eps))
     else:
         d = (None, 0, 0, 0, None, 0)
-    call("pyre_add_layernorm", resid.data_ptr(), *d, *post, gain.data_ptr(), _ptr(shift), dtype_code(gain), out.data_ptr(),
-         dtype_code(out), _ptr(rows), n, hidden, float(eps), _stream())
+    call("pyre_add_layernorm", resid, *d, *post, gain, shift, dtype_code(gain), out,
+         dtype_code(out), rows, n, hidden, float(eps), _stream())
 
 
 #: slope at which the gated unit's sigmoid is a step: max(g, 0) (u + shift)
@@ -238,7 +206,7 @@ def clipped_glu(gu: Partials, out: torch.Tensor, n: int, limit: float, slope: fl
     if gu.bias is not None:
         raise KernelError("clipped_glu: a pending bias is not supported")
     _contig("out", out)
-    call("pyre_clipped_glu", gu.data.data_ptr(), dtype_code(gu.data), gu.count, gu.stride, out.data_ptr(),
+    call("pyre_clipped_glu", gu.data, dtype_code(gu.data), gu.count, gu.stride, out,
          dtype_code(out), n, inter, float(limit), float(slope), float(shift), float(cubic), _stream())
 
 
@@ -247,7 +215,7 @@ def scale_(x: torch.Tensor, s: float) -> None:
     _dev(x)
     if x.dtype != torch.float32 or not x.is_contiguous():
         raise KernelError("scale_: contiguous float32 expected")
-    call("pyre_scale", x.data_ptr(), x.numel(), float(s), _stream())
+    call("pyre_scale", x, x.numel(), float(s), _stream())
 
 
 def _proj_args(proj: Partials, col0: int, width: int):
@@ -285,8 +253,8 @@ def unit_qkv_write(proj: Partials, col0: int, q_out: torch.Tensor, k_cache: torc
         cache_dt = dtype_code(k_cache)
     if gate_out is not None and (gate_out.dtype != torch.float32 or gate_out.numel() < n * nq or not gate_out.is_contiguous()):
         raise KernelError("unit_qkv_write: gates are contiguous float32 [N, nq]")
-    call("pyre_unit_qkv_write", *args, q_out.data_ptr(), dtype_code(q_out), _ptr(k_cache), _ptr(v_cache), cache_dt,
-         _ptr(gate_out), _ptr(slots), n, nq, nkv, dk, dv, page_size, int(bool(unit_norm)), float(eps),
+    call("pyre_unit_qkv_write", *args, q_out, dtype_code(q_out), k_cache, v_cache, cache_dt,
+         gate_out, slots, n, nq, nkv, dk, dv, page_size, int(bool(unit_norm)), float(eps),
          1 if write else 0, _stream())
 
 
@@ -354,11 +322,11 @@ def attn_biased_tile(q, out, k_cache, v_cache, gate, out_scale, tiles, n_tiles, 
         if scratch.dtype != torch.float32 or not scratch.is_contiguous() or scratch.numel() < rows * nq * splits * (dv + 4) or \
                 splits < 1 or per < 1:
             raise KernelError(f"attn_biased_tile: scratch of {rows * nq * splits * (dv + 4)} float32 elements needed")
-    call("pyre_attn_biased_tile", q.data_ptr(), out.data_ptr(), out.stride(0), dtype_code(q), k_cache.data_ptr(),
-         v_cache.data_ptr(), _ptr(gate), float(out_scale), tiles.data_ptr(), n_tiles, positions.data_ptr(),
-         seq_of_token.data_ptr(), block_table.data_ptr(), block_table.stride(0), nq, nkv, dk, dv, page_size,
-         float(scale), float(cap), _ptr(bias), int(far), int(window), int(keep_first), int(chunk), _ptr(sink),
-         int(gate_dim), _ptr(scratch), int(splits), int(per), _stream())
+    call("pyre_attn_biased_tile", q, out, out.stride(0), dtype_code(q), k_cache,
+         v_cache, gate, float(out_scale), tiles, n_tiles, positions,
+         seq_of_token, block_table, block_table.stride(0), nq, nkv, dk, dv, page_size,
+         float(scale), float(cap), bias, int(far), int(window), int(keep_first), int(chunk), sink,
+         int(gate_dim), scratch, int(splits), int(per), _stream())
 
 
 def attn_biased_spans(table_width: int, page_size: int, window: int, keep_first: int, chunk: int = 0) -> int:
@@ -385,11 +353,11 @@ def attn_biased_single(q, out, k_cache, v_cache, gate, out_scale, tokens, n, pos
         _dev(scratch)
         if scratch.dtype != torch.float32 or not scratch.is_contiguous() or scratch.numel() < n * nq * spans * (dv + 2):
             raise KernelError(f"attn_biased_single: scratch of {n * nq * spans * (dv + 2)} float32 elements needed")
-    call("pyre_attn_biased_single", q.data_ptr(), out.data_ptr(), out.stride(0), dtype_code(q), k_cache.data_ptr(),
-         v_cache.data_ptr(), _ptr(gate), float(out_scale), _ptr(tokens), n, positions.data_ptr(),
-         seq_of_token.data_ptr(), block_table.data_ptr(), block_table.stride(0), nq, nkv, dk, dv, page_size,
-         float(scale), float(cap), _ptr(bias), int(far), int(window), int(keep_first), int(chunk), _ptr(scratch), spans,
-         _ptr(sink), int(gate_dim), _stream())
+    call("pyre_attn_biased_single", q, out, out.stride(0), dtype_code(q), k_cache,
+         v_cache, gate, float(out_scale), tokens, n, positions,
+         seq_of_token, block_table, block_table.stride(0), nq, nkv, dk, dv, page_size,
+         float(scale), float(cap), bias, int(far), int(window), int(keep_first), int(chunk), scratch, spans,
+         sink, int(gate_dim), _stream())
 
 
 GLA_MAX_RANK = 512     #: the widest low-rank input of the decay (linear_attention.hip)
@@ -415,8 +383,8 @@ def gla_prepare(proj: Partials, col0: int, a2: torch.Tensor, a2_bias: torch.Tens
     if x.dtype != torch.float32 or not x.is_contiguous() or x.shape[-1] != gla_row_width(heads, dk, dv) or x.shape[0] < n \
             or proj.rows < n:
         raise KernelError("gla_prepare: x is contiguous float32 [>= n, 3*heads*dk + 2*heads*dv]")
-    call("pyre_gla_prepare", *args, a2.data_ptr(), dtype_code(a2), _ptr(a2_bias),
-         dtype_code(a2_bias) if a2_bias is not None else 0, float(tau), x.data_ptr(), n, heads, dk, dv, rank, _stream())
+    call("pyre_gla_prepare", *args, a2, dtype_code(a2), a2_bias,
+         dtype_code(a2_bias) if a2_bias is not None else 0, float(tau), x, n, heads, dk, dv, rank, _stream())
 
 
 def gla_chunks_scratch(n_tokens: int, n_seqs: int, heads: int, dk: int, dv: int) -> int:
@@ -448,14 +416,14 @@ def gla_scan(x: torch.Tensor, state: torch.Tensor, o: torch.Tensor, q_start: tor
         raise KernelError("gla_scan: shapes do not fit the head geometry")
     _i32("q_start", q_start, n_seqs + 1), _i32("state_slots", state_slots, n_seqs)
     if chunks is None:
-        call("pyre_gla_scan", x.data_ptr(), state.data_ptr(), o.data_ptr(), q_start.data_ptr(), state_slots.data_ptr(),
-             n_seqs, heads, dk, dv, float(qscale), _ptr(decay), _stream())
+        call("pyre_gla_scan", x, state, o, q_start, state_slots,
+             n_seqs, heads, dk, dv, float(qscale), decay, _stream())
         return
     n = o.shape[0]
     if chunks.dtype != torch.float32 or not chunks.is_contiguous() or chunks.numel() < gla_chunks_scratch(n, n_seqs, heads, dk, dv):
         raise KernelError("gla_scan: the chunks' scratch is contiguous float32 of gla_chunks_scratch(...) elements")
-    call("pyre_gla_chunks", x.data_ptr(), chunks.data_ptr(), state.data_ptr(), o.data_ptr(), q_start.data_ptr(),
-         state_slots.data_ptr(), n, n_seqs, int(max_tokens), heads, dk, dv, float(qscale), _stream())
+    call("pyre_gla_chunks", x, chunks, state, o, q_start,
+         state_slots, n, n_seqs, int(max_tokens), heads, dk, dv, float(qscale), _stream())
 
 
 def gla_finish(o: torch.Tensor, x: torch.Tensor, gain: torch.Tensor | None, eps: float, out_scale: float, out: torch.Tensor,
@@ -468,8 +436,8 @@ def gla_finish(o: torch.Tensor, x: torch.Tensor, gain: torch.Tensor | None, eps:
         raise KernelError("gla_finish: gain [dv] and out [>= n, >= heads*dv] expected")
     if gain is not None:
         _contig("gain", gain)
-    call("pyre_gla_finish", o.data_ptr(), x.data_ptr(), _ptr(gain), dtype_code(gain) if gain is not None else 0, float(eps), float(out_scale),
-         out.data_ptr(), dtype_code(out), out.stride(0), n, heads, dk, dv, _stream())
+    call("pyre_gla_finish", o, x, gain, dtype_code(gain) if gain is not None else 0, float(eps), float(out_scale),
+         out, dtype_code(out), out.stride(0), n, heads, dk, dv, _stream())
 
 
 def gla_finish_wide(o: torch.Tensor, x: torch.Tensor, gain: torch.Tensor, eps: float, out_scale: float, out: torch.Tensor,
@@ -483,8 +451,8 @@ def gla_finish_wide(o: torch.Tensor, x: torch.Tensor, gain: torch.Tensor, eps: f
             o.shape[-1] != heads * dv or o.shape[0] < n or x.shape[-1] != gla_row_width(heads, dk, dv) or x.shape[0] < n:
         raise KernelError("gla_finish_wide: gain [heads*dv] and out [>= n, >= heads*dv] expected")
     _contig("gain", gain)
-    call("pyre_gla_finish_wide", o.data_ptr(), x.data_ptr(), gain.data_ptr(), dtype_code(gain), float(eps), float(out_scale),
-         out.data_ptr(), dtype_code(out), out.stride(0), n, heads, dk, dv, _stream())
+    call("pyre_gla_finish_wide", o, x, gain, dtype_code(gain), float(eps), float(out_scale),
+         out, dtype_code(out), out.stride(0), n, heads, dk, dv, _stream())
 
 
 def rope_kv_write(qkv: Partials, q_out: torch.Tensor, k_cache: torch.Tensor | None,
@@ -520,8 +488,8 @@ def rope_kv_write(qkv: Partials, q_out: torch.Tensor, k_cache: torch.Tensor | No
         if cos.dim() != 2 or cos.shape[1] != rotary_dim // 2 or cos.shape != sin.shape:
             raise KernelError("rope_kv_write: cos/sin tables must be [positions, rotary_dim/2]")
         _contig("cos", cos), _contig("sin", sin)
-    call("pyre_rope_kv_write", *q, q_out.data_ptr(), dtype_code(q_out), _ptr(k_cache), _ptr(v_cache),
-         cache_dt, _ptr(cos), _ptr(sin), rotary_dim, positions.data_ptr(), _ptr(slots), n, nq, nkv, hd,
+    call("pyre_rope_kv_write", *q, q_out, dtype_code(q_out), k_cache, v_cache,
+         cache_dt, cos, sin, rotary_dim, positions, slots, n, nq, nkv, hd,
          page_size, 1 if write else 0, _stream())
 
 
@@ -534,7 +502,7 @@ def silu_mul(gu: Partials, out: torch.Tensor, n: int) -> None:
     if gu.bias is not None:
         raise KernelError("silu_mul: a pending bias is not supported")
     _contig("out", out)
-    call("pyre_silu_mul", gu.data.data_ptr(), dtype_code(gu.data), gu.count, gu.stride, out.data_ptr(),
+    call("pyre_silu_mul", gu.data, dtype_code(gu.data), gu.count, gu.stride, out,
          dtype_code(out), n, inter, _stream())
 
 
@@ -543,7 +511,7 @@ def reduce_partials(p: Partials, out: torch.Tensor, n: int) -> None:
     if out.shape[-1] != p.width or out.shape[0] < n or p.rows < n:
         raise KernelError("reduce_partials: shapes do not fit")
     _contig("out", out)
-    call("pyre_reduce_partials", *p._args(p.width), out.data_ptr(), dtype_code(out), n, p.width, _stream())
+    call("pyre_reduce_partials", *p._args(p.width), out, dtype_code(out), n, p.width, _stream())
 
 
 _FILL_PATTERNS = {(4, "zero"): 0, (2, "zero"): 0, (4, "nan"): 0x7FC00000, (2, "nan"): 0x7FC0}
@@ -558,7 +526,7 @@ def fill_rows(tensor: torch.Tensor, ids: list[int], value: float) -> None:
 
     _dev(tensor)
     _contig("tensor", tensor)
-    if tensor.dim() < 2 or tensor.dtype not in _DT:
+    if tensor.dim() < 2 or tensor.dtype not in (torch.float32, torch.bfloat16):
         raise KernelError("fill_rows: a float32 or bfloat16 tensor [outer, rows, ...] expected")
     if not ids:
         return
@@ -569,8 +537,8 @@ def fill_rows(tensor: torch.Tensor, ids: list[int], value: float) -> None:
     row_elems = tensor.stride(1)
     arr = (ctypes.c_int * len(ids))(*[int(i) for i in ids])
     with torch.cuda.device(tensor.device):
-        call("pyre_fill_rows", tensor.data_ptr(), tensor.element_size(), tensor.stride(0), outer, rows, row_elems,
-             ctypes.cast(arr, ctypes.c_void_p), len(ids), _FILL_PATTERNS[(tensor.element_size(), kind)], _stream())
+        call("pyre_fill_rows", tensor, tensor.element_size(), tensor.stride(0), outer, rows, row_elems,
+             ctypes.addressof(arr), len(ids), _FILL_PATTERNS[(tensor.element_size(), kind)], _stream())
 
 
 def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor,
@@ -588,9 +556,9 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, ou
         _i32("a_rows", a_rows, m)
     if bias is not None and bias.numel() != n_out:
         raise KernelError("gemm: bias length")
-    call("pyre_gemm_generic", a.data_ptr(), dtype_code(a), a.stride(0), _ptr(a_rows), w.data_ptr(),
-         dtype_code(w), w.stride(0), _ptr(bias), dtype_code(bias) if bias is not None else 0,
-         out.data_ptr(), dtype_code(out), out.stride(0), m, n_out, k, _stream())
+    call("pyre_gemm_generic", a, dtype_code(a), a.stride(0), a_rows, w,
+         dtype_code(w), w.stride(0), bias, dtype_code(bias) if bias is not None else 0,
+         out, dtype_code(out), out.stride(0), m, n_out, k, _stream())
 
 
 #: the most parts of k of a float32 product, and the fewest k of a part: a wave of a decode step's product is a chain of
@@ -650,7 +618,7 @@ def gemm_f32_whole(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, 
         raise KernelError(f"gemm_f32: a {tuple(a.shape)} @ w {tuple(w.shape)}.T -> out {tuple(out.shape)} do not fit {m} rows")
     if a.stride(1) != 1 or w.stride(1) != 1 or out.stride(1) != 1:
         raise KernelError("gemm_f32: rows must be contiguous")
-    call("pyre_gemm_f32_whole", a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), m, n_out, k,
+    call("pyre_gemm_f32_whole", a, a.stride(0), w, w.stride(0), out, out.stride(0), m, n_out, k,
          ksplit, _stream())
 
 
@@ -672,8 +640,8 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, out: t
         raise KernelError("gemm_f32: fewer rows than m, or partial sums that are not [ksplit, m, N]")
     if bias is not None and bias.numel() != n_out:
         raise KernelError("gemm_f32: bias length")
-    call("pyre_gemm_f32", a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), _ptr(bias),
-         dtype_code(bias) if bias is not None else 0, out.data_ptr(), out.stride(-2),
+    call("pyre_gemm_f32", a, a.stride(0), w, w.stride(0), bias,
+         dtype_code(bias) if bias is not None else 0, out, out.stride(-2),
          out.stride(0) if ksplit > 1 else 0, m, n_out, k, ksplit, _stream())
 
 
@@ -717,10 +685,10 @@ def attn_generic(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, v_ca
             args = (flat_q, flat_out, tokens[at:], positions, seq_of_token)
         else:
             args = (flat_q[at * nq * hd:], flat_out[at * nq * hd:], None, positions[at:], seq_of_token[at:])
-        call("pyre_attn_generic", args[0].data_ptr(), args[1].data_ptr(), dtype_code(q), k_cache.data_ptr(),
-             v_cache.data_ptr(), dtype_code(k_cache), _ptr(args[2]), args[3].data_ptr(), args[4].data_ptr(),
-             block_table.data_ptr(), block_table.stride(0), rows, nq, nkv, hd, page_size, float(scale),
-             int(window), max_keys, _ptr(scratch) if need else None, int(bool(matrix_cores)), _stream())
+        call("pyre_attn_generic", args[0].data_ptr(), args[1].data_ptr(), dtype_code(q), k_cache,
+             v_cache, dtype_code(k_cache), _ptr(args[2]), args[3].data_ptr(), args[4].data_ptr(),
+             block_table, block_table.stride(0), rows, nq, nkv, hd, page_size, float(scale),
+             int(window), max_keys, scratch if need else None, int(bool(matrix_cores)), _stream())
 
 
 ATTN_GENERIC_SCRATCH = 1 << 25   #: float32 elements of scratch that one launch of attn_generic may use
@@ -767,8 +735,8 @@ def attn_prefill_f32(q, out, k_cache, v_cache, tiles, n_tiles, positions, seq_of
     if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.stride(1) != 1:
         raise KernelError("attn_prefill_f32: block table must be int32 [rows, pages]")
     _i32("positions", positions), _i32("seq_of_token", seq_of_token), _i32("tiles", tiles, 2 * n_tiles)
-    call("pyre_attn_prefill_f32", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-         tiles.data_ptr(), n_tiles, positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(),
+    call("pyre_attn_prefill_f32", q, out, k_cache, v_cache,
+         tiles, n_tiles, positions, seq_of_token, block_table,
          block_table.stride(0), nq, nkv, hd, page_size, float(scale), int(window), _stream())
 
 
@@ -787,7 +755,7 @@ def argmax(logits: torch.Tensor, out: torch.Tensor, scratch: torch.Tensor | None
         scratch = torch.empty(m * ARGMAX_SCRATCH_PER_ROW, dtype=torch.int32, device=logits.device)
     if scratch.element_size() != 4 or scratch.numel() < m * ARGMAX_SCRATCH_PER_ROW or not scratch.is_contiguous():
         raise KernelError("argmax: scratch must hold 128 four-byte words per row")
-    call("pyre_argmax", logits.data_ptr(), logits.stride(0), out.data_ptr(), scratch.data_ptr(), m,
+    call("pyre_argmax", logits, logits.stride(0), out, scratch, m,
          logits.shape[1], _stream())
 
 
@@ -815,7 +783,7 @@ def argmax_static(logits: torch.Tensor, out: torch.Tensor) -> None:
     m = logits.shape[0]
     _i32("out", out, m)
     with torch.cuda.device(logits.device):
-        call("pyre_argmax_static", logits.data_ptr(), logits.stride(0), out.data_ptr(), m, logits.shape[1],
+        call("pyre_argmax_static", logits, logits.stride(0), out, m, logits.shape[1],
              _stream())
 
 
@@ -831,15 +799,15 @@ def sample(logits: torch.Tensor, temperature: torch.Tensor, uniform: torch.Tenso
         if t.dtype != torch.float32 or t.numel() < m or not t.is_contiguous():
             raise KernelError(f"sample: {name} must be contiguous float32 [M]")
     _i32("out", out, m)
-    call("pyre_sample", logits.data_ptr(), logits.stride(0), temperature.data_ptr(), uniform.data_ptr(),
-         out.data_ptr(), m, logits.shape[1], _stream())
+    call("pyre_sample", logits, logits.stride(0), temperature, uniform,
+         out, m, logits.shape[1], _stream())
 
 
 def feed_tokens(tokens: torch.Tensor, src: torch.Tensor, ids: torch.Tensor, n: int) -> None:
     """tokens[i] = ids[src[i]] for i < n with src[i] >= 0 (all int32 on the device)."""
     _dev(tokens, src, ids)
     _i32("tokens", tokens, n), _i32("src", src, n), _i32("ids", ids)
-    call("pyre_feed_tokens", tokens.data_ptr(), src.data_ptr(), ids.data_ptr(), n, _stream())
+    call("pyre_feed_tokens", tokens, src, ids, n, _stream())
 
 
 @lru_cache(maxsize=4096)
@@ -877,9 +845,9 @@ def attn_decode_work_bf16(q, out, k_cache, v_cache, work, capacity, positions, s
         raise KernelError("attn_decode_work: partial max/sum buffer too small")
     if counters.dtype != torch.int32 or counters.numel() < capacity * items:
         raise KernelError("attn_decode_work: too few counters")
-    call("pyre_attn_decode_work_bf16", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-         work.data_ptr(), capacity, positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(),
-         block_table.stride(0), part_acc.data_ptr(), part_ml.data_ptr(), counters.data_ptr(), int(bool(alone)), nq,
+    call("pyre_attn_decode_work_bf16", q, out, k_cache, v_cache,
+         work, capacity, positions, seq_of_token, block_table,
+         block_table.stride(0), part_acc, part_ml, counters, int(bool(alone)), nq,
          nkv, hd, page_size, float(scale), int(window), _stream())
 
 
@@ -917,10 +885,10 @@ def attn_decode_work_rope_bf16(qkv: Partials, cos, sin, slots, out, k_cache, v_c
         raise KernelError("attn_decode_work: partial max/sum buffer too small")
     if counters.dtype != torch.int32 or counters.numel() < capacity * items:
         raise KernelError("attn_decode_work: too few counters")
-    call("pyre_attn_decode_work_rope_bf16", args[0], args[2], args[3], args[4], args[5], cos.data_ptr(), sin.data_ptr(),
-         slots.data_ptr(), qkv.rows, int(bool(write_kv)), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-         work.data_ptr(), capacity, positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(),
-         block_table.stride(0), part_acc.data_ptr(), part_ml.data_ptr(), counters.data_ptr(), int(bool(alone)), nq,
+    call("pyre_attn_decode_work_rope_bf16", args[0], args[2], args[3], args[4], args[5], cos, sin,
+         slots, qkv.rows, int(bool(write_kv)), out, k_cache, v_cache,
+         work, capacity, positions, seq_of_token, block_table,
+         block_table.stride(0), part_acc, part_ml, counters, int(bool(alone)), nq,
          nkv, hd, page_size, float(scale), int(window), _stream())
 
 
@@ -930,8 +898,8 @@ def attn_prefill_bf16(q, out, k_cache, v_cache, tiles, n_tiles, positions, seq_o
     [n_tiles, 2] = (first token, count <= 32)."""
     _attn_common(q, out, k_cache, v_cache, positions, seq_of_token, block_table, nq, nkv, hd, page_size)
     _i32("tiles", tiles, 2 * n_tiles)
-    call("pyre_attn_prefill_bf16", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-         tiles.data_ptr(), n_tiles, positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(),
+    call("pyre_attn_prefill_bf16", q, out, k_cache, v_cache,
+         tiles, n_tiles, positions, seq_of_token, block_table,
          block_table.stride(0), nq, nkv, hd, page_size, float(scale), int(window), _stream())
 
 
@@ -956,9 +924,9 @@ def attn_prefill_work_bf16(q, out, k_cache, v_cache, work, n_items, partials, co
             raise KernelError("attn_prefill_work: partial results do not fit")
         if counters.dtype != torch.int32 or counters.numel() < n_slots * per_slot:
             raise KernelError("attn_prefill_work: too few counters")
-    call("pyre_attn_prefill_work_bf16", q.data_ptr(), out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
-         work.data_ptr(), n_items, _ptr(partials) if n_slots else None, _ptr(counters) if n_slots else None,
-         n_slots, positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(), block_table.stride(0),
+    call("pyre_attn_prefill_work_bf16", q, out, k_cache, v_cache,
+         work, n_items, partials if n_slots else None, counters if n_slots else None,
+         n_slots, positions, seq_of_token, block_table, block_table.stride(0),
          nq, nkv, hd, page_size, float(scale), int(window), _stream())
 
 
@@ -969,24 +937,12 @@ def gemm_skinny_supports(m: int, n: int, k: int, ldx: int, ldw: int) -> bool:
     return bool(lib().pyre_gemm_skinny_supports(m, n, k, ldx, ldw))
 
 
-def _skinny_common(x, w, m):
-    _dev(x, w)
-    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
-        raise KernelError("gemm_skinny: bfloat16 operands expected")
-    if x.dim() != 2 or w.dim() != 2 or x.size(1) != w.size(1) or x.size(0) < m:
-        raise KernelError(f"gemm_skinny: x {tuple(x.shape)} and w {tuple(w.shape)} do not fit {m} rows")
-    if x.stride(1) != 1 or w.stride(1) != 1:
-        raise KernelError("gemm_skinny: rows must be contiguous")
-
-
 def gemm_skinny_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, ksplit: int) -> None:
     """out[s] (float32 [ksplit, m, N]) = partial sums over k of x[0:m] @ w.T, 1 <= m <= 64."""
-    _skinny_common(x, w, m)
-    n = w.shape[0]
-    if out.dtype != torch.float32 or not out.is_contiguous() or out.numel() < ksplit * m * n or not out.is_cuda:
+    operands, (n, k) = binding.product(x, w, m)
+    if not binding.sums(out, ksplit * m * n):
         raise KernelError("gemm_skinny: out must be contiguous float32 [ksplit, m, N] on the GPU")
-    call("pyre_gemm_skinny_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), m, n,
-         w.shape[1], ksplit, _stream())
+    call("pyre_gemm_skinny_bf16", *operands, out, m, n, k, ksplit, _stream())
 
 
 def _gate_shape(unit) -> tuple[float, float, float, float]:
@@ -1005,17 +961,14 @@ def gemm_skinny_silu_bf16(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.T
     """out[0:m] (bfloat16 [m, I]) = silu(x @ gate.T) * (x @ up.T) with w_gate_up = [gate; up]. ``unit`` =
     (limit, slope, shift[, cubic]): g * sigmoid(slope * (g + cubic g^3)) * (u + shift) with g = min(gate, limit),
     u = clamp(up, -limit, limit) instead (limit <= 0: no clipping)."""
-    _skinny_common(x, w_gate_up, m)
-    two_i = w_gate_up.shape[0]
+    operands, (two_i, k) = binding.product(x, w_gate_up, m)
     if (out.dtype != torch.bfloat16 or not out.is_contiguous() or not out.is_cuda or out.dim() != 2
             or out.shape[1] * 2 != two_i or out.shape[0] < m):
         raise KernelError("gemm_skinny_silu: out must be contiguous bfloat16 [>= m, I] on the GPU")
     if unit is not None:
-        call("pyre_gemm_skinny_glu_bf16", x.data_ptr(), x.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0),
-             out.data_ptr(), m, two_i, w_gate_up.shape[1], *_gate_shape(unit), _stream())
+        call("pyre_gemm_skinny_glu_bf16", *operands, out, m, two_i, k, *_gate_shape(unit), _stream())
         return
-    call("pyre_gemm_skinny_silu_bf16", x.data_ptr(), x.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0),
-         out.data_ptr(), m, two_i, w_gate_up.shape[1], _stream())
+    call("pyre_gemm_skinny_silu_bf16", *operands, out, m, two_i, k, _stream())
 
 
 @lru_cache(maxsize=4096)
@@ -1028,12 +981,10 @@ def gemm_mid_supports(m: int, n: int, k: int, ldx: int, ldw: int) -> bool:
 def gemm_mid_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, ksplit: int, wide: bool = False) -> None:
     """out[s] (float32 [ksplit, m, N]) = partial sums over k of x[0:m] @ w.T, 1 <= m <= 256. ``wide``:
     a block takes 128 rows of w instead of 64."""
-    _skinny_common(x, w, m)
-    n = w.shape[0]
-    if out.dtype != torch.float32 or not out.is_contiguous() or out.numel() < ksplit * m * n or not out.is_cuda:
+    operands, (n, k) = binding.product(x, w, m)
+    if not binding.sums(out, ksplit * m * n):
         raise KernelError("gemm_mid: out must be contiguous float32 [ksplit, m, N] on the GPU")
-    call("pyre_gemm_mid_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), m, n,
-         w.shape[1], ksplit, int(wide), _stream())
+    call("pyre_gemm_mid_bf16", *operands, out, m, n, k, ksplit, int(wide), _stream())
 
 
 @lru_cache(maxsize=4096)
@@ -1047,17 +998,14 @@ def gemm_mid_silu_bf16(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tens
                        unit: tuple[float, float, float] | None = None) -> None:
     """out[0:m] (bfloat16 [m, I]) = silu(x @ gate.T) * (x @ up.T) with w_gate_up = [gate; up], 1 <= m <= 256;
     ``unit`` as for :func:`gemm_skinny_silu_bf16`."""
-    _skinny_common(x, w_gate_up, m)
-    two_i = w_gate_up.shape[0]
+    operands, (two_i, k) = binding.product(x, w_gate_up, m)
     if (out.dtype != torch.bfloat16 or not out.is_contiguous() or not out.is_cuda or out.dim() != 2
             or out.shape[1] * 2 != two_i or out.shape[0] < m):
         raise KernelError("gemm_mid_silu: out must be contiguous bfloat16 [>= m, I] on the GPU")
     if unit is not None:
-        call("pyre_gemm_mid_glu_bf16", x.data_ptr(), x.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0),
-             out.data_ptr(), m, two_i, w_gate_up.shape[1], *_gate_shape(unit), _stream())
+        call("pyre_gemm_mid_glu_bf16", *operands, out, m, two_i, k, *_gate_shape(unit), _stream())
         return
-    call("pyre_gemm_mid_silu_bf16", x.data_ptr(), x.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0),
-         out.data_ptr(), m, two_i, w_gate_up.shape[1], _stream())
+    call("pyre_gemm_mid_silu_bf16", *operands, out, m, two_i, k, _stream())
 
 
 @lru_cache(maxsize=4096)
@@ -1089,25 +1037,21 @@ def gemm_tile_choice(m: int, n: int, k: int, gated: bool, parts: int = 0) -> tup
 def gemm_tile_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, m: int, parts: int) -> None:
     """out[s] (float32 [parts, m, N]) = partial sums over k of x[0:m] @ w.T, in tiles of up to 256 x 256;
     ``parts`` as :func:`gemm_tile_parts` says (or another number that leaves every part 256 k)."""
-    _skinny_common(x, w, m)
-    n = w.shape[0]
-    if out.dtype != torch.float32 or not out.is_contiguous() or out.numel() < parts * m * n or not out.is_cuda:
+    operands, (n, k) = binding.product(x, w, m)
+    if not binding.sums(out, parts * m * n):
         raise KernelError("gemm_tile: out must be contiguous float32 [parts, m, N] on the GPU")
-    call("pyre_gemm_tile_bf16", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), m, n, w.shape[1], parts,
-         _stream())
+    call("pyre_gemm_tile_bf16", *operands, out, m, n, k, parts, _stream())
 
 
 def gemm_tile_glu_bf16(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor, m: int,
                        unit: tuple[float, float, float] | None = None) -> None:
     """out[0:m] (bfloat16 [m, I]) = the gated unit of x @ gate.T and x @ up.T with w_gate_up = [gate; up], in tiles of up
     to 256 x 256; ``unit`` as for :func:`gemm_skinny_silu_bf16`."""
-    _skinny_common(x, w_gate_up, m)
-    two_i = w_gate_up.shape[0]
+    operands, (two_i, k) = binding.product(x, w_gate_up, m)
     if (out.dtype != torch.bfloat16 or not out.is_contiguous() or not out.is_cuda or out.dim() != 2
             or out.shape[1] * 2 != two_i or out.shape[0] < m):
         raise KernelError("gemm_tile_glu: out must be contiguous bfloat16 [>= m, I] on the GPU")
-    call("pyre_gemm_tile_glu_bf16", x.data_ptr(), x.stride(0), w_gate_up.data_ptr(), w_gate_up.stride(0), out.data_ptr(), m,
-         two_i, w_gate_up.shape[1], *(_gate_shape(unit) if unit is not None else (0.0, 1.0, 0.0, 0.0)), _stream())
+    call("pyre_gemm_tile_glu_bf16", *operands, out, m, two_i, k, *(_gate_shape(unit) if unit is not None else (0.0, 1.0, 0.0, 0.0)), _stream())
 
 
 def read_bandwidth(device: str = "cuda:0", gib: float = 2.0, blocks: int = 4096, repeats: int = 10) -> float:
@@ -1120,11 +1064,11 @@ def read_bandwidth(device: str = "cuda:0", gib: float = 2.0, blocks: int = 4096,
     sink = torch.zeros(1, dtype=torch.int32, device=device)
     with torch.cuda.device(buf.device):
         for _ in range(2):
-            call("pyre_read_probe", buf.data_ptr(), n, blocks, sink.data_ptr(), _stream())
+            call("pyre_read_probe", buf, n, blocks, sink, _stream())
         torch.cuda.synchronize()
         t = time.perf_counter()
         for _ in range(repeats):
-            call("pyre_read_probe", buf.data_ptr(), n, blocks, sink.data_ptr(), _stream())
+            call("pyre_read_probe", buf, n, blocks, sink, _stream())
         torch.cuda.synchronize()
     return n * repeats / (time.perf_counter() - t) / 1e9
 
@@ -1164,8 +1108,8 @@ def add_tanhnorm(resid: torch.Tensor, delta: Partials | None, alpha: torch.Tenso
         raise KernelError("add_tanhnorm: at most two pending terms")
     while len(terms) < 2:
         terms.append((None, 0, 0, 0, None, 0, 1.0))
-    call("pyre_add_tanhnorm", resid.data_ptr(), *terms[0], *terms[1], alpha.data_ptr(), gain.data_ptr(), _ptr(shift),
-         dtype_code(gain), out.data_ptr(), dtype_code(out), _ptr(rows), n, hidden, _stream())
+    call("pyre_add_tanhnorm", resid, *terms[0], *terms[1], alpha, gain, shift,
+         dtype_code(gain), out, dtype_code(out), rows, n, hidden, _stream())
 
 
 def softcap_(x: torch.Tensor, cap: float) -> None:
@@ -1173,7 +1117,7 @@ def softcap_(x: torch.Tensor, cap: float) -> None:
     _dev(x)
     if x.dtype != torch.float32 or not x.is_contiguous():
         raise KernelError("softcap_: contiguous float32 expected")
-    call("pyre_softcap", x.data_ptr(), x.numel(), float(cap), _stream())
+    call("pyre_softcap", x, x.numel(), float(cap), _stream())
 
 
 def rope_tied_write(proj: Partials, col0: int, q_out: torch.Tensor, k_cache: torch.Tensor | None,
@@ -1209,10 +1153,10 @@ def rope_tied_write(proj: Partials, col0: int, q_out: torch.Tensor, k_cache: tor
             raise KernelError(f"rope_tied_write: caches {tuple(k_cache.shape)} / {tuple(v_cache.shape)} do not fit "
                               f"nkv={nkv} page={page_size} d={d}")
         cache_dt = dtype_code(k_cache)
-    call("pyre_rope_tied_write", proj.data.data_ptr(), dtype_code(proj.data), proj.count, proj.stride, proj.width, col0,
-         _ptr(proj.bias), dtype_code(proj.bias) if proj.bias is not None else 0, q_out.data_ptr(), dtype_code(q_out),
-         _ptr(k_cache), _ptr(v_cache), cache_dt, _ptr(cos) if rot else None, _ptr(sin) if rot else None, int(rot),
-         positions.data_ptr(), _ptr(slots), n, nq, nkv, d, page_size, 1 if write else 0, _stream())
+    call("pyre_rope_tied_write", proj.data, dtype_code(proj.data), proj.count, proj.stride, proj.width, col0,
+         proj.bias, dtype_code(proj.bias) if proj.bias is not None else 0, q_out, dtype_code(q_out),
+         k_cache, v_cache, cache_dt, cos if rot else None, sin if rot else None, int(rot),
+         positions, slots, n, nq, nkv, d, page_size, 1 if write else 0, _stream())
 
 
 def latent_rows(proj: Partials, n: int, rank: int, rot: int, dtype: torch.dtype, cos: torch.Tensor | None = None,
@@ -1270,8 +1214,8 @@ def latent_rows(proj: Partials, n: int, rank: int, rot: int, dtype: torch.dtype,
     if gate is not None:
         g0, gate_width, out_t = gate
         gate_out = rows_of("gate", out_t, gate_width, torch.float32)
-    call("pyre_latent_rows", proj.data.data_ptr(), dtype_code(proj.data), proj.count, proj.stride, proj.width, dtype_code(dtype),
-         _ptr(cos) if rot else None, _ptr(sin) if rot else None, int(neighbours), _ptr(positions), rank, rot, heads, dim,
+    call("pyre_latent_rows", proj.data, dtype_code(proj.data), proj.count, proj.stride, proj.width, dtype_code(dtype),
+         cos if rot else None, sin if rot else None, int(neighbours), positions, rank, rot, heads, dim,
          q_rank, q0, q_out, wide, q_gain, r0, cache, gain, slots, gate_width, g0, gate_out, float(eps), n, _stream())
 
 
@@ -1292,8 +1236,8 @@ def head_matmul(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, n: int, gat
         _contig("gate", gate)
         if gate.dtype != torch.float32 or gate.numel() < n * heads * dout:
             raise KernelError("head_matmul: the gate is float32 [>= n, heads * dout]")
-    call("pyre_head_matmul", x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(), out.data_ptr(), out.stride(0),
-         out.stride(1), _ptr(gate), dtype_code(x), n, heads, din, dout, _stream())
+    call("pyre_head_matmul", x, x.stride(0), x.stride(1), w, out, out.stride(0),
+         out.stride(1), gate, dtype_code(x), n, heads, din, dout, _stream())
 
 
 LATENT_MAX_RANK, LATENT_MAX_ROW = 512, 640  #: the longest rows that the kernels take (latent_attention.hip)
@@ -1322,9 +1266,9 @@ def latent_attn_tile(q, rows, out, tiles, n_tiles, positions, seq_of_token, bloc
     rank]``, the softmax-weighted sum of the rows' first ``rank`` elements; scores, weights and sums float32."""
     _latent_attn_args(q, rows, out, positions, seq_of_token, block_table, heads, rank, dk, page_size, sink)
     _i32("tiles", tiles, 2 * n_tiles)
-    call("pyre_latent_attn_tile", q.data_ptr(), rows.data_ptr(), out.data_ptr(), dtype_code(q), tiles.data_ptr(), n_tiles,
-         positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(), block_table.shape[1], heads, rank, dk,
-         page_size, float(scale), int(window), _ptr(sink), _stream())
+    call("pyre_latent_attn_tile", q, rows, out, dtype_code(q), tiles, n_tiles,
+         positions, seq_of_token, block_table, block_table.shape[1], heads, rank, dk,
+         page_size, float(scale), int(window), sink, _stream())
 
 
 def latent_attn_spans(table_width: int, page_size: int, window: int) -> int:
@@ -1347,9 +1291,9 @@ def latent_attn_single(q, rows, out, tokens, n, positions, seq_of_token, block_t
         if scratch is None or scratch.dtype != torch.float32 or scratch.numel() < n * heads * spans * (rank + 2):
             raise KernelError(f"latent attention: {spans} spans need {n * heads * spans * (rank + 2)} float32 of scratch")
         _dev(scratch)
-    call("pyre_latent_attn_single", q.data_ptr(), rows.data_ptr(), out.data_ptr(), dtype_code(q), _ptr(tokens), n,
-         positions.data_ptr(), seq_of_token.data_ptr(), block_table.data_ptr(), block_table.shape[1], heads, rank, dk,
-         page_size, float(scale), int(window), _ptr(sink), _ptr(scratch) if spans > 1 else None, _stream())
+    call("pyre_latent_attn_single", q, rows, out, dtype_code(q), tokens, n,
+         positions, seq_of_token, block_table, block_table.shape[1], heads, rank, dk,
+         page_size, float(scale), int(window), sink, scratch if spans > 1 else None, _stream())
 
 
 def gemm_tile_paged(rows, groups, n_groups, block_table, w, out) -> None:
@@ -1366,8 +1310,8 @@ def gemm_tile_paged(rows, groups, n_groups, block_table, w, out) -> None:
         raise KernelError(f"gemm_tile_paged: rows [pages, 1, page, row] and w [N, <= row], not {tuple(rows.shape)} and {tuple(w.shape)}")
     if out.dim() != 3 or out.shape[0] * out.shape[2] != w.shape[0] or out.shape[1] != 32 * n_groups:
         raise KernelError(f"gemm_tile_paged: out is [heads, {32 * n_groups}, {w.shape[0]} / heads], not {tuple(out.shape)}")
-    call("pyre_gemm_tile_paged_bf16", rows.data_ptr(), rows.shape[0], rows.shape[2], rows.shape[3], groups.data_ptr(), n_groups,
-         block_table.data_ptr(), block_table.shape[1], w.data_ptr(), out.data_ptr(), w.shape[0], w.shape[1], out.shape[2], _stream())
+    call("pyre_gemm_tile_paged_bf16", rows, rows.shape[0], rows.shape[2], rows.shape[3], groups, n_groups,
+         block_table, block_table.shape[1], w, out, w.shape[0], w.shape[1], out.shape[2], _stream())
 
 
 LATENT_HEADS_TOKENS = 64  #: queries of a tile of :func:`latent_heads`
@@ -1403,9 +1347,9 @@ def latent_heads(q, turned, kv, rows, out, tiles, n_tiles, block_table, scale, w
     if sink is not None and (sink.dtype != torch.float32 or sink.numel() != heads or not sink.is_contiguous()):
         raise KernelError("latent_heads: the sink is float32 [heads]")
     _i32("tiles", tiles, 5 * n_tiles), _i32("block_table", block_table)
-    call("pyre_latent_heads", q.data_ptr(), turned.data_ptr(), turned.stride(0), turned.stride(1), kv.data_ptr(), kv.shape[1], rows.data_ptr(),
-         rows.shape[3], rows.shape[2], out.data_ptr(), _ptr(gate), tiles.data_ptr(), n_tiles, block_table.data_ptr(),
-         block_table.shape[1], heads, key_dim, rot, value_dim, float(scale), int(window), _ptr(sink), _stream())
+    call("pyre_latent_heads", q, turned, turned.stride(0), turned.stride(1), kv, kv.shape[1], rows,
+         rows.shape[3], rows.shape[2], out, gate, tiles, n_tiles, block_table,
+         block_table.shape[1], heads, key_dim, rot, value_dim, float(scale), int(window), sink, _stream())
 
 
 MAX_STREAMS = 8  #: streams of a residual that the kernel takes (streams.hip)
@@ -1448,8 +1392,8 @@ def stream_norm(src: torch.Tensor, dst: torch.Tensor | None, streams: int, delta
             raise KernelError("stream_norm: dst is float32 [N, streams * H], and rows are not stored")
     if rows is not None:
         _i32("rows", rows)
-    call("pyre_stream_norm", src.data_ptr(), src.shape[1] // hidden, _ptr(dst), streams, *d, _ptr(mix), _ptr(out_w),
-         _ptr(in_w), gain.data_ptr(), _ptr(shift), int(center), float(eps), out.data_ptr(), dtype_code(out), _ptr(rows), n,
+    call("pyre_stream_norm", src, src.shape[1] // hidden, dst, streams, *d, mix, out_w,
+         in_w, gain, shift, int(center), float(eps), out, dtype_code(out), rows, n,
          hidden, _stream())
 
 
@@ -1462,8 +1406,8 @@ def poly_norm(z: Partials, abce: torch.Tensor, eps: float, out: torch.Tensor, n:
     if abce.dtype != torch.float32 or abce.numel() != 4:
         raise KernelError("poly_norm: the coefficients are float32 [4]")
     _contig("abce", abce), _contig("out", out)
-    call("pyre_poly_norm", z.data.data_ptr(), dtype_code(z.data), z.count, z.stride, abce.data_ptr(), float(eps),
-         out.data_ptr(), dtype_code(out), n, z.width, _stream())
+    call("pyre_poly_norm", z.data, dtype_code(z.data), z.count, z.stride, abce, float(eps),
+         out, dtype_code(out), n, z.width, _stream())
 
 
 ROUTE_MAX_EXPERTS = 512  #: the most experts that the routing kernel chooses among (moe.hip)
@@ -1481,7 +1425,7 @@ def route_topk(z: Partials, gates: torch.Tensor, n: int, top: int, softmax: bool
         raise KernelError("route_topk: gates are contiguous float32 [>= n, experts + extra]")
     if extra < 0 or not (0 < top <= experts <= ROUTE_MAX_EXPERTS):
         raise KernelError(f"route_topk: {top} of {experts} experts is not a choice this kernel makes")
-    call("pyre_route_topk", *z._args(z.width), gates.data_ptr(), n, experts, int(top), int(bool(softmax)), int(extra),
+    call("pyre_route_topk", *z._args(z.width), gates, n, experts, int(top), int(bool(softmax)), int(extra),
          _stream())
 
 
@@ -1497,8 +1441,8 @@ def expert_act(up: Partials, gates: torch.Tensor, out: torch.Tensor, n: int, exp
     if gates.dtype != torch.float32 or not gates.is_contiguous() or gates.shape[-1] != experts or gates.shape[0] < n:
         raise KernelError("expert_act: gates are contiguous float32 [>= n, experts]")
     _contig("out", out)
-    call("pyre_expert_act", up.data.data_ptr(), dtype_code(up.data), up.count, up.stride, gates.data_ptr(),
-         out.data_ptr(), dtype_code(out), n, experts, ff, shared_ff, _stream())
+    call("pyre_expert_act", up.data, dtype_code(up.data), up.count, up.stride, gates,
+         out, dtype_code(out), n, experts, ff, shared_ff, _stream())
 
 
 def _term_args(t: Partials | None, hidden: int, what: str):
@@ -1563,9 +1507,9 @@ def add_rms_terms(resid: torch.Tensor, delta: Partials | None, gain: torch.Tenso
             raise KernelError("add_rms_terms: the norm of the sum is an RMS norm with a gain over the hidden size")
         _dev(outer.gain), _contig("outer.gain", outer.gain)
         o = (outer.gain.data_ptr(), dtype_code(outer.gain), float(outer.eps))
-    call("pyre_add_rms_terms", resid.data_ptr(), *a, *b, float(inner[0]) if inner else 0.0, *o, _ptr(gain),
-         dtype_code(gain) if gain is not None else 0, float(eps), _ptr(out), dtype_code(out) if out is not None else 0,
-         _ptr(rows), n, hidden, _stream())
+    call("pyre_add_rms_terms", resid, *a, *b, float(inner[0]) if inner else 0.0, *o, gain,
+         dtype_code(gain) if gain is not None else 0, float(eps), out, dtype_code(out) if out is not None else 0,
+         rows, n, hidden, _stream())
 
 
 def bigram_embed(table: torch.Tensor, pairs: torch.Tensor, ids: torch.Tensor, positions: torch.Tensor,
@@ -1589,9 +1533,9 @@ def bigram_embed(table: torch.Tensor, pairs: torch.Tensor, ids: torch.Tensor, po
     _contig("table", table), _contig("pairs", pairs), _contig("out", out)
     _i32("ids", ids, n), _i32("positions", positions, n), _i32("seq_of_token", seq_of_token, n)
     _i32("q_start", q_start), _i32("state_slots", state_slots)
-    call("pyre_bigram_embed", table.data_ptr(), pairs.data_ptr(), dtype_code(table), ids.data_ptr(), positions.data_ptr(),
-         seq_of_token.data_ptr(), q_start.data_ptr(), state.data_ptr(), state_slots.data_ptr(), _ptr(places),
-         places.shape[0] if places is not None else 0, out.data_ptr(), n, hidden, int(buckets), int(mul_prev), int(mul_cur), _stream())
+    call("pyre_bigram_embed", table, pairs, dtype_code(table), ids, positions,
+         seq_of_token, q_start, state, state_slots, places,
+         places.shape[0] if places is not None else 0, out, n, hidden, int(buckets), int(mul_prev), int(mul_cur), _stream())
 
 
 CONV_MAX_TAPS = 16  #: the most taps of the short convolution (conv_attention.hip)
@@ -1656,10 +1600,10 @@ def conv_qkv_write(proj: Partials, col0: int, taps_w: torch.Tensor | None, conv_
         cache_dt = dtype_code(k_cache)
     if gate_out is not None and (gate_out.dtype != torch.float32 or gate_out.numel() < n * nq * dv or not gate_out.is_contiguous()):
         raise KernelError("conv_qkv_write: gates are contiguous float32 [N, nq*dv]")
-    call("pyre_conv_qkv_write", *args, _ptr(taps_w), taps, _ptr(conv_state) if taps > 1 else None, state_slots.data_ptr(),
-         seq_of_token.data_ptr(), q_start.data_ptr(), n_seqs, _ptr(q_gain), _ptr(k_gain), float(eps),
-         _ptr(cos) if rot else None, _ptr(sin) if rot else None, int(rot), int(bool(neighbours)), positions.data_ptr(),
-         q_out.data_ptr(), dtype_code(q_out), _ptr(k_cache), _ptr(v_cache), cache_dt, _ptr(gate_out), _ptr(slots), n, nq,
+    call("pyre_conv_qkv_write", *args, taps_w, taps, conv_state if taps > 1 else None, state_slots,
+         seq_of_token, q_start, n_seqs, q_gain, k_gain, float(eps),
+         cos if rot else None, sin if rot else None, int(rot), int(bool(neighbours)), positions,
+         q_out, dtype_code(q_out), k_cache, v_cache, cache_dt, gate_out, slots, n, nq,
          nkv, dk, dv, page_size, 1 if write else 0, int(bool(single)), _stream())
 
 
@@ -1682,8 +1626,8 @@ def retention_prepare(proj: Partials, col0: int, log_decay: torch.Tensor, cos: t
                 or cos.dim() != 2 or cos.shape[1] != rot // 2 or tuple(cos.shape) != tuple(sin.shape):
             raise KernelError("retention_prepare: cos and sin are float32 [positions, rot / 2], rot even and within the head")
         _contig("cos", cos), _contig("sin", sin)
-    call("pyre_retention_prepare", *args, log_decay.data_ptr(), _ptr(cos) if rot else None, _ptr(sin) if rot else None,
-         int(rot), int(bool(neighbours)), positions.data_ptr(), float(kscale), int(bool(silu)), x.data_ptr(), n, heads, dk,
+    call("pyre_retention_prepare", *args, log_decay, cos if rot else None, sin if rot else None,
+         int(rot), int(bool(neighbours)), positions, float(kscale), int(bool(silu)), x, n, heads, dk,
          dv, _stream())
 
 
@@ -1705,7 +1649,7 @@ def route_grouped(z: Partials, correction: torch.Tensor | None, gates: torch.Ten
     if correction is not None and (correction.dtype != torch.float32 or correction.numel() != experts or
                                    not correction.is_contiguous()):
         raise KernelError("route_grouped: the correction is contiguous float32 [experts]")
-    call("pyre_route_grouped", *z._args(experts), _ptr(correction), gates.data_ptr(), n, experts, int(top), int(groups),
+    call("pyre_route_grouped", *z._args(experts), correction, gates, n, experts, int(top), int(groups),
          int(keep_groups), _stream())
 
 
@@ -1726,8 +1670,8 @@ def expert_glu_act(gu: Partials, gates: torch.Tensor, out: torch.Tensor, n: int,
     if gates.dtype != torch.float32 or gates.dim() != 2 or gates.stride(1) != 1 or gates.shape[1] < experts or gates.shape[0] < n:
         raise KernelError("expert_glu_act: gates are float32 [>= n, >= experts] with contiguous rows")
     _contig("out", out)
-    call("pyre_expert_glu_act", gu.data.data_ptr(), dtype_code(gu.data), gu.count, gu.stride, gates.data_ptr(),
-         gates.stride(0), out.data_ptr(), dtype_code(out), n, experts, ff, int(shared_ff), int(shared_gate), _stream())
+    call("pyre_expert_glu_act", gu.data, dtype_code(gu.data), gu.count, gu.stride, gates,
+         gates.stride(0), out, dtype_code(out), n, experts, ff, int(shared_ff), int(shared_gate), _stream())
 
 
 def add_weighted_rows(p: Partials, h: torch.Tensor, gates: torch.Tensor, first: int, count: int, n: int) -> None:
@@ -1741,7 +1685,7 @@ def add_weighted_rows(p: Partials, h: torch.Tensor, gates: torch.Tensor, first: 
     if gates.dtype != torch.float32 or gates.dim() != 2 or gates.stride(1) != 1 or first < 0 or count <= 0 or \
             first + count > gates.shape[1] or gates.shape[0] < n:
         raise KernelError("add_weighted_rows: gates are float32 [>= n, >= first + count] with contiguous rows")
-    call("pyre_add_weighted_rows", p.data.data_ptr(), h.data_ptr(), dtype_code(h), h.stride(0), gates.data_ptr(),
+    call("pyre_add_weighted_rows", p.data, h, dtype_code(h), h.stride(0), gates,
          gates.stride(0), int(first), int(count), n, p.width, _stream())
 
 
@@ -1753,8 +1697,8 @@ def relu2(up: Partials, out: torch.Tensor, n: int) -> None:
     if up.rows < n or out.shape[-1] != up.width or out.shape[0] < n:
         raise KernelError("relu2: the output does not fit the product")
     _contig("out", out)
-    call("pyre_expert_act", up.data.data_ptr(), dtype_code(up.data), up.count, up.stride, None,
-         out.data_ptr(), dtype_code(out), n, 0, 4, up.width, _stream())
+    call("pyre_expert_act", up.data, dtype_code(up.data), up.count, up.stride, None,
+         out, dtype_code(out), n, 0, 4, up.width, _stream())
 
 
 def _proj_bias_args(proj: Partials, col0: int, width: int):
@@ -1808,8 +1752,8 @@ def wide_norm_qkv_write(proj: Partials, col0: int, q_gain: torch.Tensor | None, 
             raise KernelError(f"wide_norm_qkv_write: caches {tuple(k_cache.shape)} / {tuple(v_cache.shape)} do not fit "
                               f"nkv={nkv} page={page_size} dk={dk} dv={dv}")
         cache_dt = dtype_code(k_cache)
-    call("pyre_wide_norm_qkv_write", *args, _ptr(q_gain), _ptr(k_gain), float(eps), c, s, int(rot), positions.data_ptr(),
-         q_out.data_ptr(), dtype_code(q_out), _ptr(k_cache), _ptr(v_cache), cache_dt, _ptr(slots), n, nq, nkv, dk, dv,
+    call("pyre_wide_norm_qkv_write", *args, q_gain, k_gain, float(eps), c, s, int(rot), positions,
+         q_out, dtype_code(q_out), k_cache, v_cache, cache_dt, slots, n, nq, nkv, dk, dv,
          page_size, 1 if write else 0, _stream())
 
 
@@ -1855,9 +1799,9 @@ def gdr_prepare(proj: Partials, col0: int, taps_w: torch.Tensor | None, conv_sta
         if taps > 1 and (conv_state is None or conv_state.dtype != torch.float32 or not conv_state.is_contiguous() or
                          tuple(conv_state.shape[1:]) != (taps - 1, channels)):
             raise KernelError(f"gdr_prepare: the state is contiguous float32 [slots, {taps - 1}, {channels}]")
-    call("pyre_gdr_prepare", *args, _ptr(taps_w), taps, _ptr(conv_state) if taps > 1 else None, state_slots.data_ptr(),
-         seq_of_token.data_ptr(), q_start.data_ptr(), n_seqs, a2.data_ptr(), dtype_code(a2), dt_bias.data_ptr(),
-         rate.data_ptr(), g2.data_ptr(), dtype_code(g2), float(unit_eps), x.data_ptr(), n, heads, kv_heads, dk, dv,
+    call("pyre_gdr_prepare", *args, taps_w, taps, conv_state if taps > 1 else None, state_slots,
+         seq_of_token, q_start, n_seqs, a2, dtype_code(a2), dt_bias,
+         rate, g2, dtype_code(g2), float(unit_eps), x, n, heads, kv_heads, dk, dv,
          rank_a, rank_g, _stream())
 
 
@@ -1875,7 +1819,7 @@ def gdr_scan(x: torch.Tensor, state: torch.Tensor, o: torch.Tensor, q_start: tor
             o.shape[-1] != heads * dv:
         raise KernelError("gdr_scan: shapes do not fit the head geometry")
     _i32("q_start", q_start, n_seqs + 1), _i32("state_slots", state_slots, n_seqs)
-    call("pyre_gdr_scan", x.data_ptr(), state.data_ptr(), o.data_ptr(), q_start.data_ptr(), state_slots.data_ptr(), n_seqs,
+    call("pyre_gdr_scan", x, state, o, q_start, state_slots, n_seqs,
          int(max_tokens), heads, kv_heads, dk, dv, _stream())
 
 
@@ -1890,8 +1834,8 @@ def gdr_finish(o: torch.Tensor, x: torch.Tensor, gain: torch.Tensor, eps: float,
             x.shape[-1] != gdr_row_width(heads, kv_heads, dk, dv) or o.shape[-1] != heads * dv:
         raise KernelError("gdr_finish: gain [dv] and out [>= n, >= heads*dv] expected")
     _contig("gain", gain)
-    call("pyre_gdr_finish", o.data_ptr(), x.data_ptr(), gain.data_ptr(), dtype_code(gain), float(eps), float(out_scale),
-         out.data_ptr(), dtype_code(out), out.stride(0), n, heads, kv_heads, dk, dv, _stream())
+    call("pyre_gdr_finish", o, x, gain, dtype_code(gain), float(eps), float(out_scale),
+         out, dtype_code(out), out.stride(0), n, heads, kv_heads, dk, dv, _stream())
 
 
 def token_side_gate(z: Partials, table: torch.Tensor, first: int, ids: torch.Tensor, out: torch.Tensor, n: int) -> None:
@@ -1903,8 +1847,8 @@ def token_side_gate(z: Partials, table: torch.Tensor, first: int, ids: torch.Ten
     if out.shape[-1] != dim or out.shape[0] < n or z.rows < n:
         raise KernelError("token_side_gate: the output does not fit the product")
     _contig("out", out), _i32("ids", ids, n)
-    call("pyre_token_side_gate", *z._args(dim), table.data_ptr(), dtype_code(table), table.shape[1], int(first),
-         ids.data_ptr(), out.data_ptr(), dtype_code(out), n, dim, _stream())
+    call("pyre_token_side_gate", *z._args(dim), table, dtype_code(table), table.shape[1], int(first),
+         ids, out, dtype_code(out), n, dim, _stream())
 
 
 SSM_MAX_STATE = 256      #: the largest state of a channel that the selective scan's kernels take (selective_scan.hip)
@@ -1949,9 +1893,9 @@ def ssm_conv(proj: Partials, col0: int, taps_w: torch.Tensor, conv_b: torch.Tens
         raise KernelError(f"ssm_conv: x is [>= {n}, {inner}]")
     if single and n != n_seqs:
         raise KernelError(f"ssm_conv: {n} tokens of {n_seqs} requests are not one token each")
-    call("pyre_ssm_conv", *args, proj.width, int(col0), _ptr(proj.bias), taps_w.data_ptr(), taps, conv_b.data_ptr(),
-         conv_state.data_ptr() if taps > 1 else None, state_slots.data_ptr(), seq_of_token.data_ptr(), q_start.data_ptr(),
-         n_seqs, int(bool(single)), x.data_ptr(), dtype_code(x), n, inner, _stream())
+    call("pyre_ssm_conv", *args, proj.width, int(col0), proj.bias, taps_w, taps, conv_b,
+         conv_state if taps > 1 else None, state_slots, seq_of_token, q_start,
+         n_seqs, int(bool(single)), x, dtype_code(x), n, inner, _stream())
 
 
 def ssm_low(sel: Partials, rank: int, out: torch.Tensor, n: int) -> None:
@@ -1962,7 +1906,7 @@ def ssm_low(sel: Partials, rank: int, out: torch.Tensor, n: int) -> None:
     padded = out.shape[-1] if out.dtype == torch.float32 else out.shape[-1] // 2
     if out.shape[0] < n or padded < rank or (out.dtype == torch.bfloat16 and out.shape[-1] % 2):
         raise KernelError(f"ssm_low: out {tuple(out.shape)} does not hold {n} rows of {rank} columns")
-    call("pyre_ssm_low", *args, sel.width, out.data_ptr(), dtype_code(out), int(rank), int(padded), n, _stream())
+    call("pyre_ssm_low", *args, sel.width, out, dtype_code(out), int(rank), int(padded), n, _stream())
 
 
 def _ssm_common(what, x, sel, rank, gate, g0, A2, D, dt_b, state, out, n, inner, n_state):
@@ -1987,9 +1931,9 @@ def ssm_scan(z: Partials, dt_b: torch.Tensor, x: torch.Tensor, sel: Partials, ra
     if z.width != inner:
         raise KernelError("ssm_scan: the step sizes' product is as wide as the channels")
     _i32("q_start", q_start, n_seqs + 1), _i32("state_slots", state_slots, n_seqs), _dev(q_start, state_slots)
-    call("pyre_ssm_scan", *zp, dt_b.data_ptr(), x.data_ptr(), dtype_code(x), *s, sel.width, int(rank), *g, gate.width,
-         _ptr(gate.bias), int(g0), A2.data_ptr(), D.data_ptr(), state.data_ptr(), q_start.data_ptr(), state_slots.data_ptr(), n_seqs, float(out_scale),
-         out.data_ptr(), dtype_code(out), out.stride(0), inner, n_state, _stream())
+    call("pyre_ssm_scan", *zp, dt_b, x, dtype_code(x), *s, sel.width, int(rank), *g, gate.width,
+         gate.bias, int(g0), A2.data_ptr(), D.data_ptr(), state, q_start, state_slots, n_seqs, float(out_scale),
+         out, dtype_code(out), out.stride(0), inner, n_state, _stream())
 
 
 def ssm_step(dt_w: torch.Tensor, dt_b: torch.Tensor, x: torch.Tensor, sel: Partials, rank: int, gate: Partials, g0: int,
@@ -2002,6 +1946,6 @@ def ssm_step(dt_w: torch.Tensor, dt_b: torch.Tensor, x: torch.Tensor, sel: Parti
     _dev(dt_w, state_slots), _i32("state_slots", state_slots, n_seqs)
     if dt_w.dim() != 2 or dt_w.shape[0] != inner or dt_w.shape[1] < rank or dt_w.stride(1) != 1:
         raise KernelError(f"ssm_step: the step sizes' matrix is [{inner}, >= {rank}] with contiguous rows")
-    call("pyre_ssm_step", dt_w.data_ptr(), dtype_code(dt_w), dt_w.stride(0), dt_b.data_ptr(), x.data_ptr(), dtype_code(x), *s,
-         sel.width, int(rank), *g, gate.width, _ptr(gate.bias), int(g0), A2.data_ptr(), D.data_ptr(), state.data_ptr(), state_slots.data_ptr(),
-         n_seqs, float(out_scale), out.data_ptr(), dtype_code(out), out.stride(0), inner, n_state, _stream())
+    call("pyre_ssm_step", dt_w, dtype_code(dt_w), dt_w.stride(0), dt_b, x, dtype_code(x), *s,
+         sel.width, int(rank), *g, gate.width, gate.bias, int(g0), A2.data_ptr(), D.data_ptr(), state, state_slots,
+         n_seqs, float(out_scale), out, dtype_code(out), out.stride(0), inner, n_state, _stream())

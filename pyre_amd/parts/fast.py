@@ -147,7 +147,9 @@ def narrow_kernel(n: int, n_out: int, k: int, options: dict | None = None,
     device's compute units, which an engine reads once) alone; the
     thresholds in rows lie just above sizes at which decode steps are captured, so that an eager step
     and its replay at the padded size agree."""
-    opt = options or {}
+    if not options:
+        return _narrow_kernel(n, n_out, k, units, True, MID_WIDE_MIN_ROWS, True, True)
+    opt = options
     return _narrow_kernel(n, n_out, k, units, opt.get("mid_gemm", True), opt.get("mid_wide_min_rows", MID_WIDE_MIN_ROWS),
                           opt.get("skinny_gemm", True), opt.get("mid_small", True))
 
@@ -193,13 +195,16 @@ def linear(lin, ctx, x, n, out):
     rt = ctx.runtime
     if not _is_bf16(ctx, lin, x):
         return None
-    k, n_out = lin.in_features, lin.out_features
-    streams = rt.options.get("skinny_gemm", True) and ops.gemm_skinny_supports(
-        min(n, SKINNY_MAX_ROWS), n_out, k, x.stride(0), lin.weight.stride(0))
+    k, n_out, weight = lin.in_features, lin.out_features, lin.weight
+    ldx, ldw = x.stride(0), weight.stride(0)
     library = rt.options.get("library_gemm", True)
+
+    def streams() -> bool:
+        return rt.options.get("skinny_gemm", True) and ops.gemm_skinny_supports(min(n, SKINNY_MAX_ROWS), n_out, k, ldx, ldw)
+
     if out is not None:
         # float32 results wanted in place (the head's logits)
-        if streams and (n <= SKINNY_MAX_ROWS or not library):  # no split, 64 rows at a time
+        if (n <= SKINNY_MAX_ROWS or not library) and streams() and (n <= SKINNY_MAX_ROWS or not library):  # no split, 64 rows at a time
             for r0 in range(0, n, SKINNY_MAX_ROWS):
                 rows = min(SKINNY_MAX_ROWS, n - r0)
                 ops.gemm_skinny_bf16(x[r0:r0 + rows], lin.weight, out[r0:r0 + rows], rows, 1)
@@ -209,20 +214,20 @@ def linear(lin, ctx, x, n, out):
             return None
         return Partials(out.view(1, n, n_out), lin.bias)
     kernel, ks, wide = narrow_kernel(n, n_out, k, rt.options, rt.compute_units)
-    if kernel == "stream" and not streams:
+    if kernel == "stream" and not streams():
         kernel = ""
-    if kernel == "block" and not ops.gemm_mid_supports(n, n_out, k, x.stride(0), lin.weight.stride(0)):
-        kernel, ks = ("stream", skinny_ksplit(n, n_out, k, rt.compute_units)) if streams and n <= SKINNY_MAX_ROWS else ("", 0)
+    if kernel == "block" and not ops.gemm_mid_supports(n, n_out, k, ldx, ldw):
+        kernel, ks = ("stream", skinny_ksplit(n, n_out, k, rt.compute_units)) if n <= SKINNY_MAX_ROWS and streams() else ("", 0)
     if kernel:
-        buf = ctx.workspace.get(f"linear.{lin.role}.partials", (ks, n, n_out), torch.float32)
+        buf = rt.workspace.get(lin.partials_name, (ks, n, n_out), torch.float32)
         if kernel == "stream":
-            ops.gemm_skinny_bf16(x, lin.weight, buf, n, ks)
+            ops.gemm_skinny_bf16(x, weight, buf, n, ks)
         else:
-            ops.gemm_mid_bf16(x, lin.weight, buf, n, ks, wide=wide)
+            ops.gemm_mid_bf16(x, weight, buf, n, ks, wide=wide)
         return Partials(buf, lin.bias)
     if lin.role in TILE_ROLES and takes_tiles(rt, lin, n, x):
         parts = 1 if lin.whole else ops.gemm_tile_parts(n, n_out, k)
-        buf = ctx.workspace.get(f"linear.{lin.role}.partials", (parts, n, n_out), torch.float32)
+        buf = rt.workspace.get(lin.partials_name, (parts, n, n_out), torch.float32)
         ops.gemm_tile_bf16(x, lin.weight, buf, n, parts)
         return Partials(buf, lin.bias)
     if not library:

@@ -21,6 +21,7 @@ class Linear:
         self.in_features = in_features
         self.out_features = out_features
         self.role = role              #: names this product's scratch buffer
+        self.partials_name = f"linear.{role}.partials"
         self.whole = whole            #: of many rows: handed on as one sum, for a consumer that loses more by partial sums
         self.weight: torch.Tensor | None = None   # [out, in]
         self.bias: torch.Tensor | None = None

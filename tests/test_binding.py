@@ -1,0 +1,63 @@
+"""The native half of the binding: what it refuses it refuses as the checks in Python did, and an entry's own refusal comes with the
+library's message. No kernel runs here."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from pyre_amd.hip import lib
+from pyre_amd.hip.native import KernelError, binding
+
+
+def test_checks_of_operands():
+    t = torch.zeros(4, 6)
+    assert binding.dev() is None and binding.dev(None) is None
+    with pytest.raises(KernelError, match="not on a GPU"):
+        binding.dev(None, t)
+    with pytest.raises(TypeError):
+        binding.dev(3)
+    binding.contig("rows", t)
+    with pytest.raises(KernelError, match="rows must be contiguous"):
+        binding.contig("rows", t.t())
+    ids = torch.zeros(5, dtype=torch.int32)
+    binding.i32("ids", ids), binding.i32("ids", ids, 5), binding.i32("ids", ids, None)
+    with pytest.raises(KernelError, match="ids holds 5 entries, 6 needed"):
+        binding.i32("ids", ids, 6)
+    with pytest.raises(KernelError, match="ids must be int32"):
+        binding.i32("ids", ids.long())
+    with pytest.raises(KernelError, match="ids must be contiguous"):
+        binding.i32("ids", torch.zeros(6, dtype=torch.int32)[::2])
+    assert [binding.dtype_code(x) for x in (t, torch.float32, torch.bfloat16, t.bfloat16())] == [0, 0, 1, 1]
+    with pytest.raises(KernelError, match="unsupported element type"):
+        binding.dtype_code(torch.float16)
+    assert binding.ptr(None) is None and binding.ptr(t[1:]) == t.data_ptr() + 24
+    assert not binding.sums(t, 24)  # not on a GPU
+    with pytest.raises(KernelError, match="not on a GPU"):
+        binding.product(t, t, 4)
+
+
+def test_partial_sums():
+    d, bias = torch.zeros(3, 4, 6), torch.zeros(6, dtype=torch.bfloat16)
+    assert binding.partials(d, None, 6) == (d.data_ptr(), 0, 3, 24, None, 0)
+    assert binding.partials(d, bias, 6) == (d.data_ptr(), 0, 3, 24, bias.data_ptr(), 1)
+    with pytest.raises(KernelError, match="6 wide, 8 expected"):
+        binding.partials(d, None, 8)
+    with pytest.raises(KernelError, match="5 entries, 6 expected"):
+        binding.partials(d, bias[:5], 6)
+
+
+def test_entries():
+    lib.lib()
+    with pytest.raises(KernelError, match="M=0"):  # the library's own refusal
+        lib.call("pyre_gemm_mid_bf16", None, 64, None, 64, None, 0, 64, 64, 1, 0, 0)
+    with pytest.raises(KernelError, match="not on a GPU"):
+        lib.call("pyre_gemm_mid_bf16", torch.zeros(4, 4), 64, None, 64, None, 0, 64, 64, 1, 0, 0)
+    with pytest.raises(TypeError, match="takes 11 arguments, 10 given"):
+        lib.call("pyre_gemm_mid_bf16", None, 64, None, 64, None, 0, 64, 64, 1, 0)
+    with pytest.raises(TypeError):
+        lib.call("pyre_gemm_mid_bf16", None, 64.5, None, 64, None, 0, 64, 64, 1, 0, 0)
+    with pytest.raises(OverflowError):
+        lib.call("pyre_gemm_mid_bf16", None, 64, None, 64, None, 1 << 40, 64, 64, 1, 0, 0)
+    with pytest.raises(AttributeError):
+        lib.call("pyre_no_such_entry")
