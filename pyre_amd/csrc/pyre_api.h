@@ -94,8 +94,8 @@ int pyre_gemm_skinny_silu_bf16(const void* X, long ldx, const void* W, long ldw,
 int pyre_gemm_mid_supports(int M, int N, int K, long ldx, long ldw);
 int pyre_gemm_mid_bf16(const void* X, long ldx, const void* W, long ldw, float* out, int M, int N, int K,
                        int ksplit, int wide, hipStream_t stream);
-// The second of them for up to 256 rows: a block takes 64 or 96 features (pyre_gemm_mid_silu_blocks
-// blocks in all) against all rows of X; it pays where one round of blocks holds them.
+// The second of them for up to 256 rows: a block takes up to 64 or 96 features (pyre_gemm_mid_silu_blocks: the blocks that
+// hold them all so; fewer features a block where that fills the chip) against all rows of X; it pays where one round of blocks holds them.
 int pyre_gemm_mid_silu_blocks(int M, int two_i);
 int pyre_gemm_mid_silu_bf16(const void* X, long ldx, const void* W, long ldw, void* out, int M, int two_i,
                             int K, hipStream_t stream);

@@ -250,9 +250,9 @@ def gate_up_silu(lin, ctx, x, n, act, unit=None) -> bool:
         return False
     if ctx.runtime.options.get("mid_silu_min_rows", MID_SILU_MIN_ROWS) <= n <= MID_MAX_ROWS:
         # blocks of 64 features (96 where that is what it takes, up to 128 rows) against all rows,
-        # where one round of blocks holds them. Measured on the 1.5B shape: 17 us against the
-        # library's product and the SiLU-gate kernel's 29 at 65 to 128 rows, 26 against 30 at 192, 28 at 256;
-        # on the 7B shape 55 against 66 at 128, and at 256 rows, as on the 32B shape, two rounds of
+        # where one round of blocks holds them (or fewer features, so that the blocks fill the chip). Measured on the 1.5B shape:
+        # 17 to 19 us against the library's product and the SiLU-gate kernel's 29 at 65 to 128 rows, 23 against 30 at 192, 25 at 256;
+        # on the 7B shape 58 against 66 at 128, and at 256 rows, as on the 32B shape, two rounds of
         # blocks: those go to the kernel of tiles. With blocks of 32 and 64 rows of X for steps that
         # small it is ahead of the weight-streaming kernel at every size: on the 7B shape 3.20
         # against 3.23 ms a step at one request, 3.44 against 3.49 at 8, 3.77 against 3.87 at 16,
