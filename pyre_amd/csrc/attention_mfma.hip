@@ -63,7 +63,10 @@ struct KV {
   const bf16* v;     // layer slab [pages, nkv, HD, page_size]
   const int* table;  // the request's block table
   int nkv, kvh, page_size;
+  int shift = -1;    // the page size's logarithm, where it has a whole one: a division by it takes as long as a quarter of a load
+  __device__ int entry(int key) const { return shift >= 0 ? key >> shift : key / page_size; }
 };
+__device__ inline int shift_of(int page_size) { return page_size & (page_size - 1) ? -1 : __builtin_ctz(page_size); }
 
 // Per-column causal window: column c sees keys in [lo[c], hi[c]].
 template <int CT>
@@ -87,11 +90,12 @@ struct Bounds {
 // is key key0 + 8 g + 4 t + j; load_k(t, c) gives lane (r, g) the row of key
 // key0 + 8 (r / 4) + 4 t + r % 4, load_v(dt) the keys 8 g .. 8 g + 7 in its slots, and
 // tile_ok[h] stands for the chunk's keys 16 h .. 16 h + 15.
-template <int HD, int CT, bool RUNS8 = false, typename LoadK, typename LoadV>
+// `scored` is called when the chunk's keys have been multiplied.
+template <int HD, int CT, bool RUNS8 = false, typename LoadK, typename LoadV, typename Scored>
 __device__ inline void attend_core(int key0, bool edge, const bool (&tile_ok)[2], const Bounds<CT>& bd,
                                    float scale_log2, const bf16x8 (&q)[CT][HD / 32],
                                    f32x4 (&o)[HD / 16][CT], float (&m)[CT], float (&l)[CT],
-                                   LoadK&& load_k, LoadV&& load_v) {
+                                   LoadK&& load_k, LoadV&& load_v, Scored&& scored) {
   const int g = (threadIdx.x & 63) >> 4;
   // S^T tiles: rows = keys key0 + 16 t + (4 g + j), columns = lane's column r.
   f32x4 s[2][CT];
@@ -108,6 +112,7 @@ __device__ inline void attend_core(int key0, bool edge, const bool (&tile_ok)[2]
         s[t][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, q[ct][c], s[t][ct], 0, 0, 0);
     }
   }
+  scored();
 
   // Online softmax per column; P^T packed as the B operand of the second product:
   // slots 0..3 of a lane are keys 4g..4g+3 of tile 0, slots 4..7 those of tile 1.
@@ -194,7 +199,8 @@ __device__ inline void attend_chunk(const KV& kv, int key0, bool edge, const Bou
         }
         const uint4 u = {h[0].x, h[0].y, h[1].x, h[1].y};
         return __builtin_bit_cast(bf16x8, u);
-      });
+      },
+      [] {});
 }
 
 // A chunk's operands held in registers, so that the loads of the next chunk can be
@@ -227,49 +233,69 @@ struct TableWindow {
   }
 };
 
-template <int HD, bool STREAM_V>
-__device__ inline void load_chunk(const KV& kv, TableWindow& tw, int key0, ChunkRegs<HD>& cr) {
+// Where a chunk's keys and values lie for this lane: two loads' worth of look-ups, and the loads.
+struct ChunkPlace {
+  const bf16 *k, *v;
+  bool ok[2], k_ok, v_ok;
+};
+template <int HD>
+__device__ inline ChunkPlace place_chunk(const KV& kv, TableWindow& tw, int key0) {
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  ChunkPlace at;
   size_t base[2];  // (page, key/value head) of each half, in units of page_size * HD elements
   int off[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int k0 = key0 + 16 * h;
-    const int entry = k0 / kv.page_size;
+    const int entry = kv.entry(k0);
     const int page = tw.page(entry);
     off[h] = k0 - entry * kv.page_size;
-    cr.ok[h] = page >= 0;
-    base[h] = static_cast<size_t>(cr.ok[h] ? page : 0) * kv.nkv + kv.kvh;
+    at.ok[h] = page >= 0;
+    base[h] = static_cast<size_t>(at.ok[h] ? page : 0) * kv.nkv + kv.kvh;
   }
   // K: rows 0..7 of a tile are keys of the first half, rows 8..15 of the second.
   const int kh = r >> 3;
-  const bool k_ok = kh ? cr.ok[1] : cr.ok[0];
-  const bf16* kp = kv.k + ((kh ? base[1] : base[0]) * kv.page_size + (kh ? off[1] : off[0]) + 8 * ((r >> 2) & 1) + (r & 3)) * HD + 8 * g;
+  at.k_ok = kh ? at.ok[1] : at.ok[0];
+  at.k = kv.k + ((kh ? base[1] : base[0]) * kv.page_size + (kh ? off[1] : off[0]) + 8 * ((r >> 2) & 1) + (r & 3)) * HD + 8 * g;
+  // V^T: lanes g = 0, 1 take keys of the first half, g = 2, 3 of the second.
+  const int vh = g >> 1;
+  at.v_ok = vh ? at.ok[1] : at.ok[0];
+  at.v = kv.v + ((vh ? base[1] : base[0]) * HD + r) * kv.page_size + (vh ? off[1] : off[0]) + 8 * (g & 1);
+  return at;
+}
+template <int HD>
+__device__ inline void load_keys(const ChunkPlace& at, ChunkRegs<HD>& cr) {
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int c = 0; c < HD / 32; ++c) cr.k[t][c] = k_ok ? load_b128(kp + 4 * t * HD + 32 * c) : zero_b128();
-  // V^T: lanes g = 0, 1 take keys of the first half, g = 2, 3 of the second.
-  const int vh = g >> 1;
-  const bool v_ok = vh ? cr.ok[1] : cr.ok[0];
-  const bf16* vp = kv.v + ((vh ? base[1] : base[0]) * HD + r) * kv.page_size + (vh ? off[1] : off[0]) + 8 * (g & 1);
-  // STREAM_V (pages of at most 32 keys): the 16 rows of a load are whole cache lines, and
-  // these lines, read once, go past the caches. Halves of lines would come from memory twice.
+    for (int c = 0; c < HD / 32; ++c) cr.k[t][c] = at.k_ok ? load_b128(at.k + 4 * t * HD + 32 * c) : zero_b128();
+}
+// STREAM_V (pages of at most 32 keys): the 16 rows of a load are whole cache lines, and
+// these lines, read once, go past the caches. Halves of lines would come from memory twice.
+template <int HD, bool STREAM_V>
+__device__ inline void load_values(const ChunkPlace& at, int page_size, ChunkRegs<HD>& cr) {
 #pragma unroll
   for (int dt = 0; dt < HD / 16; ++dt) {
-    const bf16* p = vp + static_cast<size_t>(dt) * 16 * kv.page_size;
-    cr.v[dt] = !v_ok ? zero_b128() : STREAM_V ? load_b128_stream(p) : load_b128(p);
+    const bf16* p = at.v + static_cast<size_t>(dt) * 16 * page_size;
+    cr.v[dt] = !at.v_ok ? zero_b128() : STREAM_V ? load_b128_stream(p) : load_b128(p);
   }
 }
+template <int HD, bool STREAM_V>
+__device__ inline void load_chunk(const KV& kv, TableWindow& tw, int key0, ChunkRegs<HD>& cr) {
+  const ChunkPlace at = place_chunk<HD>(kv, tw, key0);
+  cr.ok[0] = at.ok[0], cr.ok[1] = at.ok[1];
+  load_keys<HD>(at, cr);
+  load_values<HD, STREAM_V>(at, kv.page_size, cr);
+}
 
-template <int HD, int CT>
+template <int HD, int CT, typename Scored>
 __device__ inline void attend_regs(const ChunkRegs<HD>& cr, int key0, bool edge, const Bounds<CT>& bd,
                                    float scale_log2, const bf16x8 (&q)[CT][HD / 32],
-                                   f32x4 (&o)[HD / 16][CT], float (&m)[CT], float (&l)[CT]) {
+                                   f32x4 (&o)[HD / 16][CT], float (&m)[CT], float (&l)[CT], Scored&& scored) {
   const bool ok[2] = {cr.ok[0], cr.ok[1]};
   attend_core<HD, CT, true>(
       key0, edge, ok, bd, scale_log2, q, o, m, l, [&](int t, int c) { return cr.k[t][c]; },
-      [&](int dt) { return cr.v[dt]; });
+      [&](int dt) { return cr.v[dt]; }, scored);
 }
 
 // ---------------------------------------------------------------------------
@@ -351,11 +377,17 @@ struct RopeIn {
   q, k_cache, v_cache, work, positions, seq_of_token, block_table, table_stride, part_acc, part_ml, counters, out, \
       nq, nkv, page_size, scale_log2, window
 
-template <int HD, bool STREAM_V, bool FUSED>
+template <int HD, bool STREAM_V, bool FUSED, bool ONE>
 __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, const RopeIn& rope) {
-  const int4 head_of_list = work[0];
+  // The list's head and this block's row of it (the list holds one for every block of the launch) come together.
+  const int4 head_of_list = work[0], item = work[2 * (1 + blockIdx.y)], place = work[2 * (1 + blockIdx.y) + 1];
+  // (The product's arguments with them: where they are first used they would be a trip of their own.)
+  if constexpr (FUSED)
+    asm volatile("" ::"s"(head_of_list.x), "s"(item.x), "s"(place.x), "s"(rope.qkv), "s"(rope.n_partials), "s"(rope.partial_stride), "s"(rope.bias),
+                 "s"(rope.cos_t), "s"(rope.sin_t), "s"(rope.write_kv), "s"(block_table), "s"(table_stride), "s"(nq), "s"(page_size), "s"(window));
+  else
+    asm volatile("" ::"s"(head_of_list.x), "s"(item.x), "s"(place.x));
   if (static_cast<int>(blockIdx.y) >= head_of_list.x) return;
-  const int4 item = work[2 * (1 + blockIdx.y)], place = work[2 * (1 + blockIdx.y) + 1];
   const int tok = item.x, b = item.y & 0xffff, nb = item.y >> 16, per = item.z, slot0 = item.w;
   // a list that does not fit the launch is not followed
   if (nb < 1 || nb > kMaxBlocksPerRequest || b < 0 || b >= nb || slot0 < 0 || slot0 + nb > static_cast<int>(gridDim.y) || per < 1)
@@ -370,7 +402,7 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
   const int pos = place.x;
   const int lo = window > 0 ? max(0, pos - window + 1) : 0;
 
-  KV kv{k_cache, v_cache, block_table + static_cast<size_t>(place.y) * table_stride, nkv, kvh, page_size};
+  KV kv{k_cache, v_cache, block_table + static_cast<size_t>(place.y) * table_stride, nkv, kvh, page_size, shift_of(page_size)};
   Bounds<1> bd{{lo}, {pos}};
 
   const int first = lo / kChunk, last = pos / kChunk;
@@ -392,91 +424,113 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
     // starts with both on their way.
     ChunkRegs<HD> ra, rb;
     // No entry beyond those of the chunks up to `last` is read.
-    TableWindow tw{kv.table, min(table_stride, (last * kChunk + 16) / page_size + 1), 0, -1};
-    if (begin < end) tw.fill(begin * kChunk / page_size);
+    TableWindow tw{kv.table, min(table_stride, kv.entry(last * kChunk + 16) + 1), 0, -1};
+    if (begin < end) tw.fill(kv.entry(begin * kChunk));
     // FUSED: of the waves that attend for a token and key/value head (the first group of query heads
     // only), the one whose chunks hold the token's own position writes its key and value; it does not read
     // them back but puts them into that chunk's registers (see own_key).
     const bool may_write = FUSED && qt == 0 && rope.write_kv && begin <= last && last < end;
     bool writes = false;
-    const bool ask_a = begin < end, ask_b = begin + 1 < end;
+    const bool ask_a = begin < end, ask_b = !ONE && begin + 1 < end;
     __shared__ __attribute__((aligned(16))) bf16 own_s[2][FUSED ? HD : 8];
     if constexpr (FUSED) {
-      constexpr int half = HD / 2;
+      constexpr int half = HD / 2, kItems = HD / 8;  // items of a head: four pairs each
       const int width = (nq + 2 * nkv) * HD;
       const float* row = rope.qkv + static_cast<size_t>(tok) * width;
-      auto value4 = [&](int col) {  // the product's sum with its bias, four columns from `col` (a multiple of 4) on
-        float4 v = sum_partials4<float>(row + col, static_cast<size_t>(rope.partial_stride), rope.n_partials);
-        if (rope.bias)
-          v = add4(v, rope.bias_dt == kF32 ? Vec4<float>::load(static_cast<const float*>(rope.bias) + col)
-                                           : Vec4<bf16>::load(static_cast<const bf16*>(rope.bias) + col));
-        return v;
+      // An item is four elements from `col` on and the four half a head further on: of this block's queries, then (in the block that
+      // holds the token's own position) of its key and of its value. All that a thread loads of the product is asked for first, the
+      // chunks' keys and values behind it, and nothing is waited for in between but the block table; then comes the arithmetic
+      // of rope_kv_write. (With sums made as their loads came, each of them a trip through memory before the chunks' loads, a block
+      // of its own had those on their way 4.6 us after its start, now 3.1.)
+      const bool own = qt == 0 && rope.write_kv && first + 4 * b * per <= last && last < first + 4 * (b + 1) * per;
+      const int items = kItems * (own ? nheads + 2 : nheads), n_parts = rope.n_partials;
+      constexpr int kTogether = 8;
+      struct Item {
+        float4 x[2][kTogether], c4, s4;
+        uint4 bias[2];
+        int col;
       };
-      // elements j..j+3 and half + j.. of the head at `base`: what is loaded, and the rotation of it
-      struct Pairs { float4 x1, x2, c4, s4; };
-      auto pairs_of = [&](int base, int j) {
+      auto ask_item = [&](int it, Item& x) {
+        const int h = it / kItems, j = 4 * (it % kItems);
+        x.col = (h < nheads ? head0 + h : (h == nheads ? nq : nq + nkv) + kvh) * HD + j;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int p = 0; p < kTogether; ++p)  // (parts that are not there: the last one again)
+            x.x[e][p] = Vec4<float>::load(row + x.col + e * half + static_cast<size_t>(min(p, n_parts - 1)) * rope.partial_stride);
         const size_t t = static_cast<size_t>(pos) * half + j;
-        return Pairs{value4(base + j), value4(base + j + half), Vec4<float>::load(rope.cos_t + t), Vec4<float>::load(rope.sin_t + t)};
+        x.c4 = Vec4<float>::load(rope.cos_t + t), x.s4 = Vec4<float>::load(rope.sin_t + t);
+        if (rope.bias) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            if (rope.bias_dt == kF32) {
+              x.bias[e] = *reinterpret_cast<const uint4*>(static_cast<const float*>(rope.bias) + x.col + e * half);
+            } else {
+              const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const bf16*>(rope.bias) + x.col + e * half);
+              x.bias[e].x = u.x, x.bias[e].y = u.y;
+            }
+          }
+        }
       };
-      auto rotate = [&](const Pairs& p, float4& a4, float4& b4) {
-        rotate_pair(p.x1.x, p.x2.x, p.c4.x, p.s4.x, a4.x, b4.x);
-        rotate_pair(p.x1.y, p.x2.y, p.c4.y, p.s4.y, a4.y, b4.y);
-        rotate_pair(p.x1.z, p.x2.z, p.c4.z, p.s4.z, a4.z, b4.z);
-        rotate_pair(p.x1.w, p.x2.w, p.c4.w, p.s4.w, a4.w, b4.w);
+      // the queries of this block's heads and the token's own key and value, rounded to bfloat16 as rope_kv_write stores them
+      __shared__ __attribute__((aligned(16))) bf16 q_s[16][HD + 8];
+      auto finish_item = [&](int it, const Item& x) {
+        float4 v[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          v[e] = x.x[e][0];
+#pragma unroll
+          for (int p = 1; p < kTogether; ++p)
+            if (p < n_parts) v[e] = add4(v[e], x.x[e][p]);
+          for (int p = kTogether; p < n_parts; ++p)
+            v[e] = add4(v[e], Vec4<float>::load(row + x.col + e * half + static_cast<size_t>(p) * rope.partial_stride));
+          if (rope.bias) {
+            const uint4 u = x.bias[e];
+            v[e] = add4(v[e], rope.bias_dt == kF32 ? float4{__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)}
+                                                   : float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u),
+                                                            __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u)});
+          }
+        }
+        const int h = it / kItems, j = 4 * (it % kItems);
+        float4 a4 = v[0], b4 = v[1];
+        if (h <= nheads) {
+          rotate_pair(v[0].x, v[1].x, x.c4.x, x.s4.x, a4.x, b4.x);
+          rotate_pair(v[0].y, v[1].y, x.c4.y, x.s4.y, a4.y, b4.y);
+          rotate_pair(v[0].z, v[1].z, x.c4.z, x.s4.z, a4.z, b4.z);
+          rotate_pair(v[0].w, v[1].w, x.c4.w, x.s4.w, a4.w, b4.w);
+        }
+        bf16* const dst = h < nheads ? &q_s[h][j] : &own_s[h - nheads][j];
+        Vec4<bf16>::store(dst, a4);
+        Vec4<bf16>::store(dst + half, b4);
       };
-      // First everything this thread has to load of the product: four pairs of a query (thread it of the
-      // block: head it / (HD / 8)), and in the wave that may write, four pairs of the key (lanes
-      // 0 .. HD / 8 - 1) or four elements of the value (the next HD / 4 lanes). Then the chunks' loads, which
-      // queue behind them; then the arithmetic of rope_kv_write.
       const int it = threadIdx.x;
-      const bool q_item = it < nheads * (HD / 8);
-      const bool key_lane = may_write && lane < HD / 8, value_lane = may_write && lane >= HD / 8 && lane < HD / 8 + HD / 4;
-      const float4 zero4 = {0.f, 0.f, 0.f, 0.f};
-      Pairs qp{zero4, zero4, zero4, zero4}, kp = qp;
-      float4 vv = zero4;
-      if (q_item) qp = pairs_of((head0 + it / (HD / 8)) * HD, 4 * (it % (HD / 8)));
-      if (key_lane) kp = pairs_of((nq + kvh) * HD, 4 * lane);
-      if (value_lane) vv = value4((nq + nkv + kvh) * HD + 4 * (lane - HD / 8));
-      const int slot = may_write ? rope.slots[tok] : -1;
+      Item item;
+      if (it < items) ask_item(it, item);
       if (ask_a) load_chunk<HD, STREAM_V>(kv, tw, begin * kChunk, ra);
       if (ask_b) load_chunk<HD, STREAM_V>(kv, tw, (begin + 1) * kChunk, rb);
-      // the queries of this block's heads, rounded to bfloat16 as rope_kv_write stores them
-      __shared__ __attribute__((aligned(16))) bf16 q_s[16][HD + 8];
-      static_assert(16 * (HD / 8) <= 256, "one item of the queries per thread");
-      if (q_item) {
-        float4 a4, b4;
-        rotate(qp, a4, b4);
-        const int h = it / (HD / 8), j = 4 * (it % (HD / 8));
-        Vec4<bf16>::store(&q_s[h][j], a4);
-        Vec4<bf16>::store(&q_s[h][j + half], b4);
-      }
-      // the token's own key and value, rounded likewise
-      float4 ka = zero4, kb = zero4;
-      if (key_lane) {
-        rotate(kp, ka, kb);
-        Vec4<bf16>::store(&own_s[0][4 * lane], ka);
-        Vec4<bf16>::store(&own_s[0][4 * lane + half], kb);
-      } else if (value_lane) {
-        Vec4<bf16>::store(&own_s[1][4 * (lane - HD / 8)], vv);
+      if (it < items) finish_item(it, item);
+      if (it + 256 < items) {  // 15 or 16 query heads of 128 elements, in the block with the token's own position
+        ask_item(it + 256, item);
+        finish_item(it + 256, item);
       }
       lds_barrier();  // waits for LDS alone: the chunks' loads stay on their way
 #pragma unroll
       for (int c = 0; c < HD / 32; ++c) qr[0][c] = r < nheads ? load_b128(&q_s[r][32 * c + 8 * g]) : zero_b128();
+      const int slot = may_write ? rope.slots[tok] : -1;
       writes = may_write && slot >= 0;
       if (writes) {
         const int page = slot / page_size, off = slot % page_size;
-        if (key_lane) {
-          bf16* dst = k_cache + ((static_cast<size_t>(page) * nkv + kvh) * page_size + off) * HD + 4 * lane;
-          Vec4<bf16>::store(dst, ka);
-          Vec4<bf16>::store(dst + half, kb);
-        } else if (value_lane) {
-          bf16* vrow = v_cache + ((static_cast<size_t>(page) * nkv + kvh) * HD + 4 * (lane - HD / 8)) * page_size;
-          const float vals[4] = {vv.x, vv.y, vv.z, vv.w};
+        if (lane < HD / 8) {
+          *reinterpret_cast<uint4*>(k_cache + ((static_cast<size_t>(page) * nkv + kvh) * page_size + off) * HD + 8 * lane) =
+              *reinterpret_cast<const uint4*>(&own_s[0][8 * lane]);
+        } else if (lane < HD / 8 + HD / 4) {
+          const int d = 4 * (lane - HD / 8);
+          bf16* vrow = v_cache + ((static_cast<size_t>(page) * nkv + kvh) * HD + d) * page_size;
           const bool ends = ends_its_page_run(rope.slots, tok, rope.n_rows, slot, page_size);
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             bf16* one = vrow + u * static_cast<size_t>(page_size);
-            one[off] = from_float<bf16>(vals[u]);
+            one[off] = own_s[1][d + u];
             // the step's last token of a page leaves nothing of the page's previous owner behind it
             if (ends) zero_tail(one, off + 1, page_size);
           }
@@ -516,13 +570,32 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
         cr.v[dt] = __builtin_bit_cast(bf16x8, u);
       }
     };
+    if constexpr (ONE) {
+      // One register set: the next chunk's keys are asked for when these are multiplied, its values when those are.
+      for (int c = begin; c < end; ++c) {
+        own_key(c, ra);
+        ChunkPlace next;
+        const bool more = c + 1 < end;
+        attend_regs<HD, 1>(ra, c * kChunk, c == first || c == last, bd, scale_log2, qr, o, m, l, [&] {
+          if (more) {
+            next = place_chunk<HD>(kv, tw, (c + 1) * kChunk);
+            load_keys<HD>(next, ra);
+          }
+        });
+        if (more) {
+          ra.ok[0] = next.ok[0], ra.ok[1] = next.ok[1];
+          load_values<HD, STREAM_V>(next, kv.page_size, ra);
+        }
+      }
+    } else
     for (int c = begin; c < end; c += 2) {
+      const auto nothing = [] {};
       own_key(c, ra);
-      attend_regs<HD, 1>(ra, c * kChunk, c == first || c == last, bd, scale_log2, qr, o, m, l);
+      attend_regs<HD, 1>(ra, c * kChunk, c == first || c == last, bd, scale_log2, qr, o, m, l, nothing);
       if (c + 2 < end) load_chunk<HD, STREAM_V>(kv, tw, (c + 2) * kChunk, ra);
       if (c + 1 < end) {
         own_key(c + 1, rb);
-        attend_regs<HD, 1>(rb, (c + 1) * kChunk, c + 1 == first || c + 1 == last, bd, scale_log2, qr, o, m, l);
+        attend_regs<HD, 1>(rb, (c + 1) * kChunk, c + 1 == first || c + 1 == last, bd, scale_log2, qr, o, m, l, nothing);
         if (c + 3 < end) load_chunk<HD, STREAM_V>(kv, tw, (c + 3) * kChunk, rb);
       }
     }
@@ -629,21 +702,24 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
 template <int HD, bool STREAM_V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_decode_work_alone_kernel(
     PYRE_DECODE_WORK_PARAMS) {
-  attn_decode_work_block<HD, STREAM_V, false>(PYRE_DECODE_WORK_ARGS, RopeIn{});
+  attn_decode_work_block<HD, STREAM_V, false, false>(PYRE_DECODE_WORK_ARGS, RopeIn{});
 }
 template <int HD, bool STREAM_V>
 __global__ __launch_bounds__(256, 2) void attn_decode_work_kernel(PYRE_DECODE_WORK_PARAMS) {
-  attn_decode_work_block<HD, STREAM_V, false>(PYRE_DECODE_WORK_ARGS, RopeIn{});
+  attn_decode_work_block<HD, STREAM_V, false, false>(PYRE_DECODE_WORK_ARGS, RopeIn{});
 }
-// The same two forms, finishing the q/k/v product themselves (heads of up to 128 elements).
+// The same two forms, finishing the q/k/v product themselves (heads of up to 128 elements). Where blocks share a unit there are three,
+// of one register set each (ONE), since those that do not start at once start when others end: 190 requests of 94 to 1,501 tokens
+// on the 1.5B heads are 594 blocks, of which 82 started after 17 us and ended after 31; all at once they end after 26 (31.9 us a
+// launch, now 29.4). A unit's loads on their way are what bounds them, not the sets that a wave keeps.
 template <int HD, bool STREAM_V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_decode_work_rope_alone_kernel(
     PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
-  attn_decode_work_block<HD, STREAM_V, true>(PYRE_DECODE_WORK_ARGS, rope);
+  attn_decode_work_block<HD, STREAM_V, true, false>(PYRE_DECODE_WORK_ARGS, rope);
 }
 template <int HD, bool STREAM_V>
-__global__ __launch_bounds__(256, 2) void attn_decode_work_rope_kernel(PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
-  attn_decode_work_block<HD, STREAM_V, true>(PYRE_DECODE_WORK_ARGS, rope);
+__global__ __launch_bounds__(256, 3) void attn_decode_work_rope_kernel(PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
+  attn_decode_work_block<HD, STREAM_V, true, true>(PYRE_DECODE_WORK_ARGS, rope);
 }
 #undef PYRE_DECODE_WORK_PARAMS
 #undef PYRE_DECODE_WORK_ARGS

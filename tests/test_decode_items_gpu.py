@@ -1,0 +1,16 @@
+"""The decode kernel that finishes the q/k/v product: more items of queries, key and value than a block has threads (15 and 16 query
+heads of 128 elements with the token's own position), and as many parts of the product as are asked for together, one more, and the
+most there are. The same bits as the kernels it stands for."""
+
+from __future__ import annotations
+
+import pytest
+from test_kernels_gpu import test_attn_decode_finishes_the_qkv_product_itself as check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nq,nkv", [(15, 1), (32, 2), (14, 1)])
+@pytest.mark.parametrize("ks,bias,alone", [(8, True, True), (9, False, False), (12, True, False)])
+def test_items_and_parts(nq, nkv, ks, bias, alone):
+    check(nq, nkv, 128, 16, ks, bias, 0, None, alone)
