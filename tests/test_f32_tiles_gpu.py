@@ -70,6 +70,38 @@ def test_attention_of_prompts(hd, page, window):
         assert float((out[:, h].double() - want).abs().max()) <= 2e-5
 
 
+@pytest.mark.parametrize("first,n", [(0, 1), (0, 15), (0, 16), (0, 17), (31, 1), (96, 33), (127, 2), (128, 16), (120, 49), (300, 31)])
+@pytest.mark.parametrize("nq,nkv,hd,page,window", [(5, 1, 128, 16, 0), (6, 2, 128, 16, 40), (3, 3, 160, 8, 0), (4, 2, 256, 16, 70),
+                                                   (3, 1, 30, 16, 40)])
+def test_prompts_at_the_edges_of_tokens_and_rounds(first, n, nq, nkv, hd, page, window):
+    """Blocks of sixteen tokens and rounds of two or four chunks of keys, one head and two to a block; pages that lie wholly
+    behind the window are gone from the table, and what they held is not a number."""
+    from pyre_amd.hip import ops
+
+    T = first + n
+    pages = -(-T // page)
+    k, v, q = rnd(T, nkv, hd, seed=1), rnd(T, nkv, hd, seed=2), rnd(n, nq, hd, seed=3)
+    kc = torch.full((pages, nkv, page, hd), float("nan"), device=DEV)
+    vc = torch.full((pages, nkv, hd, page), float("nan"), device=DEV)
+    for t in range(T):
+        kc[t // page, :, t % page] = k[t]
+        vc[t // page, :, :, t % page] = v[t]
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None].clone()
+    out_of_sight = (max(0, first - window + 1) // 32 * 32) // page if window else 0
+    table[0, :out_of_sight] = -1
+    kc[:out_of_sight], vc[:out_of_sight] = float("nan"), float("nan")
+    pos, seq = torch.arange(first, T, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+    tiles = torch.tensor([[t, min(32, n - t)] for t in range(0, n, 32)], dtype=torch.int32, device=DEV)
+    out = torch.full((n, nq, hd), float("nan"), device=DEV)
+    ops.attn_prefill_f32(q, out, kc, vc, tiles, len(tiles), pos, seq, table, nq, nkv, hd, page, hd ** -0.5, window)
+    i, j = torch.arange(first, T, device=DEV)[:, None], torch.arange(T, device=DEV)[None]
+    hidden = (j > i) | ((i - j >= window) if window else torch.zeros_like(j > i))
+    for h in range(nq):
+        s = (q[:, h].double() @ k[:, h * nkv // nq].double().T * hd ** -0.5).masked_fill(hidden, float("-inf"))
+        want = torch.softmax(s, 1) @ v[:, h * nkv // nq].double()
+        assert float((out[:, h].double() - want).abs().max()) <= 2e-5
+
+
 @pytest.mark.parametrize("hd,page", [(64, 16), (128, 8), (36, 4), (30, 16), (64, 6)])
 def test_keys_without_a_page_are_not_seen(hd, page):
     """An entry of -1 in the block table, and a table that ends before the step's keys do: in both forms, as in the kernels of
