@@ -20,6 +20,8 @@
 // attn_biased_tile    prompt portions: tiles of up to 32 consecutive tokens of a request, four query
 //                 heads of a key/value head per block, chunks of 32 keys through LDS, both products on
 //                 the matrix cores' float32 instruction (scores and weights stay float32).
+// attn_biased_tile16, attn_biased_tile32   the same for bfloat16 and float32 where head sizes are multiples of eight and
+//                 rows start on 16 bytes.
 // attn_biased_single  single tokens: a block per (token, up to eight query heads of a key/value head), the keys in
 //                 spans of 128 that the block's heads read together; in bfloat16 on the matrix cores, up to sixteen heads a
 //                 block, a wave per 32 keys of a span.
@@ -181,7 +183,7 @@ __device__ inline float shaped_score(float raw, float scale, float cap, const fl
 // the transposed problem, S^T[key, token] and O^T[d, token], so that a lane's sixteen scores are
 // the operands of the second product as they are.
 // VEC: both head sizes are multiples of eight and the caches start on 16 bytes, so that keys and
-// values come eight elements to a load.
+// values come eight elements to a load (bfloat16 with pages whose size is not a power of two).
 template <typename T, int NV, bool VEC>
 __global__ __launch_bounds__(kThreads) void attn_biased_tile_kernel(
     const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache, T* __restrict__ out,
@@ -397,6 +399,256 @@ __global__ __launch_bounds__(kThreads) void attn_biased_tile_kernel(
       const int d = 32 * dt + 8 * (i >> 2) + 4 * h + (i & 3);
       if (d < dv) dst[d] = from_float<T>(o[dt][i] * (gate_dim > 1 && gate ? f * grow[d] : f));
     }
+}
+
+// The same for float32 where heads are multiples of eight and rows start on 16 bytes, laid out as attention_f32_mfma.hip's: a block
+// takes sixteen tokens and two heads, on 16 x 16 x 4; of every KS chunks of 32 keys, which lie in LDS together, a
+// wave of a head takes one, by the chunk's number, and the parts are joined at the end in their order. DKP and 32 NV: the
+// head sizes padded with zeros.
+// With 32 tokens and four heads a block, a wave a head, 600 tokens of six heads were 38 blocks of four waves, each a chain of up to 19
+// chunks of 11 us whose loads waited for one another behind branches. Us a launch, biases of 1,025 distances and a cap,
+// before and now: 600 tokens of six heads of 128 205 and 53, of fourteen 209 and 66, 150 behind 600 258 and 60, sixteen 22 and 16,
+// 2,048 of 28 heads 1,354 and 786, 2,048 behind 4,000 of fourteen 1,950 and 1,410 (without biases), with a window of 1,024 378 and 359;
+// 700 of eight heads of 64 164 and 54, of 96 / 256 348 and 94. The distance from 64 bits is smaller in all of them (5.1e-7 and
+// 4.7e-7 for the first, 14.1e-7 and 8.9e-7 behind 4,000 tokens).
+template <int DKP, int NV, int KS>
+struct Tile32 {
+  static constexpr int HEADS = 2, TOKENS = 16, THREADS = 64 * HEADS * KS, KEYS = kKeys * KS, DVP = 32 * NV;
+  static constexpr int KROW = DKP + 4, VROW = kKeys + 4, KSIZE = KEYS * KROW, VSIZE = KS * DVP * VROW;
+  static constexpr int JOIN = HEADS * KS * TOKENS;  // rows that are joined: DVP + 4 sums (sixteen bytes), a maximum and a sum of weights
+  static_assert(JOIN * (DVP + 4 + 2) <= KSIZE + VSIZE, "what is joined lies where the keys and values lay");
+  static constexpr size_t LDS = sizeof(float) * (KSIZE + VSIZE) + 3 * KEYS * (sizeof(longlong2) + sizeof(int));
+};
+template <int DKP, int NV, int KS>
+__global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
+    const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache, float* __restrict__ out,
+    int out_ld, const float* __restrict__ gate, float out_scale, const int* __restrict__ tiles,
+    const int* __restrict__ positions, const int* __restrict__ seq_of_token, const int* __restrict__ block_table,
+    int table_stride, int nq, int nkv, int dk, int dv, int page_size, float scale, float cap, const float* __restrict__ bias,
+    int far, int window, int keep_first, int chunk, int bias_lds, const float* __restrict__ sink, int gate_dim) {
+  using Shape = Tile32<DKP, NV, KS>;
+  constexpr int HEADS = Shape::HEADS, TOKENS = Shape::TOKENS, THREADS = Shape::THREADS, KEYS = Shape::KEYS, DVP = Shape::DVP;
+  constexpr int KROW = Shape::KROW, VROW = Shape::VROW, OROW = DVP + 4;
+  typedef f32x4 f32x4_anywhere __attribute__((aligned(4)));
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* const Ks = lds;                     // [key][d]
+  float* const Vt = Ks + Shape::KSIZE;       // [part][d][key of the chunk]
+  longlong2* const where = reinterpret_cast<longlong2*>(Vt + Shape::VSIZE);  // of three rounds' keys: where key and value start
+  int* const pages = reinterpret_cast<int*>(where + 3 * KEYS);               // and their pages; -1: not there
+  float* const bias_s = reinterpret_cast<float*>(pages + 3 * KEYS);          // [HEADS][far + 1], if they fit
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int n_rep = nq / nkv, kvh = blockIdx.z, part = wave / HEADS, hin = blockIdx.y * HEADS + wave % HEADS;
+  const bool active = hin < n_rep;  // a wave without a head still helps loading
+  const int head = kvh * n_rep + (active ? hin : 0);
+  const int half_tile = gridDim.x - 1 - blockIdx.x;  // the last tokens, which see the most keys, first
+  const int t0 = tiles[half_tile & ~1] + TOKENS * (half_tile & 1);
+  const int ntok = min(TOKENS, tiles[half_tile | 1] - TOKENS * (half_tile & 1));
+  if (ntok <= 0) return;
+  const int pos0 = positions[t0];
+  const int* table = block_table + static_cast<size_t>(seq_of_token[t0]) * table_stride;
+
+  const bool live = active && c < ntok;
+  const int hi = c < ntok ? pos0 + c : pos0;
+  const int lo = first_seen(hi, window, chunk);
+  const int keep = window > 0 ? keep_first : 0;
+  const float* const bias_row = bias ? bias + static_cast<size_t>(head) * (far + 1) : nullptr;
+  if (bias && bias_lds && part == 0)
+    for (int i = lane; i <= far; i += 64) bias_s[wave * (far + 1) + i] = bias_row[i];
+  const float* const bias_near = bias_s + wave % HEADS * (far + 1);
+  f32x4 qr[DKP / 16];  // element 16 s + 4 g + j of the query of token c
+#pragma unroll
+  for (int s = 0; s < DKP / 16; ++s) {
+    const int d = 16 * s + 4 * g;
+    qr[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (live && d < dk) qr[s] = *reinterpret_cast<const f32x4*>(q + (static_cast<size_t>(t0 + c) * nq + head) * dk + d);
+  }
+  f32x4 o[DVP / 16];
+#pragma unroll
+  for (int dt = 0; dt < DVP / 16; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+
+  // Rounds are KS chunks with neighbouring numbers from a multiple of KS on: those of the kept first tokens, then those of the window.
+  const int lo_all = first_seen(pos0, window, chunk);  // rises with the position: the tile's first token sees furthest back
+  const int hi_all = pos0 + ntok - 1;
+  const int kept_end = min(keep, lo_all);  // keys 0 .. kept_end - 1 lie before every window
+  const int n_first = kept_end > 0 ? (kept_end - 1) / kKeys + 1 : 0;
+  const int chunk_b = max(lo_all / kKeys, n_first), last_chunk = hi_all / kKeys;
+  const int rounds_first = (n_first + KS - 1) / KS, round_b = max(chunk_b / KS, rounds_first);
+  const int n_rounds = rounds_first + max(0, last_chunk / KS - round_b + 1);
+  auto round_of = [&](int it) { return it < rounds_first ? it : round_b + (it - rounds_first); };
+  auto needed = [&](int ch) { return ch < n_first || (ch >= chunk_b && ch <= last_chunk); };
+  auto look_up = [&](int it) {  // the page of key tid of a round
+    const int key = KEYS * round_of(it) + tid, entry = key / page_size;
+    return it < n_rounds && tid < KEYS && key <= hi_all && needed(key / kKeys) && entry < table_stride ? table[entry] : -1;
+  };
+  auto note = [&](int it, int to, int page) {
+    if (tid >= KEYS) return;
+    const int at = (KEYS * round_of(it) + tid) % page_size;
+    const long long row = (static_cast<long long>(page) * nkv + kvh) * page_size + at;
+    pages[to * KEYS + tid] = page;
+    where[to * KEYS + tid] = page >= 0 ? longlong2{row * dk, row * dv} : longlong2{-1, -1};
+  };
+  // Loads without a branch: a piece that is not there is read from the queries and becomes zeros when it is stored in LDS. Values
+  // come as squares of four keys and four elements, which a thread turns over.
+  constexpr int KP = DKP / 16, VB = (NV + 1) / 2, SQUARES = KS * 8 * (DVP / 4);
+  f32x4 kp[KP], vp[VB][4];
+  unsigned kgone = 0, vgone = 0;
+  auto fetch = [&](int from) {
+    kgone = vgone = 0;
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+      const int key = (tid + THREADS * i) / (DKP / 4), d = 4 * ((tid + THREADS * i) % (DKP / 4));
+      const long long at = where[from * KEYS + key].x;
+      const bool there = at >= 0 && d < dk;
+      kp[i] = *reinterpret_cast<const f32x4*>(there ? k_cache + at + d : q);
+      kgone |= there ? 0u : 1u << i;
+    }
+#pragma unroll
+    for (int i = 0; i < VB; ++i) {
+      const int b = min(tid + THREADS * i, SQUARES - 1), d = 4 * (b / 8 % (DVP / 4)), key = kKeys * (b / 8 / (DVP / 4)) + 4 * (b % 8);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const long long at = where[from * KEYS + key + j].y;
+        const bool there = at >= 0 && d < dv;
+        vp[i][j] = *reinterpret_cast<const f32x4*>(there ? v_cache + at + d : q);
+        vgone |= there ? 0u : 1u << (4 * i + j);
+      }
+    }
+  };
+  auto put = [&]() {
+    if (__ballot(kgone | vgone)) {
+#pragma unroll
+      for (int i = 0; i < KP; ++i)
+        if (kgone >> i & 1) kp[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4 * VB; ++i)
+        if (vgone >> i & 1) vp[i / 4][i % 4] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < KP; ++i) {
+      const int key = (tid + THREADS * i) / (DKP / 4), d = 4 * ((tid + THREADS * i) % (DKP / 4));
+      *reinterpret_cast<f32x4*>(Ks + key * KROW + d) = kp[i];
+    }
+#pragma unroll
+    for (int i = 0; i < VB; ++i) {
+      const int b = tid + THREADS * i, row = b / 8 / (DVP / 4) * DVP + 4 * (b / 8 % (DVP / 4));
+      if (b < SQUARES)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          *reinterpret_cast<f32x4*>(Vt + (row + u) * VROW + 4 * (b % 8)) = f32x4{vp[i][0][u], vp[i][1][u], vp[i][2][u], vp[i][3][u]};
+    }
+  };
+  const int page0 = look_up(0), page1 = look_up(1);
+  int ahead = look_up(2);
+  note(0, 0, page0);
+  note(1, 1, page1);
+  __syncthreads();
+  fetch(0);
+  int slot = 0;
+  for (int it = 0; it < n_rounds; ++it) {
+    const int next = slot == 2 ? 0 : slot + 1, here = slot * KEYS + kKeys * part;
+    __syncthreads();  // the round before has been read by every wave
+    note(it + 2, next == 2 ? 0 : next + 1, ahead);
+    put();
+    __syncthreads();
+    if (it + 1 < n_rounds) fetch(next);
+    ahead = look_up(it + 3);
+    slot = next;
+    const int ch = KS * round_of(it) + part;
+    if (!active || !needed(ch)) continue;
+
+    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int st = 0; st < DKP / 16; ++st) {
+      f32x4 a[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) a[kt] = *reinterpret_cast<const f32x4*>(Ks + (kKeys * part + 16 * kt + c) * KROW + 16 * st + 4 * g);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kt][j], qr[st][j], s[kt], 0, 0, 0);
+    }
+    // element j of s[kt]: key 16 kt + 4 g + j of the chunk, token c
+    float bv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int dist = min(max(hi - (kKeys * ch + 16 * (i >> 2) + 4 * g + (i & 3)), 0), far);
+      bv[i] = !bias ? 0.f : bias_lds ? bias_near[dist] : bias_row[dist];
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int kk = 16 * (i >> 2) + 4 * g + (i & 3), key = kKeys * ch + kk;
+      const bool seen = key <= hi && (key >= lo || key < keep) && pages[here + kk] >= 0;
+      const float shaped = shaped_score(s[i >> 2][i & 3], scale, cap, nullptr, 0, 0) + bv[i];
+      s[i >> 2][i & 3] = seen ? shaped : -INFINITY;
+      mx = fmaxf(mx, s[i >> 2][i & 3]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m, mx);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expf(m - m_use);
+    m = m_new;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      s[i >> 2][i & 3] = expf(s[i >> 2][i & 3] - m_use);
+      sum += s[i >> 2][i & 3];
+    }
+    l = l * alpha + sum;
+#pragma unroll
+    for (int dt = 0; dt < DVP / 16; ++dt) o[dt] *= alpha;
+    constexpr int GROUP = DVP % 64 == 0 ? 4 : 2;  // tiles of d whose chains of products are in flight together
+#pragma unroll
+    for (int dt = 0; dt < DVP / 16; dt += GROUP)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        f32x4 a[GROUP];
+#pragma unroll
+        for (int t = 0; t < GROUP; ++t)
+          a[t] = *reinterpret_cast<const f32x4*>(Vt + (DVP * part + 16 * (dt + t) + c) * VROW + 16 * kt + 4 * g);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < GROUP; ++t) o[dt + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][j], s[kt][j], o[dt + t], 0, 0, 0);
+      }
+  }
+
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  float* const ml = lds + Shape::JOIN * OROW;  // [wave][token][2]
+  __syncthreads();
+#pragma unroll
+  for (int dt = 0; dt < DVP / 16; ++dt)  // element j of o[dt]: d = 16 dt + 4 g + j of token c
+    *reinterpret_cast<f32x4*>(lds + (TOKENS * wave + c) * OROW + 16 * dt + 4 * g) = o[dt];
+  if (g == 0) {
+    ml[2 * (TOKENS * wave + c)] = m;
+    ml[2 * (TOKENS * wave + c) + 1] = l;
+  }
+  __syncthreads();
+  for (int i = tid; i < HEADS * TOKENS * (DVP / 4); i += THREADS) {
+    const int d = 4 * (i % (DVP / 4)), row = i / (DVP / 4), token = row % TOKENS, which = row / TOKENS;
+    const int h = static_cast<int>(blockIdx.y) * HEADS + which;
+    if (d >= dv || token >= ntok || h >= n_rep) continue;
+    float most = -INFINITY, total = 0.f;
+#pragma unroll
+    for (int p = 0; p < KS; ++p) most = fmaxf(most, ml[2 * (TOKENS * (HEADS * p + which) + token)]);
+    f32x4 y{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < KS; ++p) {
+      const int at = TOKENS * (HEADS * p + which) + token;
+      const float weight = ml[2 * at] == -INFINITY ? 0.f : expf(ml[2 * at] - most);
+      total += weight * ml[2 * at + 1];
+      y += weight * *reinterpret_cast<const f32x4*>(lds + at * OROW + d);
+    }
+    float f = softmax_factor(most, total, sink, kvh * n_rep + h) * out_scale;
+    const float* grow = gate ? gate + (static_cast<size_t>(t0 + token) * nq + kvh * n_rep + h) * gate_dim : nullptr;
+    if (gate && gate_dim == 1) f *= grow[0];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] *= gate_dim > 1 && gate ? f * grow[d + j] : f;
+    *reinterpret_cast<f32x4_anywhere*>(out + static_cast<size_t>(t0 + token) * out_ld + (kvh * n_rep + h) * dv + d) = y;
+  }
 }
 
 // The tile kernel for bfloat16 queries and caches, on the matrix cores' 16-bit instruction with nothing rounded that
@@ -1184,6 +1436,44 @@ extern "C" int pyre_attn_biased_tile(const void* q, void* out, int out_ld, int d
   }
   const bool vec = dk % 8 == 0 && dv % 8 == 0 && reinterpret_cast<uintptr_t>(k_cache) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(v_cache) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
+  if (dt == kF32 && vec) {
+    const dim3 grid32(2 * n_tiles, (nq / nkv + 1) / 2, nkv);
+#define PYRE_TILE32(DKP, NV, KS)                                                                                          \
+  do {                                                                                                                    \
+    constexpr size_t plain = Tile32<DKP, NV, KS>::LDS;                                                                    \
+    const int near = bias && plain + sizeof(float) * 2 * (static_cast<size_t>(far) + 1) <= budget ? 1 : 0;               \
+    const size_t lds32 = plain + (near ? sizeof(float) * 2 * (far + 1) : 0);                                              \
+    static size_t raised = 64 * 1024;                                                                                     \
+    if (lds32 > raised) {                                                                                                 \
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_biased_tile32_kernel<DKP, NV, KS>),                     \
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds32)) != hipSuccess)         \
+        return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds32);                                      \
+      raised = lds32;                                                                                                     \
+    }                                                                                                                     \
+    hipLaunchKernelGGL((attn_biased_tile32_kernel<DKP, NV, KS>), grid32, dim3(128 * KS), lds32, stream,                   \
+                       static_cast<const float*>(q), static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), \
+                       static_cast<float*>(out), out_ld, gate, out_scale, tiles, positions, seq_of_token, block_table,    \
+                       table_stride, nq, nkv, dk, dv, page_size, scale, cap, bias, far, window, keep_first, chunk, near, \
+                       sink, gate_dim);                                                                                   \
+  } while (0)
+#define PYRE_TILE32_NV(DKP)                  \
+  switch (nvp) {                             \
+    case 1: PYRE_TILE32(DKP, 1, 4); break;   \
+    case 2: PYRE_TILE32(DKP, 2, 4); break;   \
+    case 4: PYRE_TILE32(DKP, 4, 4); break;   \
+    default: PYRE_TILE32(DKP, 8, 2); break;  \
+  }
+    // Waves a head by the head sizes alone, as far as LDS holds their chunks: a token's sums do not depend on the step.
+    switch (dkp / 32) {
+      case 1: PYRE_TILE32_NV(32); break;
+      case 2: PYRE_TILE32_NV(64); break;
+      case 3: PYRE_TILE32_NV(96); break;
+      default: PYRE_TILE32_NV(128); break;
+    }
+#undef PYRE_TILE32
+#undef PYRE_TILE32_NV
+    return check_launch("attn_biased_tile");
+  }
   const bool pow2_pages = (page_size & (page_size - 1)) == 0;
   if (dt == kBF16 && vec && pow2_pages) {  // the 16-bit instruction, scores and weights in 32 bits all the same
     const int ldk = dkp + kPad16, ldv = kKeys + kPad16;
@@ -1232,7 +1522,7 @@ extern "C" int pyre_attn_biased_tile(const void* q, void* out, int out_ld, int d
     return check_launch("attn_tile_join");
   }
   if (dt == kF32) {
-    if (vec) { PYRE_TILE_NV(float, true) } else { PYRE_TILE_NV(float, false) }
+    PYRE_TILE_NV(float, false)
   } else {
     if (vec) { PYRE_TILE_NV(bf16, true) } else { PYRE_TILE_NV(bf16, false) }
   }
