@@ -144,14 +144,25 @@ class LatentAttention(Mixer):
 
         def row_tiles(hb):  # the tiles of the other portions
             tiles = hb.arrays["attention.prefill_tiles"]
-            return tiles[~np.isin(hb.seq_of_token[tiles[:, 0]], hb.arrays[f"{plan}.tiles"][:, 3])]
+            made = np.zeros(hb.n_seqs, dtype=bool)
+            made[hb.arrays[f"{plan}.tiles"][:, 3]] = True
+            return tiles[~made[hb.seq_of_token[tiles[:, 0]]]]
+
+        def plain_tokens(hb):  # the range of tokens in which those lie whose attention runs over the rows themselves
+            singles, rows = hb.arrays["attention.decode_tokens"], hb.arrays[f"{plan}.row_tiles"]
+            if not len(hb.arrays[f"{plan}.tiles"]) or not (len(singles) or len(rows)):
+                return np.zeros(2, dtype=np.int32)
+            first = [int(x.min()) for x in (singles, rows[:, 0]) if len(x)]
+            last = [int(x.max()) + 1 for x in (singles, rows.sum(axis=1) - 1) if len(x)]
+            return np.asarray([min(first), max(last)], dtype=np.int32)
 
         return [*STEP_ARRAYS,
                 StepArraySpec(f"{plan}.groups", lambda n_cap, s_cap: 3 * (MOST_KEYS * n_cap // GROUP + 2 * s_cap), lambda hb: plan_groups(hb, spec)),
                 StepArraySpec(f"{plan}.tiles", lambda n_cap, s_cap: 5 * (n_cap // ops.LATENT_HEADS_TOKENS + s_cap),
                               lambda hb: plan_tiles(hb, spec)),
                 StepArraySpec(f"{plan}.rounds", lambda n_cap, s_cap: 2 * s_cap, lambda hb: plan_rounds(hb, spec)),
-                StepArraySpec(f"{plan}.row_tiles", STEP_ARRAYS[1].capacity, row_tiles)]
+                StepArraySpec(f"{plan}.row_tiles", STEP_ARRAYS[1].capacity, row_tiles),
+                StepArraySpec(f"{plan}.plain", lambda n_cap, s_cap: 2, plain_tokens)]  # once a step, not in every layer
 
     def linears(self) -> list:
         return [lin for lin in (self.inp, self.q_up, self.out) if lin is not None]
@@ -228,7 +239,7 @@ class LatentAttention(Mixer):
         made = 0
         if self.heads_up is not None and rows.numel() < 1 << 31:  # (a product's operand lies within 4 GiB)
             made = len(ctx.host.arrays[f"{self.plan_name}.tiles"])
-        a, b = self._plain_tokens(ctx.host, n) if made else (0, n)
+        a, b = ctx.host.arrays[f"{self.plan_name}.plain"].tolist() if made else (0, n)
         if b > a:
             ops.head_matmul(q[a:b], self.key_up, wide[a:b], b - a)
             o_in = ws.get("lattn.o_in", (n, heads, s.rank), ctx.dtype)
@@ -238,13 +249,6 @@ class LatentAttention(Mixer):
         if made:
             self._attend_made(ctx, q, wide[:, :, s.rank:], rows, o, cache, gate)
         return self.out.forward(ctx, o.view(n, self.o_dim), n)
-
-    def _plain_tokens(self, host, n: int) -> tuple[int, int]:
-        """The range of tokens in which those lie whose attention runs over the rows themselves."""
-        singles, tiles = host.arrays["attention.decode_tokens"], host.arrays[f"{self.plan_name}.row_tiles"]
-        first = [int(x.min()) for x in (singles, tiles[:, 0]) if len(x)]
-        last = [int(x.max()) + 1 for x in (singles, tiles.sum(axis=1) - 1) if len(x)]
-        return (min(first), max(last)) if first else (0, 0)
 
     def _attend_made(self, ctx, q, turned, rows, out, cache, gate) -> None:
         s, g0, t0 = self.spec, 0, 0
