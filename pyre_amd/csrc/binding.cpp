@@ -74,6 +74,14 @@ bool convert(PyObject* o, T& out) {
   return !PyErr_Occurred();
 }
 
+// The interpreter's lock, given up for the lifetime: an exception out of an entry takes it back too.
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 template <typename F>
 struct Entry;
 template <typename... A>
@@ -83,8 +91,10 @@ struct Entry<int (*)(A...)> {
     std::tuple<A...> v;
     if (!(convert(args[I], std::get<I>(v)) && ...)) return nullptr;
     int rc;
-    Py_BEGIN_ALLOW_THREADS rc = fn(std::get<I>(v)...);
-    Py_END_ALLOW_THREADS
+    {
+      Unlocked unlocked;
+      rc = fn(std::get<I>(v)...);
+    }
     if (rc == 0) Py_RETURN_NONE;
     raise(last_error());
     return nullptr;
@@ -95,7 +105,7 @@ struct Entry<int (*)(A...)> {
       return PyErr_Format(PyExc_TypeError, "%s takes %zu arguments, %zd given", name, sizeof...(A), n);
     try {
       return run(fn, args, std::index_sequence_for<A...>{});
-    } catch (const std::exception& e) {  // of torch, about a tensor without memory
+    } catch (const std::exception& e) {  // of torch, about a tensor without memory, or of the entry
       return PyErr_SetString(PyExc_RuntimeError, e.what()), nullptr;
     }
   }

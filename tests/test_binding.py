@@ -3,6 +3,13 @@ library's message. No kernel runs here."""
 
 from __future__ import annotations
 
+import re
+import shutil
+import subprocess
+import sys
+import textwrap
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -61,3 +68,41 @@ def test_entries():
         lib.call("pyre_gemm_mid_bf16", None, 64, None, 64, None, 1 << 40, 64, 64, 1, 0, 0)
     with pytest.raises(AttributeError):
         lib.call("pyre_no_such_entry")
+
+
+def test_an_exception_in_an_entry_is_an_error_of_the_call(tmp_path):
+    """A library whose entries throw (out of memory, say): the interpreter's lock is free while they run and held again when the
+    error is made. In a process of its own, since the library takes the kernels' place."""
+    compiler = shutil.which("g++")
+    if compiler is None:
+        pytest.skip("no C++ compiler")
+    from pyre_amd.hip import build
+
+    names = re.findall(r"X\((\w+)\)", (build.CSRC / "binding.cpp").read_text())
+    assert "gemm_mid_bf16" in names
+    source = tmp_path / "throws.cpp"
+    source.write_text("#include <new>\n" + 'extern "C" const char* pyre_last_error() { return ""; }\n' +
+                      "".join(f'extern "C" int pyre_{n}() {{ throw std::bad_alloc(); }}\n' for n in names))
+    lib_path = tmp_path / "libthrows.so"
+    subprocess.run([compiler, "-shared", "-fPIC", str(source), "-o", str(lib_path)], check=True)
+    code = textwrap.dedent(f"""
+        import threading
+        from pyre_amd.hip.native import binding
+        binding.open({str(lib_path)!r})
+        def once():
+            for _ in range(50):
+                try:
+                    binding.pyre_scale(None, 0, 1.0, None)
+                except RuntimeError as e:
+                    assert "bad_alloc" in str(e), e
+                else:
+                    raise SystemExit("no error")
+        others = [threading.Thread(target=once) for _ in range(3)]
+        [t.start() for t in others]
+        once()
+        [t.join() for t in others]
+        print("held")
+    """)
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
+                          cwd=Path(build.CSRC).parent.parent)
+    assert done.returncode == 0 and "held" in done.stdout, (done.returncode, done.stderr[-2000:])
