@@ -172,6 +172,20 @@ def build(force: bool = False, quiet: bool = False) -> Path:
     return lib
 
 
+# How the binding is compiled, but for the paths: they say where torch and this tree lie, not what is made of them.
+BINDING_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM"]
+
+
+def _cxx() -> str:
+    return os.environ.get("CXX", "g++")
+
+
+def _binding_flags() -> list[str]:
+    import torch
+
+    return [*BINDING_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+
+
 def _binding_command(out: Path) -> list[str]:
     import sysconfig
 
@@ -181,16 +195,15 @@ def _binding_command(out: Path) -> list[str]:
     rocm = Path(_hipcc()).resolve().parent.parent
     includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
                 *(p for p in (rocm / "include", Path("/opt/rocm/include")) if p.exists()), CSRC]
-    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{i}" for i in includes], str(CSRC / "binding.cpp"),
+    return [_cxx(), *_binding_flags(), *[f"-I{i}" for i in includes], str(CSRC / "binding.cpp"),
             f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-ldl", "-o", str(out)]
 
 
 def _binding_digest() -> str:
-    """What the binding is built from: its source, the declarations, torch and the interpreter."""
+    """What the binding is built from: its source, the declarations, the compiler and its flags, torch and the interpreter."""
     import torch
 
-    return _digest([CSRC / "binding.cpp", CSRC / "pyre_api.h"], f"{torch.__version__} {sys.version}")
+    return _digest([CSRC / "binding.cpp", CSRC / "pyre_api.h"], " ".join([_cxx(), *_binding_flags(), torch.__version__, sys.version]))
 
 
 def build_binding(force: bool = False, quiet: bool = False) -> Path:

@@ -106,3 +106,15 @@ def test_an_exception_in_an_entry_is_an_error_of_the_call(tmp_path):
     done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300,
                           cwd=Path(build.CSRC).parent.parent)
     assert done.returncode == 0 and "held" in done.stdout, (done.returncode, done.stderr[-2000:])
+
+
+def test_the_binding_is_stale_when_it_would_be_compiled_otherwise(monkeypatch):
+    from pyre_amd.hip import build
+
+    digests = {build._binding_digest()}
+    with monkeypatch.context() as m:
+        m.setattr(build, "BINDING_FLAGS", [*build.BINDING_FLAGS, "-g"])
+        digests.add(build._binding_digest())
+    monkeypatch.setenv("CXX", "another-compiler")
+    digests.add(build._binding_digest())
+    assert len(digests) == 3
