@@ -180,6 +180,16 @@ def _cxx() -> str:
     return os.environ.get("CXX", "g++")
 
 
+def _rocm_includes() -> list[Path]:
+    """Where HIP's headers may lie; hipcc is not needed for it (torch's headers name them, no device code is compiled)."""
+    roots = [Path(os.environ[v]) for v in ("ROCM_PATH", "HIP_PATH") if os.environ.get(v)]
+    try:
+        roots.append(Path(_hipcc()).resolve().parent.parent)
+    except BuildError:
+        pass
+    return [p for p in dict.fromkeys(r / "include" for r in [*roots, Path("/opt/rocm")]) if p.exists()]
+
+
 def _binding_flags() -> list[str]:
     import torch
 
@@ -192,9 +202,7 @@ def _binding_command(out: Path) -> list[str]:
     import torch
 
     root = Path(torch.__file__).resolve().parent
-    rocm = Path(_hipcc()).resolve().parent.parent
-    includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
-                *(p for p in (rocm / "include", Path("/opt/rocm/include")) if p.exists()), CSRC]
+    includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"], *_rocm_includes(), CSRC]
     return [_cxx(), *_binding_flags(), *[f"-I{i}" for i in includes], str(CSRC / "binding.cpp"),
             f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-ldl", "-o", str(out)]
 
@@ -215,7 +223,10 @@ def build_binding(force: bool = False, quiet: bool = False) -> Path:
         return lib
     t0 = time.time()
     tmp = out / f".{os.getpid()}.{BINDING_NAME}"
-    proc = subprocess.run(_binding_command(tmp), capture_output=True, text=True)
+    try:
+        proc = subprocess.run(_binding_command(tmp), capture_output=True, text=True)
+    except OSError as e:
+        raise BuildError(f"no C++ compiler for binding.cpp ($CXX or g++): {e}") from None
     if proc.returncode != 0:
         raise BuildError(f"the compiler failed on binding.cpp:\n{proc.stderr[-4000:]}")
     os.replace(tmp, lib)

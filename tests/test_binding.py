@@ -118,3 +118,14 @@ def test_the_binding_is_stale_when_it_would_be_compiled_otherwise(monkeypatch):
     monkeypatch.setenv("CXX", "another-compiler")
     digests.add(build._binding_digest())
     assert len(digests) == 3
+
+
+def test_the_binding_is_compiled_without_hipcc(monkeypatch, tmp_path):
+    from pyre_amd.hip import build
+
+    def missing():
+        raise build.BuildError("hipcc not found")
+
+    monkeypatch.setattr(build, "_hipcc", missing)
+    command = build._binding_command(tmp_path / "x.so")
+    assert command[0] == build._cxx() and any(c.endswith("/include") and Path(c[2:]).joinpath("hip").exists() for c in command if c.startswith("-I"))
