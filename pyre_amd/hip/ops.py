@@ -14,14 +14,14 @@ from functools import lru_cache
 import torch
 
 from pyre_amd.hip.lib import KernelError, call
-from pyre_amd.hip.native import binding
+from pyre_amd.hip.native import binding, late
 
 #: compute units that launch plans are made for when nobody names a device (an MI355X)
 DEFAULT_UNITS = 256
 
 
 #: the element type's code of a tensor or a type; what the kernels do not take is refused
-dtype_code = binding.dtype_code
+dtype_code = late(globals(), "dtype_code", "dtype_code")
 
 
 _STREAM: int | None = None
@@ -39,7 +39,8 @@ def _stream() -> int:
 
 
 # Checks of operands: every tensor lies on a GPU; a tensor is contiguous; int32, contiguous and of enough entries; its address.
-_dev, _contig, _i32, _ptr = binding.dev, binding.contig, binding.i32, binding.ptr
+_dev, _contig = late(globals(), "_dev", "dev"), late(globals(), "_contig", "contig")
+_i32, _ptr = late(globals(), "_i32", "i32"), late(globals(), "_ptr", "ptr")
 
 
 @dataclass

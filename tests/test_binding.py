@@ -108,6 +108,33 @@ def test_an_exception_in_an_entry_is_an_error_of_the_call(tmp_path):
     assert done.returncode == 0 and "held" in done.stdout, (done.returncode, done.stderr[-2000:])
 
 
+def without_compilers(tmp_path):
+    import os
+
+    return {**os.environ, "PYRE_AMD_BUILD_DIR": str(tmp_path / "empty"), "CXX": "/nowhere/g++", "HIPCC": "/nowhere/hipcc", "PATH": str(tmp_path)}
+
+
+def test_what_plans_is_imported_without_a_compiler(tmp_path):
+    """Nothing built, no compiler: the package imports and plans; the first check of an operand says what is missing."""
+    code = textwrap.dedent("""
+        import torch
+        import pyre_amd.api, pyre_amd.parts.fast
+        from pyre_amd.hip import build, ops
+        from pyre_amd.parts.attention_work import decode_capacity
+        assert decode_capacity(8, 28, 4) > 8 and ops.attn_biased_tile_plan(4, 6, 1, 600)
+        for f in (lambda: ops.dtype_code(torch.float32), lambda: ops._dev(torch.zeros(1))):
+            try:
+                f()
+            except build.BuildError as e:
+                assert "no C++ compiler" in str(e), e
+            else:
+                raise SystemExit("no error")
+    """)
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, env=without_compilers(tmp_path),
+                          cwd=Path(lib.__file__).parents[2])
+    assert done.returncode == 0, done.stderr[-2000:]
+
+
 def test_the_binding_is_stale_when_it_would_be_compiled_otherwise(monkeypatch):
     from pyre_amd.hip import build
 
@@ -129,3 +156,9 @@ def test_the_binding_is_compiled_without_hipcc(monkeypatch, tmp_path):
     monkeypatch.setattr(build, "_hipcc", missing)
     command = build._binding_command(tmp_path / "x.so")
     assert command[0] == build._cxx() and any(c.endswith("/include") and Path(c[2:]).joinpath("hip").exists() for c in command if c.startswith("-I"))
+
+
+def test_functions_of_the_binding_take_their_names_at_the_first_call():
+    from pyre_amd.hip import ops
+
+    assert ops.dtype_code(torch.bfloat16) == 1 and ops.dtype_code is binding.dtype_code
