@@ -7,7 +7,7 @@
 //
 // The product is computed transposed, out^T = W X^T, on MFMA 32x32x16: A = 32 rows of W, B = 32
 // rows of X, both read along k as they are stored. A block owns 32 RTW RW rows of W and BM = 32 to 256
-// rows of X: RW groups of XW = 1 to 4 multiplying waves (a group on RTW tiles of 32 rows of W, its wave q
+// rows of X: RW groups of XW = 1 to 4 or 6 multiplying waves (a group on RTW tiles of 32 rows of W, its wave q
 // on the rows 32 CW q .. of X, CW = 1 or 2 tiles, against all tiles of the group) and some waves that only
 // load. k is walked in stages of 64 through a ring in LDS that is filled by loads from memory
 // straight into LDS, S - 1 stages ahead; a stage holds its rows as 128-byte rows whose eight
@@ -338,6 +338,9 @@ int most_features(int M, int two_i) {
 // gate/up in 224 blocks of 40 instead of 140 of 64, 15.2 -> 12.4 at one row, 17.6 -> 14.5 at 64, 20.3 -> 17.3 at 99, 26.5 -> 22.8 at 190,
 // 28.7 -> 25.1 at 256; the 7B shape's in 237 of 80 instead of 198 of 96, 47.0 -> 45.6 at 8, 52.7 -> 48.4 at 64, 62.1 -> 57.6 at 128. The
 // 1.5B shape's q/k/v 5.1 -> 4.5 at one row, 5.9 -> 5.3 at 64, 9.1 -> 8.5 at 190, its way down 8.1 -> 7.2, 9.4 -> 8.9, 15.5 -> 14.9.
+// Of the other sizes, the kernel alone, at 1, 64, 128 and 256 rows: 32 features (8,192 of k = 2,048) 20.2 -> 16.7, 21.0 -> 16.6,
+// 25.4 -> 20.2, 35.2 -> 28.5; 48 (11,008 of 2,048) 21.6 -> 19.7, 22.5 -> 20.9, 25.9 -> 24.0, 35.8 -> 35.2; 64 (13,824 of 5,120) 46.9 -> 46.1,
+// 52.8 -> 52.4, 63.5 -> 63.2, 91.3 -> 91.2; 96 (22,016 of 4,096) 68.3 -> 65.8, 66.6 -> 65.6, 73.4 -> 72.3.
 int feature_groups(int M, int two_i) {
   const int inter = two_i / 2, units = compute_units(), most = most_features(M, two_i);
   if ((inter + most - 1) / most > units) return most / 8;
@@ -378,6 +381,8 @@ static int mid_gated(const void* X, long ldx, const void* W, long ldw, void* out
     else if (groups == 5) go(gemm_mid_kernel<1, 4, 1, 3, 5, 16, kSiluMul, 1, 4>, 13);
     else if (groups == 6) go(gemm_mid_kernel<1, 4, 1, 3, 6, 16, kSiluMul, 2, 4>, 14);
     else if (groups == 8) go(gemm_mid_kernel<1, 4, 2, 2, 8, 16, kSiluMul, 8, 4>, 16);
+    // (96 rows of X: 46.0 us at 65 and 49.0 at 96 on the 7B shape, where the 128 rows of the form below take 50.8 and 53.5)
+    else if (groups == 10 && M <= 96) go(gemm_mid_kernel<1, 3, 1, 5, 10, 12, kSiluMul, 1, 4>, 16);
     else if (groups == 10) go(gemm_mid_kernel<2, 2, 1, 5, 10, 16, kSiluMul, 2, 4>, 12);
     else if (M <= 96) go(gemm_mid_kernel<1, 3, 2, 3, 12, 12, kSiluMul, 3, 4>, 12);
     else go(gemm_mid_kernel<1, 4, 2, 3, 12, 16, kSiluMul, 2, 3>, 14);
@@ -396,7 +401,9 @@ static int mid_gated(const void* X, long ldx, const void* W, long ldw, void* out
     else if (groups == 8) go(gemm_mid_kernel<1, 1, 1, 4, 8, 4, kSiluMul, 6, 6>, 10);
     else if (groups == 10) go(gemm_mid_kernel<1, 1, 1, 5, 10, 4, kSiluMul, 7, 6>, 12);
     else if (groups == 12) go(gemm_mid_kernel<1, 1, 1, 6, 12, 4, kSiluMul, 8, 5>, 14);
-    else go(gemm_mid_kernel<1, 1, 2, 4, 16, 4, kSiluMul, 8, 4>, 12);
+    // (the 32B shape at 25 and 32 rows: 91.4 and 90.7 us, with two tiles a wave 94.0 and 93.5; with one or eight waves that only load
+    // beside these eight 93.2 and 92.1, 93.6 and 92.5)
+    else go(gemm_mid_kernel<1, 1, 1, 8, 16, 4, kSiluMul, 4, 4>, 12);
   } else {
     if (groups == 4) go(gemm_mid_kernel<1, 1, 1, 2, 4, 1, kSiluMul, 7, 8>, 9);
     else if (groups == 5) go(gemm_mid_kernel<1, 1, 1, 3, 5, 1, kSiluMul, 8, 8>, 11);

@@ -28,3 +28,9 @@ def test_features_of_a_block(m, inter, k):
     few = torch.full((len(rows), inter), float("nan"), device=DEV, dtype=torch.bfloat16)
     ops.gemm_mid_silu_bf16(x[rows].contiguous(), w, few, len(rows))
     assert torch.equal(few, out[rows])
+
+
+@pytest.mark.parametrize("inter,m", [(20473, 66), (20473, 80), (20473, 96), (24571, 96), (27643, 25), (27643, 31), (27643, 32), (27643, 64)])
+def test_few_rows_of_many_features(inter, m):
+    """80 features against the 96 rows of X that are loaded, and 128."""
+    test_features_of_a_block(m, inter, 136)
