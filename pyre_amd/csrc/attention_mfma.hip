@@ -694,8 +694,8 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
   }
 }
 
-// Two forms of the kernel. The registers of a wave (two chunks of keys and values in flight)
-// leave room for two waves per SIMD. When the step has so few requests that a block per
+// Two forms of the kernel. The registers of a wave (two chunks of keys and values in flight, of heads
+// of 128) leave room for two waves per SIMD. When the step has so few requests that a block per
 // compute unit covers them, a second block on the same unit would leave another unit idle
 // (the dispatcher fills units in order): that form keeps a unit to one block. With more
 // requests than units, two blocks per unit hide each other's latencies at start and end.
@@ -709,9 +709,16 @@ __global__ __launch_bounds__(256, 2) void attn_decode_work_kernel(PYRE_DECODE_WO
   attn_decode_work_block<HD, STREAM_V, false, false>(PYRE_DECODE_WORK_ARGS, RopeIn{});
 }
 // The same two forms, finishing the q/k/v product themselves (heads of up to 128 elements). Where blocks share a unit there are three,
-// of one register set each (ONE), since those that do not start at once start when others end: 190 requests of 94 to 1,501 tokens
+// since those that do not start at once start when others end: 190 requests of 94 to 1,501 tokens
 // on the 1.5B heads are 594 blocks, of which 82 started after 17 us and ended after 31; all at once they end after 26 (31.9 us a
-// launch, now 29.4). A unit's loads on their way are what bounds them, not the sets that a wave keeps.
+// launch, now 29.4). Heads of more than 64 elements then have registers for one chunk's set (ONE), smaller ones for both. Us a launch with
+// two blocks a unit and now, contexts of up to 512, 4,096 and 16,384 tokens, all as long and ragged (a sixteenth to all of it): the 7B heads, 128
+// requests 29.5 29.1, 21.9 20.8, 177 178, 115 114, 668 668, 422 425; 256 requests 58.8 60.3, 42.7 40.1, 348 344, 208 211, 1,328 1,310,
+// 771 786; 32B, 96 requests 48.7 40.7, 35.9 30.6, 271 269, 161 155, 1,001 1,020, 580 568; 1.5B, 190 requests 26.3 25.8, 19.0 18.3, 152
+// 153, 85 85, 564 574, 272 269 (runs of one side differ by 1 to 2 %). So many keys are bound by the unit's loads on their way, not by
+// the sets that a wave keeps; heads of 64 have half as many bytes to a set and lose by it: 129 requests of 16,384 tokens of 14 such
+// heads 193 with two blocks, 205 with three of one set, 193 with three of two (of 1,024 to 4,096, ragged, 190 requests 18.7, 18.0 and 17.3,
+// 49.6, 46.1 and 46.5; 256 25.2, 21.2 and 22.8).
 template <int HD, bool STREAM_V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_decode_work_rope_alone_kernel(
     PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
@@ -719,7 +726,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 }
 template <int HD, bool STREAM_V>
 __global__ __launch_bounds__(256, 3) void attn_decode_work_rope_kernel(PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
-  attn_decode_work_block<HD, STREAM_V, true, true>(PYRE_DECODE_WORK_ARGS, rope);
+  attn_decode_work_block<HD, STREAM_V, true, (HD > 64)>(PYRE_DECODE_WORK_ARGS, rope);
 }
 #undef PYRE_DECODE_WORK_PARAMS
 #undef PYRE_DECODE_WORK_ARGS

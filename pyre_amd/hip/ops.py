@@ -835,7 +835,8 @@ def attn_decode_work_bf16(q, out, k_cache, v_cache, work, capacity, positions, s
                           part_acc, part_ml, counters, alone, nq, nkv, hd, page_size, scale, window=0) -> None:
     """Attention of single new tokens over the paged cache from a work list (int32
     ``[1 + blocks, 8]``: see ``pyre_attn_decode_work_bf16`` in pyre_api.h) in a launch of
-    ``capacity`` blocks per key/value head, one (``alone``) or two to a compute unit.
+    ``capacity`` blocks per key/value head, one (``alone``) or two to a compute unit (three in
+    :func:`attn_decode_work_rope_bf16`).
     ``counters`` must be zero and is left at zero."""
     _attn_common(q, out, k_cache, v_cache, positions, seq_of_token, block_table, nq, nkv, hd, page_size)
     _i32("work", work, 8 * (1 + capacity))

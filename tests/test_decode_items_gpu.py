@@ -14,3 +14,10 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("ks,bias,alone", [(8, True, True), (9, False, False), (12, True, False)])
 def test_items_and_parts(nq, nkv, ks, bias, alone):
     check(nq, nkv, 128, 16, ks, bias, 0, None, alone)
+
+
+@pytest.mark.parametrize("nq,nkv,hd,page", [(14, 2, 64, 16), (7, 1, 32, 32), (12, 2, 96, 16), (14, 2, 128, 64)])
+@pytest.mark.parametrize("window,size", [(0, None), (0, 3), (70, None), (0, 40)])
+def test_forms_that_share_a_unit(nq, nkv, hd, page, window, size):
+    """Waves of no, one, two and many chunks, with one set of registers (heads of more than 64 elements) and with two."""
+    check(nq, nkv, hd, page, 2, True, window, size, False)
