@@ -1415,13 +1415,9 @@ extern "C" int pyre_attn_biased_tile(const void* q, void* out, int out_ld, int d
   const dim3 grid(n_tiles, nkv * hgroups);
 #define PYRE_TILE(T, NV, VEC)                                                                                           \
   do {                                                                                                               \
-    static size_t raised = 64 * 1024;                                                                                \
-    if (lds > raised) {                                                                                              \
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_biased_tile_kernel<T, NV, VEC>),                        \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)      \
-        return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds);                                   \
-      raised = lds;                                                                                                  \
-    }                                                                                                                \
+    static LdsLimit limit;                                                                                           \
+    if (!allow_lds(limit, reinterpret_cast<const void*>(&attn_biased_tile_kernel<T, NV, VEC>), lds))                 \
+      return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds);                                     \
     hipLaunchKernelGGL((attn_biased_tile_kernel<T, NV, VEC>), grid, dim3(kThreads), lds, stream, static_cast<const T*>(q), \
                        static_cast<const T*>(k_cache), static_cast<const T*>(v_cache), static_cast<T*>(out), out_ld, \
                        gate, out_scale, tiles, positions, seq_of_token, block_table, table_stride, nq, nkv, dk, dkp,  \
@@ -1443,13 +1439,9 @@ extern "C" int pyre_attn_biased_tile(const void* q, void* out, int out_ld, int d
     constexpr size_t plain = Tile32<DKP, NV, KS>::LDS;                                                                    \
     const int near = bias && plain + sizeof(float) * 2 * (static_cast<size_t>(far) + 1) <= budget ? 1 : 0;               \
     const size_t lds32 = plain + (near ? sizeof(float) * 2 * (far + 1) : 0);                                              \
-    static size_t raised = 64 * 1024;                                                                                     \
-    if (lds32 > raised) {                                                                                                 \
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_biased_tile32_kernel<DKP, NV, KS>),                     \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds32)) != hipSuccess)         \
-        return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds32);                                      \
-      raised = lds32;                                                                                                     \
-    }                                                                                                                     \
+    static LdsLimit limit;                                                                                                \
+    if (!allow_lds(limit, reinterpret_cast<const void*>(&attn_biased_tile32_kernel<DKP, NV, KS>), lds32))                 \
+      return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds32);                                        \
     hipLaunchKernelGGL((attn_biased_tile32_kernel<DKP, NV, KS>), grid32, dim3(128 * KS), lds32, stream,                   \
                        static_cast<const float*>(q), static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), \
                        static_cast<float*>(out), out_ld, gate, out_scale, tiles, positions, seq_of_token, block_table,    \
@@ -1494,13 +1486,9 @@ extern "C" int pyre_attn_biased_tile(const void* q, void* out, int out_ld, int d
   } while (0)
 #define PYRE_TILE16T(NV, TAB)                                                                                            \
   do {                                                                                                                   \
-    static size_t raised = 64 * 1024;                                                                                    \
-    if (lds16 > raised) {                                                                                                \
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_biased_tile16_kernel<NV, TAB>),                        \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds16)) != hipSuccess)        \
-        return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds16);                                     \
-      raised = lds16;                                                                                                    \
-    }                                                                                                                    \
+    static LdsLimit limit;                                                                                               \
+    if (!allow_lds(limit, reinterpret_cast<const void*>(&attn_biased_tile16_kernel<NV, TAB>), lds16))                    \
+      return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds16);                                       \
     hipLaunchKernelGGL((attn_biased_tile16_kernel<NV, TAB>), grid16, dim3(kThreads), lds16, stream, static_cast<const bf16*>(q), \
                        static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), static_cast<bf16*>(out),    \
                        out_ld, gate, out_scale, tiles, positions, seq_of_token, block_table, table_stride, nq, nkv, dk,  \
@@ -1560,13 +1548,9 @@ extern "C" int pyre_attn_biased_single(const void* q, void* out, int out_ld, int
     const size_t lds = sizeof(float) * 4 * nh * (128 * ev + 4);
 #define PYRE_SINGLE16(DKS, EV)                                                                                           \
   do {                                                                                                                   \
-    static size_t raised = 64 * 1024;                                                                                    \
-    if (lds > raised) {                                                                                                  \
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_biased_single16_kernel<DKS, EV>),                      \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)          \
-        return fail("attn_biased_single: the device refuses %zu bytes of LDS", lds);                                     \
-      raised = lds;                                                                                                      \
-    }                                                                                                                    \
+    static LdsLimit limit;                                                                                               \
+    if (!allow_lds(limit, reinterpret_cast<const void*>(&attn_biased_single16_kernel<DKS, EV>), lds))                    \
+      return fail("attn_biased_single: the device refuses %zu bytes of LDS", lds);                                       \
     hipLaunchKernelGGL((attn_biased_single16_kernel<DKS, EV>), dim3(n, nkv * col_groups, part ? max_spans : 1), dim3(kThreads), lds, \
                        stream, static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), \
                        static_cast<bf16*>(out), out_ld, gate, out_scale, tokens, positions, seq_of_token, block_table,   \

@@ -395,7 +395,6 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
 }
 
 constexpr int kStreamMaxRows = 32;
-constexpr int kMaxDevices = 64;
 constexpr int kSlotK = 32;  // k of a slot of the ring: rows of 128 bytes
 
 // 16 bytes per lane straight into LDS: lane x's piece lands at lds_addr + 16 x. The s_nop is the wait state that the instruction
@@ -602,15 +601,8 @@ __global__ __launch_bounds__(64 * (2 * C + kRowWaves)) void gemm_f32_stream_kern
 template <int C>
 bool launch_stream(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
                    int M, int N, int K, int kper, int parts, int chain, hipStream_t stream) {
-  static bool asked[kMaxDevices] = {};  // for that much LDS a block, once per device
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
-  if (!asked[dev]) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_stream_kernel<C>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            stream_bytes(C)) != hipSuccess)
-      return false;
-    asked[dev] = true;
-  }
+  static LdsLimit limit;
+  if (!allow_lds(limit, reinterpret_cast<const void*>(&gemm_f32_stream_kernel<C>), stream_bytes(C))) return false;
   hipLaunchKernelGGL(gemm_f32_stream_kernel<C>, dim3((N + 32 * C - 1) / (32 * C), 1, parts), dim3(64 * (2 * C + kRowWaves)), stream_bytes(C),
                      stream, A, static_cast<size_t>(lda), W, static_cast<size_t>(ldw), bias, bias_dt, out, static_cast<size_t>(ldo),
                      static_cast<size_t>(part_stride), M, N, K, kper, chain);

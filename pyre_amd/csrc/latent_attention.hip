@@ -607,12 +607,8 @@ int launch(const char* what, LatentArgs a, int blocks, int spans, hipStream_t st
   PYRE_REQUIRE(lds <= budget, "%s: %zu bytes of LDS are more than a block has", what, lds);
   const int groups = SINGLE ? (a.heads + 32 * G - 1) / (32 * G) : (a.heads + G - 1) / G;
   const auto kernel = &latent_attn_kernel<T, G, SL, NVT, KQ, SINGLE>;
-  static size_t raised = 64 * 1024;
-  if (lds > raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
-      return fail("%s: the device refuses %zu bytes of LDS", what, lds);
-    raised = lds;
-  }
+  static LdsLimit limit;
+  if (!allow_lds(limit, reinterpret_cast<const void*>(kernel), lds)) return fail("%s: the device refuses %zu bytes of LDS", what, lds);
   // prompt tiles come with those that see the most keys first: all heads of the longest start before the shorter ones,
   // which then fill the compute units that are done
   PYRE_REQUIRE(SINGLE || blocks <= 65535, "%s: %d tiles are more than a launch holds", what, blocks);

@@ -8,6 +8,8 @@
 #include <cstdarg>
 #include <cstdio>
 
+#include "pyre_lds.h"
+
 namespace pyre {
 
 constexpr int kWave = 64;
@@ -212,6 +214,17 @@ inline int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail("%s: %s", what, hipGetErrorString(e));
   return 0;
+}
+
+// Lets launches of `kernel` on the current device ask for `bytes` of LDS; `limit` is the kernel's own, static.
+inline bool allow_lds(LdsLimit& limit, const void* kernel, size_t bytes) {
+  if (bytes <= LdsLimit::kPlain) return true;
+  int device = -1;
+  const bool allowed = hipGetDevice(&device) == hipSuccess && limit.allow(device, bytes, [&](size_t most) {
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(most)) == hipSuccess;
+  });
+  if (!allowed) (void)hipGetLastError();
+  return allowed;
 }
 
 inline bool known_dtype(int dt) { return dt == kF32 || dt == kBF16; }

@@ -299,13 +299,9 @@ int launch_scan(const ScanArgs& a, const int* q_start, const int* state_slots, i
   constexpr int kCh = kThreads / L;
   constexpr size_t lds = sizeof(float) * 2 * kTile * (2 * kCh + 2 * NS * L + kCh + 1);
   static_assert(lds <= 160 * 1024, "a compute unit has 160 KB of LDS");
-  static bool raised = lds <= 64 * 1024;
-  if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&ssm_scan_kernel<L, NS, PLAIN>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
-      return fail("ssm_scan: the device refuses %zu bytes of LDS", lds);
-    raised = true;
-  }
+  static LdsLimit limit;
+  if (!allow_lds(limit, reinterpret_cast<const void*>(&ssm_scan_kernel<L, NS, PLAIN>), lds))
+    return fail("ssm_scan: the device refuses %zu bytes of LDS", lds);
   hipLaunchKernelGGL((ssm_scan_kernel<L, NS, PLAIN>), dim3((a.inner + kCh - 1) / kCh, n_seqs), dim3(2 * kThreads), lds, stream, a,
                      q_start, state_slots);
   return 0;
