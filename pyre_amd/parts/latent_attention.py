@@ -17,6 +17,8 @@ GROUP = 32
 MOST_KEYS = 64
 #: keys and values that are made at a time: a portion with more of them runs over the rows, a step with more makes them in rounds
 MADE_BYTES = 256 << 20
+#: elements of a layer's cached rows from which on every portion runs over the rows: a product's operand lies within 4 GiB
+PRODUCT_ELEMENTS = 1 << 31
 
 
 def portion_pairs(start: int, n: int, window: int) -> int:
@@ -237,7 +239,7 @@ class LatentAttention(Mixer):
             ops.latent_rows(proj, n, s.rank, s.rot_dim, ctx.dtype, queries=(0, heads, s.key_dim, q, wide), **latent)
         o = ws.get("lattn.o", (n, heads, s.value_dim), ctx.dtype)
         made = 0
-        if self.heads_up is not None and rows.numel() < 1 << 31:  # (a product's operand lies within 4 GiB)
+        if self.heads_up is not None and rows.numel() < PRODUCT_ELEMENTS:
             made = len(ctx.host.arrays[f"{self.plan_name}.tiles"])
         a, b = ctx.host.arrays[f"{self.plan_name}.plain"].tolist() if made else (0, n)
         if b > a:

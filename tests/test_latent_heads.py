@@ -165,13 +165,25 @@ def test_refusals():
         ops.gemm_tile_paged(z(4, 1, 16, 128), z(2, 3, dt=torch.int32), 2, table, z(64, 64), z(1, 32, 64))
 
 
-@pytest.mark.gpu
-def test_both_ways_in_an_engine(tmp_path):
-    """Layers whose sizes the kernels take, whole prompts, portions (short ones behind many keys run over the rows themselves), single
-    tokens and a mixture of all in a step, against the plain implementation."""
+@pytest.fixture
+def runs(monkeypatch):
+    """What the engine's layers launch: (kernel, tiles) of every call over made keys and values and over the rows."""
+    from pyre_amd.hip import ops
+
+    seen = []
+    for name, at in (("latent_heads", 6), ("latent_attn_tile", 4)):
+        def counted(*args, name=name, at=at, real=getattr(ops, name)):
+            seen.append((name, args[at]))
+            return real(*args)
+
+        monkeypatch.setattr(ops, name, counted)
+    return seen
+
+
+def both_ways(tmp_path, steps_of):
     import plain_rukosun as P
     import rukosun_models as M
-    from test_rukosun_gpu import TOL, engine_of, in_portions, one_by_one, whole, write_model
+    from test_rukosun_gpu import TOL, engine_of, write_model
     from helpers import first_bad, random_ids, replay
 
     raw = M.model(61, 64, [M.layer(M.mixer(2, 128, 64, 128, 256, 0.1, window=90, q_rank=24), 40),
@@ -180,10 +192,50 @@ def test_both_ways_in_an_engine(tmp_path):
     reqs = {r: random_ids(61, n, seed=n) for r, n in (("a", 230), ("b", 67), ("c", 33))}
     want = {r: P.forward(w, cfg, ids).float() for r, ids in reqs.items()}
     eng = engine_of(tmp_path, "bfloat16")
-    a, b, c = (reqs[r] for r in "abc")
-    mixture = [([("a", a[:150], [0, 149]), ("b", b[:66], [65])], []),
-               ([("b", b[66:], [0]), ("a", a[150:155], [0, 4]), ("c", c, list(range(33)))], ["b", "c"]),
-               ([("a", a[155:], list(range(75)))], ["a"])]
-    for steps in (whole(reqs), in_portions(reqs, [100, 3, 70]), one_by_one({"b": b}, 4), mixture):
+    for steps in steps_of(reqs):
         bad, worst = first_bad(replay(eng, steps), want, TOL["bfloat16"])
         assert bad is None, bad
+
+
+@pytest.mark.gpu
+def test_both_ways_in_an_engine(tmp_path, runs):
+    """Layers whose sizes the kernels take, whole prompts, portions (short ones behind many keys run over the rows themselves), single
+    tokens and a mixture of all in a step, against the plain implementation."""
+    from test_rukosun_gpu import in_portions, one_by_one, whole
+
+    def steps_of(reqs):
+        a, b, c = (reqs[r] for r in "abc")
+        mixture = [([("a", a[:150], [0, 149]), ("b", b[:66], [65])], []),
+                   ([("b", b[66:], [0]), ("a", a[150:155], [0, 4]), ("c", c, list(range(33)))], ["b", "c"]),
+                   ([("a", a[155:], list(range(75)))], ["a"])]
+        for steps, launched in ((whole(reqs), {"latent_heads"}), (in_portions(reqs, [100, 3, 70]), {"latent_heads", "latent_attn_tile"}),
+                                (one_by_one({"b": b}, 4), {"latent_heads"}), (mixture, {"latent_heads", "latent_attn_tile"})):
+            runs.clear()
+            yield steps
+            assert {name for name, tiles in runs if tiles} == launched
+
+    both_ways(tmp_path, steps_of)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,tiles", [(256, [6, 1, 4, 3]), (128, [3, 2, 1])])
+def test_keys_that_are_made_in_rounds(tmp_path, runs, monkeypatch, rows, tiles):
+    """A step of three prompts whose keys and values do not fit together (two rounds in each of the two layers), or for the longest
+    not even alone (which then runs over the rows; one round and two): each round's groups and tiles, in the scratch of the one before."""
+    monkeypatch.setattr(L, "MADE_BYTES", rows * 3 * 512)
+
+    def steps_of(reqs):
+        yield [([(r, ids, list(range(len(ids)))) for r, ids in reqs.items()], list(reqs))]
+        assert [t for name, t in runs if name == "latent_heads"] == tiles
+        assert [t for name, t in runs if name == "latent_attn_tile"] == ([] if len(tiles) == 4 else [8, 8])
+
+    both_ways(tmp_path, steps_of)
+
+
+@pytest.mark.gpu
+def test_a_cache_beyond_the_products_reach_is_read_row_by_row(tmp_path, runs, monkeypatch):
+    from test_rukosun_gpu import whole
+
+    monkeypatch.setattr(L, "PRODUCT_ELEMENTS", 0)
+    both_ways(tmp_path, lambda reqs: [whole(reqs)])
+    assert {name for name, _ in runs} == {"latent_attn_tile"}
