@@ -204,7 +204,7 @@ def linear(lin, ctx, x, n, out):
 
     if out is not None:
         # float32 results wanted in place (the head's logits)
-        if (n <= SKINNY_MAX_ROWS or not library) and streams() and (n <= SKINNY_MAX_ROWS or not library):  # no split, 64 rows at a time
+        if (n <= SKINNY_MAX_ROWS or not library) and streams():  # no split, 64 rows at a time
             for r0 in range(0, n, SKINNY_MAX_ROWS):
                 rows = min(SKINNY_MAX_ROWS, n - r0)
                 ops.gemm_skinny_bf16(x[r0:r0 + rows], lin.weight, out[r0:r0 + rows], rows, 1)
