@@ -40,21 +40,29 @@ def made_rows(start: int, n: int, window: int) -> int:
 
 def makes_heads(start: int, n: int, spec: LatentAttentionSpec) -> bool:
     """Whether a portion's attention runs over keys and values made of the compressed rows that it sees, or over the rows
-    themselves. Multiply-adds of a pair and head (a weight is three pieces): row + 3 rank against key + 3 value elements; of
-    a key, or a token and head: rank x (key + value elements), for every key that is seen or for every token of the
-    portion, at two and a half times the rate. Decided by a portion's own sizes, so that its result does not depend on what runs
-    beside it.
+    themselves. Decided by a portion's own sizes, so that its result does not depend on what runs beside it.
 
-    Over the rows and over made keys and values, us a layer with what goes with each (rows of 512 + 64, heads of 128 + 64 and 128, a
-    window of 1,024): 12 heads, the first 2,048 tokens 183 and 55, the next 952 120 and 48, the first 512 70 and 31, the first 16 31 and
-    24, 64 behind 1,000 113 and 44; 28 heads 335 and 96, 221 and 70, 71 and 30, 30 and 24, 113 and 52; without a window 12 heads,
-    512 tokens behind 4,000 376 and 142, 28 heads, 1,000 behind 8,000 1,357 and 406. The line: 32 tokens behind 1,000 take 111 and
-    44 alone (50 with 28 heads), but where such portions fill the chip the two are alike."""
+    Half multiply-adds of the attention kernels, which take 2.7e-9 us each of a full chip (a weight is three pieces). Over the rows a pair
+    of a query and a key costs row + 3 rank of them where made ones cost key + 3 value elements, and a token and head is carried into the
+    rows' space and out of it, rank x (key + value elements) at 4.5 times the price. To make a key costs rank / 2 a key or value element, and
+    280 more since it is written and read. Few heads do not fill the chip even with several portions: a key is then less.
+
+    Over the rows and over made keys and values, us a layer with what goes with each (heads of 128 + 64 and 128), one portion and sixteen in
+    a step. Rows of 512 + 64, a window of 1,024: 12 heads, 64 tokens behind 1,000 105 and 48, 132 and 106, 128 tokens 114 and 52, 235 and 124;
+    28 heads, 60 tokens behind 2,048 107 and 56, 238 and 213; 64 heads, 64 tokens behind 1,000 115 and 68 but 455 and 501, 32 tokens 108 and
+    69 but 243 and 454, 128 tokens 116 and 70, 902 and 629. Without a window, 64 behind 3,000 of 64 heads 268 and 141 but 1,066 and 1,481. Rows
+    of 256 + 64: 64 heads, 64 tokens behind 1,000 254 and 391 sixteen times, 28 heads 128 tokens behind 8,000 1,340 and 2,381, 256 tokens
+    2,732 and 2,487. A whole prompt pays for no key twice: 12 heads, the first 2,048 tokens 183 and 55, the first 512 70 and 31, the first 16 31
+    and 24. Of 1,392 portions, one and sixteen at a time, the line leaves 14 of those that make them more than 3 % slower for it, none of them alone
+    in its step (12 heads, sixteen times 64 tokens behind 3,000, 288 and 362; else by 12 % at most)."""
     rows = made_rows(start, n, spec.window)
-    if rows > MOST_KEYS * n + GROUP or rows * spec.num_heads * (spec.key_dim + spec.value_dim) * 2 > MADE_BYTES:
+    elements = spec.key_dim + spec.value_dim
+    if rows > MOST_KEYS * n + GROUP or rows * spec.num_heads * elements * 2 > MADE_BYTES:
         return False
     a_pair = 4 * spec.rank - spec.key_dim - 3 * spec.value_dim
-    return 5 * portion_pairs(start, n, spec.window) * a_pair > 2 * (seen_keys(start, n, spec.window) - n) * spec.rank * (spec.key_dim + spec.value_dim)
+    pairs, tokens = portion_pairs(start, n, spec.window) * a_pair, n * spec.rank * elements
+    keys = seen_keys(start, n, spec.window) * elements * (560 + spec.rank)
+    return 64 * (2 * pairs + 9 * tokens) > min(64, spec.num_heads + 32) * keys
 
 
 def made_portions(hb, spec: LatentAttentionSpec):

@@ -83,6 +83,16 @@ def test_a_step_with_more_keys_than_are_made_at_a_time_makes_them_in_rounds(monk
     assert 0 not in L.plan_tiles(hb, spec)[:, 3]  # a portion with more than fit runs over the rows
 
 
+@pytest.mark.parametrize("rank,heads,window,start,n,made", [
+    (512, 12, 1024, 0, 16, True), (512, 12, 1024, 2048, 952, True), (512, 12, 1024, 1000, 64, True), (512, 28, 0, 8000, 1000, True),
+    (512, 64, 1024, 1000, 128, True), (256, 28, 0, 8000, 256, True), (256, 12, 0, 1000, 128, True), (192, 4, 0, 0, 700, True),
+    (512, 64, 1024, 1000, 32, False), (512, 64, 1024, 1000, 64, False), (512, 64, 0, 3000, 64, False), (256, 64, 0, 1000, 64, False),
+    (256, 64, 0, 8000, 128, False), (256, 28, 0, 8000, 128, False), (192, 28, 0, 8000, 128, False), (256, 128, 1024, 1000, 64, False)])
+def test_the_way_that_is_faster_where_portions_fill_the_chip(rank, heads, window, start, n, made):
+    """Both ways measured, sixteen portions in a step: :func:`makes_heads` has the times."""
+    assert L.makes_heads(start, n, spec_of(window, rank, heads)) == made
+
+
 def test_a_portion_goes_its_way_whatever_runs_beside_it():
     spec = spec_of(1024)
     alone = L.plan_tiles(batch_of([(700, 90)]), spec)
