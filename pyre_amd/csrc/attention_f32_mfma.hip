@@ -1,7 +1,7 @@
 // Causal (optionally windowed) attention of prompt portions over the paged cache in true
-// float32 on the matrix cores (v_mfma_f32_32x32x2_f32: float32 operands, products and sums):
+// float32 on the matrix cores (v_mfma_f32_16x16x4_f32: float32 operands, products and sums):
 // the 32-bit path's attention for requests that bring more than one token. Single tokens stay
-// with attention_generic.hip, whose one block per (token, head) cannot use a 32-column tile.
+// with attention_generic.hip, whose blocks are of one token and cannot fill sixteen columns.
 //
 //   scores = (q k^T) * scale, masked to lo..pos       (pyre/model.py:109-120)
 //   probs  = softmax(scores), out = probs v            (pyre/model.py:122-123)
