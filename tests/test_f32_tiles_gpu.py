@@ -172,3 +172,35 @@ def test_k_that_ends_within_a_step_and_rows_that_start_anywhere(n, k, ks, off):
         ops.gemm_f32(pad(a[:rows], (0, whole - k)), pad(w, (0, whole - k)), None, want if ks > 1 else want[0], rows, ks)
         ops.gemm_f32(laid(a[:rows], 0), laid(w, 3 if off else 0), None, out if ks > 1 else out[0], rows, ks)
         assert torch.equal(out, want), rows
+
+
+@pytest.mark.parametrize("nq,nkv,hd,page,window", [(12, 2, 128, 16, 0), (7, 1, 64, 16, 40), (5, 5, 32, 8, 0), (6, 2, 96, 16, 70), (9, 3, 250, 16, 0),
+                                                   (4, 2, 192, 12, 33), (3, 1, 128, 3, 0), (8, 1, 256, 16, 0)])
+def test_prompts_of_many_tiles_have_the_bits_of_one_alone(nq, nkv, hd, page, window):
+    """Tiles that fill the chip run in blocks of whole tiles whose waves have two parts of the keys each, few tiles in blocks of
+    sixteen tokens and a wave for every part: first and last chunks of every part, halves of tiles that are not there."""
+    from pyre_amd.hip import ops
+
+    cases = [(0, 1), (0, 17), (0, 32), (31, 2), (32, 16), (33, 31), (64, 5), (95, 33), (127, 20), (128, 1), (129, 48), (250, 40)]
+    repeat = 90
+    pages = -(-290 // page)
+    kc, vc = rnd(len(cases) * pages, nkv, page, hd, seed=1), rnd(len(cases) * pages, nkv, hd, page, seed=2)
+    table = torch.randperm(len(cases) * pages, generator=torch.Generator().manual_seed(3)).view(len(cases), pages).int().to(DEV)
+
+    def run(which):
+        pos, seq, tiles, n = [], [], [], 0
+        for r in which:
+            first, count = cases[r]
+            tiles += [(n + t, min(32, count - t)) for t in range(0, count, 32)]
+            pos += range(first, first + count)
+            seq += [r] * count
+            n += count
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+        q = torch.cat([rnd(cases[r][1], nq, hd, seed=10 + r) for r in which])
+        out = torch.full((n, nq, hd), float("nan"), device=DEV)
+        ops.attn_prefill_f32(q, out, kc, vc, i32(tiles), len(tiles), i32(pos), i32(seq), table, nq, nkv, hd, page, hd ** -0.5, window)
+        return out
+
+    alone = torch.cat([run([r]) for r in range(len(cases))])
+    assert not bool(alone.isnan().any())
+    assert torch.equal(run(list(range(len(cases))) * repeat), alone.repeat(repeat, 1, 1))
