@@ -28,6 +28,8 @@
 //
 // Chunks start at multiples of 32 keys and spans at the token's first visible key, so the order of
 // every sum of a token depends on its own bounds alone.
+#include <algorithm>
+
 #include "pyre_api.h"
 #include "pyre_common.h"
 #include "pyre_vec4.h"
@@ -401,58 +403,64 @@ __global__ __launch_bounds__(kThreads) void attn_biased_tile_kernel(
     }
 }
 
-// The same for float32 where heads are multiples of eight and rows start on 16 bytes, laid out as attention_f32_mfma.hip's: a block
-// takes sixteen tokens and two heads, on 16 x 16 x 4; of every KS chunks of 32 keys, which lie in LDS together, a
-// wave of a head takes one, by the chunk's number, and the parts are joined at the end in their order. DKP and 32 NV: the
-// head sizes padded with zeros.
+// The same for float32 where heads are multiples of eight and rows start on 16 bytes, laid out as attention_f32_mfma.hip's, which says
+// why: a wave has sixteen tokens and a head, on 16 x 16 x 4; of every KS chunks of 32 keys each goes to a part by the chunk's number,
+// and the parts are joined at the end in their order. SHARED: a block of a whole tile and two heads, whose waves have two parts each; else
+// of sixteen tokens and two heads and a wave for every part; the same bits. DKP and 32 NV: the head sizes padded with zeros.
 // With 32 tokens and four heads a block, a wave a head, 600 tokens of six heads were 38 blocks of four waves, each a chain of up to 19
-// chunks of 11 us whose loads waited for one another behind branches. Us a launch, biases of 1,025 distances and a cap,
-// before and now: 600 tokens of six heads of 128 205 and 53, of fourteen 209 and 66, 150 behind 600 258 and 60, sixteen 22 and 16,
-// 2,048 of 28 heads 1,354 and 786, 2,048 behind 4,000 of fourteen 1,950 and 1,410 (without biases), with a window of 1,024 378 and 359;
-// 700 of eight heads of 64 164 and 54, of 96 / 256 348 and 94. The distance from 64 bits is smaller in all of them (5.1e-7 and
-// 4.7e-7 for the first, 14.1e-7 and 8.9e-7 behind 4,000 tokens).
-template <int DKP, int NV, int KS>
+// chunks of 11 us whose loads waited for one another behind branches. Us a launch so and now, biases of 1,025 distances: 600 tokens of six
+// heads of 128 205 and 46, of fourteen 209 and 49, 150 behind 600 258 and 55, 2,048 of 28 heads 1,354 and 495, 2,048 behind 4,000 of fourteen 1,950
+// and 1,061 (without biases), with a window of 1,024 378 and 250; 700 of eight heads of 64 164 and 34. Many short portions, us so, always in
+// sixteen tokens and now: 120 of sixteen tokens on fourteen heads of 128 37, 83 and 45, behind 100 others 96, 114 and 86, with a window of 64 94, 148 and
+// 94; 200 of two tokens on sixteen heads of 64 27, 77 and 33, 80, 109 and 68, 78, 151 and 79. The distance from 64 bits is smaller than with one
+// part in all of them (5.1e-7 and 4.7e-7 for the first, 14.1e-7 and 8.9e-7 behind 4,000 tokens).
+template <int DKP, int NV, int KS, bool SHARED>
 struct Tile32 {
-  static constexpr int HEADS = 2, TOKENS = 16, THREADS = 64 * HEADS * KS, KEYS = kKeys * KS, DVP = 32 * NV;
-  static constexpr int KROW = DKP + 4, VROW = kKeys + 4, KSIZE = KEYS * KROW, VSIZE = KS * DVP * VROW;
-  static constexpr int JOIN = HEADS * KS * TOKENS;  // rows that are joined: DVP + 4 sums (sixteen bytes), a maximum and a sum of weights
-  static_assert(JOIN * (DVP + 4 + 2) <= KSIZE + VSIZE, "what is joined lies where the keys and values lay");
-  static constexpr size_t LDS = sizeof(float) * (KSIZE + VSIZE) + 3 * KEYS * (sizeof(longlong2) + sizeof(int));
+  static constexpr int HEADS = 2, TOKENS = 16, HALVES = SHARED ? 2 : 1, KW = SHARED ? KS / 2 : KS, ACC = KS / KW;  // ACC: parts that a wave keeps
+  static constexpr int GROUPS = HEADS * HALVES, THREADS = 64 * GROUPS * KW, KEYS = kKeys * KW, DVP = 32 * NV;
+  static constexpr int KROW = DKP + 4, VROW = kKeys + 4, KSIZE = KEYS * KROW, VSIZE = KW * DVP * VROW;
+  static constexpr int JOINED = GROUPS * KW * TOKENS, JSIZE = JOINED * (DVP + 4 + 2 * ACC);  // rows that are joined at a time; maxima and sums behind
+  static constexpr int SIZE = KSIZE + VSIZE > JSIZE ? KSIZE + VSIZE : JSIZE;
+  static constexpr size_t LDS = sizeof(float) * SIZE + 3 * KEYS * (sizeof(longlong2) + sizeof(int));
+  static constexpr int WAVES = NV > 4 ? 1 : SHARED && DKP <= 64 && NV <= 2 ? 4 : 2;  // a SIMD
 };
-template <int DKP, int NV, int KS>
-__global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
+template <int DKP, int NV, int KS, bool SHARED>
+__global__ __launch_bounds__(128 * KS, (Tile32<DKP, NV, KS, SHARED>::WAVES)) void attn_biased_tile32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache, float* __restrict__ out,
     int out_ld, const float* __restrict__ gate, float out_scale, const int* __restrict__ tiles,
     const int* __restrict__ positions, const int* __restrict__ seq_of_token, const int* __restrict__ block_table,
     int table_stride, int nq, int nkv, int dk, int dv, int page_size, float scale, float cap, const float* __restrict__ bias,
     int far, int window, int keep_first, int chunk, int bias_lds, const float* __restrict__ sink, int gate_dim) {
-  using Shape = Tile32<DKP, NV, KS>;
-  constexpr int HEADS = Shape::HEADS, TOKENS = Shape::TOKENS, THREADS = Shape::THREADS, KEYS = Shape::KEYS, DVP = Shape::DVP;
-  constexpr int KROW = Shape::KROW, VROW = Shape::VROW, OROW = DVP + 4;
+  using Shape = Tile32<DKP, NV, KS, SHARED>;
+  constexpr int HEADS = Shape::HEADS, HALVES = Shape::HALVES, GROUPS = Shape::GROUPS, KW = Shape::KW, ACC = Shape::ACC, TOKENS = Shape::TOKENS, THREADS = Shape::THREADS, KEYS = Shape::KEYS, DVP = Shape::DVP;
+  constexpr int KROW = Shape::KROW, VROW = Shape::VROW, OROW = DVP + 4, JOINED = Shape::JOINED;
   typedef f32x4 f32x4_anywhere __attribute__((aligned(4)));
   extern __shared__ __attribute__((aligned(16))) float lds[];
   float* const Ks = lds;                     // [key][d]
   float* const Vt = Ks + Shape::KSIZE;       // [part][d][key of the chunk]
-  longlong2* const where = reinterpret_cast<longlong2*>(Vt + Shape::VSIZE);  // of three rounds' keys: where key and value start
+  longlong2* const where = reinterpret_cast<longlong2*>(lds + Shape::SIZE);  // of three rounds' keys: where key and value start
   int* const pages = reinterpret_cast<int*>(where + 3 * KEYS);               // and their pages; -1: not there
   float* const bias_s = reinterpret_cast<float*>(pages + 3 * KEYS);          // [HEADS][far + 1], if they fit
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, c = lane & 15;
-  const int n_rep = nq / nkv, kvh = blockIdx.z, part = wave / HEADS, hin = blockIdx.y * HEADS + wave % HEADS;
-  const bool active = hin < n_rep;  // a wave without a head still helps loading
-  const int head = kvh * n_rep + (active ? hin : 0);
-  const int half_tile = gridDim.x - 1 - blockIdx.x;  // the last tokens, which see the most keys, first
-  const int t0 = tiles[half_tile & ~1] + TOKENS * (half_tile & 1);
-  const int ntok = min(TOKENS, tiles[half_tile | 1] - TOKENS * (half_tile & 1));
+  const int n_rep = nq / nkv, hgroups = (n_rep + HEADS - 1) / HEADS, per_piece = hgroups * nkv;
+  const int hgroup = blockIdx.x % per_piece % hgroups, kvh = blockIdx.x % per_piece / hgroups;
+  const int part = wave / GROUPS, hin = hgroup * HEADS + wave % HEADS;
+  const int wt = HALVES == 1 ? 0 : TOKENS * (wave / HEADS % HALVES);  // the wave's first token of the block's
+  const int piece = (gridDim.x - 1 - blockIdx.x) / per_piece;  // of a tile; the last tokens, which see the most keys, first
+  const int tile = 2 * (HALVES == 1 ? piece >> 1 : piece), skip = HALVES == 1 ? TOKENS * (piece & 1) : 0;
+  const int t0 = tiles[tile] + skip, ntok = min(TOKENS * HALVES, tiles[tile + 1] - skip);
   if (ntok <= 0) return;
+  const bool active = hin < n_rep && wt < ntok;  // a wave without a head or tokens still helps loading
+  const int head = kvh * n_rep + (hin < n_rep ? hin : 0);
   const int pos0 = positions[t0];
   const int* table = block_table + static_cast<size_t>(seq_of_token[t0]) * table_stride;
 
-  const bool live = active && c < ntok;
-  const int hi = c < ntok ? pos0 + c : pos0;
+  const bool live = active && wt + c < ntok;
+  const int hi = wt + c < ntok ? pos0 + wt + c : pos0;
   const int lo = first_seen(hi, window, chunk);
   const int keep = window > 0 ? keep_first : 0;
   const float* const bias_row = bias ? bias + static_cast<size_t>(head) * (far + 1) : nullptr;
-  if (bias && bias_lds && part == 0)
+  if (bias && bias_lds && wave < HEADS)
     for (int i = lane; i <= far; i += 64) bias_s[wave * (far + 1) + i] = bias_row[i];
   const float* const bias_near = bias_s + wave % HEADS * (far + 1);
   f32x4 qr[DKP / 16];  // element 16 s + 4 g + j of the query of token c
@@ -460,23 +468,30 @@ __global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
   for (int s = 0; s < DKP / 16; ++s) {
     const int d = 16 * s + 4 * g;
     qr[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (live && d < dk) qr[s] = *reinterpret_cast<const f32x4*>(q + (static_cast<size_t>(t0 + c) * nq + head) * dk + d);
+    if (live && d < dk) qr[s] = *reinterpret_cast<const f32x4*>(q + (static_cast<size_t>(t0 + wt + c) * nq + head) * dk + d);
   }
-  f32x4 o[DVP / 16];
+  f32x4 o[ACC][DVP / 16];
+  float m[ACC], l[ACC];
 #pragma unroll
-  for (int dt = 0; dt < DVP / 16; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -INFINITY, l = 0.f;
+  for (int a = 0; a < ACC; ++a) {
+    m[a] = -INFINITY, l[a] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DVP / 16; ++dt) o[a][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
-  // Rounds are KS chunks with neighbouring numbers from a multiple of KS on: those of the kept first tokens, then those of the window.
+  // Rounds are KW chunks with neighbouring numbers from a multiple of KW on: those of the kept first tokens, then those of the window.
   const int lo_all = first_seen(pos0, window, chunk);  // rises with the position: the tile's first token sees furthest back
   const int hi_all = pos0 + ntok - 1;
   const int kept_end = min(keep, lo_all);  // keys 0 .. kept_end - 1 lie before every window
   const int n_first = kept_end > 0 ? (kept_end - 1) / kKeys + 1 : 0;
   const int chunk_b = max(lo_all / kKeys, n_first), last_chunk = hi_all / kKeys;
-  const int rounds_first = (n_first + KS - 1) / KS, round_b = max(chunk_b / KS, rounds_first);
-  const int n_rounds = rounds_first + max(0, last_chunk / KS - round_b + 1);
+  const int rounds_first = (n_first + KW - 1) / KW, round_b = max(chunk_b / KW, rounds_first);
+  const int n_rounds = rounds_first + max(0, last_chunk / KW - round_b + 1);
   auto round_of = [&](int it) { return it < rounds_first ? it : round_b + (it - rounds_first); };
   auto needed = [&](int ch) { return ch < n_first || (ch >= chunk_b && ch <= last_chunk); };
+  // The same of the wave's own tokens.
+  const int wave_lo = first_seen(pos0 + wt, window, chunk), wave_last = min(pos0 + wt + TOKENS - 1, hi_all) / kKeys;
+  auto wanted = [&](int ch) { return needed(ch) && ch <= wave_last && (kKeys * ch + kKeys > wave_lo || kKeys * ch < keep); };
   auto look_up = [&](int it) {  // the page of key tid of a round
     const int key = KEYS * round_of(it) + tid, entry = key / page_size;
     return it < n_rounds && tid < KEYS && key <= hi_all && needed(key / kKeys) && entry < table_stride ? table[entry] : -1;
@@ -490,7 +505,7 @@ __global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
   };
   // Loads without a branch: a piece that is not there is read from the queries and becomes zeros when it is stored in LDS. Values
   // come as squares of four keys and four elements, which a thread turns over.
-  constexpr int KP = DKP / 16, VB = (NV + 1) / 2, SQUARES = KS * 8 * (DVP / 4);
+  constexpr int KP = DKP / (8 * GROUPS), VB = (NV + GROUPS - 1) / GROUPS, SQUARES = KW * 8 * (DVP / 4);
   f32x4 kp[KP], vp[VB][4];
   unsigned kgone = 0, vgone = 0;
   auto fetch = [&](int from) {
@@ -544,19 +559,8 @@ __global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
   note(1, 1, page1);
   __syncthreads();
   fetch(0);
-  int slot = 0;
-  for (int it = 0; it < n_rounds; ++it) {
-    const int next = slot == 2 ? 0 : slot + 1, here = slot * KEYS + kKeys * part;
-    __syncthreads();  // the round before has been read by every wave
-    note(it + 2, next == 2 ? 0 : next + 1, ahead);
-    put();
-    __syncthreads();
-    if (it + 1 < n_rounds) fetch(next);
-    ahead = look_up(it + 3);
-    slot = next;
-    const int ch = KS * round_of(it) + part;
-    if (!active || !needed(ch)) continue;
-
+  // A chunk of the part whose turn it is, a = 0.
+  auto attend = [&](int ch, int here) __attribute__((always_inline)) {
     f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int st = 0; st < DKP / 16; ++st) {
@@ -567,6 +571,7 @@ __global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kt][j], qr[st][j], s[kt], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // element j of s[kt]: key 16 kt + 4 g + j of the chunk, token c
     float bv[8];
@@ -586,20 +591,20 @@ __global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);
+    const float m_new = fmaxf(m[0], mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = expf(m - m_use);
-    m = m_new;
+    const float alpha = expf(m[0] - m_use);
+    m[0] = m_new;
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       s[i >> 2][i & 3] = expf(s[i >> 2][i & 3] - m_use);
       sum += s[i >> 2][i & 3];
     }
-    l = l * alpha + sum;
+    l[0] = l[0] * alpha + sum;
 #pragma unroll
-    for (int dt = 0; dt < DVP / 16; ++dt) o[dt] *= alpha;
-    constexpr int GROUP = DVP % 64 == 0 ? 4 : 2;  // tiles of d whose chains of products are in flight together
+    for (int dt = 0; dt < DVP / 16; ++dt) o[0][dt] *= alpha;
+    constexpr int GROUP = DVP % 64 == 0 && DVP > 64 ? 4 : 2;  // tiles of d whose chains of products are in flight together
 #pragma unroll
     for (int dt = 0; dt < DVP / 16; dt += GROUP)
 #pragma unroll
@@ -611,43 +616,87 @@ __global__ __launch_bounds__(128 * KS) void attn_biased_tile32_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int t = 0; t < GROUP; ++t) o[dt + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][j], s[kt][j], o[dt + t], 0, 0, 0);
+          for (int t = 0; t < GROUP; ++t) o[0][dt + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][j], s[kt][j], o[0][dt + t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
       }
-  }
-
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  float* const ml = lds + Shape::JOIN * OROW;  // [wave][token][2]
-  __syncthreads();
+  };
+  // The wave's other part takes the place of this one.
+  int turned = 0;
+  auto turn = [&]() __attribute__((always_inline)) {
+    if constexpr (ACC == 2) {
+      turned ^= 1;
+      const float m0 = m[0], l0 = l[0];
+      m[0] = m[1], m[1] = m0, l[0] = l[1], l[1] = l0;
 #pragma unroll
-  for (int dt = 0; dt < DVP / 16; ++dt)  // element j of o[dt]: d = 16 dt + 4 g + j of token c
-    *reinterpret_cast<f32x4*>(lds + (TOKENS * wave + c) * OROW + 16 * dt + 4 * g) = o[dt];
-  if (g == 0) {
-    ml[2 * (TOKENS * wave + c)] = m;
-    ml[2 * (TOKENS * wave + c) + 1] = l;
-  }
-  __syncthreads();
-  for (int i = tid; i < HEADS * TOKENS * (DVP / 4); i += THREADS) {
-    const int d = 4 * (i % (DVP / 4)), row = i / (DVP / 4), token = row % TOKENS, which = row / TOKENS;
-    const int h = static_cast<int>(blockIdx.y) * HEADS + which;
-    if (d >= dv || token >= ntok || h >= n_rep) continue;
-    float most = -INFINITY, total = 0.f;
-#pragma unroll
-    for (int p = 0; p < KS; ++p) most = fmaxf(most, ml[2 * (TOKENS * (HEADS * p + which) + token)]);
-    f32x4 y{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int p = 0; p < KS; ++p) {
-      const int at = TOKENS * (HEADS * p + which) + token;
-      const float weight = ml[2 * at] == -INFINITY ? 0.f : expf(ml[2 * at] - most);
-      total += weight * ml[2 * at + 1];
-      y += weight * *reinterpret_cast<const f32x4*>(lds + at * OROW + d);
+      for (int dt = 0; dt < DVP / 16; ++dt) {
+        const f32x4 o0 = o[0][dt];
+        o[0][dt] = o[1][dt], o[1][dt] = o0;
+      }
     }
-    float f = softmax_factor(most, total, sink, kvh * n_rep + h) * out_scale;
-    const float* grow = gate ? gate + (static_cast<size_t>(t0 + token) * nq + kvh * n_rep + h) * gate_dim : nullptr;
-    if (gate && gate_dim == 1) f *= grow[0];
+  };
+  int slot = 0;
+  for (int it = 0; it < n_rounds; ++it) {
+    const int next = slot == 2 ? 0 : slot + 1, here = slot * KEYS + kKeys * part;
+    __syncthreads();  // the round before has been read by every wave
+    note(it + 2, next == 2 ? 0 : next + 1, ahead);
+    put();
+    __syncthreads();
+    if (it + 1 < n_rounds) fetch(next);
+    ahead = look_up(it + 3);
+    slot = next;
+    const int round = round_of(it), ch = KW * round + part;
+    if (round % ACC != turned) turn();
+    if (active && wanted(ch)) attend(ch, here);
+  }
+  if (turned) turn();  // o[a] is that of parts KW a .. again
 #pragma unroll
-    for (int j = 0; j < 4; ++j) y[j] *= gate_dim > 1 && gate ? f * grow[d + j] : f;
-    *reinterpret_cast<f32x4_anywhere*>(out + static_cast<size_t>(t0 + token) * out_ld + (kvh * n_rep + h) * dv + d) = y;
+  for (int a = 0; a < ACC; ++a) {
+    l[a] += __shfl_xor(l[a], 16, 64);
+    l[a] += __shfl_xor(l[a], 32, 64);
+  }
+  // The parts of a head, joined in their order: outputs of KW parts at a time.
+  float* const ml = lds + JOINED * OROW;
+  constexpr int UNITS = GROUPS * TOKENS * (DVP / 4), ITEMS = (UNITS + THREADS - 1) / THREADS;
+  f32x4 y[ITEMS];
+#pragma unroll
+  for (int a = 0; a < ACC; ++a) {
+    __syncthreads();
+#pragma unroll
+    for (int dt = 0; dt < DVP / 16; ++dt)  // element j of o[a][dt]: d = 16 dt + 4 g + j of token c
+      *reinterpret_cast<f32x4*>(lds + (TOKENS * wave + c) * OROW + 16 * dt + 4 * g) = o[a][dt];
+    if (a == 0 && g == 0) {
+#pragma unroll
+      for (int b = 0; b < ACC; ++b) {
+        ml[2 * (JOINED * b + TOKENS * wave + c)] = m[b];
+        ml[2 * (JOINED * b + TOKENS * wave + c) + 1] = l[b];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int unit = tid + THREADS * i, d = 4 * (unit % (DVP / 4)), row = unit / (DVP / 4), token = row % TOKENS, group = row / TOKENS;
+      const int in_block = TOKENS * (group / HEADS) + token, h = hgroup * HEADS + group % HEADS;
+      if (unit >= UNITS || d >= dv || in_block >= ntok || h >= n_rep) continue;
+      const auto place = [&](int p) { return JOINED * (p / KW) + TOKENS * (GROUPS * (p % KW) + group) + token; };  // of part p's maximum and sum
+      float most = -INFINITY;
+#pragma unroll
+      for (int p = 0; p < KS; ++p) most = fmaxf(most, ml[2 * place(p)]);
+      const auto weight = [&](int p) { return ml[2 * place(p)] == -INFINITY ? 0.f : expf(ml[2 * place(p)] - most); };
+      if (a == 0) y[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < KW; ++w) y[i] += weight(KW * a + w) * *reinterpret_cast<const f32x4*>(lds + (TOKENS * (GROUPS * w + group) + token) * OROW + d);
+      if (a + 1 < ACC) continue;
+      float total = 0.f;
+#pragma unroll
+      for (int p = 0; p < KS; ++p) total += weight(p) * ml[2 * place(p) + 1];
+      const int head_out = kvh * n_rep + h;
+      float f = softmax_factor(most, total, sink, head_out) * out_scale;
+      const float* grow = gate ? gate + (static_cast<size_t>(t0 + in_block) * nq + head_out) * gate_dim : nullptr;
+      if (gate && gate_dim == 1) f *= grow[0];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[i][j] *= gate_dim > 1 && gate ? f * grow[d + j] : f;
+      *reinterpret_cast<f32x4_anywhere*>(out + static_cast<size_t>(t0 + in_block) * out_ld + head_out * dv + d) = y[i];
+    }
   }
 }
 
@@ -1433,35 +1482,50 @@ extern "C" int pyre_attn_biased_tile(const void* q, void* out, int out_ld, int d
   const bool vec = dk % 8 == 0 && dv % 8 == 0 && reinterpret_cast<uintptr_t>(k_cache) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(v_cache) % 16 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
   if (dt == kF32 && vec) {
-    const dim3 grid32(2 * n_tiles, (nq / nkv + 1) / 2, nkv);
-#define PYRE_TILE32(DKP, NV, KS)                                                                                          \
+    const int hpairs = (nq / nkv + 1) / 2;
+    // Both forms have the same bits; whole tiles share what they read where their blocks fill the chip. Us in sixteen tokens and shared,
+    // heads of 128: 40 blocks 55 and 90 (150 tokens behind 600), 152 49 and 76 (600 tokens), 304 73 and 74, 98 and 84, with windows 72 and 58, 106 and
+    // 98 (two portions of 600), 512 1,171 and 1,061, 608 133 and 115, 960 88 to 272 and 45 to 192; heads of 64: 176 34 and 58 (700 tokens), 304 46 and
+    // 57, 61 and 68, with windows 46 and 32, 68 and 54, 1,128 355 and 339. Values of more than 128 elements leave no registers for two parts:
+    // 376 blocks 292 and 318, 600 254 and 309.
+    const bool shared = nvp <= 4 && static_cast<long>(n_tiles) * hpairs * nkv > compute_units();
+    const int pieces32 = shared ? 1 : 2, threads32 = nvp > 4 ? 256 : 512;  // of a tile, of a block
+    const int most = static_cast<int>(((1L << 32) - 1) / threads32 / (pieces32 * hpairs * nkv));  // tiles of a launch
+#define PYRE_TILE32_AS(DKP, NV, KS, SHARED)                                                                               \
   do {                                                                                                                    \
-    constexpr size_t plain = Tile32<DKP, NV, KS>::LDS;                                                                    \
+    constexpr size_t plain = Tile32<DKP, NV, KS, SHARED>::LDS;                                                            \
     const int near = bias && plain + sizeof(float) * 2 * (static_cast<size_t>(far) + 1) <= budget ? 1 : 0;               \
     const size_t lds32 = plain + (near ? sizeof(float) * 2 * (far + 1) : 0);                                              \
     static LdsLimit limit;                                                                                                \
-    if (!allow_lds(limit, reinterpret_cast<const void*>(&attn_biased_tile32_kernel<DKP, NV, KS>), lds32))                 \
+    if (!allow_lds(limit, reinterpret_cast<const void*>(&attn_biased_tile32_kernel<DKP, NV, KS, SHARED>), lds32))         \
       return fail("attn_biased_tile: the device refuses %zu bytes of LDS", lds32);                                        \
-    hipLaunchKernelGGL((attn_biased_tile32_kernel<DKP, NV, KS>), grid32, dim3(128 * KS), lds32, stream,                   \
-                       static_cast<const float*>(q), static_cast<const float*>(k_cache), static_cast<const float*>(v_cache), \
-                       static_cast<float*>(out), out_ld, gate, out_scale, tiles, positions, seq_of_token, block_table,    \
-                       table_stride, nq, nkv, dk, dv, page_size, scale, cap, bias, far, window, keep_first, chunk, near, \
-                       sink, gate_dim);                                                                                   \
+    for (int at = 0; at < n_tiles; at += most)                                                                            \
+      hipLaunchKernelGGL((attn_biased_tile32_kernel<DKP, NV, KS, SHARED>), dim3(pieces32 * std::min(most, n_tiles - at) * hpairs * nkv), \
+                         dim3(threads32), lds32, stream, static_cast<const float*>(q), static_cast<const float*>(k_cache), \
+                         static_cast<const float*>(v_cache), static_cast<float*>(out), out_ld, gate, out_scale,            \
+                         tiles + 2 * static_cast<size_t>(at), positions, seq_of_token, block_table, table_stride, nq, nkv, \
+                         dk, dv, page_size, scale, cap, bias, far, window, keep_first, chunk, near, sink, gate_dim);       \
+  } while (0)
+#define PYRE_TILE32(DKP, NV, KS)                     \
+  do {                                               \
+    if (shared) PYRE_TILE32_AS(DKP, NV, KS, true);   \
+    else PYRE_TILE32_AS(DKP, NV, KS, false);         \
   } while (0)
 #define PYRE_TILE32_NV(DKP)                  \
   switch (nvp) {                             \
     case 1: PYRE_TILE32(DKP, 1, 4); break;   \
     case 2: PYRE_TILE32(DKP, 2, 4); break;   \
     case 4: PYRE_TILE32(DKP, 4, 4); break;   \
-    default: PYRE_TILE32(DKP, 8, 2); break;  \
+    default: PYRE_TILE32_AS(DKP, 8, 2, false); break; \
   }
-    // Waves a head by the head sizes alone, as far as LDS holds their chunks: a token's sums do not depend on the step.
+    // Parts by the head sizes alone, as far as LDS holds their chunks: a token's sums do not depend on the step.
     switch (dkp / 32) {
       case 1: PYRE_TILE32_NV(32); break;
       case 2: PYRE_TILE32_NV(64); break;
       case 3: PYRE_TILE32_NV(96); break;
       default: PYRE_TILE32_NV(128); break;
     }
+#undef PYRE_TILE32_AS
 #undef PYRE_TILE32
 #undef PYRE_TILE32_NV
     return check_launch("attn_biased_tile");

@@ -72,3 +72,39 @@ def test_against_64_bits_however_tokens_are_cut(nq, nkv, dk, dv, page, window, k
         assert not bool(out[:, nq * dv:].any())
         outs.append(out)
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("nq,nkv,dk,dv,page,window,keep,chunk,far", [
+    (5, 1, 128, 128, 16, 0, 0, 0, 300), (6, 2, 64, 40, 16, 60, 40, 0, 33), (3, 3, 24, 64, 12, 100, 70, 0, 0), (4, 2, 96, 128, 16, 0, 0, 96, 40000),
+    (7, 1, 32, 16, 8, 1, 130, 0, 0), (8, 1, 64, 64, 16, 33, 1, 0, 64), (2, 1, 128, 200, 16, 40, 0, 0, 0)])
+def test_portions_of_many_tiles_have_the_bits_of_one_alone(nq, nkv, dk, dv, page, window, keep, chunk, far):
+    """Tiles that fill the chip run in blocks of whole tiles whose waves have two parts of the keys each, few tiles in blocks of sixteen
+    tokens and a wave for every part: first and last chunks of every part, kept tokens and windows that begin in any of them, halves
+    of tiles that are not there."""
+    from pyre_amd.hip import ops
+
+    cases = [(0, 1), (0, 17), (0, 32), (31, 2), (32, 16), (33, 31), (64, 5), (95, 33), (127, 20), (128, 1), (129, 48), (250, 40)]
+    repeat, pages = 90, -(-290 // page)
+    rnd = lambda *shape, seed: torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(DEV)  # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    kc, vc = rnd(len(cases) * pages, nkv, page, dk, seed=1), rnd(len(cases) * pages, nkv, page, dv, seed=2)
+    table = torch.randperm(len(cases) * pages, generator=torch.Generator().manual_seed(3)).view(len(cases), pages).int().to(DEV)
+    bias = rnd(nq, far + 1, seed=4) if far else None
+
+    def run(which):
+        pos, seq, tiles, n = [], [], [], 0
+        for r in which:
+            first, count = cases[r]
+            tiles += [(n + t, min(32, count - t)) for t in range(0, count, 32)]
+            pos += range(first, first + count)
+            seq += [r] * count
+            n += count
+        q = torch.cat([rnd(cases[r][1], nq * dk, seed=10 + r) for r in which])
+        out = torch.full((n, nq * dv), float("nan"), device=DEV)
+        ops.attn_biased_tile(q, out, kc, vc, None, 0.5, i32(tiles), len(tiles), i32(pos), i32(seq), table, nq, nkv, dk, dv, page, dk ** -0.5, 30.0,
+                             bias, far, window, keep, chunk)
+        return out
+
+    alone = torch.cat([run([r]) for r in range(len(cases))])
+    assert not bool(alone.isnan().any())
+    assert torch.equal(run(list(range(len(cases))) * repeat), alone.repeat(repeat, 1))
