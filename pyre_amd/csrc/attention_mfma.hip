@@ -377,7 +377,7 @@ struct RopeIn {
   q, k_cache, v_cache, work, positions, seq_of_token, block_table, table_stride, part_acc, part_ml, counters, out, \
       nq, nkv, page_size, scale_log2, window
 
-template <int HD, bool STREAM_V, bool FUSED, bool ONE>
+template <int HD, bool STREAM_V, bool FUSED, bool ONE, int kTogether = 8>
 __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, const RopeIn& rope) {
   // The list's head and this block's row of it (the list holds one for every block of the launch) come together.
   const int4 head_of_list = work[0], item = work[2 * (1 + blockIdx.y)], place = work[2 * (1 + blockIdx.y) + 1];
@@ -444,7 +444,6 @@ __device__ __forceinline__ void attn_decode_work_block(PYRE_DECODE_WORK_PARAMS, 
       // of its own had those on their way 4.6 us after its start, now 3.1.)
       const bool own = qt == 0 && rope.write_kv && first + 4 * b * per <= last && last < first + 4 * (b + 1) * per;
       const int items = kItems * (own ? nheads + 2 : nheads), n_parts = rope.n_partials;
-      constexpr int kTogether = 8;
       struct Item {
         float4 x[2][kTogether], c4, s4;
         uint4 bias[2];
@@ -719,14 +718,17 @@ __global__ __launch_bounds__(256, 2) void attn_decode_work_kernel(PYRE_DECODE_WO
 // the sets that a wave keeps; heads of 64 have half as many bytes to a set and lose by it: 129 requests of 16,384 tokens of 14 such
 // heads 193 with two blocks, 205 with three of one set, 193 with three of two (of 1,024 to 4,096, ragged, 190 requests 18.7, 18.0 and 17.3,
 // 49.6, 46.1 and 46.5; 256 25.2, 21.2 and 22.8).
+// Heads of 32 have room for five blocks (92 registers), which eight parts of the product asked for together leave no registers for: they ask for
+// four together. 8 key/value heads of 32, three or four parts, us a launch with sums as their loads came, with eight and with four together: 70 requests
+// of 4,096 tokens 52, 60 and 50, 130 of 200 12.8, 14.6 and 11.1, in a window of 512 18.1, 20.6 and 16.6; with eight parts 52 and 52, 13.4 and 12.2, 18.6 and 18.8.
 template <int HD, bool STREAM_V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void attn_decode_work_rope_alone_kernel(
     PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
   attn_decode_work_block<HD, STREAM_V, true, false>(PYRE_DECODE_WORK_ARGS, rope);
 }
 template <int HD, bool STREAM_V>
-__global__ __launch_bounds__(256, 3) void attn_decode_work_rope_kernel(PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
-  attn_decode_work_block<HD, STREAM_V, true, (HD > 64)>(PYRE_DECODE_WORK_ARGS, rope);
+__global__ __launch_bounds__(256, HD <= 32 ? 5 : 3) void attn_decode_work_rope_kernel(PYRE_DECODE_WORK_PARAMS, RopeIn rope) {
+  attn_decode_work_block<HD, STREAM_V, true, (HD > 64), HD <= 32 ? 4 : 8>(PYRE_DECODE_WORK_ARGS, rope);
 }
 #undef PYRE_DECODE_WORK_PARAMS
 #undef PYRE_DECODE_WORK_ARGS

@@ -155,7 +155,7 @@ int pyre_attn_mfma_supports(int hd, int page_size, int nq, int nkv);
 // 4 (b + 1) per - 1 of its request, counted from the first chunk that the token sees, and the
 // nb blocks of a request cover all of them. The slots of the requests are disjoint runs of nb
 // within 0..capacity-1. `alone`: a compute unit runs one block at a time (for steps of so few
-// requests that a block per unit covers them); else two, or three in the form below. The launch has
+// requests that a block per unit covers them); else two, or three (heads of 32: five) in the form below. The launch has
 // `capacity` blocks per key/value head (and group of 16 query heads); blocks past the list's
 // end exit. Scratch: part_acc [capacity, items, 16, hd] and part_ml [capacity, items, 16, 2]
 // floats, counters [capacity, items] ints that are zero before the first call and are left

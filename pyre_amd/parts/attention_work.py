@@ -16,7 +16,8 @@ import numpy as np
 
 #: compute units of the device that is planned for when nobody says (an MI355X). An engine reads
 #: its device's number once (``Runtime.compute_units``) and plans with it; a unit runs one block of
-#: the decode kernel at a time, or two, or three of the form that finishes the q/k/v product
+#: the decode kernel at a time, or two, or three (heads of 32: five) of the form that finishes the
+#: q/k/v product
 DEFAULT_UNITS = 256
 #: keys per chunk of the decode kernel, and the fewest chunks a block is given if its request has them
 DECODE_CHUNK = 32

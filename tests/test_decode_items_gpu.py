@@ -21,3 +21,10 @@ def test_items_and_parts(nq, nkv, ks, bias, alone):
 def test_forms_that_share_a_unit(nq, nkv, hd, page, window, size):
     """Waves of no, one, two and many chunks, with one set of registers (heads of more than 64 elements) and with two."""
     check(nq, nkv, hd, page, 2, True, window, size, False)
+
+
+@pytest.mark.parametrize("ks", [1, 4, 5, 8, 12])
+@pytest.mark.parametrize("alone", [True, False])
+def test_parts_of_small_heads(ks, alone):
+    """Heads of 32 elements ask for four parts together where five blocks share a unit."""
+    check(7, 1, 32, 16, ks, True, 0, None, alone)
