@@ -1,17 +1,29 @@
 // out[m, n] = sum_k X[m, k] W[n, k] in bfloat16 with float32 sums, for the many rows of prompts and mixed steps
 // (pyre/model.py:84-87,92-94,133-139 with a whole prompt as their rows).
 //
-// The product is computed transposed, out^T = W X^T, on MFMA 32x32x16: A = 32 rows of W, B = 32 rows of X, both read
+// The product is computed transposed, out^T = W X^T, on MFMA 16x16x32: A = 16 rows of W, B = 16 rows of X, both read
 // along k as they are stored. A block owns BM rows of X and BN rows of W, its WM x WN waves a part of that each; k is
 // walked in stages of 64 through a ring of S slots in LDS that loads from memory fill directly, rows of 128 bytes whose
-// eight 16-byte pieces are exchanged among themselves by the row's number, so that the operand reads of 32 lanes spread
-// over all banks. The operands of the next 16 k are read while the present ones are multiplied; the one barrier of a stage
-// stands before its last 16 k: by then every wave has read the slot for the last time, so the loads of S stages further on
-// go into it, and the next stage's slot, which everybody has waited for, is read from.
+// eight 16-byte pieces are exchanged among themselves by the row's number, so that the operand reads of 16 lanes spread
+// over all banks.
 //
-// A block takes tiles one after the other until none is left: the first loads of the next tile are on their way before
-// the results of the present one are stored. The tiles that the 32 compute units of a die work on at a time are neighbours
-// (eight tiles along m by four along n): its L2 then serves every row several times.
+// What bounds it is the card's power: with random values the clocks fall to 1.4 to 1.9 GHz. MFMA 16x16x32 needs less of it than
+// 32x32x16 (nothing but products, operands in registers: 2.0 against 1.74 PFLOP/s; operands from LDS as here 1.67 against 1.54; the
+// sums have the same bits), and less when one operand stays as it is from one instruction to the next: 2 % more. What else counts
+// is that the matrix cores never wait, so the loop has no branch and no case: the loads run on from a tile into the block's next one, and behind
+// its last one they fetch a single line that nobody reads. 4,096 x 4,096 x 8,192 takes 184 us (205 with 32x32x16, a stage's loads
+// asked for at once and waits behind conditions), the 7B shape's gate/up at 2,048 rows 408 (455), its way down 202 (226).
+//
+// Where LDS has room for two stages only, a wave's rows of W are two parts of RT0 and RT1 tiles of sixteen, and a stage is four
+// steps: the first part against k 0..31 and 32..63 of the stage, then the second part. Every operand is in registers once, read when its
+// registers are free: a slot's first part and X from the last step of the stage before to the first one of its own, its second
+// part in the two steps between. Two barriers a stage, behind the first and the third step, free them one after the other for
+// the loads of two stages further on, which have a stage and a half to arrive. With three slots and more (RT0 = all) a stage is
+// two steps, the operands of the next one are read during the present one, and the one barrier between them, behind the slot's last
+// read, frees it for the loads of S stages further on.
+//
+// A block takes tiles one after the other until none is left. The tiles that the 32 compute units of a die work on at a time
+// are neighbours (eight tiles along m by four along n): its L2 then serves every row several times.
 //
 // kF32Out: float32 [ksplit][M][N], part `ks` of k; kGated: W = gate rows, then up rows; bfloat16 [M][N / 2], the gated
 // unit of the two; kPaged: X's rows lie in the pages of a cache, 32 consecutive positions of a request at a time; bfloat16 [N / ldo][M][ldo].
@@ -50,6 +62,14 @@ __device__ inline void barrier() {
   asm volatile("s_barrier" : : : "memory");
 }
 
+// Waits for the wave's reads from LDS and for all but its last N loads and stores (Many while `behind` counts down), then for the block.
+template <int N, int Many>
+__device__ inline void sync(int& behind) {
+  asm volatile("s_cmp_gt_i32 %0, 0\n\ts_cbranch_scc1 1f\n\ts_waitcnt vmcnt(%1)\n1:\n\ts_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_barrier"
+               : : "s"(behind), "n"(N), "n"(Many) : "memory", "scc");
+  behind = __builtin_amdgcn_readfirstlane(max(behind - 1, 0));
+}
+
 enum Out { kF32Out = 0, kGated = 1, kPaged = 2 };
 
 struct TileShape {
@@ -62,22 +82,22 @@ struct TileShape {
   int table_stride, page_size;
 };
 
-template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC>
-__global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16* __restrict__ X, long ldx,
-                                                                      const bf16* __restrict__ W, long ldw,
+template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC, int RT0 = BN / WN / 16>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16* __restrict__ X, long ldx, const bf16* __restrict__ W, long ldw,
                                                                       void* __restrict__ out, TileShape sh, GateShape act) {
   constexpr int NW = WM * WN, STAGE = (BM + BN) * ROW;
-  constexpr int LX = BM / 8 / NW, LW = BN / 8 / NW, L = LX + LW;      // loads (of eight rows) of a wave and stage
-  constexpr int CT = BM / WM / 32, RT = BN / WN / 32;                 // tiles of 32 rows of X and of W of a wave
-  constexpr int STORES = CT * (OUT == kGated ? (RT + 3) / 4 : OUT == kPaged ? (RT + 1) / 2 : RT) * 4;  // stores of a wave for a whole tile
-  constexpr int MF = RT * CT, RD = RT + CT;
-  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && (OUT != kGated || RT % 2 == 0), "rows divide over the waves");
+  constexpr int RT = BN / WN / 16, CT = BM / WM / 16, RT1 = RT - RT0;  // tiles of 16 rows of W and of X of a wave
+  constexpr int LX = (BM / 8 + NW - 1) / NW, LA = 2 * WN * RT0 / NW, LB = 2 * WN * RT1 / NW;  // loads (of eight rows) of a wave: X, W's parts
+  constexpr int EARLY = LX + LA, L = EARLY + LB;
+  constexpr bool two = RT1 > 0;
+  constexpr int STORES = CT * 2 * (OUT == kF32Out ? RT / 2 : OUT == kGated ? (RT + 7) / 8 : (RT + 3) / 4);
+  static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0 && 2 * WN * RT0 % NW == 0 && 2 * WN * RT1 % NW == 0 && RT % 2 == 0 &&
+                    (two ? L : (S - 2) * L) + STORES < 64 && (S - 1) * L + LB < 64, "rows divide over the waves, waits can be counted");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[S * STAGE + NW * 4096];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int c = lane & 31, half = lane >> 5, wm = wave % WM, wn = wave / WM;
+  const int c = lane & 15, quad = lane >> 4, wm = wave % WM, wn = wave / WM;
   const int inter = sh.N / 2;
 
-  // This die's run of the tiles (blocks are dealt to the eight dies in turn), of which this block takes every step'th.
   const int tiles = sh.mt * sh.nt * sh.parts, die = blockIdx.x & 7;
   const int share = tiles >> 3, rest = tiles & 7;
   const int begin = die * share + min(die, rest), end = begin + share + (die < rest ? 1 : 0);
@@ -87,24 +107,26 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
 
   const unsigned lds_base = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds)));
   const int lrow = lane >> 3, lpiece = lane & 7;
-  unsigned offx[LX], offw[LW];
-  const char *xb, *wb;
-  int im, in, ks, stages;
-  auto place = [&](int tile) {
-    const int per = sh.mt * sh.nt;
-    ks = tile / per;
+
+  struct At { int im, in, ks, stages; };
+  auto locate = [&](int tile) {
+    const int per = sh.mt * sh.nt, ks = tile / per;
     tile -= ks * per;
     const int group = tile / (GROUP * sh.nt), first = group * GROUP, gm = min(GROUP, sh.mt - first);
     tile -= GROUP * sh.nt * group;
-    im = first + tile % gm;
-    in = tile / gm;
-    const int kbeg = ks * sh.kper;
-    stages = (min(sh.K, kbeg + sh.kper) - kbeg) / BK;
+    return At{first + tile % gm, tile / gm, ks, (min(sh.K, (ks + 1) * sh.kper) - ks * sh.kper) / BK};
+  };
+  unsigned offx[LX], offw[LA + LB];
+  const char *xb, *wb;
+  int coming = t, left;  // the tile whose stages are being asked for, and how many of them are left
+  auto place = [&](int tile) {
+    const At at_tile = locate(tile);
+    left = at_tile.stages;
     // Rows past the end are the last row once more; nobody stores what comes of them.
 #pragma unroll
     for (int i = 0; i < LX; ++i) {
-      const int row = 8 * (NW * i + wave) + lrow;
-      int at = min(im * BM + row, sh.M - 1);
+      const int row = 8 * ((NW * i + wave) % (BM / 8)) + lrow;  // (where they do not divide, some are asked for twice)
+      int at = min(at_tile.im * BM + row, sh.M - 1);
       if (OUT == kPaged) {  // (positions behind the request's last one are the last one once more)
         const int* const group = sh.groups + 3 * (at / 32);
         const int pos = min(group[1] + at % 32, group[2]);
@@ -113,182 +135,232 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
       offx[i] = static_cast<unsigned>(at) * static_cast<unsigned>(2 * ldx) + 16 * (lpiece ^ ((row >> 1) & 7));
     }
 #pragma unroll
-    for (int i = 0; i < LW; ++i) {
-      const int row = 8 * (NW * i + wave) + lrow;
+    for (int i = 0; i < LA + LB; ++i) {
+      const int lines = i < LA ? 16 * RT0 : 16 * RT1, at = 8 * (NW * (i < LA ? i : i - LA) + wave) + lrow;  // of a wave's part; in the part
+      const int row = at / lines * 16 * RT + (i < LA ? 0 : 16 * RT0) + at % lines;
       int n;
-      if (OUT == kGated) {  // 32 gate rows, then the up rows of the same features
-        const int f = in * (BN / 2) + 32 * (row >> 6) + (row & 31);
-        n = min(f, inter - 1) + ((row >> 5) & 1) * sh.up;
+      if (OUT == kGated) {  // 16 gate rows, then the up rows of the same features
+        const int f = at_tile.in * (BN / 2) + 16 * (row >> 5) + (row & 15);
+        n = min(f, inter - 1) + ((row >> 4) & 1) * sh.up;
       } else {
-        n = min(in * BN + row, sh.N - 1);
+        n = min(at_tile.in * BN + row, sh.N - 1);
       }
-      offw[i] = static_cast<unsigned>(n) * static_cast<unsigned>(2 * ldw) + 16 * (lpiece ^ ((row >> 1) & 7));
+      offw[i] = static_cast<unsigned>(n) * static_cast<unsigned>(2 * ldw) + 16 * (lpiece ^ ((at >> 1) & 7));
     }
-    xb = reinterpret_cast<const char*>(X + kbeg);
-    wb = reinterpret_cast<const char*>(W + kbeg);
+    xb = reinterpret_cast<const char*>(X + at_tile.ks * sh.kper);
+    wb = reinterpret_cast<const char*>(W + at_tile.ks * sh.kper);
   };
+  // A slot: W's first parts of all waves, their second parts, X.
   auto issue = [&](int i, unsigned slot_base) {
-    if (i < LX) load_to_lds(xb, offx[i < LX ? i : 0], slot_base + (NW * i + wave) * 1024);
-    else load_to_lds(wb, offw[i < LX ? 0 : i - LX], slot_base + BM * ROW + (NW * (i - LX) + wave) * 1024);
+    if (i < LA) load_to_lds(wb, offw[i < LA ? i : 0], slot_base + (NW * i + wave) * 1024);
+    else if (i < EARLY) load_to_lds(xb, offx[i < LA || i >= EARLY ? 0 : i - LA], slot_base + BN * ROW + (NW * (i - LA) + wave) % (BM / 8) * 1024);
+    else load_to_lds(wb, offw[i < EARLY ? 0 : i - LX], slot_base + WN * RT0 * 16 * ROW + (NW * (i - EARLY) + wave) * 1024);
   };
-  auto begin_tile = [&]() {
+  // On to the next stage to be asked for. Behind the last one of all it is that one again: what a slot holds then is not read,
+  // and every stage has the same loads before and behind it.
+  int advance = ROW;
+  auto dry = [&]() {
+    if (advance) xb -= ROW, wb -= ROW;
+    advance = 0;
+    left = 1;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      if (s < stages) {
+    for (int i = 0; i < LX; ++i) offx[i] = 0;
 #pragma unroll
-        for (int i = 0; i < L; ++i) issue(i, lds_base + s * STAGE);
-        xb += ROW;
-        wb += ROW;
-      }
+    for (int i = 0; i < LA + LB; ++i) offw[i] = 0;
+  };
+  auto next_stage = [&]() {
+    if (left == 0) {
+      if (coming + step < end) place(coming += step);
+      else dry();
     }
+    --left;
   };
 
-  const unsigned char* const xrow = lds + (wm * 32 * CT + c) * ROW;
-  const unsigned char* const wrow = lds + BM * ROW + (wn * 32 * RT + c) * ROW;
-  const int swz = (c >> 1) & 7;
-  bf16x8 a[2][RT], b[2][CT];
-  auto read = [&](int x, int kk, int buf, int slot) {
-    const int at = slot * STAGE + 16 * ((2 * kk + half) ^ swz);
-    if (x < RT) a[buf][x < RT ? x : 0] = *reinterpret_cast<const bf16x8*>(wrow + at + x * 32 * ROW);
-    else b[buf][x < RT ? 0 : x - RT] = *reinterpret_cast<const bf16x8*>(xrow + at + (x - RT) * 32 * ROW);
+  const int piece = 16 * (quad ^ ((c >> 1) & 7));
+  const unsigned char* const row0 = lds + (wn * RT0 * 16 + c) * ROW;
+  const unsigned char* const row1 = lds + (WN * RT0 + wn * RT1) * 16 * ROW + c * ROW;
+  const unsigned char* const rowx = lds + BN * ROW + (wm * CT * 16 + c) * ROW;
+  bf16x8 a0[2][RT0], a1[2][two ? RT1 : 1], b[2][CT];
+  auto get = [&](const unsigned char* row, int x, int kk, int slot) {
+    return *reinterpret_cast<const bf16x8*>(row + (piece ^ (64 * kk)) + slot * STAGE + x * 16 * ROW);
+  };
+  auto read0 = [&](int x, int kk, int slot) {  // of the first part and X
+    if (x < RT0) a0[kk][x < RT0 ? x : 0] = get(row0, x, kk, slot);
+    else b[kk][x < RT0 ? 0 : x - RT0] = get(rowx, x - RT0, kk, slot);
   };
 
   place(t);
-  begin_tile();
-  bool stored = false;  // STORES stores of every wave came after the first S stages' loads
-  while (true) {
-    if (stages < S) wait_loads<0>();
-    else if (stored) wait_loads<(S - 1) * L + STORES>();
-    else wait_loads<(S - 1) * L>();
-    barrier();
 #pragma unroll
-    for (int x = 0; x < RD; ++x) read(x, 0, 0, 0);
-    f32x16 acc[RT][CT];
+  for (int x = 0; x < S; ++x) {
+    next_stage();
+#pragma unroll
+    for (int i = 0; i < L; ++i) issue(i, lds_base + x * STAGE);
+    xb += advance, wb += advance;
+  }
+  wait_loads<LB + (S - 1) * L>();
+  barrier();
+  int behind = 0;  // of the next waits, so many have the stores of the tile before behind their loads
+  int slot = 0;
+  while (true) {
+    const At here = locate(t);
+#pragma unroll
+    for (int x = 0; x < RT0 + CT; ++x) read0(x, 0, slot);
+    f32x4 acc[RT][CT];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-      for (int q = 0; q < CT; ++q)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[r][q][i] = 0.f;
+      for (int q = 0; q < CT; ++q) acc[r][q] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    int slot = 0;
-    for (int st = 0; st < stages; ++st) {
+#pragma nounroll
+    for (int st = 0; st < here.stages; ++st) {
       const int next = slot + 1 == S ? 0 : slot + 1;
+      // Every other row of W takes X from the other end: an operand less that changes.
+      if constexpr (two) {
 #pragma unroll
-      for (int kk = 0; kk < BK / 16; ++kk) {
-        const int cur = kk & 1, nxt = cur ^ 1;
-        const bool last = kk == BK / 16 - 1;
-        bool more = false;
-        if (last) {
-          asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
-          if (st + S > stages) wait_loads<0>();
-          else if (stored && st < S - 1) wait_loads<(S - 2) * L + STORES>();
-          else wait_loads<(S - 2) * L>();
-          barrier();
-          more = st + S < stages;
-        }
-#pragma unroll
-        for (int g = 0; g < MF; ++g) {
-#pragma unroll
-          for (int x = 0; x < RD; ++x)
-            if ((RD > MF ? x * MF / RD : x) == g) read(x, last ? 0 : kk + 1, nxt, last ? next : slot);
-          acc[g / CT][g % CT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[cur][g / CT], b[cur][g % CT], acc[g / CT][g % CT], 0, 0, 0);
+        for (int g = 0; g < RT0 * CT; ++g) {
+          const int r = g / CT, q = r & 1 ? CT - 1 - g % CT : g % CT;
+          acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[0][r], b[0][q], acc[r][q], 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
-          if (last && more) {
-#pragma unroll
-            for (int i = 0; i < L; ++i)
-              if (i * MF / L == g) issue(i, lds_base + slot * STAGE);
-          }
+          if (g < RT0 + CT) read0(g, 1, slot);
         }
-        if (last && more) {
-          xb += ROW;
-          wb += ROW;
+        sync<L, L + STORES>(behind);
+        next_stage();
+#pragma unroll
+        for (int g = 0; g < RT0 * CT; ++g) {
+          const int r = g / CT, q = r & 1 ? CT - 1 - g % CT : g % CT;
+          acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[1][r], b[1][q], acc[r][q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (g < RT1) a1[0][g < RT1 ? g : 0] = get(row1, g, 0, slot);
+#pragma unroll
+          for (int i = 0; i < EARLY / 2; ++i)
+            if ((i + 1) * RT0 * CT / (EARLY / 2 + 1) == g) issue(i, lds_base + slot * STAGE);
+        }
+#pragma unroll
+        for (int g = 0; g < RT1 * CT; ++g) {
+          const int r = g / CT, q = r & 1 ? CT - 1 - g % CT : g % CT;
+          acc[RT0 + r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[0][r], b[0][q], acc[RT0 + r][q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (g < RT1) a1[1][g < RT1 ? g : 0] = get(row1, g, 1, slot);
+#pragma unroll
+          for (int i = EARLY / 2; i < EARLY; ++i)
+            if ((i - EARLY / 2 + 1) * RT1 * CT / (EARLY - EARLY / 2 + 1) == g) issue(i, lds_base + slot * STAGE);
+        }
+        sync<L, L + STORES>(behind);
+#pragma unroll
+        for (int g = 0; g < RT1 * CT; ++g) {
+          const int r = g / CT, q = r & 1 ? CT - 1 - g % CT : g % CT;
+          acc[RT0 + r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[1][r], b[1][q], acc[RT0 + r][q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (g < RT0 + CT) read0(g, 0, next);
+#pragma unroll
+          for (int i = EARLY; i < L; ++i)
+            if ((i - EARLY + 1) * RT1 * CT / (LB + 1) == g) issue(i, lds_base + slot * STAGE);
+        }
+      } else {
+#pragma unroll
+        for (int g = 0; g < RT * CT; ++g) {
+          const int r = g / CT, q = r & 1 ? CT - 1 - g % CT : g % CT;
+          acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[0][r], b[0][q], acc[r][q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (g < RT + CT) read0(g, 1, slot);
+        }
+        sync<(S - 2) * L, (S - 2) * L + STORES>(behind);
+        next_stage();
+#pragma unroll
+        for (int g = 0; g < RT * CT; ++g) {
+          const int r = g / CT, q = r & 1 ? CT - 1 - g % CT : g % CT;
+          acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[1][r], b[1][q], acc[r][q], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (g < RT + CT) read0(g, 0, next);
+#pragma unroll
+          for (int i = 0; i < L; ++i)
+            if (i * RT * CT / L == g) issue(i, lds_base + slot * STAGE);
         }
       }
+      xb += advance, wb += advance;
       slot = next;
     }
 
-    // The next tile's first loads, then this one's results. Everybody has read every slot for the last time; what the
-    // last step read ahead is not used.
-    const int m0 = im * BM, n0 = in * BN, part = ks, fcol = in * (BN / 2);
+    // (What the last step read ahead is read again.)
+    const int m0 = here.im * BM, n0 = here.in * BN, part = here.ks, fcol = here.in * (BN / 2);
     t += step;
     const bool again = t < end;
-    if (again) {
-      place(t);
-      begin_tile();
-    }
-    stored = m0 + BM <= sh.M && (OUT == kGated ? fcol + BN / 2 <= inter : n0 + BN <= sh.N);
-    // acc[r][q][4 p + j]: row 32 (RT wn + r) + 8 p + 4 half + j of the tile of W, row 32 (CT wm + q) + c of X. A piece of
+    const bool stored = m0 + BM <= sh.M && (OUT == kGated ? fcol + BN / 2 <= inter : n0 + BN <= sh.N);  // STORES stores a wave
+    // acc[r][q][j]: row 16 (RT wn + r) + 4 quad + j of the tile of W, row 16 (CT wm + q) + c of X. A piece of
     // 32 rows of 128 bytes at a time goes to the wave's LDS, its 16-byte parts exchanged by the row's number, and from
     // there eight lanes to a row to memory.
     unsigned char* const own = lds + S * STAGE + wave * 4096;
+    constexpr int WIDE = OUT == kF32Out ? 2 : OUT == kGated ? 8 : 4;  // tiles of W that make a piece
 #pragma unroll
-    for (int q = 0; q < CT; ++q)
+    for (int q = 0; q < CT; q += 2)
 #pragma unroll
-      for (int r = 0; r < RT; r += OUT == kF32Out ? 1 : 2) {
-        if (OUT == kGated && r % 4 == 2) continue;  // written with the pair before it
+      for (int r = 0; r < RT; r += WIDE) {
         asm volatile("" : : : "memory");
-        if (OUT == kGated) {
-          auto finish = [&](auto silu_) {
-            constexpr bool silu = decltype(silu_)::value;
 #pragma unroll
-            for (int pair = 0; pair < 2; ++pair) {
-              const int g = r + 2 * pair;
-              if (g >= RT) continue;
+        for (int x = 0; x < 2; ++x) {
+          if (q + x >= CT) continue;
+          const int qx = q + x < CT ? q + x : 0;
+          unsigned char* const line = own + (16 * x + c) * 128;
+          const int swz = (c >> 1) & 7;
+          if (OUT == kGated) {
+            auto finish = [&](auto silu_) {
+              constexpr bool silu = decltype(silu_)::value;
 #pragma unroll
-              for (int p = 0; p < 4; ++p) {
+              for (int u = 0; u < 4; ++u) {
+                const int g = r + 2 * u;
+                if (g >= RT) continue;
                 float y[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                  const float gate = acc[g < RT ? g : 0][q][4 * p + j], up = acc[g + 1 < RT ? g + 1 : 0][q][4 * p + j];
+                  const float gate = acc[g < RT ? g : 0][qx][j], up = acc[g + 1 < RT ? g + 1 : 0][qx][j];
                   y[j] = silu ? silu_unit(gate, up) : gated_unit(gate, up, act);
                 }
-                *reinterpret_cast<uint2*>(own + c * 128 + 16 * ((4 * pair + p) ^ (c & 7)) + 8 * half) =
+                *reinterpret_cast<uint2*>(line + 16 * ((2 * u + (quad >> 1)) ^ swz) + 8 * (quad & 1)) =
                     uint2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
               }
+            };
+            if (is_silu(act)) finish(std::true_type{});
+            else finish(std::false_type{});
+          } else if (OUT == kPaged) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              if (r + u >= RT) continue;
+              const f32x4& y = acc[r + u < RT ? r + u : 0][qx];
+              *reinterpret_cast<uint2*>(line + 16 * ((2 * u + (quad >> 1)) ^ swz) + 8 * (quad & 1)) = uint2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
             }
-          };
-          if (is_silu(act)) finish(std::true_type{});
-          else finish(std::false_type{});
-        } else if (OUT == kPaged) {
+          } else {
 #pragma unroll
-          for (int pair = 0; pair < 2; ++pair) {
-            if (r + pair >= RT) continue;
-            const f32x16& t = acc[r + pair < RT ? r + pair : 0][q];
-#pragma unroll
-            for (int p = 0; p < 4; ++p)
-              *reinterpret_cast<uint2*>(own + c * 128 + 16 * ((4 * pair + p) ^ (c & 7)) + 8 * half) =
-                  uint2{pack_bf16x2(t[4 * p], t[4 * p + 1]), pack_bf16x2(t[4 * p + 2], t[4 * p + 3])};
+            for (int u = 0; u < 2; ++u) *reinterpret_cast<f32x4*>(line + 16 * ((4 * u + quad) ^ swz)) = acc[r + u][qx];
           }
-        } else {
-#pragma unroll
-          for (int p = 0; p < 4; ++p)
-            *reinterpret_cast<f32x4*>(own + c * 128 + 16 * ((2 * p + half) ^ (c & 7))) =
-                f32x4{acc[r][q][4 * p], acc[r][q][4 * p + 1], acc[r][q][4 * p + 2], acc[r][q][4 * p + 3]};
         }
         asm volatile("" : : : "memory");
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int row = 8 * i + lrow, m = m0 + 32 * (wm * CT + q) + row;
-          const uint4 y = *reinterpret_cast<const uint4*>(own + row * 128 + 16 * (lpiece ^ (row & 7)));
+          if (q + 1 >= CT && i >= 2) continue;  // sixteen rows are left
+          const int row = 8 * i + lrow, m = m0 + 16 * (wm * CT + q) + row;
+          const uint4 y = *reinterpret_cast<const uint4*>(own + row * 128 + 16 * (lpiece ^ ((row >> 1) & 7)));
           if (OUT == kGated) {
-            const int f = fcol + 16 * (wn * RT + r) + 8 * lpiece;
+            const int f = fcol + 8 * (wn * RT + r) + 8 * lpiece;
             if (!stored && (m >= sh.M || f >= inter)) continue;
-            if (RT - r < 4 && lpiece >= 4) continue;  // a lone pair of tiles: half a row
+            if (lpiece >= RT - r) continue;  // a part of a row
             *reinterpret_cast<uint4*>(static_cast<bf16*>(out) + static_cast<size_t>(m) * sh.ldo + f) = y;
           } else if (OUT == kPaged) {
-            const int n = n0 + 32 * (wn * RT + r) + 8 * lpiece;
+            const int n = n0 + 16 * (wn * RT + r) + 8 * lpiece;
             if (!stored && (m >= sh.M || n >= sh.N)) continue;
-            if (RT - r < 2 && lpiece >= 4) continue;  // a lone tile: half a row
+            if (RT - r < 4 && lpiece >= 4) continue;  // half a row
             *reinterpret_cast<uint4*>(static_cast<bf16*>(out) + n / sh.ldo * sh.plane + static_cast<size_t>(m) * sh.ldo + n % sh.ldo) = y;
           } else {
-            const int n = n0 + 32 * (wn * RT + r) + 4 * lpiece;
+            const int n = n0 + 16 * (wn * RT + r) + 4 * lpiece;
             if (!stored && (m >= sh.M || n >= sh.N)) continue;
             *reinterpret_cast<uint4*>(static_cast<float*>(out) + part * sh.plane + static_cast<size_t>(m) * sh.ldo + n) = y;
           }
         }
       }
-    if (!again) break;
+    if (!again) {
+      wait_loads<0>();  // (nothing is to arrive in LDS that is another block's by then)
+      break;
+    }
+    behind = __builtin_amdgcn_readfirstlane(stored ? (two ? 3 : S - 1) : 0);
     if (!stored) wait_loads<0>();  // an edge's stores are not counted
   }
 }
@@ -298,35 +370,32 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
 
 namespace {
 
-// What a tile size takes, in microseconds: a launch, a round of blocks (one a compute unit) and a stage of its tiles, a
-// megabyte of results and of weights. Fitted to 24 row counts from 72 to 3,000 on nine weights (the 1.5B and 7B shapes'
-// q/k/v, attention output, gate/up and way down, and two of 8,960 x 1,536 and 5,560 x 3,584), each with 1 to 6 parts of k,
-// weights from memory: 2 to 5 % off on average. What it chooses takes 1.6 % (gated: 0.7 %) longer on average than the best
-// of all sizes and parts measured. Larger tiles need fewer bytes a product; smaller ones fill the last round better.
+// What a tile size takes, in microseconds: a launch, a round of blocks (one a compute unit), a stage of its tiles, the same again
+// where every unit has a tile (the card's power then leaves lower clocks), a megabyte of results and of weights. Fitted to 25 row
+// counts from 72 to 3,000 on nineteen weights (the 1.5B and 7B shapes' q/k/v, attention output, gate/up and way down, and others of
+// 64 to 1,536 k), each with 1 to 6 parts of k, weights from memory and launches one behind the other: 2 to 7 % off
+// on average. What it chooses takes 0.9 % (gated: 0.2 %) longer on average than the best of all sizes and parts measured. Larger
+// tiles need fewer bytes a product; smaller ones fill the last round better. A product cut in two (see TileChoice) is two of these
+// times: over 39 row counts from 257 to 12,001 on nine weights the cuts so chosen save 0.7 % on average, 1.4 % on the 7B shape's.
 struct TileCost {
   int bm, bn;
-  double launch, round, stage, out_mb, weight_mb;
+  double launch, round, stage, full, out_mb, weight_mb;
 };
-constexpr TileCost kSums[] = {{256, 256, 0.0, 3.7, 1.217, 0.167, 0.089},
-                              {256, 192, 0.6, 1.8, 1.041, 0.183, 0.107},
-                              {128, 192, 2.0, 2.1, 0.605, 0.180, 0.057},
-                              {128, 128, 1.9, 1.3, 0.471, 0.194, 0.057},
-                              {64, 128, 2.3, 1.5, 0.360, 0.168, 0.058}};
-constexpr TileCost kUnits[] = {{256, 256, 3.1, 0.0, 1.471, 0.291, 0.000},
-                               {192, 256, 5.0, 0.0, 1.219, 0.246, 0.033},
-                               {192, 192, 3.8, 1.5, 1.015, 0.400, 0.035},
-                               {128, 256, 3.9, 0.0, 0.903, 0.430, 0.018},
-                               {96, 256, 4.7, 1.1, 0.654, 0.660, 0.050},
-                               {96, 192, 4.1, 0.9, 0.586, 0.768, 0.041}};
+constexpr TileCost kSums[] = {{256, 256, 1.4, 5.0, 0.947, 0.360, 0.095, 0.015},
+                              {256, 192, 1.9, 3.8, 0.743, 0.301, 0.095, 0.006},
+                              {128, 192, 2.5, 2.0, 0.392, 0.251, 0.104, 0.065},
+                              {128, 128, 2.8, 1.4, 0.290, 0.209, 0.086, 0.053},
+                              {64, 128, 2.9, 1.0, 0.235, 0.111, 0.065, 0.049}};
+constexpr TileCost kUnits[] = {{256, 256, 3.4, 2.8, 0.871, 0.499, 0.093, 0.028},
+                               {192, 256, 3.2, 2.6, 0.630, 0.446, 0.081, 0.047},
+                               {192, 192, 3.1, 2.6, 0.680, 0.256, 0.093, 0.029},
+                               {128, 256, 2.8, 2.1, 0.438, 0.339, 0.065, 0.085},
+                               {96, 256, 2.9, 1.8, 0.319, 0.377, 0.051, 0.096},
+                               {96, 192, 3.0, 1.7, 0.251, 0.306, 0.042, 0.077}};
 // Paged rows: the sums' times (their results are half as many bytes); the product is short in k, what counts are its rounds.
 constexpr TileCost kPages[] = {kSums[0], kSums[2], kSums[3]};
 constexpr int kMaxParts = 6;
 constexpr double kReadMb = 0.2;              // the consumer's reading of a further part, a megabyte
-// A product cut in two (see TileChoice) pays for a second launch, and full rounds run at lower clocks than a nearly empty one:
-// of twenty sizes, what these sums promise came out 4.5 % lower on average, so a cut has to look that much better. One launch
-// against two, us: the 7B shape's gate/up 440 -> 417 at 1,777 rows and 278 -> 259 at 1,000, its q/k/v 135 -> 127 at 4,000 and
-// 353 -> 339 at 12,001, the 1.5B shape's gate/up 116 -> 108 at 2,048; not cut, the former's gate/up at 800 rows (262 against 281).
-constexpr double kSecondLaunchUs = 2.0, kCutCost = 1.045;
 constexpr double kMostPartsBytes = 536870912.0;  // parts of k together take no more scratch memory than this
 
 // Which tiles, in how many parts of k; and, where that leaves the last round of blocks nearly empty, a cut: tiles of `cfg`
@@ -344,7 +413,7 @@ double tile_us(const TileCost& c, int bytes, int M, int N, int K, int kper, int 
   const double tiles = static_cast<double>((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn) * parts;
   const double rounds = static_cast<double>(static_cast<long>((tiles + units - 1) / units));
   const double out_mb = rows_mb * bytes * parts;
-  return c.launch + rounds * (c.round + kper / BK * c.stage) + out_mb * c.out_mb + 2e-6 * N * static_cast<double>(K) * c.weight_mb +
+  return c.launch + rounds * (c.round + kper / BK * c.stage) + tiles / units * (kper / BK) * c.full + out_mb * c.out_mb + 2e-6 * N * static_cast<double>(K) * c.weight_mb +
          (parts - 1) * 4.0 * rows_mb * kReadMb;
 }
 
@@ -369,10 +438,10 @@ TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, 
           if (cut < 1 || cut >= (by_rows ? mt : nt)) continue;
           const int m1 = by_rows ? static_cast<int>(cut) * c.bm : M, n1 = by_rows ? N : static_cast<int>(cut) * c.bn;
           const int m2 = by_rows ? M - m1 : M, n2 = by_rows ? N : N - n1;
-          const double first = kCutCost * (tile_us(c, bytes, m1, n1, K, kper, parts) + kSecondLaunchUs);
+          const double first = tile_us(c, bytes, m1, n1, K, kper, parts);
           if (first >= best.us) continue;
           for (int j = 0; j < n_costs; ++j) {
-            const double both = first + kCutCost * tile_us(costs[j], bytes, m2, n2, K, kper, parts);
+            const double both = first + tile_us(costs[j], bytes, m2, n2, K, kper, parts);
             if (both < best.us) best = TileChoice{i, parts, kper, both, by_rows ? m1 : gated ? n1 / 2 : n1, by_rows, j};
           }
         }
@@ -387,7 +456,7 @@ struct Region {
   int m0, M, n0, N, all_m, all_n;
 };
 
-template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC>
+template <int BM, int BN, int WM, int WN, int S, int OUT, int OCC, int RT0 = BN / WN / 16>
 void launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, const Region& r, int K, int kper, int parts, GateShape act,
             hipStream_t stream) {
   const bool gated = OUT == kGated;
@@ -397,7 +466,7 @@ void launch(const bf16* X, long ldx, const bf16* W, long ldw, void* out, const R
   const int tiles = sh.mt * sh.nt * parts;
   const size_t at = static_cast<size_t>(r.m0) * r.all_n + r.n0;
   void* to = gated ? static_cast<void*>(static_cast<bf16*>(out) + at) : static_cast<void*>(static_cast<float*>(out) + at);
-  hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, S, OUT, OCC>), dim3(tiles < compute_units() ? tiles : compute_units()),
+  hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WM, WN, S, OUT, OCC, RT0>), dim3(tiles < compute_units() ? tiles : compute_units()),
                      dim3(64 * WM * WN), 0, stream, X + static_cast<size_t>(r.m0) * ldx, ldx, W + static_cast<size_t>(r.n0) * ldw, ldw, to,
                      sh, act);
 }
@@ -452,11 +521,11 @@ extern "C" int pyre_gemm_tile_bf16(const void* X, long ldx, const void* W, long 
   const bf16* w = static_cast<const bf16*>(W);
   const GateShape act{};
   launch_regions(c, M, N, [&](int cfg, const Region& r) {
-    if (cfg == 0) launch<256, 256, 4, 2, 2, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
-    else if (cfg == 1) launch<256, 192, 4, 2, 2, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
-    else if (cfg == 2) launch<128, 192, 2, 2, 3, kF32Out, 1>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
-    else if (cfg == 3) launch<128, 128, 2, 4, 4, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
-    else launch<64, 128, 1, 4, 6, kF32Out, 1>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    if (cfg == 0) launch<256, 256, 4, 2, 2, kF32Out, 2, 4>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else if (cfg == 1) launch<256, 192, 4, 2, 2, kF32Out, 2, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else if (cfg == 2) launch<128, 192, 4, 2, 3, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else if (cfg == 3) launch<128, 128, 4, 2, 4, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
+    else launch<64, 128, 2, 4, 5, kF32Out, 2>(x, ldx, w, ldw, out, r, K, c.kper, parts, act, stream);
   });
   return check_launch("gemm_tile_bf16");
 }
@@ -471,12 +540,12 @@ extern "C" int pyre_gemm_tile_glu_bf16(const void* X, long ldx, const void* W, l
   const bf16* w = static_cast<const bf16*>(W);
   const GateShape act{limit, slope, shift, cubic};
   launch_regions(c, M, two_i / 2, [&](int cfg, const Region& r) {
-    if (cfg == 0) launch<256, 256, 4, 2, 2, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
-    else if (cfg == 1) launch<192, 256, 2, 4, 2, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
-    else if (cfg == 2) launch<192, 192, 2, 3, 2, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
-    else if (cfg == 3) launch<128, 256, 2, 2, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
-    else if (cfg == 4) launch<96, 256, 1, 4, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
-    else launch<96, 192, 1, 3, 3, kGated, 1>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    if (cfg == 0) launch<256, 256, 4, 2, 2, kGated, 2, 4>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 1) launch<192, 256, 2, 4, 2, kGated, 2, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 2) launch<192, 192, 2, 3, 2, kGated, 2, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 3) launch<128, 256, 2, 4, 2, kGated, 2, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else if (cfg == 4) launch<96, 256, 2, 4, 2, kGated, 2, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
+    else launch<96, 192, 3, 2, 3, kGated, 2>(x, ldx, w, ldw, out, r, K, c.kper, 1, act, stream);
   });
   return check_launch("gemm_tile_glu_bf16");
 }
@@ -501,8 +570,8 @@ extern "C" int pyre_gemm_tile_paged_bf16(const void* X, int pages, int page_size
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, stream, static_cast<const bf16*>(X), static_cast<long>(row),
                        static_cast<const bf16*>(W), static_cast<long>(K), out, sh, GateShape{});
   };
-  if (cfg == 0) go(gemm_tile_kernel<256, 256, 4, 2, 2, kPaged, 2>, 512);
-  else if (cfg == 1) go(gemm_tile_kernel<128, 192, 2, 2, 3, kPaged, 1>, 256);
-  else go(gemm_tile_kernel<128, 128, 2, 2, 4, kPaged, 1>, 256);
+  if (cfg == 0) go(gemm_tile_kernel<256, 256, 4, 2, 2, kPaged, 2, 4>, 512);
+  else if (cfg == 1) go(gemm_tile_kernel<128, 192, 4, 2, 3, kPaged, 2>, 512);
+  else go(gemm_tile_kernel<128, 128, 2, 4, 4, kPaged, 2>, 512);
   return check_launch("gemm_tile_paged_bf16");
 }

@@ -159,6 +159,26 @@ def test_every_form_behind_a_cut(gated, tile):
     check_product(*size, gated, None, tile)
 
 
+@pytest.mark.parametrize("m,n,k", [(2100, 25616, 64), (2300, 24576, 128), (1800, 25600, 192), (3000, 16400, 320)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_blocks_that_walk_short_tiles(m, n, k, gated):
+    """Several tiles a block, of no more stages than its ring has slots: what is asked for ahead is the next tiles'."""
+    from pyre_amd.hip import ops
+
+    x, w = rnd(m, k, seed=8), rnd(n, k, seed=9, scale=0.2)
+    want = x.double() @ w.double().T
+    if gated:
+        out = torch.full((m, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops.gemm_tile_glu_bf16(x, w, out, m)
+        want = torch.nn.functional.silu(want[:, :n // 2]) * want[:, n // 2:]
+        # half a unit of the 8 bits that bfloat16 keeps, and the sums' rounding through factors that grow with the sums
+        assert bool(((out.double() - want).abs() <= want.abs() * 2.0 ** -8 + 64 * bound(k)).all())
+    else:
+        out = torch.full((1, m, n), float("nan"), device=DEV)
+        ops.gemm_tile_bf16(x, w, out, m, 1)
+        assert float((out[0].double() - want).abs().max()) <= bound(k) * float(want.std()) * 4
+
+
 @pytest.mark.parametrize("unit", [None, (7.0, 1.702, 1.0), (0.0, float("inf"), 0.0, 0.0)])
 @pytest.mark.parametrize("m,inter,k", [(1, 8, 64), (70, 8960, 128), (130, 18944, 64), (200, 18936, 64), (257, 136, 256), (300, 8960, 64),
                                        (520, 18944, 64), (1100, 1000, 128), (2049, 8968, 64)])
