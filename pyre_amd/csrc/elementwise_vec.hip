@@ -14,11 +14,18 @@ namespace {
 // ---------------------------------------------------------------------------
 // add + RMSNorm, one block per row, the row kept in registers between the passes.
 // ---------------------------------------------------------------------------
-constexpr int kNormMaxVec = 8;  // float4 per thread
+constexpr int kNormMaxVec = 8;  // float4 per thread of 256
 
 // THREADS = 256 keeps up to 8192 elements of a row in registers and suits many rows;
 // THREADS = 1024 gives a short row one float4 per thread, so that all loads of a
 // decode step's few rows are in flight at once.
+//
+// A step of few rows is a chain of trips through memory with next to no bytes: whatever is asked for is asked for at
+// once, the gain among it, the reduction is exchanges between lanes and one trip through LDS, and what the first loads need
+// comes with the launch (arguments in that order). In a graph, us at 10 parts: 1,536 elements 3.1 -> 2.7 at one row, 4.65 -> 3.3 at 190;
+// 3,584 elements 3.8 -> 3.5 and 7.7 -> 4.9. Rows get 1024 threads up to one row a compute unit (190 rows with
+// 256 threads 4.1 and 6.8; at 400 rows the two are alike). STREAM asks for four parts at a time (566 rows, 10 parts, one at a time:
+// 14.0 -> 9.8 and 26.9 -> 20.6); it has the waves that hide the gain.
 //
 // The sum of squares is added up in an order that the row's width alone fixes, whichever
 // variant runs: a row wider than 1024 elements is summed as 1024 threads would (thread t
@@ -28,29 +35,31 @@ constexpr int kNormMaxVec = 8;  // float4 per thread
 // 256 j. A position's result therefore does not depend on how many rows share the step.
 template <typename TD, typename TG, typename TO, int THREADS, int VIRT, bool STREAM>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
-    float* __restrict__ resid, const TD* __restrict__ delta, int n_partials, size_t partial_stride,
-    const float* __restrict__ bias, const TG* __restrict__ gain, TO* __restrict__ out, const int* __restrict__ rows, int hidden,
-    float eps) {
-  __shared__ float scratch[16];
+    float* __restrict__ resid, const TD* __restrict__ delta, int n_partials, int hidden, size_t partial_stride, const int* __restrict__ rows,
+    const TG* __restrict__ gain, TO* __restrict__ out, float eps, const float* __restrict__ bias) {
+  __shared__ __attribute__((aligned(16))) float scratch[16];
   const int r_out = blockIdx.x, r_in = rows ? rows[r_out] : r_out;
   const size_t in_off = static_cast<size_t>(r_in) * hidden;
   const int nvec = hidden / 4;
-  float4 v[kNormMaxVec];
+  constexpr int ITEMS = kNormMaxVec * 256 / THREADS;
+  float4 v[ITEMS], gn[ITEMS];
   float ss[VIRT];
 #pragma unroll
   for (int j = 0; j < VIRT; ++j) ss[j] = 0.f;
 #pragma unroll
-  for (int i = 0; i < kNormMaxVec; ++i) {
+  for (int i = 0; i < ITEMS; ++i) {
     const int c = threadIdx.x + i * THREADS;
     if (c >= nvec) break;
     float4 x = STREAM ? Stream4<float>::load(resid + in_off + 4 * c) : Vec4<float>::load(resid + in_off + 4 * c);
     if (delta) {
       float4 d;
       if (STREAM) {  // the same sums in the same order
-        d = Stream4<TD>::load(delta + in_off + 4 * c);
-        for (int p = 1; p < n_partials; ++p) d = add4(d, Stream4<TD>::load(delta + p * partial_stride + in_off + 4 * c));
+        d = sum_partials4_stream(delta + in_off + 4 * c, partial_stride, n_partials);
       } else {
-        d = sum_partials4<TD>(delta + in_off + 4 * c, partial_stride, n_partials);
+        PendingSum4<TD> pending;
+        pending.ask(delta + in_off + 4 * c, partial_stride, n_partials);
+        gn[i] = Vec4<TG>::load(gain + 4 * c);
+        d = pending.sum(delta + in_off + 4 * c, partial_stride, n_partials);
       }
       if (bias) d = add4(d, Vec4<float>::load(bias + 4 * c));  // all partial sums, then the bias
       x = add4(x, d);
@@ -58,35 +67,30 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
         if (STREAM) Stream4<float>::store(resid + in_off + 4 * c, x);
         else Vec4<float>::store(resid + in_off + 4 * c, x);
       }
+    } else if (!STREAM) {
+      gn[i] = Vec4<TG>::load(gain + 4 * c);
     }
     v[i] = x;
     // explicit fused multiply-adds: the same roundings in every variant of the kernel
     ss[i % VIRT] = fmaf(x.w, x.w, fmaf(x.z, x.z, fmaf(x.y, x.y, fmaf(x.x, x.x, ss[i % VIRT]))));
   }
-  float total;
-  if (VIRT == 1) {
-    total = block_sum(ss[0], scratch);
-  } else {
-    // the waves of the threads this thread stands for are wave + (THREADS / 64) j
-    const int w = threadIdx.x / kWave;
+  // the waves of the threads this thread stands for are wave + (THREADS / 64) j
 #pragma unroll
-    for (int j = 0; j < VIRT; ++j) {
-      const float s = wave_sum(ss[j]);
-      if ((threadIdx.x & (kWave - 1)) == 0) scratch[w + (THREADS / kWave) * j] = s;
-    }
-    __syncthreads();
-    total = 0.f;
-    for (int i = 0; i < VIRT * THREADS / kWave; ++i) total += scratch[i];
+  for (int j = 0; j < VIRT; ++j) {
+    const float s = full_wave_sum(ss[j]);
+    if ((threadIdx.x & (kWave - 1)) == 0) scratch[threadIdx.x / kWave + (THREADS / kWave) * j] = s;
   }
+  __syncthreads();
+  const float total = waves_sum<VIRT * THREADS / kWave>(scratch);
   const float inv = rsqrtf(total / static_cast<float>(hidden) + eps);
   const size_t out_off = static_cast<size_t>(r_out) * hidden;
 #pragma unroll
-  for (int i = 0; i < kNormMaxVec; ++i) {
+  for (int i = 0; i < ITEMS; ++i) {
     const int c = threadIdx.x + i * THREADS;
     if (c >= nvec) break;
-    const float4 gn = Vec4<TG>::load(gain + 4 * c);
-    const float4 x = v[i];
-    const float4 y{x.x * inv * gn.x, x.y * inv * gn.y, x.z * inv * gn.z, x.w * inv * gn.w};
+    if (STREAM) gn[i] = Vec4<TG>::load(gain + 4 * c);
+    const float4 x = v[i], g = gn[i];
+    const float4 y{x.x * inv * g.x, x.y * inv * g.y, x.z * inv * g.z, x.w * inv * g.w};
     if (STREAM) Stream4<TO>::store(out + out_off + 4 * c, y);
     else Vec4<TO>::store(out + out_off + 4 * c, y);
   }
@@ -95,12 +99,12 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
 // ---------------------------------------------------------------------------
 // rotary + cache write, four pairs per item; grid (tokens, ceil(items / 256)).
 // ---------------------------------------------------------------------------
+// (The arguments that the first loads need come first: those are in registers when the kernel starts.)
 template <typename TI, typename TC, bool STREAM>
 __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
-    const TI* __restrict__ qkv, int n_partials, size_t partial_stride, const void* __restrict__ bias,
-    int bias_dt, TC* __restrict__ q_out, TC* __restrict__ k_cache, TC* __restrict__ v_cache,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t, const int* __restrict__ positions,
-    const int* __restrict__ slots, int nq, int nkv, int hd, int page_size, int write_kv) {
+    const TI* __restrict__ qkv, size_t partial_stride, int n_partials, int nq, int nkv, int hd, const void* __restrict__ bias,
+    const int* __restrict__ positions, const int* __restrict__ slots, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    int bias_dt, int page_size, TC* __restrict__ q_out, TC* __restrict__ k_cache, TC* __restrict__ v_cache) {
   const int n = blockIdx.x;
   const int half = hd / 2, hv = half / 4;            // vec4 pairs per head
   const int n_rot = (nq + nkv) * hv, n_items = n_rot + nkv * (hd / 4);
@@ -108,31 +112,49 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
   if (it >= n_items) return;
   const int width = (nq + 2 * nkv) * hd;
   const size_t in_row = static_cast<size_t>(n) * width;
-  const int slot = write_kv ? slots[n] : -1;
-  const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
+  const int slot = slots ? slots[n] : -1;
 
-  auto value4 = [&](int col) {
-    float4 v;
+  // Whatever is asked for is asked for before anything is waited for (a step of few tokens is all waiting): the product's parts, the
+  // bias, the tables' row.
+  struct Value {
+    PendingSum4<TI> parts;
+    uint4 bias;
+  };
+  auto ask4 = [&](Value& v, int col) {
     if (STREAM) {  // the product's rows of a step of many tokens are read once: past the caches
-      v = Stream4<TI>::load(qkv + in_row + col);
-      for (int p = 1; p < n_partials; ++p) v = add4(v, Stream4<TI>::load(qkv + p * partial_stride + in_row + col));
+      v.parts.v[0] = sum_partials4_stream(qkv + in_row + col, partial_stride, n_partials);
     } else {
-      v = sum_partials4<TI>(qkv + in_row + col, partial_stride, n_partials);
+      v.parts.ask(qkv + in_row + col, partial_stride, n_partials);
     }
-    if (bias) {  // col is a multiple of 4: one load of four
-      v = add4(v, bias_dt == kF32 ? Vec4<float>::load(static_cast<const float*>(bias) + col)
-                                  : Vec4<bf16>::load(static_cast<const bf16*>(bias) + col));
+    if (bias) {  // col is a multiple of 4: one load of four, as they are
+      if (bias_dt == kF32) {
+        v.bias = *reinterpret_cast<const uint4*>(static_cast<const float*>(bias) + col);
+      } else {
+        const uint2 u = *reinterpret_cast<const uint2*>(static_cast<const bf16*>(bias) + col);
+        v.bias.x = u.x, v.bias.y = u.y;
+      }
     }
-    return v;
+  };
+  auto value4 = [&](const Value& v, int col) {
+    const float4 s = STREAM ? v.parts.v[0] : v.parts.sum(qkv + in_row + col, partial_stride, n_partials);
+    if (!bias) return s;
+    const uint4 u = v.bias;
+    return add4(s, bias_dt == kF32 ? float4{__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)}
+                                   : float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                                            __uint_as_float(u.y & 0xffff0000u)});
   };
 
   if (it < n_rot) {
     const int head = it / hv, j = 4 * (it % hv);
-    if (head >= nq && slot < 0) return;
     const int base = head * hd;
-    const float4 x1 = value4(base + j), x2 = value4(base + j + half);
+    Value p1, p2;
+    ask4(p1, base + j);
+    ask4(p2, base + j + half);
     const size_t t = static_cast<size_t>(positions[n]) * half + j;
     const float4 c = Vec4<float>::load(cos_t + t), s = Vec4<float>::load(sin_t + t);
+    const float4 x1 = value4(p1, base + j), x2 = value4(p2, base + j + half);
+    if (head >= nq && slot < 0) return;
+    const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
     float4 a, b;
     rotate_pair(x1.x, x2.x, c.x, s.x, a.x, b.x);
     rotate_pair(x1.y, x2.y, c.y, s.y, a.y, b.y);
@@ -142,10 +164,14 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
                         : k_cache + ((static_cast<size_t>(page) * nkv + (head - nq)) * page_size + off) * hd;
     Vec4<TC>::store(dst + j, a);
     Vec4<TC>::store(dst + j + half, b);
-  } else if (slot >= 0) {
+  } else {
     const int e = 4 * (it - n_rot);
     const int kvh = e / hd, d = e % hd;
-    const float4 v = value4((nq + nkv) * hd + e);
+    Value pv;
+    ask4(pv, (nq + nkv) * hd + e);
+    const float4 v = value4(pv, (nq + nkv) * hd + e);
+    if (slot < 0) return;
+    const int page = slot / page_size, off = slot % page_size;
     TC* row = v_cache + ((static_cast<size_t>(page) * nkv + kvh) * hd + d) * page_size;
     row[off] = from_float<TC>(v.x);
     row[page_size + off] = from_float<TC>(v.y);
@@ -217,11 +243,11 @@ bool add_rmsnorm_vec(float* resid, const void* delta, int delta_dt, int n_partia
   if (bias && (!delta || reinterpret_cast<uintptr_t>(bias) % 16)) return false;
   // Which variant runs depends on the number of rows; what it computes does not (see the kernel).
   const bool wide = hidden > 1024;
-  const bool few = n <= 128 && wide;  // a decode step: spread each row over more threads
+  const bool few = n <= compute_units() && wide;  // a row a unit: spread over more threads
 #define PYRE_NORM_LAUNCH(THREADS, VIRT, STREAM)                                                                      \
   hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TG, TO, THREADS, VIRT, STREAM>), dim3(n), dim3(THREADS), 0, stream, \
-                     resid, static_cast<const TD*>(delta), n_partials, static_cast<size_t>(partial_stride), bias,    \
-                     static_cast<const TG*>(gain), static_cast<TO*>(out), rows, hidden, eps)
+                     resid, static_cast<const TD*>(delta), n_partials, hidden, static_cast<size_t>(partial_stride), rows, \
+                     static_cast<const TG*>(gain), static_cast<TO*>(out), eps, bias)
   PYRE_DISPATCH(delta_dt, TD, PYRE_DISPATCH(gain_dt, TG, PYRE_DISPATCH(out_dt, TO, {
     const bool many = n >= 512;  // more bytes than the caches keep for the next kernel
     if (few) PYRE_NORM_LAUNCH(1024, 1, false);
@@ -246,10 +272,9 @@ bool rope_kv_write_vec(const void* qkv, int qkv_dt, int n_partials, long partial
 #define PYRE_ROPE_LAUNCH(STREAM)                                                                                   \
   PYRE_DISPATCH(qkv_dt, TI, PYRE_DISPATCH(q_dt, TC,                                                               \
       hipLaunchKernelGGL((rope_kv_write_vec_kernel<TI, TC, STREAM>), grid, dim3(256), 0, stream,                  \
-                         static_cast<const TI*>(qkv), n_partials, static_cast<size_t>(partial_stride), bias,      \
-                         bias_dt, static_cast<TC*>(q_out), static_cast<TC*>(k_cache),                             \
-                         static_cast<TC*>(v_cache), cos_t, sin_t, positions, slots, nq, nkv, hd, page_size,       \
-                         write_kv)))
+                         static_cast<const TI*>(qkv), static_cast<size_t>(partial_stride), n_partials, nq, nkv, hd, bias,  \
+                         positions, write_kv ? slots : nullptr, cos_t, sin_t, bias_dt, page_size, static_cast<TC*>(q_out), \
+                         static_cast<TC*>(k_cache), static_cast<TC*>(v_cache))))
   if (n >= 512) {
     PYRE_ROPE_LAUNCH(true);
   } else {

@@ -168,6 +168,42 @@ __device__ inline float lanes_sum(float v) {
   return v;
 }
 
+// wave_sum where all 64 lanes are there, with the same additions in the same order and no trip through LDS for any of them: halves and
+// quarters of the wave change places, then the lanes of sixteen turn by 8 and by 4 (equal to the exchange with the
+// lane 4 away, since lanes 8 apart hold the same by then). Six exchanges through LDS are a chain of 0.3 us.
+__device__ inline float full_wave_sum(float v) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(halves[0]) + __uint_as_float(halves[1]);
+  const auto quarters = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(quarters[0]) + __uint_as_float(quarters[1]);
+  v += lane_exchange<0x128>(v);  // row_ror:8
+  v += lane_exchange<0x124>(v);  // row_ror:4
+  v += lane_exchange<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v += lane_exchange<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  return v;
+}
+
+// block_sum's value for blocks of N waves that all arrive, the waves' results read from LDS together. `scratch` is N floats on 16
+// bytes that the block uses for nothing else (no barrier stands before their first use).
+template <int N>
+__device__ inline float waves_sum(const float* scratch) {
+  float s[N];
+#pragma unroll
+  for (int i = 0; i < N; i += 4) *reinterpret_cast<float4*>(s + i) = *reinterpret_cast<const float4*>(scratch + i);
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) t += s[i];
+  return t;
+}
+template <int N>
+__device__ inline float row_sum(float v, float* scratch) {
+  static_assert(N % 4 == 0, "read four at a time");
+  v = full_wave_sum(v);
+  if ((threadIdx.x & (kWave - 1)) == 0) scratch[threadIdx.x / kWave] = v;
+  __syncthreads();
+  return waves_sum<N>(scratch);
+}
+
 // Block-wide reductions for blocks of up to 1024 threads (16 waves). `scratch`
 // is 16 floats of LDS. Every thread receives the result; the order of the
 // additions is fixed by the thread layout alone.

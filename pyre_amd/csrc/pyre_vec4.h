@@ -65,25 +65,45 @@ __device__ inline float4 add4(float4 a, float4 b) { return float4{a.x + b.x, a.y
 // lie `stride` elements apart. Up to kAtOnce loads are in flight together: a kernel that only
 // passes a few rows on spends its time waiting for loads, one round trip after the other.
 constexpr int kAtOnce = 12;
+// The loads and the sum apart, for whoever asks for something else between the two.
+template <typename T>
+struct PendingSum4 {
+  float4 v[kAtOnce];
+  __device__ inline void ask(const T* src, size_t stride, int n) {
+#pragma unroll
+    for (int p = 0; p < kAtOnce; ++p)
+      if (p < n) v[p] = Vec4<T>::load(src + p * stride);
+  }
+  __device__ inline float4 sum(const T* src, size_t stride, int n) const {
+    float4 s = v[0];
+#pragma unroll
+    for (int p = 1; p < kAtOnce; ++p)
+      if (p < n) s = add4(s, v[p]);
+    for (int p = kAtOnce; p < n; ++p) s = add4(s, Vec4<T>::load(src + p * stride));
+    return s;
+  }
+};
 template <typename T>
 __device__ inline float4 sum_partials4(const T* src, size_t stride, int n) {
-  float4 v[kAtOnce];
-#pragma unroll
-  for (int p = 0; p < kAtOnce; ++p)
-    if (p < n) v[p] = Vec4<T>::load(src + p * stride);
-  float4 s = v[0];
-#pragma unroll
-  for (int p = 1; p < kAtOnce; ++p)
-    if (p < n) s = add4(s, v[p]);
-  for (int p = kAtOnce; p < n; ++p) s = add4(s, Vec4<T>::load(src + p * stride));
-  return s;
+  PendingSum4<T> pending;
+  pending.ask(src, stride, n);
+  return pending.sum(src, stride, n);
 }
 
-// The same sum of loads past the caches, in the same order.
+// The same sum of loads past the caches, in the same order, four of them under way at a time (rows in such numbers hide a trip
+// through memory behind each other, not one for each of ten parts).
 template <typename T>
 __device__ inline float4 sum_partials4_stream(const T* src, size_t stride, int n) {
   float4 s = Stream4<T>::load(src);
-  for (int p = 1; p < n; ++p) s = add4(s, Stream4<T>::load(src + p * stride));
+  for (int p = 1; p < n; p += 4) {
+    float4 v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (p + i < n) v[i] = Stream4<T>::load(src + (p + i) * stride);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (p + i < n) s = add4(s, v[i]);
+  }
   return s;
 }
 

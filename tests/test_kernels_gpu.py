@@ -108,6 +108,47 @@ def test_add_rmsnorm_row_does_not_depend_on_row_count(dtype, hidden):
     assert torch.equal(g_many, out_many.flip(0))
 
 
+@pytest.mark.parametrize("parts", [1, 2, 5, 6, 13])
+@pytest.mark.parametrize("many", [256, 257, 511, 512])
+def test_row_kernels_forms_for_rows_at_their_edges(many, parts):
+    """The norm's forms (a row a compute unit, 256 threads a row, past the caches) and the rotary kernel's two add a product's parts in
+    one order, however many of them are asked for together: the bits of the first rows alone."""
+    ops = _ops()
+    from pyre_amd.hip.ops import Partials
+
+    few = 3
+    for hidden in (1000, 1028, 8192):
+        resid, delta, gain = rnd(many, hidden, seed=1), rnd(parts, many, hidden, seed=2), rnd(hidden, seed=4) + 1
+        out, r = torch.empty(many, hidden, device=DEV), resid.clone()
+        ops.add_rmsnorm(r, Partials(delta), gain, 1e-6, out)
+        want = resid.double() + delta.double().sum(0)
+        assert torch.allclose(r.double(), want, atol=3e-6 * parts)
+        assert torch.allclose(out.double(), want * torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + 1e-6) * gain.double(), atol=2e-5, rtol=1e-5)
+        out3, r3 = torch.empty(few, hidden, device=DEV), resid[:few].clone()
+        ops.add_rmsnorm(r3, Partials(delta[:, :few].contiguous()), gain, 1e-6, out3)
+        assert torch.equal(r3, r[:few]) and torch.equal(out3, out[:few])
+    nq, nkv, hd, page = 3, 1, 16, 16
+    width, pages = (nq + 2 * nkv) * hd, many // page + 2
+    for dt in (torch.float32, torch.bfloat16):
+        qkv, bias = rnd(parts, many, width, seed=5), rnd(width, seed=6, dtype=dt)
+        cos, sin = rnd(many, hd // 2, seed=7), rnd(many, hd // 2, seed=8)
+        got = []
+        for n in (many, few):
+            q = torch.empty(n, nq * hd, device=DEV, dtype=dt)
+            kc, vc = (torch.zeros(pages, nkv, *shape, device=DEV, dtype=dt) for shape in ((page, hd), (hd, page)))
+            at = i32(list(range(n)))
+            ops.rope_kv_write(Partials(qkv[:, :n].contiguous(), bias), q, kc, vc, cos, sin, hd, at, at, n, nq, nkv, hd, page)
+            got.append((q[:few], kc[0, :, :few], vc[0, :, :, :few]))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+        x = (qkv.double().sum(0) + bias.double())[:few].view(few, nq + 2 * nkv, hd)
+        a, b, c, s = x[..., :hd // 2], x[..., hd // 2:], cos[:few, None].double(), sin[:few, None].double()
+        turned = torch.cat([a * c - b * s, b * c + a * s], -1)
+        tol = 2e-5 if dt == torch.float32 else 2.0 ** -8 * float(x.abs().max()) * 4
+        assert torch.allclose(got[0][0].double().view(few, nq, hd), turned[:, :nq], atol=tol)
+        assert torch.allclose(got[0][1].double().transpose(0, 1), turned[:, nq:nq + nkv], atol=tol)
+        assert torch.allclose(got[0][2].double().permute(2, 0, 1), x[:, nq + nkv:], atol=tol)
+
+
 @pytest.mark.parametrize("adt,wdt", [("float32", "float32"), ("bfloat16", "bfloat16"), ("bfloat16", "float32")])
 @pytest.mark.parametrize("m,n,k", [(1, 37, 50), (5, 130, 257), (77, 200, 64), (130, 65, 1000)])
 def test_gemm_generic(adt, wdt, m, n, k):
