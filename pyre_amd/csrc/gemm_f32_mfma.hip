@@ -243,28 +243,44 @@ __global__ __launch_bounds__(256) void gemm_f32_short_kernel(const float* __rest
 // A chain of instructions ends after `chain` steps and is added to the total in float32. A block that walks all parts of k
 // (where the rows alone fill the chip) ends its chains where the parts end: the bits of the consumer's sum of partial sums, which
 // then do not go through memory (WHOLE: every part's sum comes down by itself, as in memory).
-template <int BM, int BN, int WM, int WN, int SL, int OCC, bool TAIL, bool WHOLE>
-__global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
-    const float* A, long lda, const float* W, long ldw, const void* __restrict__ bias,
-    int bias_dt, float* __restrict__ out, size_t ldo, size_t part_stride, int M, int N, int K, int kper, int chain, int mt, int nt) {
+struct TileArgs {
+  const float* A;
+  long lda;
+  const float* W;
+  long ldw;
+  const void* bias;
+  int bias_dt;
+  float* out;
+  size_t ldo, part_stride;
+  int M, N, K, kper, chain, nt;
+};
+template <int BM, int BN, int SL>
+constexpr int tile_bytes() { return 2 * 3 * 2 * SL * (16 * (BM + BN) + 64 / SL); }
+
+// Block `block` of `blocks`, whose tiles begin at row `row0` of A.
+template <int BM, int BN, int WM, int WN, int SL, bool TAIL, bool WHOLE>
+__device__ inline void gemm_f32_tile(unsigned char* const lds, const TileArgs& s, int row0, int mt, int block, int blocks) {
   constexpr int R = BM + BN, KP = 2 * SL, P = KP * R / 256, ROWS = 16 * R + 64 / SL, PLANE = KP * ROWS, BUF = 3 * PLANE;
   constexpr int CT = BM / WM / 32, RT = BN / WN / 32;
-  static_assert(WM * WN == 4 && KP * R % 256 == 0, "four waves, whose threads bring equally many pieces");
-  __shared__ __attribute__((aligned(64))) unsigned char lds[2 * BUF];
+  static_assert(WM * WN == 4 && KP * R % 256 == 0 && 2 * BUF == tile_bytes<BM, BN, SL>(), "four waves, whose threads bring equally many pieces");
+  const float *const A = s.A, *const W = s.W;
+  const long lda = s.lda, ldw = s.ldw;
+  const size_t ldo = s.ldo;
+  const int M = s.M, N = s.N, chain = s.chain, nt = s.nt;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 31, half = lane >> 5, wm = wave % WM, wn = wave / WM;
   // Blocks are dealt to the eight dies in turn: a die's blocks are neighbours, eight tiles along m by some along n.
-  const int die = blockIdx.x & 7, share = gridDim.x >> 3, rest = gridDim.x & 7;
-  int t = die * share + min(die, rest) + (blockIdx.x >> 3);
+  const int die = block & 7, share = blocks >> 3, rest = blocks & 7;
+  int t = die * share + min(die, rest) + (block >> 3);
   const int per = mt * nt, ks = t / per;
   t -= ks * per;
   const int group = t / (8 * nt), first = 8 * group, gm = min(8, mt - first);
   t -= 8 * nt * group;
-  const int m0 = (first + t % gm) * BM, n0 = (t / gm) * BN;
-  const int kbeg = ks * kper, kend = min(K, kbeg + kper), len = kend - kbeg, steps = (len + BK - 1) / BK;
+  const int m0 = row0 + (first + t % gm) * BM, n0 = (t / gm) * BN;
+  const int kbeg = ks * s.kper, kend = min(s.K, kbeg + s.kper), len = kend - kbeg, steps = (len + BK - 1) / BK;
   const int slots = (steps + SL - 1) / SL;
-  out += ks * part_stride;
-  if (ks) bias = nullptr;  // the bias belongs to one part only
+  float* const out = s.out + ks * s.part_stride;
+  const void* const bias = ks ? nullptr : s.bias;  // the bias belongs to one part only
 
   const float* src[P];
   unsigned dst[P];
@@ -391,7 +407,24 @@ __global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(
         bad |= store4(f32x4{total[r][q][4 * i], total[r][q][4 * i + 1], total[r][q][4 * i + 2], total[r][q][4 * i + 3]}, !WHOLE,
                       out + static_cast<size_t>(m + 32 * q) * ldo, rows_of_16, n + 32 * r + 8 * i, N);
   }
-  finish<WHOLE>(bad, A + kbeg, lda, W + kbeg, ldw, bias, bias_dt, out, ldo, m, CT, M, n, RT, N, len, chain);
+  finish<WHOLE>(bad, A + kbeg, lda, W + kbeg, ldw, bias, s.bias_dt, out, ldo, m, CT, M, n, RT, N, len, chain);
+}
+
+template <int BM, int BN, int SL, int OCC, bool TAIL, bool WHOLE>
+__global__ __launch_bounds__(256, OCC) void gemm_f32_tile_kernel(const TileArgs s, int mt) {
+  __shared__ __attribute__((aligned(64))) unsigned char lds[tile_bytes<BM, BN, SL>()];
+  gemm_f32_tile<BM, BN, 2, 2, SL, TAIL, WHOLE>(lds, s, 0, mt, blockIdx.x, gridDim.x);
+}
+
+// Tiles of 128 x 128 for the first 128 mt rows, the first `big` blocks, and of 64 x 128 for up to 64 rows behind them: where those would
+// be half of a tile's rows or less, and so that the last round of blocks has smaller ones to fill it with.
+template <bool TAIL, bool WHOLE>
+__global__ __launch_bounds__(256, 2) void gemm_f32_mixed_kernel(const TileArgs s, int mt, int big) {
+  __shared__ __attribute__((aligned(64))) unsigned char lds[tile_bytes<64, 128, 2>()];
+  static_assert(tile_bytes<128, 128, 1>() <= tile_bytes<64, 128, 2>(), "room for either");
+  const int block = blockIdx.x;
+  if (block < big) gemm_f32_tile<128, 128, 2, 2, 1, TAIL, WHOLE>(lds, s, 0, mt, block, big);
+  else gemm_f32_tile<64, 128, 2, 2, 2, TAIL, WHOLE>(lds, s, 128 * mt, 1, block - big, gridDim.x - big);
 }
 
 constexpr int kStreamMaxRows = 32;
@@ -635,6 +668,30 @@ constexpr double kMacsPerUs = 3.9e5;    // of a compute unit
 constexpr double kBytesPerUs = 5e6;     // of memory, both ways
 constexpr double kFillUs = 0.004;       // a k of a block's chain before the unit's other blocks hide it
 
+// 128 x 128 and, for the last rows, 64 x 128, in one launch (us, one size of tiles and the two: the 1.5B shape's gate/up 250 and 225 at 650
+// rows, its way down 107 and 100 at 566, 87 and 82 at 400, q/k/v 25 and 21 at 270, the head 1,551 and 1,501 at 566; the 7B shape's
+// gate/up 899 and 851, its way down 439 and 418, at 150 rows 175 and 146). Against tiles of 64 x 128 alone only where that says a
+// tenth less: at 8 % less it was slower (the 7B shape's gate/up at 150 rows 369 and 398, the 1.5B shape's at 400 162 and 177).
+constexpr int kMixed = kSizes;
+constexpr double kMixedLeast = 0.9;
+
+// How many tiles of 128 x 128 the busiest unit's tiles are worth where `big` of them and then `small` ones, each worth 0.6, go to
+// whichever unit is free.
+double mixed_rounds(long big, long small) {
+  const double cost = kTiles[1].cost * kTiles[1].bm / kTiles[0].bm;
+  const long units = compute_units();
+  long n[2] = {units - big % units, big % units};
+  double level[2] = {static_cast<double>(big / units), static_cast<double>(big / units + 1)};
+  double most = n[1] ? level[1] : level[0];
+  while (small > 0) {
+    const int i = n[1] && level[1] < level[0] ? 1 : 0;
+    level[i] += cost;
+    if (level[i] > most) most = level[i];
+    small -= n[i];
+  }
+  return most;
+}
+
 // The tile size for so many rows and `parts` parts of kper, and what it takes in microseconds.
 int best_tile(int M, int N, int kper, int parts, double* us) {
   int best = 0;
@@ -643,6 +700,11 @@ int best_tile(int M, int N, int kper, int parts, double* us) {
     const long tiles = static_cast<long>((M + kTiles[i].bm - 1) / kTiles[i].bm) * ((N + kTiles[i].bn - 1) / kTiles[i].bn) * parts;
     const double work = kTiles[i].cost * kTiles[i].bm * kTiles[i].bn * kper * ((tiles + compute_units() - 1) / compute_units());
     if (work < least) least = work, best = i;
+  }
+  if (M > 128 && M % 128 > 0 && M % 128 <= 64) {
+    const long columns = static_cast<long>((N + 127) / 128) * parts;
+    const double work = 128.0 * 128.0 * kper * mixed_rounds(M / 128 * columns, columns);
+    if (work < (best == 1 ? kMixedLeast : 1.0) * least) least = work, best = kMixed;
   }
   if (us) *us = least / kMacsPerUs + 8.0 * parts * M * static_cast<double>(N) / kBytesPerUs + kFillUs * kper;
   return best;
@@ -658,17 +720,26 @@ bool takes_whole(int M, int N, int K, long lda, long ldw) {
 // Chains of `chain` steps. `whole`: in one part, whose chains are the parts of a product in several.
 void launch_tiles(const float* A, long lda, const float* W, long ldw, const void* bias, int bias_dt, float* out, long ldo, long part_stride,
                   int M, int N, int K, int kper, int parts, int chain, bool whole, hipStream_t stream) {
-  const auto tile = [&](auto kernel, int bm, int bn) {
-    const int mt = (M + bm - 1) / bm, nt = (N + bn - 1) / bn;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * nt * parts), dim3(256), 0, stream, A, lda, W, ldw, bias, bias_dt, out,
-                       static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, chain, mt, nt);
-  };
-  const int best = best_tile(M, N, kper, parts, nullptr);
+  const int nt = (N + 127) / 128, best = best_tile(M, N, kper, parts, nullptr);
   const bool tail = K % BK != 0;
-#define PYRE_F32_TILE(BM, BN, SL, OCC)                                                    \
-  tile(whole  ? gemm_f32_tile_kernel<BM, BN, 2, 2, SL, OCC, false, true>                  \
-       : tail ? gemm_f32_tile_kernel<BM, BN, 2, 2, SL, OCC, true, false>                  \
-              : gemm_f32_tile_kernel<BM, BN, 2, 2, SL, OCC, false, false>, BM, BN)
+  TileArgs s{A, lda, W, ldw, bias, bias_dt, out, static_cast<size_t>(ldo), static_cast<size_t>(part_stride), M, N, K, kper, chain, nt};
+  if (best == kMixed) {
+    const int mt = M / 128, big = mt * nt * parts;
+    const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(big + nt * parts), dim3(256), 0, stream, s, mt, big); };
+    if (whole) go(gemm_f32_mixed_kernel<false, true>);
+    else if (tail) go(gemm_f32_mixed_kernel<true, false>);
+    else go(gemm_f32_mixed_kernel<false, false>);
+    return;
+  }
+  const auto tile = [&](auto kernel, int bm, int bn) {
+    const int mt = (M + bm - 1) / bm;
+    s.nt = (N + bn - 1) / bn;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(mt) * s.nt * parts), dim3(256), 0, stream, s, mt);
+  };
+#define PYRE_F32_TILE(BM, BN, SL, OCC)                                              \
+  tile(whole  ? gemm_f32_tile_kernel<BM, BN, SL, OCC, false, true>                  \
+       : tail ? gemm_f32_tile_kernel<BM, BN, SL, OCC, true, false>                  \
+              : gemm_f32_tile_kernel<BM, BN, SL, OCC, false, false>, BM, BN)
   if (best == 0) PYRE_F32_TILE(128, 128, 1, 2);
   else if (best == 1) PYRE_F32_TILE(64, 128, 2, 2);
   else PYRE_F32_TILE(64, 64, 2, 3);
@@ -697,7 +768,13 @@ extern "C" int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int k
 extern "C" int pyre_gemm_f32_tile_choice(int M, int N, int K, int ksplit) {
   PYRE_REQUIRE(M > 0 && N > 0 && K > 0 && ksplit > 0, "gemm_f32_tile_choice: bad sizes");
   const int i = best_tile(M, N, part_of(K, ksplit), ksplit, nullptr);
-  return 1000 * kTiles[i].bm + kTiles[i].bn;
+  return i == kMixed ? 1000 * 128 + 128 : 1000 * kTiles[i].bm + kTiles[i].bn;
+}
+
+// Whether up to 64 rows behind those that fill tiles of 128 go to tiles of 64 x 128.
+extern "C" int pyre_gemm_f32_tile_mixed(int M, int N, int K, int ksplit) {
+  PYRE_REQUIRE(M > 0 && N > 0 && K > 0 && ksplit > 0, "gemm_f32_tile_mixed: bad sizes");
+  return best_tile(M, N, part_of(K, ksplit), ksplit, nullptr) == kMixed;
 }
 
 extern "C" int pyre_gemm_f32_whole(const float* A, long lda, const float* W, long ldw, float* out, long ldo, int M, int N, int K,

@@ -74,6 +74,8 @@ int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw, const void
 int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int ksplit);
 // The tiles that a product of more than 32 rows in ksplit parts is made of: 1000 x rows + columns.
 int pyre_gemm_f32_tile_choice(int M, int N, int K, int ksplit);
+// 1 if the last rows of such a product, up to 64 behind those that fill tiles of 128, are made in tiles of 64.
+int pyre_gemm_f32_tile_mixed(int M, int N, int K, int ksplit);
 int pyre_gemm_f32_whole(const float* A, long lda, const float* W, long ldw, float* out, long ldo, int M, int N, int K, int ksplit,
                         hipStream_t stream);
 

@@ -29,6 +29,7 @@ _SIGNATURES = {
     "pyre_gemm_mid_silu_blocks": [I, I],
     "pyre_gemm_f32_adds": [I, I, I, L, L, I],
     "pyre_gemm_f32_tile_choice": [I, I, I, I],
+    "pyre_gemm_f32_tile_mixed": [I, I, I, I],
     "pyre_gemm_tile_supports": [I, I, I, L, L],
     "pyre_gemm_tile_parts": [I, I, I],
     "pyre_attn_biased_spans": [I, I, I, I],

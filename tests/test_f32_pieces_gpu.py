@@ -204,3 +204,38 @@ def test_every_size_of_tiles(m, n, tile, k, off):
     same = torch.ones(m, n, dtype=torch.bool, device=DEV)
     same[list(rows)], same[:, list(cols)] = False, False
     assert torch.equal(got[same], out[same])
+
+
+@pytest.mark.parametrize("m,n,k,ks", [(129, 32768, 160, 1), (192, 32768, 157, 1), (566, 2048, 1536, 8), (400, 1500, 8960, 14), (260, 20000, 160, 2)])
+def test_last_rows_in_smaller_tiles(m, n, k, ks):
+    """Tiles of 128 rows with tiles of 64 behind them in one launch: the bits of a product of the last rows alone, bias, rows and columns past
+    the end, a part's end within a step, sums of all parts, and numbers that are not finite in either kind of tile."""
+    from pyre_amd.hip import ops
+    from pyre_amd.hip.lib import lib
+
+    assert lib().pyre_gemm_f32_tile_mixed(m, n, k, ks) == 1
+    a, w = operands(m, n, k, 0)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(1)).to(DEV)
+    a[1, 3], a[m - 1, 2] = float("inf"), 1e33
+    shape = (ks, m, n) if ks > 1 else (m, n)
+    out = torch.full(shape, float("nan"), device=DEV)
+    ops.gemm_f32(a, w, bias, out, m, ks)
+    for rows in (torch.arange(0, 100), torch.arange(m - 100, m)):
+        assert lib().pyre_gemm_f32_tile_mixed(100, n, k, ks) == 0
+        want = torch.empty(shape[:-2] + (100, n), device=DEV)
+        ops.gemm_f32(a[rows.to(DEV)].contiguous(), w, bias, want, 100, ks)
+        assert torch.equal(out[..., rows.to(DEV), :].nan_to_num(), want.nan_to_num())
+    exact = a.double() @ w.double().T + bias.double()
+    got = (out.double().sum(0) if ks > 1 else out.double())
+    fine = torch.ones(m, dtype=torch.bool, device=DEV)
+    fine[[1, m - 1]] = False
+    scale = a.double().abs() @ w.double().abs().T + bias.double().abs()
+    assert bool(((got - exact)[fine].abs() <= 2.0 ** -21 * scale[fine]).all())
+    if k % 16 == 0 and ks > 1:
+        plain, whole = torch.empty(shape, device=DEV), torch.empty(m, n, device=DEV)
+        ops.gemm_f32(a, w, None, plain, m, ks)
+        ops.gemm_f32_whole(a, w, whole, m, ks)
+        total = plain[0].clone()
+        for p in plain[1:]:
+            total += p
+        assert torch.equal(whole.nan_to_num(), total.nan_to_num())
