@@ -33,6 +33,7 @@
 #include "pyre_api.h"
 #include "pyre_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 using namespace pyre;
@@ -396,6 +397,9 @@ constexpr TileCost kUnits[] = {{256, 256, 3.4, 2.8, 0.871, 0.499, 0.093, 0.028},
 constexpr TileCost kPages[] = {kSums[0], kSums[2], kSums[3]};
 constexpr int kMaxParts = 6;
 constexpr double kReadMb = 0.2;              // the consumer's reading of a further part, a megabyte
+// Megabytes a microsecond that weights come with at the most: a head's few last rows are a second pass over
+// weights that no cache holds (151,936 x 1,536, 54 rows: 92 us, 70 without this; 566 rows cut behind 512 took 346 us, whole 302).
+constexpr double kMbPerUs = 5.0;
 constexpr double kMostPartsBytes = 536870912.0;  // parts of k together take no more scratch memory than this
 
 // Which tiles, in how many parts of k; and, where that leaves the last round of blocks nearly empty, a cut: tiles of `cfg`
@@ -440,8 +444,9 @@ TileChoice choose(const TileCost* costs, int n_costs, bool gated, int M, int N, 
           const int m2 = by_rows ? M - m1 : M, n2 = by_rows ? N : N - n1;
           const double first = tile_us(c, bytes, m1, n1, K, kper, parts);
           if (first >= best.us) continue;
+          const double again = by_rows ? 2e-6 * N * static_cast<double>(K) / kMbPerUs : 0.0;
           for (int j = 0; j < n_costs; ++j) {
-            const double both = first + tile_us(costs[j], bytes, m2, n2, K, kper, parts);
+            const double both = first + std::max(tile_us(costs[j], bytes, m2, n2, K, kper, parts), again);
             if (both < best.us) best = TileChoice{i, parts, kper, both, by_rows ? m1 : gated ? n1 / 2 : n1, by_rows, j};
           }
         }

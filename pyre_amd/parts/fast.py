@@ -4,8 +4,8 @@ Each function returns None / False when its fast path does not take the case
 (element type, sizes, alignment); the caller then runs the general kernel.
 Nothing here changes what is computed, only by which kernel. Sizes that no kernel
 of this framework takes go to the vendor's BLAS through ``torch.mm``, as the
-reference's products do (`pyre/model.py:84-87` are ``nn.Linear``), and so do the
-head's logits of many rows; the true 32-bit path never comes here.
+reference's products do (`pyre/model.py:84-87` are ``nn.Linear``); the true 32-bit
+path never comes here.
 """
 
 from __future__ import annotations
@@ -203,12 +203,18 @@ def linear(lin, ctx, x, n, out):
         return rt.options.get("skinny_gemm", True) and ops.gemm_skinny_supports(min(n, SKINNY_MAX_ROWS), n_out, k, ldx, ldw)
 
     if out is not None:
-        # float32 results wanted in place (the head's logits)
-        if (n <= SKINNY_MAX_ROWS or not library) and streams():  # no split, 64 rows at a time
+        # float32 results wanted in place (the head's logits). Of more rows than a block of the weight-streaming kernel keeps (a large
+        # decode step, every row of a portion) in tiles, whole: against the library's product, us on the 1.5B and 7B shapes' heads,
+        # 114 and 131, 221 and 232 at 65 rows, 144 and 153, 277 and 293 at 190, 155 and 168, 292 and 326 at 256, 237 and 275, 466
+        # and 563 at 512, 1,078 and 1,160, 2,120 and 2,212 at 2,400; behind by up to 4 % where a row of tiles of 256 is nearly empty (257
+        # rows 208 and 199, 566 309 and 305, 634 and 617).
+        if takes_tiles(rt, lin, n, x) and out.is_contiguous() and out.data_ptr() % 16 == 0:
+            ops.gemm_tile_bf16(x, weight, out, n, 1)
+        elif (n <= SKINNY_MAX_ROWS or not library) and streams():  # no split, 64 rows at a time
             for r0 in range(0, n, SKINNY_MAX_ROWS):
                 rows = min(SKINNY_MAX_ROWS, n - r0)
                 ops.gemm_skinny_bf16(x[r0:r0 + rows], lin.weight, out[r0:r0 + rows], rows, 1)
-        elif library:  # many rows (a large decode step, or every row of a portion): one pass over the weights
+        elif library:
             torch.mm(x if n == x.shape[0] else x[:n], lin.weight.t(), out_dtype=torch.float32, out=out)
         else:
             return None

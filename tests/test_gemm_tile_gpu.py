@@ -282,3 +282,26 @@ def test_a_step_with_weights_that_are_views():
         eng = Engine.from_state(cfg, state, EngineConfig(max_cached_tokens=1024, max_num_batched_tokens=512, max_model_len=512))
         rows.append(eng.step([Entry("a", ids, list(range(300)))]).clone())
     assert float(((rows[0] - rows[1]).abs().amax(1) / rows[1].abs().amax(1)).max()) <= 2e-2
+
+
+@pytest.mark.parametrize("m,view", [(64, False), (65, False), (190, False), (257, False), (190, True)])
+def test_logits_of_many_rows_without_the_library(m, view, monkeypatch):
+    """The head's float32 results in place, on both sides of the rows that the weight-streaming kernel takes; weights that do
+    not lie on 16 bytes are the library's."""
+    from types import SimpleNamespace
+
+    from pyre_amd.hip import ops
+    from pyre_amd.parts import fast
+
+    n, k = 20016, 192
+    x, w = rnd(m + 3, k, seed=1), rnd(n * k + 8, seed=2)
+    weight = w[4:n * k + 4].view(n, k) if view else w[:n * k].view(n, k)
+    lin = SimpleNamespace(in_features=k, out_features=n, weight=weight, bias=None, role="head")
+    rt = SimpleNamespace(dtype=torch.bfloat16, options={}, compute_units=ops.compute_units())
+    called, mm = [], torch.mm
+    monkeypatch.setattr(torch, "mm", lambda *a, **b: (called.append(1), mm(*a, **b))[1])
+    out = torch.full((m, n), float("nan"), device=DEV)
+    p = fast.linear(lin, SimpleNamespace(runtime=rt), x, m, out)
+    assert bool(called) == view
+    want = x[:m].double() @ weight.double().T
+    assert float((p.data[0].double() - want).abs().max()) <= bound(k) * float(want.std()) * 4
