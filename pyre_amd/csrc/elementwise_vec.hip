@@ -54,7 +54,7 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
     if (delta) {
       float4 d;
       if (STREAM) {  // the same sums in the same order
-        d = sum_partials4_stream(delta + in_off + 4 * c, partial_stride, n_partials);
+        d = sum_many_partials4_stream(delta + in_off + 4 * c, partial_stride, n_partials);
       } else {
         PendingSum4<TD> pending;
         pending.ask(delta + in_off + 4 * c, partial_stride, n_partials);
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
   };
   auto ask4 = [&](Value& v, int col) {
     if (STREAM) {  // the product's rows of a step of many tokens are read once: past the caches
-      v.parts.v[0] = sum_partials4_stream(qkv + in_row + col, partial_stride, n_partials);
+      v.parts.v[0] = sum_many_partials4_stream(qkv + in_row + col, partial_stride, n_partials);
     } else {
       v.parts.ask(qkv + in_row + col, partial_stride, n_partials);
     }

@@ -126,6 +126,25 @@ def takes_tiles(rt, lin, n: int, x=None) -> bool:
     return ops.gemm_tile_supports(n, lin.out_features, lin.in_features, lin.in_features if x is None else x.stride(0), lin.weight.stride(0))
 
 
+#: rows from which, and the k and the weights' elements up to which, a product of few rows is ahead in tiles
+FEW_TILES_MIN_ROWS, FEW_TILES_MAX_K, FEW_TILES_MAX_WEIGHTS = 129, 4608, 17 << 20
+
+
+def few_tiles(n: int, n_out: int, k: int) -> int:
+    """In how many parts of k the kernel of tiles makes a product of so few rows that a block could keep them all, where it is ahead of the
+    one that does so, else 0. From 129 rows on what a block takes from L2 (all rows again for every 64 or 128 rows of
+    W) bounds that kernel, and tiles of 64 x 128 fill the chip with fewer parts for the consumer to read. In a graph, weights from memory, us
+    there and here, at 129 to 150, 192 and 256 rows: the 1.5B shape's q/k/v 7.8 and 6.8, 8.3 and 7.0, 9.7 and 7.5, its attention output 7.6 and
+    6.5, 8.3 and 6.8, 9.6 and 7.1; the 7B shape's q/k/v 15.1 and 15.5 (7 parts and 2), 17.1 and 16.7, 19.2 and 17.4, its attention output 13.6 and 12.9
+    (8 parts and 3), 14.7 and 13.6, 17.7 and 15.2; 3,072 x 4,608 14.4 and 14.4 (9 parts and 3), 15.6 and 15.5, 18.7 and 16.7. At 128 rows they are
+    about alike; longer k and larger weights stay with it: the ways down (1.5B 13.1 and 14.7, 14.7 and 15.9, 17.4 and 17.0; 7B 41.7 and
+    45.4, 42.5 and 50.0, 50.3 and 51.1) and the 32B shape's (o 20.0 and 22.4, 21.8 and 24.3, 25.8 and 24.8). The parts are those of
+    the next multiple of 64 rows, at which such decode steps are captured."""
+    if not FEW_TILES_MIN_ROWS <= n <= MID_MAX_ROWS or k > FEW_TILES_MAX_K or n_out * k > FEW_TILES_MAX_WEIGHTS:
+        return 0
+    return ops.gemm_tile_parts(-(-n // 64) * 64, n_out, k)
+
+
 def library_takes(lin, rt, n: int) -> bool:
     """Whether the 16-bit product of ``n`` rows (more than the weight-streaming kernel's) and this weight is left to the BLAS
     library once no kernel for few rows takes it."""
@@ -224,7 +243,10 @@ def linear(lin, ctx, x, n, out):
         kernel = ""
     if kernel == "block" and not ops.gemm_mid_supports(n, n_out, k, ldx, ldw):
         kernel, ks = ("stream", skinny_ksplit(n, n_out, k, rt.compute_units)) if n <= SKINNY_MAX_ROWS and streams() else ("", 0)
-    if kernel:
+    parts = 0
+    if kernel == "block" and rt.options.get("mid_gemm", True) != 2 and lin.role in TILE_ROLES and not lin.whole and takes_tiles(rt, lin, n, x):
+        parts = few_tiles(n, n_out, k)
+    if kernel and not parts:
         buf = rt.workspace.get(lin.partials_name, (ks, n, n_out), torch.float32)
         if kernel == "stream":
             ops.gemm_skinny_bf16(x, weight, buf, n, ks)
@@ -232,7 +254,7 @@ def linear(lin, ctx, x, n, out):
             ops.gemm_mid_bf16(x, weight, buf, n, ks, wide=wide)
         return Partials(buf, lin.bias)
     if lin.role in TILE_ROLES and takes_tiles(rt, lin, n, x):
-        parts = 1 if lin.whole else ops.gemm_tile_parts(n, n_out, k)
+        parts = parts or (1 if lin.whole else ops.gemm_tile_parts(n, n_out, k))
         buf = rt.workspace.get(lin.partials_name, (parts, n, n_out), torch.float32)
         ops.gemm_tile_bf16(x, lin.weight, buf, n, parts)
         return Partials(buf, lin.bias)

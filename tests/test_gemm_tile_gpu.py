@@ -305,3 +305,24 @@ def test_logits_of_many_rows_without_the_library(m, view, monkeypatch):
     assert bool(called) == view
     want = x[:m].double() @ weight.double().T
     assert float((p.data[0].double() - want).abs().max()) <= bound(k) * float(want.std()) * 4
+
+
+@pytest.mark.parametrize("n,k", [(1536, 1536), (2048, 1536), (4608, 3584), (3072, 4608), (1024, 1024), (48, 768)])
+def test_few_rows_in_tiles_agree_with_their_captured_size(n, k):
+    """From 129 rows on: a row of an eager step has the bits that it has in the padded one, and the sums are right."""
+    from types import SimpleNamespace
+
+    from pyre_amd.hip import ops
+    from pyre_amd.parts import fast
+
+    weight, x = rnd(n, k, seed=2), rnd(256, k, seed=1)
+    want = x.double() @ weight.double().T
+    buffers = {}
+    workspace = SimpleNamespace(get=lambda name, shape, dtype: buffers.setdefault((name, shape), torch.full(shape, float("nan"), dtype=dtype, device=DEV)))
+    rt = SimpleNamespace(dtype=torch.bfloat16, options={}, compute_units=ops.compute_units(), workspace=workspace)
+    lin = SimpleNamespace(in_features=k, out_features=n, weight=weight, bias=None, role="attn.out", whole=False, partials_name="p")
+    for captured, eager in ((128, 100), (192, 129), (192, 150), (256, 193), (256, 255)):
+        got = [fast.linear(lin, SimpleNamespace(runtime=rt), x[:m], m, None).data.clone() for m in (captured, eager)]
+        assert got[0].shape[0] == got[1].shape[0] and torch.equal(got[0][:, :eager], got[1])
+        assert fast.few_tiles(captured, n, k) == (0 if captured == 128 else got[0].shape[0])
+        assert float((got[0].double().sum(0) - want[:captured]).abs().max()) <= bound(k) * float(want.std()) * 4
