@@ -20,7 +20,7 @@ template <int THREADS>
 __device__ inline Poly poly_of_row(float s2, float s4, float s6, const float* abce, float eps, int width, float* scratch) {
   const float inv_n = 1.f / static_cast<float>(width);
   // the three block sums with one barrier pair: every wave leaves its three sums, everybody adds them in order
-  s2 = wave_sum(s2), s4 = wave_sum(s4), s6 = wave_sum(s6);
+  s2 = full_wave_sum(s2), s4 = full_wave_sum(s4), s6 = full_wave_sum(s6);
   const int w = threadIdx.x / kWave;
   constexpr int kWaves = THREADS / kWave;
   if (threadIdx.x % kWave == 0) scratch[w] = s2, scratch[kWaves + w] = s4, scratch[2 * kWaves + w] = s6;

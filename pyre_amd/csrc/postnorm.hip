@@ -106,7 +106,7 @@ template <typename TA, typename TG, typename TO, int THREADS, int ITEMS, bool ST
 __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
     float* __restrict__ resid, Term a, Term b, float inner_eps, const TG* __restrict__ outer_gain, float outer_eps,
     const TG* __restrict__ out_gain, float out_eps, TO* __restrict__ out, const int* __restrict__ rows, int hidden) {
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[4][16];  // of each sum its own
   const int r_out = blockIdx.x, r_in = rows ? rows[r_out] : r_out, tid = threadIdx.x;
   const size_t row = static_cast<size_t>(r_in) * hidden;
   const float inv_n = 1.f / static_cast<float>(hidden);
@@ -122,14 +122,14 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
     if constexpr (kTogether)
       r[k] = i >= hidden ? float4{0.f, 0.f, 0.f, 0.f} : STREAM ? Stream4<float>::load(resid + row + i) : Vec4<float>::load(resid + row + i);
   }
-  auto inv_rms = [&](const float4 (&v)[ITEMS], float e) {
+  auto inv_rms = [&](const float4 (&v)[ITEMS], float e, int at) {
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k)
       if (4 * (tid + k * THREADS) < hidden) ss += (v[k].x * v[k].x + v[k].y * v[k].y) + (v[k].z * v[k].z + v[k].w * v[k].w);
-    return 1.f / sqrtf(block_sum(ss, scratch) * inv_n + e);
+    return 1.f / sqrtf(row_sum<THREADS / kWave>(ss, scratch[at]) * inv_n + e);
   };
-  auto take = [&](const Term& t) {
+  auto take = [&](const Term& t, int at) {
     float4 v[ITEMS];
     const TA* src = static_cast<const TA*>(t.data) + row;
 #pragma unroll
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
              : STREAM    ? sum_partials4_stream(src + i, t.stride, t.n_partials)
                          : sum_partials4(src + i, t.stride, t.n_partials);
     }
-    const float f = t.gain ? inv_rms(v, inner_eps) * t.scale : t.scale;
+    const float f = t.gain ? inv_rms(v, inner_eps, at) * t.scale : t.scale;
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
@@ -149,10 +149,10 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
       y[k] = float4{y[k].x + v[k].x * f * g.x, y[k].y + v[k].y * f * g.y, y[k].z + v[k].z * f * g.z, y[k].w + v[k].w * f * g.w};
     }
   };
-  if (a.data) take(a);
-  if (b.data) take(b);
+  if (a.data) take(a, 0);
+  if (b.data) take(b, 1);
   if (outer_gain) {
-    const float f = inv_rms(y, outer_eps);
+    const float f = inv_rms(y, outer_eps, 2);
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
       const int i = 4 * (tid + k * THREADS);
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(THREADS) void add_rms_terms_vec_kernel(
     }
   }
   if (!out) return;
-  const float f = out_gain ? inv_rms(y, out_eps) : 1.f;
+  const float f = out_gain ? inv_rms(y, out_eps, 3) : 1.f;
   const size_t orow = static_cast<size_t>(r_out) * hidden;
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {

@@ -28,7 +28,7 @@ __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
     const float* __restrict__ gain, const float* __restrict__ shift, int center, float eps, TO* __restrict__ out,
     const int* __restrict__ picked, int hidden) {
   constexpr int W = VEC ? 4 : 1;
-  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float scratch[2][16];
   const int r_out = blockIdx.x, r_in = picked ? picked[r_out] : r_out, tid = threadIdx.x;
   const size_t row = static_cast<size_t>(r_in) * hidden;
   const float inv_n = 1.f / static_cast<float>(hidden);
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
     for (int k = 0; k < ITEMS; ++k)
 #pragma unroll
       for (int e = 0; e < W; ++e) sum += u[k][e];  // elements behind the row's end are zero
-    mean = block_sum(sum, scratch) * inv_n;
+    mean = row_sum<THREADS / kWave>(sum, scratch[0]) * inv_n;
   }
   float ss = 0.f;
 #pragma unroll
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(THREADS) void stream_norm_kernel(
     if (W * (tid + k * THREADS) < hidden)
 #pragma unroll
       for (int e = 0; e < W; ++e) ss += (u[k][e] - mean) * (u[k][e] - mean);
-  const float inv = 1.f / sqrtf(block_sum(ss, scratch) * inv_n + eps);
+  const float inv = 1.f / sqrtf(row_sum<THREADS / kWave>(ss, scratch[1]) * inv_n + eps);
   const size_t orow = static_cast<size_t>(r_out) * hidden;
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
