@@ -244,7 +244,8 @@ def linear(lin, ctx, x, n, out):
     if kernel == "block" and not ops.gemm_mid_supports(n, n_out, k, ldx, ldw):
         kernel, ks = ("stream", skinny_ksplit(n, n_out, k, rt.compute_units)) if n <= SKINNY_MAX_ROWS and streams() else ("", 0)
     parts = 0
-    if kernel == "block" and rt.options.get("mid_gemm", True) != 2 and lin.role in TILE_ROLES and not lin.whole and takes_tiles(rt, lin, n, x):
+    if (kernel == "block" and n >= FEW_TILES_MIN_ROWS and rt.options.get("mid_gemm", True) != 2 and lin.role in TILE_ROLES
+            and not lin.whole and takes_tiles(rt, lin, n, x)):
         parts = few_tiles(n, n_out, k)
     if kernel and not parts:
         buf = rt.workspace.get(lin.partials_name, (ks, n, n_out), torch.float32)
