@@ -110,17 +110,13 @@ TILE_ROLES = LIBRARY_F32_ROLES | {"ffn.down"}
 def takes_tiles(rt, lin, n: int, x=None) -> bool:
     """Whether a 16-bit product of ``n`` rows goes to the kernel of tiles of up to 256 x 256 (`gemm_tile.hip`): all of more
     rows than the weight-streaming kernel takes whose sizes it supports and whose operands lie on 16 bytes (``x`` None: rows like a
-    workspace's; a weight that its owner hands over may be a view). Against the BLAS library's products (us here and there,
-    weights from memory, the gated unit and the reading of partial sums with them): the 7B shape's way down 107 and 141 at 566
-    rows, 241 and 360 at 2,048, 469 and 537 at 4,096, 936 and 880 at 8,192; its gate/up 156 and 153, 454 and 550, 888 and 868,
-    1,717 and 1,780; the 1.5B shape's way down 26 and 31 at 566, 60 and 67 at 2,048, 107 and 103 at 4,096; its gate/up 38 and 43,
-    109 and 138, 200 and 225; the 32B shape's way down 190 and 246, 496 and 447, 1,037 and 897, at 8,192 1,932 and 2,289.
-    Where the line could be drawn otherwise: q/k/v and attention output are ahead up to about 1,000 rows (7B: 28 and 33, 26 and
-    25 at 566) and behind from there on (71 and 65, 58 and 51 at 2,048; 128 and 123, 94 and 89 at 4,096; worst the 1.5B shape's
-    q/k/v, 32 and 25 at 3,000). All products of a layer together are 824 and 1,024 us for 2,048 rows of the 7B shape, 1,578 and
-    1,618 for 4,096, 3,070 and 3,047 for 8,192; 206 and 247, 367 and 383, 651 and 690 of the 1.5B shape; 1,654 and 1,729, 3,276
-    and 3,216, 6,286 and 6,804 of the 32B shape (at 3,000 rows 2,409 and 2,297: 1.23 PFLOP/s in its way down where the library
-    has 1.48)."""
+    workspace's; a weight that its owner hands over may be a view). Against the BLAS library's products (us here and there, the
+    gated unit with them, launches one behind the other): the 7B shape's q/k/v 26 and 35 at 566 rows, 64 and 68 at 2,048, 113 and 122
+    at 4,096, 204 and 212 at 8,192; its attention output 27 and 28, 50 and 53, 86 and 90, 160 and 169; its gate/up 159 and 185, 413 and
+    553, 790 and 872, 1,528 and 1,778; its way down 89 and 143, 214 and 350, 396 and 670, 781 and 1,214. The 1.5B shape's q/k/v 12 and 21,
+    20 and 23, 34 and 32, 47 and 54; its gate/up 32 and 46, 97 and 138, 183 and 215, 346 and 428; its way down 23 and 39, 50 and 66, 85 and
+    99, 159 and 168. The 32B shape's gate/up 295 and 317, 831 and 1,068, 1,608 and 1,939, 3,139 and 3,586; its way down 163 and 252, 437 and
+    450, 849 and 896, 1,650 and 2,241. A consumer's reading of more parts than one, up to six at 566 rows, comes to it (0.2 us a megabyte)."""
     if not rt.options.get("tile_gemm", True) or n <= SKINNY_MAX_ROWS or lin.weight.data_ptr() % 16 or (x is not None and x.data_ptr() % 16):
         return False
     return ops.gemm_tile_supports(n, lin.out_features, lin.in_features, lin.in_features if x is None else x.stride(0), lin.weight.stride(0))
