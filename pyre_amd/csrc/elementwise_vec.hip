@@ -24,8 +24,11 @@ constexpr int kNormMaxVec = 8;  // float4 per thread of 256
 // once, the gain among it, the reduction is exchanges between lanes and one trip through LDS, and what the first loads need
 // comes with the launch (arguments in that order). In a graph, us at 10 parts: 1,536 elements 3.1 -> 2.7 at one row, 4.65 -> 3.3 at 190;
 // 3,584 elements 3.8 -> 3.5 and 7.7 -> 4.9. Rows get 1024 threads up to one row a compute unit (190 rows with
-// 256 threads 4.1 and 6.8; at 400 rows the two are alike). STREAM asks for four parts at a time (566 rows, 10 parts, one at a time:
-// 14.0 -> 9.8 and 26.9 -> 20.6); it has the waves that hide the gain.
+// 256 threads 4.1 and 6.8; at 400 rows the two are alike). STREAM has the waves that hide the gain. FOUR: it asks for four parts at a
+// time, for three parts and more of so few rows that a trip through memory for each part is not hidden: one at a time and four, us at 566
+// rows and 10 parts 11.6 and 8.3, 26.2 and 19.8. Two parts gain nothing by it (566 rows of 1,536 elements 4.0 and 4.2, of 4,096 8.45 and 8.7),
+// and where rows and parts are many it takes the caches' order from the reads: 2,048 rows of 2,048 in 10 parts 33.8 and
+// 39.3, 1,300 of 4,096 46.7 and 49.5. The line (rows times parts below 12,000) is where the two are alike over seven widths.
 //
 // The sum of squares is added up in an order that the row's width alone fixes, whichever
 // variant runs: a row wider than 1024 elements is summed as 1024 threads would (thread t
@@ -33,7 +36,7 @@ constexpr int kNormMaxVec = 8;  // float4 per thread of 256
 // reduced by the butterfly of wave_sum; the 16 results are added in ascending order).
 // The 256-thread variant then plays VIRT = 4 of those threads per thread: t = thread +
 // 256 j. A position's result therefore does not depend on how many rows share the step.
-template <typename TD, typename TG, typename TO, int THREADS, int VIRT, bool STREAM>
+template <typename TD, typename TG, typename TO, int THREADS, int VIRT, bool STREAM, bool FOUR = false>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
     float* __restrict__ resid, const TD* __restrict__ delta, int n_partials, int hidden, size_t partial_stride, const int* __restrict__ rows,
     const TG* __restrict__ gain, TO* __restrict__ out, float eps, const float* __restrict__ bias) {
@@ -54,7 +57,8 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
     if (delta) {
       float4 d;
       if (STREAM) {  // the same sums in the same order
-        d = sum_many_partials4_stream(delta + in_off + 4 * c, partial_stride, n_partials);
+        d = FOUR ? sum_many_partials4_stream(delta + in_off + 4 * c, partial_stride, n_partials)
+                 : sum_partials4_stream(delta + in_off + 4 * c, partial_stride, n_partials);
       } else {
         PendingSum4<TD> pending;
         pending.ask(delta + in_off + 4 * c, partial_stride, n_partials);
@@ -100,7 +104,14 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(
 // rotary + cache write, four pairs per item; grid (tokens, ceil(items / 256)).
 // ---------------------------------------------------------------------------
 // (The arguments that the first loads need come first: those are in registers when the kernel starts.)
-template <typename TI, typename TC, bool STREAM>
+// How the product's parts are read; they are always added in one order. kTogether: both values' parts and all else is asked for before
+// anything is waited for. That takes 124 registers (kEach 62), so it is for as many blocks as the compute units then hold, four each (two
+// parts, us with kEach and kTogether: 28 query and 4 key/value heads, three blocks a row, 4.6 and 4.1 at 256 rows, 5.3 and 6.0 at 400; 12 and 2,
+// two blocks, 4.9 and 4.7 at 400; 40 and 8, four blocks, 7.6 and 8.5 at 400). kEach: one value after the other. From 512 rows on past the caches,
+// one part at a time (kStream) or four (kStreamFour), for three parts and more of less than 1,200 rows (12 and 2 heads, us: 7 parts of 700
+// rows 13.5 and 9.9, 2 parts of 566 rows 4.9 and 5.4, 7 parts of 28 and 4 heads at 2,048 rows 54.9 and 57.0).
+enum Read { kTogether, kEach, kStream, kStreamFour };
+template <typename TI, typename TC, Read READ>
 __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
     const TI* __restrict__ qkv, size_t partial_stride, int n_partials, int nq, int nkv, int hd, const void* __restrict__ bias,
     const int* __restrict__ positions, const int* __restrict__ slots, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
@@ -109,7 +120,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
   const int half = hd / 2, hv = half / 4;            // vec4 pairs per head
   const int n_rot = (nq + nkv) * hv, n_items = n_rot + nkv * (hd / 4);
   const int it = blockIdx.y * 256 + threadIdx.x;
-  if (it >= n_items) return;
+  if (it >= (slots ? n_items : nq * hv)) return;  // (no slots: the cache is another layer's)
   const int width = (nq + 2 * nkv) * hd;
   const size_t in_row = static_cast<size_t>(n) * width;
   const int slot = slots ? slots[n] : -1;
@@ -121,11 +132,11 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
     uint4 bias;
   };
   auto ask4 = [&](Value& v, int col) {
-    if (STREAM) {  // the product's rows of a step of many tokens are read once: past the caches
-      v.parts.v[0] = sum_many_partials4_stream(qkv + in_row + col, partial_stride, n_partials);
-    } else {
-      v.parts.ask(qkv + in_row + col, partial_stride, n_partials);
-    }
+    const TI* const src = qkv + in_row + col;
+    if (READ == kStreamFour) v.parts.v[0] = sum_many_partials4_stream(src, partial_stride, n_partials);
+    else if (READ == kStream) v.parts.v[0] = sum_partials4_stream(src, partial_stride, n_partials);
+    else if (READ == kEach) v.parts.v[0] = sum_partials4(src, partial_stride, n_partials);
+    else v.parts.ask(src, partial_stride, n_partials);
     if (bias) {  // col is a multiple of 4: one load of four, as they are
       if (bias_dt == kF32) {
         v.bias = *reinterpret_cast<const uint4*>(static_cast<const float*>(bias) + col);
@@ -136,12 +147,17 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
     }
   };
   auto value4 = [&](const Value& v, int col) {
-    const float4 s = STREAM ? v.parts.v[0] : v.parts.sum(qkv + in_row + col, partial_stride, n_partials);
+    const float4 s = READ != kTogether ? v.parts.v[0] : v.parts.sum(qkv + in_row + col, partial_stride, n_partials);
     if (!bias) return s;
     const uint4 u = v.bias;
     return add4(s, bias_dt == kF32 ? float4{__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)}
                                    : float4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
                                             __uint_as_float(u.y & 0xffff0000u)});
+  };
+
+  int page = 0, off = 0;
+  auto place = [&] {
+    if (slot >= 0) page = slot / page_size, off = slot % page_size;
   };
 
   if (it < n_rot) {
@@ -152,9 +168,10 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
     ask4(p2, base + j + half);
     const size_t t = static_cast<size_t>(positions[n]) * half + j;
     const float4 c = Vec4<float>::load(cos_t + t), s = Vec4<float>::load(sin_t + t);
+    if (READ != kTogether) place();
     const float4 x1 = value4(p1, base + j), x2 = value4(p2, base + j + half);
+    if (READ == kTogether) place();
     if (head >= nq && slot < 0) return;
-    const int page = slot >= 0 ? slot / page_size : 0, off = slot >= 0 ? slot % page_size : 0;
     float4 a, b;
     rotate_pair(x1.x, x2.x, c.x, s.x, a.x, b.x);
     rotate_pair(x1.y, x2.y, c.y, s.y, a.y, b.y);
@@ -169,9 +186,10 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
     const int kvh = e / hd, d = e % hd;
     Value pv;
     ask4(pv, (nq + nkv) * hd + e);
+    if (READ != kTogether) place();
     const float4 v = value4(pv, (nq + nkv) * hd + e);
+    if (READ == kTogether) place();
     if (slot < 0) return;
-    const int page = slot / page_size, off = slot % page_size;
     TC* row = v_cache + ((static_cast<size_t>(page) * nkv + kvh) * hd + d) * page_size;
     row[off] = from_float<TC>(v.x);
     row[page_size + off] = from_float<TC>(v.y);
@@ -244,13 +262,16 @@ bool add_rmsnorm_vec(float* resid, const void* delta, int delta_dt, int n_partia
   // Which variant runs depends on the number of rows; what it computes does not (see the kernel).
   const bool wide = hidden > 1024;
   const bool few = n <= compute_units() && wide;  // a row a unit: spread over more threads
-#define PYRE_NORM_LAUNCH(THREADS, VIRT, STREAM)                                                                      \
-  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TG, TO, THREADS, VIRT, STREAM>), dim3(n), dim3(THREADS), 0, stream, \
+#define PYRE_NORM_LAUNCH(THREADS, VIRT, ...)                                                                         \
+  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TG, TO, THREADS, VIRT, __VA_ARGS__>), dim3(n), dim3(THREADS), 0, stream, \
                      resid, static_cast<const TD*>(delta), n_partials, hidden, static_cast<size_t>(partial_stride), rows, \
                      static_cast<const TG*>(gain), static_cast<TO*>(out), eps, bias)
   PYRE_DISPATCH(delta_dt, TD, PYRE_DISPATCH(gain_dt, TG, PYRE_DISPATCH(out_dt, TO, {
     const bool many = n >= 512;  // more bytes than the caches keep for the next kernel
+    const bool four = n_partials > 2 && static_cast<long>(n) * n_partials < 12000;
     if (few) PYRE_NORM_LAUNCH(1024, 1, false);
+    else if (wide && many && four) PYRE_NORM_LAUNCH(256, 4, true, true);
+    else if (many && four) PYRE_NORM_LAUNCH(256, 1, true, true);
     else if (wide && many) PYRE_NORM_LAUNCH(256, 4, true);
     else if (wide) PYRE_NORM_LAUNCH(256, 4, false);
     else if (many) PYRE_NORM_LAUNCH(256, 1, true);
@@ -269,16 +290,19 @@ bool rope_kv_write_vec(const void* qkv, int qkv_dt, int n_partials, long partial
   const int items = (nq + nkv) * (hd / 8) + nkv * (hd / 4);
   const dim3 grid(n, (items + 255) / 256);
   if (grid.y > 65535) return false;
-#define PYRE_ROPE_LAUNCH(STREAM)                                                                                   \
+#define PYRE_ROPE_LAUNCH(READ)                                                                                   \
   PYRE_DISPATCH(qkv_dt, TI, PYRE_DISPATCH(q_dt, TC,                                                               \
-      hipLaunchKernelGGL((rope_kv_write_vec_kernel<TI, TC, STREAM>), grid, dim3(256), 0, stream,                  \
+      hipLaunchKernelGGL((rope_kv_write_vec_kernel<TI, TC, READ>), grid, dim3(256), 0, stream,                  \
                          static_cast<const TI*>(qkv), static_cast<size_t>(partial_stride), n_partials, nq, nkv, hd, bias,  \
                          positions, write_kv ? slots : nullptr, cos_t, sin_t, bias_dt, page_size, static_cast<TC*>(q_out), \
                          static_cast<TC*>(k_cache), static_cast<TC*>(v_cache))))
   if (n >= 512) {
-    PYRE_ROPE_LAUNCH(true);
+    if (n_partials > 2 && n < 1200) PYRE_ROPE_LAUNCH(kStreamFour);
+    else PYRE_ROPE_LAUNCH(kStream);
+  } else if (static_cast<int>(n * grid.y) <= 4 * compute_units()) {
+    PYRE_ROPE_LAUNCH(kTogether);
   } else {
-    PYRE_ROPE_LAUNCH(false);
+    PYRE_ROPE_LAUNCH(kEach);
   }
 #undef PYRE_ROPE_LAUNCH
   return true;

@@ -149,6 +149,61 @@ def test_row_kernels_forms_for_rows_at_their_edges(many, parts):
         assert torch.allclose(got[0][2].double().permute(2, 0, 1), x[:, nq + nkv:], atol=tol)
 
 
+@pytest.mark.parametrize("many,parts", [(512, 2), (512, 3), (1199, 3), (1200, 3), (1199, 10), (1200, 10), (2048, 6)])
+def test_row_kernels_read_parts_one_or_four_at_a_time(many, parts):
+    """From 512 rows on the norm and the rotary kernel ask for a product's parts one or four at a time: the bits of the last rows alone."""
+    ops = _ops()
+    from pyre_amd.hip.ops import Partials
+
+    few = 5
+    for hidden in (512, 1536):
+        resid, delta, gain = rnd(many, hidden, seed=1), rnd(parts, many, hidden, seed=2), rnd(hidden, seed=4) + 1
+        out, r = torch.empty(many, hidden, device=DEV), resid.clone()
+        ops.add_rmsnorm(r, Partials(delta), gain, 1e-6, out)
+        out5, r5 = torch.empty(few, hidden, device=DEV), resid[-few:].clone()
+        ops.add_rmsnorm(r5, Partials(delta[:, -few:].contiguous()), gain, 1e-6, out5)
+        assert torch.equal(r5, r[-few:]) and torch.equal(out5, out[-few:])
+    check_rope_rows(ops, many, few, parts, 3, 1, 16)
+
+
+@pytest.mark.parametrize("nq,nkv,hd,rows", [(28, 4, 128, 341), (28, 4, 128, 342), (12, 2, 128, 511), (40, 8, 128, 256), (40, 8, 128, 257)])
+def test_rotary_on_both_sides_of_four_blocks_a_unit(nq, nkv, hd, rows):
+    """Up to four blocks a compute unit everything is asked for together, beyond one value after the other: the same bits."""
+    for parts in (1, 2, 13):
+        check_rope_rows(_ops(), rows, 3, parts, nq, nkv, hd)
+
+
+def check_rope_rows(ops, many, few, parts, nq, nkv, hd):
+    """The last rows of many have the bits that they have alone, with a cache and (the queries) without."""
+    from pyre_amd.hip.ops import Partials
+
+    width, page = (nq + 2 * nkv) * hd, 16
+    for dt in (torch.float32, torch.bfloat16):
+        qkv, bias = rnd(parts, many, width, seed=5), rnd(width, seed=6, dtype=dt)
+        cos, sin = rnd(many, hd // 2, seed=7), rnd(many, hd // 2, seed=8)
+        got = []
+        for lo in (0, many - few):
+            n = many - lo
+            at, slots = i32(list(range(lo, many))), i32(list(range(n)))
+            kc, vc = (torch.zeros(n // page + 1, nkv, *shape, device=DEV, dtype=dt) for shape in ((page, hd), (hd, page)))
+            q, alone = (torch.full((n, nq * hd), float("nan"), device=DEV, dtype=dt) for _ in range(2))
+            part = Partials(qkv[:, lo:].contiguous(), bias)
+            ops.rope_kv_write(part, q, kc, vc, cos, sin, hd, at, slots, n, nq, nkv, hd, page)
+            ops.rope_kv_write(part, alone, None, None, cos, sin, hd, at, None, n, nq, nkv, hd, page)
+            assert torch.equal(q, alone)
+            k, v = kc.transpose(1, 2).reshape(-1, nkv, hd)[:n], vc.permute(0, 3, 1, 2).reshape(-1, nkv, hd)[:n]
+            got.append((q[-few:], k[-few:], v[-few:]))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+        x = (qkv.double().sum(0) + bias.double())[-few:].view(few, nq + 2 * nkv, hd)
+        a, b, c, s = x[..., :hd // 2], x[..., hd // 2:], cos[-few:, None].double(), sin[-few:, None].double()
+        turned = torch.cat([a * c - b * s, b * c + a * s], -1)
+        # float32: the roundings of up to 13 additions and a rotation of values of up to 8 sqrt(parts); bfloat16: half a unit of 8 bits, twice
+        tol = 2e-5 if dt == torch.float32 else 2.0 ** -8 * float(x.abs().max()) * 4
+        assert torch.allclose(got[0][0].double().view(few, nq, hd), turned[:, :nq], atol=tol)
+        assert torch.allclose(got[0][1].double(), turned[:, nq:nq + nkv], atol=tol)
+        assert torch.allclose(got[0][2].double(), x[:, nq + nkv:], atol=tol)
+
+
 @pytest.mark.parametrize("adt,wdt", [("float32", "float32"), ("bfloat16", "bfloat16"), ("bfloat16", "float32")])
 @pytest.mark.parametrize("m,n,k", [(1, 37, 50), (5, 130, 257), (77, 200, 64), (130, 65, 1000)])
 def test_gemm_generic(adt, wdt, m, n, k):
