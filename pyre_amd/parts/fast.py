@@ -141,6 +141,28 @@ def few_tiles(n: int, n_out: int, k: int) -> int:
     return ops.gemm_tile_parts(-(-n // 64) * 64, n_out, k)
 
 
+#: features of a head from which its product of many rows is made in tiles, and the k up to which one of any size is
+HEAD_TILES_MIN_FEATURES, HEAD_TILES_MAX_SHORT_K = 120_000, 512
+#: whole rows of tiles of 256 -> the k up to which the head's product is made in tiles where up to 64 rows stand behind them
+HEAD_TILES_MAX_K_BEHIND = {1: 5120, 2: 2048}
+
+
+def head_in_tiles(n: int, n_out: int, k: int) -> bool:
+    """Whether the logits of ``n`` rows, more than the weight-streaming kernel takes, are made in tiles rather than by the library's product. k is
+    not split (the results go to their place), so a head of fewer features than about two rounds of tiles leaves a round
+    nearly empty here and there, and up to 64 rows behind whole rows of tiles of 256 cost a row of tiles of their own, the more the longer k.
+    Us in tiles and by the library: 151,936 x 1,536 111 and 128 at 65 rows, 142 and 152 at 190, 153 and 164 at 256, 179 and 197 at 257, 228 and
+    278 at 512, 282 and 304 at 513, 1,065 and 1,157 at 2,400; 152,064 x 3,584 219 and 231, 269 and 294, 289 and 322, 399 and 433, 459 and 554, but 609
+    and 588 at 513, 619 and 606 at 566 (from 577 rows on 620 and 694), 2,111 and 2,199 at 2,400; 152,064 x 5,120 866 and 816 at 513, 872 and 840 at 566;
+    151,936 x 8,192 941 and 866 at 257. 32,000 x 2,048 33 and 26 at 129, 48 and 37 at 257, though 55 and 57 at 512; 64,000 x 4,096 behind by 15 % at
+    257 and at 513, 100,352 x 4,096 by 11 % at 257, 128,256 x 4,096 ahead by 10 % there. With k of up to 512, where the results bound both,
+    ahead but for a few sizes that are alike, 3 % behind at worst (32,000 features: 0.47 of the library's time at 65 rows, 0.9 at 512)."""
+    if k <= HEAD_TILES_MAX_SHORT_K:
+        return True
+    whole, behind = divmod(n, 256)
+    return n_out >= HEAD_TILES_MIN_FEATURES and not (1 <= behind <= 64 and k > HEAD_TILES_MAX_K_BEHIND.get(whole, k))
+
+
 def library_takes(lin, rt, n: int) -> bool:
     """Whether the 16-bit product of ``n`` rows (more than the weight-streaming kernel's) and this weight is left to the BLAS
     library once no kernel for few rows takes it."""
@@ -218,18 +240,16 @@ def linear(lin, ctx, x, n, out):
         return rt.options.get("skinny_gemm", True) and ops.gemm_skinny_supports(min(n, SKINNY_MAX_ROWS), n_out, k, ldx, ldw)
 
     if out is not None:
-        # float32 results wanted in place (the head's logits). Of more rows than a block of the weight-streaming kernel keeps (a large
-        # decode step, every row of a portion) in tiles, whole: against the library's product, us on the 1.5B and 7B shapes' heads,
-        # 114 and 131, 221 and 232 at 65 rows, 144 and 153, 277 and 293 at 190, 155 and 168, 292 and 326 at 256, 237 and 275, 466
-        # and 563 at 512, 1,078 and 1,160, 2,120 and 2,212 at 2,400; behind by up to 4 % where a row of tiles of 256 is nearly empty (257
-        # rows 208 and 199, 566 309 and 305, 634 and 617).
-        if takes_tiles(rt, lin, n, x) and out.is_contiguous() and out.data_ptr() % 16 == 0:
+        # float32 results wanted in place (the head's logits): of more rows than a block of the weight-streaming kernel keeps (a large
+        # decode step, every row of a portion) in tiles, whole, where those are ahead of the library's product.
+        if ((not library or head_in_tiles(n, n_out, k)) and takes_tiles(rt, lin, n, x) and out.is_contiguous()
+                and out.data_ptr() % 16 == 0):
             ops.gemm_tile_bf16(x, weight, out, n, 1)
         elif (n <= SKINNY_MAX_ROWS or not library) and streams():  # no split, 64 rows at a time
             for r0 in range(0, n, SKINNY_MAX_ROWS):
                 rows = min(SKINNY_MAX_ROWS, n - r0)
                 ops.gemm_skinny_bf16(x[r0:r0 + rows], lin.weight, out[r0:r0 + rows], rows, 1)
-        elif library:
+        elif library:  # one pass over the weights
             torch.mm(x if n == x.shape[0] else x[:n], lin.weight.t(), out_dtype=torch.float32, out=out)
         else:
             return None

@@ -247,6 +247,29 @@ def test_which_kernel_takes_a_product_is_a_function_of_its_sizes():
             assert len({narrow_kernel(n, *shape) for n in range(lo + 1, hi + 1)}) == 1, (shape, lo, hi)
 
 
+@pytest.mark.parametrize("n_out,k", [(151936, 1536), (152064, 3584), (152064, 5120), (128256, 4096), (100352, 4096), (64000, 2048), (32000, 2048), (32000, 512),
+                                     (20016, 192), (120000, 2048)])
+@pytest.mark.parametrize("n", [65, 128, 190, 256, 257, 320, 321, 512, 513, 566, 576, 577, 634, 769, 2400])
+def test_which_kernel_makes_the_logits_of_many_rows(n, n_out, k, monkeypatch):
+    """The head's product in place: in tiles where those were measured ahead, else the library's."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from pyre_amd.parts import fast
+
+    made = []
+    monkeypatch.setattr(fast.ops, "gemm_tile_bf16", lambda *a: made.append("tiles"))
+    monkeypatch.setattr(torch, "mm", lambda *a, **b: made.append("library"))
+    x, weight = (torch.empty(r, k, dtype=torch.bfloat16, device="meta") for r in (n, n_out))
+    out = torch.empty(n, n_out, device="meta")
+    lin = SimpleNamespace(in_features=k, out_features=n_out, weight=weight, bias=None, role="head")
+    rt = SimpleNamespace(dtype=torch.bfloat16, options={}, compute_units=DEFAULT_UNITS)
+    fast.linear(lin, SimpleNamespace(runtime=rt), x, n, out)
+    few_behind = (512 < n <= 576 and k > 2048) or (256 < n <= 320 and k > 5120)
+    assert made == ["tiles" if k <= 512 or (n_out >= 120000 and not few_behind) else "library"]
+
+
 @pytest.mark.parametrize("role,bias,k,left", [("attn.qkv", True, 1536, False), ("ffn.down", False, 8960, False), ("ffn.gate_up", False, 1536, False),
                                               ("ffn.gate_up", True, 1536, True), ("moe.up", False, 1536, True), ("attn.out", False, 1000, True)])
 def test_what_is_left_to_the_library(role, bias, k, left):
