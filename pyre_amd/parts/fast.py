@@ -129,13 +129,15 @@ FEW_TILES_MIN_ROWS, FEW_TILES_MAX_K, FEW_TILES_MAX_WEIGHTS = 129, 4608, 17 << 20
 def few_tiles(n: int, n_out: int, k: int) -> int:
     """In how many parts of k the kernel of tiles makes a product of so few rows that a block could keep them all, where it is ahead of the
     one that does so, else 0. From 129 rows on what a block takes from L2 (all rows again for every 64 or 128 rows of
-    W) bounds that kernel, and tiles of 64 x 128 fill the chip with fewer parts for the consumer to read. In a graph, weights from memory, us
-    there and here, at 129 to 150, 192 and 256 rows: the 1.5B shape's q/k/v 7.8 and 6.8, 8.3 and 7.0, 9.7 and 7.5, its attention output 7.6 and
-    6.5, 8.3 and 6.8, 9.6 and 7.1; the 7B shape's q/k/v 15.1 and 15.5 (7 parts and 2), 17.1 and 16.7, 19.2 and 17.4, its attention output 13.6 and 12.9
-    (8 parts and 3), 14.7 and 13.6, 17.7 and 15.2; 3,072 x 4,608 14.4 and 14.4 (9 parts and 3), 15.6 and 15.5, 18.7 and 16.7. At 128 rows they are
-    about alike; longer k and larger weights stay with it: the ways down (1.5B 13.1 and 14.7, 14.7 and 15.9, 17.4 and 17.0; 7B 41.7 and
-    45.4, 42.5 and 50.0, 50.3 and 51.1) and the 32B shape's (o 20.0 and 22.4, 21.8 and 24.3, 25.8 and 24.8). The parts are those of
-    the next multiple of 64 rows, at which such decode steps are captured."""
+    W) bounds that kernel, and tiles of 64 x 128 fill the chip with fewer parts for the consumer to read. In a graph, weights from memory, the norm that
+    reads the parts with it, us there and here at 129, 192 and 256 rows: the 1.5B shape's q/k/v 12.1 and 11.1, 13.3 and 12.3, 15.7 and 13.0, its
+    attention output 11.3 and 10.2, 12.7 and 11.2, 14.8 and 12.4; the 7B shape's q/k/v (7 parts, and 2 or 3) 22.9 and 19.0, 24.0 and 20.8, 26.6 and 22.5
+    (the products alone 15.4 and 14.9, 15.9 and 16.3, 19.0 and 17.0), its attention output (8 parts, and 3 or 4) 20.9 and 17.1, 22.6 and 18.1, 24.6 and
+    20.5; 3,072 x 4,608 22.0 and 18.1, 23.4 and 19.6, 24.9 and 21.6; 1,024 x 4,608 13.0 and 11.7, 15.0 and 12.7, 17.5 and 13.8; 4,096 x 4,096 23.1 and 19.4, 23.2
+    and 21.6, 26.6 and 21.6; 8,192 x 2,048 22.4 and 20.8, 23.9 and 22.5, 27.9 and 22.9, the least that is gained within these limits. At 128 rows they
+    are about alike. Beyond the limits the products alone (1.5B way down 13.1 and 14.7, 14.7 and 15.9, 17.4 and 17.0; 7B 41.7 and 45.4, 42.5
+    and 50.0, 50.3 and 51.1; the 32B shape's attention output 20.0 and 22.4, 21.8 and 24.3, 25.8 and 24.8) leave less to gain; 4,608 x 4,096 is ahead by 3 to 14 %
+    with its consumer. The parts are those of the next multiple of 64 rows, at which such decode steps are captured."""
     if not FEW_TILES_MIN_ROWS <= n <= MID_MAX_ROWS or k > FEW_TILES_MAX_K or n_out * k > FEW_TILES_MAX_WEIGHTS:
         return 0
     return ops.gemm_tile_parts(-(-n // 64) * 64, n_out, k)
@@ -205,7 +207,7 @@ def _narrow_kernel(n: int, n_out: int, k: int, units: int, block, wide_min_rows:
         # 4.43 against 4.47 ms at 32 requests, 5.20 against 5.29 at 48, 5.74 against 5.88 at 64 (at 8
         # and 16: 3.46 against 3.44, 3.79 against 3.77); of the 32B shape 35.5 against 36.2 at 64.
         # Against 64 rows of the weights a block: 7.78 against 7.94 ms at 96 requests, 8.86 against
-        # 8.90 at 128, 12.56 against 12.63 at 192, 15.25 against 15.34 at 256.
+        # 8.90 at 128, and where every product was made by this kernel 12.56 against 12.63 at 192, 15.25 against 15.34 at 256.
         ks = mid_ksplit(n_out, k, 128, units)
         if ks and 4 * -(-n_out // 128) * ks >= 3 * units:
             return "block", ks, True

@@ -247,6 +247,47 @@ def test_which_kernel_takes_a_product_is_a_function_of_its_sizes():
             assert len({narrow_kernel(n, *shape) for n in range(lo + 1, hi + 1)}) == 1, (shape, lo, hi)
 
 
+@pytest.mark.parametrize("n_out,k,few", [(2048, 1536, True), (1536, 1536, True), (4608, 3584, True), (3072, 4608, True), (1024, 4608, True), (1024, 4672, False),
+                                         (4352, 4096, True), (4368, 4096, False), (1536, 8960, False), (3584, 18944, False), (5120, 5120, False)])
+def test_which_kernel_a_product_of_few_rows_ends_up_with(n_out, k, few, monkeypatch):
+    """`narrow_kernel` and then `few_tiles`: up to 128 rows the kernel that keeps all rows in a block, from 129 to 256 the one of tiles in the
+    parts of the next multiple of 64 rows where k and the weights are within its limits, beyond 256 rows tiles; the same
+    at an eager step's rows and at those at which it is captured."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from pyre_amd.engine.batch import DECODE_ROW_BUCKETS
+    from pyre_amd.parts import fast
+
+    made = []
+    monkeypatch.setattr(fast.ops, "gemm_mid_bf16", lambda x, w, out, m, ks, wide=False: made.append(("block", ks, wide)))
+    monkeypatch.setattr(fast.ops, "gemm_tile_bf16", lambda x, w, out, m, parts: made.append(("tiles", parts, False)))
+    workspace = SimpleNamespace(get=lambda name, shape, dtype: torch.empty(shape, dtype=dtype, device="meta"))
+    rt = SimpleNamespace(dtype=torch.bfloat16, options={}, compute_units=DEFAULT_UNITS, workspace=workspace)
+    lin = SimpleNamespace(in_features=k, out_features=n_out, weight=torch.empty(n_out, k, dtype=torch.bfloat16, device="meta"), bias=None,
+                          role="attn.out", whole=False, partials_name="p")
+
+    def choice(n, **changed):
+        for name, value in changed.items():
+            monkeypatch.setattr(lin, name, value)
+        made.clear()
+        p = fast.linear(lin, SimpleNamespace(runtime=rt), torch.empty(n, k, dtype=torch.bfloat16, device="meta"), n, None)
+        assert len(made) == 1 and p.data.shape == (made[0][1], n, n_out)
+        return made[0]
+
+    for n in (65, 128):
+        assert choice(n)[0] == "block"
+    for n in (129, 150, 192, 193, 256):
+        assert choice(n) == (("tiles", fast.ops.gemm_tile_parts(-(-n // 64) * 64, n_out, k), False) if few else fast.narrow_kernel(n, n_out, k))
+    assert choice(257) == ("tiles", fast.ops.gemm_tile_parts(257, n_out, k), False)
+    edges = [b for b in DECODE_ROW_BUCKETS if 64 <= b <= 256]
+    for lo, hi in zip(edges, edges[1:]):
+        assert len({choice(n) for n in range(lo + 1, hi + 1)}) == 1
+    assert choice(200, whole=True) == fast.narrow_kernel(200, n_out, k)
+    assert choice(200, whole=False, role="ffn.gate_up") == fast.narrow_kernel(200, n_out, k)
+
+
 @pytest.mark.parametrize("n_out,k", [(151936, 1536), (152064, 3584), (152064, 5120), (128256, 4096), (100352, 4096), (64000, 2048), (32000, 2048), (32000, 512),
                                      (20016, 192), (120000, 2048)])
 @pytest.mark.parametrize("n", [65, 128, 190, 256, 257, 320, 321, 512, 513, 566, 576, 577, 634, 769, 2400])
