@@ -768,7 +768,7 @@ extern "C" int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int k
 extern "C" int pyre_gemm_f32_tile_choice(int M, int N, int K, int ksplit) {
   PYRE_REQUIRE(M > 0 && N > 0 && K > 0 && ksplit > 0, "gemm_f32_tile_choice: bad sizes");
   const int i = best_tile(M, N, part_of(K, ksplit), ksplit, nullptr);
-  return i == kMixed ? 1000 * 128 + 128 : 1000 * kTiles[i].bm + kTiles[i].bn;
+  return i == kMixed ? 1000 * (128 + 64) + 128 : 1000 * kTiles[i].bm + kTiles[i].bn;
 }
 
 // Whether up to 64 rows behind those that fill tiles of 128 go to tiles of 64 x 128.

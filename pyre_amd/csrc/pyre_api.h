@@ -72,7 +72,8 @@ int pyre_gemm_f32(const float* A, long lda, const float* W, long ldw, const void
 // the sum of the parts in their order, as a consumer of pyre_gemm_f32's partial sums forms it, bit for bit. More than 16
 // rows, K a multiple of 16, rows on 16 bytes.
 int pyre_gemm_f32_adds(int M, int N, int K, long lda, long ldw, int ksplit);
-// The tiles that a product of more than 32 rows in ksplit parts is made of: 1000 x rows + columns.
+// The tiles that a product of more than 32 rows in ksplit parts is made of: 1000 x rows + columns; 192128 for tiles of 128 x 128 and,
+// for the last rows, of 64 x 128.
 int pyre_gemm_f32_tile_choice(int M, int N, int K, int ksplit);
 // 1 if the last rows of such a product, up to 64 behind those that fill tiles of 128, are made in tiles of 64.
 int pyre_gemm_f32_tile_mixed(int M, int N, int K, int ksplit);

@@ -209,7 +209,7 @@ def test_every_size_of_tiles(m, n, tile, k, off):
 @pytest.mark.parametrize("m,n,k,ks", [(129, 32768, 160, 1), (192, 32768, 157, 1), (566, 2048, 1536, 8), (400, 1500, 8960, 14), (260, 20000, 160, 2)])
 def test_last_rows_in_smaller_tiles(m, n, k, ks):
     """Tiles of 128 rows with tiles of 64 behind them in one launch: the bits of a product of the last rows alone, bias, rows and columns past
-    the end, a part's end within a step, sums of all parts, and numbers that are not finite in either kind of tile."""
+    the end, a part's end within a step, and numbers that are not finite in either kind of tile; one launch for all parts in tiles of one size."""
     from pyre_amd.hip import ops
     from pyre_amd.hip.lib import lib
 
@@ -239,3 +239,36 @@ def test_last_rows_in_smaller_tiles(m, n, k, ks):
         for p in plain[1:]:
             total += p
         assert torch.equal(whole.nan_to_num(), total.nan_to_num())
+
+
+@pytest.mark.parametrize("m,n,k,ks", [(129, 32768, 160, 2), (192, 32700, 320, 3), (2049, 2048, 1536, 8), (2112, 2048, 1536, 8), (2305, 3584, 3584, 9)])
+def test_last_rows_in_smaller_tiles_with_all_parts_added(m, n, k, ks):
+    """The same tiles where a block adds all parts of k up itself: the bits of the parts added in their order, in the rows of the large
+    tiles and of the small ones, whole rows and columns past the end, numbers that are not finite or beyond the pieces in both."""
+    from pyre_amd.hip import ops
+    from pyre_amd.hip.lib import lib
+
+    assert lib().pyre_gemm_f32_tile_choice(m, n, k, 1) == 192128 and lib().pyre_gemm_f32_tile_mixed(m, n, k, 1) == 1
+    a, w = operands(m, n, k, 0)
+    behind = m // 128 * 128  # the first row of a small tile
+    for row, value, places in ((3, float("inf"), (k // 2,)), (40, 2e35, range(0, k, 7)), (100, float("nan"), (1,)), (behind - 1, 3e38, (3,)),
+                               (behind, -3e38, (k - 2,)), (m - 1, 1e30, (2, k // 2))):
+        a[row, list(places)] = value
+    if m - behind > 60:
+        a[behind + 33, 5], a[behind + 40, k - 1] = float("-inf"), float("nan")
+    w[n - 1, 4], w[n // 2, k - 3] = 1e33, -2e31
+    parts, whole = torch.full((ks, m, n), float("nan"), device=DEV), torch.full((m, n), float("nan"), device=DEV)
+    ops.gemm_f32(a, w, None, parts, m, ks)
+    ops.gemm_f32_whole(a, w, whole, m, ks)
+    want = parts[0].clone()
+    for p in parts[1:]:
+        want += p
+    assert torch.equal(whole.isnan(), want.isnan()) and torch.equal(whole.nan_to_num(), want.nan_to_num())
+    rows = torch.tensor(sorted({0, 3, 40, 100, behind - 2, behind - 1, behind, m - 1, *range(m - 70, m)}), device=DEV)  # in tiles of one size
+    assert lib().pyre_gemm_f32_tile_choice(len(rows), n, k, ks) != 192128
+    few = torch.empty(ks, len(rows), n, device=DEV)
+    ops.gemm_f32(a[rows].contiguous(), w, None, few, len(rows), ks)
+    assert torch.equal(few.nan_to_num(), parts[:, rows].nan_to_num())
+    exact = a[rows].double() @ w.double().T
+    fine, scale = exact.abs() < 1e38, a[rows].double().abs() @ w.double().abs().T
+    assert bool(((whole[rows].double() - exact)[fine].abs() <= 2.0 ** -21 * scale[fine]).all())
