@@ -57,8 +57,8 @@ def test_larger_sums(m, n, k, rows):
 
 
 #: the forms of the kernel: rows of x and of w of a tile, and the stages of 64 k that its ring holds
-SUMS = {(256, 256): 2, (256, 192): 2, (128, 192): 3, (128, 128): 4, (64, 128): 6}
-UNITS = {(256, 256): 2, (192, 256): 2, (192, 192): 2, (128, 256): 3, (96, 256): 3, (96, 192): 3}
+SUMS = {(256, 256): 2, (256, 192): 2, (128, 192): 3, (128, 128): 4, (64, 128): 5}
+UNITS = {(256, 256): 2, (192, 256): 2, (192, 192): 2, (128, 256): 2, (96, 256): 2, (96, 192): 3}
 CASES = ("whole tiles", "a row more", "columns past the end", "fewer stages than slots", "an edge before a whole tile")
 
 
@@ -139,9 +139,14 @@ def check_product(m, n, k, gated, tile, rest=None):
         assert float((out.double().sum(0) - want).abs().max()) <= bound(k) * max(1.0, k ** 0.5) * 4
 
 
-#: what the planner gives to no form: its smallest tiles are for products of one round, some of them for longer k only
-NEVER = {(False, (64, 128), CASES[4]), (True, (96, 192), CASES[4]), (False, (128, 192), CASES[3]), (True, (192, 192), CASES[3]),
-         (True, (96, 256), CASES[3]), (True, (96, 192), CASES[3])}
+#: what the planner gives to no form: its smallest tiles of gated units are for products of one round
+NEVER = {(True, (96, 192), CASES[4])}
+
+
+@pytest.mark.parametrize("gated,tile,case", sorted(NEVER))
+def test_what_no_form_is_given(gated, tile, case):
+    """What the next test leaves out is not there to be taken: with other costs of the tiles it has to be looked at again."""
+    assert (tile, case) not in sizes_of_every_form(gated)
 
 
 @pytest.mark.parametrize("gated,tile,case", [(g, t, c) for g, forms in ((False, SUMS), (True, UNITS)) for t in forms for c in CASES
@@ -162,8 +167,12 @@ def test_every_form_behind_a_cut(gated, tile):
 @pytest.mark.parametrize("m,n,k", [(2100, 25616, 64), (2300, 24576, 128), (1800, 25600, 192), (3000, 16400, 320)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_blocks_that_walk_short_tiles(m, n, k, gated):
-    """Several tiles a block, of no more stages than its ring has slots: what is asked for ahead is the next tiles'."""
+    """Several tiles of one to five stages a block, in rings of two slots (k = 64 and 128: no more stages than those): what is asked for
+    ahead is the next tiles'."""
     from pyre_amd.hip import ops
+
+    (rows, cols), _, _, _ = ops.gemm_tile_choice(m, n, k, gated, 1)
+    assert (UNITS if gated else SUMS)[rows, cols] == 2 and m // rows * (n // cols) > ops.compute_units()
 
     x, w = rnd(m, k, seed=8), rnd(n, k, seed=9, scale=0.2)
     want = x.double() @ w.double().T
@@ -177,6 +186,25 @@ def test_blocks_that_walk_short_tiles(m, n, k, gated):
         out = torch.full((1, m, n), float("nan"), device=DEV)
         ops.gemm_tile_bf16(x, w, out, m, 1)
         assert float((out[0].double() - want).abs().max()) <= bound(k) * float(want.std()) * 4
+
+
+@pytest.mark.parametrize("tile,m,n,k", [((128, 192), 641, 21808, 64), ((128, 192), 769, 18704, 128), ((128, 192), 769, 19088, 192),
+                                        ((128, 128), 129, 24912, 64), ((128, 128), 257, 16848, 128), ((128, 128), 257, 16592, 192),
+                                        ((128, 128), 257, 16496, 256), ((64, 128), 267, 11392, 64), ((64, 128), 170, 18608, 128),
+                                        ((64, 128), 190, 17808, 192), ((64, 128), 192, 18560, 256), ((64, 128), 192, 20720, 320)])
+def test_blocks_that_walk_short_tiles_in_longer_rings(tile, m, n, k):
+    """Several tiles a block, of no more stages than its ring of three to five slots has: the tiles behind the next one are asked for already, and
+    stores of several tiles stand among the loads that are counted, or (at an edge) do not."""
+    from pyre_amd.hip import ops
+
+    says, cut, _, _ = ops.gemm_tile_choice(m, n, k, False, 1)
+    assert says == tile and not cut and k // 64 <= SUMS[tile] and -(-m // tile[0]) * -(-n // tile[1]) > ops.compute_units()
+    x, w = rnd(m, k + 24, seed=1)[:, 8:k + 8], rnd(n, k + 8, seed=2)[:, :k]
+    want = x.double() @ w.double().T
+    for _ in range(3):
+        out = torch.full((1, m, n), float("nan"), device=DEV)
+        ops.gemm_tile_bf16(x, w, out, m, 1)
+        assert float((out[0].double() - want).abs().max()) <= bound(k) * max(1.0, k ** 0.5) * 4
 
 
 @pytest.mark.parametrize("unit", [None, (7.0, 1.702, 1.0), (0.0, float("inf"), 0.0, 0.0)])
