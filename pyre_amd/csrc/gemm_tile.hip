@@ -41,7 +41,6 @@ using namespace pyre;
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 constexpr int BK = 64;             // k of a stage
@@ -94,6 +93,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_tile_kernel(const bf16
   constexpr int STORES = CT * 2 * (OUT == kF32Out ? RT / 2 : OUT == kGated ? (RT + 7) / 8 : (RT + 3) / 4);
   static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0 && 2 * WN * RT0 % NW == 0 && 2 * WN * RT1 % NW == 0 && RT % 2 == 0 &&
                     (two ? L : (S - 2) * L) + STORES < 64 && (S - 1) * L + LB < 64, "rows divide over the waves, waits can be counted");
+  static_assert(RT0 * CT >= RT0 + CT && (!two || (S == 2 && RT1 * CT >= RT0 + CT && RT0 * CT >= RT1)),
+                "a step has a product for every operand that is read during it");
   __shared__ __attribute__((aligned(1024))) unsigned char lds[S * STAGE + NW * 4096];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, quad = lane >> 4, wm = wave % WM, wn = wave / WM;
@@ -398,7 +399,7 @@ constexpr TileCost kPages[] = {kSums[0], kSums[2], kSums[3]};
 constexpr int kMaxParts = 6;
 constexpr double kReadMb = 0.2;              // the consumer's reading of a further part, a megabyte
 // Megabytes a microsecond that weights come with at the most: a head's few last rows are a second pass over
-// weights that no cache holds (151,936 x 1,536, 54 rows: 92 us, 70 without this; 566 rows cut behind 512 took 346 us, whole 302).
+// weights that no cache holds (151,936 x 1,536, 54 rows: 92 us, 70 without this; 566 rows cut behind 512 took 346 us, whole 309).
 constexpr double kMbPerUs = 5.0;
 constexpr double kMostPartsBytes = 536870912.0;  // parts of k together take no more scratch memory than this
 
