@@ -130,8 +130,8 @@ class Engine:
         time the vendor libraries' kernels for each distinct many-row 16-bit product of
         this model that is left to them (:func:`pyre_amd.parts.fast.library_takes`: of the
         shapes that the framework's own kernels take none) and remember the fastest (torch's
-        TunableOp). Other row counts keep the libraries' own choice, and so do the head's
-        float32 logits. Returns the number of products tuned."""
+        TunableOp). Other row counts keep the libraries' own choice, and so do the logits of
+        heads whose product of many rows is the library's (:func:`pyre_amd.parts.fast.head_in_tiles`). Returns the number of products tuned."""
         import os
         import tempfile
 

@@ -4,7 +4,8 @@ Each function returns None / False when its fast path does not take the case
 (element type, sizes, alignment); the caller then runs the general kernel.
 Nothing here changes what is computed, only by which kernel. Sizes that no kernel
 of this framework takes go to the vendor's BLAS through ``torch.mm``, as the
-reference's products do (`pyre/model.py:84-87` are ``nn.Linear``); the true 32-bit
+reference's products do (`pyre/model.py:84-87` are ``nn.Linear``), and so do the
+logits of many rows where that is ahead (:func:`head_in_tiles`); the true 32-bit
 path never comes here.
 """
 
@@ -77,7 +78,8 @@ def mid_ksplit(n_out: int, k: int, block_rows: int = 64, units: int = DEFAULT_UN
     takes at least two parts of 384 k or more (shorter parts gain nothing and cost the consumer
     another addend; measured on the 1.5B, 7B and 32B shapes: q/k/v, the
     attention output and the feed-forward's way down take 9 to 20 us where the library takes 19
-    to 31, and 60 against 100 at 7B's way down; the wide gate/up product stays with the library)."""
+    to 31, and 60 against 100 at 7B's way down; a product too wide for that, gate/up without the gate in its
+    epilogue, is not this kernel's)."""
     blocks = -(-n_out // block_rows)
     ks = min(units // blocks, k // 384, MID_MAX_KSPLIT)
     while ks > 1 and (ks - 1) * (-(-(-(-k // ks)) // 64) * 64) >= k:
@@ -182,7 +184,8 @@ def narrow_kernel(n: int, n_out: int, k: int, options: dict | None = None,
     """Which of our kernels takes a 16-bit product of ``n`` rows whose result is handed on as partial
     sums: ("stream", parts of k, False) for the weight-streaming kernel, ("block", parts, wide) for the
     kernel that keeps the step's rows in a block (``wide``: 128 rows of the weights a block instead
-    of 64), ("", 0, False) for neither (the kernel of tiles then, or the BLAS library). A function of the sizes (and of the
+    of 64), ("", 0, False) for neither (the kernel of tiles then, or the BLAS library). From 129 rows on products of short k that it
+    answers "block" for are made in tiles after all (:func:`few_tiles`). A function of the sizes (and of the
     device's compute units, which an engine reads once) alone; the
     thresholds in rows lie just above sizes at which decode steps are captured, so that an eager step
     and its replay at the padded size agree."""
