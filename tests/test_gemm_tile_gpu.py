@@ -354,3 +354,34 @@ def test_few_rows_in_tiles_agree_with_their_captured_size(n, k):
         assert got[0].shape[0] == got[1].shape[0] and torch.equal(got[0][:, :eager], got[1])
         assert fast.few_tiles(captured, n, k) == (0 if captured == 128 else got[0].shape[0])
         assert float((got[0].double().sum(0) - want[:captured]).abs().max()) <= bound(k) * float(want.std()) * 4
+
+
+@pytest.mark.parametrize("n,k", [(2048, 4096), (8000, 8192), (16000, 5120), (32000, 2048), (64000, 1024), (100352, 2560)])
+def test_the_librarys_logits_in_a_graph(n, k):
+    """The heads of fewer features are the library's product, in captured steps (up to 256 rows) too: every replay has the bits of the eager
+    product of the rows that are there by then, with eager work on the same memory and synchronizations between the replays."""
+    from types import SimpleNamespace
+
+    from pyre_amd.hip import ops
+    from pyre_amd.parts import fast
+
+    weight = rnd(n, k, seed=2, scale=0.02)
+    lin = SimpleNamespace(in_features=k, out_features=n, weight=weight, bias=None, role="head")
+    ctx = SimpleNamespace(runtime=SimpleNamespace(dtype=torch.bfloat16, options={}, compute_units=ops.compute_units()))
+    for m in (96, 128, 192, 256):
+        assert not fast.head_in_tiles(m, n, k)
+        x, out, eager = rnd(m, k, seed=m), torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+        fast.linear(lin, ctx, x, m, out)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            fast.linear(lin, ctx, x, m, out)
+        for i in range(5):
+            x.copy_(rnd(m, k, seed=1000 + i))
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            fast.linear(lin, ctx, x, m, eager)
+            want = x.double() @ weight.double().T if i == 4 else None
+            assert torch.equal(out, eager)
+        assert float((out.double() - want).abs().max()) <= bound(k) * float(want.std()) * 4
